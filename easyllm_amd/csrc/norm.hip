@@ -419,11 +419,12 @@ extern "C" int ezl_rmsnorm_fwd(const void* x, const void* residual, const void* 
     }
     const int tpr = tpr_for((int)h);
     const int nchunk = ((int)h + tpr * 8 - 1) / (tpr * 8);
+    // whole row slots only: with tpr = 192 (1024 < h <= 1536) a 256-thread block would hold one slot and a third of another
     const int rpb = 256 / tpr;
     int64_t grid = (rows + rpb - 1) / rpb;
     if (grid > 256 * 16) grid = 256 * 16;
 #define LAUNCH(NC, RES)                                                                                             \
-    hipLaunchKernelGGL((rmsnorm_fwd_kernel<NC, RES>), dim3((unsigned)grid), dim3(256), 0, st, (const bf16_t*)x,      \
+    hipLaunchKernelGGL((rmsnorm_fwd_kernel<NC, RES>), dim3((unsigned)grid), dim3(rpb * tpr), 0, st, (const bf16_t*)x, \
                        (const bf16_t*)residual, (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, \
                        (int)rows, (int)h, eps, tpr)
     if (residual) {
