@@ -11,14 +11,16 @@
 // (2 stages x 2 operands x 32 KiB).  An operand whose reduction dimension is the strided one is kept as it lies in
 // memory ([k][256]) and read with ds_read_b64_tr_b16 (the LDS transpose read), so nothing is ever transposed in HBM.
 //
-// Main kernel (K % 64 == 0): MFMA 16x16x32 (8x4 tiles per wave); tiles go HBM -> LDS directly
-// (buffer_load_dwordx4 ... lds, no staging registers, no ds_write); bank conflicts are avoided by an XOR swizzle applied on
-// the global-address side.  A K tile is consumed in four phases (k half x M half) of 16 MFMAs; the fragments of the
-// next phase are read during the current one, the barrier that publishes the next stage sits in front of the last
-// phase, and the loads of tile kt+2 are issued under that phase's MFMAs.  A second kernel with register staging,
-// padded tiles and MFMA 32x32x16 covers K tails (K % 64 != 0).
-// The forward form and the fp32 weight-gradient form on long reductions run a 4-wave variant of the main kernel (128x128
-// wave tiles, one wave per SIMD).
+// Main kernels: MFMA 16x16x32; tiles go HBM -> LDS directly (buffer_load_dwordx4 ... lds, no staging registers, no ds_write);
+// bank conflicts are avoided by an XOR swizzle applied on the global-address side.  In the 8-wave kernel a K tile is consumed
+// in four phases (k half x M half) of 16 MFMAs; the fragments of the next phase are read during the current one, the barrier
+// that publishes the next stage sits in front of the last phase, and the loads of tile kt+2 are issued under that phase's
+// MFMAs.  The forward form and the fp32 weight-gradient form on long reductions run a 4-wave variant (128x128 wave tiles,
+// one wave per SIMD).
+// K tails (K % 64 != 0: a weight gradient over an odd number of tokens, a forward over a width like 688): the lanes of the
+// last K tile's loads that lie past K get an offset outside the buffer, which reads as zero; nothing else differs.  (A register-
+// staged kernel with padded tiles used to cover them; fp32 weight gradients of a 2048-wide layer over 4000 tokens, of which it
+// could not split the last round, took 1310 us against 960, a 1376-long input gradient in one launch instead of two 84 against 21.)
 // Blocks are renumbered so that each XCD (own L2) works on a contiguous band of tiles, 8 tiles tall.
 //
 // Tile counts that leave the last round of workgroups mostly empty (320 tiles on 256 CUs, or 64 tiles in all) are evened out
@@ -30,86 +32,9 @@
 
 namespace {
 
-// =================================================================================================
-// K-tail kernel: register-staged loads, padded tiles
-// =================================================================================================
 constexpr int BM = 256, BN = 256, BK = 64;
-constexpr int LDK = BK + 8;     // row stride (elements) of a k-contiguous tile  [256][72]
-constexpr int LDN = 256 + 32;   // row stride (elements) of a k-major tile       [64][288]
-constexpr int TILE = 256 * LDK; // == 64 * LDN elements per operand per stage
-static_assert(TILE == 64 * LDN, "both tile layouts must have the same footprint");
 
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-
-// ---- global -> register staging of one operand tile (2048 x 128-bit chunks over NT threads) ----
-template <bool KC, int NT, bool KTAIL>
-struct Stager {
-    static constexpr int NCH = 2048 / NT;   // chunks per thread
-    static constexpr int RSTEP = NT / 8;    // KC: tile rows between two chunks of a thread
-    static constexpr int KSTEP = NT / 32;   // non-KC: k rows between two chunks of a thread
-    uint32_t off[NCH];  // element offsets of this thread's chunks at k = 0
-    int kpos;           // (KC) k column of all chunks / (non-KC) k row of chunk 0
-    // dim = extent of the non-reduction dimension, first = first row/col of the block tile
-    __device__ __forceinline__ void init(int tid, int first, int dim, int64_t ld) {
-        if (KC) {
-            kpos = (tid & 7) * 8;
-#pragma unroll
-            for (int i = 0; i < NCH; ++i) {
-                int r = first + (tid >> 3) + RSTEP * i;
-                r = r < dim ? r : dim - 1;  // rows past the edge re-read the last row; their results are never stored
-                off[i] = (uint32_t)((int64_t)r * ld + kpos);
-            }
-        } else {
-            kpos = tid >> 5;
-            int c = first + (tid & 31) * 8;
-            c = c + 8 <= dim ? c : dim - 8;
-#pragma unroll
-            for (int i = 0; i < NCH; ++i) off[i] = (uint32_t)((int64_t)(kpos + KSTEP * i) * ld + c);
-        }
-    }
-    // k0 = first k of the tile; kadv = element offset of that k (k0 for KC, k0 * ld otherwise)
-    __device__ __forceinline__ void load(const bf16_t* __restrict__ base, int k0, int64_t kadv, int K, bf16x8* r) const {
-        const bf16_t* p = base + kadv;
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            if (KTAIL) {
-                const bool ok = KC ? (k0 + kpos < K) : (k0 + kpos + KSTEP * i < K);
-                bf16x8 z;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) z[j] = (bf16_t)0.0f;
-                r[i] = ok ? *reinterpret_cast<const bf16x8*>(p + off[i]) : z;
-            } else {
-                r[i] = *reinterpret_cast<const bf16x8*>(p + off[i]);
-            }
-        }
-    }
-    __device__ __forceinline__ void store(bf16_t* __restrict__ s, int tid, const bf16x8* r) const {
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            if (KC) *reinterpret_cast<bf16x8*>(s + ((tid >> 3) + RSTEP * i) * LDK + (tid & 7) * 8) = r[i];
-            else *reinterpret_cast<bf16x8*>(s + ((tid >> 5) + KSTEP * i) * LDN + (tid & 31) * 8) = r[i];
-        }
-    }
-};
-
-// ---- LDS -> MFMA operand fragment: 32 rows(or cols) x 16 k, lane holds 8 k of one row ----------
-// lane l: row = l & 31, k = 8 * (l >> 5) + 0..7
-template <bool KC>
-__device__ __forceinline__ bf16x8 frag(const bf16_t* __restrict__ s, int row0, int ks, int lane) {
-    if (KC) {
-        return *reinterpret_cast<const bf16x8*>(s + (row0 + (lane & 31)) * LDK + ks * 16 + (lane >> 5) * 8);
-    } else {
-        // a 16-lane group reads a 4(k) x 16(row) block; lane i of the group receives column i
-        const int q = lane >> 4;
-        const bf16_t* p = s + (ks * 16 + (q >> 1) * 8 + ((lane & 15) >> 2)) * LDN + row0 + (q & 1) * 16 + ((lane & 3) << 2);
-        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
-        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * LDN));
-        bf16x8 v;
-        v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
-        v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
-        return v;
-    }
-}
 
 template <typename OutT> __device__ __forceinline__ void store_out(OutT* p, float v, bool accumulate);
 template <> __device__ __forceinline__ void store_out<bf16_t>(bf16_t* p, float v, bool accumulate) {
@@ -118,110 +43,6 @@ template <> __device__ __forceinline__ void store_out<bf16_t>(bf16_t* p, float v
 template <> __device__ __forceinline__ void store_out<float>(float* p, float v, bool accumulate) {
     *p = accumulate ? v + *p : v;
 }
-
-// WAVES_M x WAVES_N waves tile the 256x256 block; a wave owns (256/WAVES_M) x (256/WAVES_N)
-template <bool A_KC, bool B_KC, typename OutT, bool KTAIL, int WAVES_M, int WAVES_N>
-__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-                                                                      OutT* __restrict__ C, int M, int N, int K, int64_t lda,
-                                                                      int64_t ldb, int64_t ldc, int accumulate, int tiles_m,
-                                                                      int tiles_n) {
-    constexpr int NT = WAVES_M * WAVES_N * 64;
-    constexpr int TM = BM / WAVES_M / 32, TN = BN / WAVES_N / 32;  // MFMA tiles per wave
-    __shared__ __attribute__((aligned(16))) bf16_t smem[4 * TILE];  // A0 B0 A1 B1
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-
-    // XCD-aware renumbering: hardware deals consecutive block ids round-robin to the 8 XCDs
-    const int nblocks = tiles_m * tiles_n;
-    int pid = blockIdx.x;
-    {
-        const int per = nblocks >> 3, rem = nblocks & 7, xcd = pid & 7, idx = pid >> 3;
-        pid = xcd * per + (xcd < rem ? xcd : rem) + idx;
-    }
-    constexpr int GROUP_M = 8;
-    const int group_size = GROUP_M * tiles_n;
-    const int group = pid / group_size;
-    const int first_m = group * GROUP_M;
-    const int gm = tiles_m - first_m < GROUP_M ? tiles_m - first_m : GROUP_M;
-    const int tm = first_m + (pid % group_size) % gm;
-    const int tn = (pid % group_size) / gm;
-    const int m0 = tm * BM, n0 = tn * BN;
-
-    Stager<A_KC, NT, KTAIL> sa;
-    Stager<B_KC, NT, KTAIL> sb;
-    // per-thread offsets are 32-bit and relative to the block's first row / column: operands of any size are addressable
-    A += A_KC ? (int64_t)m0 * lda : (int64_t)m0;
-    B += B_KC ? (int64_t)n0 * ldb : (int64_t)n0;
-    sa.init(tid, 0, M - m0, lda);
-    sb.init(tid, 0, N - n0, ldb);
-    constexpr int NCH = 2048 / NT;
-    bf16x8 ra[NCH], rb[NCH];
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    const int nk = (K + BK - 1) / BK;
-    const int64_t astep = A_KC ? BK : (int64_t)BK * lda;
-    const int64_t bstep = B_KC ? BK : (int64_t)BK * ldb;
-
-    sa.load(A, 0, 0, K, ra);
-    sb.load(B, 0, 0, K, rb);
-    sa.store(smem, tid, ra);
-    sb.store(smem + TILE, tid, rb);
-    if (nk > 1) {
-        sa.load(A, BK, astep, K, ra);
-        sb.load(B, BK, bstep, K, rb);
-    }
-    __syncthreads();
-
-    for (int kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        const bf16_t* sA = smem + cur * 2 * TILE;
-        const bf16_t* sB = sA + TILE;
-        if (kt + 1 < nk) {  // tile kt+1 sits in registers: park it in the other stage
-            sa.store(smem + (cur ^ 1) * 2 * TILE, tid, ra);
-            sb.store(smem + (cur ^ 1) * 2 * TILE + TILE, tid, rb);
-        }
-        if (kt + 2 < nk) {  // and start fetching tile kt+2, to land during this step's MFMAs
-            sa.load(A, (kt + 2) * BK, (int64_t)(kt + 2) * astep, K, ra);
-            sb.load(B, (kt + 2) * BK, (int64_t)(kt + 2) * bstep, K, rb);
-        }
-#pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
-            bf16x8 fa[TM], fb[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i] = frag<A_KC>(sA, wm * (TM * 32) + i * 32, ks, lane);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) fb[j] = frag<B_KC>(sB, wn * (TN * 32) + j * 32, ks, lane);
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-
-    // epilogue: lane holds column (lane & 31); register r is row 8*(r/4) + 4*(lane>>5) + r%4
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int col = n0 + wn * (TN * 32) + j * 32 + (lane & 31);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm * (TM * 32) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row < M && col < N) store_out<OutT>(C + (int64_t)row * ldc + col, acc[i][j][r], accumulate != 0);
-            }
-        }
-    }
-}
-
 
 // =================================================================================================
 // main kernel: direct-to-LDS loads, XOR-swizzled tiles
@@ -241,7 +62,7 @@ __device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int& 
     tn = (pid % group_size) / gm;
 }
 
-// Work split of a launch whose main kernel runs (K % 64 == 0): tile ids below `full` are one workgroup each; every later
+// Work split of a launch: tile ids below `full` are one workgroup each; every later
 // tile is computed by `nsplit` workgroups that each take a contiguous share of the K tiles and leave an fp32 partial tile.
 struct SplitPlan {
     int full, nsplit;
@@ -253,26 +74,38 @@ struct SplitPlan {
 #define SG_VMEM_R 0x020
 #define SG_DS_R 0x100
 
-// One operand tile = 32 wave-instructions of 1 KiB each (buffer_load_dwordx4 ... lds: lane l lands at base + 16 l).
-//   k-contiguous tile [256 rows][64 k]:  instruction q covers rows 8q..8q+7; chunk c of row r sits in slot c ^ ((r>>1)&7)
-//   k-major tile      [64 k][256 cols]:  instruction q covers k rows 2q, 2q+1; chunk c of k row sits in slot c ^ kmajor_swizzle(k)
+// chunk (16 B) permutation of a k-major tile row: keeps the transpose reads of one wave instruction (four k rows x 32 B in each
+// of four k octets) on distinct banks.  Rows of 128 or more columns all start at bank 0; a 64-column row is half the banks
+// wide, so the row's parity already separates two of the four rows.
+template <int R>
+__device__ __forceinline__ int kmajor_swizzle(int krow) {
+    if (R >= 128) return ((krow & 3) << 2) ^ (((krow >> 3) & 1) << 1);
+    return (((krow >> 1) & 1) << 2) ^ (((krow >> 3) & 1) << 1);
+}
+
+// One operand tile of R rows (k-contiguous) or columns (k-major) = R / 8 wave-instructions of 1 KiB each
+// (buffer_load_dwordx4 ... lds: lane l lands at base + 16 l).
+//   k-contiguous tile [R rows][64 k]:  instruction q covers rows 8q..8q+7; chunk c of row r sits in slot c ^ ((r>>1)&7)
+//   k-major tile      [64 k][R cols]:  instruction q covers 512 / R k rows; chunk c of k row sits in slot c ^ kmajor_swizzle(k)
 // Wave w issues instructions q = w*NI .. w*NI+NI-1, i.e. one contiguous NI KiB piece of the tile: M0 (the LDS base) is
-// written once per tile and the instruction offset i*1024 selects the KiB.  That offset is also added to the global
-// address, so the per-lane byte offsets are stored with i*1024 already subtracted; they are kept 4 KiB high (and the
+// written once per 4 KiB and the instruction offset (i & 3) * 1024 selects the KiB.  That offset is also added to the global
+// address, so the per-lane byte offsets are stored with it already subtracted; they are kept 4 KiB high (and the
 // buffer's base 4 KiB low) so that they stay non-negative.  The address is buffer base (scalar, advanced per K tile) +
 // 32-bit lane offset + immediate: no vector address arithmetic inside the K loop.
 // The buffer form of the load is used rather than the global one because the compiler books a global load to LDS as a
 // flat access that may touch both memories, and while one is in flight it turns every counted wait on the LDS fragment
 // reads into a full drain (lgkmcnt(0)); with buffer loads the waits inside the K loop are exact counts.
-// chunk (16 B) permutation of a k-major tile row: keeps the transpose reads of one wave instruction on distinct banks
-__device__ __forceinline__ int kmajor_swizzle(int krow) { return ((krow & 3) << 2) ^ (((krow >> 3) & 1) << 1); }
+constexpr uint32_t kBufBytes = 0x80000000u;  // every tile is addressed as a 2 GiB buffer: an offset of kBufBytes reads as zero
 
-template <bool KC, int NW>
-struct Loader {
-    static constexpr int NI = 32 / NW;
-    static_assert(NI * 1024 <= 4096, "instruction offsets are limited to 12 bits");
+template <bool KC, int R, int NW, bool KTAIL>
+struct TileLoader {
+    static constexpr int NI = R / 8 / NW;
+    static constexpr int CPR = R / 8;       // k-major: chunks per k row
+    static constexpr int KPI = 64 / CPR;    // k-major: k rows per instruction
     uint32_t off[NI];  // byte offsets from (operand base + k advance - 4096)
-    __device__ __forceinline__ void init(int lane, int wave, int first, int dim, int64_t ld) {
+    // dim: rows (columns) of the operand from this tile's first on; those past the edge re-read the last one, their results
+    // are never stored
+    __device__ __forceinline__ void init(int lane, int wave, int dim, int64_t ld) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int q = wave * NI + i;
@@ -280,38 +113,44 @@ struct Loader {
             if (KC) {
                 const int row = 8 * q + (lane >> 3);
                 const int c = (lane & 7) ^ ((row >> 1) & 7);
-                int gr = first + row;
-                gr = gr < dim ? gr : dim - 1;
+                const int gr = row < dim ? row : dim - 1;
                 e = (int64_t)gr * ld + c * 8;
             } else {
-                const int krow = 2 * q + (lane >> 5);
-                const int c = (lane & 31) ^ kmajor_swizzle(krow);
-                int col = first + c * 8;
+                const int krow = KPI * q + lane / CPR;
+                const int c = (lane % CPR) ^ kmajor_swizzle<R>(krow);
+                int col = c * 8;
                 col = col + 8 <= dim ? col : dim - 8;
                 e = (int64_t)krow * ld + col;
             }
-            off[i] = (uint32_t)(e * 2 + 4096 - i * 1024);
+            off[i] = (uint32_t)(e * 2 + 4096 - (i & 3) * 1024);
         }
     }
-    // gbase: operand base advanced to the tile's first k, as a byte pointer
-    template <int I>
-    __device__ __forceinline__ void issue_one(__amdgpu_buffer_rsrc_t gbase, bf16_t* piece) const {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(gbase, (lds_void*)piece, 16, off[I], 0, I * 1024, 0);
+    // gtile: the operand advanced to the tile's first k
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t base(const bf16_t* gtile) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(gtile)) - 4096, 0, kBufBytes, 0x00020000);
     }
-    __device__ __forceinline__ void issue(const bf16_t* __restrict__ gtile, bf16_t* stage, int wave) const {
-        // an unbounded raw buffer that starts 4 KiB below the tile
-        const __amdgpu_buffer_rsrc_t gbase = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<char*>(reinterpret_cast<const char*>(gtile)) - 4096, 0, 0xffffffffu, 0x00020000);
-        bf16_t* piece = stage + wave * (NI * 512);
-        issue_one<0>(gbase, piece);
-        if constexpr (NI > 1) issue_one<1>(gbase, piece);
-        if constexpr (NI > 2) issue_one<2>(gbase, piece);
-        if constexpr (NI > 3) issue_one<3>(gbase, piece);
+    // kv: how many of the tile's 64 k exist (looked at with KTAIL only; more than 64 is fine)
+    template <int I>
+    __device__ __forceinline__ void issue_at(__amdgpu_buffer_rsrc_t g, bf16_t* stage, int lane, int wave, int kv) const {
+        uint32_t o = off[I];
+        if (KTAIL && kv < BK) {
+            const int q = wave * NI + I;
+            const int k = KC ? ((lane & 7) ^ (((8 * q + (lane >> 3)) >> 1) & 7)) * 8 : KPI * q + lane / CPR;
+            o = k < kv ? o : kBufBytes;
+        }
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(g, (lds_void*)(stage + wave * (NI * 512) + (I >> 2) * 2048), 16, o, 0, (I & 3) * 1024, 0);
+    }
+    template <int I = 0>
+    __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t g, bf16_t* stage, int lane, int wave, int kv) const {
+        if constexpr (I < NI) {
+            issue_at<I>(g, stage, lane, wave, kv);
+            issue<I + 1>(g, stage, lane, wave, kv);
+        }
     }
 };
 
 // ---- LDS -> MFMA 16x16x32 operand fragment: 16 rows (or columns) x 32 k; lane l holds row l & 15, k = 8 (l >> 4) + 0..7 ----
-template <bool KC>
+template <bool KC, int R>
 __device__ __forceinline__ bf16x8 sfrag(const bf16_t* __restrict__ s, int row0, int ks, int lane) {
     if (KC) {
         const int row = row0 + (lane & 15);
@@ -321,10 +160,10 @@ __device__ __forceinline__ bf16x8 sfrag(const bf16_t* __restrict__ s, int row0, 
         // a 16-lane group reads an 8(k) x 16(row) block as two 4 x 16 transpose reads; lane i of the group receives column i
         const int krow = ks * 32 + (lane >> 4) * 8 + ((lane & 15) >> 2);
         const int col = row0 + ((lane & 3) << 2);
-        const int c = (col >> 3) ^ kmajor_swizzle(krow);
-        const bf16_t* p = s + krow * 256 + c * 8 + (col & 7);
+        const int c = (col >> 3) ^ kmajor_swizzle<R>(krow);
+        const bf16_t* p = s + krow * R + c * 8 + (col & 7);
         const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
-        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * 256));  // k + 4: same swizzle
+        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * R));  // k + 4: same swizzle
         bf16x8 v;
         v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
         v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
@@ -364,20 +203,37 @@ template <> struct Out4<float> { typedef f32x4 type; };
 //
 // MULTI: the reduction runs over up to three (A, B) pairs in turn, C (=|+=) A0 B0 + A1 B1 + A2 B2, all pairs with the same
 // leading dimensions: the input gradient of several linears that share their input (q / k / v, gate / up) in one launch,
-// summed in fp32, instead of one launch per pair that reads and rewrites the bf16 result.  K is the total reduction
-// length; pair 1 starts at K tile t1, pair 2 at t2 (INT_MAX when absent).
+// summed in fp32, instead of one launch per pair that reads and rewrites the bf16 result.  The kernel's K is pair 0's
+// length; pair 1 starts at K tile t1, pair 2 at t2 (nk when absent), nk tiles in all.
 struct KSegments {
     const bf16_t* A1;
     const bf16_t* B1;
     const bf16_t* A2;
     const bf16_t* B2;
-    int t1, t2;
+    int t1, t2, nk;
+    int K1, K2;
 };
 
-template <bool A_KC, bool B_KC, typename OutT, bool MULTI = false>
+// the (A, B) pair of K tile t, the tile's index inside it and how many of its 64 k exist: scalar selects
+template <bool MULTI>
+__device__ __forceinline__ void pick_segment(const bf16_t* A, const bf16_t* B, int K, const KSegments& seg, int& t, int& kv,
+                                             const bf16_t*& Ab, const bf16_t*& Bb) {
+    Ab = A;
+    Bb = B;
+    if constexpr (MULTI) {
+        const bool s1 = t >= seg.t1, s2 = t >= seg.t2;
+        Ab = s2 ? seg.A2 : (s1 ? seg.A1 : A);
+        Bb = s2 ? seg.B2 : (s1 ? seg.B1 : B);
+        t -= s2 ? seg.t2 : (s1 ? seg.t1 : 0);
+        K = s2 ? seg.K2 : (s1 ? seg.K1 : K);
+    }
+    kv = K - t * BK;
+}
+
+template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
 __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                        int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
-                                                       int tiles_m, int tiles_n, const SplitPlan plan, const KSegments seg = KSegments()) {
+                                                       int tiles_m, int tiles_n, const SplitPlan plan, const KSegments seg) {
     constexpr int NW = 8, WAVES_N = 4;
     __shared__ __attribute__((aligned(1024))) bf16_t smem[4 * DTILE];  // A0 B0 A1 B1
     const int tid = threadIdx.x, lane = tid & 63;
@@ -398,14 +254,14 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
     tile_of(pid, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
 
-    Loader<A_KC, NW> la;
-    Loader<B_KC, NW> lb;
+    TileLoader<A_KC, BM, NW, KTAIL> la;
+    TileLoader<B_KC, BN, NW, KTAIL> lb;
     // per-lane offsets are 32-bit and relative to the block's first row / column (a scalar 64-bit advance of the operand
     // base), so operands of more than 2^31 elements are addressable
     const int64_t a_blk = A_KC ? (int64_t)m0 * lda : (int64_t)m0;
     const int64_t b_blk = B_KC ? (int64_t)n0 * ldb : (int64_t)n0;
-    la.init(lane, wave, 0, M - m0, lda);
-    lb.init(lane, wave, 0, N - n0, ldb);
+    la.init(lane, wave, M - m0, lda);
+    lb.init(lane, wave, N - n0, ldb);
 
     f32x4 acc[8][4];
 #pragma unroll
@@ -415,7 +271,7 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
-    int nk = K / BK, kt0 = 0;  // this workgroup's K tiles: kt0 .. kt0 + nk - 1
+    int nk = MULTI ? seg.nk : (K + BK - 1) / BK, kt0 = 0;  // this workgroup's K tiles: kt0 .. kt0 + nk - 1
     if (split) {
         kt0 = (int)((int64_t)nk * part / plan.nsplit);
         nk = (int)((int64_t)nk * (part + 1) / plan.nsplit) - kt0;
@@ -427,11 +283,11 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
     bf16x8 fa[2][4], fb[2][4];
     auto read_a = [&](const bf16_t* sA, int ks, int half, int buf) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) fa[buf][i] = sfrag<A_KC>(sA, arow + half * 64 + i * 16, ks, lane);
+        for (int i = 0; i < 4; ++i) fa[buf][i] = sfrag<A_KC, 256>(sA, arow + half * 64 + i * 16, ks, lane);
     };
     auto read_b = [&](const bf16_t* sA, int ks, int buf) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) fb[buf][j] = sfrag<B_KC>(sA + DTILE, brow + j * 16, ks, lane);
+        for (int j = 0; j < 4; ++j) fb[buf][j] = sfrag<B_KC, 256>(sA + DTILE, brow + j * 16, ks, lane);
     };
     // B is the first MFMA operand: the accumulator then holds C^T fragments, i.e. a lane owns 4 consecutive columns of one
     // row of C, which it can store as one vector.
@@ -443,17 +299,12 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
                 acc[half * 4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[bbuf][j], fa[abuf][i], acc[half * 4 + i][j], 0, 0, 0);
     };
     auto issue_tile = [&](int t, int stage) {
-        const bf16_t* Ab = A;
-        const bf16_t* Bb = B;
+        const bf16_t *Ab, *Bb;
+        int kv;
         t += kt0;
-        if constexpr (MULTI) {  // scalar selects: which pair K tile t belongs to
-            const bool s1 = t >= seg.t1, s2 = t >= seg.t2;
-            Ab = s2 ? seg.A2 : (s1 ? seg.A1 : A);
-            Bb = s2 ? seg.B2 : (s1 ? seg.B1 : B);
-            t -= s2 ? seg.t2 : (s1 ? seg.t1 : 0);
-        }
-        la.issue(Ab + a_blk + (int64_t)t * astep, smem + stage * 2 * DTILE, wave);
-        lb.issue(Bb + b_blk + (int64_t)t * bstep, smem + stage * 2 * DTILE + DTILE, wave);
+        pick_segment<MULTI>(A, B, K, seg, t, kv, Ab, Bb);
+        la.issue(la.base(Ab + a_blk + (int64_t)t * astep), smem + stage * 2 * DTILE, lane, wave, kv);
+        lb.issue(lb.base(Bb + b_blk + (int64_t)t * bstep), smem + stage * 2 * DTILE + DTILE, lane, wave, kv);
     };
 
     issue_tile(0, 0);
@@ -461,7 +312,7 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
     // Pull the remaining kernel arguments into registers now: a scalar load still in flight inside the K loop shares the
     // counter of the LDS reads and would turn every counted wait on them into a full drain.
     asm volatile("" ::"s"(C), "s"(ldc), "s"(accumulate), "s"(plan.partial), "s"(plan.full), "s"(plan.nsplit));
-    if constexpr (MULTI) asm volatile("" ::"s"(seg.A1), "s"(seg.B1), "s"(seg.A2), "s"(seg.B2), "s"(seg.t1), "s"(seg.t2));
+    if constexpr (MULTI) asm volatile("" ::"s"(seg.A1), "s"(seg.B1), "s"(seg.A2), "s"(seg.B2), "s"(seg.t1), "s"(seg.t2), "s"(seg.K1), "s"(seg.K2));
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     __syncthreads();
     read_b(smem, 0, 0);
@@ -621,42 +472,9 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-// one operand tile for 4 waves: wave w issues instructions q = 8 w .. 8 w + 7 (8 KiB), in two groups of four that share an
-// LDS base (the instruction offset reaches 4 KiB)
-template <bool KC>
-struct Loader4 {
-    uint32_t off[8];
-    __device__ __forceinline__ void init(int lane, int wave, int dim, int64_t ld) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int q = wave * 8 + i;
-            int64_t e;
-            if (KC) {
-                const int row = 8 * q + (lane >> 3);
-                const int c = (lane & 7) ^ ((row >> 1) & 7);
-                const int gr = row < dim ? row : dim - 1;
-                e = (int64_t)gr * ld + c * 8;
-            } else {
-                const int krow = 2 * q + (lane >> 5);
-                const int c = (lane & 31) ^ kmajor_swizzle(krow);
-                int col = c * 8;
-                col = col + 8 <= dim ? col : dim - 8;
-                e = (int64_t)krow * ld + col;
-            }
-            off[i] = (uint32_t)(e * 2 + 4096 - (i & 3) * 1024);
-        }
-    }
-    // gbase: buffer that starts 4 KiB below the tile
-    template <int I>
-    __device__ __forceinline__ void issue_one(__amdgpu_buffer_rsrc_t gbase, bf16_t* stage, int wave) const {
-        bf16_t* piece = stage + wave * 4096 + (I >> 2) * 2048;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(gbase, (lds_void*)piece, 16, off[I], 0, (I & 3) * 1024, 0);
-    }
-};
-
 // C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base) and, for bf16, its
 // tile-relative byte offsets must fit 31 bits: the host side checks.
-template <bool A_KC, bool B_KC, typename OutT>
+template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                          int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
                                                          int tiles_m, int tiles_n, const SplitPlan plan) {
@@ -679,8 +497,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     tile_of(pid, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
 
-    Loader4<A_KC> la;
-    Loader4<B_KC> lb;
+    TileLoader<A_KC, BM, 4, KTAIL> la;
+    TileLoader<B_KC, BN, 4, KTAIL> lb;
     const int64_t a_blk = A_KC ? (int64_t)m0 * lda : (int64_t)m0;
     const int64_t b_blk = B_KC ? (int64_t)n0 * ldb : (int64_t)n0;
     la.init(lane, wave, M - m0, lda);
@@ -694,7 +512,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
-    int nk = K / BK, kt0 = 0;  // this workgroup's K tiles: kt0 .. kt0 + nk - 1
+    int nk = (K + BK - 1) / BK, kt0 = 0;  // this workgroup's K tiles: kt0 .. kt0 + nk - 1
     if (split) {
         kt0 = (int)((int64_t)nk * part / plan.nsplit);
         nk = (int)((int64_t)nk * (part + 1) / plan.nsplit) - kt0;
@@ -707,22 +525,22 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     // fragment f of a k half: f < 8 the B fragment f, else the A fragment f - 8
     auto read_frag = [&](const bf16_t* sA, int ks, int buf, auto F) {
         constexpr int f = decltype(F)::value;
-        if constexpr (f < 8) fb[buf][f] = sfrag<B_KC>(sA + DTILE, brow + f * 16, ks, lane);
-        else fa[buf][f - 8] = sfrag<A_KC>(sA, arow + (f - 8) * 16, ks, lane);
+        if constexpr (f < 8) fb[buf][f] = sfrag<B_KC, 256>(sA + DTILE, brow + f * 16, ks, lane);
+        else fa[buf][f - 8] = sfrag<A_KC, 256>(sA, arow + (f - 8) * 16, ks, lane);
     };
     __amdgpu_buffer_rsrc_t ga, gb;
+    int kv = BK;
     auto tile_bases = [&](int t) {
         t += kt0;
-        ga = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(A + a_blk + (int64_t)t * astep)) - 4096, 0,
-                                               0xffffffffu, 0x00020000);
-        gb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(B + b_blk + (int64_t)t * bstep)) - 4096, 0,
-                                               0xffffffffu, 0x00020000);
+        kv = K - t * BK;
+        ga = la.base(A + a_blk + (int64_t)t * astep);
+        gb = lb.base(B + b_blk + (int64_t)t * bstep);
     };
     // load l of a tile pair: l < 8 piece l of the A tile, else piece l - 8 of the B tile
     auto issue_load = [&](int stage, auto L) {
         constexpr int l = decltype(L)::value;
-        if constexpr (l < 8) la.template issue_one<l>(ga, smem + stage * 2 * DTILE, wave);
-        else lb.template issue_one<l - 8>(gb, smem + stage * 2 * DTILE + DTILE, wave);
+        if constexpr (l < 8) la.template issue_at<l>(ga, smem + stage * 2 * DTILE, lane, wave, kv);
+        else lb.template issue_at<l - 8>(gb, smem + stage * 2 * DTILE + DTILE, lane, wave, kv);
     };
     auto issue_tile = [&](int t, int stage) {
         tile_bases(t);
@@ -942,9 +760,9 @@ SplitPlan make_plan(int64_t tiles, int64_t nk, void* workspace, int64_t workspac
     return p;
 }
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % BK != 0) return 0;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    SplitPlan p = make_plan(tiles, K / BK, (void*)16, INT64_MAX);
+    SplitPlan p = make_plan(tiles, (K + BK - 1) / BK, (void*)16, INT64_MAX);
     return p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
 }
 
@@ -952,39 +770,41 @@ int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
 // against 103 at 64, 179 against 194 at 128)
 constexpr int kW4MinKTiles = 48;
 
+template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
+void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
+                 void* workspace, int64_t workspace_bytes, hipStream_t st) {
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, nk = (K + BK - 1) / BK;
+    const SplitPlan plan = make_plan((int64_t)tiles_m * tiles_n, nk, workspace, workspace_bytes);
+    const int split_tiles = tiles_m * tiles_n - plan.full;
+    const dim3 grid((unsigned)(plan.full + split_tiles * plan.nsplit));
+    bool w4 = false;
+    // The 4-wave kernel: forward form with a bf16 result, and weight-gradient form with an fp32 result (inside the steps
+    // 0.4 - 0.8 % faster than the 8-wave kernel although a single launch at K = 4096 is not: it moves a third fewer LDS
+    // bytes, and the steps are bound by power).  With a k-strided B only (input gradients) it gained nothing.
+    if constexpr ((A_KC && B_KC && sizeof(OutT) == 2) || (!A_KC && !B_KC && sizeof(OutT) == 4)) {
+        const int vec = 16 / (int)sizeof(OutT);
+        // (a launch that is split tiles only is judged by the length of a share)
+        const int w4_ktiles = plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk;
+        w4 = w4_ktiles >= kW4MinKTiles && N % vec == 0 && ldc % vec == 0 && ezl_aligned16(C) &&
+             (int64_t)ldc * (int64_t)sizeof(OutT) * BM < (1LL << 31);  // tile-relative byte offsets of C fit 31 bits
+        if (w4)
+            hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, KTAIL>), grid, dim3(256), 0, st, (const bf16_t*)A, (const bf16_t*)B, (OutT*)C,
+                               M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan);
+    }
+    if (!w4)
+        hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, false, KTAIL>), grid, dim3(512), 0, st, (const bf16_t*)A, (const bf16_t*)B,
+                           (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan, KSegments());
+    if (plan.nsplit > 1)
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, st, (OutT*)C, M, N, ldc,
+                           accumulate, tiles_m, tiles_n, plan);
+}
 template <bool A_KC, bool B_KC, typename OutT>
 void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
             void* workspace, int64_t workspace_bytes, hipStream_t st) {
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const dim3 grid((unsigned)(tiles_m * tiles_n)), block(512);
-    if (K % BK == 0) {
-        const SplitPlan plan = make_plan((int64_t)tiles_m * tiles_n, K / BK, workspace, workspace_bytes);
-        const int split_tiles = tiles_m * tiles_n - plan.full;
-        // The 4-wave kernel: forward form with a bf16 result, and weight-gradient form with an fp32 result (inside the steps
-        // 0.4 - 0.8 % faster than the 8-wave kernel although a single launch at K = 4096 is not: it moves a third fewer LDS
-        // bytes, and the steps are bound by power).  With a k-strided B only (input gradients) it gained nothing.
-        if constexpr ((A_KC && B_KC && sizeof(OutT) == 2) || (!A_KC && !B_KC && sizeof(OutT) == 4)) {
-            const int vec = 16 / (int)sizeof(OutT);
-            // (a launch that is split tiles only is judged by the length of a share)
-            const int w4_ktiles = plan.nsplit > 1 && plan.full == 0 ? K / BK / plan.nsplit : K / BK;
-            if (w4_ktiles >= kW4MinKTiles && N % vec == 0 && ldc % vec == 0 && ezl_aligned16(C) &&
-                (int64_t)ldc * (int64_t)sizeof(OutT) * BM < (1LL << 31)) {  // tile-relative byte offsets of C fit 31 bits
-                hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT>), dim3((unsigned)(plan.full + split_tiles * plan.nsplit)), dim3(256), 0, st,
-                                   (const bf16_t*)A, (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan);
-                if (plan.nsplit > 1)
-                    hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, st, (OutT*)C, M, N,
-                                       ldc, accumulate, tiles_m, tiles_n, plan);
-                return;
-            }
-        }
-        hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT>), dim3((unsigned)(plan.full + split_tiles * plan.nsplit)), block, 0, st,
-                           (const bf16_t*)A, (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan);
-        if (plan.nsplit > 1)
-            hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, st, (OutT*)C, M, N, ldc,
-                               accumulate, tiles_m, tiles_n, plan);
-    } else
-        hipLaunchKernelGGL((gemm_staged_kernel<A_KC, B_KC, OutT, true, 2, 4>), grid, block, 0, st, (const bf16_t*)A,
-                           (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n);
+    if (K % BK == 0)
+        launch_form<A_KC, B_KC, OutT, false>(A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
+    else
+        launch_form<A_KC, B_KC, OutT, true>(A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
 }
 
 // C = 0 for an empty reduction (a fill kernel rather than a memset node, so the call can be captured into a graph)
@@ -1053,17 +873,18 @@ extern "C" int ezl_gemm_bf16(const void* A, const void* B, void* C, int64_t M, i
 
 // C (=|+=) sum_i A[i] * B[i] over `count` operand pairs that share M, N and the leading dimensions; K[i] is the reduction
 // length of pair i.  The input gradient dx = sum_i dy_i W_i of linears that share their input is one such sum.  With up to
-// three pairs in the (a_kc = 1, b_kc = 0, bf16 output) form and every K[i] a positive multiple of 64 it is a single launch
-// that adds the products in fp32 and rounds once; otherwise the pairs go out as ezl_gemm_bf16 calls that accumulate into C.
+// three pairs in the (a_kc = 1, b_kc = 0, bf16 output) form and every K[i] positive it is a single launch that adds the
+// products in fp32 and rounds once; otherwise the pairs go out as ezl_gemm_bf16 calls that accumulate into C.
 extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void* const* B, void* C, int64_t M, int64_t N,
                                     const int64_t* K, int64_t lda, int64_t ldb, int64_t ldc, int a_kc, int b_kc, int out_dtype,
                                     int accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
     EZL_REQUIRE(count >= 1 && A && B && K, EZL_EINVAL, "ezl_gemm_bf16_ksplit: bad count or null argument array");
-    bool one_launch = count <= 3 && a_kc == 1 && b_kc == 0 && out_dtype == 0 && M > 0 && N > 0;
+    bool one_launch = count <= 3 && a_kc == 1 && b_kc == 0 && out_dtype == 0 && M > 0 && N > 0, tail = false;
     int64_t ktot = 0;
     for (int i = 0; i < count; ++i) {
         EZL_REQUIRE(K[i] >= 0, EZL_EINVAL, "ezl_gemm_bf16_ksplit: negative size");
-        one_launch = one_launch && K[i] > 0 && K[i] % BK == 0;
+        one_launch = one_launch && K[i] > 0;
+        tail = tail || K[i] % BK != 0;
         ktot += K[i];
     }
     if (!one_launch || count == 1) {
@@ -1078,6 +899,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
         EZL_REQUIRE(A[i] && B[i], EZL_EINVAL, "ezl_gemm_bf16: null pointer");
         EZL_REQUIRE(ezl_aligned16(A[i]) && ezl_aligned16(B[i]) && lda % 8 == 0 && ldb % 8 == 0, EZL_EINVAL,
                     "ezl_gemm_bf16: operands must be 16-byte aligned with leading dimensions that are multiples of 8");
+        EZL_REQUIRE(K[i] % 8 == 0, EZL_EUNSUPPORTED, "ezl_gemm_bf16: contiguous extent of A must be a multiple of 8");
         EZL_REQUIRE(lda >= K[i] && lda < (1LL << 22) && ldb < (1LL << 22), EZL_EUNSUPPORTED,
                     "ezl_gemm_bf16: leading dimension too small, or 2^22 or more");
     }
@@ -1086,17 +908,23 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     EZL_REQUIRE(tiles < (1LL << 31), EZL_EUNSUPPORTED, "ezl_gemm_bf16: too many tiles");
     KSegments seg;
-    seg.A1 = (const bf16_t*)A[1]; seg.B1 = (const bf16_t*)B[1];
-    seg.t1 = (int)(K[0] / BK);
-    seg.A2 = count > 2 ? (const bf16_t*)A[2] : seg.A1; seg.B2 = count > 2 ? (const bf16_t*)B[2] : seg.B1;
-    seg.t2 = count > 2 ? (int)((K[0] + K[1]) / BK) : 0x7fffffff;
+    auto ktiles = [&](int i) { return (int)((K[i] + BK - 1) / BK); };
+    seg.A1 = (const bf16_t*)A[1]; seg.B1 = (const bf16_t*)B[1]; seg.K1 = (int)K[1];
+    seg.t1 = ktiles(0);
+    seg.t2 = seg.nk = seg.t1 + ktiles(1);
+    if (count > 2) seg.nk += ktiles(2);
+    seg.A2 = count > 2 ? (const bf16_t*)A[2] : seg.A1; seg.B2 = count > 2 ? (const bf16_t*)B[2] : seg.B1; seg.K2 = count > 2 ? (int)K[2] : 0;
     const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
-    const SplitPlan plan = make_plan(tiles, ktot / BK, workspace, workspace_bytes);
+    const SplitPlan plan = make_plan(tiles, (ktot + BK - 1) / BK, workspace, workspace_bytes);
     const int split_tiles = (int)tiles - plan.full;
-    hipLaunchKernelGGL((gemm_d2l_kernel<true, false, bf16_t, true>), dim3((unsigned)(plan.full + split_tiles * plan.nsplit)), dim3(512), 0,
-                       (hipStream_t)stream, (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)ktot, lda, ldb, ldc,
-                       accumulate, tiles_m, tiles_n, plan, seg);
+#define EZL_MULTI(KT)                                                                                                                      \
+    hipLaunchKernelGGL((gemm_d2l_kernel<true, false, bf16_t, true, KT>), dim3((unsigned)(plan.full + split_tiles * plan.nsplit)), dim3(512), 0, \
+                       (hipStream_t)stream, (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc,     \
+                       accumulate, tiles_m, tiles_n, plan, seg)
+    if (tail) EZL_MULTI(true);
+    else EZL_MULTI(false);
+#undef EZL_MULTI
     if (plan.nsplit > 1)
         hipLaunchKernelGGL((gemm_split_reduce_kernel<bf16_t>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, (hipStream_t)stream,
                            (bf16_t*)C, (int)M, (int)N, ldc, accumulate, tiles_m, tiles_n, plan);

@@ -32,3 +32,50 @@ def test_rmsnorm_fwd_widths_that_do_not_divide_a_block(K, rows, h, fused):
     ref = z.float() * ref_rstd[:, None] * w.float()
     assert ((y.float() - ref).abs() <= ref.abs() * (2 ** -8) + 1e-6).all()
     assert torch.allclose(rstd, ref_rstd, rtol=1e-5)
+
+
+# ---- GEMM ------------------------------------------------------------------------------------------------------------
+def gemm_bound(A, B):
+    """Per element: K products of bf16 values are exact in fp32; summing K of them in any order is off by at most
+    K 2^-24 sum|a b| (taken 4 times too large); one rounding to bf16 on top where the result is bf16."""
+    K = A.shape[1]
+    return A.float().abs() @ B.float().abs() * (4 * K * 2.0 ** -24)
+
+
+def check_gemm(K, form, M, N, Kd, accumulate=False, seed=0):
+    """form 0 forward, 1 input gradient, 2 weight gradient with an fp32 result, 3 weight gradient with a bf16 result."""
+    A = rnd(M, Kd, seed=seed) if form < 2 else rnd(Kd, M, seed=seed).t()
+    B = rnd(N, Kd, seed=seed + 1).t() if form == 0 else rnd(Kd, N, seed=seed + 1)
+    dt = torch.float32 if form == 2 else torch.bfloat16
+    out = rnd(M, N, seed=seed + 2).to(dt) if accumulate else torch.full((M, N), float("nan"), device="cuda", dtype=dt)
+    ref = A.float() @ B.float() + (out.float() if accumulate else 0)
+    lda, ldb = max(A.stride()), max(B.stride())
+    K.gemm(A if form < 2 else A.t(), B.t() if form == 0 else B, M, N, Kd, lda, ldb, form < 2, form == 0, out=out, accumulate=accumulate)
+    tol = gemm_bound(A, B) + (ref.abs() * 2.0 ** -8 if dt == torch.bfloat16 else ref.abs() * 2.0 ** -22) + 1e-6
+    worst = ((out.float() - ref).abs() - tol).max().item()
+    assert worst <= 0, (form, M, N, Kd, accumulate, worst)
+
+
+@pytest.mark.parametrize("form,M,N,Kd", [
+    (0, 1024, 256, 688), (0, 300, 520, 8), (0, 256, 256, 56), (0, 256, 264, 4104), (1, 1024, 256, 688), (1, 257, 512, 72),
+    (2, 688, 256, 1531), (2, 256, 4096, 1), (2, 264, 248, 4097), (2, 512, 512, 63), (3, 256, 264, 65)])
+def test_gemm_k_tails(K, form, M, N, Kd):
+    """Reductions that are no multiple of the 64-wide K tile: the last tile's missing k read as zero."""
+    print("gemm", form, M, N, Kd, flush=True)
+    check_gemm(K, form, M, N, Kd)
+    check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
+
+
+@pytest.mark.parametrize("T,n_in,outs", [(300, 256, (688, 688)), (1024, 256, (256, 64, 72)), (129, 520, (8, 1000, 120))])
+def test_gemm_input_gradient_over_pairs_with_k_tails(K, T, n_in, outs):
+    print("dgrad multi", T, n_in, outs, flush=True)
+    ld = max(outs)
+    dys = [torch.zeros(T, ld, device="cuda", dtype=torch.bfloat16)[:, :o].copy_(rnd(T, o, seed=i)) for i, o in enumerate(outs)]
+    for dy, o in zip(dys, outs):  # what follows a row's valid part must not reach the result
+        if o < ld:
+            torch.as_strided(dy, (T, ld - o), (ld, 1), dy.storage_offset() + o).fill_(float("nan"))
+    ws = [rnd(o, n_in, seed=10 + i) for i, o in enumerate(outs)]
+    dx = K.linear_dgrad_multi(dys, ws)
+    A, B = torch.cat([d.contiguous() for d in dys], 1), torch.cat(ws, 0)
+    ref = A.float() @ B.float()
+    assert ((dx.float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
