@@ -19,22 +19,18 @@
 // one wave per SIMD).
 // K tails (K % 64 != 0: a weight gradient over an odd number of tokens, a forward over a width like 688): the lanes of the
 // last K tile's loads that lie past K get an offset outside the buffer, which reads as zero; nothing else differs.  (A register-
-// staged kernel with padded tiles used to cover them; fp32 weight gradients of a 2048-wide layer over 4000 tokens, of which it
-// could not split the last round, took 1310 us against 960, a 1376-long input gradient in one launch instead of two 84 against 21.)
+// staged kernel used to cover them, without split last rounds and without the one-launch input gradient: a training step over
+// 4 x 1000 tokens at h = 2048 took 4977 us with it and 4626 with these.)
 // Blocks are renumbered so that each XCD (own L2) works on a contiguous band of tiles, 8 tiles tall.
 //
 // Tile counts that leave the last round of workgroups mostly empty (320 tiles on 256 CUs, or 64 tiles in all) are evened out
 // by splitting the reduction of the tiles of that last round over several workgroups (given a workspace): each writes an
 // fp32 partial tile and a small kernel adds the partials in a fixed order, so results stay bit-reproducible.
-#include "common.h"
-
-#include <type_traits>
+//
+// Products that do not fill the chip with 256 x 256 tiles run on the smaller tiles of gemm_small.hip (see choose_plan).
+#include "gemm_tile.h"
 
 namespace {
-
-constexpr int BM = 256, BN = 256, BK = 64;
-
-typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
 template <typename OutT> __device__ __forceinline__ void store_out(OutT* p, float v, bool accumulate);
 template <> __device__ __forceinline__ void store_out<bf16_t>(bf16_t* p, float v, bool accumulate) {
@@ -49,19 +45,6 @@ template <> __device__ __forceinline__ void store_out<float>(float* p, float v, 
 // =================================================================================================
 constexpr int DTILE = 256 * 64;  // elements per operand per stage of the swizzled layout (32 KiB)
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-// tile id (in the banded order described above) -> tile coordinates
-__device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-    constexpr int GROUP_M = 8;
-    const int group_size = GROUP_M * tiles_n;
-    const int group = pid / group_size;
-    const int first_m = group * GROUP_M;
-    const int gm = tiles_m - first_m < GROUP_M ? tiles_m - first_m : GROUP_M;
-    tm = first_m + (pid % group_size) % gm;
-    tn = (pid % group_size) / gm;
-}
-
 // Work split of a launch: tile ids below `full` are one workgroup each; every later
 // tile is computed by `nsplit` workgroups that each take a contiguous share of the K tiles and leave an fp32 partial tile.
 struct SplitPlan {
@@ -73,103 +56,6 @@ struct SplitPlan {
 #define SG_MFMA 0x008
 #define SG_VMEM_R 0x020
 #define SG_DS_R 0x100
-
-// chunk (16 B) permutation of a k-major tile row: keeps the transpose reads of one wave instruction (four k rows x 32 B in each
-// of four k octets) on distinct banks.  Rows of 128 or more columns all start at bank 0; a 64-column row is half the banks
-// wide, so the row's parity already separates two of the four rows.
-template <int R>
-__device__ __forceinline__ int kmajor_swizzle(int krow) {
-    if (R >= 128) return ((krow & 3) << 2) ^ (((krow >> 3) & 1) << 1);
-    return (((krow >> 1) & 1) << 2) ^ (((krow >> 3) & 1) << 1);
-}
-
-// One operand tile of R rows (k-contiguous) or columns (k-major) = R / 8 wave-instructions of 1 KiB each
-// (buffer_load_dwordx4 ... lds: lane l lands at base + 16 l).
-//   k-contiguous tile [R rows][64 k]:  instruction q covers rows 8q..8q+7; chunk c of row r sits in slot c ^ ((r>>1)&7)
-//   k-major tile      [64 k][R cols]:  instruction q covers 512 / R k rows; chunk c of k row sits in slot c ^ kmajor_swizzle(k)
-// Wave w issues instructions q = w*NI .. w*NI+NI-1, i.e. one contiguous NI KiB piece of the tile: M0 (the LDS base) is
-// written once per 4 KiB and the instruction offset (i & 3) * 1024 selects the KiB.  That offset is also added to the global
-// address, so the per-lane byte offsets are stored with it already subtracted; they are kept 4 KiB high (and the
-// buffer's base 4 KiB low) so that they stay non-negative.  The address is buffer base (scalar, advanced per K tile) +
-// 32-bit lane offset + immediate: no vector address arithmetic inside the K loop.
-// The buffer form of the load is used rather than the global one because the compiler books a global load to LDS as a
-// flat access that may touch both memories, and while one is in flight it turns every counted wait on the LDS fragment
-// reads into a full drain (lgkmcnt(0)); with buffer loads the waits inside the K loop are exact counts.
-constexpr uint32_t kBufBytes = 0x80000000u;  // every tile is addressed as a 2 GiB buffer: an offset of kBufBytes reads as zero
-
-template <bool KC, int R, int NW, bool KTAIL>
-struct TileLoader {
-    static constexpr int NI = R / 8 / NW;
-    static constexpr int CPR = R / 8;       // k-major: chunks per k row
-    static constexpr int KPI = 64 / CPR;    // k-major: k rows per instruction
-    uint32_t off[NI];  // byte offsets from (operand base + k advance - 4096)
-    // dim: rows (columns) of the operand from this tile's first on; those past the edge re-read the last one, their results
-    // are never stored
-    __device__ __forceinline__ void init(int lane, int wave, int dim, int64_t ld) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int q = wave * NI + i;
-            int64_t e;
-            if (KC) {
-                const int row = 8 * q + (lane >> 3);
-                const int c = (lane & 7) ^ ((row >> 1) & 7);
-                const int gr = row < dim ? row : dim - 1;
-                e = (int64_t)gr * ld + c * 8;
-            } else {
-                const int krow = KPI * q + lane / CPR;
-                const int c = (lane % CPR) ^ kmajor_swizzle<R>(krow);
-                int col = c * 8;
-                col = col + 8 <= dim ? col : dim - 8;
-                e = (int64_t)krow * ld + col;
-            }
-            off[i] = (uint32_t)(e * 2 + 4096 - (i & 3) * 1024);
-        }
-    }
-    // gtile: the operand advanced to the tile's first k
-    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t base(const bf16_t* gtile) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(gtile)) - 4096, 0, kBufBytes, 0x00020000);
-    }
-    // kv: how many of the tile's 64 k exist (looked at with KTAIL only; more than 64 is fine)
-    template <int I>
-    __device__ __forceinline__ void issue_at(__amdgpu_buffer_rsrc_t g, bf16_t* stage, int lane, int wave, int kv) const {
-        uint32_t o = off[I];
-        if (KTAIL && kv < BK) {
-            const int q = wave * NI + I;
-            const int k = KC ? ((lane & 7) ^ (((8 * q + (lane >> 3)) >> 1) & 7)) * 8 : KPI * q + lane / CPR;
-            o = k < kv ? o : kBufBytes;
-        }
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(g, (lds_void*)(stage + wave * (NI * 512) + (I >> 2) * 2048), 16, o, 0, (I & 3) * 1024, 0);
-    }
-    template <int I = 0>
-    __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t g, bf16_t* stage, int lane, int wave, int kv) const {
-        if constexpr (I < NI) {
-            issue_at<I>(g, stage, lane, wave, kv);
-            issue<I + 1>(g, stage, lane, wave, kv);
-        }
-    }
-};
-
-// ---- LDS -> MFMA 16x16x32 operand fragment: 16 rows (or columns) x 32 k; lane l holds row l & 15, k = 8 (l >> 4) + 0..7 ----
-template <bool KC, int R>
-__device__ __forceinline__ bf16x8 sfrag(const bf16_t* __restrict__ s, int row0, int ks, int lane) {
-    if (KC) {
-        const int row = row0 + (lane & 15);
-        const int c = (ks * 4 + (lane >> 4)) ^ ((row >> 1) & 7);
-        return *reinterpret_cast<const bf16x8*>(s + row * 64 + c * 8);
-    } else {
-        // a 16-lane group reads an 8(k) x 16(row) block as two 4 x 16 transpose reads; lane i of the group receives column i
-        const int krow = ks * 32 + (lane >> 4) * 8 + ((lane & 15) >> 2);
-        const int col = row0 + ((lane & 3) << 2);
-        const int c = (col >> 3) ^ kmajor_swizzle<R>(krow);
-        const bf16_t* p = s + krow * R + c * 8 + (col & 7);
-        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
-        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * R));  // k + 4: same swizzle
-        bf16x8 v;
-        v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
-        v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
-        return v;
-    }
-}
 
 // Instruction-scheduling recipe for one phase (compile-time unrolled): one MFMA, then up to PER LDS reads while reads are
 // left, then up to PER_V global->LDS loads while loads are left.
@@ -192,44 +78,11 @@ struct SchedPhase {
     }
 };
 
-template <typename OutT> struct Out4;
-template <> struct Out4<bf16_t> { typedef bf16x4 type; };
-template <> struct Out4<float> { typedef f32x4 type; };
-
 // 8 waves (2 x 4), each owning 128 x 64 of the 256 x 256 block tile as 8 x 4 MFMA 16x16x32 tiles.  The 16x16x32 shape is
 // used because it sustains a higher clock than 32x32x16 under the board's power limit (fewer accumulator-register
 // accesses per flop).  A 64-wide K tile is worked off in four phases (k half, M half): a phase issues 16 MFMAs on 4 A and
 // 4 B fragments while the fragments of the next phase are read from LDS into the other register set.
 //
-// MULTI: the reduction runs over up to three (A, B) pairs in turn, C (=|+=) A0 B0 + A1 B1 + A2 B2, all pairs with the same
-// leading dimensions: the input gradient of several linears that share their input (q / k / v, gate / up) in one launch,
-// summed in fp32, instead of one launch per pair that reads and rewrites the bf16 result.  The kernel's K is pair 0's
-// length; pair 1 starts at K tile t1, pair 2 at t2 (nk when absent), nk tiles in all.
-struct KSegments {
-    const bf16_t* A1;
-    const bf16_t* B1;
-    const bf16_t* A2;
-    const bf16_t* B2;
-    int t1, t2, nk;
-    int K1, K2;
-};
-
-// the (A, B) pair of K tile t, the tile's index inside it and how many of its 64 k exist: scalar selects
-template <bool MULTI>
-__device__ __forceinline__ void pick_segment(const bf16_t* A, const bf16_t* B, int K, const KSegments& seg, int& t, int& kv,
-                                             const bf16_t*& Ab, const bf16_t*& Bb) {
-    Ab = A;
-    Bb = B;
-    if constexpr (MULTI) {
-        const bool s1 = t >= seg.t1, s2 = t >= seg.t2;
-        Ab = s2 ? seg.A2 : (s1 ? seg.A1 : A);
-        Bb = s2 ? seg.B2 : (s1 ? seg.B1 : B);
-        t -= s2 ? seg.t2 : (s1 ? seg.t1 : 0);
-        K = s2 ? seg.K2 : (s1 ? seg.K1 : K);
-    }
-    kv = K - t * BK;
-}
-
 template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
 __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                        int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
@@ -464,14 +317,6 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // back; the 8-wave kernel 1.05).  Used for the forward form (both operands k-contiguous, bf16 result) and for the
 // weight-gradient form with an fp32 result on long reductions; for input gradients and short reductions the 8-wave
 // kernel, which hides more of the prologue and the epilogue, is as fast or faster.
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
 // C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base) and, for bf16, its
 // tile-relative byte offsets must fit 31 bits: the host side checks.
 template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
@@ -759,11 +604,91 @@ SplitPlan make_plan(int64_t tiles, int64_t nk, void* workspace, int64_t workspac
     p.full = (int)(tiles - r); p.nsplit = s; p.partial = (float*)workspace;
     return p;
 }
+
+// ---- which tile shape, and over how many workgroups a tile's reduction is split ------------------------------------------
+// The time of a launch is estimated for every shape as rounds x (K tiles x rate + fixed) and the cheapest one taken.  The
+// rates (us per 64-wide K tile of one workgroup per CU, or of two sharing a CU; the lower figure with the chip nearly empty,
+// the higher one full: clock and L2 bandwidth give way) and fixed costs (us: first load, epilogue, a workgroup's start) are
+// fits to products timed back to back:
+//                 few workgroups      chip full         fixed     from (M x N x K, us)
+//   256 x 256     1.00                1.30              12        4096^3 96, 4096 x 4096 x 11008 239, 1531 x 11008 x 4096 115
+//   256 x 128     0.60                0.77               6        2048 x 768 x 768 12.5, x 2048 25; 4000 x 2048 x 2048 31, x 5504 71;
+//                                                                 1531 x 4096 x 4096 (3/4 full) 46, x 22016 227
+//   128 x 128     0.64 (one per CU)   0.98 (two)         3        2048 x 768 x 768 10.4, x 2048 23; 4000 x 2048 x 2048 35, x 5504 87
+//   64 x 64       0.33 (one per CU)   0.40 (two)         3        1024 x 256 x 256 3.8, x 768 6.4; 1167 x 1024 x 1024 8.9, x 5632 38
+//   64 x 64 by 8 waves  0.19          0.27               3.2      1024 x 256 x 768 5.3, 256 x 256 x 1024 5.7, 1024 x 1024 x 1167 7.3
+// A split reduction adds a launch and a trip of the fp32 partial tiles through the caches (2048 x 768 x 4096 as 256 x 128 tiles
+// split four ways: 26, of which 10 for that).
+constexpr double kReduceFixed = 4.0, kReduceBytesPerUs = 8e6;
+double reduce_cost(int64_t tiles, int64_t tile_elems, int64_t nsplit) {
+    return kReduceFixed + (double)tiles * tile_elems * nsplit * 8 / kReduceBytesPerUs;
+}
+double cost_256(int64_t tiles, int64_t nk, bool split_ok) {
+    const SplitPlan p = make_plan(tiles, nk, split_ok ? (void*)16 : nullptr, INT64_MAX);
+    auto round = [&](int64_t groups, int64_t k) { return k * (1.0 + 0.3 * groups / kCus) + 12; };
+    double t = (p.full / kCus) * round(kCus, nk);
+    if (p.full % kCus) t += round(p.full % kCus, nk);
+    if (p.nsplit > 1) {
+        const int64_t r = tiles - p.full;
+        t += round(r * p.nsplit, (nk + p.nsplit - 1) / p.nsplit) + reduce_cost(r, BM * BN, p.nsplit);
+    }
+    return t;
+}
+double cost_small(int kind, int64_t tiles, int64_t nk, int64_t nsplit) {
+    const int64_t groups = tiles * nsplit, share = (nk + nsplit - 1) / nsplit;
+    const bool two = kind == kTile128 || kind == kTile64;  // workgroups per CU
+    const double low = kind == kTile256x128 ? 0.60 : kind == kTile128 ? 0.64 : kind == kTile64 ? 0.33 : 0.19;
+    const double high = kind == kTile256x128 ? 0.77 : kind == kTile128 ? 0.98 : kind == kTile64 ? 0.40 : 0.27;
+    const double fixed = kind == kTile256x128 ? 6 : kind == kTile64Waves ? 3.2 : 3;
+    const int64_t slots = two ? 2 * kCus : kCus, rest = groups % slots;
+    double t = (groups / slots) * (share * high + fixed);
+    const double fill = (double)rest / kCus;  // (one workgroup per CU: the rate holds until the chip is nearly full)
+    if (rest) t += share * (two ? (rest > kCus ? high : low) : low + (high - low) * fill * fill * fill) + fixed;
+    if (nsplit > 1) t += reduce_cost(tiles, gemm_kind_bm(kind) * gemm_kind_bn(kind), nsplit);
+    return t;
+}
+
+int64_t tiles_of(int kind, int64_t M, int64_t N) {
+    const int64_t bm = gemm_kind_bm(kind), bn = gemm_kind_bn(kind);
+    return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+}
+// `count` products over the same nk K tiles in one launch (256 x 256 takes one product); `room`: workspace bytes
+GemmPlan choose_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room) {
+    GemmPlan best = {kTile256, 1};
+    double t_best = 1e30;
+    if (count == 1) {
+        const int64_t tiles = tiles_of(kTile256, M[0], N[0]);
+        const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
+        const int64_t need = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * 4 : 0;
+        t_best = cost_256(tiles, nk, need <= room);
+    }
+    for (int kind = kTile256x128; kind < kGemmKinds; ++kind) {
+        int64_t tiles = 0;
+        for (int i = 0; i < count; ++i) tiles += tiles_of(kind, M[i], N[i]);
+        if (tiles * 16 >= (1LL << 31)) continue;
+        for (int64_t s = 1; s <= 16; ++s) {
+            if (s > 1 && (kind == kTile64Waves || nk / s < 4 || tiles * s > 4 * kCus ||
+                          tiles * s * gemm_kind_bm(kind) * gemm_kind_bn(kind) * 4 > room))
+                break;
+            const double t = cost_small(kind, tiles, nk, s);
+            if (t < t_best) {
+                t_best = t;
+                best.kind = kind;
+                best.nsplit = (int)s;
+            }
+        }
+    }
+    return best;
+}
+// workspace of a product's plan; the 256 x 256 kernels' own where a launch has to fall back to them
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    SplitPlan p = make_plan(tiles, (K + BK - 1) / BK, (void*)16, INT64_MAX);
-    return p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
+    const int64_t nk = (K + BK - 1) / BK, tiles = tiles_of(kTile256, M, N);
+    const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
+    const int64_t big = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
+    const GemmPlan q = choose_plan(1, &M, &N, nk, INT64_MAX);
+    const int64_t small = q.nsplit > 1 ? tiles_of(q.kind, M, N) * q.nsplit * gemm_kind_bm(q.kind) * gemm_kind_bn(q.kind) * (int64_t)sizeof(float) : 0;
+    return q.kind == kTile256 ? big : (big > small ? big : small);
 }
 
 // the 4-wave kernel pays off from this many K tiles on (4096 x 4096 x K, forward form: 57 against 54 us at 32 tiles, 98
@@ -798,9 +723,29 @@ void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int
         hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, st, (OutT*)C, M, N, ldc,
                            accumulate, tiles_m, tiles_n, plan);
 }
+// the smaller-tile kernels store at 31-bit byte offsets inside a tile
+template <typename OutT>
+bool small_stores_ok(int64_t ldc) {
+    return ldc * (int64_t)sizeof(OutT) * 256 < (1LL << 31);
+}
 template <bool A_KC, bool B_KC, typename OutT>
 void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
             void* workspace, int64_t workspace_bytes, hipStream_t st) {
+    constexpr int form = A_KC ? (B_KC ? 0 : 1) : (sizeof(OutT) == 4 ? 2 : 3);
+    if constexpr (A_KC ? sizeof(OutT) == 2 : !B_KC) {
+        if (small_stores_ok<OutT>(ldc)) {
+            const int64_t m = M, n = N;
+            const GemmPlan plan = choose_plan(1, &m, &n, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
+            if (plan.kind != kTile256) {
+                GemmSmallArgs a = {};
+                a.p[0] = {(const bf16_t*)A, (const bf16_t*)B, C, lda, ldb, ldc, M, N, 0, 0, 0, accumulate};
+                a.K = K;
+                a.partial = (float*)workspace;
+                gemm_small_launch(form, false, plan, a, 1, st);
+                return;
+            }
+        }
+    }
     if (K % BK == 0)
         launch_form<A_KC, B_KC, OutT, false>(A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
     else
@@ -916,6 +861,19 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     seg.A2 = count > 2 ? (const bf16_t*)A[2] : seg.A1; seg.B2 = count > 2 ? (const bf16_t*)B[2] : seg.B1; seg.K2 = count > 2 ? (int)K[2] : 0;
     const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
+    if (small_stores_ok<bf16_t>(ldc)) {
+        const GemmPlan small = choose_plan(1, &M, &N, (ktot + BK - 1) / BK, workspace ? workspace_bytes : 0);
+        if (small.kind != kTile256) {
+            GemmSmallArgs a = {};
+            a.p[0] = {(const bf16_t*)A[0], (const bf16_t*)B[0], C, lda, ldb, ldc, (int)M, (int)N, 0, 0, 0, accumulate};
+            a.K = (int)K[0];
+            a.partial = (float*)workspace;
+            a.seg = seg;
+            gemm_small_launch(1, true, small, a, 1, (hipStream_t)stream);
+            EZL_LAUNCH_CHECK("ezl_gemm_bf16_ksplit");
+            return EZL_OK;
+        }
+    }
     const SplitPlan plan = make_plan(tiles, (ktot + BK - 1) / BK, workspace, workspace_bytes);
     const int split_tiles = (int)tiles - plan.full;
 #define EZL_MULTI(KT)                                                                                                                      \

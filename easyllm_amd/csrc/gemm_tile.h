@@ -1,0 +1,195 @@
+// Device code shared by the GEMM kernels (gemm.hip, gemm_small.hip): operand tiles in LDS, MFMA fragments, K segments.
+#pragma once
+#include "common.h"
+
+#include <type_traits>
+
+// MULTI: the reduction runs over up to three (A, B) pairs in turn, C (=|+=) A0 B0 + A1 B1 + A2 B2, all pairs with the same
+// leading dimensions: the input gradient of several linears that share their input (q / k / v, gate / up) in one launch,
+// summed in fp32, instead of one launch per pair that reads and rewrites the bf16 result.  The kernel's K is pair 0's
+// length; pair 1 starts at K tile t1, pair 2 at t2 (nk when absent), nk tiles in all.
+struct KSegments {
+    const bf16_t* A1;
+    const bf16_t* B1;
+    const bf16_t* A2;
+    const bf16_t* B2;
+    int t1, t2, nk;
+    int K1, K2;
+};
+
+namespace {
+
+constexpr int BM = 256, BN = 256, BK = 64;
+
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+typedef __attribute__((address_space(3))) void lds_void;
+
+// tile id (in the banded order described above) -> tile coordinates
+__device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
+    constexpr int GROUP_M = 8;
+    const int group_size = GROUP_M * tiles_n;
+    const int group = pid / group_size;
+    const int first_m = group * GROUP_M;
+    const int gm = tiles_m - first_m < GROUP_M ? tiles_m - first_m : GROUP_M;
+    tm = first_m + (pid % group_size) % gm;
+    tn = (pid % group_size) / gm;
+}
+
+// chunk (16 B) permutation of a k-major tile row: keeps the transpose reads of one wave instruction (four k rows x 32 B in each
+// of four k octets) on distinct banks.  Rows of 128 or more columns all start at bank 0; a 64-column row is half the banks
+// wide, so the row's parity already separates two of the four rows.
+template <int R>
+__device__ __forceinline__ int kmajor_swizzle(int krow) {
+    if (R >= 128) return ((krow & 3) << 2) ^ (((krow >> 3) & 1) << 1);
+    return (((krow >> 1) & 1) << 2) ^ (((krow >> 3) & 1) << 1);
+}
+
+// One operand tile of R rows (k-contiguous) or columns (k-major) = R / 8 wave-instructions of 1 KiB each
+// (buffer_load_dwordx4 ... lds: lane l lands at base + 16 l).
+//   k-contiguous tile [R rows][64 k]:  instruction q covers rows 8q..8q+7; chunk c of row r sits in slot c ^ ((r>>1)&7)
+//   k-major tile      [64 k][R cols]:  instruction q covers 512 / R k rows; chunk c of k row sits in slot c ^ kmajor_swizzle(k)
+// Wave w issues instructions q = w*NI .. w*NI+NI-1, i.e. one contiguous NI KiB piece of the tile: M0 (the LDS base) is
+// written once per 4 KiB and the instruction offset (i & 3) * 1024 selects the KiB.  That offset is also added to the global
+// address, so the per-lane byte offsets are stored with it already subtracted; they are kept 4 KiB high (and the
+// buffer's base 4 KiB low) so that they stay non-negative.  The address is buffer base (scalar, advanced per K tile) +
+// 32-bit lane offset + immediate: no vector address arithmetic inside the K loop.
+// The buffer form of the load is used rather than the global one because the compiler books a global load to LDS as a
+// flat access that may touch both memories, and while one is in flight it turns every counted wait on the LDS fragment
+// reads into a full drain (lgkmcnt(0)); with buffer loads the waits inside the K loop are exact counts.
+constexpr uint32_t kBufBytes = 0x80000000u;  // every tile is addressed as a 2 GiB buffer: an offset of kBufBytes reads as zero
+
+template <bool KC, int R, int NW, bool KTAIL>
+struct TileLoader {
+    static constexpr int NI = R / 8 / NW;
+    static constexpr int CPR = R / 8;       // k-major: chunks per k row
+    static constexpr int KPI = 64 / CPR;    // k-major: k rows per instruction
+    uint32_t off[NI];  // byte offsets from (operand base + k advance - 4096)
+    // dim: rows (columns) of the operand from this tile's first on; those past the edge re-read the last one, their results
+    // are never stored
+    __device__ __forceinline__ void init(int lane, int wave, int dim, int64_t ld) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int q = wave * NI + i;
+            int64_t e;
+            if (KC) {
+                const int row = 8 * q + (lane >> 3);
+                const int c = (lane & 7) ^ ((row >> 1) & 7);
+                const int gr = row < dim ? row : dim - 1;
+                e = (int64_t)gr * ld + c * 8;
+            } else {
+                const int krow = KPI * q + lane / CPR;
+                const int c = (lane % CPR) ^ kmajor_swizzle<R>(krow);
+                int col = c * 8;
+                col = col + 8 <= dim ? col : dim - 8;
+                e = (int64_t)krow * ld + col;
+            }
+            off[i] = (uint32_t)(e * 2 + 4096 - (i & 3) * 1024);
+        }
+    }
+    // gtile: the operand advanced to the tile's first k
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t base(const bf16_t* gtile) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(gtile)) - 4096, 0, kBufBytes, 0x00020000);
+    }
+    // kv: how many of the tile's 64 k exist (looked at with KTAIL only; more than 64 is fine)
+    template <int I>
+    __device__ __forceinline__ void issue_at(__amdgpu_buffer_rsrc_t g, bf16_t* stage, int lane, int wave, int kv) const {
+        uint32_t o = off[I];
+        if (KTAIL && kv < BK) {
+            const int q = wave * NI + I;
+            const int k = KC ? ((lane & 7) ^ (((8 * q + (lane >> 3)) >> 1) & 7)) * 8 : KPI * q + lane / CPR;
+            o = k < kv ? o : kBufBytes;
+        }
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(g, (lds_void*)(stage + wave * (NI * 512) + (I >> 2) * 2048), 16, o, 0, (I & 3) * 1024, 0);
+    }
+    template <int I = 0>
+    __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t g, bf16_t* stage, int lane, int wave, int kv) const {
+        if constexpr (I < NI) {
+            issue_at<I>(g, stage, lane, wave, kv);
+            issue<I + 1>(g, stage, lane, wave, kv);
+        }
+    }
+};
+
+// ---- LDS -> MFMA 16x16x32 operand fragment: 16 rows (or columns) x 32 k; lane l holds row l & 15, k = 8 (l >> 4) + 0..7 ----
+template <bool KC, int R>
+__device__ __forceinline__ bf16x8 sfrag(const bf16_t* __restrict__ s, int row0, int ks, int lane) {
+    if (KC) {
+        const int row = row0 + (lane & 15);
+        const int c = (ks * 4 + (lane >> 4)) ^ ((row >> 1) & 7);
+        return *reinterpret_cast<const bf16x8*>(s + row * 64 + c * 8);
+    } else {
+        // a 16-lane group reads an 8(k) x 16(row) block as two 4 x 16 transpose reads; lane i of the group receives column i
+        const int krow = ks * 32 + (lane >> 4) * 8 + ((lane & 15) >> 2);
+        const int col = row0 + ((lane & 3) << 2);
+        const int c = (col >> 3) ^ kmajor_swizzle<R>(krow);
+        const bf16_t* p = s + krow * R + c * 8 + (col & 7);
+        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
+        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * R));  // k + 4: same swizzle
+        bf16x8 v;
+        v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
+        v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
+        return v;
+    }
+}
+
+// the (A, B) pair of K tile t, the tile's index inside it and how many of its 64 k exist: scalar selects
+template <bool MULTI>
+__device__ __forceinline__ void pick_segment(const bf16_t* A, const bf16_t* B, int K, const KSegments& seg, int& t, int& kv,
+                                             const bf16_t*& Ab, const bf16_t*& Bb) {
+    Ab = A;
+    Bb = B;
+    if constexpr (MULTI) {
+        const bool s1 = t >= seg.t1, s2 = t >= seg.t2;
+        Ab = s2 ? seg.A2 : (s1 ? seg.A1 : A);
+        Bb = s2 ? seg.B2 : (s1 ? seg.B1 : B);
+        t -= s2 ? seg.t2 : (s1 ? seg.t1 : 0);
+        K = s2 ? seg.K2 : (s1 ? seg.K1 : K);
+    }
+    kv = K - t * BK;
+}
+
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+template <typename OutT> struct Out4;
+template <> struct Out4<bf16_t> { typedef bf16x4 type; };
+template <> struct Out4<float> { typedef f32x4 type; };
+
+}  // namespace
+
+// One product of a launch of the smaller-tile kernels (gemm_small.hip).
+struct GemmProblem {
+    const bf16_t* A;
+    const bf16_t* B;
+    void* C;
+    int64_t lda, ldb, ldc;
+    int M, N;
+    int tiles_m, tiles_n, first;  // tile grid, and the launch-wide id of its first tile (INT_MAX: no such product)
+    int accumulate;
+};
+
+// A launch: up to three independent products over the same K, or (K segments) one product over up to three operand pairs.
+constexpr int kMaxProblems = 3;
+struct GemmSmallArgs {
+    GemmProblem p[kMaxProblems];
+    int ntiles, K, nsplit;
+    float* partial;  // nsplit > 1: [ntiles][nsplit][tile] fp32
+    KSegments seg;
+};
+
+// Tile shapes of gemm_small.hip, and 0 for the 256 x 256 kernels of gemm.hip.
+enum GemmKind { kTile256 = 0, kTile256x128 = 1, kTile128 = 2, kTile64 = 3, kTile64Waves = 4, kGemmKinds = 5 };
+struct GemmPlan {
+    int kind, nsplit;
+};
+// form 0: A, B k-contiguous, bf16 result; 1: A k-contiguous, bf16 result (multi: over K segments); 2 / 3: neither, fp32 / bf16
+// result.  Sets the tile grids in `a` and launches; 256 rows of every problem's C must span less than 2 GiB.
+__attribute__((visibility("hidden"))) void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs& a, int count,
+                                                             hipStream_t stream);
+inline int64_t gemm_kind_bm(int kind) { return kind <= kTile256x128 ? 256 : (kind == kTile128 ? 128 : 64); }
+inline int64_t gemm_kind_bn(int kind) { return kind == kTile256 ? 256 : (kind <= kTile128 ? 128 : 64); }

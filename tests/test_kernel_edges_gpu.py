@@ -79,3 +79,51 @@ def test_gemm_input_gradient_over_pairs_with_k_tails(K, T, n_in, outs):
     A, B = torch.cat([d.contiguous() for d in dys], 1), torch.cat(ws, 0)
     ref = A.float() @ B.float()
     assert ((dx.float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
+
+
+@pytest.mark.parametrize("form,M,N,Kd", [
+    # 64 x 64, the waves share the reduction: fewer and more K tiles than waves, a ragged tail, one row, one vector of columns
+    (0, 65, 72, 1000), (2, 256, 264, 1531), (1, 1, 8, 520), (3, 8, 64, 449), (0, 64, 64, 64),
+    # 64 x 64: one and several K tiles per stage ring
+    (0, 1167, 1024, 1024), (1, 1000, 2056, 200), (2, 2048, 776, 2048), (3, 1544, 1032, 64),
+    # 128 x 128, whole and split
+    (1, 1167, 2816, 1032), (2, 2824, 1000, 1167), (0, 4100, 1800, 512), (2, 1024, 1032, 12000), (3, 1024, 1024, 9001),
+    # 256 x 128: one to four K tiles, tails, ragged edges, split
+    (0, 4001, 2056, 2048), (1, 1531, 4096, 712), (0, 4096, 2048, 64), (1, 4096, 2048, 128), (2, 4096, 2048, 192), (0, 4096, 2048, 200),
+    (1, 700, 3080, 5128), (3, 2048, 2048, 4000)])
+def test_gemm_smaller_tiles(K, form, M, N, Kd):
+    print("gemm", form, M, N, Kd, flush=True)
+    check_gemm(K, form, M, N, Kd)
+    check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
+
+
+@pytest.mark.parametrize("T,n_in,outs", [(1167, 1024, (1024, 256, 256)), (2048, 768, (2048, 2056)), (700, 3072, (3072, 1024, 1032)),
+                                         (4000, 2048, (2048, 2048, 2056)), (1024, 256, (256, 256, 256))])
+def test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs):
+    print("dgrad multi", T, n_in, outs, flush=True)
+    ld = max(outs)
+    dys = [torch.empty(T, ld, device="cuda", dtype=torch.bfloat16)[:, :o].copy_(rnd(T, o, seed=i)) for i, o in enumerate(outs)]
+    ws = [rnd(o, n_in, seed=10 + i) for i, o in enumerate(outs)]
+    A, B = torch.cat([d.contiguous() for d in dys], 1), torch.cat(ws, 0)
+    ref = A.float() @ B.float()
+    dx = K.linear_dgrad_multi(dys, ws)
+    assert ((dx.float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
+    K.linear_dgrad_multi(dys, ws, out=dx, accumulate=True)
+    assert ((dx.float() - 2 * ref).abs() <= 2 * gemm_bound(A, B) + ref.abs() * 2.0 ** -6 + 1e-6).all()
+
+
+def test_gemm_smaller_tiles_leave_what_is_outside_the_result_alone(K):
+    """The stores past a tile's last row or column drop out: neighbours of a result that is a view stay as they were."""
+    for form, M, N, Kd, extra in ((0, 65, 72, 1000, 16), (0, 1001, 1000, 1024, 16), (0, 4001, 2056, 256, 16), (2, 1000, 1000, 1100, 16),
+                                  (0, 65, 71, 1000, 9), (0, 1001, 1003, 1024, 11), (0, 4001, 2049, 256, 13), (0, 700, 3075, 3072, 9)):
+        dt = torch.float32 if form == 2 else torch.bfloat16  # (odd widths: element-wise stores)
+        big = torch.full((M + 3, N + extra), 7.0, device="cuda", dtype=dt)
+        A = rnd(M, Kd, seed=1) if form == 0 else rnd(Kd, M, seed=1)
+        B = rnd(N, Kd, seed=2) if form == 0 else rnd(Kd, N, seed=2)
+        K.gemm(A, B, M, N, Kd, A.stride(0), B.stride(0), form == 0, form == 0, out=big[1:M + 1, 8:N + 8])
+        Af, Bf = (A, B.t()) if form == 0 else (A.t(), B)
+        ref = Af.float() @ Bf.float()
+        assert ((big[1:M + 1, 8:N + 8].float() - ref).abs() <= gemm_bound(Af, Bf) + ref.abs() * 2.0 ** -8 + 1e-6).all(), (form, M, N, Kd)
+        border = big.clone()
+        border[1:M + 1, 8:N + 8] = 7.0
+        assert (border == 7.0).all(), (form, M, N, Kd)
