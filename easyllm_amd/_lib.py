@@ -3,6 +3,7 @@
 There is no fallback: if the library is missing, or a call fails, a RuntimeError is raised.
 """
 import ctypes
+import functools
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -63,6 +64,7 @@ _SPECIAL = {
 }
 
 _lib = None
+_functions = {}
 
 
 def exported_symbols():
@@ -82,6 +84,7 @@ def load():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = ctypes.c_int
+            _functions[name] = fn
         for name, (argtypes, restype) in _SPECIAL.items():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
@@ -92,10 +95,11 @@ def load():
 
 def call(name, *args):
     """Calls an int-returning entry point and raises RuntimeError with the library's message on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    if _lib is None:
+        load()
+    rc = _functions[name](*args)
     if rc != 0:
-        msg = lib.ezl_last_error()
+        msg = _lib.ezl_last_error()
         raise RuntimeError("%s failed (%d): %s" % (name, rc, msg.decode() if msg else "?"))
 
 
@@ -115,6 +119,7 @@ def attn_bwd_workspace_bytes(total_tokens, ndocs, nq, nk, d):
     return load().ezl_attn_bwd_workspace_bytes(total_tokens, ndocs, nq, nk, d)
 
 
+@functools.lru_cache(maxsize=1024)  # a function of the sizes alone
 def gemm_workspace_bytes(M, N, K):
     return load().ezl_gemm_workspace_bytes(M, N, K)
 

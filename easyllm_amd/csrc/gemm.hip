@@ -653,7 +653,7 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
     return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 // `count` products over the same nk K tiles in one launch (256 x 256 takes one product); `room`: workspace bytes
-GemmPlan choose_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room) {
+GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room) {
     GemmPlan best = {kTile256, 1};
     double t_best = 1e30;
     if (count == 1) {
@@ -680,13 +680,24 @@ GemmPlan choose_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, 
     }
     return best;
 }
+// The search takes 3 us, as long as a small product: a thread remembers its last 256 products by their sizes.
+GemmPlan choose_plan(int64_t M, int64_t N, int64_t nk, int64_t room) {
+    struct Entry {
+        int64_t M, N, nk, room;
+        GemmPlan plan;
+    };
+    static thread_local Entry memo[256] = {};
+    Entry& e = memo[(uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ nk * 0x165667B19E3779F9ull) >> 56];
+    if (e.M != M || e.N != N || e.nk != nk || e.room != room) e = {M, N, nk, room, find_plan(1, &M, &N, nk, room)};
+    return e.plan;
+}
 // workspace of a product's plan; the 256 x 256 kernels' own where a launch has to fall back to them
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int64_t nk = (K + BK - 1) / BK, tiles = tiles_of(kTile256, M, N);
     const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
     const int64_t big = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
-    const GemmPlan q = choose_plan(1, &M, &N, nk, INT64_MAX);
+    const GemmPlan q = choose_plan(M, N, nk, INT64_MAX);
     const int64_t small = q.nsplit > 1 ? tiles_of(q.kind, M, N) * q.nsplit * gemm_kind_bm(q.kind) * gemm_kind_bn(q.kind) * (int64_t)sizeof(float) : 0;
     return q.kind == kTile256 ? big : (big > small ? big : small);
 }
@@ -734,8 +745,7 @@ void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t 
     constexpr int form = A_KC ? (B_KC ? 0 : 1) : (sizeof(OutT) == 4 ? 2 : 3);
     if constexpr (A_KC ? sizeof(OutT) == 2 : !B_KC) {
         if (small_stores_ok<OutT>(ldc)) {
-            const int64_t m = M, n = N;
-            const GemmPlan plan = choose_plan(1, &m, &n, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
+            const GemmPlan plan = choose_plan(M, N, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
             if (plan.kind != kTile256) {
                 GemmSmallArgs a = {};
                 a.p[0] = {(const bf16_t*)A, (const bf16_t*)B, C, lda, ldb, ldc, M, N, 0, 0, 0, accumulate};
@@ -862,7 +872,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
     if (small_stores_ok<bf16_t>(ldc)) {
-        const GemmPlan small = choose_plan(1, &M, &N, (ktot + BK - 1) / BK, workspace ? workspace_bytes : 0);
+        const GemmPlan small = choose_plan(M, N, (ktot + BK - 1) / BK, workspace ? workspace_bytes : 0);
         if (small.kind != kTile256) {
             GemmSmallArgs a = {};
             a.p[0] = {(const bf16_t*)A[0], (const bf16_t*)B[0], C, lda, ldb, ldc, (int)M, (int)N, 0, 0, 0, accumulate};

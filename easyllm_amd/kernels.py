@@ -12,12 +12,15 @@ from . import _lib
 BF16 = torch.bfloat16
 
 
+# A launch of a small kernel costs the GPU 2 - 5 us, so what a wrapper spends around it is what a small model's step takes:
+# addresses and the stream go to ctypes as plain integers, and messages are only put together when they are raised.
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device as its raw handle (torch.cuda.current_stream() builds an object for it)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need(cond, msg):
@@ -26,7 +29,8 @@ def _need(cond, msg):
 
 
 def _bf16c(t, name):
-    _need(t.is_cuda and t.dtype == BF16 and t.is_contiguous(), "%s must be a contiguous bf16 GPU tensor" % name)
+    if not (t.dtype is BF16 and t.is_contiguous() and t.is_cuda):
+        raise ValueError("%s must be a contiguous bf16 GPU tensor" % name)
 
 
 # ------------------------------------------------------------------------------------- RMSNorm
@@ -224,9 +228,10 @@ def cast_f32_to_bf16(x):
 
 # ------------------------------------------------------------------------------------- GEMM
 def _rows_ld(t, name):
-    _need(t.is_cuda and t.dtype == BF16 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1],
-          "%s must be a bf16 2-D GPU tensor with unit inner stride" % name)
-    return t.stride(0)
+    st = t.stride()
+    if not (len(st) == 2 and st[1] == 1 and st[0] >= t.shape[1] and t.dtype is BF16 and t.is_cuda):
+        raise ValueError("%s must be a bf16 2-D GPU tensor with unit inner stride" % name)
+    return st[0]
 
 
 def gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out=None, out_dtype=BF16, accumulate=False):
@@ -242,30 +247,36 @@ def _span(t):
 
 def _extent_ok(t, rows, cols, ld):
     """True when a [rows x cols] operand with leading dimension ld lies inside tensor t."""
+    if t.shape == (rows, cols) and t.stride(0) == ld:
+        return ld >= cols
     if rows == 0 or cols == 0:
         return True
     return ld >= cols and _span(t) >= (rows - 1) * ld + cols
 
 
 def _gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out, out_dtype, accumulate):
-    _need(not (accumulate and out is None), "GEMM: accumulate needs the buffer to add to (out=...)")
+    if out is None:
+        _need(not accumulate, "GEMM: accumulate needs the buffer to add to (out=...)")
     for t, name in ((A, "A"), (B, "B")):
-        _need(t.is_cuda and t.dtype == BF16 and t.stride(-1) == 1, "GEMM operand %s must be a bf16 GPU tensor with unit inner stride" % name)
+        if not (t.dtype is BF16 and t.is_cuda and t.stride(-1) == 1):
+            raise ValueError("GEMM operand %s must be a bf16 GPU tensor with unit inner stride" % name)
     # A is M x K stored [m][k] (a_kc) or [k][m]; B is N x K stored [n][k] (b_kc) or [k][n]
     _need(_extent_ok(A, M, K, lda) if a_kc else _extent_ok(A, K, M, lda), "GEMM: A is smaller than M x K with this leading dimension")
     _need(_extent_ok(B, N, K, ldb) if b_kc else _extent_ok(B, K, N, ldb), "GEMM: B is smaller than N x K with this leading dimension")
     if out is None:
-        out = torch.empty(M, N, dtype=out_dtype, device=A.device)
-    _need(out.is_cuda and out.dim() == 2 and out.stride(1) == 1 and tuple(out.shape) == (M, N), "bad GEMM output")
-    _need(out.dtype in (BF16, torch.float32), "GEMM output must be bf16 or fp32")
+        out = torch.empty((M, N), dtype=out_dtype, device=A.device)
+    ost = out.stride()
+    _need(out.is_cuda and len(ost) == 2 and ost[1] == 1 and out.shape == (M, N), "bad GEMM output")
+    bf16_out = out.dtype is BF16
+    _need(bf16_out or out.dtype is torch.float32, "GEMM output must be bf16 or fp32")
     ws, ws_bytes = _gemm_workspace(M, N, K, A.device)
-    _lib.call("ezl_gemm_bf16", _p(A), _p(B), _p(out), M, N, K, lda, ldb, out.stride(0), 1 if a_kc else 0, 1 if b_kc else 0,
-              0 if out.dtype == BF16 else 1, 1 if accumulate else 0, _p(ws), ws_bytes, _stream())
+    _lib.call("ezl_gemm_bf16", A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, lda, ldb, ost[0], 1 if a_kc else 0, 1 if b_kc else 0,
+              0 if bf16_out else 1, 1 if accumulate else 0, _p(ws), ws_bytes, _stream())
     return out
 
 
 def _gemm_workspace(M, N, K, device):
-    """fp32 partial tiles for shapes whose last round of output tiles would leave most of the chip idle (None otherwise)."""
+    """fp32 partial tiles for shapes whose reductions are split over several workgroups (None otherwise)."""
     nbytes = _lib.gemm_workspace_bytes(M, N, K)
     return (torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes) if nbytes else (None, 0)
 
@@ -287,7 +298,6 @@ def linear_dgrad(dy2d, w, out=None, accumulate=False):
 def linear_dgrad_multi(dy2ds, ws, out=None, accumulate=False):
     """dx[T, in] (=|+=) sum_i dy_i[T, out_i] @ w_i[out_i, in]: the input gradient of linears that share their input.
     One launch when the dy_i share a row stride and the w_i theirs; otherwise one accumulating GEMM per pair."""
-    import ctypes
     n = len(dy2ds)
     _need(n == len(ws) and n >= 1, "linear_dgrad_multi: list lengths differ")
     _need(not (accumulate and out is None), "linear_dgrad_multi: accumulate needs the buffer to add to (out=...)")
@@ -304,7 +314,8 @@ def linear_dgrad_multi(dy2ds, ws, out=None, accumulate=False):
         out = torch.empty(T, n_in, dtype=BF16, device=dy2ds[0].device)
     _need(out.is_cuda and out.dim() == 2 and out.stride(1) == 1 and tuple(out.shape) == (T, n_in) and out.dtype == BF16, "bad GEMM output")
     wsp, wsp_bytes = _gemm_workspace(T, n_in, sum(w.shape[0] for w in ws), out.device)
-    _lib.call("ezl_gemm_bf16_ksplit", n, (ctypes.c_void_p * n)(*[_p(dy) for dy in dy2ds]), (ctypes.c_void_p * n)(*[_p(w) for w in ws]),
+    _lib.call("ezl_gemm_bf16_ksplit", n, (ctypes.c_void_p * n)(*[dy.data_ptr() for dy in dy2ds]),
+              (ctypes.c_void_p * n)(*[w.data_ptr() for w in ws]),
               _p(out), T, n_in, (ctypes.c_int64 * n)(*[w.shape[0] for w in ws]), ldas[0], ldbs[0], out.stride(0), 1, 0, 0,
               1 if accumulate else 0, _p(wsp), wsp_bytes, _stream())
     return out
@@ -341,9 +352,10 @@ def bias_grad(dy, main_grad=None, accumulate=False):
 # ------------------------------------------------------------------------------------- attention
 def _tok_strides(t, b):
     """(seq_stride, batch_stride) of a [s, b, heads, d] tensor whose heads*d block is contiguous."""
-    _need(t.is_cuda and t.dtype == BF16 and t.dim() == 4 and t.stride(3) == 1 and t.stride(2) == t.shape[3],
-          "attention tensors must be bf16 [s, b, heads, d] with contiguous heads*d")
-    return t.stride(0), (t.stride(1) if b > 1 else 0)
+    st = t.stride()
+    if not (len(st) == 4 and st[3] == 1 and st[2] == t.shape[3] and t.dtype is BF16 and t.is_cuda):
+        raise ValueError("attention tensors must be bf16 [s, b, heads, d] with contiguous heads*d")
+    return st[0], (st[1] if b > 1 else 0)
 
 
 def _cu_arg(cu_seqlens, b):
@@ -502,7 +514,8 @@ def scale_by_scalar_(x, scalar):
 
 # ------------------------------------------------------------------------------------- optimizer step
 def _f32c(t, name):
-    _need(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous(), "%s must be a contiguous fp32 GPU tensor" % name)
+    if not (t.dtype is torch.float32 and t.is_contiguous() and t.is_cuda):
+        raise ValueError("%s must be a contiguous fp32 GPU tensor" % name)
 
 
 def sumsq_partials():
@@ -530,7 +543,8 @@ def adamw_step(master, exp_avg, exp_avg_sq, grad, param, lr, beta1, beta2, eps, 
     """In-place AdamW update of (master, exp_avg, exp_avg_sq) from fp32 grad; param (bf16 or None) is refreshed from master."""
     for t, n in ((master, "master"), (exp_avg, "exp_avg"), (exp_avg_sq, "exp_avg_sq"), (grad, "grad")):
         _f32c(t, n)
-        _need(t.numel() == master.numel(), "%s size mismatch" % n)
+        if t.numel() != master.numel():
+            raise ValueError("%s size mismatch" % n)
     if param is not None:
         _bf16c(param, "param")
         _need(param.numel() == master.numel(), "param size mismatch")
