@@ -77,13 +77,13 @@ def cpu_baseline(w, flops):
 
 
 class GemmTimer:
-    """Per-launch timing of the GEMM kernel: while installed, every launch that goes through kernels.gemm or
+    """Per-launch timing of the GEMM kernels: while installed, every launch that goes through kernels.gemm, kernels.gemm_group or
     kernels.linear_dgrad_multi is bracketed by two events on the launch stream and (flops, start, end) is recorded."""
 
     def __init__(self, kernels):
         import torch
         self.kernels, self.torch, self.records = kernels, torch, []
-        self._gemm, self._multi = kernels.gemm, kernels.linear_dgrad_multi
+        self._gemm, self._multi, self._group = kernels.gemm, kernels.linear_dgrad_multi, kernels.gemm_group
 
     def __enter__(self):
         torch = self.torch
@@ -107,11 +107,18 @@ class GemmTimer:
             self.records.append((2.0 * dy2ds[0].shape[0] * ws[0].shape[1] * sum(w.shape[0] for w in ws), start, end))
             return out
 
-        self.kernels.gemm, self.kernels.linear_dgrad_multi = gemm, multi
+        def group(As, Bs, Ms, Ns, K, *a, **kw):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            self._group(As, Bs, Ms, Ns, K, *a, **kw)
+            end.record()
+            self.records.append((2.0 * K * sum(m * n for m, n in zip(Ms, Ns)), start, end))
+
+        self.kernels.gemm, self.kernels.linear_dgrad_multi, self.kernels.gemm_group = gemm, multi, group
         return self
 
     def __exit__(self, *exc):
-        self.kernels.gemm, self.kernels.linear_dgrad_multi = self._gemm, self._multi
+        self.kernels.gemm, self.kernels.linear_dgrad_multi, self.kernels.gemm_group = self._gemm, self._multi, self._group
         return False
 
 

@@ -34,6 +34,8 @@ SIGNATURES = {
     "ezl_bias_grad": [_vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp],
     "ezl_gemm_bf16": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _vp, _i64, _vp],
     "ezl_gemm_bf16_ksplit": [_i32, _vpp, _vpp, _vp, _i64, _i64, _i64p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _vp, _i64, _vp],
+    "ezl_gemm_bf16_group": [_i32, _vpp, _vpp, _vpp, _i64p, _i64p, _i64, _i64p, _i64p, _i64p, _i32, _i32, _i32, ctypes.POINTER(_i32), _vp,
+                            _i64, _vp],
     "ezl_attn_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i64p, _vp],
     "ezl_attn_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _f32,
                      _i64p, _vp, _i64, _vp],
@@ -59,6 +61,7 @@ _SPECIAL = {
     "ezl_embed_scatter_add_workspace_bytes": ([_i64, _i64], _i64),
     "ezl_attn_bwd_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64], _i64),
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
+    "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
     "ezl_sumsq_partials": ([], _i64),
     "ezl_location_idx_rows": ([_i64, _i64, _i64], _i64),
 }
@@ -122,6 +125,12 @@ def attn_bwd_workspace_bytes(total_tokens, ndocs, nq, nk, d):
 @functools.lru_cache(maxsize=1024)  # a function of the sizes alone
 def gemm_workspace_bytes(M, N, K):
     return load().ezl_gemm_workspace_bytes(M, N, K)
+
+
+@functools.lru_cache(maxsize=1024)
+def gemm_group_workspace_bytes(Ms, Ns, K):
+    n = len(Ms)
+    return load().ezl_gemm_group_workspace_bytes(n, (_i64 * n)(*Ms), (_i64 * n)(*Ns), K)
 
 
 def sumsq_partials():

@@ -653,7 +653,7 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
     return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 // `count` products over the same nk K tiles in one launch (256 x 256 takes one product); `room`: workspace bytes
-GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room) {
+GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr) {
     GemmPlan best = {kTile256, 1};
     double t_best = 1e30;
     if (count == 1) {
@@ -678,6 +678,7 @@ GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, in
             }
         }
     }
+    if (time) *time = t_best;
     return best;
 }
 // The search takes 3 us, as long as a small product: a thread remembers its last 256 products by their sizes.
@@ -691,6 +692,48 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t nk, int64_t room) {
     if (e.M != M || e.N != N || e.nk != nk || e.room != room) e = {M, N, nk, room, find_plan(1, &M, &N, nk, room)};
     return e.plan;
 }
+int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const int64_t* N) {
+    int64_t tiles = 0;
+    for (int i = 0; i < count; ++i) tiles += tiles_of(p.kind, M[i], N[i]);
+    return p.nsplit > 1 ? tiles * p.nsplit * gemm_kind_bm(p.kind) * gemm_kind_bn(p.kind) * (int64_t)sizeof(float) : 0;
+}
+// Products that share a reduction length (q / k / v or gate / up of one input, and their weight gradients) in one launch?  Worth
+// it where each of them leaves CUs idle: 1024 tokens at h = 256, q + k + v forward 3 x 4.7 us alone.  The launches of a long
+// batch fill the chip one by one, with the better 256 x 256 tiles (at 4096 tokens and h = 4096 one launch for q / k / v
+// measured 0.14 ms per four-layer step slower), and the estimate says so.
+constexpr double kLaunchGap = 2.5;  // us between two launches of a stream: ramp down, ramp up
+bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
+    struct Entry {
+        int64_t M[kMaxProblems], N[kMaxProblems], K, room;
+        GemmPlan plan;
+        int count;
+        bool one;
+    };
+    static thread_local Entry memo[64] = {};
+    uint64_t hash = K * 0x165667B19E3779F9ull + count;
+    for (int i = 0; i < count; ++i) hash = (hash ^ (uint64_t)M[i]) * 0x9E3779B97F4A7C15ull + (uint64_t)N[i] * 0xC2B2AE3D27D4EB4Full;
+    Entry& e = memo[hash >> 58];
+    bool same = e.count == count && e.K == K && e.room == room;
+    for (int i = 0; i < count && same; ++i) same = e.M[i] == M[i] && e.N[i] == N[i];
+    if (!same) {
+        const int64_t nk = (K + BK - 1) / BK;
+        double apart = kLaunchGap * (count - 1), together;
+        for (int i = 0; i < count; ++i) {
+            double t;
+            find_plan(1, &M[i], &N[i], nk, room, &t);
+            apart += t;
+            e.M[i] = M[i];
+            e.N[i] = N[i];
+        }
+        e.plan = find_plan(count, M, N, nk, room, &together);
+        e.one = together < apart;
+        e.K = K;
+        e.room = room;
+        e.count = count;
+    }
+    plan = e.plan;
+    return e.one;
+}
 // workspace of a product's plan; the 256 x 256 kernels' own where a launch has to fall back to them
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -698,7 +741,7 @@ int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
     const int64_t big = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
     const GemmPlan q = choose_plan(M, N, nk, INT64_MAX);
-    const int64_t small = q.nsplit > 1 ? tiles_of(q.kind, M, N) * q.nsplit * gemm_kind_bm(q.kind) * gemm_kind_bn(q.kind) * (int64_t)sizeof(float) : 0;
+    const int64_t small = small_plan_bytes(q, 1, &M, &N);
     return q.kind == kTile256 ? big : (big > small ? big : small);
 }
 
@@ -772,6 +815,23 @@ __global__ __launch_bounds__(256) void zero_c_kernel(OutT* __restrict__ C, int64
 }  // namespace
 
 
+static int check_operands(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int a_kc,
+                          int b_kc) {
+    EZL_REQUIRE(A && B, EZL_EINVAL, "ezl_gemm_bf16: null pointer");
+    EZL_REQUIRE(ezl_aligned16(A) && ezl_aligned16(B) && lda % 8 == 0 && ldb % 8 == 0, EZL_EINVAL,
+                "ezl_gemm_bf16: operands must be 16-byte aligned with leading dimensions that are multiples of 8");
+    // every 128-bit chunk must lie wholly inside or wholly outside the matrix
+    EZL_REQUIRE(a_kc ? (K % 8 == 0) : (M % 8 == 0), EZL_EUNSUPPORTED, "ezl_gemm_bf16: contiguous extent of A must be a multiple of 8");
+    EZL_REQUIRE(b_kc ? (K % 8 == 0) : (N % 8 == 0), EZL_EUNSUPPORTED, "ezl_gemm_bf16: contiguous extent of B must be a multiple of 8");
+    EZL_REQUIRE(lda >= (a_kc ? K : M) && ldb >= (b_kc ? K : N) && ldc >= N, EZL_EINVAL, "ezl_gemm_bf16: leading dimension too small");
+    // 32-bit byte offsets inside one 256-row (or 64-k-row) tile; the tile bases advance in 64 bits
+    EZL_REQUIRE(lda < (1LL << 22) && ldb < (1LL << 22) && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31), EZL_EUNSUPPORTED,
+                "ezl_gemm_bf16: a dimension of 2^31 or more, or a leading dimension of 2^22 or more");
+    const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    EZL_REQUIRE(tiles < (1LL << 31), EZL_EUNSUPPORTED, "ezl_gemm_bf16: too many tiles");
+    return EZL_OK;
+}
+
 // a_kc / b_kc: 1 if the operand's reduction index is its contiguous one
 //   A: a_kc ? A[m * lda + k] : A[k * lda + m]        B: b_kc ? B[n * ldb + k] : B[k * ldb + n]
 // out_dtype: 0 bf16, 1 fp32.  accumulate: C += A*B instead of C = A*B.
@@ -794,18 +854,7 @@ extern "C" int ezl_gemm_bf16(const void* A, const void* B, void* C, int64_t M, i
         }
         return EZL_OK;
     }
-    EZL_REQUIRE(A && B, EZL_EINVAL, "ezl_gemm_bf16: null pointer");
-    EZL_REQUIRE(ezl_aligned16(A) && ezl_aligned16(B) && lda % 8 == 0 && ldb % 8 == 0, EZL_EINVAL,
-                "ezl_gemm_bf16: operands must be 16-byte aligned with leading dimensions that are multiples of 8");
-    // every 128-bit chunk must lie wholly inside or wholly outside the matrix
-    EZL_REQUIRE(a_kc ? (K % 8 == 0) : (M % 8 == 0), EZL_EUNSUPPORTED, "ezl_gemm_bf16: contiguous extent of A must be a multiple of 8");
-    EZL_REQUIRE(b_kc ? (K % 8 == 0) : (N % 8 == 0), EZL_EUNSUPPORTED, "ezl_gemm_bf16: contiguous extent of B must be a multiple of 8");
-    EZL_REQUIRE(lda >= (a_kc ? K : M) && ldb >= (b_kc ? K : N) && ldc >= N, EZL_EINVAL, "ezl_gemm_bf16: leading dimension too small");
-    // 32-bit byte offsets inside one 256-row (or 64-k-row) tile; the tile bases advance in 64 bits
-    EZL_REQUIRE(lda < (1LL << 22) && ldb < (1LL << 22) && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31), EZL_EUNSUPPORTED,
-                "ezl_gemm_bf16: a dimension of 2^31 or more, or a leading dimension of 2^22 or more");
-    const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    EZL_REQUIRE(tiles < (1LL << 31), EZL_EUNSUPPORTED, "ezl_gemm_bf16: too many tiles");
+    if (const int rc = check_operands(A, B, M, N, K, lda, ldb, ldc, a_kc, b_kc)) return rc;
     hipStream_t st = (hipStream_t)stream;
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
 #define EZL_GEMM_CASE(AK, BKC, OT) \
@@ -897,5 +946,47 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
         hipLaunchKernelGGL((gemm_split_reduce_kernel<bf16_t>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, (hipStream_t)stream,
                            (bf16_t*)C, (int)M, (int)N, ldc, accumulate, tiles_m, tiles_n, plan);
     EZL_LAUNCH_CHECK("ezl_gemm_bf16_ksplit");
+    return EZL_OK;
+}
+
+// Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch.
+// ezl_gemm_group_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
+extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
+    if (count < 2 || count > kMaxProblems || !M || !N || K <= 0) return -1;
+    for (int i = 0; i < count; ++i)
+        if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
+    GemmPlan plan;
+    if (!group_plan(count, M, N, K, INT64_MAX, plan)) return -1;
+    return small_plan_bytes(plan, count, M, N);
+}
+
+extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
+                                   int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,
+                                   const int* accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
+    EZL_REQUIRE(count >= 1 && count <= kMaxProblems && A && B && C && M && N && lda && ldb && ldc && accumulate && K > 0, EZL_EINVAL,
+                "ezl_gemm_bf16_group: bad count, null argument array or empty reduction");
+    EZL_REQUIRE((out_dtype == 0 && (a_kc || !b_kc)) || (out_dtype == 1 && !a_kc && !b_kc), EZL_EUNSUPPORTED,
+                "ezl_gemm_bf16_group: forms are forward, input gradient and weight gradient");
+    EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16_group: workspace must be 16-byte aligned");
+    GemmSmallArgs a = {};
+    int64_t tiles = 0;
+    for (int i = 0; i < count; ++i) {
+        EZL_REQUIRE(C[i] && M[i] > 0 && N[i] > 0, EZL_EINVAL, "ezl_gemm_bf16_group: null pointer or empty product");
+        if (const int rc = check_operands(A[i], B[i], M[i], N[i], K, lda[i], ldb[i], ldc[i], a_kc, b_kc)) return rc;
+        EZL_REQUIRE(out_dtype == 0 ? small_stores_ok<bf16_t>(ldc[i]) : small_stores_ok<float>(ldc[i]), EZL_EUNSUPPORTED,
+                    "ezl_gemm_bf16_group: leading dimension of C too large");
+        a.p[i] = {(const bf16_t*)A[i], (const bf16_t*)B[i], C[i], lda[i], ldb[i], ldc[i], (int)M[i], (int)N[i], 0, 0, 0, accumulate[i]};
+        tiles += tiles_of(kTile64, M[i], N[i]);
+    }
+    EZL_REQUIRE(tiles < (1LL << 27), EZL_EUNSUPPORTED, "ezl_gemm_bf16_group: too many tiles");
+    GemmPlan plan;
+    group_plan(count, M, N, K, INT64_MAX, plan);
+    if (small_plan_bytes(plan, count, M, N) > (workspace ? workspace_bytes : 0)) group_plan(count, M, N, K, 0, plan);
+    if (plan.kind == kTile256) plan = {kTile256x128, 1};  // (a group of one: these kernels take one or more)
+    a.K = (int)K;
+    a.partial = (float*)workspace;
+    const int form = a_kc ? (b_kc ? 0 : 1) : (out_dtype == 1 ? 2 : 3);
+    gemm_small_launch(form, false, plan, a, count, (hipStream_t)stream);
+    EZL_LAUNCH_CHECK("ezl_gemm_bf16_group");
     return EZL_OK;
 }

@@ -69,14 +69,13 @@ class FanOutLinearFunction(torch.autograd.Function):
     def forward(ctx, x, *weights):
         x2d = x.reshape(-1, x.shape[-1])
         ctx.save_for_backward(x, *weights)
-        return tuple(K.linear_fwd(x2d, w).view(*x.shape[:-1], w.shape[0]) for w in weights)
+        return tuple(y.view(*x.shape[:-1], y.shape[1]) for y in K.linear_fwd_multi(x2d, weights))
 
     @staticmethod
     def backward(ctx, *dys):
         x, *weights = ctx.saved_tensors
         x2d = x.reshape(-1, x.shape[-1])
         dx = None
-        grads = []
         dy2ds = []
         for dy in dys:
             if dy is None:
@@ -88,18 +87,13 @@ class FanOutLinearFunction(torch.autograd.Function):
             pairs = [(dy2d, w) for dy2d, w in zip(dy2ds, weights) if dy2d is not None]
             if pairs:
                 dx = K.linear_dgrad_multi([a for a, _ in pairs], [b for _, b in pairs])
-        for i, (dy2d, w) in enumerate(zip(dy2ds, weights)):
-            if dy2d is None:
-                grads.append(None)
-                continue
-            dw = None
-            if ctx.needs_input_grad[1 + i]:
-                mg, acc = _main_grad_target(w)
-                if mg is not None:
-                    K.linear_wgrad(dy2d, x2d, out=mg, accumulate=acc)
-                else:
-                    dw = K.linear_wgrad(dy2d, x2d)
-            grads.append(dw)
+        wanted = [i for i, dy2d in enumerate(dy2ds) if dy2d is not None and ctx.needs_input_grad[1 + i]]
+        grads = [None] * len(weights)
+        if wanted:
+            targets = [_main_grad_target(weights[i]) for i in wanted]
+            dws = K.linear_wgrad_multi([dy2ds[i] for i in wanted], x2d, [mg for mg, _ in targets], [acc for _, acc in targets])
+            for i, (mg, _), dw in zip(wanted, targets, dws):
+                grads[i] = dw if mg is None else None
         return (None if dx is None else dx.view(x.shape),) + tuple(grads)
 
 

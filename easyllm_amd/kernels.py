@@ -328,6 +328,61 @@ def linear_wgrad(dy2d, x2d, out=None, accumulate=False):
     return gemm(dy2d, x2d, dy2d.shape[1], x2d.shape[1], dy2d.shape[0], lda, ldb, False, False, out=out, accumulate=accumulate)
 
 
+def gemm_group(As, Bs, Ms, Ns, K, ldas, ldbs, a_kc, b_kc, outs, accumulates, ws_bytes):
+    """Products over one reduction length in one launch; ws_bytes as gemm_group_workspace_bytes says for these sizes.  Operands
+    and outputs have been checked by the callers below."""
+    n = len(As)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=outs[0].device) if ws_bytes else None
+    i64n, vpn = ctypes.c_int64 * n, ctypes.c_void_p * n
+    _lib.call("ezl_gemm_bf16_group", n, vpn(*[t.data_ptr() for t in As]), vpn(*[t.data_ptr() for t in Bs]),
+              vpn(*[t.data_ptr() for t in outs]), i64n(*Ms), i64n(*Ns), K, i64n(*ldas), i64n(*ldbs), i64n(*[t.stride(0) for t in outs]),
+              1 if a_kc else 0, 1 if b_kc else 0, 0 if outs[0].dtype is BF16 else 1, (ctypes.c_int * n)(*accumulates), _p(ws), ws_bytes,
+              _stream())
+
+
+def _group_ws(Ms, Ns, K):
+    """Workspace bytes of one launch for these products, or -1: separate launches (also for empty ones)."""
+    if not 2 <= len(Ms) <= 3 or K == 0:
+        return -1
+    return _lib.gemm_group_workspace_bytes(Ms, Ns, K)
+
+
+def linear_fwd_multi(x2d, ws):
+    """[x2d @ w_i^T]: linears that share their input, in one launch where that is faster."""
+    T, n_in = x2d.shape
+    Ns = tuple(w.shape[0] for w in ws)
+    nbytes = _group_ws((T,) * len(ws), Ns, n_in)
+    if nbytes < 0:
+        return [linear_fwd(x2d, w) for w in ws]
+    lda, ldbs = _rows_ld(x2d, "x"), [_rows_ld(w, "w") for w in ws]
+    for w in ws:
+        _need(w.shape[1] == n_in, "linear_fwd: inner dimensions differ")
+    outs = [torch.empty((T, n), dtype=BF16, device=x2d.device) for n in Ns]
+    gemm_group([x2d] * len(ws), ws, (T,) * len(ws), Ns, n_in, [lda] * len(ws), ldbs, True, True, outs, [0] * len(ws), nbytes)
+    return outs
+
+
+def linear_wgrad_multi(dy2ds, x2d, outs, accumulates):
+    """dw_i (=|+=) dy_i^T @ x for linears that share their input; outs[i] None: a new bf16 tensor.  Returns the dw_i."""
+    T, n_in = x2d.shape
+    Ms = tuple(dy.shape[1] for dy in dy2ds)
+    n = len(dy2ds)
+    nbytes = _group_ws(Ms, (n_in,) * n, T) if len({None if o is None else o.dtype for o in outs}) == 1 else -1
+    if nbytes < 0:
+        return [linear_wgrad(dy, x2d, out=o, accumulate=acc) for dy, o, acc in zip(dy2ds, outs, accumulates)]
+    ldas, ldb = [_rows_ld(dy, "dy") for dy in dy2ds], _rows_ld(x2d, "x")
+    res = []
+    for dy, o, m in zip(dy2ds, outs, Ms):
+        _need(dy.shape[0] == T, "linear_wgrad: token counts differ")
+        if o is None:
+            o = torch.empty((m, n_in), dtype=BF16, device=x2d.device)
+        st = o.stride()
+        _need(o.is_cuda and o.shape == (m, n_in) and st[1] == 1 and (o.dtype is BF16 or o.dtype is torch.float32), "bad GEMM output")
+        res.append(o)
+    gemm_group(dy2ds, [x2d] * n, Ms, (n_in,) * n, T, ldas, [ldb] * n, False, False, res, [1 if a else 0 for a in accumulates], nbytes)
+    return res
+
+
 def bias_add(x, bias):
     _bf16c(x, "x"); _bf16c(bias, "bias")
     n = x.shape[-1]

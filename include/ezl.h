@@ -122,6 +122,15 @@ int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void* const* B, 
                          int64_t lda, int64_t ldb, int64_t ldc, int a_kc, int b_kc, int out_dtype, int accumulate, void* workspace,
                          int64_t workspace_bytes, void* stream);
 
+/* Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch: q / k / v (gate / up) of
+ * one input, or their weight gradients, where each alone would leave most of the chip idle.  The workspace query returns -1
+ * where separate calls are estimated to be faster (the call itself always makes one launch).  Forms: forward, input gradient
+ * (bf16 results) and weight gradient (bf16 or fp32); all arrays are HOST arrays of `count` entries. */
+int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K);
+int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
+                        int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,
+                        const int* accumulate, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* bias of a linear layer: column_parallel_linear.py:43-44 (out = x + bias) and :100 (db = sum_rows dy);
  * db goes to exactly one of db_bf16 [n] or db_f32 [n] (added to when accumulate != 0). */
 int ezl_bias_add(const void* x, const void* bias, void* out, int64_t rows, int64_t n, void* stream);

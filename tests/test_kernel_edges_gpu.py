@@ -127,3 +127,27 @@ def test_gemm_smaller_tiles_leave_what_is_outside_the_result_alone(K):
         border = big.clone()
         border[1:M + 1, 8:N + 8] = 7.0
         assert (border == 7.0).all(), (form, M, N, Kd)
+
+
+@pytest.mark.parametrize("T,n_in,outs", [(1024, 256, (256, 256, 256)), (1167, 1024, (1024, 256, 264)), (389, 768, (2048, 2056)),
+                                         (17, 264, (8, 1000, 72)), (4000, 2048, (2048, 512, 512)), (9000, 256, (256, 512))])
+def test_gemm_products_in_one_launch(K, T, n_in, outs):
+    """q / k / v (gate / up) forward and weight gradients as one launch, each against its own reference; and accumulation
+    switched per product."""
+    print("gemm group", T, n_in, outs, flush=True)
+    from easyllm_amd import _lib
+    x, ws = rnd(T, n_in, seed=1), [rnd(o, n_in, seed=2 + i) for i, o in enumerate(outs)]
+    n = len(outs)
+    assert _lib.gemm_group_workspace_bytes((T,) * n, outs, n_in) >= 0 or T > 4000
+    for y, w in zip(K.linear_fwd_multi(x, ws), ws):
+        ref = x.float() @ w.float().t()
+        assert ((y.float() - ref).abs() <= gemm_bound(x, w.t()) + ref.abs() * 2.0 ** -8 + 1e-6).all()
+    dys = [rnd(T, o, seed=7 + i) for i, o in enumerate(outs)]
+    for dt in (torch.float32, None):
+        accs = [i % 2 == 1 and dt is not None for i in range(n)]
+        mgs = [None if dt is None else torch.full((o, n_in), 3.0, device="cuda", dtype=dt) for o in outs]
+        for dw, dy, acc in zip(K.linear_wgrad_multi(dys, x, mgs, accs), dys, accs):
+            ref = dy.float().t() @ x.float() + (3.0 if acc else 0.0)
+            assert dw.dtype == (dt or torch.bfloat16)
+            tol = gemm_bound(dy.t(), x) + ref.abs() * (2.0 ** -22 if dt else 2.0 ** -8) + 1e-6
+            assert ((dw.float() - ref).abs() <= tol).all()
