@@ -50,6 +50,8 @@ SIGNATURES = {
     "ezl_sumsq_f32": [_vp, _i64, _vp, _vp],
     "ezl_clip_coef": [_vp, _i64, _f32, _vp, _vp],
     "ezl_build_location_idx": [_vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64],
+    "ezl_sumsq_list": [_i32, _vpp, _i64p, _vp, _vp],
+    "ezl_adamw_list": [_i32, _vpp, _vpp, _vpp, _vpp, _vpp, _i64p, _f32, _f32, _f32, _f32, _f32, _i64, _i32, _vp, _vp],
     "ezl_adamw_step": [_vp, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _i32, _vp, _vp],
 }
 _SPECIAL = {
@@ -63,6 +65,7 @@ _SPECIAL = {
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
     "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
     "ezl_sumsq_partials": ([], _i64),
+    "ezl_sumsq_list_partials": ([_i32], _i64),
     "ezl_location_idx_rows": ([_i64, _i64, _i64], _i64),
 }
 
@@ -135,6 +138,10 @@ def gemm_group_workspace_bytes(Ms, Ns, K):
 
 def sumsq_partials():
     return load().ezl_sumsq_partials()
+
+
+def sumsq_list_partials(count):
+    return load().ezl_sumsq_list_partials(count)
 
 
 def location_idx_rows(seq_length, num_epochs, tokens_per_epoch):

@@ -51,6 +51,11 @@ __global__ __launch_bounds__(kSumsqBlock) void sumsq_partial_kernel(const float*
     }
 }
 
+__global__ __launch_bounds__(256) void zero_f32_kernel(float* __restrict__ x, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) x[i] = 0.f;
+}
+
 // out[0] = sqrt(sum partials), out[1] = clip coefficient: max_norm / (norm + 1e-6) if that is below one, else 1
 __global__ __launch_bounds__(1024) void clip_coef_kernel(const float* __restrict__ partials, int64_t count, float max_norm,
                                                          float* __restrict__ out) {
@@ -86,59 +91,142 @@ __device__ __forceinline__ void adam_one(float& p, float& m, float& v, float g, 
     p = p - a.lr * update;
 }
 
-__global__ __launch_bounds__(kOptBlock) void adamw_kernel(float* __restrict__ master, float* __restrict__ exp_avg,
-                                                         float* __restrict__ exp_avg_sq, const float* __restrict__ grad,
-                                                         bf16_t* __restrict__ param, int64_t n, AdamArgs a,
-                                                         const float* __restrict__ norm_coef) {
-    const float coef = norm_coef ? norm_coef[1] : 1.0f;
-    const int64_t n4 = n >> 2;
-    const int64_t stride = (int64_t)gridDim.x * kOptBlock;
-    auto update = [&](int64_t i, f32x4 p, f32x4 m, f32x4 v, const f32x4 g) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float pk = p[k], mk = m[k], vk = v[k];
-            adam_one(pk, mk, vk, g[k] * coef, a);
-            p[k] = pk; m[k] = mk; v[k] = vk;
-        }
-        reinterpret_cast<f32x4*>(master)[i] = p;
-        reinterpret_cast<f32x4*>(exp_avg)[i] = m;
-        reinterpret_cast<f32x4*>(exp_avg_sq)[i] = v;
-        if (param) {
-            bf16x4 o;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = (bf16_t)p[k];
-            reinterpret_cast<bf16x4*>(param)[i] = o;
-        }
-    };
-    int64_t i = (int64_t)blockIdx.x * kOptBlock + threadIdx.x;
-    for (; i + stride < n4; i += 2 * stride) {  // two vectors of every stream in flight per thread
-        const int64_t j = i + stride;
-        const f32x4 p0 = reinterpret_cast<f32x4*>(master)[i], p1 = reinterpret_cast<f32x4*>(master)[j];
-        const f32x4 m0 = reinterpret_cast<f32x4*>(exp_avg)[i], m1 = reinterpret_cast<f32x4*>(exp_avg)[j];
-        const f32x4 v0 = reinterpret_cast<f32x4*>(exp_avg_sq)[i], v1 = reinterpret_cast<f32x4*>(exp_avg_sq)[j];
-        const f32x4 g0 = reinterpret_cast<const f32x4*>(grad)[i], g1 = reinterpret_cast<const f32x4*>(grad)[j];
-        update(i, p0, m0, v0, g0);
-        update(j, p1, m1, v1, g1);
+// ---- lists of tensors in one launch ----------------------------------------------------------------------------------
+// A stack has tens of tensors, most of them small (a norm weight is 3 - 16 KB): one launch per tensor left the update of a
+// 63 M parameter stack at 42 launches of which half moved next to nothing.  A list of up to kListMax tensors is cut into
+// chunks of kChunk elements, numbered through, that a fixed grid of blocks walks in steps of its size (so the chunks of a
+// block, and with them the order of the norm's sums, depend on the list alone).  16 bytes per lane, four vectors of every
+// stream in flight per thread.
+constexpr int kListMax = 48;
+constexpr int kChunk = 4096;             // elements: 4 vectors x 4 floats x 256 threads
+constexpr int kListBlocks = 2048;        // 8 per CU
+
+struct TensorList {
+    float* a[kListMax];                  // fp32: the gradient (norm), or master / moments / gradient (update)
+    float* m[kListMax];
+    float* v[kListMax];
+    const float* g[kListMax];
+    bf16_t* param[kListMax];             // may be null
+    int64_t n[kListMax];
+    int first[kListMax];                 // launch-wide number of the tensor's first chunk
+    int count, chunks;
+};
+
+__device__ __forceinline__ int tensor_of(const TensorList& l, int chunk) {  // scalar bisection
+    int lo = 0, hi = l.count;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (l.first[mid] <= chunk) lo = mid;
+        else hi = mid;
     }
-    if (i < n4)
-        update(i, reinterpret_cast<f32x4*>(master)[i], reinterpret_cast<f32x4*>(exp_avg)[i], reinterpret_cast<f32x4*>(exp_avg_sq)[i],
-               reinterpret_cast<const f32x4*>(grad)[i]);
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-        const int64_t i = (n4 << 2) + threadIdx.x;
-        float p = master[i], m = exp_avg[i], v = exp_avg_sq[i];
-        adam_one(p, m, v, grad[i] * coef, a);
-        master[i] = p;
-        exp_avg[i] = m;
-        exp_avg_sq[i] = v;
-        if (param) param[i] = (bf16_t)p;
+    return lo;
+}
+
+__global__ __launch_bounds__(kOptBlock) void sumsq_list_kernel(const TensorList l, float* __restrict__ partials) {
+    __shared__ float red[kOptBlock / 64];
+    float acc = 0.f;
+    for (int chunk = blockIdx.x; chunk < l.chunks; chunk += gridDim.x) {
+        const int t = tensor_of(l, chunk);
+        const float* g = l.g[t];
+        const int64_t base = (int64_t)(chunk - l.first[t]) * kChunk, left = l.n[t] - base;
+        if (left >= kChunk) {
+            f32x4 x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const f32x4*>(g + base + (u * kOptBlock + threadIdx.x) * 4);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc += x[u][0] * x[u][0] + x[u][1] * x[u][1] + x[u][2] * x[u][2] + x[u][3] * x[u][3];
+        } else {
+            for (int64_t i = threadIdx.x; i < left; i += kOptBlock) acc += g[base + i] * g[base + i];
+        }
+    }
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float t = 0.f;
+#pragma unroll
+        for (int k = 0; k < kOptBlock / 64; ++k) t += red[k];
+        partials[blockIdx.x] = t;
     }
 }
 
-inline unsigned opt_grid(int64_t n4, int64_t cap) {
-    int64_t g = (n4 + kOptBlock - 1) / kOptBlock;
-    if (g > cap) g = cap;
-    if (g < 1) g = 1;
-    return (unsigned)g;
+// The state is touched once per step and is far larger than the last-level cache: streaming loads and stores.
+__device__ __forceinline__ f32x4 ld_stream(const float* p, int i) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + i); }
+__device__ __forceinline__ void st_stream(float* p, int i, f32x4 x) { __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(p) + i); }
+
+// Bound by HBM: 30 B per parameter.  465 M parameters, norm + update: 3.30 ms with one launch per tensor and two vectors in
+// flight per stream (4.8 TB/s), 2.71 with this (5.8), 2.67 with the streaming hint (5.9); 1024 or 4096 blocks are no different.
+__global__ __launch_bounds__(kOptBlock) void adamw_list_kernel(const TensorList l, const AdamArgs a, const float* __restrict__ norm_coef) {
+    const float coef = norm_coef ? norm_coef[1] : 1.0f;
+    for (int chunk = blockIdx.x; chunk < l.chunks; chunk += gridDim.x) {
+        const int t = tensor_of(l, chunk);
+        const int64_t base = (int64_t)(chunk - l.first[t]) * kChunk, left = l.n[t] - base;
+        float *pp = l.a[t] + base, *pm = l.m[t] + base, *pv = l.v[t] + base;
+        const float* pg = l.g[t] + base;
+        bf16_t* pw = l.param[t] ? l.param[t] + base : nullptr;
+        if (left >= kChunk) {
+            f32x4 p[4], m[4], v[4], g[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = u * kOptBlock + threadIdx.x;
+                p[u] = ld_stream(pp, i); m[u] = ld_stream(pm, i); v[u] = ld_stream(pv, i); g[u] = ld_stream(pg, i);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = u * kOptBlock + threadIdx.x;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float pk = p[u][k], mk = m[u][k], vk = v[u][k];
+                    adam_one(pk, mk, vk, g[u][k] * coef, a);
+                    p[u][k] = pk; m[u][k] = mk; v[u][k] = vk;
+                }
+                st_stream(pp, i, p[u]); st_stream(pm, i, m[u]); st_stream(pv, i, v[u]);
+                if (pw) {
+                    bf16x4 o;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) o[k] = (bf16_t)p[u][k];
+                    reinterpret_cast<bf16x4*>(pw)[i] = o;
+                }
+            }
+        } else {
+            for (int64_t i = threadIdx.x; i < left; i += kOptBlock) {
+                float p = pp[i], m = pm[i], v = pv[i];
+                adam_one(p, m, v, pg[i] * coef, a);
+                pp[i] = p; pm[i] = m; pv[i] = v;
+                if (pw) pw[i] = (bf16_t)p;
+            }
+        }
+    }
+}
+
+AdamArgs adam_args(float lr, float beta1, float beta2, float eps, float weight_decay, int64_t step, int bias_correction) {
+    AdamArgs a;
+    a.lr = lr; a.beta1 = beta1; a.beta2 = beta2; a.eps = eps; a.weight_decay = weight_decay;
+    a.inv_bc1 = bias_correction ? (float)(1.0 / (1.0 - pow((double)beta1, (double)step))) : 1.0f;
+    a.inv_bc2 = bias_correction ? (float)(1.0 / (1.0 - pow((double)beta2, (double)step))) : 1.0f;
+    return a;
+}
+
+// calls launch(list, number of blocks) for every kListMax non-empty tensors of 0 .. count - 1; fill(list, slot, i) sets the pointers
+template <class Fill, class Launch>
+void for_each_list(int count, const int64_t* n, Fill fill, Launch launch) {
+    TensorList l;
+    l.count = l.chunks = 0;
+    auto flush = [&]() {
+        if (l.count) launch(l, (unsigned)(l.chunks < kListBlocks ? l.chunks : kListBlocks));
+        l.count = l.chunks = 0;
+    };
+    for (int i = 0; i < count; ++i) {
+        if (n[i] == 0) continue;
+        const int64_t chunks = (n[i] + kChunk - 1) / kChunk;
+        if (l.count == kListMax || l.chunks + chunks >= (1LL << 30)) flush();
+        fill(l, l.count, i);
+        l.n[l.count] = n[i];
+        l.first[l.count] = l.chunks;
+        l.chunks += (int)chunks;
+        ++l.count;
+    }
+    flush();
 }
 
 }  // namespace
@@ -171,13 +259,57 @@ extern "C" int ezl_adamw_step(void* master, void* exp_avg, void* exp_avg_sq, con
     EZL_REQUIRE(ezl_aligned16(master) && ezl_aligned16(exp_avg) && ezl_aligned16(exp_avg_sq) && ezl_aligned16(grad) &&
                     (((uintptr_t)param_bf16 & 7) == 0),
                 EZL_EINVAL, "ezl_adamw_step: fp32 buffers must be 16-byte aligned, the bf16 weight 8-byte aligned");
-    if (n == 0) return EZL_OK;
-    AdamArgs a;
-    a.lr = lr; a.beta1 = beta1; a.beta2 = beta2; a.eps = eps; a.weight_decay = weight_decay;
-    a.inv_bc1 = bias_correction ? (float)(1.0 / (1.0 - pow((double)beta1, (double)step))) : 1.0f;
-    a.inv_bc2 = bias_correction ? (float)(1.0 / (1.0 - pow((double)beta2, (double)step))) : 1.0f;
-    hipLaunchKernelGGL(adamw_kernel, dim3(opt_grid(n >> 2, 256 * 16)), dim3(kOptBlock), 0, (hipStream_t)stream, (float*)master,
-                       (float*)exp_avg, (float*)exp_avg_sq, (const float*)grad, (bf16_t*)param_bf16, n, a, (const float*)norm_coef);
+    const int64_t one[1] = {n};
+    const AdamArgs a = adam_args(lr, beta1, beta2, eps, weight_decay, step, bias_correction);
+    for_each_list(1, one, [&](TensorList& l, int s, int) {
+        l.a[s] = (float*)master; l.m[s] = (float*)exp_avg; l.v[s] = (float*)exp_avg_sq; l.g[s] = (const float*)grad; l.param[s] = (bf16_t*)param_bf16;
+    }, [&](const TensorList& l, unsigned blocks) {
+        hipLaunchKernelGGL(adamw_list_kernel, dim3(blocks), dim3(kOptBlock), 0, (hipStream_t)stream, l, a, (const float*)norm_coef);
+    });
     EZL_LAUNCH_CHECK("ezl_adamw_step");
+    return EZL_OK;
+}
+
+// fp32 slots that ezl_sumsq_list fills for a list of `count` tensors
+extern "C" int64_t ezl_sumsq_list_partials(int count) { return count < 0 ? -1 : ((int64_t)count + kListMax - 1) / kListMax * kListBlocks; }
+
+extern "C" int ezl_sumsq_list(int count, const void* const* x, const int64_t* n, void* partials, void* stream) {
+    EZL_REQUIRE(count >= 0 && (count == 0 || (x && n && partials)), EZL_EINVAL, "ezl_sumsq_list: bad count or null argument array");
+    for (int i = 0; i < count; ++i)
+        EZL_REQUIRE(n[i] >= 0 && n[i] < (1LL << 40) && (n[i] == 0 || x[i]) && ezl_aligned16(x[i]), EZL_EINVAL,
+                    "ezl_sumsq_list: null or misaligned tensor");
+    float* out = (float*)partials;
+    float* const end = out + ezl_sumsq_list_partials(count);
+    for_each_list(count, n, [&](TensorList& l, int s, int i) { l.g[s] = (const float*)x[i]; }, [&](const TensorList& l, unsigned blocks) {
+        hipLaunchKernelGGL(sumsq_list_kernel, dim3(blocks), dim3(kOptBlock), 0, (hipStream_t)stream, l, out);
+        out += blocks;
+    });
+    if (out < end)  // slots of blocks that were not needed (a fill kernel, not a memset node)
+        hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((end - out + 255) / 256)), dim3(256), 0, (hipStream_t)stream, out, (int)(end - out));
+    EZL_LAUNCH_CHECK("ezl_sumsq_list");
+    return EZL_OK;
+}
+
+extern "C" int ezl_adamw_list(int count, void* const* master, void* const* exp_avg, void* const* exp_avg_sq, const void* const* grad,
+                              void* const* param_bf16, const int64_t* n, float lr, float beta1, float beta2, float eps, float weight_decay,
+                              int64_t step, int bias_correction, const void* norm_coef, void* stream) {
+    EZL_REQUIRE(count >= 0 && (count == 0 || (master && exp_avg && exp_avg_sq && grad && param_bf16 && n)), EZL_EINVAL,
+                "ezl_adamw_list: bad count or null argument array");
+    EZL_REQUIRE(step >= 1, EZL_EINVAL, "ezl_adamw_list: step counts from 1");
+    for (int i = 0; i < count; ++i) {
+        EZL_REQUIRE(n[i] >= 0 && n[i] < (1LL << 40) && (n[i] == 0 || (master[i] && exp_avg[i] && exp_avg_sq[i] && grad[i])), EZL_EINVAL,
+                    "ezl_adamw_list: null pointer");
+        EZL_REQUIRE(ezl_aligned16(master[i]) && ezl_aligned16(exp_avg[i]) && ezl_aligned16(exp_avg_sq[i]) && ezl_aligned16(grad[i]) &&
+                        (((uintptr_t)param_bf16[i] & 7) == 0),
+                    EZL_EINVAL, "ezl_adamw_list: fp32 buffers must be 16-byte aligned, the bf16 weight 8-byte aligned");
+    }
+    const AdamArgs a = adam_args(lr, beta1, beta2, eps, weight_decay, step, bias_correction);
+    for_each_list(count, n, [&](TensorList& l, int s, int i) {
+        l.a[s] = (float*)master[i]; l.m[s] = (float*)exp_avg[i]; l.v[s] = (float*)exp_avg_sq[i]; l.g[s] = (const float*)grad[i];
+        l.param[s] = (bf16_t*)param_bf16[i];
+    }, [&](const TensorList& l, unsigned blocks) {
+        hipLaunchKernelGGL(adamw_list_kernel, dim3(blocks), dim3(kOptBlock), 0, (hipStream_t)stream, l, a, (const float*)norm_coef);
+    });
+    EZL_LAUNCH_CHECK("ezl_adamw_list");
     return EZL_OK;
 }

@@ -577,6 +577,10 @@ def sumsq_partials():
     return int(_lib.sumsq_partials())
 
 
+def sumsq_list_partials(count):
+    return int(_lib.sumsq_list_partials(count))
+
+
 def sumsq(x, partials_row):
     """partials_row (fp32 [sumsq_partials()]) <- per-block sums of x^2."""
     _f32c(x, "x"); _f32c(partials_row, "partials")
@@ -609,3 +613,37 @@ def adamw_step(master, exp_avg, exp_avg_sq, grad, param, lr, beta1, beta2, eps, 
     _lib.call("ezl_adamw_step", _p(master), _p(exp_avg), _p(exp_avg_sq), _p(grad), _p(param), master.numel(), float(lr),
               float(beta1), float(beta2), float(eps), float(weight_decay), int(step), 1 if bias_correction else 0,
               _p(norm_coef), _stream())
+
+
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
+
+
+def sumsq_list(xs, partials):
+    """partials (fp32 [_lib.sumsq_list_partials(len(xs))]) <- sums of squares of a list of fp32 tensors."""
+    for x in xs:
+        _f32c(x, "x")
+    _f32c(partials, "partials")
+    _need(partials.numel() == _lib.sumsq_list_partials(len(xs)), "partials have the wrong length")
+    _lib.call("ezl_sumsq_list", len(xs), _pointers(xs), (ctypes.c_int64 * len(xs))(*[x.numel() for x in xs]), _p(partials), _stream())
+
+
+def adamw_list(masters, exp_avgs, exp_avg_sqs, grads, params, lr, beta1, beta2, eps, weight_decay, step, bias_correction=True,
+               norm_coef=None):
+    """adamw_step over lists of tensors (params: bf16 or None entries) in one launch per 48 of them."""
+    ns = [t.numel() for t in masters]
+    for ts, name in ((masters, "master"), (exp_avgs, "exp_avg"), (exp_avg_sqs, "exp_avg_sq"), (grads, "grad")):
+        for t, n in zip(ts, ns):
+            _f32c(t, name)
+            if t.numel() != n:
+                raise ValueError("%s size mismatch" % name)
+    for t, n in zip(params, ns):
+        if t is not None:
+            _bf16c(t, "param")
+            _need(t.numel() == n, "param size mismatch")
+    if norm_coef is not None:
+        _f32c(norm_coef, "norm_coef")
+        _need(norm_coef.numel() == 2, "norm_coef must hold (norm, coefficient)")
+    _lib.call("ezl_adamw_list", len(ns), _pointers(masters), _pointers(exp_avgs), _pointers(exp_avg_sqs), _pointers(grads), _pointers(params),
+              (ctypes.c_int64 * len(ns))(*ns), float(lr), float(beta1), float(beta2), float(eps), float(weight_decay), int(step),
+              1 if bias_correction else 0, _p(norm_coef), _stream())

@@ -74,7 +74,7 @@ class FusedAdam:
                                  "exp_avg_sq": torch.zeros_like(p, dtype=torch.float32)}
         n = sum(len(g["params"]) for g in self.param_groups)
         dev = self.param_groups[0]["params"][0].device if n else torch.device("cpu")
-        self._partials = torch.zeros(max(n, 1), K.sumsq_partials(), dtype=torch.float32, device=dev) if n else None
+        self._partials = torch.zeros(K.sumsq_list_partials(n), dtype=torch.float32, device=dev) if n else None
         self._norm_coef = torch.ones(2, dtype=torch.float32, device=dev) if n else None
 
     def _all_params(self):
@@ -84,9 +84,8 @@ class FusedAdam:
 
     def global_grad_norm(self, max_norm):
         """(norm, coefficient) of all main_grads as a device tensor; max_norm <= 0 disables clipping (coefficient 1)."""
-        for i, (_, p) in enumerate(self._all_params()):
-            K.sumsq(p.main_grad.view(-1), self._partials[i])
-        return K.clip_coef(self._partials.view(-1), max_norm, out=self._norm_coef)
+        K.sumsq_list([p.main_grad for _, p in self._all_params()], self._partials)
+        return K.clip_coef(self._partials, max_norm, out=self._norm_coef)
 
     def step(self, clip_grad=0.0):
         norm_coef = self.global_grad_norm(clip_grad) if clip_grad and clip_grad > 0 else None
@@ -95,11 +94,11 @@ class FusedAdam:
                 continue
             group["step"] += 1
             b1, b2 = group["betas"]
-            for p in group["params"]:
-                st = self.state[p]
-                K.adamw_step(st["master"].view(-1), st["exp_avg"].view(-1), st["exp_avg_sq"].view(-1), p.main_grad.view(-1),
-                             p.data.view(-1) if p.dtype == torch.bfloat16 else None, group["lr"], b1, b2, group["eps"],
-                             group["weight_decay"], group["step"], group["bias_correction"], norm_coef)
+            states = [self.state[p] for p in group["params"]]
+            K.adamw_list([st["master"] for st in states], [st["exp_avg"] for st in states], [st["exp_avg_sq"] for st in states],
+                         [p.main_grad for p in group["params"]], [p.data if p.dtype == torch.bfloat16 else None for p in group["params"]],
+                         group["lr"], b1, b2, group["eps"], group["weight_decay"], group["step"], group["bias_correction"], norm_coef)
+            for p, st in zip(group["params"], states):
                 if p.dtype != torch.bfloat16:
                     p.data.copy_(st["master"])
         return norm_coef

@@ -203,6 +203,14 @@ int ezl_clip_coef(const void* partials, int64_t count, float max_norm, void* nor
 int ezl_adamw_step(void* master, void* exp_avg, void* exp_avg_sq, const void* grad, void* param_bf16, int64_t n, float lr,
                    float beta1, float beta2, float eps, float weight_decay, int64_t step, int bias_correction,
                    const void* norm_coef, void* stream);
+/* The same over a list of tensors in one launch per 48 of them.  ezl_sumsq_list fills ezl_sumsq_list_partials(count) fp32 slots
+ * (any slots past the launched blocks are zeroed) for ezl_clip_coef; the arrays are HOST arrays of `count` entries, entries
+ * of param_bf16 may be NULL. */
+int64_t ezl_sumsq_list_partials(int count);
+int ezl_sumsq_list(int count, const void* const* x, const int64_t* n, void* partials, void* stream);
+int ezl_adamw_list(int count, void* const* master, void* const* exp_avg, void* const* exp_avg_sq, const void* const* grad,
+                   void* const* param_bf16, const int64_t* n, float lr, float beta1, float beta2, float eps, float weight_decay,
+                   int64_t step, int bias_correction, const void* norm_coef, void* stream);
 
 /* ---- packed-sequence sample index (host code, no GPU): llm/data/cores/helpers.cpp:36-122 `build_location_idx`
  *      (python twin llm/data/nlp_dataset.py:424-463) ----

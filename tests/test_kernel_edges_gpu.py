@@ -151,3 +151,26 @@ def test_gemm_products_in_one_launch(K, T, n_in, outs):
             assert dw.dtype == (dt or torch.bfloat16)
             tol = gemm_bound(dy.t(), x) + ref.abs() * (2.0 ** -22 if dt else 2.0 ** -8) + 1e-6
             assert ((dw.float() - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("sizes", [[1], [4096, 4095, 4097, 3], [0, 8, 0, 70001], [1 + 37 * i for i in range(101)]])
+def test_optimizer_over_lists_of_tensors(K, sizes):
+    """Chunk edges, empty tensors and more tensors than one launch takes: the norm against fp64, the update bit for bit against
+    the single-tensor call."""
+    print("optimizer lists", len(sizes), flush=True)
+    gs = [torch.randn(n, device="cuda") for n in sizes]
+    partials = torch.full((K.sumsq_list_partials(len(sizes)),), float("nan"), device="cuda")
+    K.sumsq_list(gs, partials)
+    want = sum(g.double().square().sum().item() for g in gs)
+    assert abs(partials.double().sum().item() - want) <= 1e-5 * want
+    coef = torch.tensor([5.0, 0.5], device="cuda")
+    one = [[torch.randn(n, device="cuda") for n in sizes] for _ in range(2)] + [[torch.rand(n, device="cuda") for n in sizes]]
+    lst = [[t.clone() for t in ts] for ts in one]
+    params = [torch.zeros(n, device="cuda", dtype=torch.bfloat16) if i % 3 else None for i, n in enumerate(sizes)]
+    params1 = [None if p is None else p.clone() for p in params]
+    K.adamw_list(*lst, gs, params, 1e-2, 0.9, 0.95, 1e-8, 0.1, 3, True, coef)
+    for i in range(len(sizes)):
+        K.adamw_step(one[0][i], one[1][i], one[2][i], gs[i], params1[i], 1e-2, 0.9, 0.95, 1e-8, 0.1, 3, True, coef)
+        assert all(torch.equal(a[i], b[i]) for a, b in zip(one, lst))
+        if params[i] is not None:
+            assert torch.equal(params[i], params1[i]) and torch.equal(params[i], lst[0][i].bfloat16())
