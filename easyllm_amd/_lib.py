@@ -13,6 +13,22 @@ _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_
 _i64p = ctypes.POINTER(ctypes.c_int64)
 _vpp = ctypes.POINTER(ctypes.c_void_p)
 
+
+
+class Layer(ctypes.Structure):
+    """struct ezl_layer"""
+    _fields_ = ([(n, _i64) for n in ("s", "b", "h", "nq", "nk", "d", "f", "ndocs", "npos")] + [(n, _f32) for n in ("eps1", "eps2", "scale")]
+                + [(n, _vp) for n in ("ln1", "wq", "wk", "wv", "bq", "bk", "bv", "wo", "ln2", "wg", "wu", "wd", "cos", "sin", "position_ids",
+                                      "cu_seqlens")])
+
+
+class LayerGrad(ctypes.Structure):
+    """struct ezl_layer_grad"""
+    _fields_ = [("f32", _vp), ("bf16", _vp), ("accumulate", _i32)]
+
+
+_layerp = ctypes.POINTER(Layer)
+
 # name -> argtypes; the single source of truth for the symbol table on the Python side
 SIGNATURES = {
     "ezl_rmsnorm_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp],
@@ -50,6 +66,8 @@ SIGNATURES = {
     "ezl_sumsq_f32": [_vp, _i64, _vp, _vp],
     "ezl_clip_coef": [_vp, _i64, _f32, _vp, _vp],
     "ezl_build_location_idx": [_vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64],
+    "ezl_layer_fwd": [_layerp, _vp, _vp, _vp, _vp, _vp],
+    "ezl_layer_bwd": [_layerp, _vp, _vp, _vp, _vp, _vp, ctypes.POINTER(LayerGrad), _vp],
     "ezl_sumsq_list": [_i32, _vpp, _i64p, _vp, _vp],
     "ezl_adamw_list": [_i32, _vpp, _vpp, _vpp, _vpp, _vpp, _i64p, _f32, _f32, _f32, _f32, _f32, _i64, _i32, _vp, _vp],
     "ezl_adamw_step": [_vp, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _i32, _vp, _vp],
@@ -64,6 +82,7 @@ _SPECIAL = {
     "ezl_attn_bwd_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64], _i64),
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
     "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
+    "ezl_layer_bytes": ([_layerp, _i32], _i64),
     "ezl_sumsq_partials": ([], _i64),
     "ezl_sumsq_list_partials": ([_i32], _i64),
     "ezl_location_idx_rows": ([_i64, _i64, _i64], _i64),
@@ -134,6 +153,10 @@ def gemm_workspace_bytes(M, N, K):
 def gemm_group_workspace_bytes(Ms, Ns, K):
     n = len(Ms)
     return load().ezl_gemm_group_workspace_bytes(n, (_i64 * n)(*Ms), (_i64 * n)(*Ns), K)
+
+
+def layer_bytes(layer, which):
+    return load().ezl_layer_bytes(ctypes.byref(layer), which)
 
 
 def sumsq_partials():

@@ -2,6 +2,7 @@
 // SwiGLU, rotary embedding, token-embedding gather / scatter-add, [b,s,h] <-> [s,b,h] row moves,
 // bf16 add and bf16 <-> fp32 casts.  All use 128-bit accesses (8 bf16 per lane).
 #include "common.h"
+#include "qkv_bias.h"
 
 namespace {
 
@@ -521,7 +522,106 @@ __global__ __launch_bounds__(kBlock) void bias_grad_partial_kernel(const bf16_t*
     for (int k = 0; k < 8; ++k) partial[(int64_t)blockIdx.y * n + col + k] = acc[k];
 }
 
+// q / k / v projections (rows of nq, nk, nk heads) + their biases, q and k rotated: bias_add (rounded to bf16) and the rotation
+// above in one pass.  An item is 8 low-half + 8 high-half elements of one head of one row.
+struct QkvBias {
+    const bf16_t *x[3], *bias[3];
+    bf16_t* out[3];
+};
+__global__ __launch_bounds__(kBlock) void bias_rope_kernel(const QkvBias a, const float* __restrict__ cosb, const float* __restrict__ sinb,
+                                                           const int64_t* __restrict__ position_ids, int64_t rows, int s, int b, int nq,
+                                                           int nk, int d, int64_t npos) {
+    const int half = d >> 1, per_head = half >> 3, nheads = nq + 2 * nk;
+    const int64_t items = rows * nheads * per_head;
+    for (int64_t it = (int64_t)blockIdx.x * kBlock + threadIdx.x; it < items; it += (int64_t)gridDim.x * kBlock) {
+        const int j8 = (int)(it % per_head);
+        const int64_t rh = it / per_head;
+        int head = (int)(rh % nheads);
+        const int64_t row = rh / nheads;
+        const int which = head < nq ? 0 : (head < nq + nk ? 1 : 2);
+        head -= which == 0 ? 0 : (which == 1 ? nq : nq + nk);
+        const int col = head * d + j8 * 8;
+        const int64_t at = row * (int64_t)((which == 0 ? nq : nk) * d) + col;
+        const bf16_t* x = which == 0 ? a.x[0] : (which == 1 ? a.x[1] : a.x[2]);
+        const bf16_t* bias = which == 0 ? a.bias[0] : (which == 1 ? a.bias[1] : a.bias[2]);
+        bf16_t* out = which == 0 ? a.out[0] : (which == 1 ? a.out[1] : a.out[2]);
+        float lo[8], hi[8], bl[8], bh[8];
+        unpack8(ld_bf16x8(x + at), lo);
+        unpack8(ld_bf16x8(x + at + half), hi);
+        unpack8(ld_bf16x8(bias + col), bl);
+        unpack8(ld_bf16x8(bias + col + half), bh);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            lo[k] = (float)(bf16_t)(lo[k] + bl[k]);
+            hi[k] = (float)(bf16_t)(hi[k] + bh[k]);
+        }
+        if (which < 2) {
+            int64_t pos = position_ids ? position_ids[(row % b) * s + row / b] : row / b;
+            pos = pos < 0 ? 0 : (pos >= npos ? npos - 1 : pos);
+            const float *cp = cosb + pos * half + j8 * 8, *sp = sinb + pos * half + j8 * 8;
+            const f32x4 c0 = *reinterpret_cast<const f32x4*>(cp), c1 = *reinterpret_cast<const f32x4*>(cp + 4);
+            const f32x4 s0 = *reinterpret_cast<const f32x4*>(sp), s1 = *reinterpret_cast<const f32x4*>(sp + 4);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float cs = k < 4 ? c0[k] : c1[k - 4], sn = k < 4 ? s0[k] : s1[k - 4];
+                const float x1 = lo[k], x2 = hi[k];
+                lo[k] = x1 * cs - x2 * sn;
+                hi[k] = x2 * cs + x1 * sn;
+            }
+        }
+        st_bf16x8(out + at, pack8(lo));
+        st_bf16x8(out + at + half, pack8(hi));
+    }
+}
+
+// the column sums of a [rows, qw + 2 kw] partial table, written to three targets
+__global__ __launch_bounds__(256) void qkv_bias_fold_kernel(const float* __restrict__ partial, int nrows, int qw, int kw, const QkvBiasGrad g) {
+    const int ncols = qw + 2 * kw, col = blockIdx.x * 256 + threadIdx.x;
+    if (col >= ncols) return;
+    float acc = 0.f;  // in the order of ezl_colsum_kernel: 16 interleaved groups of rows, then the groups
+#pragma unroll 4
+    for (int g0 = 0; g0 < 16; ++g0) {
+        float v = 0.f;
+        for (int r = g0; r < nrows; r += 16) v += partial[(size_t)r * ncols + col];
+        acc += v;
+    }
+    const int which = col < qw ? 0 : (col < qw + kw ? 1 : 2);
+    const int c = col - (which == 0 ? 0 : (which == 1 ? qw : qw + kw));
+    float* f = which == 0 ? g.f32[0] : (which == 1 ? g.f32[1] : g.f32[2]);
+    bf16_t* h = which == 0 ? g.bf16[0] : (which == 1 ? g.bf16[1] : g.bf16[2]);
+    const int accumulate = which == 0 ? g.accumulate[0] : (which == 1 ? g.accumulate[1] : g.accumulate[2]);
+    if (f) f[c] = accumulate ? f[c] + acc : acc;
+    else if (h) h[c] = (bf16_t)acc;
+}
+
 }  // namespace
+
+int qkv_bias_rope(const void* const* x, const void* const* bias, void* const* out, int64_t nq, int64_t nk, int64_t d, const void* cos_table,
+                  const void* sin_table, const void* position_ids, int64_t s, int64_t b, int64_t npos, hipStream_t stream) {
+    EZL_REQUIRE(d % 16 == 0 && npos >= 1 && (position_ids || npos >= s) && cos_table && sin_table, EZL_EUNSUPPORTED,
+                "q / k / v bias + rotation: bad head dim or rotary tables");
+    QkvBias a;
+    for (int i = 0; i < 3; ++i) {
+        EZL_REQUIRE(x[i] && bias[i] && out[i] && ezl_aligned16(x[i]) && ezl_aligned16(bias[i]) && ezl_aligned16(out[i]), EZL_EINVAL,
+                    "q / k / v bias + rotation: null or misaligned pointer");
+        a.x[i] = (const bf16_t*)x[i]; a.bias[i] = (const bf16_t*)bias[i]; a.out[i] = (bf16_t*)out[i];
+    }
+    hipLaunchKernelGGL(bias_rope_kernel, dim3(grid_for(s * b * (nq + 2 * nk) * (d / 16), kBlock)), dim3(kBlock), 0, stream, a,
+                       (const float*)cos_table, (const float*)sin_table, (const int64_t*)position_ids, s * b, (int)s, (int)b, (int)nq,
+                       (int)nk, (int)d, npos);
+    EZL_LAUNCH_CHECK("q / k / v bias + rotation");
+    return EZL_OK;
+}
+
+int qkv_bias_grad(const void* dqkv, const QkvBiasGrad& g, int64_t rows, int64_t qw, int64_t kw, void* workspace, hipStream_t stream) {
+    const int64_t n = qw + 2 * kw;
+    const dim3 grid((unsigned)((n / 8 + kBlock - 1) / kBlock), 64);
+    hipLaunchKernelGGL(bias_grad_partial_kernel, grid, dim3(kBlock), 0, stream, (const bf16_t*)dqkv, (float*)workspace, rows, (int)n);
+    hipLaunchKernelGGL(qkv_bias_fold_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, (const float*)workspace, 64, (int)qw,
+                       (int)kw, g);
+    EZL_LAUNCH_CHECK("q / k / v bias gradient");
+    return EZL_OK;
+}
 
 extern "C" int ezl_swiglu_fwd(const void* gate, const void* up, void* out, int64_t n, void* stream) {
     EZL_REQUIRE(n >= 0 && n % 8 == 0, EZL_EUNSUPPORTED, "ezl_swiglu_fwd: n must be a multiple of 8");

@@ -310,6 +310,44 @@ def flash_attention_unpadded(q, k, v, key_padding_mask, scale=None):
 
 
 # --------------------------------------------------------------------------------------------
+# a whole decoder layer: llama/transformer.py:747-803
+# --------------------------------------------------------------------------------------------
+class DecoderLayerFunction(torch.autograd.Function):
+    """x [s, b, h] -> layer(x) with all launches made by one native call, and one for the backward: for layers whose kernels
+    take less time than the Python between them.  `plan` = (heads, f, eps, scale); params = (ln1, q, k, v, o, ln2, gate, up,
+    down[, q / k / v biases])."""
+
+    @staticmethod
+    def forward(ctx, x, plan, cos, sin, position_ids, cu_seqlens, *params):
+        x = x.contiguous()
+        desc = K.layer_desc(x.shape, *plan, params[:9], params[9:] or None, cos, sin, position_ids, cu_seqlens)
+        y, saved = K.layer_fwd(desc, x)
+        ctx.save_for_backward(x, saved, cos, sin, position_ids, cu_seqlens, *params)
+        ctx.plan = plan
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, saved, cos, sin, position_ids, cu_seqlens, *params = ctx.saved_tensors
+        desc = K.layer_desc(x.shape, *ctx.plan, params[:9], params[9:] or None, cos, sin, position_ids, cu_seqlens)
+        targets, grads = [], []
+        for i, p in enumerate(params):
+            needed = ctx.needs_input_grad[6 + i]
+            mg, acc = _main_grad_target(p) if needed else (None, False)
+            grad = None
+            if mg is None and (needed or p.dim() == 1):  # (a norm's kernel writes its weight gradient in any case)
+                grad = torch.empty_like(p)
+            targets.append((mg, grad, acc) if mg is not None or grad is not None else None)
+            grads.append(grad if needed else None)
+        dx = K.layer_bwd(desc, x, dy.contiguous(), saved, targets)
+        return (dx if ctx.needs_input_grad[0] else None, None, None, None, None, None, *grads)
+
+
+def decoder_layer(x, plan, cos, sin, position_ids, cu_seqlens, params):
+    return DecoderLayerFunction.apply(x, plan, cos, sin, position_ids, cu_seqlens, *params)
+
+
+# --------------------------------------------------------------------------------------------
 # embedding: base_modules/layers/vocab_parallel_emb.py:106-137
 # --------------------------------------------------------------------------------------------
 class EmbeddingFunction(torch.autograd.Function):

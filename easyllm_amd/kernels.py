@@ -647,3 +647,64 @@ def adamw_list(masters, exp_avgs, exp_avg_sqs, grads, params, lr, beta1, beta2, 
     _lib.call("ezl_adamw_list", len(ns), _pointers(masters), _pointers(exp_avgs), _pointers(exp_avg_sqs), _pointers(grads), _pointers(params),
               (ctypes.c_int64 * len(ns))(*ns), float(lr), float(beta1), float(beta2), float(eps), float(weight_decay), int(step),
               1 if bias_correction else 0, _p(norm_coef), _stream())
+
+
+# ------------------------------------------------------------------------------------- one decoder layer per call
+def layer_desc(shape, heads, f, eps, scale, weights, biases, cos, sin, position_ids, cu_seqlens):
+    """struct ezl_layer for activations of `shape` (s, b, h): heads = (nq, nk, d), weights = (ln1, q, k, v, o, ln2, gate, up, down),
+    biases of q / k / v or None.  The tensors have to outlive the call that it is made for."""
+    s, b, h = shape
+    nq, nk, d = heads
+    ln1, wq, wk, wv, wo, ln2, wg, wu, wd = weights
+    for w, n_out, n_in in ((wq, nq * d, h), (wk, nk * d, h), (wv, nk * d, h), (wo, h, nq * d), (wg, f, h), (wu, f, h), (wd, h, f)):
+        if not (w.dtype is BF16 and w.shape == (n_out, n_in) and w.is_contiguous() and w.is_cuda):
+            raise ValueError("layer: a weight is not a contiguous bf16 GPU tensor of the layer's size")
+    for w in (ln1, ln2):
+        _bf16c(w, "norm weight")
+        _need(w.numel() == h, "norm weight size mismatch")
+    bq = bk = bv = None
+    if biases is not None:
+        for t, n in zip(biases, (nq * d, nk * d, nk * d)):
+            _bf16c(t, "bias")
+            _need(t.numel() == n, "bias size mismatch")
+        bq, bk, bv = (t.data_ptr() for t in biases)
+    if position_ids is not None:
+        _need(position_ids.is_cuda and position_ids.dtype is torch.int64 and position_ids.is_contiguous()
+              and position_ids.shape == (b, s), "position_ids must be int64 [b, s]")
+    _need(cos.shape == sin.shape and cos.shape[1] == d // 2 and cos.dtype is torch.float32, "bad cos/sin table")
+    cu, ndocs = _cu_arg(cu_seqlens, b)
+    return _lib.Layer(s, b, h, nq, nk, d, f, ndocs, cos.shape[0], eps[0], eps[1], scale, ln1.data_ptr(), wq.data_ptr(), wk.data_ptr(),
+                      wv.data_ptr(), bq, bk, bv, wo.data_ptr(), ln2.data_ptr(), wg.data_ptr(), wu.data_ptr(), wd.data_ptr(), cos.data_ptr(),
+                      sin.data_ptr(), _p(position_ids), _p(cu))
+
+
+def layer_fwd(desc, x):
+    """-> (y, saved block)"""
+    _bf16c(x, "x")
+    y = torch.empty_like(x)
+    saved = torch.empty(_lib.layer_bytes(desc, 0), dtype=torch.uint8, device=x.device)
+    temp = torch.empty(_lib.layer_bytes(desc, 1), dtype=torch.uint8, device=x.device)
+    _lib.call("ezl_layer_fwd", ctypes.byref(desc), x.data_ptr(), y.data_ptr(), saved.data_ptr(), temp.data_ptr(), _stream())
+    return y, saved
+
+
+def layer_bwd(desc, x, dy, saved, grads):
+    """grads: per parameter (ln1, q, k, v, o, ln2, gate, up, down[, biases]) an (fp32 buffer, bf16 tensor, accumulate) triple, the
+    first or the second None, or None for no gradient.  Returns dx."""
+    _bf16c(x, "x"); _bf16c(dy, "dy")
+    _need(dy.shape == x.shape, "layer_bwd: shape mismatch")
+    arr = (_lib.LayerGrad * 12)()
+    for slot, g in zip(arr, grads):
+        if g is not None:
+            f32, bf16, acc = g
+            if f32 is not None:
+                _f32c(f32, "main_grad")
+                slot.f32 = f32.data_ptr()
+            else:
+                _bf16c(bf16, "gradient")
+                slot.bf16 = bf16.data_ptr()
+            slot.accumulate = 1 if acc else 0
+    dx = torch.empty_like(x)
+    temp = torch.empty(_lib.layer_bytes(desc, 2), dtype=torch.uint8, device=x.device)
+    _lib.call("ezl_layer_bwd", ctypes.byref(desc), x.data_ptr(), dy.data_ptr(), dx.data_ptr(), saved.data_ptr(), temp.data_ptr(), arr, _stream())
+    return dx

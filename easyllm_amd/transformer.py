@@ -18,7 +18,7 @@ import torch
 
 from . import dist_env
 from . import functional as F_
-from .layers import (ColumnParallelLinear, RowParallelLinear, GLU_ACTIVATIONS, build_layer_norm,
+from .layers import (ColumnParallelLinear, RMSNorm, RowParallelLinear, GLU_ACTIVATIONS, build_layer_norm,
                      get_initializer_from_cfg, get_torch_dtype)
 from .positional_embeddings import RotaryEmbedding, apply_rotary_pos_emb
 
@@ -162,9 +162,9 @@ class ParallelAttention(torch.nn.Module):
             query_layer, key_layer, value_layer = F_.fan_out_linear(hidden_states, self.q_proj.weight, self.k_proj.weight,
                                                                     self.v_proj.weight)
         elif not self.qkv_pack:
-            query_layer, _ = self.q_proj(hidden_states)
-            key_layer, _ = self.k_proj(hidden_states)
-            value_layer, _ = self.v_proj(hidden_states)
+            projections = (self.q_proj, self.k_proj, self.v_proj)
+            query_layer, key_layer, value_layer = (
+                F_.bias_add(y, p.bias) for y, p in zip(F_.fan_out_linear(hidden_states, *(p.weight for p in projections)), projections))
         else:
             qkv_layer, _ = self.wqkv(hidden_states)  # q | k | v along the last dim (:427-429)
             query_layer = qkv_layer[..., :self.q_size]
@@ -240,9 +240,54 @@ class ParallelTransformerLayer(torch.nn.Module):
             onnx_safe=onnx_safe, sync_tp_duplicated_parameters=sync_tp_duplicated_parameters,
             sequence_parallel=sequence_parallel)
         self.alibi = None
+        # Layers of up to this many forward FLOPs make all their launches in one native call (see _native_inputs).
+        self.native_call_flops = 1e12
+
+    def _native_inputs(self, hidden_states, attention_mask, cu_seqlens, position_ids):
+        """The arguments of functional.decoder_layer if this call can be one native call, else None.
+
+        It pays where the host's work per launch (10 - 20 us through a module, an autograd node and a wrapper; 3 us from native
+        code) exceeds the kernels' own time: two layers at h = 256 on 1024 tokens, forward + loss + backward, 1.6 ms of which
+        0.57 are kernels.  1e12 FLOPs are 0.8 ms of kernels, where the host is ahead either way; larger layers keep the
+        composed form, whose activations and gradients are freed one by one.  Only the plain layer qualifies: its own
+        submodules, unhooked, separate q / k / v projections, no o bias, no key padding mask."""
+        attn, mlp = self.self_attn, self.mlp
+        if (type(attn) is not ParallelAttention or type(mlp) is not ParallelMLP or attn.qkv_pack or self.apply_residual_connection_post_layernorm
+                or (attention_mask is not None and cu_seqlens is None) or not hidden_states.is_cuda
+                or hidden_states.dtype is not torch.bfloat16 or hidden_states.dim() != 3):
+            return None
+        q, k, v, o, gate, up, down = attn.q_proj, attn.k_proj, attn.v_proj, attn.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj
+        ln1, ln2, core, rotary = self.input_layernorm, self.post_attention_layernorm, attn.core_attention_flash, attn.rotary_emb
+        nq, nk = attn.num_attention_heads_per_partition, attn.num_kv_attention_heads_per_partition
+        d, f = attn.hidden_size_per_attention_head, gate.weight.shape[0]
+        s, b, h = hidden_states.shape
+        if 2.0 * s * b * h * ((2 * nq + 2 * nk) * d + 3 * f) > self.native_call_flops or s * b == 0 or o.bias is not None:
+            return None
+        for m, cls in ((attn, ParallelAttention), (mlp, ParallelMLP), (q, ColumnParallelLinear), (k, ColumnParallelLinear),
+                       (v, ColumnParallelLinear), (o, RowParallelLinear), (gate, ColumnParallelLinear), (up, ColumnParallelLinear),
+                       (down, RowParallelLinear), (ln1, RMSNorm), (ln2, RMSNorm), (core, FlashAttention), (rotary, RotaryEmbedding)):
+            if type(m) is not cls or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
+                return None
+        params = (ln1.weight, q.weight, k.weight, v.weight, o.weight, ln2.weight, gate.weight, up.weight, down.weight)
+        if q.bias is not None:
+            params += (q.bias, k.bias, v.bias)
+        for p in params:
+            if p.dtype is not torch.bfloat16 or not p.is_contiguous() or not p.is_cuda:
+                return None
+        if mlp.activation_func is not GLU_ACTIVATIONS["silu"] or not core.causal or torch.nn.modules.module._has_any_global_hook():
+            return None
+        cos, sin = rotary.tables(s, hidden_states.device)
+        if cu_seqlens is not None:
+            cu_seqlens = cu_seqlens.view(-1).int()
+        scale = core.softmax_scale if core.softmax_scale is not None else d ** -0.5
+        return hidden_states, ((nq, nk, d), f, (ln1.eps, ln2.eps), scale), cos, sin, position_ids, cu_seqlens, params
 
     def forward(self, hidden_states, attention_mask, cu_seqlens=None, position_ids=None, layer_past=None,
                 get_key_value=False):
+        if layer_past is None and not get_key_value:
+            native = self._native_inputs(hidden_states, attention_mask, cu_seqlens, position_ids)
+            if native is not None:
+                return F_.decoder_layer(*native)
         hidden_states, layernorm_output = self.input_layernorm.forward_keep_input(hidden_states)
         attention_output, attention_bias = self.self_attn(layernorm_output, attention_mask, cu_seqlens, position_ids,
                                                           layer_past=layer_past, get_key_value=get_key_value, alibi=self.alibi)

@@ -221,6 +221,35 @@ int64_t ezl_location_idx_rows(int64_t seq_length, int64_t num_epochs, int64_t to
 int ezl_build_location_idx(const int32_t* sizes, int64_t n_sizes, const int32_t* doc_idx, int64_t n_doc_idx, int64_t seq_length,
                            int64_t num_epochs, int64_t tokens_per_epoch, int32_t* out, int64_t out_rows);
 
+/* ---- one decoder layer per call: ParallelTransformerLayer.forward, llama/transformer.py:747-803, and its backward ----
+ * The launches of the entry points above in the layer's order, for callers whose layers are small enough for the host's work
+ * per call to matter.  Same kernels, same results.  Activations [s, b, h] (token row = s_idx * b + b_idx), contiguous. */
+typedef struct {
+    int64_t s, b, h, nq, nk, d, f;        /* tokens, hidden, query / kv heads, head dim, MLP width */
+    int64_t ndocs, npos;                  /* documents (b when cu_seqlens is NULL), rows of the rotary tables */
+    float eps1, eps2, scale;              /* norms' epsilons, softmax scale */
+    const void *ln1, *wq, *wk, *wv;       /* weights [out, in] bf16 */
+    const void *bq, *bk, *bv;             /* biases of q / k / v, or all NULL */
+    const void *wo, *ln2, *wg, *wu, *wd;
+    const void *cos, *sin;                /* fp32 [npos, d / 2] */
+    const void* position_ids;             /* int64 [b, s] or NULL */
+    const void* cu_seqlens;               /* int32 [ndocs + 1] or NULL */
+} ezl_layer;
+/* where a parameter's gradient goes: an fp32 buffer (overwritten, or added to when accumulate != 0), else a bf16 one, else
+ * (both NULL; not for the norms) nowhere */
+typedef struct {
+    void *f32, *bf16;
+    int accumulate;
+} ezl_layer_grad;
+enum { EZL_G_LN1, EZL_G_Q, EZL_G_K, EZL_G_V, EZL_G_O, EZL_G_LN2, EZL_G_GATE, EZL_G_UP, EZL_G_DOWN, EZL_G_BQ, EZL_G_BK, EZL_G_BV, EZL_G_COUNT };
+/* device bytes of the blocks below (256-byte aligned bases): which 0 = saved, 1 = forward temp, 2 = backward temp; -1: bad sizes */
+int64_t ezl_layer_bytes(const ezl_layer* layer, int which);
+/* y = layer(x); `saved` is what ezl_layer_bwd needs, `temp` is free again when the call's work is done */
+int ezl_layer_fwd(const ezl_layer* layer, const void* x, void* y, void* saved, void* temp, void* stream);
+/* grads: EZL_G_COUNT entries */
+int ezl_layer_bwd(const ezl_layer* layer, const void* x, const void* dy, void* dx, const void* saved, void* temp,
+                  const ezl_layer_grad* grads, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -174,3 +174,70 @@ def test_optimizer_over_lists_of_tensors(K, sizes):
         assert all(torch.equal(a[i], b[i]) for a, b in zip(one, lst))
         if params[i] is not None:
             assert torch.equal(params[i], params1[i]) and torch.equal(params[i], lst[0][i].bfloat16())
+
+
+@pytest.mark.parametrize("name", ["mha", "gqa", "bias", "bf16_grads", "packed", "frozen", "checkpoint"])
+def test_layer_in_one_native_call_equals_the_composed_layer(name):
+    """Same kernels in the same order: loss and every gradient bit for bit, except where the composed form rounds once more
+    (unequal q / kv widths: the input gradients of q, k and v are added in bf16 instead of in fp32)."""
+    from easyllm_amd import data, runner
+    h, nq = 256, 4
+    nk = 1 if name in ("gqa", "packed") else 4
+    kw = dict(num_layers=2, hidden_size=h, num_attention_heads=nq, num_kv_attention_heads=nk, intermediate_size=688, vocab_size=512,
+              seq_length=192, bf16=True, checkpoint_activations=name == "checkpoint")
+    if name == "bias":
+        kw["transformer_layer_params"] = {"attention_qkv_bias": True}
+    b, s = (1, 384) if name == "packed" else (2, 192)
+    tokens = torch.randint(0, 512, (b, s), generator=torch.Generator().manual_seed(1)).cuda()
+    labels = torch.randint(0, 512, (b, s), generator=torch.Generator().manual_seed(2)).cuda()
+    pos = torch.arange(s).expand(b, s).contiguous().cuda()
+    inputs = (tokens, pos, None)
+    if name == "packed":
+        cu = [0, 100, 101, 384]
+        inputs = (tokens, torch.tensor([data.get_position_ids(cu)]).cuda(), None, torch.tensor(cu).cuda())
+    results = []
+    for flops in (1e12, 0.0):
+        torch.manual_seed(3)
+        model = runner.build_model({"type": "llama_custom", "kwargs": dict(kw)}).cuda()
+        for m in model.modules():
+            if hasattr(m, "native_call_flops"):
+                m.native_call_flops = flops
+        with torch.no_grad():
+            for p in model.parameters():
+                if p.dim() == 1:
+                    p.add_(0.1 * torch.randn_like(p))
+        if name == "frozen":
+            for n, p in model.named_parameters():
+                p.requires_grad_("q_proj" in n or "layernorm" in n or "up_proj" in n)
+        if name != "bf16_grads":
+            runner.attach_main_grads(model)
+        nodes = []
+        out = model(inputs)
+        fn = out.grad_fn
+        while fn is not None:
+            nodes.append(type(fn).__name__)
+            fn = fn.next_functions[0][0] if fn.next_functions else None
+        if name != "checkpoint":
+            assert any("DecoderLayer" in n for n in nodes) == (flops > 0)
+        for _ in range(2):  # the second pass adds to the gradients
+            loss = runner.forward_step(model, inputs, (labels, torch.ones(b, s, device="cuda")))
+        grads = {n: (p.main_grad if hasattr(p, "main_grad") else p.grad) for n, p in model.named_parameters() if p.requires_grad}
+        results.append((out.float(), loss, {n: g.float() for n, g in grads.items()}))
+    (out1, loss1, g1), (out0, loss0, g0) = results
+    assert torch.equal(out1, out0) and torch.equal(loss1, loss0) and g1.keys() == g0.keys()
+    for n in g0:
+        if nk == nq:
+            assert torch.equal(g1[n], g0[n]), n
+        else:  # 2 roundings of 2^-9 each in one layer's input gradient, carried through the layers below
+            assert (g1[n] - g0[n]).norm() <= 2e-2 * g0[n].norm(), n
+
+
+def test_a_hooked_submodule_keeps_the_composed_layer():
+    from easyllm_amd import runner
+    model = runner.build_model({"type": "llama_custom", "kwargs": dict(num_layers=1, hidden_size=128, num_attention_heads=2, intermediate_size=256,
+                                                                       vocab_size=512, seq_length=64, bf16=True)}).cuda()
+    seen = []
+    model.get_submodule("3").mlp.register_forward_hook(lambda m, i, o: seen.append(o[0].shape))
+    tokens = torch.randint(0, 512, (1, 64)).cuda()
+    model((tokens, torch.arange(64).view(1, 64).cuda(), None))
+    assert seen == [torch.Size([64, 1, 128])]
