@@ -4,6 +4,8 @@
 #include "common.h"
 #include "qkv_bias.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -170,12 +172,22 @@ __global__ __launch_bounds__(kBlock) void embed_gather_kernel(const int64_t* __r
 //   cnt[V]   rows per id                      first[V]  smallest row holding the id (its block does the sum)
 //   off[V]   start of the id's bucket         bucket[T] rows grouped by id (order inside a group: as the atomics fell)
 // The owner block of an id sorts that id's bucket by row number before summing, so the order the atomics produced never
-// reaches the result.
-constexpr int kBucketLds = 1024;  // buckets up to this size are sorted in LDS by rank; longer ones through a row bitmap
+// reaches the result.  Ids with more than kOwnedRows rows (a padding token, frequent words) are left to several blocks each,
+// a slice of the columns per block.
+constexpr int kOwnedRows = 32;
+inline int64_t embed_heavy_max(int64_t rows) { return rows / kOwnedRows + 1; }  // more ids than this cannot be that frequent
+
+// The lanes of the wave that hold the same id as its first active lane (a run of padding is all of them), and whether this lane
+// is one of them: their atomics on one address become one.
+__device__ __forceinline__ bool same_as_first_lane(int id, unsigned long long& mask) {
+    const bool same = id == __builtin_amdgcn_readfirstlane(id);
+    mask = __ballot(same);
+    return same;
+}
 
 __global__ __launch_bounds__(kBlock) void embed_tables_init_kernel(int* __restrict__ cnt, int* __restrict__ first,
                                                                    int* __restrict__ fill, int* __restrict__ cursor, int64_t V) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *cursor = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 2) cursor[threadIdx.x] = 0;  // next free bucket entry, number of frequent ids
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < V; i += (int64_t)gridDim.x * kBlock) {
         cnt[i] = 0;
         fill[i] = 0;
@@ -188,8 +200,14 @@ __global__ __launch_bounds__(kBlock) void embed_count_kernel(const int64_t* __re
     for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < rows; r += (int64_t)gridDim.x * kBlock) {
         const int64_t id = ids[r];
         if (id < 0 || id >= V) continue;
-        atomicAdd(cnt + id, 1);
-        atomicMin(first + id, (int)r);
+        unsigned long long mask;
+        if (!same_as_first_lane((int)id, mask)) {
+            atomicAdd(cnt + id, 1);
+            atomicMin(first + id, (int)r);
+        } else if ((int)(threadIdx.x & 63) == __builtin_ctzll(mask)) {  // the lowest lane holds the smallest row
+            atomicAdd(cnt + id, (int)__popcll(mask));
+            atomicMin(first + id, (int)r);
+        }
     }
 }
 
@@ -198,11 +216,14 @@ __global__ __launch_bounds__(kBlock) void embed_count_kernel(const int64_t* __re
 // takes the next cnt[id] entries from a running cursor; no prefix sum over the vocabulary is needed.
 __global__ __launch_bounds__(kBlock) void embed_assign_kernel(const int64_t* __restrict__ ids, const int* __restrict__ cnt,
                                                               const int* __restrict__ first, int* __restrict__ off,
-                                                              int* __restrict__ cursor, int64_t rows, int64_t V) {
+                                                              int* __restrict__ cursor, int* __restrict__ heavy, int64_t rows,
+                                                              int64_t V) {
     for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < rows; r += (int64_t)gridDim.x * kBlock) {
         const int64_t id = ids[r];
         if (id < 0 || id >= V || first[id] != (int)r) continue;
-        off[id] = atomicAdd(cursor, cnt[id]);
+        const int n = cnt[id];
+        off[id] = atomicAdd(cursor, n);
+        if (n > kOwnedRows) heavy[atomicAdd(cursor + 1, 1)] = (int)id;
     }
 }
 
@@ -212,7 +233,17 @@ __global__ __launch_bounds__(kBlock) void embed_bucket_kernel(const int64_t* __r
     for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < rows; r += (int64_t)gridDim.x * kBlock) {
         const int64_t id = ids[r];
         if (id < 0 || id >= V) continue;
-        bucket[off[id] + atomicAdd(fill + id, 1)] = (int)r;
+        unsigned long long mask;
+        int at;
+        if (!same_as_first_lane((int)id, mask)) {
+            at = atomicAdd(fill + id, 1);
+        } else {
+            const int lane = threadIdx.x & 63, leader = __builtin_ctzll(mask);
+            int base = 0;
+            if (lane == leader) base = atomicAdd(fill + id, (int)__popcll(mask));
+            at = __builtin_amdgcn_readlane(base, leader) + (int)__popcll(mask & ((1ull << lane) - 1));
+        }
+        bucket[off[id] + at] = (int)r;
     }
 }
 
@@ -230,27 +261,110 @@ __global__ __launch_bounds__(kBlock) void zero_f32x4_kernel(f32x4* __restrict__ 
 
 // overwrite: dW[id] = sum instead of dW[id] += sum, and the rows of ids that do not occur are zero-filled (the whole
 // [V, h] gradient is then defined by this launch: no separate fill pass).
-constexpr int kWindowRows = 2048;  // an id with more than kBucketLds rows is ordered through a bitmap over this many row numbers
+constexpr int kWindowRows = 2048;  // a frequent id's rows are put in order through a bitmap over this many row numbers
 
+// One frequent id, columns col0 + 2 thread, + 1: a thread walks the id's rows in order with up to 24 rows' loads in flight (one
+// register each), so that the time is the latency of n / 24 loads rather than of n / 4.  (1000 padding rows of 4000, h = 2048:
+// the scatter kernel 430 -> 79 us.)
+__device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY, float* __restrict__ dW, const int* __restrict__ mine, int n,
+                                                  int64_t id, int col0, int64_t rows, int h, int overwrite, int* list, unsigned* bits, int& wtot) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int col = col0 + 2 * threadIdx.x;
+    const bool live = col < h;
+    const int lane_col = live ? col : 0;
+    float a0 = 0.f, a1 = 0.f;
+    // rows are put in order a window at a time: every lane of the first wave owns one 32-row word of a bitmap, counts its bits,
+    // and after a scan over the wave writes its rows into the ordered list
+    for (int64_t w0 = 0; w0 < rows; w0 += kWindowRows) {
+        __syncthreads();  // the previous window's (or id's) LDS use is over
+        if (threadIdx.x < 64) bits[threadIdx.x] = 0u;
+        __syncthreads();
+        for (int i = threadIdx.x; i < n; i += kBlock) {
+            const int64_t r = (int64_t)mine[i] - w0;
+            if (r >= 0 && r < kWindowRows) atomicOr(&bits[r >> 5], 1u << (r & 31));
+        }
+        __syncthreads();
+        if (wv == 0) {
+            unsigned m = bits[lane];
+            const int mine_n = __builtin_popcount(m);
+            int incl = mine_n;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += v;
+            }
+            if (lane == 63) wtot = incl;
+            int pos = incl - mine_n;
+            while (m) {
+                list[pos++] = (int)w0 + 32 * lane + __builtin_ctz(m);
+                m &= m - 1;
+            }
+        }
+        __syncthreads();
+        const int m = wtot;
+        int i = 0;
+        auto batch = [&](auto N) {
+            constexpr int U = decltype(N)::value;
+            for (; i + U <= m; i += U) {
+                bf16x2 v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {  // (scalar row offset + one lane offset: no address registers per row)
+                    const int64_t row = __builtin_amdgcn_readfirstlane(list[i + u]);
+                    v[u] = *reinterpret_cast<const bf16x2*>(dY + row * h + lane_col);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    a0 += (float)v[u][0];
+                    a1 += (float)v[u][1];
+                }
+            }
+        };
+        batch(std::integral_constant<int, 24>{});
+        batch(std::integral_constant<int, 4>{});
+        batch(std::integral_constant<int, 1>{});
+    }
+    if (live) {
+        f32x2* dst = reinterpret_cast<f32x2*>(dW + id * h + col);
+        f32x2 o = {a0, a1};
+        if (!overwrite) {
+            const f32x2 old = *dst;
+            o[0] += old[0];
+            o[1] += old[1];
+        }
+        *dst = o;
+    }
+}
+
+// (rows of up to 4096: six waves per SIMD, as the zero fill wants them)
 template <int MAXC>
-__global__ __launch_bounds__(kBlock) void embed_scatter_bucket_kernel(const int64_t* __restrict__ ids, const bf16_t* __restrict__ dY,
+__global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucket_kernel(const int64_t* __restrict__ ids, const bf16_t* __restrict__ dY,
                                                                       float* __restrict__ dW, const int* __restrict__ cnt,
                                                                       const int* __restrict__ first, const int* __restrict__ off,
-                                                                      const int* __restrict__ bucket, int64_t rows, int h,
-                                                                      int64_t V, int overwrite) {
-    static_assert(kWindowRows == 32 * 64 && kWindowRows >= kBucketLds, "one bitmap word per lane of the first wave");
-    __shared__ int list[kWindowRows];  // rows of the current id in increasing order (first kBucketLds entries double as `sorted`)
-    __shared__ int raw[kBucketLds];
+                                                                      const int* __restrict__ bucket, const int* __restrict__ cursor,
+                                                                      const int* __restrict__ heavy, int64_t rows, int h, int64_t V,
+                                                                      int overwrite) {
+    static_assert(kWindowRows == 32 * 64, "one bitmap word per lane of the first wave");
+    __shared__ int list[kWindowRows];  // rows of the current id in increasing order
+    __shared__ int raw[kBlock];
     __shared__ unsigned bits[64];
     __shared__ int wtot;
     int* sorted = list;
     const int h8 = h >> 3;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int helpers = (int)gridDim.x < 512 ? (int)gridDim.x : 512;
+    if ((int)blockIdx.x < helpers) {  // the frequent ids first, as they take longest; the other blocks need not even look
+        const int slices = (h + 2 * kBlock - 1) / (2 * kBlock), items = cursor[1] * slices;
+        for (int it = blockIdx.x; it < items; it += helpers) {
+            const int id = heavy[it / slices];
+            embed_frequent_id(dY, dW, bucket + off[id], cnt[id], id, (it % slices) * 2 * kBlock, rows, h, overwrite, list, bits, wtot);
+        }
+        __syncthreads();
+    }
     for (int64_t t = blockIdx.x; t < rows; t += gridDim.x) {
         const int64_t id = ids[t];
         if (id < 0 || id >= V) continue;
         if (first[id] != (int)t) continue;  // the block of the smallest row of an id owns it (uniform over the block)
         const int n = cnt[id];
+        if (n > kOwnedRows) continue;
         const int* mine = bucket + off[id];
         float acc[MAXC][8];
 #pragma unroll
@@ -298,50 +412,18 @@ __global__ __launch_bounds__(kBlock) void embed_scatter_bucket_kernel(const int6
         };
         if (n == 1) {
             add_row(t);
-        } else if (n <= kBucketLds) {
+        } else {
             __syncthreads();  // the previous id's LDS use is over
-            for (int i = threadIdx.x; i < n; i += kBlock) raw[i] = mine[i];
+            if ((int)threadIdx.x < n) raw[threadIdx.x] = mine[threadIdx.x];
             __syncthreads();
-            for (int i = threadIdx.x; i < n; i += kBlock) {  // rows are distinct: rank = number of smaller rows
-                const int v = raw[i];
+            if ((int)threadIdx.x < n) {  // rows are distinct: rank = number of smaller rows
+                const int v = raw[threadIdx.x];
                 int rank = 0;
                 for (int j = 0; j < n; ++j) rank += raw[j] < v;
                 sorted[rank] = v;
             }
             __syncthreads();
             add_rows(sorted, n);
-        } else {
-            // A frequent id (padding, say): its rows are put in order through a bitmap over row numbers, a window of
-            // kWindowRows rows at a time -- every lane of the first wave owns one 32-row word, counts its bits, and after a
-            // scan over the wave writes its rows into the ordered list.  n / kBlock bucket reads per thread and window.
-            for (int64_t w0 = 0; w0 < rows; w0 += kWindowRows) {
-                __syncthreads();  // the previous window's (or id's) LDS use is over
-                if (threadIdx.x < 64) bits[threadIdx.x] = 0u;
-                __syncthreads();
-                for (int i = threadIdx.x; i < n; i += kBlock) {
-                    const int64_t r = (int64_t)mine[i] - w0;
-                    if (r >= 0 && r < kWindowRows) atomicOr(&bits[r >> 5], 1u << (r & 31));
-                }
-                __syncthreads();
-                if (wv == 0) {
-                    unsigned m = bits[lane];
-                    const int mine_n = __builtin_popcount(m);
-                    int incl = mine_n;
-#pragma unroll
-                    for (int o = 1; o < 64; o <<= 1) {
-                        const int v = __shfl_up(incl, o, 64);
-                        if (lane >= o) incl += v;
-                    }
-                    if (lane == 63) wtot = incl;
-                    int pos = incl - mine_n;
-                    while (m) {
-                        list[pos++] = (int)w0 + 32 * lane + __builtin_ctz(m);
-                        m &= m - 1;
-                    }
-                }
-                __syncthreads();
-                add_rows(list, wtot);
-            }
         }
 #pragma unroll
         for (int c = 0; c < MAXC; ++c) {
@@ -723,7 +805,7 @@ extern "C" int ezl_embed_gather(const void* ids, const void* weight, void* out, 
 
 extern "C" int64_t ezl_embed_scatter_add_workspace_bytes(int64_t rows, int64_t vocab) {
     if (rows < 0 || vocab <= 0) return -1;
-    return (4 * vocab + rows + 4) * (int64_t)sizeof(int);
+    return (4 * vocab + rows + 4 + embed_heavy_max(rows)) * (int64_t)sizeof(int);
 }
 
 extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dweight_f32, void* workspace, int64_t workspace_bytes,
@@ -745,12 +827,13 @@ extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dwei
     int* fill = off + vocab;
     int* bucket = fill + vocab;
     int* cursor = bucket + rows;
+    int* heavy = cursor + 4;
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(embed_tables_init_kernel, dim3(grid_for(vocab, kBlock, 1024)), dim3(kBlock), 0, st, cnt, first, fill, cursor, vocab);
     hipLaunchKernelGGL(embed_count_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, cnt, first,
                        rows, vocab);
     hipLaunchKernelGGL(embed_assign_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, cnt, first, off,
-                       cursor, rows, vocab);
+                       cursor, heavy, rows, vocab);
     hipLaunchKernelGGL(embed_bucket_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, off, fill,
                        bucket, rows, vocab);
     EZL_LAUNCH_CHECK("ezl_embed_scatter_add(tables)");
@@ -768,13 +851,13 @@ extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dwei
     const dim3 grid(grid_for(overwrite ? (rows > vocab ? rows : vocab) : rows, 1));
     if (h <= 8 * kBlock * 2)
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<2>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (float*)dweight_f32, cnt, first, off, bucket, rows, (int)h, vocab, overwrite);
+                           (float*)dweight_f32, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
     else if (h <= 8 * kBlock * 4)
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<4>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (float*)dweight_f32, cnt, first, off, bucket, rows, (int)h, vocab, overwrite);
+                           (float*)dweight_f32, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
     else
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<8>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (float*)dweight_f32, cnt, first, off, bucket, rows, (int)h, vocab, overwrite);
+                           (float*)dweight_f32, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
     EZL_LAUNCH_CHECK("ezl_embed_scatter_add");
     return EZL_OK;
 }
