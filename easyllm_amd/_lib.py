@@ -60,6 +60,7 @@ SIGNATURES = {
     "ezl_ce_prepare": [_vp, _vp, _i32, _i64, _vp, _vp, _i64, _vp],
     "ezl_ce_fwd": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "ezl_ce_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
+    "ezl_ce_loss": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "ezl_ce_fused": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "ezl_ce_reduce": [_vp, _vp, _vp, _vp, _i64, _vp],
     "ezl_scale_by_scalar": [_vp, _vp, _i64, _i32, _vp],

@@ -7,6 +7,7 @@
 //   * ezl_ce_bwd          (softmax - onehot[valid]) * grad_out                        (cross_entropy.py:91-112)
 //   * ezl_ce_fused        loss rows AND d loss / d logits in one visit of the logits, for the
 //                         mean-reduced loss: grad = (softmax - onehot) * w / N
+//   * ezl_ce_loss         the loss rows of ezl_ce_fused alone: scoring and validation
 //   * ezl_ce_reduce       loss = sum(loss_row * w) / N                                (losses.py:55)
 // A row of logits (bf16 or fp32) is owned by one 512-thread block.  When the row fits 64 KiB of
 // LDS it is staged there during the max pass, so HBM sees one read and (for bwd/fused) one write.
@@ -457,6 +458,68 @@ __global__ __launch_bounds__(kWideBlock) void ce_fused_wide_kernel(const bf16_t*
     __builtin_amdgcn_s_waitcnt(0x0F70);  // no LDS write of this block may still be in flight when it ends
 }
 
+// Loss rows without a gradient: maximum and sum in one pass over the row (each thread rescales its sum when its maximum moves),
+// four vectors in flight per thread.  Bound by HBM: 8192 x 32000 in fp32 214 us (4.9 TB/s), against 585 for the fused kernel, which
+// reads the row three times (twice from cache) and writes the gradient.
+template <typename T>
+__global__ __launch_bounds__(kCeBlock) void ce_loss_kernel(const T* __restrict__ logits, const int64_t* __restrict__ labels,
+                                                           const float* __restrict__ weights, float* __restrict__ loss, int64_t rows, int V,
+                                                           int vend) {
+    __shared__ float red[kCeWaves];
+    const int v8 = V >> 3;
+    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        if (weights[r] == 0.f) {  // ignored position
+            if (threadIdx.x == 0) loss[r] = 0.f;
+            continue;
+        }
+        const T* xrow = logits + r * V;
+        float m = -INFINITY, s = 0.f;
+        auto fold = [&](const float (&f)[4][8]) {  // columns past vend and vectors past the row hold -inf
+            float mn = m;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) mn = fmaxf(mn, f[u][k]);
+            if (mn == -INFINITY) return;
+            const float mb = mn * kLog2e;
+            s *= __builtin_amdgcn_exp2f(m * kLog2e - mb);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) s += __builtin_amdgcn_exp2f(f[u][k] * kLog2e - mb);
+            m = mn;
+        };
+        for (int i = threadIdx.x; i < v8; i += 4 * kCeBlock) {
+            float f[4][8];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int j = i + u * kCeBlock;
+                if (j < v8) {
+                    Vec8<T>::load(xrow + (int64_t)j * 8, f[u]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) f[u][k] = -INFINITY;
+                }
+            }
+            if ((i + 3 * kCeBlock) * 8 + 8 > vend) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)
+                        if ((i + u * kCeBlock) * 8 + k >= vend) f[u][k] = -INFINITY;
+            }
+            fold(f);
+        }
+        const float mrow = block_max(m, red);
+        s = block_sum(m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - mrow) * kLog2e), red);
+        if (threadIdx.x == 0) {
+            const int64_t t = labels[r];
+            const bool masked = t < 0 || t >= vend;
+            loss[r] = masked ? logf(s) : (mrow + logf(s)) - (float)xrow[t];
+        }
+    }
+}
+
 // weights[i] = mask[i] * (labels[i] != ignore_index); count[0] = sum(weights) -- one block, fixed order
 __global__ __launch_bounds__(1024) void ce_prepare_kernel(const int64_t* __restrict__ labels, const void* __restrict__ mask,
                                                           int mask_dtype, int64_t ignore_index, float* __restrict__ weights,
@@ -617,6 +680,24 @@ extern "C" int ezl_ce_fused(const void* logits, const void* labels, const void* 
     }
 #undef LAUNCH
     EZL_LAUNCH_CHECK("ezl_ce_fused");
+    return EZL_OK;
+}
+
+extern "C" int ezl_ce_loss(const void* logits, const void* labels, const void* weights, void* loss_rows, int64_t rows, int64_t vocab,
+                           int64_t cut_size, int dtype, void* stream) {
+    int rc = ce_check("ezl_ce_loss", logits, rows, vocab, cut_size, dtype);
+    if (rc) return rc;
+    EZL_REQUIRE(rows == 0 || (labels && weights && loss_rows), EZL_EINVAL, "ezl_ce_loss: null pointer");
+    if (rows == 0) return EZL_OK;
+    const int V = (int)vocab, vend = (int)(vocab - cut_size);
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == 0)
+        hipLaunchKernelGGL((ce_loss_kernel<bf16_t>), dim3(ce_grid(rows)), dim3(kCeBlock), 0, st, (const bf16_t*)logits, (const int64_t*)labels,
+                           (const float*)weights, (float*)loss_rows, rows, V, vend);
+    else
+        hipLaunchKernelGGL((ce_loss_kernel<float>), dim3(ce_grid(rows)), dim3(kCeBlock), 0, st, (const float*)logits, (const int64_t*)labels,
+                           (const float*)weights, (float*)loss_rows, rows, V, vend);
+    EZL_LAUNCH_CHECK("ezl_ce_loss");
     return EZL_OK;
 }
 

@@ -214,8 +214,6 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 #undef EZL_STEP
 #undef EZL_PHASE_SCHED
 
-    // epilogue: acc[i][j] register r is C[m0 + arow + 16 i + (lane & 15)][n0 + brow + 16 j + 4 (lane >> 4) + r]
-    typedef typename Out4<OutT>::type out4_t;
     if (split) {  // this workgroup's share of the reduction, as a dense fp32 tile; gemm_split_reduce_kernel adds the shares
         float* tile = plan.partial + ((size_t)(pid - plan.full) * plan.nsplit + part) * (size_t)(BM * BN);
 #pragma unroll
@@ -225,74 +223,24 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
                 *reinterpret_cast<f32x4*>(tile + (arow + i * 16 + (lane & 15)) * BN + brow + j * 16 + 4 * (lane >> 4)) = acc[i][j];
         return;
     }
-    if constexpr (sizeof(OutT) == 2) {
-        // bf16: 8-byte stores of 4 columns reach only half the write bandwidth of 16-byte ones (3.8 vs 6.7 TB/s on a
-        // 4096 x 32000 output).  Lanes l and l ^ 16 trade halves of two neighbouring column tiles, so that the lane of
-        // the even 16-lane row ends up with 8 consecutive columns of tile 2 jp and its partner with those of tile 2 jp + 1.
-        if ((N % 8 == 0) && (ldc % 8 == 0) && (((uintptr_t)C & 15) == 0)) {
-            const int g = lane >> 4;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int row = m0 + arow + i * 16 + (lane & 15);
-#pragma unroll
-                for (int jp = 0; jp < 2; ++jp) {
-                    float lo[4], hi[4];  // columns +0..3 and +4..7 of this lane's 8
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float ta = acc[i][2 * jp][r], tb = acc[i][2 * jp + 1][r];  // scalars: a bit_cast of a vector element reads element 0
-                        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(ta), __float_as_uint(tb), false, false);
-                        lo[r] = __uint_as_float(sw[0]);
-                        hi[r] = __uint_as_float(sw[1]);
-                    }
-                    const int col = n0 + brow + (2 * jp + (g & 1)) * 16 + 8 * (g >> 1);
-                    if (row >= M || col >= N) continue;
-                    bf16_t* dst = C + (int64_t)row * ldc + col;
-                    bf16x8 v;
-                    if (accumulate) {
-                        const bf16x8 old = *reinterpret_cast<const bf16x8*>(dst);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            v[r] = (bf16_t)(lo[r] + (float)old[r]);
-                            v[4 + r] = (bf16_t)(hi[r] + (float)old[4 + r]);
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            v[r] = (bf16_t)lo[r];
-                            v[4 + r] = (bf16_t)hi[r];
-                        }
-                    }
-                    *reinterpret_cast<bf16x8*>(dst) = v;
-                }
-            }
-            return;
-        }
+    const int mrem = M - m0 < BM ? M - m0 : BM, nrem = N - n0;
+    OutT* Ct = C + (int64_t)m0 * ldc + n0;
+    if (N % 8 == 0 && ldc % (16 / (int)sizeof(OutT)) == 0 && ((uintptr_t)C & 15) == 0 && ldc < (1 << 21) / ((int)sizeof(OutT) / 2)) {
+        store_tile_flags<8, 4, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ldc, mrem, nrem, arow, brow, lane, accumulate);
+        return;
     }
-    const bool vec_ok = (N % 4 == 0) && (ldc % 4 == 0) && (((uintptr_t)C & 15) == 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int row = m0 + arow + i * 16 + (lane & 15);
+    for (int i = 0; i < 8; ++i) {  // any width, alignment and row stride: element by element
+        const int row = arow + i * 16 + (lane & 15);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int col = n0 + brow + j * 16 + 4 * (lane >> 4);
-            if (row >= M || col >= N) continue;
-            OutT* dst = C + (int64_t)row * ldc + col;
-            if (vec_ok) {
-                out4_t v;
-                if (accumulate) {
-                    const out4_t old = *reinterpret_cast<const out4_t*>(dst);
+            const int col = brow + j * 16 + 4 * (lane >> 4);
+            if (row >= mrem || col >= nrem) continue;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = (OutT)(acc[i][j][r] + (float)old[r]);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = (OutT)acc[i][j][r];
-                }
-                *reinterpret_cast<out4_t*>(dst) = v;
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (col + r < N) store_out<OutT>(dst + r, acc[i][j][r], accumulate != 0);
-            }
+            for (int r = 0; r < 4; ++r)
+                if (col + r < nrem)
+                    store_out<OutT>(Ct + (int64_t)row * ldc + col + r, accumulate & kRoundResult ? (float)(bf16_t)acc[i][j][r] : acc[i][j][r],
+                                    (accumulate & 1) != 0);
         }
     }
 }
@@ -462,83 +410,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
-    if constexpr (sizeof(OutT) == 4) {  // fp32 results (weight gradients): the 4 columns a lane owns as one 16-byte store
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int row = m0 + arow + i * 16 + (lane & 15);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int col = n0 + brow + j * 16 + 4 * (lane >> 4);
-                if (row >= M || col >= N) continue;
-                float* dst = C + (int64_t)row * ldc + col;
-                f32x4 v = acc[i][j];
-                if (accumulate) {
-                    const f32x4 old = *reinterpret_cast<const f32x4*>(dst);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] += old[r];
-                }
-                *reinterpret_cast<f32x4*>(dst) = v;
-            }
-        }
-    } else {
-
-    // epilogue: acc[i][j] register r is C[m0 + arow + 16 i + (lane & 15)][n0 + brow + 16 j + 4 (lane >> 4) + r]
-    // C is addressed as a buffer that starts at the tile's corner and ends behind the tile's last valid row: a store to a row
-    // past M drops out by the buffer's range check, one to a column past N by an offset that is out of range.  The epilogue is
-    // thus straight-line code (no branch per store, and `accumulate` decided once), whose 32 independent chains of
-    // register moves, conversions and stores the compiler interleaves; with a branch per store it took twice as long.
-    constexpr int SZ = 2;
     const int mrem = M - m0 < BM ? M - m0 : BM;
-    const __amdgpu_buffer_rsrc_t cbuf = __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<char*>(C + (int64_t)m0 * ldc + n0), 0, (uint32_t)(((int64_t)mrem * ldc - n0) * SZ), 0x00020000);
-    const uint32_t row_off = (uint32_t)(arow + (lane & 15)) * (uint32_t)(ldc * SZ);
-    const uint32_t row_step = (uint32_t)(16 * ldc * SZ);  // scalar: rows 16 i
-    constexpr uint32_t kOut = 0x80000000u;
-    auto epilogue = [&](auto ACC) {
-        constexpr bool accum = decltype(ACC)::value;
-        {  // lanes l and l ^ 16 trade halves of two neighbouring column tiles: 16-byte stores
-            const int g = lane >> 4;
-            uint32_t voff[4];
-#pragma unroll
-            for (int jp = 0; jp < 4; ++jp) {
-                const int col = brow + (2 * jp + (g & 1)) * 16 + 8 * (g >> 1);
-                voff[jp] = n0 + col < N ? row_off + (uint32_t)col * SZ : kOut;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-#pragma unroll
-                for (int jp = 0; jp < 4; ++jp) {
-                    float lo[4], hi[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float ta = acc[i][2 * jp][r], tb = acc[i][2 * jp + 1][r];
-                        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(ta), __float_as_uint(tb), false, false);
-                        lo[r] = __uint_as_float(sw[0]);
-                        hi[r] = __uint_as_float(sw[1]);
-                    }
-                    bf16x8 v;
-                    if constexpr (accum) {
-                        const bf16x8 old = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff[jp], i * row_step, 0));
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            v[r] = (bf16_t)(lo[r] + (float)old[r]);
-                            v[4 + r] = (bf16_t)(hi[r] + (float)old[4 + r]);
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            v[r] = (bf16_t)lo[r];
-                            v[4 + r] = (bf16_t)hi[r];
-                        }
-                    }
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, voff[jp], i * row_step, 0);
-                }
-            }
-        }
-    };
-    if (accumulate) epilogue(std::true_type{});
-    else epilogue(std::false_type{});
-    }
+    OutT* Ct = C + (int64_t)m0 * ldc + n0;
+    store_tile_flags<8, 8, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ldc, mrem, N - n0, arow, brow, lane, accumulate);
 }
 
 // C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order.  One block per 16 rows of a tile: a thread owns 16
@@ -563,6 +437,11 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(OutT* __restrict
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[4 * q + e] += x[e];
         }
+    }
+    if (accumulate & kRoundResult) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = (float)(bf16_t)v[e];
+        accumulate = 0;
     }
     OutT* dst = C + (int64_t)row * ldc + col;
     if (col + 16 <= N && ldc % 8 == 0 && ((uintptr_t)C & 15) == 0) {  // whole 16-column piece, 16-byte aligned
@@ -760,7 +639,7 @@ void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int
     // The 4-wave kernel: forward form with a bf16 result, and weight-gradient form with an fp32 result (inside the steps
     // 0.4 - 0.8 % faster than the 8-wave kernel although a single launch at K = 4096 is not: it moves a third fewer LDS
     // bytes, and the steps are bound by power).  With a k-strided B only (input gradients) it gained nothing.
-    if constexpr ((A_KC && B_KC && sizeof(OutT) == 2) || (!A_KC && !B_KC && sizeof(OutT) == 4)) {
+    if constexpr ((A_KC && B_KC) || (!A_KC && !B_KC && sizeof(OutT) == 4)) {
         const int vec = 16 / (int)sizeof(OutT);
         // (a launch that is split tiles only is judged by the length of a share)
         const int w4_ktiles = plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk;
@@ -785,8 +664,8 @@ bool small_stores_ok(int64_t ldc) {
 template <bool A_KC, bool B_KC, typename OutT>
 void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
             void* workspace, int64_t workspace_bytes, hipStream_t st) {
-    constexpr int form = A_KC ? (B_KC ? 0 : 1) : (sizeof(OutT) == 4 ? 2 : 3);
-    if constexpr (A_KC ? sizeof(OutT) == 2 : !B_KC) {
+    constexpr int form = A_KC ? (B_KC ? (sizeof(OutT) == 4 ? 4 : 0) : 1) : (sizeof(OutT) == 4 ? 2 : 3);
+    if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC) {
         if (small_stores_ok<OutT>(ldc)) {
             const GemmPlan plan = choose_plan(M, N, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
             if (plan.kind != kTile256) {
@@ -834,7 +713,7 @@ static int check_operands(const void* A, const void* B, int64_t M, int64_t N, in
 
 // a_kc / b_kc: 1 if the operand's reduction index is its contiguous one
 //   A: a_kc ? A[m * lda + k] : A[k * lda + m]        B: b_kc ? B[n * ldb + k] : B[k * ldb + n]
-// out_dtype: 0 bf16, 1 fp32.  accumulate: C += A*B instead of C = A*B.
+// out_dtype: 0 bf16, 1 fp32, 2 fp32 holding bf16 values (forward form, no accumulation).  accumulate: C += A*B instead of C = A*B.
 // bytes of workspace with which a launch of this shape evens out a mostly empty last round of tiles (0: none needed)
 extern "C" int64_t ezl_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) { return plan_bytes(M, N, K); }
 
@@ -842,12 +721,18 @@ extern "C" int ezl_gemm_bf16(const void* A, const void* B, void* C, int64_t M, i
                              int64_t ldc, int a_kc, int b_kc, int out_dtype, int accumulate, void* workspace,
                              int64_t workspace_bytes, void* stream) {
     EZL_REQUIRE(M >= 0 && N >= 0 && K >= 0, EZL_EINVAL, "ezl_gemm_bf16: negative size");
-    EZL_REQUIRE(out_dtype == 0 || out_dtype == 1, EZL_EUNSUPPORTED, "ezl_gemm_bf16: out_dtype must be 0 (bf16) or 1 (fp32)");
+    EZL_REQUIRE(out_dtype == 0 || out_dtype == 1 || (out_dtype == 2 && a_kc && b_kc && !accumulate), EZL_EUNSUPPORTED,
+                "ezl_gemm_bf16: out_dtype must be 0 (bf16), 1 (fp32) or, for an overwriting forward product, 2 (bf16 values as fp32)");
+    if (accumulate) accumulate = 1;
+    if (out_dtype == 2) {
+        out_dtype = 1;
+        accumulate = kRoundResult;
+    }
     if (M == 0 || N == 0) return EZL_OK;
     EZL_REQUIRE(C, EZL_EINVAL, "ezl_gemm_bf16: null pointer");
     if (K == 0) {  // empty reduction (a weight gradient over zero tokens): C = 0, or C unchanged when accumulating
         EZL_REQUIRE(ldc >= N, EZL_EINVAL, "ezl_gemm_bf16: leading dimension too small");
-        if (!accumulate) {
+        if (accumulate != 1) {
             if (out_dtype == 0) hipLaunchKernelGGL(zero_c_kernel<bf16_t>, dim3(256), dim3(256), 0, (hipStream_t)stream, (bf16_t*)C, M, N, ldc);
             else hipLaunchKernelGGL(zero_c_kernel<float>, dim3(256), dim3(256), 0, (hipStream_t)stream, (float*)C, M, N, ldc);
             EZL_LAUNCH_CHECK("ezl_gemm_bf16(zero)");

@@ -41,80 +41,6 @@ __device__ __forceinline__ GemmProblem problem_of(const GemmSmallArgs& a, int ti
     return p;
 }
 
-// acc[i][j] register r is C[m0 + row0 + 16 i + (lane & 15)][n0 + col0 + 16 j + 4 (lane >> 4) + r].
-// C is addressed as a buffer that starts at the tile's corner and ends behind the last valid element of its last valid row: a
-// store past either edge drops out by the range check (for columns: an offset that is out of range), so the code is
-// straight-line.  bf16: lanes l and l ^ 16 trade halves of two neighbouring column tiles, 16-byte stores.  VEC = false (rows
-// that do not start on 16 bytes, or a width that is no multiple of 8): one element per store.
-template <int TM, int TN, typename OutT, bool ACC, bool VEC>
-__device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT* C, int64_t ldc, int mrem, int nrem, int row0, int col0,
-                                                int lane) {
-    constexpr int SZ = (int)sizeof(OutT);
-    constexpr uint32_t kOut = 0x80000000u;
-    const __amdgpu_buffer_rsrc_t cbuf = __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<char*>(C), 0, (uint32_t)(((int64_t)(mrem - 1) * ldc + nrem) * SZ), 0x00020000);
-    const uint32_t row_off = (uint32_t)(row0 + (lane & 15)) * (uint32_t)(ldc * SZ);
-    const uint32_t row_step = (uint32_t)(16 * ldc * SZ);
-    if constexpr (!VEC) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int col = col0 + j * 16 + 4 * (lane >> 4) + r;
-                    const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
-                    float v = acc[i][j][r];
-                    if constexpr (SZ == 2) {
-                        if constexpr (ACC) v += (float)__builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(cbuf, voff, i * row_step, 0));
-                        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (bf16_t)v), cbuf, voff, i * row_step, 0);
-                    } else {
-                        if constexpr (ACC) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(cbuf, voff, i * row_step, 0));
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), cbuf, voff, i * row_step, 0);
-                    }
-                }
-    } else if constexpr (SZ == 2) {
-        const int g = lane >> 4;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-#pragma unroll
-            for (int jp = 0; jp < TN / 2; ++jp) {
-                const int col = col0 + (2 * jp + (g & 1)) * 16 + 8 * (g >> 1);
-                const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
-                float v[8];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float ta = acc[i][2 * jp][r], tb = acc[i][2 * jp + 1][r];
-                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(ta), __float_as_uint(tb), false, false);
-                    v[r] = __uint_as_float(sw[0]);
-                    v[4 + r] = __uint_as_float(sw[1]);
-                }
-                if constexpr (ACC) {
-                    const bf16x8 old = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff, i * row_step, 0));
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) v[r] += (float)old[r];
-                }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, voff, i * row_step, 0);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int col = col0 + j * 16 + 4 * (lane >> 4);
-                const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
-                f32x4 v = acc[i][j];
-                if constexpr (ACC) {
-                    const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff, i * row_step, 0));
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] += old[r];
-                }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, voff, i * row_step, 0);
-            }
-        }
-    }
-}
 template <typename OutT>
 __device__ __forceinline__ bool vector_stores(const GemmProblem& p) {
     return p.N % 8 == 0 && p.ldc % (16 / (int)sizeof(OutT)) == 0 && ((uintptr_t)p.C & 15) == 0;
@@ -123,13 +49,8 @@ template <int TM, int TN, typename OutT>
 __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], const GemmProblem& p, int m0, int n0, int row0, int col0, int lane) {
     OutT* C = (OutT*)p.C + (int64_t)m0 * p.ldc + n0;
     const int mrem = p.M - m0 < 256 ? p.M - m0 : 256, nrem = p.N - n0;  // (no tile is taller: the range fits 31 bits)
-    if (vector_stores<OutT>(p)) {
-        if (p.accumulate) store_tile_impl<TM, TN, OutT, true, true>(acc, C, p.ldc, mrem, nrem, row0, col0, lane);
-        else store_tile_impl<TM, TN, OutT, false, true>(acc, C, p.ldc, mrem, nrem, row0, col0, lane);
-    } else {
-        if (p.accumulate) store_tile_impl<TM, TN, OutT, true, false>(acc, C, p.ldc, mrem, nrem, row0, col0, lane);
-        else store_tile_impl<TM, TN, OutT, false, false>(acc, C, p.ldc, mrem, nrem, row0, col0, lane);
-    }
+    if (vector_stores<OutT>(p)) store_tile_flags<TM, TN, OutT, true, sizeof(OutT) == 4>(acc, C, p.ldc, mrem, nrem, row0, col0, lane, p.accumulate);
+    else store_tile_flags<TM, TN, OutT, false, sizeof(OutT) == 4>(acc, C, p.ldc, mrem, nrem, row0, col0, lane, p.accumulate);
 }
 
 // this workgroup's share of the reduction, as a dense fp32 tile; small_reduce_kernel adds the shares
@@ -457,13 +378,18 @@ __global__ __launch_bounds__(256) void small_reduce_kernel(const GemmSmallArgs a
 #pragma unroll
         for (int r = 0; r < 4; ++r) { v[r] += x[r]; v[4 + r] += y[r]; }
     }
+    if (p.accumulate & kRoundResult) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[r] = (float)(bf16_t)v[r];
+    }
+    const bool accumulate = p.accumulate & 1;
     OutT* dst = (OutT*)p.C + (int64_t)row * p.ldc + col;
     if (!vector_stores<OutT>(p)) {
 #pragma unroll
         for (int r = 0; r < 8; ++r)
-            if (col + r < p.N) dst[r] = (OutT)(p.accumulate ? v[r] + (float)dst[r] : v[r]);
+            if (col + r < p.N) dst[r] = (OutT)(accumulate ? v[r] + (float)dst[r] : v[r]);
     } else if constexpr (sizeof(OutT) == 2) {
-        if (p.accumulate) {
+        if (accumulate) {
             const bf16x8 old = ld_bf16x8((const bf16_t*)dst);
 #pragma unroll
             for (int r = 0; r < 8; ++r) v[r] += (float)old[r];
@@ -475,7 +401,7 @@ __global__ __launch_bounds__(256) void small_reduce_kernel(const GemmSmallArgs a
             f32x4 o;
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[r] = v[4 * h + r];
-            if (p.accumulate) o += *reinterpret_cast<const f32x4*>(dst + 4 * h);
+            if (accumulate) o += *reinterpret_cast<const f32x4*>(dst + 4 * h);
             *reinterpret_cast<f32x4*>(dst + 4 * h) = o;
         }
     }
@@ -522,6 +448,7 @@ void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs
     if (form == 0) launch_kind<true, true, bf16_t, false>(plan.kind, a, tail, stream);
     else if (form == 1 && multi) launch_kind<true, false, bf16_t, true>(plan.kind, a, tail, stream);
     else if (form == 1) launch_kind<true, false, bf16_t, false>(plan.kind, a, tail, stream);
+    else if (form == 4) launch_kind<true, true, float, false>(plan.kind, a, tail, stream);
     else if (form == 2) launch_kind<false, false, float, false>(plan.kind, a, tail, stream);
     else launch_kind<false, false, bf16_t, false>(plan.kind, a, tail, stream);
 }

@@ -17,6 +17,9 @@ struct KSegments {
     int K1, K2;
 };
 
+// Kernels take it in place of `accumulate`: an fp32 result is rounded to bf16 first (logits that are handed out in fp32).
+constexpr int kRoundResult = 2;
+
 namespace {
 
 constexpr int BM = 256, BN = 256, BK = 64;
@@ -156,9 +159,94 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-template <typename OutT> struct Out4;
-template <> struct Out4<bf16_t> { typedef bf16x4 type; };
-template <> struct Out4<float> { typedef f32x4 type; };
+// acc[i][j] register r is C[m0 + row0 + 16 i + (lane & 15)][n0 + col0 + 16 j + 4 (lane >> 4) + r].
+// C is addressed as a buffer that starts at the tile's corner and ends behind the last valid element of its last valid row: a
+// store past either edge drops out by the range check (for columns: an offset that is out of range), so the code is
+// straight-line (a branch per store instead: 4000 x 32000 x 2048 with an fp32 result 632 us against 482; a weight gradient of
+// 32000 x 4096 over 1531 tokens 420 against 405).  bf16: lanes l and l ^ 16 trade halves of two neighbouring column tiles, 16-byte stores.  VEC = false (rows
+// that do not start on 16 bytes, or a width that is no multiple of 8): one element per store.
+template <int TM, int TN, typename OutT, bool ACC, bool VEC, bool ROUND = false>
+__device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT* C, int64_t ldc, int mrem, int nrem, int row0, int col0,
+                                                int lane) {
+    constexpr int SZ = (int)sizeof(OutT);
+    constexpr uint32_t kOut = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t cbuf = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<char*>(C), 0, (uint32_t)(((int64_t)(mrem - 1) * ldc + nrem) * SZ), 0x00020000);
+    const uint32_t row_off = (uint32_t)(row0 + (lane & 15)) * (uint32_t)(ldc * SZ);
+    const uint32_t row_step = (uint32_t)(16 * ldc * SZ);
+    if constexpr (!VEC) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int col = col0 + j * 16 + 4 * (lane >> 4) + r;
+                    const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
+                    float v = acc[i][j][r];
+                    if constexpr (ROUND) v = (float)(bf16_t)v;
+                    if constexpr (SZ == 2) {
+                        if constexpr (ACC) v += (float)__builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(cbuf, voff, i * row_step, 0));
+                        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (bf16_t)v), cbuf, voff, i * row_step, 0);
+                    } else {
+                        if constexpr (ACC) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(cbuf, voff, i * row_step, 0));
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), cbuf, voff, i * row_step, 0);
+                    }
+                }
+    } else if constexpr (SZ == 2) {
+        const int g = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int jp = 0; jp < TN / 2; ++jp) {
+                const int col = col0 + (2 * jp + (g & 1)) * 16 + 8 * (g >> 1);
+                const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
+                float v[8];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float ta = acc[i][2 * jp][r], tb = acc[i][2 * jp + 1][r];
+                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(ta), __float_as_uint(tb), false, false);
+                    v[r] = __uint_as_float(sw[0]);
+                    v[4 + r] = __uint_as_float(sw[1]);
+                }
+                if constexpr (ACC) {
+                    const bf16x8 old = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff, i * row_step, 0));
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) v[r] += (float)old[r];
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, voff, i * row_step, 0);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int col = col0 + j * 16 + 4 * (lane >> 4);
+                const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
+                f32x4 v = acc[i][j];
+                if constexpr (ROUND)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = (float)(bf16_t)v[r];
+                if constexpr (ACC) {
+                    const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff, i * row_step, 0));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] += old[r];
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, voff, i * row_step, 0);
+            }
+        }
+    }
+}
+
+// as above with the kernel's flags: bit 0 accumulate, kRoundResult (only where the form has it: MAY_ROUND)
+template <int TM, int TN, typename OutT, bool VEC, bool MAY_ROUND>
+__device__ __forceinline__ void store_tile_flags(const f32x4 (&acc)[TM][TN], OutT* C, int64_t ldc, int mrem, int nrem, int row0, int col0,
+                                                 int lane, int flags) {
+    if (flags & 1) store_tile_impl<TM, TN, OutT, true, VEC>(acc, C, ldc, mrem, nrem, row0, col0, lane);
+    else if (MAY_ROUND && (flags & kRoundResult)) store_tile_impl<TM, TN, OutT, false, VEC, true>(acc, C, ldc, mrem, nrem, row0, col0, lane);
+    else store_tile_impl<TM, TN, OutT, false, VEC>(acc, C, ldc, mrem, nrem, row0, col0, lane);
+}
 
 }  // namespace
 
@@ -188,7 +276,7 @@ struct GemmPlan {
     int kind, nsplit;
 };
 // form 0: A, B k-contiguous, bf16 result; 1: A k-contiguous, bf16 result (multi: over K segments); 2 / 3: neither, fp32 / bf16
-// result.  Sets the tile grids in `a` and launches; 256 rows of every problem's C must span less than 2 GiB.
+// result; 4: as 0 with an fp32 result.  Sets the tile grids in `a` and launches; 256 rows of every problem's C must span less than 2 GiB.
 __attribute__((visibility("hidden"))) void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs& a, int count,
                                                              hipStream_t stream);
 inline int64_t gemm_kind_bm(int kind) { return kind <= kTile256x128 ? 256 : (kind == kTile128 ? 128 : 64); }

@@ -60,6 +60,24 @@ def linear(x, weight):
     return LinearFunction.apply(x, weight)
 
 
+class LinearFp32OutputFunction(torch.autograd.Function):
+    """to_fp32(linear(x, weight)) without the bf16 tensor in between: same values, the product's epilogue writes them in fp32."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        y = K.linear_fwd(x.reshape(-1, x.shape[-1]), weight, fp32_output=True)
+        ctx.save_for_backward(x, weight)
+        return y.view(*x.shape[:-1], weight.shape[0])
+
+    @staticmethod
+    def backward(ctx, dy):
+        return LinearFunction.backward(ctx, K.cast_f32_to_bf16(dy.contiguous()))
+
+
+def linear_fp32_output(x, weight):
+    return LinearFp32OutputFunction.apply(x, weight)
+
+
 class FanOutLinearFunction(torch.autograd.Function):
     """One input through several bias-free linears (q/k/v, or gate/up): y_i = x W_i^T.  The input gradient
     sum_i dy_i W_i is one GEMM whose reduction runs over all (dy_i, W_i) pairs (fp32 sum, one rounding) instead of one
@@ -535,4 +553,8 @@ class FusedCrossEntropyLossFunction(torch.autograd.Function):
 
 
 def fused_cross_entropy_loss(logits, labels, loss_mask=None, cut_size=None, ignore_index=-100, inplace=False):
+    if not (torch.is_grad_enabled() and logits.requires_grad):  # nobody will ask for the gradient: the loss alone
+        logits, labels = logits.contiguous(), labels.contiguous()
+        weights, count = K.ce_prepare(labels, None if loss_mask is None else loss_mask.contiguous(), ignore_index)
+        return K.ce_reduce(K.ce_loss(logits, labels, weights, cut_size), weights, count)
     return FusedCrossEntropyLossFunction.apply(logits, labels, loss_mask, cut_size, ignore_index, inplace)

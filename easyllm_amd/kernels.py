@@ -234,8 +234,9 @@ def _rows_ld(t, name):
     return st[0]
 
 
-def gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out=None, out_dtype=BF16, accumulate=False):
-    return _gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out, out_dtype, accumulate)
+def gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out=None, out_dtype=BF16, accumulate=False, rounded=False):
+    """rounded: an fp32 result that holds the bf16-rounded values (forward form, no accumulation)."""
+    return _gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out, out_dtype, accumulate, rounded)
 
 
 def _span(t):
@@ -254,7 +255,7 @@ def _extent_ok(t, rows, cols, ld):
     return ld >= cols and _span(t) >= (rows - 1) * ld + cols
 
 
-def _gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out, out_dtype, accumulate):
+def _gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out, out_dtype, accumulate, rounded=False):
     if out is None:
         _need(not accumulate, "GEMM: accumulate needs the buffer to add to (out=...)")
     for t, name in ((A, "A"), (B, "B")):
@@ -271,7 +272,7 @@ def _gemm(A, B, M, N, K, lda, ldb, a_kc, b_kc, out, out_dtype, accumulate):
     _need(bf16_out or out.dtype is torch.float32, "GEMM output must be bf16 or fp32")
     ws, ws_bytes = _gemm_workspace(M, N, K, A.device)
     _lib.call("ezl_gemm_bf16", A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, lda, ldb, ost[0], 1 if a_kc else 0, 1 if b_kc else 0,
-              0 if bf16_out else 1, 1 if accumulate else 0, _p(ws), ws_bytes, _stream())
+              0 if bf16_out else (2 if rounded else 1), 1 if accumulate else 0, _p(ws), ws_bytes, _stream())
     return out
 
 
@@ -281,10 +282,12 @@ def _gemm_workspace(M, N, K, device):
     return (torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes) if nbytes else (None, 0)
 
 
-def linear_fwd(x2d, w):
-    """y[T, out] = x[T, in] @ w[out, in]^T"""
+def linear_fwd(x2d, w, fp32_output=False):
+    """y[T, out] = x[T, in] @ w[out, in]^T; fp32_output: the bf16 result's values in an fp32 tensor."""
     lda, ldb = _rows_ld(x2d, "x"), _rows_ld(w, "w")
     _need(x2d.shape[1] == w.shape[1], "linear_fwd: inner dimensions differ")
+    if fp32_output:
+        return gemm(x2d, w, x2d.shape[0], w.shape[0], x2d.shape[1], lda, ldb, True, True, out_dtype=torch.float32, rounded=True)
     return gemm(x2d, w, x2d.shape[0], w.shape[0], x2d.shape[1], lda, ldb, True, True)
 
 
@@ -552,6 +555,18 @@ def ce_fused(logits, labels, weights, count, cut_size=0, inplace=True):
     _lib.call("ezl_ce_fused", _p(logits), _p(labels), _p(weights), _p(count), _p(loss_rows), _p(grad), rows, V, cut_size or 0,
               _logits_dtype(logits), _stream())
     return loss_rows, grad
+
+
+def ce_loss(logits, labels, weights, cut_size=0):
+    """-> loss_rows fp32 [rows], as ce_fused gives them"""
+    V = logits.shape[-1]
+    rows = logits.numel() // V
+    _labels(labels, rows)
+    _f32c(weights, "weights")
+    _need(weights.numel() == rows, "one weight per row")
+    loss_rows = torch.empty(rows, dtype=torch.float32, device=logits.device)
+    _lib.call("ezl_ce_loss", _p(logits), _p(labels), _p(weights), _p(loss_rows), rows, V, cut_size or 0, _logits_dtype(logits), _stream())
+    return loss_rows
 
 
 def ce_reduce(loss_rows, weights, count):

@@ -77,6 +77,8 @@ class LlamaModelPipe(torch.nn.Module):
         for idx, spec in enumerate(self.specs):
             if isinstance(spec, LayerSpec):
                 module = spec.build()
+                if self.specs[idx + 1:] == [float16_to_fp32] and isinstance(module, EmbedddingPipeNoTied):
+                    module.fp32_output = True
                 self.add_module(str(idx), module)
                 self.forward_funcs.append(module)
             elif isinstance(spec, torch.nn.Module):

@@ -4,13 +4,16 @@ from . import functional as F_
 from .word_embedings import EmbeddingPipe
 
 
-def parallel_lm_logits(input_, word_embeddings_weight, parallel_output, bias=None, sequence_parallel=False):
+def parallel_lm_logits(input_, word_embeddings_weight, parallel_output, bias=None, sequence_parallel=False, fp32_output=False):
     """logits = input @ W^T with W [V, h]; TP=1 so no gather is needed either way (:68-71)."""
     if sequence_parallel:
         input_parallel = dist_env.gather_from_sequence_parallel_region(input_, tensor_parallel_output_grad=True)
     else:
         input_parallel = dist_env.copy_to_tensor_model_parallel_region(input_)
-    logits_parallel = F_.linear(input_parallel, word_embeddings_weight)
+    if fp32_output and bias is None:
+        logits_parallel = F_.linear_fp32_output(input_parallel, word_embeddings_weight)
+    else:
+        logits_parallel = F_.linear(input_parallel, word_embeddings_weight)
     if bias is not None:
         logits_parallel = F_.bias_add(logits_parallel, bias)
     if parallel_output:
@@ -22,7 +25,10 @@ class EmbedddingPipeNoTied(EmbeddingPipe):
     def __init__(self, *args, parallel_output=True, **kwargs):
         super().__init__(*args, **kwargs)
         self.parallel_output = parallel_output
+        self.fp32_output = False  # set by a model whose next stage is float16_to_fp32: logits in fp32 straight from the product
 
     def forward(self, lm_output, **kwargs):
+        # (a hook on this module sees the bf16 logits that it would without that)
+        fp32_output = self.fp32_output and not (self._forward_hooks or self._backward_hooks or self._backward_pre_hooks)
         return parallel_lm_logits(lm_output, self.word_embeddings_weight, self.parallel_output,
-                                  sequence_parallel=self.sequence_parallel)
+                                  sequence_parallel=self.sequence_parallel, fp32_output=fp32_output)

@@ -105,7 +105,8 @@ int ezl_cast_f32_to_bf16(const void* in, void* out, int64_t n, void* stream);
  *      row_parallel_linear.py:113; llama/lm_head.py:62 ----
  * C[M,N] (=|+=) A * B, bf16 operands, fp32 accumulation.
  *   A: a_kc ? A[m*lda + k] : A[k*lda + m]     B: b_kc ? B[n*ldb + k] : B[k*ldb + n]
- * out_dtype 0 = bf16, 1 = fp32.
+ * out_dtype 0 = bf16, 1 = fp32, 2 = fp32 holding the bf16-rounded values (forward form, accumulate = 0: the logits of
+ * llama/llama.py:187-188 without a separate cast).
  * workspace (optional, may be NULL): ezl_gemm_workspace_bytes(M, N, K) bytes of device memory, 16-byte aligned.  With it, a
  * tile count that leaves the last round of workgroups mostly empty (320 output tiles of 256 x 256 on 256 CUs, or 64 tiles
  * in all) is evened out: the reduction of those last tiles is split over several workgroups whose fp32 partial tiles are
@@ -183,6 +184,8 @@ int ezl_ce_fwd(const void* logits, const void* labels, void* loss, void* lse, in
                int dtype, void* stream);
 int ezl_ce_bwd(const void* logits, const void* labels, const void* lse, const void* grad_out, void* grad, int64_t rows,
                int64_t vocab, int64_t cut_size, int dtype, void* stream);
+int ezl_ce_loss(const void* logits, const void* labels, const void* weights, void* loss_rows, int64_t rows, int64_t vocab,
+                int64_t cut_size, int dtype, void* stream);
 int ezl_ce_fused(const void* logits, const void* labels, const void* weights, const void* count, void* loss_rows, void* grad,
                  int64_t rows, int64_t vocab, int64_t cut_size, int dtype, void* stream);
 int ezl_ce_reduce(const void* loss_rows, const void* weights, const void* count, void* loss_out, int64_t n, void* stream);

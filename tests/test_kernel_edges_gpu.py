@@ -241,3 +241,52 @@ def test_a_hooked_submodule_keeps_the_composed_layer():
     tokens = torch.randint(0, 512, (1, 64)).cuda()
     model((tokens, torch.arange(64).view(1, 64).cuda(), None))
     assert seen == [torch.Size([64, 1, 128])]
+
+
+@pytest.mark.parametrize("M,N,Kd", [(1024, 256, 256), (1167, 50304, 1024), (300, 1003, 72), (4096, 4096, 3136), (64, 72, 2000), (700, 3072, 3072)])
+def test_gemm_forward_with_an_fp32_result_of_bf16_values(K, M, N, Kd):
+    """Bit for bit the cast of the bf16 result: same kernels per shape (or one that adds the K tiles in the same order), same rounding.
+    Where the two fall to different splits of the reduction: one bf16 step."""
+    print("gemm rounded fp32", M, N, Kd, flush=True)
+    x, w = rnd(M, Kd, seed=1), rnd(N, Kd, seed=2)
+    y, f = K.linear_fwd(x, w), K.linear_fwd(x, w, fp32_output=True)
+    assert f.dtype == torch.float32 and torch.equal(f, f.bfloat16().float())
+    assert torch.equal(f, y.float())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,V,cut", [(1, 8, 0), (37, 1000, 0), (5, 16384 + 8, 3), (300, 32000, 0), (9, 152064, 1000), (3, 2048, 2047)])
+def test_loss_without_gradient_equals_the_fused_loss(K, rows, V, cut, dtype):
+    """Same sums in another order: 1e-6 relative; ignored rows contribute exactly nothing, whatever they hold."""
+    print("ce loss", rows, V, cut, dtype, flush=True)
+    logits = (torch.randn(rows, V, device="cuda") * 4).to(dtype)
+    labels = torch.randint(0, V, (rows,), device="cuda")  # (some fall into the cut columns: masked)
+    weights = (torch.rand(rows, device="cuda") < 0.8).float()
+    weights[0] = 1.0
+    logits[weights == 0] = float("nan")
+    count = weights.sum().view(1)
+    want, _ = K.ce_fused(logits.clone(), labels, weights, count, cut, inplace=True)
+    got = K.ce_loss(logits, labels, weights, cut)
+    assert torch.allclose(got, want, rtol=1e-6, atol=2e-6)
+    assert (got[weights == 0] == 0).all()
+
+
+def test_default_fp32_logits_are_the_cast_of_the_bf16_ones():
+    from easyllm_amd import runner
+    kw = dict(num_layers=1, hidden_size=256, num_attention_heads=4, intermediate_size=512, vocab_size=1000, seq_length=64, bf16=True)
+    tokens, pos = torch.randint(0, 1000, (2, 64)).cuda(), torch.arange(64).expand(2, 64).contiguous().cuda()
+    target = (tokens, torch.ones(2, 64, device="cuda"))
+    outs = []
+    for fp32 in (True, False):
+        torch.manual_seed(0)
+        model = runner.build_model({"type": "llama_custom", "kwargs": dict(kw, fp32_logits=fp32)}).cuda()
+        with torch.no_grad():
+            no_grad_loss = model.loss_fn(model((tokens, pos, None)), target)
+        out = model((tokens, pos, None))
+        loss = model.loss_fn(out, target)
+        loss.backward()
+        assert abs(no_grad_loss.item() - loss.item()) <= 1e-6 * loss.item()
+        outs.append((out, {n: p.grad for n, p in model.named_parameters()}))
+    assert outs[0][0].dtype == torch.float32 and torch.equal(outs[0][0], outs[1][0].float())
+    for n in outs[0][1]:  # the logits' gradient is rounded to bf16 once either way, from exponentials of two kernels
+        assert (outs[0][1][n].float() - outs[1][1][n].float()).norm() <= 2e-2 * outs[1][1][n].float().norm(), n
