@@ -709,9 +709,12 @@ def layer_bwd(desc, x, dy, saved, grads):
     _bf16c(x, "x"); _bf16c(dy, "dy")
     _need(dy.shape == x.shape, "layer_bwd: shape mismatch")
     arr = (_lib.LayerGrad * 12)()
-    for slot, g in zip(arr, grads):
+    q, k = (desc.nq * desc.d, desc.nk * desc.d)
+    h, f = desc.h, desc.f
+    for slot, g, n in zip(arr, grads, (h, q * h, k * h, k * h, h * q, h, f * h, f * h, h * f, q, k, k)):
         if g is not None:
             f32, bf16, acc = g
+            _need((bf16 if f32 is None else f32).numel() == n, "layer_bwd: a gradient buffer is not of its parameter's size")
             if f32 is not None:
                 _f32c(f32, "main_grad")
                 slot.f32 = f32.data_ptr()

@@ -18,7 +18,7 @@ from .default_cfg import update_model_cfg
 from .layers import LayerSpec, build_layer_norm
 from .lm_head import EmbedddingPipeNoTied
 from .registry import LOSS_REGISTRY, MODULE_ZOO_REGISTRY
-from .transformer import ParallelTransformerLayerPipe
+from .transformer import ParallelTransformerLayerPipe, is_plain
 from .word_embedings import EmbeddingPipe
 from . import losses as _losses  # noqa: F401  (registers 'softmax_cross_entropy')
 
@@ -77,8 +77,6 @@ class LlamaModelPipe(torch.nn.Module):
         for idx, spec in enumerate(self.specs):
             if isinstance(spec, LayerSpec):
                 module = spec.build()
-                if self.specs[idx + 1:] == [float16_to_fp32] and isinstance(module, EmbedddingPipeNoTied):
-                    module.fp32_output = True
                 self.add_module(str(idx), module)
                 self.forward_funcs.append(module)
             elif isinstance(spec, torch.nn.Module):
@@ -120,8 +118,12 @@ class LlamaModelPipe(torch.nn.Module):
         def exec_range(start, end):
             def run(*inputs):
                 inputs = inputs[0] if len(inputs) == 1 else inputs
-                for f in funcs_all[start:end]:
-                    inputs = f(inputs)
+                for i in range(start, end):
+                    f = funcs_all[i]
+                    if i + 1 < n and funcs_all[i + 1] is float16_to_fp32 and is_plain(f, EmbedddingPipeNoTied):
+                        inputs = f(inputs, fp32_output=True)  # (the cast then has nothing to do)
+                    else:
+                        inputs = f(inputs)
                 return inputs
             return run
 

@@ -25,10 +25,8 @@ class EmbedddingPipeNoTied(EmbeddingPipe):
     def __init__(self, *args, parallel_output=True, **kwargs):
         super().__init__(*args, **kwargs)
         self.parallel_output = parallel_output
-        self.fp32_output = False  # set by a model whose next stage is float16_to_fp32: logits in fp32 straight from the product
 
-    def forward(self, lm_output, **kwargs):
-        # (a hook on this module sees the bf16 logits that it would without that)
-        fp32_output = self.fp32_output and not (self._forward_hooks or self._backward_hooks or self._backward_pre_hooks)
+    def forward(self, lm_output, fp32_output=False, **kwargs):
+        """fp32_output: the bf16 logits' values in fp32, straight from the product."""
         return parallel_lm_logits(lm_output, self.word_embeddings_weight, self.parallel_output,
                                   sequence_parallel=self.sequence_parallel, fp32_output=fp32_output)

@@ -26,6 +26,12 @@ _POSITION_TYPES = ("rotary", "absolute", "alibi", "flash", "dynamicntk")
 _MASK_TYPES = ("causal", "padding", "prefix", "custom")
 
 
+def is_plain(module, cls):
+    """Exactly this class, with no hook or replaced forward that skipping its __call__ would leave out."""
+    return not (type(module) is not cls or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                or module._backward_pre_hooks or "forward" in module.__dict__ or torch.nn.modules.module._has_any_global_hook())
+
+
 class FlashAttention(torch.nn.Module):
     """Causal softmax(q k^T * scale) v over packed documents (the flash_attn_varlen_* seam)."""
 
@@ -163,8 +169,11 @@ class ParallelAttention(torch.nn.Module):
                                                                     self.v_proj.weight)
         elif not self.qkv_pack:
             projections = (self.q_proj, self.k_proj, self.v_proj)
-            query_layer, key_layer, value_layer = (
-                F_.bias_add(y, p.bias) for y, p in zip(F_.fan_out_linear(hidden_states, *(p.weight for p in projections)), projections))
+            if all(is_plain(p, ColumnParallelLinear) for p in projections):  # one launch where that is faster, one input gradient
+                ys = F_.fan_out_linear(hidden_states, *(p.weight for p in projections))
+                query_layer, key_layer, value_layer = (F_.bias_add(y, p.bias) for y, p in zip(ys, projections))
+            else:
+                query_layer, key_layer, value_layer = (p(hidden_states)[0] for p in projections)
         else:
             qkv_layer, _ = self.wqkv(hidden_states)  # q | k | v along the last dim (:427-429)
             query_layer = qkv_layer[..., :self.q_size]
@@ -266,7 +275,7 @@ class ParallelTransformerLayer(torch.nn.Module):
         for m, cls in ((attn, ParallelAttention), (mlp, ParallelMLP), (q, ColumnParallelLinear), (k, ColumnParallelLinear),
                        (v, ColumnParallelLinear), (o, RowParallelLinear), (gate, ColumnParallelLinear), (up, ColumnParallelLinear),
                        (down, RowParallelLinear), (ln1, RMSNorm), (ln2, RMSNorm), (core, FlashAttention), (rotary, RotaryEmbedding)):
-            if type(m) is not cls or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
+            if not is_plain(m, cls):
                 return None
         params = (ln1.weight, q.weight, k.weight, v.weight, o.weight, ln2.weight, gate.weight, up.weight, down.weight)
         if q.bias is not None:
@@ -274,7 +283,10 @@ class ParallelTransformerLayer(torch.nn.Module):
         for p in params:
             if p.dtype is not torch.bfloat16 or not p.is_contiguous() or not p.is_cuda:
                 return None
-        if mlp.activation_func is not GLU_ACTIVATIONS["silu"] or not core.causal or torch.nn.modules.module._has_any_global_hook():
+            mg = getattr(p, "main_grad", None)
+            if mg is not None and not (mg.dtype is torch.float32 and mg.shape == p.shape and mg.is_contiguous()):
+                return None
+        if mlp.activation_func is not GLU_ACTIVATIONS["silu"] or not core.causal:
             return None
         cos, sin = rotary.tables(s, hidden_states.device)
         if cu_seqlens is not None:

@@ -243,6 +243,40 @@ def test_a_hooked_submodule_keeps_the_composed_layer():
     assert seen == [torch.Size([64, 1, 128])]
 
 
+def test_hooks_on_biased_projections_and_on_the_head_run():
+    """They see what the modules return by themselves: q with its bias, logits in bf16."""
+    from easyllm_amd import runner
+    model = runner.build_model({"type": "llama_custom", "kwargs": dict(
+        num_layers=1, hidden_size=128, num_attention_heads=2, intermediate_size=256, vocab_size=512, seq_length=64, bf16=True,
+        transformer_layer_params={"attention_qkv_bias": True})}).cuda()
+    head = model.get_submodule("6")
+    seen = {}
+    tokens = torch.randint(0, 512, (1, 64)).cuda()
+    inputs = (tokens, torch.arange(64).view(1, 64).cuda(), None)
+    plain = model(inputs)
+    hooks = [model.get_submodule("3").self_attn.q_proj.register_forward_hook(lambda m, i, o: seen.update(q=o[0].shape)),
+             head.register_forward_hook(lambda m, i, o: seen.update(logits=o))]
+    hooked = model(inputs)
+    assert seen["q"] == torch.Size([64, 1, 128]) and seen["logits"].dtype == torch.bfloat16
+    assert plain.dtype == hooked.dtype == torch.float32 and torch.equal(hooked, seen["logits"].float()) and torch.equal(hooked, plain)
+    for hook in hooks:
+        hook.remove()
+    assert head(rnd(1, 64, 128)).dtype == torch.bfloat16
+
+
+def test_gradient_buffers_of_another_size_are_refused():
+    from easyllm_amd import runner
+    model = runner.build_model({"type": "llama_custom", "kwargs": dict(num_layers=1, hidden_size=128, num_attention_heads=2, intermediate_size=256,
+                                                                       vocab_size=512, seq_length=64, bf16=True,
+                                                                       checkpoint_activations=False)}).cuda()
+    tokens = torch.randint(0, 512, (1, 64)).cuda()
+    out = model((tokens, torch.arange(64).view(1, 64).cuda(), None))
+    runner.attach_main_grads(model)
+    model.get_submodule("3").mlp.up_proj.weight.main_grad = torch.zeros(255, 128, device="cuda")
+    with pytest.raises(ValueError, match="gradient buffer"):
+        out.sum().backward()
+
+
 @pytest.mark.parametrize("M,N,Kd", [(1024, 256, 256), (1167, 50304, 1024), (300, 1003, 72), (4096, 4096, 3136), (64, 72, 2000), (700, 3072, 3072)])
 def test_gemm_forward_with_an_fp32_result_of_bf16_values(K, M, N, Kd):
     """Bit for bit the cast of the bf16 result: same kernels per shape (or one that adds the K tiles in the same order), same rounding.
