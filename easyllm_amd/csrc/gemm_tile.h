@@ -165,6 +165,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // straight-line (a branch per store instead: 4000 x 32000 x 2048 with an fp32 result 632 us against 482; a weight gradient of
 // 32000 x 4096 over 1531 tokens 420 against 405).  bf16: lanes l and l ^ 16 trade halves of two neighbouring column tiles, 16-byte stores.  VEC = false (rows
 // that do not start on 16 bytes, or a width that is no multiple of 8): one element per store.
+// The row step is part of the vector offset: with a scalar offset register the compiler leaves no wait state between a 16-byte
+// buffer store and the next write of its data registers, and the hardware needs one (seen as lanes 12 - 15 of a row group holding
+// the next value's bits where such a write came right behind).
 template <int TM, int TN, typename OutT, bool ACC, bool VEC, bool ROUND = false>
 __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT* C, int64_t ldc, int mrem, int nrem, int row0, int col0,
                                                 int lane) {
@@ -186,11 +189,11 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
                     float v = acc[i][j][r];
                     if constexpr (ROUND) v = (float)(bf16_t)v;
                     if constexpr (SZ == 2) {
-                        if constexpr (ACC) v += (float)__builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(cbuf, voff, i * row_step, 0));
-                        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (bf16_t)v), cbuf, voff, i * row_step, 0);
+                        if constexpr (ACC) v += (float)__builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(cbuf, voff + i * row_step, 0, 0));
+                        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (bf16_t)v), cbuf, voff + i * row_step, 0, 0);
                     } else {
-                        if constexpr (ACC) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(cbuf, voff, i * row_step, 0));
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), cbuf, voff, i * row_step, 0);
+                        if constexpr (ACC) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(cbuf, voff + i * row_step, 0, 0));
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), cbuf, voff + i * row_step, 0, 0);
                     }
                 }
     } else if constexpr (SZ == 2) {
@@ -210,11 +213,11 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
                     v[4 + r] = __uint_as_float(sw[1]);
                 }
                 if constexpr (ACC) {
-                    const bf16x8 old = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff, i * row_step, 0));
+                    const bf16x8 old = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff + i * row_step, 0, 0));
 #pragma unroll
                     for (int r = 0; r < 8; ++r) v[r] += (float)old[r];
                 }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, voff, i * row_step, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, voff + i * row_step, 0, 0);
             }
         }
     } else {
@@ -229,11 +232,11 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] = (float)(bf16_t)v[r];
                 if constexpr (ACC) {
-                    const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff, i * row_step, 0));
+                    const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff + i * row_step, 0, 0));
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] += old[r];
                 }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, voff, i * row_step, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, voff + i * row_step, 0, 0);
             }
         }
     }
