@@ -15,8 +15,7 @@
 // bank conflicts are avoided by an XOR swizzle applied on the global-address side.  In the 8-wave kernel a K tile is consumed
 // in four phases (k half x M half) of 16 MFMAs; the fragments of the next phase are read during the current one, the barrier
 // that publishes the next stage sits in front of the last phase, and the loads of tile kt+2 are issued under that phase's
-// MFMAs.  The forward form and the fp32 weight-gradient form on long reductions run a 4-wave variant (128x128 wave tiles,
-// one wave per SIMD).
+// MFMAs.  Long reductions run a 4-wave variant (128x128 wave tiles, one wave per SIMD; see w4_pays).
 // K tails (K % 64 != 0: a weight gradient over an odd number of tokens, a forward over a width like 688): the lanes of the
 // last K tile's loads that lie past K get an offset outside the buffer, which reads as zero; nothing else differs.  (A register-
 // staged kernel used to cover them, without split last rounds and without the one-launch input gradient: a training step over
@@ -262,98 +261,112 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // the CU's address unit takes 16 cycles per 1 KiB wave load, i.e. the four waves' loads keep it busy for all of phase B,
 // and issued any faster they fill its queue and the issuing wave stalls with its MFMAs behind it (measured on all-zero
 // operands, 4096 x 4096 x K: 0.96 us per K tile with this spacing, 1.12 with one load every second MFMA, 1.23 back to
-// back; the 8-wave kernel 1.05).  Used for the forward form (both operands k-contiguous, bf16 result) and for the
-// weight-gradient form with an fp32 result on long reductions; for input gradients and short reductions the 8-wave
-// kernel, which hides more of the prologue and the epilogue, is as fast or faster.
-// C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base) and, for bf16, its
-// tile-relative byte offsets must fit 31 bits: the host side checks.
-template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
+// back; the 8-wave kernel 1.05).
+// A workgroup works off items blockIdx.x, + gridDim.x, ... as one stream of K tiles: the last two K tiles of an item bring in the
+// first two of the next, and the finished accumulators are stored while those are on their way (their wait is a count that
+// leaves the stores in flight).  With one workgroup per tile a tile cost 14 us on top of its K tiles - a workgroup's start, the first
+// loads, the stores drained before its LDS is free - which is a third of it at 32 K tiles: 4000 x 32000 x 2048 444 -> 407 us,
+// 8192 x 32000 x 1024 517 -> 460, 4096 x 11008 x 2048 143 -> 134, 8192 x 32000 x 5120 1974 -> 1947; the weight gradient 32000 x 4096 x
+// 4096 911 -> 885.  What is left there is the power limit: longer K loops run at 1.2 - 1.35 us per K tile instead of 0.96.
+// C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base), its tile-relative byte offsets
+// must fit 31 bits, and every item must have two K tiles or more: the host side checks.
+template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                          int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
-                                                         int tiles_m, int tiles_n, const SplitPlan plan) {
+                                                         int tiles_m, int tiles_n, int items, const SplitPlan plan, const KSegments seg) {
     __shared__ __attribute__((aligned(1024))) bf16_t smem[4 * DTILE];  // A0 B0 A1 B1
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-
-    int pid = blockIdx.x, part = 0;
-    const bool split = pid >= plan.full;
-    if (!split) {  // XCD-aware renumbering over the whole-tile workgroups
-        const int per = plan.full >> 3, rem = plan.full & 7, xcd = pid & 7, idx = pid >> 3;
-        pid = xcd * per + (xcd < rem ? xcd : rem) + idx;
-    } else {  // a tile of the split last round: this workgroup's share of its K tiles
-        const int u = pid - plan.full;
-        pid = plan.full + u / plan.nsplit;
-        part = u - (pid - plan.full) * plan.nsplit;
-    }
-    int tm, tn;
-    tile_of(pid, tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
-
-    TileLoader<A_KC, BM, 4, KTAIL> la;
-    TileLoader<B_KC, BN, 4, KTAIL> lb;
-    const int64_t a_blk = A_KC ? (int64_t)m0 * lda : (int64_t)m0;
-    const int64_t b_blk = B_KC ? (int64_t)n0 * ldb : (int64_t)n0;
-    la.init(lane, wave, M - m0, lda);
-    lb.init(lane, wave, N - n0, ldb);
-
-    f32x4 acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
-
-    int nk = (K + BK - 1) / BK, kt0 = 0;  // this workgroup's K tiles: kt0 .. kt0 + nk - 1
-    if (split) {
-        kt0 = (int)((int64_t)nk * part / plan.nsplit);
-        nk = (int)((int64_t)nk * (part + 1) / plan.nsplit) - kt0;
-    }
+    const int nk_all = MULTI ? seg.nk : (K + BK - 1) / BK;
     const int64_t astep = A_KC ? BK : (int64_t)BK * lda;
     const int64_t bstep = B_KC ? BK : (int64_t)BK * ldb;
     const int arow = wm * 128, brow = wn * 128;
 
+    struct Item {  // a whole tile, or a tile of the split last round with this workgroup's share of its K tiles
+        int m0, n0, kt0, nk;
+        int slot;  // >= 0: place of the partial tile
+        int64_t a_blk, b_blk;
+    };
+    auto item_of = [&](int u) {
+        Item it;
+        it.kt0 = 0; it.nk = nk_all; it.slot = -1;
+        int pid = u;
+        if (u < plan.full) {  // XCD-aware renumbering over the whole tiles (a grid smaller than the items is a multiple of 8)
+            const int per = plan.full >> 3, rem = plan.full & 7, xcd = u & 7, idx = u >> 3;
+            pid = xcd * per + (xcd < rem ? xcd : rem) + idx;
+        } else {
+            it.slot = u - plan.full;
+            const int t = it.slot / plan.nsplit, part = it.slot - t * plan.nsplit;
+            pid = plan.full + t;
+            it.kt0 = (int)((int64_t)nk_all * part / plan.nsplit);
+            it.nk = (int)((int64_t)nk_all * (part + 1) / plan.nsplit) - it.kt0;
+        }
+        int tm, tn;
+        tile_of(pid, tiles_m, tiles_n, tm, tn);
+        // (scalar registers: the buffer bases are made of them)
+        it.m0 = __builtin_amdgcn_readfirstlane(tm * BM);
+        it.n0 = __builtin_amdgcn_readfirstlane(tn * BN);
+        it.kt0 = __builtin_amdgcn_readfirstlane(it.kt0);
+        it.nk = __builtin_amdgcn_readfirstlane(it.nk);
+        it.slot = __builtin_amdgcn_readfirstlane(it.slot);
+        it.a_blk = A_KC ? (int64_t)it.m0 * lda : (int64_t)it.m0;
+        it.b_blk = B_KC ? (int64_t)it.n0 * ldb : (int64_t)it.n0;
+        return it;
+    };
+    int u = blockIdx.x;
+    Item it = item_of(u);
+
+    TileLoader<A_KC, BM, 4, KTAIL> la;
+    TileLoader<B_KC, BN, 4, KTAIL> lb;
+    la.init(lane, wave, M - it.m0, lda);
+    lb.init(lane, wave, N - it.n0, ldb);
+
+    FragReader<A_KC> ra;
+    FragReader<B_KC> rb;
+    ra.init(arow, lane);
+    rb.init(brow, lane);
+
+    f32x4 acc[8][8];
     bf16x8 fa[2][8], fb[2][8];
     // fragment f of a k half: f < 8 the B fragment f, else the A fragment f - 8
     auto read_frag = [&](const bf16_t* sA, int ks, int buf, auto F) {
         constexpr int f = decltype(F)::value;
-        if constexpr (f < 8) fb[buf][f] = sfrag<B_KC, 256>(sA + DTILE, brow + f * 16, ks, lane);
-        else fa[buf][f - 8] = sfrag<A_KC, 256>(sA, arow + (f - 8) * 16, ks, lane);
+        if constexpr (f < 8) fb[buf][f] = rb.template read<f>(sA + DTILE, ks);
+        else fa[buf][f - 8] = ra.template read<f - 8>(sA, ks);
     };
     __amdgpu_buffer_rsrc_t ga, gb;
     int kv = BK;
-    auto tile_bases = [&](int t) {
-        t += kt0;
-        kv = K - t * BK;
-        ga = la.base(A + a_blk + (int64_t)t * astep);
-        gb = lb.base(B + b_blk + (int64_t)t * bstep);
+    auto tile_bases = [&](const Item& x, int t) {
+        const bf16_t *Ab, *Bb;
+        t += x.kt0;
+        pick_segment<MULTI>(A, B, K, seg, t, kv, Ab, Bb);
+        ga = la.base(Ab + x.a_blk + (int64_t)t * astep);
+        gb = lb.base(Bb + x.b_blk + (int64_t)t * bstep);
     };
     // load l of a tile pair: l < 8 piece l of the A tile, else piece l - 8 of the B tile
-    auto issue_load = [&](int stage, auto L) {
+    auto issue_load = [&](bf16_t* st, auto L) {
         constexpr int l = decltype(L)::value;
-        if constexpr (l < 8) la.template issue_at<l>(ga, smem + stage * 2 * DTILE, lane, wave, kv);
-        else lb.template issue_at<l - 8>(gb, smem + stage * 2 * DTILE + DTILE, lane, wave, kv);
-    };
-    auto issue_tile = [&](int t, int stage) {
-        tile_bases(t);
-        static_for<0, 16>([&](auto L) { issue_load(stage, L); });
+        if constexpr (l < 8) la.template issue_at<l>(ga, st, lane, wave, kv);
+        else lb.template issue_at<l - 8>(gb, st + DTILE, lane, wave, kv);
     };
 
-    issue_tile(0, 0);
-    if (nk > 1) issue_tile(1, 1);
+    tile_bases(it, 0);
+    static_for<0, 16>([&](auto L) { issue_load(smem, L); });
+    tile_bases(it, 1);
+    static_for<0, 16>([&](auto L) { issue_load(smem + 2 * DTILE, L); });
     // the remaining kernel arguments, pulled into registers now (a scalar load in flight inside the K loop would share the
     // counter of the LDS reads)
-    asm volatile("" ::"s"(C), "s"(ldc), "s"(accumulate), "s"(plan.partial), "s"(plan.full), "s"(plan.nsplit));
-    if (nk > 1) __builtin_amdgcn_s_waitcnt(0x4070);  // vmcnt(16) lgkmcnt(0): tile 0 has landed, tile 1 is still on its way
-    else __builtin_amdgcn_s_waitcnt(0x0070);         // vmcnt(0) lgkmcnt(0)
+    asm volatile("" ::"s"(C), "s"(ldc), "s"(accumulate), "s"(plan.partial), "s"(plan.full), "s"(plan.nsplit), "s"(items), "s"(M), "s"(N),
+                 "s"(tiles_m), "s"(tiles_n));
+    if constexpr (MULTI) asm volatile("" ::"s"(seg.A1), "s"(seg.B1), "s"(seg.A2), "s"(seg.B2), "s"(seg.t1), "s"(seg.t2), "s"(seg.K1), "s"(seg.K2));
+    __builtin_amdgcn_s_waitcnt(0x4070);  // vmcnt(16) lgkmcnt(0): K tile 0 has landed, K tile 1 is still on its way
     __syncthreads();
     static_for<0, 16>([&](auto F) { read_frag(smem, 0, 0, F); });
 
     constexpr int RSTEP = 2;  // a fragment read every RSTEP MFMAs (16 reads: the first half of a phase)
     constexpr int LSTEP = 4;  // a tile load every LSTEP MFMAs (16 loads: all of phase B)
-    auto phase_a = [&](int kt) {
-        const bf16_t* sA = smem + (kt & 1) * 2 * DTILE;
+    auto phase_a = [&](const bf16_t* sA) {
         static_for<0, 64>([&](auto S) {
             constexpr int m = decltype(S)::value, i = m >> 3, j = m & 7;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0][i], acc[i][j], 0, 0, 0);
@@ -361,58 +374,83 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-    auto phase_b = [&](int kt, auto HAS_NEXT, auto DO_LOAD) {
-        constexpr bool has_next = decltype(HAS_NEXT)::value, do_load = decltype(DO_LOAD)::value;
-        const int cur = kt & 1;
-        const bf16_t* sN = smem + (cur ^ 1) * 2 * DTILE;
-        if constexpr (do_load) tile_bases(kt + 2);
+    auto phase_b = [&](const bf16_t* sN, bf16_t* sL) {
         static_for<0, 64>([&](auto S) {
             constexpr int m = decltype(S)::value, i = m >> 3, j = m & 7;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[1][i], acc[i][j], 0, 0, 0);
-            if constexpr (has_next && m % RSTEP == 0 && m / RSTEP < 16) read_frag(sN, 0, 0, std::integral_constant<int, m / RSTEP>{});
-            if constexpr (do_load && m % LSTEP == LSTEP - 1) issue_load(cur, std::integral_constant<int, m / LSTEP>{});
+            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sN, 0, 0, std::integral_constant<int, m / RSTEP>{});
+            if constexpr (m % LSTEP == LSTEP - 1) issue_load(sL, std::integral_constant<int, m / LSTEP>{});
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-    auto publish = [&]() {
-        __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): the next tile has landed, this wave's reads are done
+    auto publish = [&](auto LEFT) {  // all but this wave's LEFT newest accesses are done: the next K tile has landed; so are its LDS reads
+        constexpr int left = decltype(LEFT)::value;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (left & 15) | ((left >> 4) << 14));
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
     };
-    phase_a(0);
-    publish();
-    int kt = 0;
-    for (; kt + 2 < nk; ++kt) {
-        phase_b(kt, std::true_type{}, std::true_type{});
-        phase_a(kt + 1);
-        publish();
-    }
-    if (kt + 1 < nk) {
-        phase_b(kt, std::true_type{}, std::false_type{});
-        phase_a(kt + 1);
-        publish();
-        ++kt;
-    }
-    phase_b(kt, std::false_type{}, std::false_type{});
-
-    if (split) {  // this workgroup's share of the reduction, as a dense fp32 tile; gemm_split_reduce_kernel adds the shares
-        float* tile = plan.partial + ((size_t)(pid - plan.full) * plan.nsplit + part) * (size_t)(BM * BN);
+    // stores of a finished tile that are newer than the loads of the next tile's second K tile (a count holds at most 63)
+    constexpr int STORES = sizeof(OutT) == 2 ? 32 : 63;
+    typedef std::integral_constant<int, 0> none;
+    int s0 = 0, s1 = 2 * DTILE;  // stages of K tiles kt and kt + 1
+    auto flip = [&]() {
+        const int x = s0;
+        s0 = s1;
+        s1 = x;
+        asm volatile("" : "+s"(s0), "+s"(s1));  // (the fragment reads are restrict-qualified: a refilled stage must not look like the same address)
+    };
+    for (bool first = true;; first = false) {
+        const int next_u = u + (int)gridDim.x;
+        const bool more = next_u < items;
+        const Item next = more ? item_of(next_u) : it;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                *reinterpret_cast<f32x4*>(tile + (arow + i * 16 + (lane & 15)) * BN + brow + j * 16 + 4 * (lane >> 4)) = acc[i][j];
-        return;
+            for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        phase_a(smem + s0);
+        if (first) publish(none{});
+        else publish(std::integral_constant<int, STORES>{});
+        for (int kt = 2; kt < it.nk; ++kt) {
+            tile_bases(it, kt);
+            phase_b(smem + s1, smem + s0);
+            phase_a(smem + s1);
+            publish(none{});
+            flip();
+        }
+        // the last two K tiles bring in the first two of the next tile (the last item's: its own again, into stages nobody reads)
+        if (min(M - next.m0, BM) != min(M - it.m0, BM)) la.init(lane, wave, M - next.m0, lda);
+        if (min(N - next.n0, BN) != min(N - it.n0, BN)) lb.init(lane, wave, N - next.n0, ldb);
+        tile_bases(next, 0);
+        phase_b(smem + s1, smem + s0);
+        phase_a(smem + s1);
+        publish(none{});
+        flip();
+        tile_bases(next, 1);
+        phase_b(smem + s1, smem + s0);
+        flip();
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
+        int64_t ld = ldc;
+        asm volatile("" : "+s"(ld));  // (the stores' offsets are not kept over the K loop)
+        if (it.slot >= 0) {  // a share of the reduction, as a dense fp32 tile; gemm_split_reduce_kernel adds the shares
+            float* tile = plan.partial + (size_t)it.slot * (size_t)(BM * BN);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    *reinterpret_cast<f32x4*>(tile + (arow + i * 16 + (lane & 15)) * BN + brow + j * 16 + 4 * (lane >> 4)) = from_agprs<64>(acc[i][j]);
+        } else {
+            const int mrem = M - it.m0 < BM ? M - it.m0 : BM;
+            OutT* Ct = C + (int64_t)it.m0 * ld + it.n0;
+            store_tile_flags<8, 8, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ld, mrem, N - it.n0, arow, brow, lane, accumulate);
+        }
+        if (!more) break;
+        it = next;
+        u = next_u;
     }
-    // the accumulators stay in their AGPRs until here (otherwise the last phase copies each finished tile out to VGPRs
-    // right behind its MFMA and runs out of registers)
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
-    const int mrem = M - m0 < BM ? M - m0 : BM;
-    OutT* Ct = C + (int64_t)m0 * ldc + n0;
-    store_tile_flags<8, 8, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ldc, mrem, N - n0, arow, brow, lane, accumulate);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the last item's loads of a next tile (its own again) may not outlive the workgroup's LDS
 }
 
 // C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order.  One block per 16 rows of a tile: a thread owns 16
@@ -624,9 +662,37 @@ int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     return q.kind == kTile256 ? big : (big > small ? big : small);
 }
 
-// the 4-wave kernel pays off from this many K tiles on (4096 x 4096 x K, forward form: 57 against 54 us at 32 tiles, 98
-// against 103 at 64, 179 against 194 at 128)
-constexpr int kW4MinKTiles = 48;
+// Which 256 x 256 kernel: the 4-wave one moves a third fewer LDS bytes (the chip is bound by power on long products) and, with
+// one workgroup per CU walking over several tiles, hides a tile's first loads and its stores; the 8-wave one hides more inside a
+// single tile.  Speed of the 4-wave kernel over the 8-wave one, M x N x K:
+//   forward            one tile per CU: 4096 x 4096 x 2048 (32 K tiles) 0.95, x 4096 1.05, x 8192 1.08
+//                      several: 8192 x 32000 x 1024 (16) 1.12, 8192 x 8192 x 1536 1.10, 4000 x 32000 x 2048 1.09
+//   weight gradient    11008 x 4096 x 1024 (16) 1.08, 32000 x 4096 x 1024 1.13, 13824 x 5120 x 2048 1.04, but with the rows of B 16 KiB
+//                      (or a multiple) apart 32000 x 8192 x 1536 0.94, 28672 x 8192 x 1536 0.96
+//   input gradient     4096 x 8192 x 8192 (128) 1.01, 4096 x 28672 x 8192 0.97, 8192 x 13824 x 5120 0.95; 4096 x 4096 x 11008 (172) 1.02,
+//                      4096 x 8192 x 28672 1.04, 16384 x 4096 x 32000 1.03
+//   ... over segments  4096 x 4096 x 2 * 11008 (344) 0.97, 16384 x 4096 x 2 * 4096 0.95; 4096 x 8192 x 2 * 20480 (640) 1.03, x 2 * 28672 1.04
+// items: workgroup-sized pieces of the launch; nk: K tiles of a piece
+enum class Form { forward, weight_gradient, input_gradient, input_gradient_segments };
+bool w4_pays(Form form, int64_t nk, int64_t items, int64_t ldb) {
+    switch (form) {
+        case Form::forward: return nk >= 48 || (nk >= 16 && items > kCus);
+        case Form::weight_gradient: return nk >= 48 || (nk >= 16 && items > kCus && ldb % 8192 != 0);
+        case Form::input_gradient: return nk >= 160;
+        default: return nk >= 512;
+    }
+}
+// Workgroups of a 4-wave launch: one per CU, each walking over its tiles, while the K loop is short against a tile's ends; one per
+// tile on longer ones and over many rounds, where the hardware's order of dispatch keeps the workgroups that share operands together
+// (as weight gradients, one per tile against one per CU: 32000 x 5120 x 8192, 128 K tiles, 2164 us against 2314; 11008 x 4096 x
+// 4096, 64 K tiles, 291 against 283).
+dim3 w4_grid(int64_t nk, int64_t items) { return dim3((unsigned)(nk <= 64 && items > kCus && items <= 16 * kCus ? kCus : items)); }
+// its stores: 16 bytes each, at 31-bit byte offsets inside a tile
+template <typename OutT>
+bool w4_stores_ok(const void* C, int64_t N, int64_t ldc) {
+    const int vec = 16 / (int)sizeof(OutT);
+    return N % vec == 0 && ldc % vec == 0 && ezl_aligned16(C) && ldc * (int64_t)sizeof(OutT) * BM < (1LL << 31);
+}
 
 template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
 void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
@@ -634,24 +700,20 @@ void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, nk = (K + BK - 1) / BK;
     const SplitPlan plan = make_plan((int64_t)tiles_m * tiles_n, nk, workspace, workspace_bytes);
     const int split_tiles = tiles_m * tiles_n - plan.full;
-    const dim3 grid((unsigned)(plan.full + split_tiles * plan.nsplit));
+    const int items = plan.full + split_tiles * plan.nsplit;
     bool w4 = false;
-    // The 4-wave kernel: forward form with a bf16 result, and weight-gradient form with an fp32 result (inside the steps
-    // 0.4 - 0.8 % faster than the 8-wave kernel although a single launch at K = 4096 is not: it moves a third fewer LDS
-    // bytes, and the steps are bound by power).  With a k-strided B only (input gradients) it gained nothing.
-    if constexpr ((A_KC && B_KC) || (!A_KC && !B_KC && sizeof(OutT) == 4)) {
-        const int vec = 16 / (int)sizeof(OutT);
+    // (bf16 weight gradients and fp32 input gradients stay with the 8-wave kernel)
+    if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC && sizeof(OutT) == 4) {
+        constexpr Form form = !A_KC ? Form::weight_gradient : (B_KC ? Form::forward : Form::input_gradient);
         // (a launch that is split tiles only is judged by the length of a share)
-        const int w4_ktiles = plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk;
-        w4 = w4_ktiles >= kW4MinKTiles && N % vec == 0 && ldc % vec == 0 && ezl_aligned16(C) &&
-             (int64_t)ldc * (int64_t)sizeof(OutT) * BM < (1LL << 31);  // tile-relative byte offsets of C fit 31 bits
+        w4 = w4_pays(form, plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk, items, ldb) && w4_stores_ok<OutT>(C, N, ldc);
         if (w4)
-            hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, KTAIL>), grid, dim3(256), 0, st, (const bf16_t*)A, (const bf16_t*)B, (OutT*)C,
-                               M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan);
+            hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, false, KTAIL>), w4_grid(nk, items), dim3(256), 0, st, (const bf16_t*)A,
+                               (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, items, plan, KSegments());
     }
     if (!w4)
-        hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, false, KTAIL>), grid, dim3(512), 0, st, (const bf16_t*)A, (const bf16_t*)B,
-                           (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan, KSegments());
+        hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, false, KTAIL>), dim3((unsigned)items), dim3(512), 0, st, (const bf16_t*)A,
+                           (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan, KSegments());
     if (plan.nsplit > 1)
         hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, st, (OutT*)C, M, N, ldc,
                            accumulate, tiles_m, tiles_n, plan);
@@ -820,10 +882,20 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     }
     const SplitPlan plan = make_plan(tiles, (ktot + BK - 1) / BK, workspace, workspace_bytes);
     const int split_tiles = (int)tiles - plan.full;
-#define EZL_MULTI(KT)                                                                                                                      \
-    hipLaunchKernelGGL((gemm_d2l_kernel<true, false, bf16_t, true, KT>), dim3((unsigned)(plan.full + split_tiles * plan.nsplit)), dim3(512), 0, \
-                       (hipStream_t)stream, (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc,     \
-                       accumulate, tiles_m, tiles_n, plan, seg)
+    const int items = plan.full + split_tiles * plan.nsplit;
+    const int share = plan.nsplit > 1 && plan.full == 0 ? seg.nk / plan.nsplit : seg.nk;
+    const bool w4 = w4_pays(Form::input_gradient_segments, share, items, ldb) && w4_stores_ok<bf16_t>(C, N, ldc);
+#define EZL_MULTI(KT)                                                                                                                        \
+    do {                                                                                                                                     \
+        if (w4)                                                                                                                              \
+            hipLaunchKernelGGL((gemm_w4_kernel<true, false, bf16_t, true, KT>), w4_grid(seg.nk, items), dim3(256), 0, (hipStream_t)stream,    \
+                               (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate,    \
+                               tiles_m, tiles_n, items, plan, seg);                                                                          \
+        else                                                                                                                                 \
+            hipLaunchKernelGGL((gemm_d2l_kernel<true, false, bf16_t, true, KT>), dim3((unsigned)items), dim3(512), 0, (hipStream_t)stream,   \
+                               (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate,    \
+                               tiles_m, tiles_n, plan, seg);                                                                                 \
+    } while (0)
     if (tail) EZL_MULTI(true);
     else EZL_MULTI(false);
 #undef EZL_MULTI

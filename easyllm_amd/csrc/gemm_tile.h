@@ -135,6 +135,45 @@ __device__ __forceinline__ bf16x8 sfrag(const bf16_t* __restrict__ s, int row0, 
     }
 }
 
+// The eight fragments of a wave's 128 rows (columns) in a 256-wide tile.  What a fragment's address is made of per lane is computed once and hidden
+// from the compiler, which otherwise rebuilds it per read in a loop over stages (48 vector instructions per K tile of the 4-wave
+// kernel, 5 % of its time); the rest is the read's immediate offset.
+template <bool KC>
+struct FragReader {
+    static constexpr int R = 256;
+    int off[KC ? 2 : 8];  // elements: k-contiguous per k half, k-major per fragment (its chunk permutation mixes with the fragment's index)
+    __device__ __forceinline__ void init(int row0, int lane) {
+        if constexpr (KC) {
+            const int row = row0 + (lane & 15);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) off[ks] = row * 64 + (((ks * 4 + (lane >> 4)) ^ ((row >> 1) & 7)) * 8);
+        } else {
+            const int krow = (lane >> 4) * 8 + ((lane & 15) >> 2);
+#pragma unroll
+            for (int f = 0; f < 8; ++f) {
+                const int col = row0 + f * 16 + ((lane & 3) << 2);
+                off[f] = krow * R + ((col >> 3) ^ kmajor_swizzle<R>(krow)) * 8 + (col & 7);
+            }
+        }
+#pragma unroll
+        for (int& o : off) asm volatile("" : "+v"(o));
+    }
+    template <int F>
+    __device__ __forceinline__ bf16x8 read(const bf16_t* __restrict__ s, int ks) const {
+        if constexpr (KC) {
+            return *reinterpret_cast<const bf16x8*>(s + off[ks] + F * 16 * 64);
+        } else {
+            const bf16_t* p = s + off[F] + ks * 32 * R;
+            const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
+            const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * R));
+            bf16x8 v;
+            v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
+            v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
+            return v;
+        }
+    }
+};
+
 // the (A, B) pair of K tile t, the tile's index inside it and how many of its 64 k exist: scalar selects
 template <bool MULTI>
 __device__ __forceinline__ void pick_segment(const bf16_t* A, const bf16_t* B, int K, const KSegments& seg, int& t, int& kv,
@@ -159,12 +198,21 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// Tiles of 64 accumulators are the 4-wave kernel's, which take all AGPRs: they are copied out here, row by row (with a
+// scheduling barrier behind each).  Copied any earlier, behind their MFMA or all of them before the first store, they spill.
+template <int ACCUMULATORS>
+__device__ __forceinline__ f32x4 from_agprs(f32x4 x) {
+    if constexpr (ACCUMULATORS >= 64) asm volatile("" : "+a"(x));
+    return x;
+}
+
 // acc[i][j] register r is C[m0 + row0 + 16 i + (lane & 15)][n0 + col0 + 16 j + 4 (lane >> 4) + r].
 // C is addressed as a buffer that starts at the tile's corner and ends behind the last valid element of its last valid row: a
 // store past either edge drops out by the range check (for columns: an offset that is out of range), so the code is
 // straight-line (a branch per store instead: 4000 x 32000 x 2048 with an fp32 result 632 us against 482; a weight gradient of
 // 32000 x 4096 over 1531 tokens 420 against 405).  bf16: lanes l and l ^ 16 trade halves of two neighbouring column tiles, 16-byte stores.  VEC = false (rows
 // that do not start on 16 bytes, or a width that is no multiple of 8): one element per store.
+// A row's old values (ACC) are fetched in front of the stores of the row before it: an access waits for all older ones.
 // The row step is part of the vector offset: with a scalar offset register the compiler leaves no wait state between a 16-byte
 // buffer store and the next write of its data registers, and the hardware needs one (seen as lanes 12 - 15 of a row group holding
 // the next value's bits where such a write came right behind).
@@ -198,46 +246,68 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
                 }
     } else if constexpr (SZ == 2) {
         const int g = lane >> 4;
+        const auto offset = [&](int jp) {
+            const int col = col0 + (2 * jp + (g & 1)) * 16 + 8 * (g >> 1);
+            return col < nrem ? row_off + (uint32_t)col * SZ : kOut;
+        };
+        u32x4 old[2][TN / 2];
+        const auto fetch = [&](int i) {
+#pragma unroll
+            for (int jp = 0; jp < TN / 2; ++jp) old[i & 1][jp] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, offset(jp) + i * row_step, 0, 0));
+        };
+        if constexpr (ACC) fetch(0);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
+            if constexpr (ACC)
+                if (i + 1 < TM) fetch(i + 1);
 #pragma unroll
             for (int jp = 0; jp < TN / 2; ++jp) {
-                const int col = col0 + (2 * jp + (g & 1)) * 16 + 8 * (g >> 1);
-                const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
+                const f32x4 va = from_agprs<TM * TN>(acc[i][2 * jp]), vb = from_agprs<TM * TN>(acc[i][2 * jp + 1]);
                 float v[8];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float ta = acc[i][2 * jp][r], tb = acc[i][2 * jp + 1][r];
-                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(ta), __float_as_uint(tb), false, false);
+                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(va[r]), __float_as_uint(vb[r]), false, false);
                     v[r] = __uint_as_float(sw[0]);
                     v[4 + r] = __uint_as_float(sw[1]);
                 }
                 if constexpr (ACC) {
-                    const bf16x8 old = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff + i * row_step, 0, 0));
+                    const bf16x8 o = __builtin_bit_cast(bf16x8, old[i & 1][jp]);
 #pragma unroll
-                    for (int r = 0; r < 8; ++r) v[r] += (float)old[r];
+                    for (int r = 0; r < 8; ++r) v[r] += (float)o[r];
                 }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, voff + i * row_step, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, offset(jp) + i * row_step, 0, 0);
             }
+            if constexpr (TM * TN >= 64) __builtin_amdgcn_sched_barrier(0);
         }
     } else {
+        const auto offset = [&](int j) {
+            const int col = col0 + j * 16 + 4 * (lane >> 4);
+            return col < nrem ? row_off + (uint32_t)col * SZ : kOut;
+        };
+        u32x4 old[2][TN];
+        const auto fetch = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) old[i & 1][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, offset(j) + i * row_step, 0, 0));
+        };
+        if constexpr (ACC) fetch(0);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
+            if constexpr (ACC)
+                if (i + 1 < TM) fetch(i + 1);
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                const int col = col0 + j * 16 + 4 * (lane >> 4);
-                const uint32_t voff = col < nrem ? row_off + (uint32_t)col * SZ : kOut;
-                f32x4 v = acc[i][j];
+                f32x4 v = from_agprs<TM * TN>(acc[i][j]);
                 if constexpr (ROUND)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] = (float)(bf16_t)v[r];
                 if constexpr (ACC) {
-                    const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(cbuf, voff + i * row_step, 0, 0));
+                    const f32x4 o = __builtin_bit_cast(f32x4, old[i & 1][j]);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] += old[r];
+                    for (int r = 0; r < 4; ++r) v[r] += o[r];
                 }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, voff + i * row_step, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, offset(j) + i * row_step, 0, 0);
             }
+            if constexpr (TM * TN >= 64) __builtin_amdgcn_sched_barrier(0);
         }
     }
 }

@@ -129,6 +129,35 @@ def test_gemm_smaller_tiles_leave_what_is_outside_the_result_alone(K):
         assert (border == 7.0).all(), (form, M, N, Kd)
 
 
+@pytest.mark.parametrize("form,M,N,Kd", [
+    # several tiles per workgroup: ragged edges, K tails, a split last round, one K tile more or less than where the rule changes
+    (0, 5000, 20000, 1096), (0, 4096, 8192, 1024), (0, 4000, 17000, 4096), (0, 4000, 17000, 4104), (2, 5000, 20008, 1100), (2, 4096, 4352, 4160),
+    # one workgroup per tile: whole rounds and split ones, input gradients
+    (0, 4096, 4096, 8200), (2, 3000, 3080, 9000), (1, 4100, 5128, 10248), (1, 4096, 4096, 10240), (2, 8192, 8192, 2048)])
+def test_gemm_four_wave_kernel(K, form, M, N, Kd):
+    print("gemm", form, M, N, Kd, flush=True)
+    check_gemm(K, form, M, N, Kd)
+    check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
+    if form == 0:
+        x, w = rnd(M, Kd, seed=1), rnd(N, Kd, seed=2)
+        f = K.linear_fwd(x, w, fp32_output=True)
+        tol = gemm_bound(x, w.t()) + f.abs() * 2.0 ** -8 + 1e-6
+        assert torch.equal(f, f.bfloat16().float()) and ((f - x.float() @ w.float().t()).abs() <= tol).all()
+
+
+def test_gemm_four_wave_kernel_over_pairs(K):
+    T, n_in, outs = 4100, 4104, (16392, 16392)
+    print("dgrad multi", T, n_in, outs, flush=True)
+    dys = [rnd(T, o, seed=i) for i, o in enumerate(outs)]
+    ws = [rnd(o, n_in, seed=10 + i) for i, o in enumerate(outs)]
+    A, B = torch.cat(dys, 1), torch.cat(ws, 0)
+    ref, bound = A.float() @ B.float(), gemm_bound(A, B)
+    dx = K.linear_dgrad_multi(dys, ws)
+    assert ((dx.float() - ref).abs() <= bound + ref.abs() * 2.0 ** -8 + 1e-6).all()
+    K.linear_dgrad_multi(dys, ws, out=dx, accumulate=True)
+    assert ((dx.float() - 2 * ref).abs() <= 2 * bound + ref.abs() * 2.0 ** -6 + 1e-6).all()
+
+
 @pytest.mark.parametrize("T,n_in,outs", [(1024, 256, (256, 256, 256)), (1167, 1024, (1024, 256, 264)), (389, 768, (2048, 2056)),
                                          (17, 264, (8, 1000, 72)), (4000, 2048, (2048, 512, 512)), (9000, 256, (256, 512))])
 def test_gemm_products_in_one_launch(K, T, n_in, outs):
