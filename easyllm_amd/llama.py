@@ -105,14 +105,17 @@ class LlamaModelPipe(torch.nn.Module):
     def get_seq_len(self, forward_input):
         return forward_input[0].shape[1]  # first (and only) pipeline stage: tokens [b, s]
 
-    def forward(self, forward_input):
+    def forward(self, forward_input, cast_logits=True):
+        """cast_logits=False: the logits as the head computed them, in bf16, also where fp32_logits asks for an fp32 copy."""
         seq_len = self.get_seq_len(forward_input)
         if self.size_map is not None:
             self.skip_checkpoint_layer_range = self.start_checkpoint_layer_idx + self.get_checkpoint_range(seq_len)
-        return self._forward_specs(forward_input)
+        return self._forward_specs(forward_input, cast_logits)
 
-    def _forward_specs(self, x):
+    def _forward_specs(self, x, cast_logits=True):
         funcs_all = self.forward_funcs
+        if not cast_logits and funcs_all[-1] is float16_to_fp32:
+            funcs_all = funcs_all[:-1]
         n = len(funcs_all)
 
         def exec_range(start, end):

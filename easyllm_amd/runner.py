@@ -9,7 +9,9 @@ number of accumulation steps and ZeRO partitioning are DeepSpeed's and are not r
 import torch
 
 from .registry import MODULE_ZOO_REGISTRY
-from . import llama as _llama  # noqa: F401  (registers the model builders)
+from . import llama as _llama  # (registers the model builders)
+from .losses import CrossEntropy
+from .transformer import is_plain
 
 
 def build_model(cfg):
@@ -33,9 +35,19 @@ def zero_main_grads(model):
         p.grad = None
 
 
+def _logits_stay_inside(model):
+    """Nobody but this framework's own fused loss sees the model's output: no hook, subclass or other loss in between.
+
+    fp32_logits then only costs passes over memory: the fp32 logits hold bf16 values, the loss computes in fp32 from either, and
+    its fp32 gradient is rounded to bf16 before the head's products.  Without the copies 4 x 1000 tokens at V = 32000 save 0.47 ms
+    of 3.38 (a cast of the gradient, 146 us, and half the bytes of the head's result and of the loss)."""
+    return (is_plain(model, _llama.LlamaModelPipe) and type(model.loss_fn) is CrossEntropy and model.loss_fn.fused
+            and is_plain(model.forward_funcs[-2], _llama.EmbedddingPipeNoTied))
+
+
 def forward_step(model, inputs, labels):
     """One micro-batch: returns the loss tensor after backward has run."""
-    output = model(inputs)
+    output = model(inputs, cast_logits=False) if _logits_stay_inside(model) else model(inputs)
     loss = model.loss_fn(output, labels)
     loss.backward()
     return loss

@@ -353,3 +353,31 @@ def test_default_fp32_logits_are_the_cast_of_the_bf16_ones():
     assert outs[0][0].dtype == torch.float32 and torch.equal(outs[0][0], outs[1][0].float())
     for n in outs[0][1]:  # the logits' gradient is rounded to bf16 once either way, from exponentials of two kernels
         assert (outs[0][1][n].float() - outs[1][1][n].float()).norm() <= 2e-2 * outs[1][1][n].float().norm(), n
+
+
+@pytest.mark.parametrize("ignored", [0.0, 0.3])
+def test_a_training_step_needs_no_fp32_copy_of_the_logits(ignored):
+    """forward_step with the default fp32 logits against its own composition: the same values in, fp32 inside, one rounding of the
+    logits' gradient.  The two loss kernels add in another order: 1e-6 of the loss, and values of the rounded gradient that fall to the
+    other side; the 12 bf16 tensors between it and the lowest weight gradient may each do so by one step, 2^-8 of a value, at
+    most, independently of each other: sqrt(12) 2^-8."""
+    from easyllm_amd import runner
+    kw = dict(num_layers=1, hidden_size=256, num_attention_heads=4, intermediate_size=512, vocab_size=1000, seq_length=64, bf16=True)
+    tokens, pos = torch.randint(0, 1000, (2, 64)).cuda(), torch.arange(64).expand(2, 64).contiguous().cuda()
+    labels = torch.randint(0, 1000, (2, 64)).cuda()
+    labels[torch.rand(2, 64, device="cuda") < ignored] = -100
+    target = (labels, torch.ones(2, 64, device="cuda"))
+    results = []
+    for composed in (True, False):
+        torch.manual_seed(0)
+        model = runner.build_model({"type": "llama_custom", "kwargs": dict(kw)}).cuda()
+        seen = []
+        if composed:  # a hook on the model sees fp32 logits, as before
+            model.register_forward_hook(lambda m, i, o: seen.append(o.dtype))
+        loss = runner.forward_step(model, (tokens, pos, None), target)
+        assert seen == [torch.float32] * composed
+        results.append((loss, {n: p.grad.float() for n, p in model.named_parameters()}))
+    (loss0, g0), (loss1, g1) = results
+    assert abs(loss0.item() - loss1.item()) <= 1e-6 * loss0.item()
+    for n in g0:
+        assert (g0[n] - g1[n]).norm() <= 12 ** 0.5 * 2.0 ** -8 * g0[n].norm(), n
