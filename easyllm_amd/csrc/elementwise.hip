@@ -266,7 +266,8 @@ constexpr int kWindowRows = 2048;  // a frequent id's rows are put in order thro
 // One frequent id, columns col0 + 2 thread, + 1: a thread walks the id's rows in order with up to 24 rows' loads in flight (one
 // register each), so that the time is the latency of n / 24 loads rather than of n / 4.  (1000 padding rows of 4000, h = 2048:
 // the scatter kernel 430 -> 79 us.)
-__device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY, float* __restrict__ dW, const int* __restrict__ mine, int n,
+template <typename OutT>
+__device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY, OutT* __restrict__ dW, const int* __restrict__ mine, int n,
                                                   int64_t id, int col0, int64_t rows, int h, int overwrite, int* list, unsigned* bits, int& wtot) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int col = col0 + 2 * threadIdx.x;
@@ -323,7 +324,10 @@ __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY,
         batch(std::integral_constant<int, 4>{});
         batch(std::integral_constant<int, 1>{});
     }
-    if (live) {
+    if (!live) return;
+    if constexpr (sizeof(OutT) == 2) {
+        *reinterpret_cast<bf16x2*>(dW + id * h + col) = bf16x2{(bf16_t)a0, (bf16_t)a1};
+    } else {
         f32x2* dst = reinterpret_cast<f32x2*>(dW + id * h + col);
         f32x2 o = {a0, a1};
         if (!overwrite) {
@@ -336,9 +340,13 @@ __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY,
 }
 
 // (rows of up to 4096: six waves per SIMD, as the zero fill wants them)
-template <int MAXC>
+// OutT bf16: the fp32 sums are rounded once as they are stored.  A gradient without an fp32 buffer behind it used to be written in
+// fp32, read by a cast and written again, five times the bytes of the result.  Gradient
+// of [V, h] over T rows, with the cast and now: 50304 x 1024, T 1167 98 -> 33 us; 32000 x 4096, T 4096 263 -> 59; 152064 x 5120
+// 1548 -> 304 (5.1 TB/s, on either side of the flat fill's line).
+template <int MAXC, typename OutT>
 __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucket_kernel(const int64_t* __restrict__ ids, const bf16_t* __restrict__ dY,
-                                                                      float* __restrict__ dW, const int* __restrict__ cnt,
+                                                                      OutT* __restrict__ dW, const int* __restrict__ cnt,
                                                                       const int* __restrict__ first, const int* __restrict__ off,
                                                                       const int* __restrict__ bucket, const int* __restrict__ cursor,
                                                                       const int* __restrict__ heavy, int64_t rows, int h, int64_t V,
@@ -429,19 +437,23 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
         for (int c = 0; c < MAXC; ++c) {
             const int col = (c * kBlock + threadIdx.x);
             if (col < h8) {
-                float* dst = dW + id * h + col * 8;
-                f32x4 lo, hi;
-                if (overwrite) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) { lo[k] = acc[c][k]; hi[k] = acc[c][4 + k]; }
+                OutT* dst = dW + id * h + col * 8;
+                if constexpr (sizeof(OutT) == 2) {
+                    st_bf16x8(dst, pack8(acc[c]));
                 } else {
-                    lo = *reinterpret_cast<f32x4*>(dst);
-                    hi = *reinterpret_cast<f32x4*>(dst + 4);
+                    f32x4 lo, hi;
+                    if (overwrite) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) { lo[k] += acc[c][k]; hi[k] += acc[c][4 + k]; }
+                        for (int k = 0; k < 4; ++k) { lo[k] = acc[c][k]; hi[k] = acc[c][4 + k]; }
+                    } else {
+                        lo = *reinterpret_cast<f32x4*>(dst);
+                        hi = *reinterpret_cast<f32x4*>(dst + 4);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) { lo[k] += acc[c][k]; hi[k] += acc[c][4 + k]; }
+                    }
+                    *reinterpret_cast<f32x4*>(dst) = lo;
+                    *reinterpret_cast<f32x4*>(dst + 4) = hi;
                 }
-                *reinterpret_cast<f32x4*>(dst) = lo;
-                *reinterpret_cast<f32x4*>(dst + 4) = hi;
             }
         }
     }
@@ -459,7 +471,7 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
             for (int r = 0; r < m; ++r) {
                 if (raw[r] != 0) continue;
                 f32x4* dst = reinterpret_cast<f32x4*>(dW + (v0 + (int64_t)r * gridDim.x) * h);
-                for (int i = threadIdx.x; i < (h >> 2); i += kBlock) __builtin_nontemporal_store(z, dst + i);
+                for (int i = threadIdx.x; i < h * (int)sizeof(OutT) / 16; i += kBlock) __builtin_nontemporal_store(z, dst + i);
             }
         }
     }
@@ -808,19 +820,21 @@ extern "C" int64_t ezl_embed_scatter_add_workspace_bytes(int64_t rows, int64_t v
     return (4 * vocab + rows + 4 + embed_heavy_max(rows)) * (int64_t)sizeof(int);
 }
 
-extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dweight_f32, void* workspace, int64_t workspace_bytes,
-                                     int64_t rows, int64_t h, int64_t vocab, int accumulate, void* stream) {
+namespace {
+template <typename OutT>
+int embed_gradient(const char* name, const void* ids, const void* dy, void* dweight, void* workspace, int64_t workspace_bytes, int64_t rows,
+                   int64_t h, int64_t vocab, int accumulate, void* stream) {
     EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h < (1LL << 31) && vocab > 0, EZL_EUNSUPPORTED,
-                "ezl_embed_scatter_add: h must be a multiple of 8");
-    EZL_REQUIRE((rows == 0 || (ids && dy && dweight_f32)) && ezl_aligned16(dy), EZL_EINVAL,
-                "ezl_embed_scatter_add: null or misaligned pointer");
+                "%s: h must be a multiple of 8", name);
+    EZL_REQUIRE((rows == 0 || (ids && dy && dweight)) && ezl_aligned16(dy), EZL_EINVAL,
+                "%s: null or misaligned pointer", name);
     if (rows == 0 && accumulate) return EZL_OK;
-    EZL_REQUIRE(dweight_f32, EZL_EINVAL, "ezl_embed_scatter_add: null or misaligned pointer");
-    EZL_REQUIRE(h <= 8192 * 2, EZL_EUNSUPPORTED, "ezl_embed_scatter_add: h must be <= 16384");
-    EZL_REQUIRE(rows < (1LL << 31) && vocab < (1LL << 31), EZL_EUNSUPPORTED, "ezl_embed_scatter_add: more than 2^31 rows or ids");
-    EZL_REQUIRE(((uintptr_t)dweight_f32 & 15) == 0, EZL_EINVAL, "ezl_embed_scatter_add: dweight must be 16-byte aligned");
+    EZL_REQUIRE(dweight, EZL_EINVAL, "%s: null or misaligned pointer", name);
+    EZL_REQUIRE(h <= 8192 * 2, EZL_EUNSUPPORTED, "%s: h must be <= 16384", name);
+    EZL_REQUIRE(rows < (1LL << 31) && vocab < (1LL << 31), EZL_EUNSUPPORTED, "%s: more than 2^31 rows or ids", name);
+    EZL_REQUIRE(((uintptr_t)dweight & 15) == 0, EZL_EINVAL, "%s: dweight must be 16-byte aligned", name);
     EZL_REQUIRE(workspace && ((uintptr_t)workspace & 3) == 0 && workspace_bytes >= ezl_embed_scatter_add_workspace_bytes(rows, vocab),
-                EZL_EINVAL, "ezl_embed_scatter_add: workspace missing or smaller than ezl_embed_scatter_add_workspace_bytes()");
+                EZL_EINVAL, "%s: workspace missing or smaller than ezl_embed_scatter_add_workspace_bytes()", name);
     int* cnt = (int*)workspace;
     int* first = cnt + vocab;
     int* off = first + vocab;
@@ -836,30 +850,41 @@ extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dwei
                        cursor, heavy, rows, vocab);
     hipLaunchKernelGGL(embed_bucket_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, off, fill,
                        bucket, rows, vocab);
-    EZL_LAUNCH_CHECK("ezl_embed_scatter_add(tables)");
+    EZL_LAUNCH_CHECK(name);
     // one workgroup per token row (accumulate) or per vocabulary row, whichever is more: the zero fill of the rows that
     // received nothing is most of the traffic when the result overwrites the buffer
     // Overwriting a large table ([152064, 5120] fp32 = 3.1 GB, say) is mostly a zero fill, and a flat fill kernel in front
     // of the adding form writes it faster than the per-row fill inside the scatter kernel does (measured 502 against 580 us
     // at that size); for a table of 0.5 GB the fused form wins (99 against 116 us) because the two parts overlap.
-    const bool flat_fill = !accumulate && vocab * h >= (int64_t)1 << 28;
+    const bool flat_fill = !accumulate && vocab * h * (int64_t)sizeof(OutT) >= (int64_t)1 << 30;
     if (flat_fill) {
-        const int64_t n4 = vocab * h / 4;
-        hipLaunchKernelGGL(zero_f32x4_kernel, dim3(grid_for(n4, 4 * kBlock, (int64_t)1 << 20)), dim3(kBlock), 0, st, (f32x4*)dweight_f32, n4);
+        const int64_t n4 = vocab * h * (int64_t)sizeof(OutT) / 16;
+        hipLaunchKernelGGL(zero_f32x4_kernel, dim3(grid_for(n4, 4 * kBlock, (int64_t)1 << 20)), dim3(kBlock), 0, st, (f32x4*)dweight, n4);
     }
     const int overwrite = accumulate || flat_fill ? 0 : 1;
     const dim3 grid(grid_for(overwrite ? (rows > vocab ? rows : vocab) : rows, 1));
     if (h <= 8 * kBlock * 2)
-        hipLaunchKernelGGL((embed_scatter_bucket_kernel<2>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (float*)dweight_f32, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
+        hipLaunchKernelGGL((embed_scatter_bucket_kernel<2, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
+                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
     else if (h <= 8 * kBlock * 4)
-        hipLaunchKernelGGL((embed_scatter_bucket_kernel<4>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (float*)dweight_f32, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
+        hipLaunchKernelGGL((embed_scatter_bucket_kernel<4, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
+                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
     else
-        hipLaunchKernelGGL((embed_scatter_bucket_kernel<8>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (float*)dweight_f32, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
-    EZL_LAUNCH_CHECK("ezl_embed_scatter_add");
+        hipLaunchKernelGGL((embed_scatter_bucket_kernel<8, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
+                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
+    EZL_LAUNCH_CHECK(name);
     return EZL_OK;
+}
+}  // namespace
+
+extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dweight_f32, void* workspace, int64_t workspace_bytes,
+                                     int64_t rows, int64_t h, int64_t vocab, int accumulate, void* stream) {
+    return embed_gradient<float>("ezl_embed_scatter_add", ids, dy, dweight_f32, workspace, workspace_bytes, rows, h, vocab, accumulate, stream);
+}
+
+extern "C" int ezl_embed_grad_bf16(const void* ids, const void* dy, void* dweight_bf16, void* workspace, int64_t workspace_bytes,
+                                   int64_t rows, int64_t h, int64_t vocab, void* stream) {
+    return embed_gradient<bf16_t>("ezl_embed_grad_bf16", ids, dy, dweight_bf16, workspace, workspace_bytes, rows, h, vocab, 0, stream);
 }
 
 extern "C" int ezl_transpose01(const void* x, void* y, int64_t d0, int64_t d1, int64_t inner, void* stream) {

@@ -384,9 +384,7 @@ class EmbeddingFunction(torch.autograd.Function):
         if mg is not None:
             K.embed_scatter_add(ids, dout.contiguous(), mg, accumulate=acc)
             return None, None
-        buf = torch.empty(weight.shape, dtype=torch.float32, device=weight.device)
-        K.embed_scatter_add(ids, dout.contiguous(), buf, accumulate=False)
-        return None, K.cast_f32_to_bf16(buf)
+        return None, K.embed_grad_bf16(ids, dout.contiguous(), weight.shape[0])
 
 
 def _raise_for_id_flag(bad, ids, num_embeddings):

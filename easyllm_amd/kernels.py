@@ -193,6 +193,19 @@ def embed_scatter_add(ids, dy, dweight_f32, accumulate=True):
     _lib.call("ezl_embed_scatter_add", _p(ids), _p(dy), _p(dweight_f32), _p(ws), ws_bytes, ids.numel(), h, V, 1 if accumulate else 0, _stream())
 
 
+def embed_grad_bf16(ids, dy, vocab):
+    """-> bf16 [vocab, h]: what embed_scatter_add(accumulate=False) writes, each sum rounded once."""
+    _need(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous(), "ids must be contiguous int64 on the GPU")
+    _bf16c(dy, "dy")
+    h = dy.shape[-1]
+    _need(dy.numel() == ids.numel() * h, "one dy row per id")
+    dweight = torch.empty((vocab, h), dtype=BF16, device=dy.device)
+    ws_bytes = _lib.embed_scatter_add_workspace_bytes(ids.numel(), vocab)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dy.device)
+    _lib.call("ezl_embed_grad_bf16", _p(ids), _p(dy), _p(dweight), _p(ws), ws_bytes, ids.numel(), h, vocab, _stream())
+    return dweight
+
+
 # ------------------------------------------------------------------------------------- plumbing
 def transpose01(x):
     _bf16c(x, "x")

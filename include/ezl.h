@@ -94,6 +94,9 @@ int ezl_embed_gather(const void* ids, const void* weight, void* out, void* bad_f
 int64_t ezl_embed_scatter_add_workspace_bytes(int64_t rows, int64_t vocab);
 int ezl_embed_scatter_add(const void* ids, const void* dy, void* dweight_f32, void* workspace, int64_t workspace_bytes,
                           int64_t rows, int64_t h, int64_t vocab, int accumulate, void* stream);
+/* the overwriting form into a bf16 gradient: the same fp32 sums, rounded once */
+int ezl_embed_grad_bf16(const void* ids, const void* dy, void* dweight_bf16, void* workspace, int64_t workspace_bytes,
+                        int64_t rows, int64_t h, int64_t vocab, void* stream);
 
 /* ---- layout / dtype plumbing of llama/llama.py:145-188 (transpose, undo, float16_to_fp32) ---- */
 int ezl_transpose01(const void* x, void* y, int64_t d0, int64_t d1, int64_t inner, void* stream); /* y[j,i,:] = x[i,j,:] */

@@ -381,3 +381,18 @@ def test_a_training_step_needs_no_fp32_copy_of_the_logits(ignored):
     assert abs(loss0.item() - loss1.item()) <= 1e-6 * loss0.item()
     for n in g0:
         assert (g0[n] - g1[n]).norm() <= 12 ** 0.5 * 2.0 ** -8 * g0[n].norm(), n
+
+
+@pytest.mark.parametrize("V,h,rows,frequent", [(1, 8, 1, 0), (50, 64, 600, 0), (4099, 1024, 1167, 0), (4099, 1032, 1167, 700), (700, 4104, 130, 40),
+                                               (90, 8200, 300, 100), (70000, 8192, 257, 33), (333, 512, 0, 0)])
+def test_embedding_gradient_in_bf16_is_the_fp32_one_rounded(K, V, h, rows, frequent):
+    """Every register depth of the kernel, frequent ids (more than 32 rows), a table of more than 1 GiB (cleared by a fill of its
+    own) and an empty batch.  The sums run in fp32 in row order in both forms: equal bit for bit."""
+    print("embedding gradient bf16", V, h, rows, frequent, flush=True)
+    ids = torch.randint(0, V, (rows,), generator=torch.Generator().manual_seed(rows + h))
+    ids[:frequent] = V // 2
+    ids, dy = ids.cuda(), rnd(rows, h, seed=4)
+    ref = torch.full((V, h), 3.5, device="cuda")
+    K.embed_scatter_add(ids, dy, ref, accumulate=False)
+    got = K.embed_grad_bf16(ids, dy, V)
+    assert got.dtype is torch.bfloat16 and torch.equal(got, ref.bfloat16())
