@@ -906,7 +906,21 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     return EZL_OK;
 }
 
-// Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch.
+namespace {
+// Whether two results of a group share memory (one weight used by two projections: one gradient buffer): in one launch their tiles
+// would be read and written in any order.  Address ranges are compared, so interleaved column blocks count as sharing.
+bool results_meet(int count, void* const* C, const int64_t* M, const int64_t* N, const int64_t* ldc, int64_t size) {
+    for (int i = 1; i < count; ++i)
+        for (int j = 0; j < i; ++j) {
+            const char *a = (const char*)C[i], *b = (const char*)C[j];
+            if (a < b + ((M[j] - 1) * ldc[j] + N[j]) * size && b < a + ((M[i] - 1) * ldc[i] + N[i]) * size) return true;
+        }
+    return false;
+}
+}  // namespace
+
+// Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch; one after the other where their
+// results share memory.
 // ezl_gemm_group_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
 extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
     if (count < 2 || count > kMaxProblems || !M || !N || K <= 0) return -1;
@@ -936,6 +950,13 @@ extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* 
         tiles += tiles_of(kTile64, M[i], N[i]);
     }
     EZL_REQUIRE(tiles < (1LL << 27), EZL_EUNSUPPORTED, "ezl_gemm_bf16_group: too many tiles");
+    if (results_meet(count, C, M, N, ldc, out_dtype == 0 ? 2 : 4)) {
+        for (int i = 0; i < count; ++i)
+            if (const int rc = ezl_gemm_bf16(A[i], B[i], C[i], M[i], N[i], K, lda[i], ldb[i], ldc[i], a_kc, b_kc, out_dtype, accumulate[i],
+                                             workspace, workspace_bytes, stream))
+                return rc;
+        return EZL_OK;
+    }
     GemmPlan plan;
     group_plan(count, M, N, K, INT64_MAX, plan);
     if (small_plan_bytes(plan, count, M, N) > (workspace ? workspace_bytes : 0)) group_plan(count, M, N, K, 0, plan);

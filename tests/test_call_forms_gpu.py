@@ -1,0 +1,78 @@
+"""Forms of calls that a fast path must answer as the general one does: shared and odd buffers, replaced parts, values that are not
+finite."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from easyllm_amd import kernels
+    return kernels
+
+
+def rnd(*shape, seed=0, scale=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device="cuda") * scale).bfloat16()
+
+
+def product_bound(A, B):
+    """Products of bf16 values are exact in fp32; summing K of them in any order is off by at most K 2^-24 sum|a b| (taken 4 times
+    too large)."""
+    return A.float().abs() @ B.float().abs() * (4 * A.shape[1] * 2.0 ** -24)
+
+
+def small_model(**kw):
+    from easyllm_amd import runner
+    torch.manual_seed(3)
+    cfg = dict(num_layers=1, hidden_size=256, num_attention_heads=4, intermediate_size=688, vocab_size=512, seq_length=192, bf16=True,
+               checkpoint_activations=False)
+    cfg.update(kw)
+    model = runner.build_model({"type": "llama_custom", "kwargs": cfg}).cuda()
+    with torch.no_grad():
+        for p in model.parameters():
+            if p.dim() == 1:
+                p.add_(0.1 * torch.randn_like(p))
+    return model
+
+
+def small_batch(b=2, s=192, vocab=512):
+    g = torch.Generator().manual_seed(1)
+    tokens, labels = torch.randint(0, vocab, (b, s), generator=g).cuda(), torch.randint(0, vocab, (b, s), generator=g).cuda()
+    return (tokens, torch.arange(s).expand(b, s).contiguous().cuda(), None), (labels, torch.ones(b, s, device="cuda"))
+
+
+def decoder_layer(model):
+    return next(m for m in model.modules() if hasattr(m, "native_call_flops"))
+
+
+# ---- results of one launch that share memory ---------------------------------------------------------------------------
+@pytest.mark.parametrize("T,n_in,n_out,count", [(1024, 256, 256, 3), (1167, 1024, 256, 2), (4000, 2048, 512, 3), (9000, 256, 512, 2)])
+def test_weight_gradients_of_one_weight_used_several_times(K, T, n_in, n_out, count):
+    """One buffer for several products, at sizes where they would otherwise share a launch: they are added one after the other."""
+    from easyllm_amd import _lib
+    print("one weight, several uses", T, n_in, n_out, count, flush=True)
+    assert _lib.gemm_group_workspace_bytes((n_out,) * count, (n_in,) * count, T) >= 0
+    x, dys = rnd(T, n_in, seed=1), [rnd(T, n_out, seed=2 + i) for i in range(count)]
+    total = sum(dys[i].double().t() @ x.double() for i in range(count))
+    bound = sum(product_bound(dy.t(), x) for dy in dys) + total.abs() * 2.0 ** -20 + 1e-5
+    for first in (False, True):
+        mg = torch.full((n_out, n_in), 3.0, device="cuda")
+        K.linear_wgrad_multi(dys, x, [mg] * count, [first] + [True] * (count - 1))
+        assert ((mg - (total + 3.0 * first)).abs() <= bound).all()
+
+
+def test_a_weight_shared_by_two_projections_through_autograd():
+    from easyllm_amd import functional as F_
+    T, n = 1024, 256
+    x = rnd(T, n, seed=1)
+    w = torch.nn.Parameter(rnd(n, n, seed=2))
+    w.main_grad, w.main_grad_fresh = torch.full((n, n), 7.0, device="cuda"), True
+    dys = [rnd(T, n, seed=3 + i) for i in range(2)]
+    torch.autograd.backward(F_.fan_out_linear(x, w, w), dys)
+    ref = sum(dy.double().t() @ x.double() for dy in dys)
+    bound = sum(product_bound(dy.t(), x) for dy in dys) + ref.abs() * 2.0 ** -20 + 1e-5
+    assert ((w.main_grad - ref).abs() <= bound).all() and not w.main_grad_fresh
