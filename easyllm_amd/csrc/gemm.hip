@@ -920,7 +920,7 @@ bool results_meet(int count, void* const* C, const int64_t* M, const int64_t* N,
 }  // namespace
 
 // Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch; one after the other where their
-// results share memory.
+// results share memory or have rows too far apart.
 // ezl_gemm_group_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
 extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
     if (count < 2 || count > kMaxProblems || !M || !N || K <= 0) return -1;
@@ -941,16 +941,17 @@ extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* 
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16_group: workspace must be 16-byte aligned");
     GemmSmallArgs a = {};
     int64_t tiles = 0;
+    bool apart = false;
     for (int i = 0; i < count; ++i) {
         EZL_REQUIRE(C[i] && M[i] > 0 && N[i] > 0, EZL_EINVAL, "ezl_gemm_bf16_group: null pointer or empty product");
         if (const int rc = check_operands(A[i], B[i], M[i], N[i], K, lda[i], ldb[i], ldc[i], a_kc, b_kc)) return rc;
-        EZL_REQUIRE(out_dtype == 0 ? small_stores_ok<bf16_t>(ldc[i]) : small_stores_ok<float>(ldc[i]), EZL_EUNSUPPORTED,
-                    "ezl_gemm_bf16_group: leading dimension of C too large");
+        // (rows of C too far apart for the smaller tiles' stores: ezl_gemm_bf16 has kernels for them)
+        apart = apart || !(out_dtype == 0 ? small_stores_ok<bf16_t>(ldc[i]) : small_stores_ok<float>(ldc[i]));
         a.p[i] = {(const bf16_t*)A[i], (const bf16_t*)B[i], C[i], lda[i], ldb[i], ldc[i], (int)M[i], (int)N[i], 0, 0, 0, accumulate[i]};
         tiles += tiles_of(kTile64, M[i], N[i]);
     }
     EZL_REQUIRE(tiles < (1LL << 27), EZL_EUNSUPPORTED, "ezl_gemm_bf16_group: too many tiles");
-    if (results_meet(count, C, M, N, ldc, out_dtype == 0 ? 2 : 4)) {
+    if (apart || results_meet(count, C, M, N, ldc, out_dtype == 0 ? 2 : 4)) {
         for (int i = 0; i < count; ++i)
             if (const int rc = ezl_gemm_bf16(A[i], B[i], C[i], M[i], N[i], K, lda[i], ldb[i], ldc[i], a_kc, b_kc, out_dtype, accumulate[i],
                                              workspace, workspace_bytes, stream))

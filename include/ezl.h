@@ -129,8 +129,8 @@ int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void* const* B, 
 /* Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch: q / k / v (gate / up) of
  * one input, or their weight gradients, where each alone would leave most of the chip idle.  The workspace query returns -1
  * where separate calls are estimated to be faster (the call itself makes one launch all the same, except that products whose results
- * share memory go out one after the other, in the order of the list).  Forms: forward, input gradient
- * (bf16 results) and weight gradient (bf16 or fp32); all arrays are HOST arrays of `count` entries. */
+ * share memory, or any with result rows 8 MiB or more apart, go out one after the other, in the order of the list).  Forms: forward,
+ * input gradient (bf16 results) and weight gradient (bf16 or fp32); all arrays are HOST arrays of `count` entries. */
 int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K);
 int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
                         int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,

@@ -76,3 +76,19 @@ def test_a_weight_shared_by_two_projections_through_autograd():
     ref = sum(dy.double().t() @ x.double() for dy in dys)
     bound = sum(product_bound(dy.t(), x) for dy in dys) + ref.abs() * 2.0 ** -20 + 1e-5
     assert ((w.main_grad - ref).abs() <= bound).all() and not w.main_grad_fresh
+
+
+def test_weight_gradients_into_buffers_with_far_apart_rows(K):
+    """Rows 8 MiB apart are more than the smaller-tile kernels' offsets reach: such results are stored by the others."""
+    from easyllm_amd import _lib
+    T, n_in, outs, ld = 1024, 264, (8, 16), 1 << 21
+    assert _lib.gemm_group_workspace_bytes(outs, (n_in,) * 2, T) >= 0
+    x, dys = rnd(T, n_in, seed=1), [rnd(T, o, seed=2 + i) for i, o in enumerate(outs)]
+    bufs = [torch.full((o * ld,), 5.0, device="cuda") for o in outs]
+    mgs = [b.as_strided((o, n_in), (ld, 1)) for b, o in zip(bufs, outs)]
+    K.linear_wgrad_multi(dys, x, mgs, [False, True])
+    for mg, buf, dy, old in zip(mgs, bufs, dys, (0.0, 5.0)):
+        ref = dy.double().t() @ x.double() + old
+        assert ((mg - ref).abs() <= product_bound(dy.t(), x) + ref.abs() * 2.0 ** -20 + 1e-5).all()
+        mg.fill_(5.0)
+        assert (buf == 5.0).all()
