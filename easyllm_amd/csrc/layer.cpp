@@ -134,6 +134,28 @@ int weight_gradients(int count, const void* const* dy, int64_t ld, const void* x
     return EZL_OK;
 }
 
+// elements of the parameters, in the order of the gradient list
+void parameter_sizes(const Dims& m, int64_t (&n)[EZL_G_COUNT]) {
+    n[EZL_G_LN1] = n[EZL_G_LN2] = m.h;
+    n[EZL_G_Q] = n[EZL_G_O] = m.qw * m.h;
+    n[EZL_G_K] = n[EZL_G_V] = m.kw * m.h;
+    n[EZL_G_GATE] = n[EZL_G_UP] = n[EZL_G_DOWN] = m.f * m.h;
+    n[EZL_G_BQ] = m.qw;
+    n[EZL_G_BK] = n[EZL_G_BV] = m.kw;
+}
+bool gradients_meet(const Dims& m, const ezl_layer_grad* g) {
+    int64_t n[EZL_G_COUNT];
+    parameter_sizes(m, n);
+    const char *from[EZL_G_COUNT], *to[EZL_G_COUNT];
+    for (int i = 0; i < EZL_G_COUNT; ++i) {
+        from[i] = (const char*)(g[i].f32 ? g[i].f32 : g[i].bf16);
+        to[i] = from[i] + (from[i] ? n[i] * (g[i].f32 ? 4 : 2) : 0);
+        for (int j = 0; j < i; ++j)
+            if (from[i] < to[j] && from[j] < to[i]) return true;
+    }
+    return false;
+}
+
 int check(const char* name, const ezl_layer* l) {
     EZL_REQUIRE(l, EZL_EINVAL, "%s: null argument", name);
     EZL_REQUIRE(l->s > 0 && l->b > 0 && l->h > 0 && l->nq > 0 && l->nk > 0 && l->nq % l->nk == 0 && l->d > 0 && l->f > 0 && l->ndocs > 0,
@@ -200,6 +222,7 @@ extern "C" int ezl_layer_bwd(const ezl_layer* l, const void* x, const void* dy, 
     const BackwardTemp t(*l, m, temp);
     EZL_REQUIRE((g[EZL_G_LN1].f32 || g[EZL_G_LN1].bf16) && (g[EZL_G_LN2].f32 || g[EZL_G_LN2].bf16), EZL_EINVAL,
                 "ezl_layer_bwd: the norm weights' gradients are part of their kernels");
+    EZL_REQUIRE(!gradients_meet(m, g), EZL_EINVAL, "ezl_layer_bwd: two gradients share memory (they are written in the kernels' order)");
     // y = sum + down(act): dy goes to both
     EZL_TRY(ezl_gemm_bf16(dy, l->wd, t.dact, m.T, m.f, m.h, m.h, m.f, m.f, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
     {

@@ -348,16 +348,27 @@ class DecoderLayerFunction(torch.autograd.Function):
     def backward(ctx, dy):
         x, saved, cos, sin, position_ids, cu_seqlens, *params = ctx.saved_tensors
         desc = K.layer_desc(x.shape, *ctx.plan, params[:9], params[9:] or None, cos, sin, position_ids, cu_seqlens)
-        targets, grads = [], []
+        # The kernels write the gradients in their own order (down first, ln1 last), several in one launch, while the accumulate
+        # flags hold for the order of the list: where a buffer occurs again (a parameter in two places), only its first gradient
+        # is written there by the kernels, the others are added afterwards.
+        targets, grads, again, taken = [], [], [], set()
         for i, p in enumerate(params):
             needed = ctx.needs_input_grad[6 + i]
             mg, acc = _main_grad_target(p) if needed else (None, False)
             grad = None
+            if mg is not None:
+                address = mg.data_ptr()
+                if address in taken:
+                    again.append((mg, acc, torch.empty_like(p, dtype=torch.float32)))
+                    mg, acc = again[-1][2], False
+                taken.add(address)
             if mg is None and (needed or p.dim() == 1):  # (a norm's kernel writes its weight gradient in any case)
                 grad = torch.empty_like(p)
             targets.append((mg, grad, acc) if mg is not None or grad is not None else None)
             grads.append(grad if needed else None)
         dx = K.layer_bwd(desc, x, dy.contiguous(), saved, targets)
+        for mg, acc, part in again:
+            mg.add_(part.view(mg.shape)) if acc else mg.copy_(part.view(mg.shape))
         return (dx if ctx.needs_input_grad[0] else None, None, None, None, None, None, *grads)
 
 

@@ -253,7 +253,7 @@ enum { EZL_G_LN1, EZL_G_Q, EZL_G_K, EZL_G_V, EZL_G_O, EZL_G_LN2, EZL_G_GATE, EZL
 int64_t ezl_layer_bytes(const ezl_layer* layer, int which);
 /* y = layer(x); `saved` is what ezl_layer_bwd needs, `temp` is free again when the call's work is done */
 int ezl_layer_fwd(const ezl_layer* layer, const void* x, void* y, void* saved, void* temp, void* stream);
-/* grads: EZL_G_COUNT entries */
+/* grads: EZL_G_COUNT entries, no two of which share memory (they are written in the kernels' order, several in one launch) */
 int ezl_layer_bwd(const ezl_layer* layer, const void* x, const void* dy, void* dx, const void* saved, void* temp,
                   const ezl_layer_grad* grads, void* stream);
 

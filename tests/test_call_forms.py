@@ -1,0 +1,69 @@
+"""Forms of calls that a fast path must answer as the general one does, where that can be seen without a GPU."""
+import ctypes
+
+import pytest
+import torch
+
+from easyllm_amd import _lib
+from easyllm_amd import functional as F_
+
+
+# the order in which a layer's backward writes its parameters' gradients (down, gate, up, ln2, o, q / k / v biases, q, k, v, ln1)
+_WRITE_ORDER = (8, 6, 7, 5, 4, 9, 10, 11, 1, 2, 3, 0)
+
+
+def _layer_with_fake_kernels(monkeypatch, params):
+    """decoder_layer whose backward writes i + 1 as the gradient of parameter i, in the kernels' order and all reads of old values
+    of a launch before its writes (the q / k / v and gate / up gradients are one launch each)."""
+    def bwd(desc, x, dy, saved, targets):
+        for launch in ((8,), (6, 7), (5,), (4,), (9, 10, 11), (1, 2, 3), (0,)):
+            new = []
+            for i in launch:
+                if i < len(targets) and targets[i] is not None:
+                    f32, bf16, acc = targets[i]
+                    out = bf16 if f32 is None else f32
+                    new.append((out, out + (i + 1) if acc else torch.full_like(out, i + 1)))
+            for out, value in new:
+                out.copy_(value)
+        return torch.ones_like(x)
+
+    monkeypatch.setattr(F_.K, "layer_desc", lambda *a: None)
+    monkeypatch.setattr(F_.K, "layer_fwd", lambda desc, x: (x.clone(), torch.empty(0)))
+    monkeypatch.setattr(F_.K, "layer_bwd", bwd)
+    x = torch.ones(2, 1, 4, requires_grad=True)
+    return F_.decoder_layer(x, (), torch.ones(1), torch.ones(1), None, None, tuple(params))
+
+
+@pytest.mark.parametrize("fresh", [True, False])
+@pytest.mark.parametrize("tied", [(0, 5), (1, 2), (2, 3), (6, 7), (10, 11), (1, 4), (0, 5, 1), (6, 7, 8)])
+def test_a_parameter_that_occurs_twice_in_a_layer_gets_both_gradients(monkeypatch, tied, fresh):
+    assert sorted(_WRITE_ORDER) == list(range(12))
+    params = [torch.nn.Parameter(torch.zeros(4)) for _ in range(12)]
+    for i in tied[1:]:
+        params[i] = params[tied[0]]
+    for p in params:
+        p.main_grad = torch.full((4,), 100.0)
+        p.main_grad_fresh = fresh
+    _layer_with_fake_kernels(monkeypatch, params).sum().backward()
+    for p in set(params):
+        want = sum(i + 1 for i in range(12) if params[i] is p) + (0 if fresh else 100)
+        assert torch.equal(p.main_grad, torch.full((4,), float(want))) and p.grad is None and not p.main_grad_fresh
+
+
+def test_a_parameter_that_occurs_twice_in_a_layer_without_gradient_buffers(monkeypatch):
+    params = [torch.nn.Parameter(torch.zeros(4)) for _ in range(9)]
+    params[5], params[3] = params[0], params[2]
+    _layer_with_fake_kernels(monkeypatch, params).sum().backward()
+    assert params[0].grad[0] == 1 + 6 and params[2].grad[0] == 3 + 4 and params[1].grad[0] == 2
+
+
+def test_layer_gradients_that_share_memory_are_refused():
+    """The kernels write in their own order, several results in one launch; nothing is launched for such a call."""
+    _lib.load()
+    layer = _lib.Layer(s=8, b=1, h=64, nq=1, nk=1, d=64, f=64, ndocs=1, npos=8)
+    grads = (_lib.LayerGrad * 12)()
+    for i in range(9):
+        grads[i].f32 = 0x100000 * (i + 1)
+    grads[3].f32 = grads[2].f32 + 64 * 64 * 4 - 4  # v starts on the last element of k
+    with pytest.raises(RuntimeError, match="share memory"):
+        _lib.call("ezl_layer_bwd", ctypes.byref(layer), 256, 256, 256, 256, 256, grads, None)

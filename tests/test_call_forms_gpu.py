@@ -92,3 +92,39 @@ def test_weight_gradients_into_buffers_with_far_apart_rows(K):
         assert ((mg - ref).abs() <= product_bound(dy.t(), x) + ref.abs() * 2.0 ** -20 + 1e-5).all()
         mg.fill_(5.0)
         assert (buf == 5.0).all()
+
+
+@pytest.mark.parametrize("tied", ["norms", "k_v", "gate_up", "q_o", "biases"])
+@pytest.mark.parametrize("fresh", [True, False])
+def test_a_layer_with_a_shared_parameter_against_the_composed_layer(tied, fresh):
+    """The same activations and gradients of activations bit for bit; the weight gradients from the same bf16 values, summed in
+    fp32 in another order at most: 1e-5 of their norm."""
+    from easyllm_amd import runner
+    print("shared parameter", tied, fresh, flush=True)
+    results = []
+    for flops in (1e12, 0.0):
+        model = small_model(num_layers=2, **({"transformer_layer_params": {"attention_qkv_bias": True}} if tied == "biases" else {}))
+        for m in model.modules():
+            if hasattr(m, "native_call_flops"):
+                m.native_call_flops = flops
+                attn, mlp = m.self_attn, m.mlp
+                if tied == "norms":
+                    m.post_attention_layernorm.weight = m.input_layernorm.weight
+                elif tied == "k_v":
+                    attn.v_proj.weight = attn.k_proj.weight
+                elif tied == "gate_up":
+                    mlp.up_proj.weight = mlp.gate_proj.weight
+                elif tied == "q_o":
+                    attn.o_proj.weight = attn.q_proj.weight
+                else:
+                    attn.v_proj.bias = attn.k_proj.bias = attn.q_proj.bias
+        runner.attach_main_grads(model)
+        for p in model.parameters():
+            p.main_grad.fill_(3.0)
+            p.main_grad_fresh = fresh
+        loss = runner.forward_step(model, *small_batch())
+        results.append((loss, {n: p.main_grad for n, p in model.named_parameters()}))
+    (loss1, g1), (loss0, g0) = results
+    assert torch.equal(loss1, loss0) and g1.keys() == g0.keys()
+    for n in g0:
+        assert (g1[n] - g0[n]).norm() <= 1e-5 * g0[n].norm(), n
