@@ -207,9 +207,25 @@ AdamArgs adam_args(float lr, float beta1, float beta2, float eps, float weight_d
     return a;
 }
 
-// calls launch(list, number of blocks) for every kListMax non-empty tensors of 0 .. count - 1; fill(list, slot, i) sets the pointers
-template <class Fill, class Launch>
-void for_each_list(int count, const int64_t* n, Fill fill, Launch launch) {
+// Whether an update of the list writes memory that tensor `slot` is made of: a parameter that occurs twice is updated twice, one
+// launch after the other.
+bool updates_meet(const TensorList& l, int slot) {
+    auto meet = [&](const void* const* streams, int size) {
+        const char* p = (const char*)streams[slot];
+        for (int i = 0; i < slot && p; ++i) {
+            const char* q = (const char*)streams[i];
+            if (q && p < q + l.n[i] * size && q < p + l.n[slot] * size) return true;
+        }
+        return false;
+    };
+    return meet((const void* const*)l.a, 4) || meet((const void* const*)l.m, 4) || meet((const void* const*)l.v, 4) ||
+           meet((const void* const*)l.param, 2);
+}
+
+// calls launch(list, number of blocks) for every kListMax non-empty tensors of 0 .. count - 1, and earlier in front of a tensor
+// that must_wait(list, slot); fill(list, slot, i) sets the pointers
+template <class Fill, class Wait, class Launch>
+void for_each_list(int count, const int64_t* n, Fill fill, Wait must_wait, Launch launch) {
     TensorList l;
     l.count = l.chunks = 0;
     auto flush = [&]() {
@@ -222,6 +238,11 @@ void for_each_list(int count, const int64_t* n, Fill fill, Launch launch) {
         if (l.count == kListMax || l.chunks + chunks >= (1LL << 30)) flush();
         fill(l, l.count, i);
         l.n[l.count] = n[i];
+        if (must_wait(l, l.count)) {
+            flush();
+            fill(l, 0, i);
+            l.n[0] = n[i];
+        }
         l.first[l.count] = l.chunks;
         l.chunks += (int)chunks;
         ++l.count;
@@ -263,7 +284,7 @@ extern "C" int ezl_adamw_step(void* master, void* exp_avg, void* exp_avg_sq, con
     const AdamArgs a = adam_args(lr, beta1, beta2, eps, weight_decay, step, bias_correction);
     for_each_list(1, one, [&](TensorList& l, int s, int) {
         l.a[s] = (float*)master; l.m[s] = (float*)exp_avg; l.v[s] = (float*)exp_avg_sq; l.g[s] = (const float*)grad; l.param[s] = (bf16_t*)param_bf16;
-    }, [&](const TensorList& l, unsigned blocks) {
+    }, updates_meet, [&](const TensorList& l, unsigned blocks) {
         hipLaunchKernelGGL(adamw_list_kernel, dim3(blocks), dim3(kOptBlock), 0, (hipStream_t)stream, l, a, (const float*)norm_coef);
     });
     EZL_LAUNCH_CHECK("ezl_adamw_step");
@@ -280,7 +301,8 @@ extern "C" int ezl_sumsq_list(int count, const void* const* x, const int64_t* n,
                     "ezl_sumsq_list: null or misaligned tensor");
     float* out = (float*)partials;
     float* const end = out + ezl_sumsq_list_partials(count);
-    for_each_list(count, n, [&](TensorList& l, int s, int i) { l.g[s] = (const float*)x[i]; }, [&](const TensorList& l, unsigned blocks) {
+    for_each_list(count, n, [&](TensorList& l, int s, int i) { l.g[s] = (const float*)x[i]; }, [](const TensorList&, int) { return false; },
+                  [&](const TensorList& l, unsigned blocks) {
         hipLaunchKernelGGL(sumsq_list_kernel, dim3(blocks), dim3(kOptBlock), 0, (hipStream_t)stream, l, out);
         out += blocks;
     });
@@ -307,7 +329,7 @@ extern "C" int ezl_adamw_list(int count, void* const* master, void* const* exp_a
     for_each_list(count, n, [&](TensorList& l, int s, int i) {
         l.a[s] = (float*)master[i]; l.m[s] = (float*)exp_avg[i]; l.v[s] = (float*)exp_avg_sq[i]; l.g[s] = (const float*)grad[i];
         l.param[s] = (bf16_t*)param_bf16[i];
-    }, [&](const TensorList& l, unsigned blocks) {
+    }, updates_meet, [&](const TensorList& l, unsigned blocks) {
         hipLaunchKernelGGL(adamw_list_kernel, dim3(blocks), dim3(kOptBlock), 0, (hipStream_t)stream, l, a, (const float*)norm_coef);
     });
     EZL_LAUNCH_CHECK("ezl_adamw_list");

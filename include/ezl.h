@@ -210,7 +210,8 @@ int ezl_clip_coef(const void* partials, int64_t count, float max_norm, void* nor
 int ezl_adamw_step(void* master, void* exp_avg, void* exp_avg_sq, const void* grad, void* param_bf16, int64_t n, float lr,
                    float beta1, float beta2, float eps, float weight_decay, int64_t step, int bias_correction,
                    const void* norm_coef, void* stream);
-/* The same over a list of tensors in one launch per 48 of them.  ezl_sumsq_list fills ezl_sumsq_list_partials(count) fp32 slots
+/* The same over a list of tensors in one launch per 48 of them (a tensor that shares memory with an earlier one starts a new
+ * launch: the updates are made in the order of the list).  ezl_sumsq_list fills ezl_sumsq_list_partials(count) fp32 slots
  * (any slots past the launched blocks are zeroed) for ezl_clip_coef; the arrays are HOST arrays of `count` entries, entries
  * of param_bf16 may be NULL. */
 int64_t ezl_sumsq_list_partials(int count);

@@ -128,3 +128,23 @@ def test_a_layer_with_a_shared_parameter_against_the_composed_layer(tied, fresh)
     assert torch.equal(loss1, loss0) and g1.keys() == g0.keys()
     for n in g0:
         assert (g1[n] - g0[n]).norm() <= 1e-5 * g0[n].norm(), n
+
+
+# ---- optimizer lists ---------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("order", [(0, 1, 0), (0, 0, 0, 0), tuple(range(50)) + (3, 49, 3), (1,) * 60])
+def test_a_tensor_that_occurs_twice_in_an_optimizer_list_is_updated_twice(K, order):
+    """One after the other, as single-tensor calls in the order of the list: bit for bit."""
+    print("optimizer list with repetitions", len(order), flush=True)
+    sizes = [70001 if i == 0 else 4096 * (1 + i % 3) + i for i in range(max(order) + 1)]
+    sides = []
+    for _ in range(2):
+        torch.manual_seed(5)
+        sides.append([[torch.randn(n, device="cuda") for n in sizes], [torch.randn(n, device="cuda") for n in sizes],
+                      [torch.rand(n, device="cuda") for n in sizes], [torch.randn(n, device="cuda") for n in sizes],
+                      [torch.zeros(n, device="cuda", dtype=torch.bfloat16) for n in sizes]])
+    coef = torch.tensor([5.0, 0.5], device="cuda")
+    a, b = sides
+    K.adamw_list(*[[ts[i] for i in order] for ts in a], 1e-2, 0.9, 0.95, 1e-8, 0.1, 3, True, coef)
+    for i in order:
+        K.adamw_step(*[ts[i] for ts in b], 1e-2, 0.9, 0.95, 1e-8, 0.1, 3, True, coef)
+    assert all(torch.equal(x, y) for xs, ys in zip(a, b) for x, y in zip(xs, ys))
