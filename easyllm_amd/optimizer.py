@@ -84,8 +84,10 @@ class FusedAdam:
 
     def global_grad_norm(self, max_norm):
         """(norm, coefficient) of all main_grads as a device tensor; max_norm <= 0 disables clipping (coefficient 1)."""
-        K.sumsq_list([p.main_grad for _, p in self._all_params()], self._partials)
-        return K.clip_coef(self._partials, max_norm, out=self._norm_coef)
+        grads = [p.main_grad for _, p in self._all_params()]
+        partials = self._partials[:K.sumsq_list_partials(len(grads))]  # (parameters may have been taken out of their groups)
+        K.sumsq_list(grads, partials)
+        return K.clip_coef(partials, max_norm, out=self._norm_coef)
 
     def step(self, clip_grad=0.0):
         norm_coef = self.global_grad_norm(clip_grad) if clip_grad and clip_grad > 0 else None

@@ -148,3 +148,19 @@ def test_a_tensor_that_occurs_twice_in_an_optimizer_list_is_updated_twice(K, ord
     for i in order:
         K.adamw_step(*[ts[i] for ts in b], 1e-2, 0.9, 0.95, 1e-8, 0.1, 3, True, coef)
     assert all(torch.equal(x, y) for xs, ys in zip(a, b) for x, y in zip(xs, ys))
+
+
+def test_the_gradient_norm_after_parameters_were_taken_out_of_a_group():
+    """Fewer tensors than the optimizer was built with, over the edge of what one launch takes."""
+    from easyllm_amd import optimizer
+    params = []
+    for i in range(50):
+        p = torch.nn.Parameter(rnd(100 + i, seed=i))
+        p.main_grad = torch.randn(100 + i, device="cuda")
+        params.append(p)
+    opt = optimizer.FusedAdam([{"params": params}])
+    opt.global_grad_norm(1.0)
+    for keep in (50, 48, 3):
+        del opt.param_groups[0]["params"][keep:]
+        want = torch.stack([p.main_grad.double().square().sum() for p in params[:keep]]).sum().sqrt()
+        assert abs(opt.global_grad_norm(1.0)[0] - want) <= 1e-5 * want
