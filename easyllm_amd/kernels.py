@@ -660,6 +660,8 @@ def adamw_list(masters, exp_avgs, exp_avg_sqs, grads, params, lr, beta1, beta2, 
                norm_coef=None):
     """adamw_step over lists of tensors (params: bf16 or None entries) in one launch per 48 of them."""
     ns = [t.numel() for t in masters]
+    for ts in (exp_avgs, exp_avg_sqs, grads, params):
+        _need(len(ts) == len(ns), "adamw_list: the lists need one entry per tensor")
     for ts, name in ((masters, "master"), (exp_avgs, "exp_avg"), (exp_avg_sqs, "exp_avg_sq"), (grads, "grad")):
         for t, n in zip(ts, ns):
             _f32c(t, name)

@@ -164,3 +164,11 @@ def test_the_gradient_norm_after_parameters_were_taken_out_of_a_group():
         del opt.param_groups[0]["params"][keep:]
         want = torch.stack([p.main_grad.double().square().sum() for p in params[:keep]]).sum().sqrt()
         assert abs(opt.global_grad_norm(1.0)[0] - want) <= 1e-5 * want
+
+
+def test_optimizer_lists_of_different_lengths_are_refused(K):
+    lists = [[torch.zeros(8, device="cuda") for _ in range(2)] for _ in range(4)] + [[None, None]]
+    for short in range(5):
+        args = [ts[:1] if i == short else ts for i, ts in enumerate(lists)]
+        with pytest.raises(ValueError, match="one entry per tensor"):
+            K.adamw_list(*args, 1e-2, 0.9, 0.95, 1e-8, 0.1, 3)
