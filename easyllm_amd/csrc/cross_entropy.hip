@@ -480,8 +480,8 @@ __global__ __launch_bounds__(kCeBlock) void ce_loss_kernel(const T* __restrict__
             for (int u = 0; u < 4; ++u)
 #pragma unroll
                 for (int k = 0; k < 8; ++k) mn = fmaxf(mn, f[u][k]);
-            if (mn == -INFINITY) return;
-            const float mb = mn * kLog2e;
+            // (a thread that has seen -inf only takes them off 0: exp2(-inf) is 0, and a NaN, which the maximum passes over, stays one)
+            const float mb = mn == -INFINITY ? 0.f : mn * kLog2e;
             s *= __builtin_amdgcn_exp2f(m * kLog2e - mb);
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(kCeBlock) void ce_loss_kernel(const T* __restrict__
             fold(f);
         }
         const float mrow = block_max(m, red);
-        s = block_sum(m == -INFINITY ? 0.f : s * __builtin_amdgcn_exp2f((m - mrow) * kLog2e), red);
+        s = block_sum(s * __builtin_amdgcn_exp2f((m - mrow) * kLog2e), red);
         if (threadIdx.x == 0) {
             const int64_t t = labels[r];
             const bool masked = t < 0 || t >= vend;

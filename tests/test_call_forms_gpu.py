@@ -172,3 +172,37 @@ def test_optimizer_lists_of_different_lengths_are_refused(K):
         args = [ts[:1] if i == short else ts for i, ts in enumerate(lists)]
         with pytest.raises(ValueError, match="one entry per tensor"):
             K.adamw_list(*args, 1e-2, 0.9, 0.95, 1e-8, 0.1, 3)
+
+
+# ---- loss without gradient ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V,cut", [(8, 0), (1000, 0), (4096, 8), (32000, 0), (16392, 3)])
+def test_loss_without_gradient_on_values_that_are_not_finite(K, V, cut, dtype):
+    """Row by row what the loss with gradient gives, NaN for NaN; -inf in a counted column is a probability of zero."""
+    print("ce loss, not finite", V, cut, dtype, flush=True)
+    nan, inf = float("nan"), float("inf")
+    rows = 10
+    logits = (torch.randn(rows, V, device="cuda", generator=torch.Generator(device="cuda").manual_seed(V)) * 4).to(dtype)
+    labels = torch.full((rows,), V - cut - 1, device="cuda")
+    logits[0, :8] = nan           # one vector of one thread, and nothing else of that thread if the row is short
+    logits[1] = nan
+    logits[2] = nan
+    labels[2] = V                 # (a label outside the vocabulary)
+    logits[3, V - cut - 1] = nan  # a single column, the last one
+    logits[4, :V // 2] = -inf     # finite
+    logits[5] = -inf
+    logits[6] = -inf
+    labels[6] = -1
+    logits[7, 0] = inf
+    logits[8, :8] = -inf
+    logits[8, 7] = nan
+    if V - cut - 1 > 8:
+        logits[9, 1:V - cut - 1] = -inf  # finite
+    if cut:
+        logits[9, V - cut:] = nan        # (columns that are cut off are not looked at)
+    weights = torch.ones(rows, device="cuda")
+    want, _ = K.ce_fused(logits.clone(), labels, weights, weights.sum().view(1), cut, inplace=True)
+    got = K.ce_loss(logits, labels, weights, cut)
+    print(got.tolist(), want.tolist(), flush=True)
+    assert torch.allclose(got, want, rtol=1e-6, atol=2e-6, equal_nan=True)
+    assert got[[0, 1, 2, 3, 8]].isnan().all()
