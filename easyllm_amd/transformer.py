@@ -286,8 +286,8 @@ class ParallelTransformerLayer(torch.nn.Module):
             mg = getattr(p, "main_grad", None)
             if mg is not None and not (mg.dtype is torch.float32 and mg.shape == p.shape and mg.is_contiguous()):
                 return None
-        if mlp.activation_func is not GLU_ACTIVATIONS["silu"] or not core.causal:
-            return None
+        if mlp.activation_func is not GLU_ACTIVATIONS["silu"] or not core.causal or (core.training and core.dropout_p != 0.0):
+            return None  # (the composed layer refuses what is not built)
         cos, sin = rotary.tables(s, hidden_states.device)
         if cu_seqlens is not None:
             cu_seqlens = cu_seqlens.view(-1).int()

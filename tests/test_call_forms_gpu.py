@@ -206,3 +206,15 @@ def test_loss_without_gradient_on_values_that_are_not_finite(K, V, cut, dtype):
     print(got.tolist(), want.tolist(), flush=True)
     assert torch.allclose(got, want, rtol=1e-6, atol=2e-6, equal_nan=True)
     assert got[[0, 1, 2, 3, 8]].isnan().all()
+
+
+# ---- parts of a layer that a native call must not pass by --------------------------------------------------------------
+def test_attention_dropout_is_refused_in_training():
+    model, (inputs, _) = small_model(), small_batch()
+    core = decoder_layer(model).self_attn.core_attention_flash
+    core.dropout_p = 0.1
+    with pytest.raises(NotImplementedError, match="dropout"):
+        model(inputs)
+    out = model.eval()(inputs)
+    core.dropout_p = 0.0
+    assert torch.equal(out, model(inputs))
