@@ -18,7 +18,7 @@ from .default_cfg import update_model_cfg
 from .layers import LayerSpec, build_layer_norm
 from .lm_head import EmbedddingPipeNoTied
 from .registry import LOSS_REGISTRY, MODULE_ZOO_REGISTRY
-from .transformer import ParallelTransformerLayerPipe, is_plain
+from .transformer import ParallelTransformerLayerPipe, is_plain, passed_by_when_plain
 from .word_embedings import EmbeddingPipe
 from . import losses as _losses  # noqa: F401  (registers 'softmax_cross_entropy')
 
@@ -181,6 +181,8 @@ class LlamaModelPipe(torch.nn.Module):
             specs.append(float16_to_fp32)
         return specs
 
+
+passed_by_when_plain(EmbedddingPipeNoTied, LlamaModelPipe)
 
 _LLAMA_MODELS = {
     "llama_7b": {"num_layers": 32, "hidden_size": 4096, "num_attention_heads": 32},

@@ -26,10 +26,41 @@ _POSITION_TYPES = ("rotary", "absolute", "alibi", "flash", "dynamicntk")
 _MASK_TYPES = ("causal", "padding", "prefix", "custom")
 
 
+_METHODS = {}  # class that a fast path may pass by -> ((name, method), ...) as defined
+_NAMES = {}    # ... -> names that its modules must not replace for themselves
+
+
+def passed_by_when_plain(*classes):
+    """Notes the methods of these classes, for is_plain to find a replaced one."""
+    for cls in classes:
+        names = {n for c in cls.__mro__ if c not in torch.nn.Module.__mro__ for n in vars(c) if n[:2] != "__"}
+        _METHODS[cls] = tuple((n, getattr(cls, n)) for n in sorted(names) if callable(getattr(cls, n)))
+        _NAMES[cls] = frozenset(n for n, _ in _METHODS[cls]) | {"_call_impl", "_compiled_call_impl"}
+
+
+def are_plain(pairs):
+    """(module, class) pairs: each exactly of its class, with no hook and no method replaced, on the module or on the class, that
+    passing its __call__ by would leave out."""
+    if torch.nn.modules.module._has_any_global_hook():
+        return False
+    classes = set()
+    for module, cls in pairs:
+        if type(module) is not cls:
+            return False
+        own = module.__dict__
+        if (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or not own.keys().isdisjoint(_NAMES[cls])):
+            return False
+        classes.add(cls)
+    for cls in classes:
+        for name, method in _METHODS[cls]:
+            if getattr(cls, name) is not method:
+                return False
+    return True
+
+
 def is_plain(module, cls):
-    """Exactly this class, with no hook or replaced forward that skipping its __call__ would leave out."""
-    return not (type(module) is not cls or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
-                or module._backward_pre_hooks or "forward" in module.__dict__ or torch.nn.modules.module._has_any_global_hook())
+    return are_plain(((module, cls),))
 
 
 class FlashAttention(torch.nn.Module):
@@ -272,11 +303,10 @@ class ParallelTransformerLayer(torch.nn.Module):
         s, b, h = hidden_states.shape
         if 2.0 * s * b * h * ((2 * nq + 2 * nk) * d + 3 * f) > self.native_call_flops or s * b == 0 or o.bias is not None:
             return None
-        for m, cls in ((attn, ParallelAttention), (mlp, ParallelMLP), (q, ColumnParallelLinear), (k, ColumnParallelLinear),
-                       (v, ColumnParallelLinear), (o, RowParallelLinear), (gate, ColumnParallelLinear), (up, ColumnParallelLinear),
-                       (down, RowParallelLinear), (ln1, RMSNorm), (ln2, RMSNorm), (core, FlashAttention), (rotary, RotaryEmbedding)):
-            if not is_plain(m, cls):
-                return None
+        if not are_plain(((attn, ParallelAttention), (mlp, ParallelMLP), (q, ColumnParallelLinear), (k, ColumnParallelLinear),
+                          (v, ColumnParallelLinear), (o, RowParallelLinear), (gate, ColumnParallelLinear), (up, ColumnParallelLinear),
+                          (down, RowParallelLinear), (ln1, RMSNorm), (ln2, RMSNorm), (core, FlashAttention), (rotary, RotaryEmbedding))):
+            return None
         params = (ln1.weight, q.weight, k.weight, v.weight, o.weight, ln2.weight, gate.weight, up.weight, down.weight)
         if q.bias is not None:
             params += (q.bias, k.bias, v.bias)
@@ -333,3 +363,6 @@ class ParallelTransformerLayerPipe(ParallelTransformerLayer):
             return super().forward(hidden_states, attention_mask, cu_seqlens, position_ids, **kwargs), attention_mask, \
                 cu_seqlens, position_ids
         raise RuntimeError("Received more inputs than understood.")
+
+
+passed_by_when_plain(RMSNorm, ColumnParallelLinear, RowParallelLinear, RotaryEmbedding, FlashAttention, ParallelMLP, ParallelAttention)

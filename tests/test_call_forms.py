@@ -67,3 +67,35 @@ def test_layer_gradients_that_share_memory_are_refused():
     grads[3].f32 = grads[2].f32 + 64 * 64 * 4 - 4  # v starts on the last element of k
     with pytest.raises(RuntimeError, match="share memory"):
         _lib.call("ezl_layer_bwd", ctypes.byref(layer), 256, 256, 256, 256, 256, grads, None)
+
+
+def test_a_module_with_replaced_parts_is_not_plain(monkeypatch):
+    from easyllm_amd import layers, transformer
+    linear = lambda: layers.ColumnParallelLinear(8, 8, bias=False, use_cpu_initialization=True, params_dtype=torch.bfloat16)
+    plain = lambda m, cls=layers.ColumnParallelLinear: transformer.is_plain(m, cls)
+    norm = layers.RMSNorm(False, 8)
+    assert plain(linear()) and plain(norm, layers.RMSNorm) and not plain(norm)
+    for name in ("forward", "_call_impl", "_compiled_call_impl"):
+        m = linear()
+        m.__dict__[name] = m.forward
+        assert not plain(m)
+    for name in ("forward_keep_input", "forward_with_residual"):
+        replaced = layers.RMSNorm(False, 8)
+        replaced.__dict__[name] = norm.forward
+        assert not plain(replaced, layers.RMSNorm)
+    m = linear()
+    handle = m.register_forward_hook(lambda *a: None)
+    assert not plain(m)
+    handle.remove()
+    assert plain(m)
+    monkeypatch.setattr(layers.ColumnParallelLinear, "forward", lambda self, x: (x, None))
+    assert not plain(m) and plain(norm, layers.RMSNorm)
+
+
+def test_a_replaced_loss_sees_the_logits_that_the_model_returns(monkeypatch):
+    from easyllm_amd import losses, runner
+    model = runner.build_model({"type": "llama_custom", "kwargs": dict(num_layers=1, hidden_size=64, num_attention_heads=1, intermediate_size=64,
+                                                                       vocab_size=64, seq_length=8, bf16=True)})
+    assert runner._logits_stay_inside(model)
+    monkeypatch.setattr(losses.CrossEntropy, "__call__", lambda self, output, labels: output.sum())
+    assert not runner._logits_stay_inside(model)

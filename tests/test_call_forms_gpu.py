@@ -218,3 +218,26 @@ def test_attention_dropout_is_refused_in_training():
     out = model.eval()(inputs)
     core.dropout_p = 0.0
     assert torch.equal(out, model(inputs))
+
+
+@pytest.mark.parametrize("part,method", [("input_layernorm", "forward_keep_input"), ("post_attention_layernorm", "forward_with_residual"),
+                                         ("self_attn.core_attention_flash", "forward_sb"), ("self_attn.rotary_emb", "tables"),
+                                         ("self_attn", "forward"), ("mlp", "forward"), ("mlp.down_proj", "forward")])
+@pytest.mark.parametrize("on_class", [False, True])
+def test_a_replaced_method_of_a_submodule_is_called(monkeypatch, part, method, on_class):
+    model, (inputs, _) = small_model(), small_batch()
+    want = model(inputs)
+    module = decoder_layer(model).get_submodule(part)
+    calls = []
+    original = getattr(type(module), method)
+    if on_class:
+        def replaced(self, *a, **kw):
+            calls.append(method)
+            return original(self, *a, **kw)
+        monkeypatch.setattr(type(module), method, replaced)
+    else:
+        def replaced(*a, **kw):
+            calls.append(method)
+            return original(module, *a, **kw)
+        monkeypatch.setattr(module, method, replaced)
+    assert torch.equal(model(inputs), want) and calls
