@@ -543,27 +543,29 @@ def vocab_parallel_cross_entropy(vocab_parallel_logits, target, cut_size=None):
 
 class FusedCrossEntropyLossFunction(torch.autograd.Function):
     """sum(loss_i * w_i) / sum(w), w = loss_mask * (label != -100), with d loss / d logits produced
-    in the same visit of the logits (written to a new buffer, or over the logits when `inplace`)."""
+    in the same visit of the logits (written to a new buffer, or over the logits when `inplace`).  Without `want_grad` nobody
+    will ask for it: the loss alone."""
 
     @staticmethod
-    def forward(ctx, logits, labels, loss_mask, cut_size, ignore_index, inplace):
+    def forward(ctx, logits, labels, loss_mask, cut_size, ignore_index, inplace, want_grad=True):
         logits = logits.contiguous()
         labels = labels.contiguous()
         weights, count = K.ce_prepare(labels, None if loss_mask is None else loss_mask.contiguous(), ignore_index)
+        if not want_grad:
+            return K.ce_reduce(K.ce_loss(logits, labels, weights, cut_size), weights, count)
         loss_rows, grad = K.ce_fused(logits, labels, weights, count, cut_size or 0, inplace=inplace)
         ctx.save_for_backward(grad)
         return K.ce_reduce(loss_rows, weights, count)
 
     @staticmethod
     def backward(ctx, grad_out):
+        if not ctx.saved_tensors:  # (only the mask asked for a gradient, and has none)
+            return (None,) * 7
         (grad,) = ctx.saved_tensors
         K.scale_by_scalar_(grad, grad_out.reshape(1).float().contiguous())
-        return grad, None, None, None, None, None
+        return grad, None, None, None, None, None, None
 
 
 def fused_cross_entropy_loss(logits, labels, loss_mask=None, cut_size=None, ignore_index=-100, inplace=False):
-    if not (torch.is_grad_enabled() and logits.requires_grad):  # nobody will ask for the gradient: the loss alone
-        logits, labels = logits.contiguous(), labels.contiguous()
-        weights, count = K.ce_prepare(labels, None if loss_mask is None else loss_mask.contiguous(), ignore_index)
-        return K.ce_reduce(K.ce_loss(logits, labels, weights, cut_size), weights, count)
-    return FusedCrossEntropyLossFunction.apply(logits, labels, loss_mask, cut_size, ignore_index, inplace)
+    return FusedCrossEntropyLossFunction.apply(logits, labels, loss_mask, cut_size, ignore_index, inplace,
+                                               torch.is_grad_enabled() and logits.requires_grad)

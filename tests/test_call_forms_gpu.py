@@ -241,3 +241,25 @@ def test_a_replaced_method_of_a_submodule_is_called(monkeypatch, part, method, o
             return original(module, *a, **kw)
         monkeypatch.setattr(module, method, replaced)
     assert torch.equal(model(inputs), want) and calls
+
+
+def test_forward_mode_through_the_fused_loss_is_refused():
+    """Also where no reverse-mode gradient is wanted: a tangent must not be dropped without a word."""
+    import torch.autograd.forward_ad as fwAD
+    from easyllm_amd import functional as F_
+    logits, labels = rnd(4, 64), torch.arange(4, device="cuda")
+    with fwAD.dual_level():
+        dual = fwAD.make_dual(logits, rnd(4, 64, seed=1))
+        with pytest.raises(RuntimeError, match="(?i)forward"):
+            F_.fused_cross_entropy_loss(dual, labels)
+
+
+def test_a_loss_of_which_only_the_mask_wants_a_gradient():
+    from easyllm_amd import functional as F_
+    mask = torch.ones(4, device="cuda", requires_grad=True)
+    logits, labels = rnd(4, 64), torch.arange(4, device="cuda")
+    loss = F_.fused_cross_entropy_loss(logits, labels, mask)
+    loss.backward()  # (the mask is not differentiated)
+    assert mask.grad is None
+    ref = torch.nn.functional.cross_entropy(logits.float(), labels)
+    assert abs(loss.item() - ref.item()) <= 1e-5 * ref.item()
