@@ -190,6 +190,12 @@ class ParallelAttention(torch.nn.Module):
             raise NotImplementedError("position_embedding_type=%r: the llama step uses 'rotary' (default_cfg.py:22)"
                                       % (position_embedding_type,))
 
+    @staticmethod
+    def _adds_all_biases(projections):
+        """Plain projections that each have a bias and add it themselves."""
+        return (are_plain([(p, ColumnParallelLinear) for p in projections])
+                and all(p.bias is not None and not p.skip_bias_add for p in projections))
+
     def forward(self, hidden_states, attention_mask, cu_seqlens=None, position_ids=None, layer_past=None,
                 get_key_value=False, alibi=None):
         # hidden_states [s, b, h]
@@ -200,7 +206,7 @@ class ParallelAttention(torch.nn.Module):
                                                                     self.v_proj.weight)
         elif not self.qkv_pack:
             projections = (self.q_proj, self.k_proj, self.v_proj)
-            if all(is_plain(p, ColumnParallelLinear) for p in projections):  # one launch where that is faster, one input gradient
+            if self._adds_all_biases(projections):  # one launch where that is faster, one input gradient
                 ys = F_.fan_out_linear(hidden_states, *(p.weight for p in projections))
                 query_layer, key_layer, value_layer = (F_.bias_add(y, p.bias) for y, p in zip(ys, projections))
             else:
@@ -290,7 +296,7 @@ class ParallelTransformerLayer(torch.nn.Module):
         code) exceeds the kernels' own time: two layers at h = 256 on 1024 tokens, forward + loss + backward, 1.6 ms of which
         0.57 are kernels.  1e12 FLOPs are 0.8 ms of kernels, where the host is ahead either way; larger layers keep the
         composed form, whose activations and gradients are freed one by one.  Only the plain layer qualifies: its own
-        submodules, unhooked, separate q / k / v projections, no o bias, no key padding mask."""
+        submodules, unhooked, separate q / k / v projections with all biases or none, no o or down bias, no key padding mask."""
         attn, mlp = self.self_attn, self.mlp
         if (type(attn) is not ParallelAttention or type(mlp) is not ParallelMLP or attn.qkv_pack or self.apply_residual_connection_post_layernorm
                 or (attention_mask is not None and cu_seqlens is None) or not hidden_states.is_cuda
@@ -301,7 +307,7 @@ class ParallelTransformerLayer(torch.nn.Module):
         nq, nk = attn.num_attention_heads_per_partition, attn.num_kv_attention_heads_per_partition
         d, f = attn.hidden_size_per_attention_head, gate.weight.shape[0]
         s, b, h = hidden_states.shape
-        if 2.0 * s * b * h * ((2 * nq + 2 * nk) * d + 3 * f) > self.native_call_flops or s * b == 0 or o.bias is not None:
+        if 2.0 * s * b * h * ((2 * nq + 2 * nk) * d + 3 * f) > self.native_call_flops or s * b == 0 or o.bias is not None or down.bias is not None:
             return None
         if not are_plain(((attn, ParallelAttention), (mlp, ParallelMLP), (q, ColumnParallelLinear), (k, ColumnParallelLinear),
                           (v, ColumnParallelLinear), (o, RowParallelLinear), (gate, ColumnParallelLinear), (up, ColumnParallelLinear),
@@ -309,6 +315,8 @@ class ParallelTransformerLayer(torch.nn.Module):
             return None
         params = (ln1.weight, q.weight, k.weight, v.weight, o.weight, ln2.weight, gate.weight, up.weight, down.weight)
         if q.bias is not None:
+            if not attn._adds_all_biases((q, k, v)):
+                return None
             params += (q.bias, k.bias, v.bias)
         for p in params:
             if p.dtype is not torch.bfloat16 or not p.is_contiguous() or not p.is_cuda:

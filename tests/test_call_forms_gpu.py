@@ -263,3 +263,52 @@ def test_a_loss_of_which_only_the_mask_wants_a_gradient():
     assert mask.grad is None
     ref = torch.nn.functional.cross_entropy(logits.float(), labels)
     assert abs(loss.item() - ref.item()) <= 1e-5 * ref.item()
+
+
+@pytest.mark.parametrize("without", [("k_proj",), ("k_proj", "v_proj")])
+@pytest.mark.parametrize("flops", [1e12, 0.0])
+def test_projections_of_which_some_have_no_bias(without, flops):
+    """As with biases of zero there (the sum with a zero bias is exact)."""
+    results = []
+    for removed in (True, False):
+        model, batch = small_model(transformer_layer_params={"attention_qkv_bias": True}), small_batch()
+        layer = decoder_layer(model)
+        layer.native_call_flops = flops
+        for name in without:
+            proj = layer.self_attn.get_submodule(name)
+            if removed:
+                proj.bias = None
+            else:
+                with torch.no_grad():
+                    proj.bias.zero_()
+        out = model(batch[0])
+        loss = model.loss_fn(out, batch[1])
+        loss.backward()
+        results.append((out, loss, {n: p.grad.float() for n, p in model.named_parameters()}))
+    (out1, loss1, g1), (out0, loss0, g0) = results
+    assert torch.equal(out1, out0) and torch.equal(loss1, loss0) and set(g0) - set(g1) == {n for n in g0 if n.split(".")[-2] in without and n.endswith("bias")}
+    for n in g1:  # (the input gradient of three separate projections is added in bf16: a rounding or two)
+        assert (g1[n] - g0[n]).norm() <= 2e-2 * g0[n].norm(), n
+
+
+def test_a_projection_that_leaves_its_bias_to_the_caller():
+    """skip_bias_add: the projection's bias is not added by it, and the attention drops what it returns beside its result."""
+    model, (inputs, _) = small_model(transformer_layer_params={"attention_qkv_bias": True}), small_batch()
+    k = decoder_layer(model).self_attn.k_proj
+    k.skip_bias_add = True
+    out = model(inputs)
+    k.skip_bias_add = False
+    with torch.no_grad():
+        k.bias.zero_()
+    assert torch.equal(out, model(inputs))
+
+
+def test_a_down_projection_with_a_bias_of_its_own():
+    model, (inputs, _) = small_model(), small_batch()
+    down = decoder_layer(model).mlp.down_proj
+    down.bias, down.skip_bias_add = torch.nn.Parameter(rnd(256, seed=5)), False
+    out = model(inputs)
+    decoder_layer(model).native_call_flops = 0.0
+    assert torch.equal(out, model(inputs))
+    down.bias = None
+    assert not torch.equal(out, model(inputs))
