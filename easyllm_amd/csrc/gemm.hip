@@ -830,6 +830,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
                                     const int64_t* K, int64_t lda, int64_t ldb, int64_t ldc, int a_kc, int b_kc, int out_dtype,
                                     int accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
     EZL_REQUIRE(count >= 1 && A && B && K, EZL_EINVAL, "ezl_gemm_bf16_ksplit: bad count or null argument array");
+    accumulate = accumulate ? 1 : 0;  // (the kernels take a bit field)
     bool one_launch = count <= 3 && a_kc == 1 && b_kc == 0 && out_dtype == 0 && M > 0 && N > 0, tail = false;
     int64_t ktot = 0;
     for (int i = 0; i < count; ++i) {
@@ -947,7 +948,7 @@ extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* 
         if (const int rc = check_operands(A[i], B[i], M[i], N[i], K, lda[i], ldb[i], ldc[i], a_kc, b_kc)) return rc;
         // (rows of C too far apart for the smaller tiles' stores: ezl_gemm_bf16 has kernels for them)
         apart = apart || !(out_dtype == 0 ? small_stores_ok<bf16_t>(ldc[i]) : small_stores_ok<float>(ldc[i]));
-        a.p[i] = {(const bf16_t*)A[i], (const bf16_t*)B[i], C[i], lda[i], ldb[i], ldc[i], (int)M[i], (int)N[i], 0, 0, 0, accumulate[i]};
+        a.p[i] = {(const bf16_t*)A[i], (const bf16_t*)B[i], C[i], lda[i], ldb[i], ldc[i], (int)M[i], (int)N[i], 0, 0, 0, accumulate[i] ? 1 : 0};
         tiles += tiles_of(kTile64, M[i], N[i]);
     }
     EZL_REQUIRE(tiles < (1LL << 27), EZL_EUNSUPPORTED, "ezl_gemm_bf16_group: too many tiles");

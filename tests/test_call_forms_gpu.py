@@ -312,3 +312,40 @@ def test_a_down_projection_with_a_bias_of_its_own():
     assert torch.equal(out, model(inputs))
     down.bias = None
     assert not torch.equal(out, model(inputs))
+
+
+# ---- C entries ---------------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("flag", [1, 2, -1, 3])
+@pytest.mark.parametrize("entry,T,n_in,outs", [("ksplit", 1024, 256, (256, 64)), ("ksplit", 4096, 5120, (4096, 1024)), ("ksplit", 300, 264, (256,)),
+                                               ("group", 1024, 256, (256, 64)), ("group", 9000, 256, (256, 512)), ("single", 1024, 256, (256,))])
+def test_any_nonzero_accumulate_flag_adds(K, entry, T, n_in, outs, flag):
+    from easyllm_amd import _lib
+    print("accumulate", entry, T, n_in, outs, flag, flush=True)
+    n = len(outs)
+    vp, i64 = ctypes.c_void_p * n, ctypes.c_int64 * n
+    ptr = lambda ts: vp(*[t.data_ptr() for t in ts])
+    ld = max(outs)
+    dys = [torch.empty(T, ld, device="cuda", dtype=torch.bfloat16)[:, :o].copy_(rnd(T, o, seed=i)) for i, o in enumerate(outs)]
+    ws = torch.empty(64 << 20, device="cuda", dtype=torch.uint8)
+    if entry == "ksplit":
+        weights = [rnd(o, n_in, seed=9 + i) for i, o in enumerate(outs)]
+        out = [torch.full((T, n_in), 3.0, device="cuda", dtype=torch.bfloat16)]
+        _lib.call("ezl_gemm_bf16_ksplit", n, ptr(dys), ptr(weights), out[0].data_ptr(), T, n_in, i64(*outs), ld, n_in, n_in, 1, 0, 0, flag,
+                  ws.data_ptr(), ws.numel(), None)
+        torch.cuda.synchronize()
+        ref = [3.0 + sum(dy.float() @ w.float() for dy, w in zip(dys, weights))]
+        bound = [sum(product_bound(dy, w) for dy, w in zip(dys, weights)) + ref[0].abs() * 2.0 ** -8 + 1e-5]
+    else:
+        x = rnd(T, n_in, seed=9)
+        out = [torch.full((o, n_in), 3.0, device="cuda") for o in outs]
+        if entry == "group":
+            _lib.call("ezl_gemm_bf16_group", n, ptr(dys), vp(*[x.data_ptr()] * n), ptr(out), i64(*outs), i64(*[n_in] * n), T, i64(*[ld] * n),
+                      i64(*[n_in] * n), i64(*[n_in] * n), 0, 0, 1, (ctypes.c_int * n)(*[flag] * n), ws.data_ptr(), ws.numel(), None)
+        else:
+            _lib.call("ezl_gemm_bf16", dys[0].data_ptr(), x.data_ptr(), out[0].data_ptr(), outs[0], n_in, T, ld, n_in, n_in, 0, 0, 1, flag,
+                      ws.data_ptr(), ws.numel(), None)
+        torch.cuda.synchronize()
+        ref = [3.0 + dy.float().t() @ x.float() for dy in dys]
+        bound = [product_bound(dy.t(), x) + r.abs() * 2.0 ** -20 + 1e-5 for dy, r in zip(dys, ref)]
+    for o, r, tol in zip(out, ref, bound):
+        assert ((o.float() - r).abs() <= tol).all()
