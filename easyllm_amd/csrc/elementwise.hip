@@ -259,70 +259,112 @@ __global__ __launch_bounds__(kBlock) void zero_f32x4_kernel(f32x4* __restrict__ 
     }
 }
 
-// overwrite: dW[id] = sum instead of dW[id] += sum, and the rows of ids that do not occur are zero-filled (the whole
-// [V, h] gradient is then defined by this launch: no separate fill pass).
-constexpr int kWindowRows = 2048;  // a frequent id's rows are put in order through a bitmap over this many row numbers
+// What putting the rows of a frequent id in order needs of LDS.
+constexpr int kListRows = 2048;               // rows in order at a time
+constexpr int kWindowWords = 2048;            // words of the bitmap over row numbers
+constexpr int kWindowRows = 32 * kWindowWords;
+constexpr int kFrequentBlocks = 1024;         // 512: each of 3971 ids 33 times, h = 4096, 448 us instead of 341
+struct EmbedOrder {
+    alignas(16) int list[kListRows];
+    int raw[kBlock];
+    unsigned bits[kWindowWords];
+    int wave_total[kBlock / 64];
+};
 
 // One frequent id, columns col0 + 2 thread, + 1: a thread walks the id's rows in order with up to 24 rows' loads in flight (one
 // register each), so that the time is the latency of n / 24 loads rather than of n / 4.  (1000 padding rows of 4000, h = 2048:
 // the scatter kernel 430 -> 79 us.)
+// Every slice of the columns puts the rows in order for itself, which must not cost more than adding them: up to one row per thread
+// by rank, whatever the batch; more through a bitmap over 65536 row numbers at a time.  The whole gradient, added to a buffer, of
+// T rows of 4096 by one block per id, by column slices over bitmap windows of 2048 rows, and so: T = 131072, each id 33 times
+// 334, 3473, 340 us; 300 times 474, 1043, 310; 3000 times 3335, 922, 636; T = 16384, ids by Zipf's law 950, 164, 148.
 template <typename OutT>
 __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY, OutT* __restrict__ dW, const int* __restrict__ mine, int n,
-                                                  int64_t id, int col0, int64_t rows, int h, int overwrite, int* list, unsigned* bits, int& wtot) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int col = col0 + 2 * threadIdx.x;
+                                                  int64_t id, int col0, int64_t rows, int h, int overwrite, EmbedOrder& o) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int col = col0 + 2 * tid;
     const bool live = col < h;
     const int lane_col = live ? col : 0;
     float a0 = 0.f, a1 = 0.f;
-    // rows are put in order a window at a time: every lane of the first wave owns one 32-row word of a bitmap, counts its bits,
-    // and after a scan over the wave writes its rows into the ordered list
-    for (int64_t w0 = 0; w0 < rows; w0 += kWindowRows) {
+    for (int64_t w0 = 0; w0 < rows; w0 += n <= kBlock ? rows : kWindowRows) {
         __syncthreads();  // the previous window's (or id's) LDS use is over
-        if (threadIdx.x < 64) bits[threadIdx.x] = 0u;
-        __syncthreads();
-        for (int i = threadIdx.x; i < n; i += kBlock) {
-            const int64_t r = (int64_t)mine[i] - w0;
-            if (r >= 0 && r < kWindowRows) atomicOr(&bits[r >> 5], 1u << (r & 31));
+        int m = 0;  // rows of the window
+        // a thread owns `per` consecutive words of the bitmap; their bits, counted and scanned over the block, say where its rows go
+        const int words = rows - w0 < kWindowRows ? (int)((rows - w0 + 31) >> 5) : kWindowWords, per = (words + kBlock - 1) / kBlock;
+        const int last = (tid + 1) * per < words ? (tid + 1) * per : words;
+        if (n <= kBlock) {  // rows are distinct: rank = number of smaller rows
+            const int v = tid < n ? mine[tid] : 0x7fffffff;
+            o.raw[tid] = v;
+            __syncthreads();
+            int rank = 0;
+            for (int j = 0; j < n; ++j) rank += o.raw[j] < v;
+            if (tid < n) o.list[rank] = v;
+            m = n;
+        } else {
+            for (int i = tid; i < words; i += kBlock) o.bits[i] = 0u;
+            __syncthreads();
+            for (int i = tid; i < n; i += kBlock) {
+                const int64_t r = (int64_t)mine[i] - w0;
+                if (r >= 0 && r < kWindowRows) atomicOr(&o.bits[r >> 5], 1u << (r & 31));
+            }
+            __syncthreads();
+            int count = 0;
+            for (int i = tid * per; i < last; ++i) count += __builtin_popcount(o.bits[i]);
+            int end = count;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int v = __shfl_up(end, d, 64);
+                if (lane >= d) end += v;
+            }
+            if (lane == 63) o.wave_total[wv] = end;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kBlock / 64; ++i) {
+                if (i < wv) end += o.wave_total[i];
+                m += o.wave_total[i];
+            }
+            m = __builtin_amdgcn_readfirstlane(m);
+            o.raw[tid] = end - count;  // (not a register each while rows are added)
         }
-        __syncthreads();
-        if (wv == 0) {
-            unsigned m = bits[lane];
-            const int mine_n = __builtin_popcount(m);
-            int incl = mine_n;
+        for (int at = 0; at < m; at += kListRows) {
+            if (at) __syncthreads();  // the rows before these are added
+            if (n > kBlock) {
+                int q = o.raw[tid] - at;
+                for (int i = tid * per; i < last && q < kListRows; ++i) {
+                    unsigned w = o.bits[i];
+                    if (q + 32 <= 0) {
+                        q += __builtin_popcount(w);
+                        continue;
+                    }
+                    for (; w; w &= w - 1, ++q)
+                        if (q >= 0 && q < kListRows) o.list[q] = (int)w0 + 32 * i + __builtin_ctz(w);
+                }
+            }
+            __syncthreads();
+            const int listed = m - at < kListRows ? m - at : kListRows;
+            int i = 0;
+            auto batch = [&](auto N) {
+                constexpr int U = decltype(N)::value;
+                for (; i + U <= listed; i += U) {
+                    bf16x2 v[U];
+                    int at_row[U];
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(incl, o, 64);
-                if (lane >= o) incl += v;
-            }
-            if (lane == 63) wtot = incl;
-            int pos = incl - mine_n;
-            while (m) {
-                list[pos++] = (int)w0 + 32 * lane + __builtin_ctz(m);
-                m &= m - 1;
-            }
+                    for (int u = 0; u < U; ++u) at_row[u] = __builtin_amdgcn_readfirstlane(o.list[i + u]);
+#pragma unroll
+                    for (int u = 0; u < U; ++u)  // (scalar row address + one lane offset: no address registers per row)
+                        v[u] = reinterpret_cast<const bf16x2*>(dY + (int64_t)at_row[u] * h)[lane_col >> 1];
+                    __builtin_amdgcn_sched_barrier(0);  // (or the loads are waited for one by one to save registers: 1000 rows 264 us)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        a0 += (float)v[u][0];
+                        a1 += (float)v[u][1];
+                    }
+                }
+            };
+            batch(std::integral_constant<int, 24>{});
+            batch(std::integral_constant<int, 4>{});
+            batch(std::integral_constant<int, 1>{});
         }
-        __syncthreads();
-        const int m = wtot;
-        int i = 0;
-        auto batch = [&](auto N) {
-            constexpr int U = decltype(N)::value;
-            for (; i + U <= m; i += U) {
-                bf16x2 v[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {  // (scalar row offset + one lane offset: no address registers per row)
-                    const int64_t row = __builtin_amdgcn_readfirstlane(list[i + u]);
-                    v[u] = *reinterpret_cast<const bf16x2*>(dY + row * h + lane_col);
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    a0 += (float)v[u][0];
-                    a1 += (float)v[u][1];
-                }
-            }
-        };
-        batch(std::integral_constant<int, 24>{});
-        batch(std::integral_constant<int, 4>{});
-        batch(std::integral_constant<int, 1>{});
     }
     if (!live) return;
     if constexpr (sizeof(OutT) == 2) {
@@ -339,6 +381,8 @@ __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY,
     }
 }
 
+// overwrite: dW[id] = sum instead of dW[id] += sum, and the rows of ids that do not occur are zero-filled (the whole
+// [V, h] gradient is then defined by this launch: no separate fill pass).
 // (rows of up to 4096: six waves per SIMD, as the zero fill wants them)
 // OutT bf16: the fp32 sums are rounded once as they are stored.  A gradient without an fp32 buffer behind it used to be written in
 // fp32, read by a cast and written again, five times the bytes of the result.  Gradient
@@ -351,19 +395,15 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
                                                                       const int* __restrict__ bucket, const int* __restrict__ cursor,
                                                                       const int* __restrict__ heavy, int64_t rows, int h, int64_t V,
                                                                       int overwrite) {
-    static_assert(kWindowRows == 32 * 64, "one bitmap word per lane of the first wave");
-    __shared__ int list[kWindowRows];  // rows of the current id in increasing order
-    __shared__ int raw[kBlock];
-    __shared__ unsigned bits[64];
-    __shared__ int wtot;
-    int* sorted = list;
+    __shared__ EmbedOrder order;
+    int *const raw = order.raw, *const sorted = order.list;  // rows of the current id as they are found, and in increasing order
     const int h8 = h >> 3;
-    const int helpers = (int)gridDim.x < 512 ? (int)gridDim.x : 512;
+    const int helpers = (int)gridDim.x < kFrequentBlocks ? (int)gridDim.x : kFrequentBlocks;
     if ((int)blockIdx.x < helpers) {  // the frequent ids first, as they take longest; the other blocks need not even look
         const int slices = (h + 2 * kBlock - 1) / (2 * kBlock), items = cursor[1] * slices;
         for (int it = blockIdx.x; it < items; it += helpers) {
             const int id = heavy[it / slices];
-            embed_frequent_id(dY, dW, bucket + off[id], cnt[id], id, (it % slices) * 2 * kBlock, rows, h, overwrite, list, bits, wtot);
+            embed_frequent_id(dY, dW, bucket + off[id], cnt[id], id, (it % slices) * 2 * kBlock, rows, h, overwrite, order);
         }
         __syncthreads();
     }

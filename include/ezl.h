@@ -86,7 +86,8 @@ int ezl_rope_apply_pair(const void* q, void* q_out, int64_t nq, int64_t q_in_str
  * scatter_add: dweight_f32[id] (+)= sum of dy[r] over rows with ids[r] == id, fp32, added in increasing row order whatever
  * the launch does (bit-reproducible).  accumulate != 0 adds to what the buffer holds; accumulate == 0 overwrites it and
  * zero-fills the rows of ids that do not occur, so the whole [vocab, h] gradient is written by the call.  Work is linear
- * in `rows`; an id that occurs n > 32 times is summed in n consecutive row visits by h / 512 workgroups.  workspace:
+ * in `rows` for batches of up to 65536; an id that occurs n > 32 times is summed in n consecutive row visits by h / 512 workgroups,
+ * which for n > 256 look through the id's rows once per 65536 rows of the batch.  workspace:
  * ezl_embed_scatter_add_workspace_bytes(rows, vocab) bytes of device memory, 4-byte aligned, contents irrelevant before
  * and after. */
 int ezl_embed_gather(const void* ids, const void* weight, void* out, void* bad_flag, int64_t rows, int64_t h, int64_t vocab,

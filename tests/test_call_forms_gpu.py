@@ -349,3 +349,32 @@ def test_any_nonzero_accumulate_flag_adds(K, entry, T, n_in, outs, flag):
         bound = [product_bound(dy.t(), x) + r.abs() * 2.0 ** -20 + 1e-5 for dy, r in zip(dys, ref)]
     for o, r, tol in zip(out, ref, bound):
         assert ((o.float() - r).abs() <= tol).all()
+
+
+# ---- embedding gradient ------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("V,h,rows,counts", [
+    (500, 64, 5000, (33, 256, 257, 1024, 1025, 2000)),      # ids on both sides of every limit of the ordering
+    (40, 520, 9000, (2048, 2049, 3000, 40)),                # more rows of one id than the ordered list holds
+    (300, 8, 140000, (33, 300, 2048, 65536, 60000)),        # several bitmap windows, full and nearly empty ones
+    (3, 16, 65537, (65536,)), (2, 8, 131072, (131071, 1))])
+def test_embedding_gradient_with_frequent_ids(K, V, h, rows, counts, accumulate):
+    """Against the same sums taken in row order one row at a time (fp32, in the given order: bit for bit)."""
+    print("embedding gradient, frequent ids", V, h, rows, counts, accumulate, flush=True)
+    g = torch.Generator().manual_seed(rows)
+    ids = torch.randint(len(counts), max(V, len(counts) + 1), (rows,), generator=g)
+    where = torch.randperm(rows, generator=g)
+    at = 0
+    for i, n in enumerate(counts):
+        ids[where[at:at + n]] = i
+        at += n
+    dy = torch.randn(rows, h, generator=g).bfloat16()
+    old = torch.randn(V, h, generator=g)
+    ref = torch.zeros(V, h)
+    for i in ids.unique().tolist():
+        ref[i] = torch.from_numpy(dy[ids == i].float().numpy().cumsum(axis=0, dtype="float32")[-1])
+    out = old.cuda()
+    K.embed_scatter_add(ids.cuda(), dy.cuda(), out, accumulate=accumulate)
+    assert torch.equal(out.cpu(), ref + old if accumulate else ref)
+    if not accumulate:
+        assert torch.equal(K.embed_grad_bf16(ids.cuda(), dy.cuda(), V).cpu(), ref.bfloat16())
