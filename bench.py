@@ -180,7 +180,8 @@ def measure(name, steps, warmup, mode, input_check):
     median_ms = per_step[len(per_step) // 2] if len(per_step) % 2 else 0.5 * (per_step[len(per_step) // 2 - 1] + per_step[len(per_step) // 2])
 
     # Second pass of the same K steps with every GEMM launch bracketed by two timing events on the launch stream.  The
-    # events serialise the queue (about 20 us per launch), so they are kept out of the pass that `value` comes from.
+    # events serialise the queue (about 20 us per launch), so they are kept out of the pass that `value` comes from; the GEMM's
+    # share is its share of this second pass.
     for m in model.modules():  # small layers launch from one native call, where no launch can be bracketed
         if hasattr(m, "native_call_flops"):
             m.native_call_flops = 0.0
@@ -200,7 +201,7 @@ def measure(name, steps, warmup, mode, input_check):
                tok_s=tokens_per_step * steps / elapsed, tflops=flops * steps / elapsed / 1e12,
                recomputed_layers=model.recompute_count, gemm_launches=len(timing) // max(steps, 1),
                gemm_tflops=gemm_flops / (gemm_ms * 1e-3) / 1e12 if gemm_ms > 0 else 0.0,
-               gemm_avg_launch_us=gemm_ms * 1e3 / max(len(timing), 1), gemm_share=gemm_ms / steps / ms_per_step,
+               gemm_avg_launch_us=gemm_ms * 1e3 / max(len(timing), 1), gemm_share=gemm_ms * 1e-3 / elapsed_instrumented,
                instrumented_ms_per_step=elapsed_instrumented / steps * 1e3)
     return fig, model
 
