@@ -352,6 +352,23 @@ def test_any_nonzero_accumulate_flag_adds(K, entry, T, n_in, outs, flag):
 
 
 # ---- embedding gradient ------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("T,K_,outs", [(1024, 256, (256, 256, 256)), (17, 264, (8, 1000, 72)), (389, 2056, (768, 264)), (300, 5000, (128, 64))])
+def test_input_gradients_in_one_launch(K, T, K_, outs):
+    """The form of the group call that no wrapper uses: dy_i[T, K] w_i[K, n_i] in bf16, accumulation per product."""
+    print("gemm group input gradients", T, K_, outs, flush=True)
+    from easyllm_amd import _lib
+    n = len(outs)
+    nbytes = _lib.gemm_group_workspace_bytes((T,) * n, outs, K_)
+    assert nbytes >= 0
+    dys, ws = [rnd(T, K_, seed=i) for i in range(n)], [rnd(K_, o, seed=10 + i) for i, o in enumerate(outs)]
+    dxs = [torch.full((T, o), 3.0, device="cuda", dtype=torch.bfloat16) for o in outs]
+    accs = [i % 2 for i in range(n)]
+    K.gemm_group(dys, ws, (T,) * n, outs, K_, [K_] * n, outs, True, False, dxs, accs, nbytes)
+    for dx, dy, w, acc in zip(dxs, dys, ws, accs):
+        ref = dy.float() @ w.float() + 3.0 * acc
+        assert ((dx.float() - ref).abs() <= product_bound(dy, w) + ref.abs() * 2.0 ** -8 + 1e-6).all()
+
+
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("V,h,rows,counts", [
     (500, 64, 5000, (33, 256, 257, 1024, 1025, 2000)),      # ids on both sides of every limit of the ordering
