@@ -2,8 +2,8 @@
 // narrow layers, weight gradients of narrow layers.  Same operand forms, LDS layouts and fragments.
 //
 // What a tile shape costs: the CU's address unit takes 16 cycles per 1 KiB wave load, so a 64-wide K tile of the operands
-// takes 16 (BM + BN) / 8 cycles to fetch and BM BN / 64 cycles of MFMA (16x16x32, 16 cycles each, four SIMDs).  256 x 256:
-// 1024 against 4096 / 4 = 1024 per SIMD pair; 256 x 128: 768 against 1024; 128 x 128: 512 against 512; 64 x 64: 256 against 128.
+// takes 16 (BM + BN) / 8 cycles to fetch and BM BN / 32 cycles of MFMA (16x16x32, 16 cycles each, four SIMDs).  256 x 256:
+// 1024 against 2048; 256 x 128: 768 against 1024; 128 x 128: 512 against 512; 64 x 64: 256 against 128.
 // The smaller the tile, the more the fetch binds; what it buys is workgroups.
 #include "gemm_tile.h"
 
