@@ -617,16 +617,20 @@ int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const i
 // Products that share a reduction length (q / k / v or gate / up of one input, and their weight gradients) in one launch?  Worth
 // it where each of them leaves CUs idle: 1024 tokens at h = 256, q + k + v forward 3 x 4.7 us alone.  The launches of a long
 // batch fill the chip one by one, with the better 256 x 256 tiles (at 4096 tokens and h = 4096 one launch for q / k / v
-// measured 0.14 ms per four-layer step slower).  The estimate flatters the one launch where the products are long, so there it has
-// to win by a tenth.  Estimated ratio -> measured time apart and together, us (T tokens, width / widths; f forward, w weight gradient):
-//   apart under 115 us      f 3072, 2048 / 3 x 2048 0.99 -> 98, 91; f 1024, 2048 / 2 x 5504 1.00 -> 61, 57; f 1531, 1024 / 2 x 2816 0.93 ->
-//                           37, 31; w 512, 8192 / 8192, 2 x 1024 0.96 -> 145, 134; f 8192, 1024 / 2 x 2816 0.98 -> 115, 104
-//   longer, 0.9 and below   f 2048, 4096 / 4096, 2 x 1024 0.86 -> 114, 104; w 6144, 2048 / 3 x 2048 0.85 -> 173, 158; f 2048, 5120 / 3 x 5120
-//                           0.81 -> 300, 286; w 8192, 2048 / 2 x 5504 0.90 -> 361, 337; at worst f 1024, 4096 / 2 x 11008 0.88 -> 162, 169
-//   longer, above 0.9       f 3072, 2048 / 2 x 5504 0.91 -> 140, 154; f 6144, 2048 / 2 x 5504 0.98 -> 234, 281; f 4096, 5120 / 3 x 5120 1.00 ->
-//                           537, 551; w the same 0.98 -> 577, 595; at best f 3072, 8192 / 8192, 2 x 1024 0.93 -> 462, 429
+// measured 0.14 ms per four-layer step slower).  Between launches of the smaller tiles the estimates compare well; against the 256 x 256
+// kernels they flatter the one launch, which has to win by a tenth where each product alone takes those.  Estimated ratio -> measured
+// time apart and together, us (T tokens, width / widths; f forward, w weight gradient):
+//   smaller tiles alone     f 3072, 8192 / 8192, 2 x 1024 0.93 -> 462, 429; w 512, 8192 / 8192, 2 x 1024 0.96 -> 145, 134; f 8192, 1024 /
+//                           2 x 2816 0.98 -> 115, 104; w 1378, 4608 / 2 x 12288 0.99 -> 380, 370; at worst w 9200, 2048 / 3 x 2048 0.94 ->
+//                           242, 254
+//   256 x 256, to 0.9       f 2048, 5120 / 3 x 5120 0.81 -> 300, 286; w 14955, 3200 / 3 x 3200 0.82 -> 1028, 960; w 8192, 2048 / 2 x 5504
+//                           0.90 -> 361, 337; at worst w 2792, 1664 / 2 x 5504 0.86 -> 126, 132
+//   256 x 256, above        f 3072, 2048 / 2 x 5504 0.91 -> 140, 154; f 3600, 3072 / 3 x 3072 0.96 -> 188, 209; f 4797, 1664 / 2 x 5792 0.99 ->
+//                           151, 184; f 4096, 5120 / 3 x 5120 1.00 -> 537, 551; at best f 270, 7552 / 2 x 23872 0.91 -> 365, 330
+// Over 220 groups of widths 256 - 8192 and 256 - 16384 tokens with ratios of 0.72 - 1.08: 0.27 % behind the faster of the two on
+// average; by any estimated gain 0.74 %, by any gain where the products apart take under 115 us and a tenth above 0.65 %.
 constexpr double kLaunchGap = 2.5;  // us between two launches of a stream: ramp down, ramp up
-constexpr double kShortApart = 115, kLongMargin = 0.9;
+constexpr double kMargin256 = 0.9;
 bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
     struct Entry {
         int64_t M[kMaxProblems], N[kMaxProblems], K, room;
@@ -643,15 +647,16 @@ bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_
     if (!same) {
         const int64_t nk = (K + BK - 1) / BK;
         double apart = kLaunchGap * (count - 1), together;
+        bool all_256 = true;
         for (int i = 0; i < count; ++i) {
             double t;
-            find_plan(1, &M[i], &N[i], nk, room, &t);
+            all_256 = find_plan(1, &M[i], &N[i], nk, room, &t).kind == kTile256 && all_256;
             apart += t;
             e.M[i] = M[i];
             e.N[i] = N[i];
         }
         e.plan = find_plan(count, M, N, nk, room, &together);
-        e.one = together < (apart < kShortApart ? apart : kLongMargin * apart);
+        e.one = together < (all_256 ? kMargin256 * apart : apart);
         e.K = K;
         e.room = room;
         e.count = count;

@@ -103,8 +103,9 @@ def test_a_replaced_loss_sees_the_logits_that_the_model_returns(monkeypatch):
 
 @pytest.mark.parametrize("T,h,outs,forward,weight_gradient", [
     (1024, 256, (256, 256, 256), True, True), (3072, 2048, (2048, 2048, 2048), True, True), (2048, 4096, (4096, 1024, 1024), True, True),
-    (4096, 5120, (5120, 5120, 5120), False, False), (4096, 4096, (4096, 4096, 4096), False, False), (6144, 2048, (5504, 5504), False, True)])
-def test_long_products_share_a_launch_only_by_a_margin(T, h, outs, forward, weight_gradient):
+    (4096, 5120, (5120, 5120, 5120), False, False), (4096, 4096, (4096, 4096, 4096), False, False), (6144, 2048, (5504, 5504), False, True),
+    (1378, 4608, (12288, 12288), False, True), (3600, 3072, (3072, 3072, 3072), False, True)])
+def test_products_of_256_tiles_share_a_launch_only_by_a_margin(T, h, outs, forward, weight_gradient):
     n = len(outs)
     assert (_lib.gemm_group_workspace_bytes((T,) * n, outs, h) >= 0) == forward
     assert (_lib.gemm_group_workspace_bytes(outs, (h,) * n, T) >= 0) == weight_gradient
