@@ -154,8 +154,9 @@ __global__ __launch_bounds__(kOptBlock) void sumsq_list_kernel(const TensorList 
 __device__ __forceinline__ f32x4 ld_stream(const float* p, int i) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + i); }
 __device__ __forceinline__ void st_stream(float* p, int i, f32x4 x) { __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(p) + i); }
 
-// Bound by HBM: 30 B per parameter.  465 M parameters, norm + update: 3.30 ms with one launch per tensor and two vectors in
-// flight per stream (4.8 TB/s), 2.71 with this (5.8), 2.67 with the streaming hint (5.9); 1024 or 4096 blocks are no different.
+// Bound by HBM: 30 B per parameter, 4 more for the norm.  465 M parameters, norm + update: 3.39 - 3.51 ms with one launch per tensor
+// and two vectors in flight per stream, 3.15 with this, 3.13 - 3.10 with the streaming hint (5.1 TB/s: the update 2.75 ms, the norm
+// 0.37); a training iteration of 63 M parameters 3.06 -> 2.96 ms by the hint.  1024 or 4096 blocks are no different.
 __global__ __launch_bounds__(kOptBlock) void adamw_list_kernel(const TensorList l, const AdamArgs a, const float* __restrict__ norm_coef) {
     const float coef = norm_coef ? norm_coef[1] : 1.0f;
     for (int chunk = blockIdx.x; chunk < l.chunks; chunk += gridDim.x) {
