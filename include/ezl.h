@@ -232,7 +232,8 @@ int ezl_build_location_idx(const int32_t* sizes, int64_t n_sizes, const int32_t*
 
 /* ---- one decoder layer per call: ParallelTransformerLayer.forward, llama/transformer.py:747-803, and its backward ----
  * The launches of the entry points above in the layer's order, for callers whose layers are small enough for the host's work
- * per call to matter.  Same kernels, same results.  Activations [s, b, h] (token row = s_idx * b + b_idx), contiguous. */
+ * per call to matter.  The kernels are those of the entry points; the input gradient of q / k / v is one sum over all three, rounded
+ * once (ezl_gemm_bf16_ksplit).  Activations [s, b, h] (token row = s_idx * b + b_idx), contiguous. */
 typedef struct {
     int64_t s, b, h, nq, nk, d, f;        /* tokens, hidden, query / kv heads, head dim, MLP width */
     int64_t ndocs, npos;                  /* documents (b when cu_seqlens is NULL), rows of the rotary tables */
