@@ -28,6 +28,7 @@
 //
 // Products that do not fill the chip with 256 x 256 tiles run on the smaller tiles of gemm_small.hip (see choose_plan).
 #include "gemm_tile.h"
+#include "gemm_list.h"
 
 namespace {
 
@@ -631,12 +632,16 @@ int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const i
 // average; by any estimated gain 0.74 %, by any gain where the products apart take under 115 us and a tenth above 0.65 %.
 constexpr double kLaunchGap = 2.5;  // us between two launches of a stream: ramp down, ramp up
 constexpr double kMargin256 = 0.9;
-bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
+struct GroupTimes {
+    GemmPlan plan;           // of the one launch
+    double together, apart;  // estimated us
+    bool one;
+};
+GroupTimes group_times(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room) {
     struct Entry {
         int64_t M[kMaxProblems], N[kMaxProblems], K, room;
-        GemmPlan plan;
+        GroupTimes times;
         int count;
-        bool one;
     };
     static thread_local Entry memo[64] = {};
     uint64_t hash = K * 0x165667B19E3779F9ull + count;
@@ -646,23 +651,29 @@ bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_
     for (int i = 0; i < count && same; ++i) same = e.M[i] == M[i] && e.N[i] == N[i];
     if (!same) {
         const int64_t nk = (K + BK - 1) / BK;
-        double apart = kLaunchGap * (count - 1), together;
+        GroupTimes& g = e.times;
+        g.apart = kLaunchGap * (count - 1);
         bool all_256 = true;
         for (int i = 0; i < count; ++i) {
             double t;
             all_256 = find_plan(1, &M[i], &N[i], nk, room, &t).kind == kTile256 && all_256;
-            apart += t;
+            g.apart += t;
             e.M[i] = M[i];
             e.N[i] = N[i];
         }
-        e.plan = find_plan(count, M, N, nk, room, &together);
-        e.one = together < (all_256 ? kMargin256 * apart : apart);
+        g.plan = find_plan(count, M, N, nk, room, &g.together);
+        if (all_256) g.together /= kMargin256;
+        g.one = g.together < g.apart;
         e.K = K;
         e.room = room;
         e.count = count;
     }
-    plan = e.plan;
-    return e.one;
+    return e.times;
+}
+bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
+    const GroupTimes g = group_times(count, M, N, K, room);
+    plan = g.plan;
+    return g.one;
 }
 // workspace of a product's plan; the 256 x 256 kernels' own where a launch has to fall back to them
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
@@ -936,8 +947,10 @@ bool results_meet(int count, void* const* C, const int64_t* M, const int64_t* N,
 // Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch; one after the other where their
 // results share memory or have rows too far apart.
 // ezl_gemm_group_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
+constexpr int kGroupMax = 3;  // q / k / v
+static_assert(kGemmListMax == kMaxProblems, "a list goes out in one launch");
 extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
-    if (count < 2 || count > kMaxProblems || !M || !N || K <= 0) return -1;
+    if (count < 2 || count > kGroupMax || !M || !N || K <= 0) return -1;
     for (int i = 0; i < count; ++i)
         if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
     GemmPlan plan;
@@ -948,6 +961,27 @@ extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, c
 extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
                                    int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,
                                    const int* accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
+    EZL_REQUIRE(count <= kGroupMax, EZL_EINVAL, "ezl_gemm_bf16_group: bad count, null argument array or empty reduction");
+    return gemm_list(count, A, B, C, M, N, K, lda, ldb, ldc, a_kc, b_kc, out_dtype, accumulate, workspace, workspace_bytes, stream);
+}
+
+// A decoder layer's weight gradients all reduce over its tokens.  Behind one another each of them is a launch that fills a part of the
+// chip (2 x 512 tokens at h = 256: 16 to 132 workgroups, four launches of 8 us), as one list of tiles they fill it together.
+int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* M, const int64_t* N, int64_t K) {
+    double in_pieces = kLaunchGap * (pieces - 1);
+    int count = 0;
+    for (int p = 0; p < pieces; ++p) {
+        const GroupTimes g = group_times(counts[p], M + count, N + count, K, INT64_MAX);
+        in_pieces += g.one ? g.together : g.apart;
+        count += counts[p];
+    }
+    const GroupTimes all = group_times(count, M, N, K, INT64_MAX);
+    return all.together < in_pieces ? small_plan_bytes(all.plan, count, M, N) : -1;
+}
+
+int gemm_list(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N, int64_t K,
+              const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype, const int* accumulate,
+              void* workspace, int64_t workspace_bytes, void* stream) {
     EZL_REQUIRE(count >= 1 && count <= kMaxProblems && A && B && C && M && N && lda && ldb && ldc && accumulate && K > 0, EZL_EINVAL,
                 "ezl_gemm_bf16_group: bad count, null argument array or empty reduction");
     EZL_REQUIRE((out_dtype == 0 && (a_kc || !b_kc)) || (out_dtype == 1 && !a_kc && !b_kc), EZL_EUNSUPPORTED,

@@ -35,10 +35,10 @@ __device__ __forceinline__ void tile_and_part(const GemmSmallArgs& a, int& tile,
     tile -= part * a.ntiles;
 }
 __device__ __forceinline__ GemmProblem problem_of(const GemmSmallArgs& a, int tile) {
-    GemmProblem p = a.p[0];
-    if (tile >= a.p[1].first) p = a.p[1];
-    if (tile >= a.p[2].first) p = a.p[2];
-    return p;
+    int i = 0;
+#pragma unroll
+    for (int j = 1; j < kMaxProblems; ++j) i += tile >= a.first[j];
+    return a.p[i];
 }
 
 template <typename OutT>
@@ -433,13 +433,12 @@ void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs
     for (int i = 0; i < kMaxProblems; ++i) {
         GemmProblem& p = a.p[i];
         if (i >= count) {
-            p = a.p[0];
-            p.first = 0x7fffffff;
+            a.first[i] = 0x7fffffff;
             continue;
         }
         p.tiles_m = (p.M + bm - 1) / bm;
         p.tiles_n = (p.N + bn - 1) / bn;
-        p.first = a.ntiles;
+        p.first = a.first[i] = a.ntiles;
         a.ntiles += p.tiles_m * p.tiles_n;
     }
     a.nsplit = plan.nsplit;

@@ -330,14 +330,16 @@ struct GemmProblem {
     void* C;
     int64_t lda, ldb, ldc;
     int M, N;
-    int tiles_m, tiles_n, first;  // tile grid, and the launch-wide id of its first tile (INT_MAX: no such product)
+    int tiles_m, tiles_n, first;  // tile grid, and the launch-wide id of its first tile
     int accumulate;
 };
 
-// A launch: up to three independent products over the same K, or (K segments) one product over up to three operand pairs.
-constexpr int kMaxProblems = 3;
+// A launch: independent products over the same K (up to the seven weight gradients of a decoder layer), or (K segments) one
+// product over up to three operand pairs.
+constexpr int kMaxProblems = 7;
 struct GemmSmallArgs {
     GemmProblem p[kMaxProblems];
+    int first[kMaxProblems];  // as in p (INT_MAX: no such product), together: one scalar load brings all of them
     int ntiles, K, nsplit;
     float* partial;  // nsplit > 1: [ntiles][nsplit][tile] fp32
     KSegments seg;

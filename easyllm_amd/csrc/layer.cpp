@@ -9,6 +9,7 @@
 // Memory: activations that backward needs lie in one `saved` block, everything else in one `temp` block; both are the caller's
 // and laid out by the same arithmetic in forward and backward (bump allocation, 256-byte steps).
 #include "common.h"
+#include "gemm_list.h"
 #include "qkv_bias.h"
 #include "../../include/ezl.h"
 
@@ -55,6 +56,24 @@ int64_t products_ws(int count, const int64_t* M, const int64_t* N, int64_t K) {
     return w;
 }
 
+// Sizes of a layer's weight gradients dw_i[n_i, k_i], which all reduce over the T tokens: q, k, v, o, gate, up, down.
+struct WeightGradients {
+    int64_t n[kGemmListMax], k[kGemmListMax];
+    explicit WeightGradients(const Dims& m)
+        : n{m.qw, m.kw, m.kw, m.h, m.f, m.f, m.h}, k{m.h, m.h, m.h, m.qw, m.h, m.h, m.f} {}
+    // workspace of all of them in one launch behind everything else; -1 where it is faster to launch them as their operands
+    // appear (q / k / v, o, gate / up, down).  elem: bytes of a result.  Results of much more than the last-level cache (256 MB)
+    // are better written in pieces, which drain into memory under the products between them: a layer's backward with 309 and 356 MB of
+    // them in one launch and in pieces 301 against 312 us, 1060 against 1102; with 410 - 670 MB 406 against 398, 790 against 779, 968
+    // against 1006, 524 against 484, 575 against 534.
+    int64_t list_bytes(int64_t T, int elem) const {
+        static const int counts[4] = {3, 1, 2, 1};
+        int64_t results = 0;
+        for (int i = 0; i < kGemmListMax; ++i) results += n[i] * k[i] * elem;
+        return results > (384LL << 20) ? -1 : gemm_list_workspace_bytes(4, counts, n, k, T);
+    }
+};
+
 struct ForwardTemp {
     void *wide, *bias_in, *ws;
     int64_t ws_bytes, bytes;
@@ -90,6 +109,7 @@ struct BackwardTemp {
         w = max64(w, ezl_rmsnorm_bwd_workspace_bytes(m.T, m.h));
         w = max64(w, ezl_attn_bwd_workspace_bytes(m.T, l.ndocs, m.nq, m.nk, m.d));
         if (l.bq) w = max64(w, ezl_bias_grad_workspace_bytes(m.T, m.qw + 2 * m.kw));
+        w = max64(w, WeightGradients(m).list_bytes(m.T, 2));
         ws_bytes = w;
         ws = b.take(ws_bytes);
         bytes = b.used;
@@ -132,6 +152,16 @@ int weight_gradients(int count, const void* const* dy, int64_t ld, const void* x
         if (out[i])
             EZL_TRY(ezl_gemm_bf16(dy[i], x, out[i], n[i], k, T, ld, k, k, 0, 0, g[i].f32 ? 1 : 0, acc[i], ws, ws_bytes, st));
     return EZL_OK;
+}
+
+// gradient list entries of the weights, in WeightGradients' order
+constexpr int kWeights[kGemmListMax] = {EZL_G_Q, EZL_G_K, EZL_G_V, EZL_G_O, EZL_G_GATE, EZL_G_UP, EZL_G_DOWN};
+
+// all weight gradients in one launch: all wanted, in one type, and estimated to be faster than piece by piece
+bool in_one_list(const Dims& m, const ezl_layer_grad* g) {
+    for (int i : kWeights)
+        if (!(g[i].f32 || g[i].bf16) || (g[i].f32 != nullptr) != (g[EZL_G_Q].f32 != nullptr)) return false;
+    return WeightGradients(m).list_bytes(m.T, g[EZL_G_Q].f32 ? 4 : 2) >= 0;
 }
 
 // elements of the parameters, in the order of the gradient list
@@ -223,9 +253,10 @@ extern "C" int ezl_layer_bwd(const ezl_layer* l, const void* x, const void* dy, 
     EZL_REQUIRE((g[EZL_G_LN1].f32 || g[EZL_G_LN1].bf16) && (g[EZL_G_LN2].f32 || g[EZL_G_LN2].bf16), EZL_EINVAL,
                 "ezl_layer_bwd: the norm weights' gradients are part of their kernels");
     EZL_REQUIRE(!gradients_meet(m, g), EZL_EINVAL, "ezl_layer_bwd: two gradients share memory (they are written in the kernels' order)");
+    const bool one_list = in_one_list(m, g);  // then their operands stay where they are to the end
     // y = sum + down(act): dy goes to both
     EZL_TRY(ezl_gemm_bf16(dy, l->wd, t.dact, m.T, m.f, m.h, m.h, m.f, m.f, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
-    {
+    if (!one_list) {
         const void* d[1] = {dy};
         EZL_TRY(weight_gradients(1, d, m.h, a.act, &g[EZL_G_DOWN], m.T, &m.h, m.f, t.ws, t.ws_bytes, st));
     }
@@ -234,13 +265,13 @@ extern "C" int ezl_layer_bwd(const ezl_layer* l, const void* x, const void* dy, 
         const void *d[2] = {t.dgate, t.dup}, *w[2] = {l->wg, l->wu};
         const int64_t n[2] = {m.f, m.f};
         EZL_TRY(ezl_gemm_bf16_ksplit(2, d, w, t.dn, m.T, m.h, n, m.f, m.h, m.h, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
-        EZL_TRY(weight_gradients(2, d, m.f, a.n2, &g[EZL_G_GATE], m.T, n, m.h, t.ws, t.ws_bytes, st));
+        if (!one_list) EZL_TRY(weight_gradients(2, d, m.f, a.n2, &g[EZL_G_GATE], m.T, n, m.h, t.ws, t.ws_bytes, st));
     }
     EZL_TRY(ezl_rmsnorm_bwd(t.dn, a.sum, l->ln2, a.rstd2, dy, t.dsum, g[EZL_G_LN2].f32 ? nullptr : g[EZL_G_LN2].bf16, g[EZL_G_LN2].f32,
                             g[EZL_G_LN2].accumulate, t.ws, t.ws_bytes, m.T, m.h, st));
     // sum = x + o(ctx)
     EZL_TRY(ezl_gemm_bf16(t.dsum, l->wo, t.dctx, m.T, m.qw, m.h, m.h, m.qw, m.qw, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
-    {
+    if (!one_list) {
         const void* d[1] = {t.dsum};
         EZL_TRY(weight_gradients(1, d, m.h, a.ctx, &g[EZL_G_O], m.T, &m.h, m.qw, t.ws, t.ws_bytes, st));
     }
@@ -264,7 +295,21 @@ extern "C" int ezl_layer_bwd(const ezl_layer* l, const void* x, const void* dy, 
             EZL_TRY(qkv_bias_grad(t.dqkv, gb, m.T, m.qw, m.kw, t.ws, (hipStream_t)st));
         }
         EZL_TRY(ezl_gemm_bf16_ksplit(3, d, w, t.dn, m.T, m.h, n, S, m.h, m.h, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
-        EZL_TRY(weight_gradients(3, d, S, a.n1, &g[EZL_G_Q], m.T, n, m.h, t.ws, t.ws_bytes, st));
+        if (!one_list) EZL_TRY(weight_gradients(3, d, S, a.n1, &g[EZL_G_Q], m.T, n, m.h, t.ws, t.ws_bytes, st));
+    }
+    if (one_list) {
+        const WeightGradients w(m);
+        const void *d[kGemmListMax] = {dq, dk, dv, t.dsum, t.dgate, t.dup, dy};
+        const void *x[kGemmListMax] = {a.n1, a.n1, a.n1, a.ctx, a.n2, a.n2, a.act};
+        const int64_t ld[kGemmListMax] = {S, S, S, m.h, m.f, m.f, m.h};
+        void* out[kGemmListMax];
+        int acc[kGemmListMax];
+        for (int i = 0; i < kGemmListMax; ++i) {
+            const ezl_layer_grad& target = g[kWeights[i]];
+            out[i] = target.f32 ? target.f32 : target.bf16;
+            acc[i] = target.accumulate;
+        }
+        EZL_TRY(gemm_list(kGemmListMax, d, x, out, w.n, w.k, m.T, ld, w.k, w.k, 0, 0, g[EZL_G_Q].f32 ? 1 : 0, acc, t.ws, t.ws_bytes, st));
     }
     return ezl_rmsnorm_bwd(t.dn, x, l->ln1, a.rstd1, t.dsum, dx, g[EZL_G_LN1].f32 ? nullptr : g[EZL_G_LN1].bf16, g[EZL_G_LN1].f32,
                            g[EZL_G_LN1].accumulate, t.ws, t.ws_bytes, m.T, m.h, st);

@@ -182,6 +182,36 @@ def test_gemm_products_in_one_launch(K, T, n_in, outs):
             assert ((dw.float() - ref).abs() <= tol).all()
 
 
+@pytest.mark.parametrize("h,nq,nk,f,b,s,main_grads", [(64, 1, 1, 72, 1, 3, True), (256, 4, 1, 688, 2, 511, True), (768, 12, 12, 2048, 2, 1024, True),
+                                                      (1024, 16, 4, 2816, 3, 389, False), (1024, 8, 8, 2816, 1, 4000, True),
+                                                      (256, 4, 4, 1000, 1, 16001, True)])
+def test_weight_gradients_of_a_layer_in_one_launch(h, nq, nk, f, b, s, main_grads):
+    """A layer's seven weight gradients as one list of tiles (at these sizes: one, two or several K tiles per wave, K tails, 64, 128 and
+    256 x 128 tiles, split reductions), overwritten and then added to, against the composed layer's separate products: activations and
+    their gradients are the same bits, the sums over the tokens are in fp32 in another order (bf16 results: one rounding apart)."""
+    from easyllm_amd import runner
+    print("weight gradients of a layer", h, f, b, s, flush=True)
+    results = []
+    for flops in (1e13, 0.0):
+        torch.manual_seed(5)
+        model = runner.build_model({"type": "llama_custom", "kwargs": dict(
+            num_layers=1, hidden_size=h, num_attention_heads=nq, num_kv_attention_heads=nk, intermediate_size=f, vocab_size=512, seq_length=s,
+            bf16=True, checkpoint_activations=False)}).cuda()
+        layer = next(m for m in model.modules() if hasattr(m, "native_call_flops"))
+        layer.native_call_flops = flops
+        if main_grads:
+            runner.attach_main_grads(model)
+        g = torch.Generator().manual_seed(1)
+        tokens, labels = (torch.randint(0, 512, (b, s), generator=g).cuda() for _ in range(2))
+        for _ in range(2 if main_grads else 1):  # the second pass adds
+            runner.forward_step(model, (tokens, torch.arange(s).expand(b, s).contiguous().cuda(), None), (labels, torch.ones(b, s, device="cuda")))
+        results.append({n: (p.main_grad if main_grads else p.grad.float()) for n, p in layer.named_parameters() if p.dim() == 2})
+    got, want = results
+    assert len(want) == 7
+    for n in want:
+        assert (got[n] - want[n]).norm() <= (1e-5 if main_grads else 2.0 ** -8) * want[n].norm(), n
+
+
 @pytest.mark.parametrize("sizes", [[1], [4096, 4095, 4097, 3], [0, 8, 0, 70001], [1 + 37 * i for i in range(101)]])
 def test_optimizer_over_lists_of_tensors(K, sizes):
     """Chunk edges, empty tensors and more tensors than one launch takes: the norm against fp64, the update bit for bit against
