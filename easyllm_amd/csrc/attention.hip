@@ -20,9 +20,11 @@
 // LDS rows are padded to (d*2 + 48) bytes, which keeps both the 128-bit row reads and the transpose
 // reads free of bank conflicts.  K/V (or Q/dO) tiles are double buffered and filled through
 // registers one tile ahead.  dQ uses its own pass instead of atomics, so results are deterministic.
-#include "common.h"
-
-#include <type_traits>
+//
+// Launches that leave CUs idle: the forward and the dQ kernel also exist with the key tiles shared out to two groups of four
+// waves, dQ and dK/dV as one launch, and attention_small.hip has both with 32 rows per workgroup.  Which is taken follows from
+// the number of blocks and the document length alone (attn_small_pays, fwd_key_groups_pay, bwd_one_launch_pays).
+#include "attention_tile.h"
 
 namespace {
 
@@ -30,321 +32,30 @@ constexpr int kThreads = 256;
 #ifndef EZL_DKDV_MIN_BLOCKS
 #define EZL_DKDV_MIN_BLOCKS 512  // dK/dV workgroups wanted before (kv head, key block) pairs stop being split
 #endif
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
-
-typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-typedef __attribute__((address_space(3))) void lds_void;
-
-struct AttnParams {
-    const bf16_t* q; const bf16_t* k; const bf16_t* v; const bf16_t* o; const bf16_t* dout;
-    bf16_t* out; bf16_t* dq; bf16_t* dk; bf16_t* dv;
-    float* lse; float* delta;
-    float* part;  // dK/dV kernel with nsplit > 1: fp32 partial sums [nsplit][2 (dK, dV)][T][nk][d]
-    int nsplit;   // workgroups that share a (kv head, key block): each takes nq / nk / nsplit of the group's query heads
-    const int* cu;
-    int ndocs, s_len, T, nq, nk;
-    float scale;
-    int64_t q_ss, q_sb, k_ss, k_sb, v_ss, v_sb, o_ss, o_sb;          // forward tensors
-    int64_t do_ss, do_sb, dq_ss, dq_sb, dk_ss, dk_sb, dv_ss, dv_sb;  // backward tensors
-};
-
-__device__ __forceinline__ int64_t tok_off(int n, int s_len, int64_t ss, int64_t sb) {
-    const int b = n / s_len;
-    return (int64_t)b * sb + (int64_t)(n - b * s_len) * ss;
-}
-
-// Work list of the three kernels.  A document is cut at batch-row boundaries (the reference's collator never emits one
-// that crosses a row: it appends every row's length to that row's boundaries), so inside a piece token i lives at
-// tok_off(piece_start) + i * seq_stride and no per-token division is needed.  A piece of n tokens has ceil(n / 128) blocks;
-// block j of a piece (queries, or keys counted from the piece's END for the dK/dV kernel) walks j + 1 blocks of the other
-// operand, so its running time grows with j.
-//
-// Blocks are handed out longest first over ALL pieces and heads (rank 0 = the largest j anywhere): the hardware starts
-// workgroups in the order of their ids, and with the long blocks of some head started late -- as happens when ids run head
-// by head -- the last of them finish long after everything else (98 instead of 66 block-times for 4 heads x 32 blocks on
-// the 64 slots of an XCD).  rank -> (piece, j): level j holds the pieces with more than j blocks, levels are laid out from
-// the highest down; the level is found by bisection on count(j) = number of blocks with index >= j, the piece inside the
-// level by a prefix sum, both computed by the whole workgroup (every thread must call this, before any other use of LDS).
-// Dense batches (no cu_seqlens) have a closed form.
-__device__ __forceinline__ int doc_bounds(const int* __restrict__ cu, int d, int s_len, int T, int& e) {
-    int a = cu ? cu[d] : d * s_len;
-    e = cu ? cu[d + 1] : (d + 1) * s_len;
-    a = a < 0 ? 0 : a;
-    e = e > T ? T : e;
-    return a;
-}
-
-struct BlockSearch {
-    int* s_wave;  // [16]
-    int tid, nthr, lane, wv, nwaves;
-    // sum over the workgroup; uniform result
-    __device__ __forceinline__ int reduce(int v) const {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        __syncthreads();  // s_wave of the previous reduction has been read
-        if (lane == 0) s_wave[wv] = v;
-        __syncthreads();
-        int t = 0;
-        for (int i = 0; i < nwaves; ++i) t += s_wave[i];
-        return t;
-    }
-};
-
-// lds: kFindBlockInts ints of LDS for the search.  It is handed in by the kernel, carved from its one LDS array, instead of
-// being declared here: with several LDS variables in a kernel the compiler tags every LDS access with the variable it
-// belongs to and thereby drops the no-alias tags of the fragment reads, after which each read waits for all tile loads in
-// flight (vmcnt(0)) because it might alias their destination.
-constexpr int kFindBlockInts = 20;
-__device__ __forceinline__ bool find_block(const int* __restrict__ cu, int ndocs, int s_len, int T, int rank, int blk_rows,
-                                           int& doc_start, int& doc_len, int& blk, int* lds) {
-    const int nb_row = (s_len + blk_rows - 1) / blk_rows;
-    if (!cu) {  // every piece is a whole batch row: level j holds all ndocs rows
-        if (rank >= ndocs * nb_row) return false;
-        blk = nb_row - 1 - rank / ndocs;
-        doc_start = (rank % ndocs) * s_len;
-        doc_len = s_len;
-        return true;
-    }
-    int* s_wave = lds;        // [16]
-    int* s_found = lds + 16;  // [4]
-    BlockSearch bs;
-    bs.s_wave = s_wave;
-    bs.tid = threadIdx.x; bs.nthr = blockDim.x; bs.lane = bs.tid & 63; bs.wv = bs.tid >> 6; bs.nwaves = bs.nthr >> 6;
-    // blocks with index >= j over this thread's documents (pieces enumerated on the fly; one piece unless a document
-    // crosses a batch row)
-    auto count_ge = [&](int j) {
-        int c = 0;
-        for (int d = bs.tid; d < ndocs; d += bs.nthr) {
-            int e;
-            const int a = doc_bounds(cu, d, s_len, T, e);
-            for (int x = a; x < e;) {
-                const int row_end = (x / s_len + 1) * s_len;
-                const int e1 = e < row_end ? e : row_end;
-                const int nb = (e1 - x + blk_rows - 1) / blk_rows;
-                c += nb > j ? nb - j : 0;
-                x = e1;
-            }
-        }
-        return bs.reduce(c);
-    };
-    if (rank >= count_ge(0)) return false;
-    int lo = 0, hi = nb_row, c_hi = 0;  // count(lo) > rank >= count(hi)
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        const int c = count_ge(mid);
-        if (c > rank) lo = mid;
-        else { hi = mid; c_hi = c; }
-    }
-    const int j = lo;
-    const int want = rank - c_hi;  // the want-th piece (in document order) that has more than j blocks
-    if (bs.tid == 0) s_found[0] = 0;
-    int base = 0;
-    for (int d0 = 0; d0 < ndocs; d0 += bs.nthr) {
-        const int d = d0 + bs.tid;
-        int mine = 0, a = 0, e = 0;
-        if (d < ndocs) {
-            a = doc_bounds(cu, d, s_len, T, e);
-            for (int x = a; x < e;) {
-                const int row_end = (x / s_len + 1) * s_len;
-                const int e1 = e < row_end ? e : row_end;
-                mine += (e1 - x + blk_rows - 1) / blk_rows > j;
-                x = e1;
-            }
-        }
-        int incl = mine;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64);
-            if (bs.lane >= o) incl += v;
-        }
-        __syncthreads();
-        if (bs.lane == 63) s_wave[bs.wv] = incl;
-        __syncthreads();
-        int before = 0, total = 0;
-        for (int i = 0; i < bs.nwaves; ++i) {
-            const int v = s_wave[i];
-            before += i < bs.wv ? v : 0;
-            total += v;
-        }
-        const int first = base + before + incl - mine;  // rank inside the level of this thread's first qualifying piece
-        if (mine > 0 && want >= first && want < first + mine) {
-            int rel = want - first;
-            for (int x = a; x < e;) {
-                const int row_end = (x / s_len + 1) * s_len;
-                const int e1 = e < row_end ? e : row_end;
-                if ((e1 - x + blk_rows - 1) / blk_rows > j) {
-                    if (rel == 0) {
-                        s_found[1] = x;
-                        s_found[2] = e1 - x;
-                        s_found[0] = 1;
-                        break;
-                    }
-                    --rel;
-                }
-                x = e1;
-            }
-        }
-        base += total;
-        if (want < base) break;  // uniform
-    }
-    __syncthreads();
-    if (!s_found[0]) return false;
-    doc_start = __builtin_amdgcn_readfirstlane(s_found[1]);
-    doc_len = __builtin_amdgcn_readfirstlane(s_found[2]);
-    blk = j;
-    return true;
-}
-
-// The hardware deals consecutive workgroups (x fastest, then y) round-robin to the 8 XCDs, each with an L2 of its own.
-// With the plain (block, head) numbering every XCD would touch the K / V rows of every head and its L2 would keep missing;
-// renumbered, an XCD owns nheads / 8 heads, and inside an XCD the ids run over ranks (longest blocks first, see above) with
-// the XCD's heads innermost: blocks of equal length of all its heads start together and walk the keys in step.
-// by: head, rank: position in the longest-first work list of one head.
-__device__ __forceinline__ void xcd_head_blocks(int nheads, int& rank, int& by) {
-    const int lin = blockIdx.y * gridDim.x + blockIdx.x;
-    if ((nheads & 7) == 0) {
-        const int hpx = nheads >> 3, idx = lin >> 3;
-        by = (lin & 7) * hpx + idx % hpx;
-        rank = idx / hpx;
-    } else {
-        by = lin % nheads;
-        rank = lin / nheads;
-    }
-}
-
-template <int D>
-struct Tile {
-    static constexpr int LD = D + 24;             // padded row stride in elements
-    static constexpr int CH = D / 8;              // 128-bit chunks per row
-    static constexpr int ROWS = 64;
-    static constexpr int ELEMS = ROWS * LD;
-
-    // ---- tile rows straight from global memory into LDS (buffer_load ... lds, 16 bytes per lane) ----
-    // One wave instruction fills 1 KiB of consecutive LDS, i.e. 1024 / (2 LD) padded rows: instruction q of a tile covers
-    // bytes 1024 q .. 1024 q + 1023 of its LDS image, and the lane that falls on row padding re-reads the row's first chunk.
-    // Rows at or past the document's end re-read its last row: finite values that only ever meet masked probabilities.
-    // NWAVES waves share the NQ instructions of a tile: wave w issues q = w, w + NWAVES, ...
-    static constexpr int NQ = (ROWS * LD * 2 + 1023) / 1024;
-    static_assert(ROWS * LD * 2 % 1024 == 0, "a tile is a whole number of 1 KiB pieces");
-    template <int NWAVES>
-    struct Direct {
-        static constexpr int NJ = (NQ + NWAVES - 1) / NWAVES;
-        uint32_t off[NJ];  // global byte offset of this lane's chunk from the tile's first row, per instruction
-        // last: last valid row of the tile (63, or fewer in a document's ragged last tile: later rows re-read it)
-        __device__ __forceinline__ void init(int64_t ss, int lane, int wave, int last) {
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const int q = wave + NWAVES * j;
-                const int byte = q * 1024 + lane * 16;
-                int row = byte / (LD * 2);
-                int colb = byte - row * (LD * 2);
-                colb = colb < D * 2 ? colb : 0;
-                row = row < last ? row : last;
-                off[j] = (uint32_t)row * (uint32_t)(ss * 2) + (uint32_t)colb;
-            }
-        }
-        // tile_rows: global address of the tile's first row (head column included); stage: its LDS image
-        __device__ __forceinline__ void issue(const bf16_t* tile_rows, bf16_t* stage, int wave) const {
-            // (the buffer form of the load: while a global load to LDS is in flight the compiler, which books it as a flat
-            // access, turns every counted wait on LDS reads into a full drain)
-            const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<char*>(reinterpret_cast<const char*>(tile_rows)), 0, 0xffffffffu, 0x00020000);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const int q = wave + NWAVES * j;
-                if (q < NQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(g, (lds_void*)(stage + q * 512), 16, off[j], 0, 0, 0);
-            }
-        }
-    };
-    // operand whose k index is d:   lane -> row (row0 + lane&31), d = kd*16 + 8*(lane>>5) ..+7
-    static __device__ __forceinline__ bf16x8 frag_kc(const bf16_t* __restrict__ s, int row0, int kd, int lane) {
-        return *reinterpret_cast<const bf16x8*>(s + (row0 + (lane & 31)) * LD + kd * 16 + (lane >> 5) * 8);
-    }
-    // operand whose k index is the tile row: lane -> d column (col0 + lane&31); k values are tile rows
-    // krow0 + 4g + {0..3} and krow0 + 8 + 4g + {0..3}, g = lane>>5 -- the order in which a 32x32
-    // accumulator block holds 16 consecutive rows, so accumulators convert straight to the B operand.
-    static __device__ __forceinline__ bf16x8 frag_tr(const bf16_t* __restrict__ s, int krow0, int col0, int lane) {
-        const int q = lane >> 4;
-        const bf16_t* p = s + (krow0 + 4 * (lane >> 5) + ((lane & 15) >> 2)) * LD + col0 + (q & 1) * 16 + ((lane & 3) << 2);
-        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p));
-        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 8 * LD));
-        bf16x8 v;
-        v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
-        v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
-        return v;
-    }
-    // ---- fragments of the 16x16x32 MFMA (l16 = lane & 15, j4 = lane >> 4) ----
-    // (the tile pointers are __restrict__ so that the reads carry a no-alias tag: an untagged LDS read waits for every tile
-    // load in flight)
-    // A operand whose k index is d: 16 tile rows row0 .., d = 32 ds + 8 j4 .. + 7
-    static __device__ __forceinline__ bf16x8 frag_kc16(const bf16_t* __restrict__ s, int row0, int ds, int lane) {
-        return *reinterpret_cast<const bf16x8*>(s + (row0 + (lane & 15)) * LD + ds * 32 + (lane >> 4) * 8);
-    }
-    // A operand whose k index is the tile row: lane -> d column col0 + l16; k slots 8 j4 + e are tile rows krow0 + 4 j4 + e
-    // (e < 4) and krow0 + 16 + 4 j4 + e - 4 (e >= 4): the order in which two stacked 16-row accumulator tiles hold them
-    static __device__ __forceinline__ bf16x8 frag_tr16(const bf16_t* __restrict__ s, int krow0, int col0, int lane) {
-        const bf16_t* a = s + (krow0 + 4 * (lane >> 4) + ((lane & 15) >> 2)) * LD + col0 + ((lane & 3) << 2);
-        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(a));
-        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(a + 16 * LD));
-        bf16x8 v;
-        v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
-        v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
-        return v;
-    }
-};
-
-// registers 8t .. 8t+7 of an accumulator block as a bf16 B operand
-__device__ __forceinline__ bf16x8 acc_to_b(const f32x16& a, int t) {
-    bf16x8 v;
-    if (t == 0) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (bf16_t)a[e];
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (bf16_t)a[8 + e];
-    }
-    return v;
-}
-
-// row of register r inside a 32-row accumulator block
-__device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
-
-// one operand row per lane, straight from global memory, as D/16 B-operand fragments
-template <int D>
-__device__ __forceinline__ void load_row_frags(const bf16_t* __restrict__ rowp, int lane, bf16x8* f) {
-#pragma unroll
-    for (int kd = 0; kd < D / 16; ++kd) f[kd] = *reinterpret_cast<const bf16x8*>(rowp + kd * 16 + (lane >> 5) * 8);
-}
 
 // =================================================================================================
 // forward
 // =================================================================================================
-// f(integral_constant<int, I>) for I = I0 .. N-1, so that the body sees its index as a constant expression
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
 // The loop over the key tiles below the diagonal is software-pipelined inside each wave: iteration t issues the MFMAs of
 // S(t+1) = K(t+1) Q^T and then of O += V(t) P(t), one per step, and between them the vector ALU work that turns S(t) into
 // P(t) and, once S(t+1) is complete, takes its row maxima.  A sched_barrier after every step keeps that interleaving.  The
 // K tiles therefore run one tile ahead of the V tiles in LDS.  The two tiles on the diagonal are done afterwards, one at a
 // time with the mask.
-template <int D>
-__global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
+// KG = 2: two groups of four waves share out the key tiles (group g takes g, g + 2, ...), each with its own stages in LDS; their sums are
+// brought together at the end.  Half the chain per workgroup, at one workgroup of eight waves per CU instead of two of four.
+template <int D, int KG>
+__global__ __launch_bounds__(kThreads * KG, 2) void attn_fwd_kernel(AttnParams p) {
     using TL = Tile<D>;
-    // K0 V0 K1 V1: tile t of K or V in stage t & 1; then the block search's scratch
-    __shared__ __attribute__((aligned(16))) bf16_t smem[4 * TL::ELEMS + 2 * kFindBlockInts];
+    // per key group K0 V0 K1 V1: tile t of K or V in stage t & 1; then the block search's scratch
+    __shared__ __attribute__((aligned(16))) bf16_t smem_all[KG * 4 * TL::ELEMS + 2 * kFindBlockInts];
     int doc_start, doc_len, qb;
     int bx, by;
     xcd_head_blocks(p.nq, bx, by);
-    if (!find_block(p.cu, p.ndocs, p.s_len, p.T, bx, 128, doc_start, doc_len, qb, reinterpret_cast<int*>(smem + 4 * TL::ELEMS)))
+    if (!find_block(p.cu, p.ndocs, p.s_len, p.T, bx, 128, doc_start, doc_len, qb, reinterpret_cast<int*>(smem_all + KG * 4 * TL::ELEMS)))
         return;  // bx = rank: longest rows first
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    bf16_t* smem = smem_all + kg * 4 * TL::ELEMS;
     const int hq = by, hk = hq / (p.nq / p.nk);
     const int q0 = qb * 128, qw0 = q0 + wave * 32;
     const int qi = qw0 + (lane & 31);                        // this lane's query (document relative)
@@ -353,8 +64,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
     load_row_frags<D>(p.q + tok_off(qtok, p.s_len, p.q_ss, p.q_sb) + (int64_t)hq * D, lane, qf);
 
     const int kend = (q0 + 128 < doc_len ? q0 + 128 : doc_len);
-    const int ntiles = (kend + 63) / 64;
-    const int nmain = 2 * qb;  // tiles wholly below the diagonal for every query of the workgroup
+    // this key group's tiles: t = 0 .. ntiles - 1 stands for tile KG t + kg of the document
+    const int ntiles = ((kend + 63) / 64 - kg + KG - 1) / KG;
+    const int nmain = 2 * qb / KG;  // of which wholly below the diagonal for every query of the workgroup
+    constexpr int NDIAG = 2 / KG;   // at most that many on the diagonal
     const int64_t kh = (int64_t)hk * D;
     const bf16_t* kbase = p.k + tok_off(doc_start, p.s_len, p.k_ss, p.k_sb) + kh;
     const bf16_t* vbase = p.v + tok_off(doc_start, p.s_len, p.v_ss, p.v_sb) + kh;
@@ -363,7 +76,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
     vld.init(p.v_ss, lane, wave, 63);
     // which: 0 = K tile t, 1 = V tile t
     auto issue_one = [&](int t, int which) {
-        const int row0 = t * 64;
+        const int row0 = (KG * t + kg) * 64;
         bf16_t* dst = smem + (t & 1) * 2 * TL::ELEMS + which * TL::ELEMS;
         const bf16_t* src = (which ? vbase + (int64_t)row0 * p.v_ss : kbase + (int64_t)row0 * p.k_ss);
         if (row0 + 64 <= doc_len) {
@@ -375,8 +88,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
             e.issue(src, dst, wave);
         }
     };
-    issue_one(0, 0);
-    issue_one(0, 1);
+    if (KG == 1 || ntiles > 0) {
+        issue_one(0, 0);
+        issue_one(0, 1);
+    }
     if (ntiles > 1) issue_one(1, 0);
     // every load issued so far (the per-lane operand rows included) has landed before the loop starts
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -398,10 +113,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
     auto scores1 = [&](int t, f32x16 (&s)[2]) {
         const bf16_t* sK = smem + (t & 1) * 2 * TL::ELEMS;
         bf16x8 fk[2][4];
-        constexpr int KG = D / 64, NG = 2 * KG;
+        constexpr int KGRP = D / 64, NG = 2 * KGRP;
         auto ldk = [&](int g, int buf) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) fk[buf][i] = TL::frag_kc(sK, (g / KG) * 32, (g % KG) * 4 + i, lane);
+            for (int i = 0; i < 4; ++i) fk[buf][i] = TL::frag_kc(sK, (g / KGRP) * 32, (g % KGRP) * 4 + i, lane);
         };
         ldk(0, 0);
 #pragma unroll
@@ -413,7 +128,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
             if (g + 1 < NG) ldk(g + 1, (g + 1) & 1);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                s[g / KG] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fk[g & 1][i], qf[(g % KG) * 4 + i], s[g / KG], 0, 0, 0);
+                s[g / KGRP] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fk[g & 1][i], qf[(g % KGRP) * 4 + i], s[g / KGRP], 0, 0, 0);
         }
     };
     auto rowmax = [&](const f32x16 (&s)[2]) {
@@ -449,7 +164,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
         // K stage t & 1: K(t) was last read by the scores of the previous iteration (t = 0: by scores1 above), i.e. before
         // the barrier every wave has passed since
         if (t + 2 < ntiles) issue_one(t + 2, 0);
-        issue_one(t + 1, 1);                      // V stage (t+1) & 1: V(t-1) likewise; t + 1 <= nmain < ntiles
+        if (KG == 1 || t + 1 < ntiles) issue_one(t + 1, 1);  // V stage (t+1) & 1: V(t-1) likewise; (KG == 1: t + 1 <= nmain < ntiles)
         {
             const bf16_t* sK = smem + ((t + 1) & 1) * 2 * TL::ELEMS;
             const bf16_t* sV = smem + (t & 1) * 2 * TL::ELEMS + TL::ELEMS;
@@ -515,12 +230,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
         __syncthreads();
     }
     // ---- the tiles on the diagonal; cur holds S(nmain) ----
-    for (int t = nmain; t < ntiles; ++t) {
+    for (int t = nmain; t < (KG == 1 ? ntiles : nmain + NDIAG); ++t) {
         if (t + 2 < ntiles) issue_one(t + 2, 0);
         if (t + 1 < ntiles) issue_one(t + 1, 1);
         const bf16_t* sV = smem + (t & 1) * 2 * TL::ELEMS + TL::ELEMS;
-        const int key0 = t * 64;
-        if (key0 <= qw0 + 31) {  // otherwise every key of the tile is after every query of this wave
+        const int key0 = (KG * t + kg) * 64;
+        if (t < ntiles && key0 <= qw0 + 31) {  // otherwise every key of the tile is after every query of this wave
             bf16x8 fv[2][D / 32];
             auto ldv = [&](int g, int buf) {
 #pragma unroll
@@ -557,24 +272,50 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
                     oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[g & 1][db], pfr, oacc[db], 0, 0, 0);
             }
         }
-        if (t + 1 < ntiles && (t + 1) * 64 <= qw0 + 31) scores1(t + 1, cur);  // K(t+1) arrived before the previous barrier
+        if (t + 1 < ntiles && (KG * (t + 1) + kg) * 64 <= qw0 + 31) scores1(t + 1, cur);  // K(t+1) arrived before the previous barrier
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
     }
-    const float ltot = lsum + __shfl_xor(lsum, 32, 64);
+    float ltot = lsum + __shfl_xor(lsum, 32, 64);
+    int db0 = 0;
+    constexpr int NDB = D / 32 / KG;  // 32-wide pieces of O that a wave finishes
+    if constexpr (KG == 2) {
+        // the two key groups' sums, brought to a common reference point: each wave finishes half of O, for which its partner in
+        // the other group leaves its half in LDS (every wave is past its last tile since the barrier above)
+        float* park = reinterpret_cast<float*>(smem_all) + wave * (2 * (NDB * 16 + 2) * 64) + lane;
+        float* mine = park + kg * ((NDB * 16 + 2) * 64);
+        float* other = park + (1 - kg) * ((NDB * 16 + 2) * 64);
+        db0 = kg * NDB;
+#pragma unroll
+        for (int i = 0; i < NDB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mine[(i * 16 + r) * 64] = kg ? oacc[i][r] : oacc[NDB + i][r];
+        mine[NDB * 16 * 64] = m;
+        mine[(NDB * 16 + 1) * 64] = ltot;
+        __syncthreads();
+        const float m1 = other[NDB * 16 * 64], l1 = other[(NDB * 16 + 1) * 64];
+        const float mt = fmaxf(m, m1), ref = mt == -INFINITY ? 0.f : mt;
+        const float a0 = __builtin_amdgcn_exp2f((m - ref) * sl2), a1 = __builtin_amdgcn_exp2f((m1 - ref) * sl2);
+        m = mt;
+        ltot = kg ? l1 * a1 + ltot * a0 : ltot * a0 + l1 * a1;
+#pragma unroll
+        for (int i = 0; i < NDB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[i][r] = (kg ? oacc[NDB + i][r] : oacc[i][r]) * a0 + other[(i * 16 + r) * 64] * a1;
+    }
     if (qi < doc_len) {
         const float inv = 1.0f / ltot;
         bf16_t* orow = p.out + tok_off(doc_start + qi, p.s_len, p.o_ss, p.o_sb) + (int64_t)hq * D;
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db)
+        for (int db = 0; db < NDB; ++db)
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
                 bf16x4 w;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) w[e] = (bf16_t)(oacc[db][r4 * 4 + e] * inv);
-                *reinterpret_cast<bf16x4*>(orow + db * 32 + 8 * r4 + 4 * (lane >> 5)) = w;
+                *reinterpret_cast<bf16x4*>(orow + (db0 + db) * 32 + 8 * r4 + 4 * (lane >> 5)) = w;
             }
-        if (lane < 32) p.lse[(int64_t)hq * p.T + doc_start + qi] = m * p.scale + __builtin_amdgcn_logf(ltot) * kLn2;
+        if (kg == 0 && lane < 32) p.lse[(int64_t)hq * p.T + doc_start + qi] = m * p.scale + __builtin_amdgcn_logf(ltot) * kLn2;
     }
 }
 
@@ -587,22 +328,25 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
 // registers; the two partial dK / dV of a key group are added through LDS at the end, always in the same order.
 constexpr int kDkdvThreads = 512;
 
+// LDS: K V rows of the block's 128 keys, (Q dO) tiles x 2 stages, [stage][lse*log2e | delta][64 queries] floats, block search
 template <int D>
-__global__ __launch_bounds__(kDkdvThreads) void attn_bwd_dkdv_kernel(AttnParams p) {
+constexpr int kDkdvTiles = 2 * 128 * Tile<D>::LD + 4 * Tile<D>::ELEMS;
+template <int D>
+constexpr int kDkdvLds = kDkdvTiles<D> + 2 * (2 * 2 * 64) + 2 * kFindBlockInts;
+
+// OWN_DELTA: delta = rowsum(dO * O) is computed with the dO tiles instead of read
+template <int D, bool OWN_DELTA>
+__device__ __forceinline__ void dkdv_block(const AttnParams& p, int bx, int by, bf16_t* smem) {
     using TL = Tile<D>;
     constexpr int LD = TL::LD, CH = TL::CH;
     constexpr int KV_ELEMS = 128 * LD;     // K (or V) rows of the block's 128 keys
     constexpr int STAGE = 2 * TL::ELEMS;   // Q tile + dO tile, 64 rows each
     constexpr int NCH_KV = 128 * CH / kDkdvThreads, NCH_Q = 64 * CH / kDkdvThreads;
-    __shared__ __attribute__((aligned(16))) bf16_t smem[2 * KV_ELEMS + 2 * STAGE];  // K V | (Q dO) x 2 stages
-    __shared__ __attribute__((aligned(16))) float sstat[2][2][64];                   // [stage][lse*log2e | delta][query]
-    static_assert(sizeof(bf16_t) * (2 * KV_ELEMS + 2 * STAGE) >= sizeof(float) * 4 * 2 * (D / 32) * 16 * 64,
+    float(*sstat)[2][64] = reinterpret_cast<float(*)[2][64]>(smem + kDkdvTiles<D>);
+    static_assert(sizeof(bf16_t) * kDkdvTiles<D> >= sizeof(float) * 4 * 2 * (D / 32) * 16 * 64,
                   "the final reduction parks four waves' accumulators in the tile memory");
     int doc_start, doc_len, kbk;
-    int bx, by;
-    xcd_head_blocks(p.nk * p.nsplit, bx, by);
-    __shared__ int s_find[kFindBlockInts];  // (no tile loads straight into LDS in this kernel: several LDS variables do no harm)
-    if (!find_block(p.cu, p.ndocs, p.s_len, p.T, bx, 128, doc_start, doc_len, kbk, s_find)) return;
+    if (!find_block(p.cu, p.ndocs, p.s_len, p.T, bx, 128, doc_start, doc_len, kbk, reinterpret_cast<int*>(smem + kDkdvLds<D> - 2 * kFindBlockInts))) return;
     kbk = (doc_len + 127) / 128 - 1 - kbk;  // rank 0 = most blocks of queries to walk = the piece's first keys
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wave & 3, half = wave >> 2;
@@ -650,7 +394,8 @@ __global__ __launch_bounds__(kDkdvThreads) void attn_bwd_dkdv_kernel(AttnParams 
 
     const bf16_t* qdoc = p.q + tok_off(doc_start, p.s_len, p.q_ss, p.q_sb);
     const bf16_t* dodoc = p.dout + tok_off(doc_start, p.s_len, p.do_ss, p.do_sb);
-    bf16x8 rq[NCH_Q], rdo[NCH_Q];
+    const bf16_t* odoc = p.o + tok_off(doc_start, p.s_len, p.o_ss, p.o_sb);
+    bf16x8 rq[NCH_Q], rdo[NCH_Q], ro[OWN_DELTA ? NCH_Q : 1];
     float rstat = 0.f;  // threads 0..63: lse*log2e of query tid; 64..127: delta of query tid-64
     auto load_iter = [&](int it) {
         const int hq = hq0 + it / nqt;
@@ -662,8 +407,9 @@ __global__ __launch_bounds__(kDkdvThreads) void attn_bwd_dkdv_kernel(AttnParams 
             n = n < doc_len ? n : doc_len - 1;
             rq[i] = *reinterpret_cast<const bf16x8*>(qdoc + (int64_t)hq * D + (int64_t)n * p.q_ss + (c % CH) * 8);
             rdo[i] = *reinterpret_cast<const bf16x8*>(dodoc + (int64_t)hq * D + (int64_t)n * p.do_ss + (c % CH) * 8);
+            if constexpr (OWN_DELTA) ro[i] = *reinterpret_cast<const bf16x8*>(odoc + (int64_t)hq * D + (int64_t)n * p.o_ss + (c % CH) * 8);
         }
-        if (tid < 128) {
+        if (tid < (OWN_DELTA ? 64 : 128)) {
             const int n = doc_start + row0 + (tid & 63);
             rstat = 0.f;
             if (n < tok_end) rstat = tid < 64 ? p.lse[(int64_t)hq * p.T + n] * kLog2e : p.delta[(int64_t)hq * p.T + n];
@@ -677,7 +423,18 @@ __global__ __launch_bounds__(kDkdvThreads) void attn_bwd_dkdv_kernel(AttnParams 
             *reinterpret_cast<bf16x8*>(sq + (c / CH) * LD + (c % CH) * 8) = rq[i];
             *reinterpret_cast<bf16x8*>(sq + TL::ELEMS + (c / CH) * LD + (c % CH) * 8) = rdo[i];
         }
-        if (tid < 128) sstat[stage][tid >> 6][tid & 63] = rstat;
+        if constexpr (OWN_DELTA) {
+#pragma unroll
+            for (int i = 0; i < NCH_Q; ++i) {  // the CH lanes that hold a row are neighbours
+                float sum = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sum += (float)ro[i][e] * (float)rdo[i][e];
+#pragma unroll
+                for (int x = 1; x < CH; x <<= 1) sum += __shfl_xor(sum, x, 64);
+                if (tid % CH == 0) sstat[stage][1][(tid + kDkdvThreads * i) / CH] = sum;
+            }
+        }
+        if (tid < (OWN_DELTA ? 64 : 128)) sstat[stage][tid >> 6][tid & 63] = rstat;
     };
     load_iter(0);
     store_iter(0);
@@ -824,6 +581,14 @@ __global__ __launch_bounds__(kDkdvThreads) void attn_bwd_dkdv_kernel(AttnParams 
     }
 }
 
+template <int D>
+__global__ __launch_bounds__(kDkdvThreads) void attn_bwd_dkdv_kernel(AttnParams p) {
+    __shared__ __attribute__((aligned(16))) bf16_t smem[kDkdvLds<D>];
+    int bx, by;
+    xcd_head_blocks(p.nk * p.nsplit, bx, by);
+    dkdv_block<D, false>(p, bx, by, smem);
+}
+
 // dK = scale * sum_parts partial dK, dV = sum_parts partial dV, parts added in index order; one thread per 8 columns
 template <int D>
 __global__ __launch_bounds__(kThreads) void attn_dkdv_combine_kernel(AttnParams p) {
@@ -862,16 +627,18 @@ __global__ __launch_bounds__(kThreads) void attn_dkdv_combine_kernel(AttnParams 
 // A fragment read from LDS feeds two MFMAs (the two query groups), as one 32x32x16 fragment feeds one MFMA of twice the work.
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-template <int D>
-__global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) {
+// LDS: per key group K0 V0 K1 V1, then the block search's scratch
+template <int D, int KG>
+constexpr int kDqLds = KG * 4 * Tile<D>::ELEMS + 2 * kFindBlockInts;
+
+template <int D, int KG>
+__device__ __forceinline__ void dq_block(const AttnParams& p, int bx, int by, bf16_t* smem_all) {
     using TL = Tile<D>;
-    constexpr int LD = TL::LD;
-    __shared__ __attribute__((aligned(16))) bf16_t smem[4 * TL::ELEMS + 2 * kFindBlockInts];  // K0 V0 K1 V1, block search scratch
     int doc_start, doc_len, qb;
-    int bx, by;
-    xcd_head_blocks(p.nq, bx, by);
-    if (!find_block(p.cu, p.ndocs, p.s_len, p.T, bx, 128, doc_start, doc_len, qb, reinterpret_cast<int*>(smem + 4 * TL::ELEMS))) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (!find_block(p.cu, p.ndocs, p.s_len, p.T, bx, 128, doc_start, doc_len, qb, reinterpret_cast<int*>(smem_all + KG * 4 * TL::ELEMS))) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    bf16_t* smem = smem_all + kgrp * 4 * TL::ELEMS;
     const int hq = by, hk = hq / (p.nq / p.nk);
     const int q0 = qb * 128, qw0 = q0 + wave * 32;
     const int j4 = lane >> 4, l16 = lane & 15;
@@ -900,11 +667,12 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) 
         acc += __shfl_xor(acc, 32, 64);
         dlt[qg] = acc;
         lse2[qg] = p.lse[(int64_t)hq * p.T + qtok] * kLog2e;
-        if (j4 == 0 && qi[qg] < doc_len) p.delta[(int64_t)hq * p.T + doc_start + qi[qg]] = acc;
+        if (kgrp == 0 && j4 == 0 && qi[qg] < doc_len) p.delta[(int64_t)hq * p.T + doc_start + qi[qg]] = acc;
     }
 
     const int kend = (q0 + 128 < doc_len ? q0 + 128 : doc_len);
-    const int ntiles = (kend + 63) / 64;
+    const int ntiles_all = (kend + 63) / 64;
+    const int ntiles = (ntiles_all - kgrp + KG - 1) / KG;  // this key group's: t = 0 .. stands for tile KG t + kgrp of the document
     const int64_t kh = (int64_t)hk * D;
     const bf16_t* kbase = p.k + tok_off(doc_start, p.s_len, p.k_ss, p.k_sb) + kh;
     const bf16_t* vbase = p.v + tok_off(doc_start, p.s_len, p.v_ss, p.v_sb) + kh;
@@ -912,7 +680,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) 
     kld.init(p.k_ss, lane, wave, 63);
     vld.init(p.v_ss, lane, wave, 63);
     auto issue_tile = [&](int t, int stage) {
-        const int row0 = t * 64;
+        const int row0 = (KG * t + kgrp) * 64;
         bf16_t* sk = smem + stage * 2 * TL::ELEMS;
         if (row0 + 64 <= doc_len) {
             kld.issue(kbase + (int64_t)row0 * p.k_ss, sk, wave);
@@ -925,7 +693,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) 
             ve.issue(vbase + (int64_t)row0 * p.v_ss, sk + TL::ELEMS, wave);
         }
     };
-    issue_tile(0, 0);
+    if (KG == 1 || ntiles > 0) issue_tile(0, 0);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
 
@@ -938,13 +706,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) 
             for (int r = 0; r < 4; ++r) dqacc[i][qg][r] = 0.f;
     const float sl2 = p.scale * kLog2e;
 
-    for (int t = 0; t < ntiles; ++t) {
+    for (int t = 0; t < (ntiles_all + KG - 1) / KG; ++t) {
         const int cur = t & 1;
         const bf16_t* sK = smem + cur * 2 * TL::ELEMS;
         const bf16_t* sV = sK + TL::ELEMS;
         if (t + 1 < ntiles) issue_tile(t + 1, cur ^ 1);  // that stage was last read before the barrier that ended tile t-1
-        const int key0 = t * 64;
-        if (key0 <= qw0 + 31) {
+        const int key0 = (KG * t + kgrp) * 64;
+        if ((KG == 1 || t < ntiles) && key0 <= qw0 + 31) {
             const bool on_diag = key0 + 63 > qw0;
 #pragma unroll
             for (int pb = 0; pb < 2; ++pb) {  // 32 keys at a time
@@ -1009,26 +777,74 @@ __global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) 
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces of the next tile are in LDS
         __syncthreads();
     }
+    int dt0 = 0;
+    constexpr int NDT_OUT = D / 16 / KG;  // 16-wide pieces of dQ that a wave finishes
+    if constexpr (KG == 2) {
+        // each wave finishes half of dQ, for which its partner in the other key group leaves its half in LDS (every wave is past its
+        // last tile since the barrier above)
+        float* park = reinterpret_cast<float*>(smem_all) + wave * (2 * NDT_OUT * 2 * 4 * 64) + lane * 4;
+        float* mine = park + kgrp * (NDT_OUT * 2 * 4 * 64);
+        float* other = park + (1 - kgrp) * (NDT_OUT * 2 * 4 * 64);
+        dt0 = kgrp * NDT_OUT;
+#pragma unroll
+        for (int i = 0; i < NDT_OUT; ++i)
+#pragma unroll
+            for (int qg = 0; qg < 2; ++qg) *reinterpret_cast<f32x4v*>(mine + (i * 2 + qg) * 256) = kgrp ? dqacc[i][qg] : dqacc[NDT_OUT + i][qg];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NDT_OUT; ++i)
+#pragma unroll
+            for (int qg = 0; qg < 2; ++qg)
+                dqacc[i][qg] = (kgrp ? dqacc[NDT_OUT + i][qg] : dqacc[i][qg]) + *reinterpret_cast<const f32x4v*>(other + (i * 2 + qg) * 256);
+    }
 #pragma unroll
     for (int qg = 0; qg < 2; ++qg) {
         if (qi[qg] >= doc_len) continue;
         bf16_t* dqrow = p.dq + tok_off(doc_start + qi[qg], p.s_len, p.dq_ss, p.dq_sb) + (int64_t)hq * D;
 #pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) {
+        for (int dt = 0; dt < NDT_OUT; ++dt) {
             bf16x4 w;
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[e] = (bf16_t)(dqacc[dt][qg][e] * p.scale);
-            *reinterpret_cast<bf16x4*>(dqrow + dt * 16 + 4 * j4) = w;
+            *reinterpret_cast<bf16x4*>(dqrow + (dt0 + dt) * 16 + 4 * j4) = w;
         }
     }
 }
+
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(AttnParams p) {
+    __shared__ __attribute__((aligned(16))) bf16_t smem[kDqLds<D, 1>];
+    int bx, by;
+    xcd_head_blocks(p.nq, bx, by);
+    dq_block<D, 1>(p, bx, by, smem);
+}
+
+// Both in one launch: workgroups 0 .. key_blocks - 1 are dK/dV blocks, the others dQ blocks with their key tiles shared out to
+// two groups of four waves.
+template <int D>
+__global__ __launch_bounds__(kDkdvThreads) void attn_bwd_both_kernel(AttnParams p, int key_blocks) {
+    __shared__ __attribute__((aligned(16))) bf16_t smem[kDkdvLds<D> > kDqLds<D, 2> ? kDkdvLds<D> : kDqLds<D, 2>];
+    int bx, by;
+    const int lin = blockIdx.x;
+    if (lin < key_blocks) {
+        heads_of(lin, p.nk * p.nsplit, bx, by);
+        dkdv_block<D, true>(p, bx, by, smem);
+    } else {
+        heads_of(lin - key_blocks, p.nq, bx, by);
+        dq_block<D, 2>(p, bx, by, smem);
+    }
+}
 // (explicit: the launches below alone have left the host-side launch stubs of some of these kernels undefined)
-template __global__ void attn_fwd_kernel<128>(AttnParams);
-template __global__ void attn_fwd_kernel<64>(AttnParams);
+template __global__ void attn_fwd_kernel<128, 1>(AttnParams);
+template __global__ void attn_fwd_kernel<64, 1>(AttnParams);
+template __global__ void attn_fwd_kernel<128, 2>(AttnParams);
+template __global__ void attn_fwd_kernel<64, 2>(AttnParams);
 template __global__ void attn_bwd_dkdv_kernel<128>(AttnParams);
 template __global__ void attn_bwd_dkdv_kernel<64>(AttnParams);
 template __global__ void attn_dkdv_combine_kernel<128>(AttnParams);
 template __global__ void attn_dkdv_combine_kernel<64>(AttnParams);
+template __global__ void attn_bwd_both_kernel<128>(AttnParams, int);
+template __global__ void attn_bwd_both_kernel<64>(AttnParams, int);
 template __global__ void attn_bwd_dq_kernel<128>(AttnParams);
 template __global__ void attn_bwd_dq_kernel<64>(AttnParams);
 
@@ -1043,6 +859,27 @@ int check_common(const char* name, int64_t T, int64_t s_len, int64_t nq, int64_t
     return EZL_OK;
 }
 
+}  // namespace
+
+namespace {
+// blocks: 128-row blocks of the launch; s_len: the longest document there can be.  While about every CU has one workgroup, a launch takes
+// its longest chain of tiles: sharing it out to two groups of waves pays for their sums being brought together where it has
+// six tiles or more, and with some CUs having two workgroups where it has many.  us, one group against two:
+//   d 64:  13 / 3 x 400 (130 blocks) 10.5, 9.8; 19 / 8 x 222 (266) 9.7, 12.9; 12 / 2 x 1024 (192) 18.9, 15.8; 22 / 3 x 558 (308) 14.4, 16.8;
+//          12 / 2 x 1541 (300) 27.4, 21.9; 18 / 2784 (396) 44.5, 34.8; 16 / 2 x 2048 (512) 34.8, 33.1
+//   d 128: 26 / 3 x 190 (130) 9.3, 10.3; 13 / 3 x 535 (169) 17.3, 17.1; 8 / 3206 (208) 51.1, 43.1; 24 / 2 x 700 (264) 20.7, 22.0; 32 / 1531
+//          (384) 37.5, 33.3; 36 / 4 x 384 (432) 19.7, 24.8; 31 / 1721 (434) 43.5, 44.0; 32 / 4096 (1024) 152, 166
+bool fwd_key_groups_pay(int64_t blocks, int64_t s_len) { return blocks <= 256 ? s_len >= 384 : blocks <= 384 && s_len >= 1024; }
+// dQ and dK/dV in one launch (dQ with two key groups): they fill each other's idle CUs and share their tails, at the price of one workgroup
+// of eight waves per CU for dQ and of the extra reads of O for dK/dV, which costs more once either kernel fills the chip (at d = 128 some
+// registers spill as well).  us, two launches against one:
+//   d 64:  10 / 2 x 194 (40 blocks) 18.8, 10.3; 13 / 3 x 400 (130) 27.9, 19.5; 12 / 2 x 1024 (192) 47.4, 28.8; 19 / 8 x 222 (266) 26.1, 29.8;
+//          22 / 3 x 558 (308) 37.5, 38.0; 12 / 2 x 1541 (300) 70, 59; 18 / 2784 (396) 115, 106; 12 / 8192 (768) 458, 473
+//   d 128: 33 / 3 x 92 (99) 21.0, 14.3; 26 / 3 x 190 (130) 27.6, 23.6; 8 / 4 x 512 (128) 42.3, 30.1; 31 / 8 x 83 (186) 24.2, 28.6; 13 / 3 x 535
+//          (169) 48.7, 39.0; 15 / 2219 (270) 140, 118; 32 / 1337 (352) 93.9, 94.6; 32 / 1531 (384) 107, 113; 16 / 4 x 1000 (512) 95, 113
+bool bwd_one_launch_pays(int64_t blocks, int64_t s_len, int64_t d) {
+    return blocks <= 128 || (blocks <= 256 && s_len >= 384) || (blocks <= (d == 64 ? 384 : 288) && s_len >= 1024);
+}
 }  // namespace
 
 // strides[8]: q_seq, q_batch, k_seq, k_batch, v_seq, v_batch, out_seq, out_batch (elements)
@@ -1060,9 +897,20 @@ extern "C" int ezl_attn_fwd(const void* q, const void* k, const void* v, void* o
     p.scale = scale;
     p.q_ss = strides[0]; p.q_sb = strides[1]; p.k_ss = strides[2]; p.k_sb = strides[3];
     p.v_ss = strides[4]; p.v_sb = strides[5]; p.o_ss = strides[6]; p.o_sb = strides[7];
+    if (attn_small_pays(total_tokens, s_len, nq, d, false)) {
+        attn_small_fwd(p, (int)d, (hipStream_t)stream);
+        EZL_LAUNCH_CHECK("ezl_attn_fwd");
+        return EZL_OK;
+    }
     const dim3 grid((unsigned)((total_tokens + 127) / 128 + ndocs + total_tokens / s_len), (unsigned)nq);
-    if (d == 128) hipLaunchKernelGGL(attn_fwd_kernel<128>, grid, dim3(kThreads), 0, (hipStream_t)stream, p);
-    else hipLaunchKernelGGL(attn_fwd_kernel<64>, grid, dim3(kThreads), 0, (hipStream_t)stream, p);
+    hipStream_t st = (hipStream_t)stream;
+    if (fwd_key_groups_pay(total_tokens / s_len * ((s_len + 127) / 128) * nq, s_len)) {
+        if (d == 128) hipLaunchKernelGGL((attn_fwd_kernel<128, 2>), grid, dim3(2 * kThreads), 0, st, p);
+        else hipLaunchKernelGGL((attn_fwd_kernel<64, 2>), grid, dim3(2 * kThreads), 0, st, p);
+    } else {
+        if (d == 128) hipLaunchKernelGGL((attn_fwd_kernel<128, 1>), grid, dim3(kThreads), 0, st, p);
+        else hipLaunchKernelGGL((attn_fwd_kernel<64, 1>), grid, dim3(kThreads), 0, st, p);
+    }
     EZL_LAUNCH_CHECK("ezl_attn_fwd");
     return EZL_OK;
 }
@@ -1113,13 +961,29 @@ extern "C" int ezl_attn_bwd(const void* q, const void* k, const void* v, const v
     p.do_ss = strides[8]; p.do_sb = strides[9]; p.dq_ss = strides[10]; p.dq_sb = strides[11];
     p.dk_ss = strides[12]; p.dk_sb = strides[13]; p.dv_ss = strides[14]; p.dv_sb = strides[15];
     hipStream_t st = (hipStream_t)stream;
+    if (attn_small_pays(total_tokens, s_len, nq, d, true)) {
+        attn_small_bwd(p, (int)d, st);
+        EZL_LAUNCH_CHECK("ezl_attn_bwd");
+        return EZL_OK;
+    }
     const unsigned nblk = (unsigned)((total_tokens + 127) / 128 + ndocs + total_tokens / s_len);
     const dim3 gridq(nblk, (unsigned)nq);
     const dim3 gridk(nblk, (unsigned)(nk * p.nsplit));
     int64_t gc = (total_tokens * nk * d / 8 + kThreads - 1) / kThreads;
     if (gc > 256 * 16) gc = 256 * 16;
-    // the dQ kernel goes first: it also produces delta = rowsum(dO * O), which the dK/dV kernel reads
-    if (d == 128) {
+    const bool both = bwd_one_launch_pays(total_tokens / s_len * ((s_len + 127) / 128) * nq, s_len, d);
+    // otherwise the dQ kernel goes first: it also produces delta = rowsum(dO * O), which the dK/dV kernel reads
+    if (both) {
+        const int key_blocks = (int)(nblk * nk * p.nsplit);
+        const dim3 grid((unsigned)(key_blocks + nblk * nq));
+        if (d == 128) {
+            hipLaunchKernelGGL(attn_bwd_both_kernel<128>, grid, dim3(kDkdvThreads), 0, st, p, key_blocks);
+            if (p.nsplit > 1) hipLaunchKernelGGL(attn_dkdv_combine_kernel<128>, dim3((unsigned)gc), dim3(kThreads), 0, st, p);
+        } else {
+            hipLaunchKernelGGL(attn_bwd_both_kernel<64>, grid, dim3(kDkdvThreads), 0, st, p, key_blocks);
+            if (p.nsplit > 1) hipLaunchKernelGGL(attn_dkdv_combine_kernel<64>, dim3((unsigned)gc), dim3(kThreads), 0, st, p);
+        }
+    } else if (d == 128) {
         hipLaunchKernelGGL(attn_bwd_dq_kernel<128>, gridq, dim3(kThreads), 0, st, p);
         hipLaunchKernelGGL(attn_bwd_dkdv_kernel<128>, gridk, dim3(kDkdvThreads), 0, st, p);
         if (p.nsplit > 1) hipLaunchKernelGGL(attn_dkdv_combine_kernel<128>, dim3((unsigned)gc), dim3(kThreads), 0, st, p);

@@ -8,7 +8,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB_DIR = os.path.join(PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libezl.so")
-SOURCES = ["api.cpp", "data_index.cpp", "norm.hip", "elementwise.hip", "cross_entropy.hip", "gemm.hip", "gemm_small.hip", "attention.hip", "optimizer.hip", "layer.cpp"]
+SOURCES = ["api.cpp", "data_index.cpp", "norm.hip", "elementwise.hip", "cross_entropy.hip", "gemm.hip", "gemm_small.hip", "attention.hip", "attention_small.hip", "optimizer.hip", "layer.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
          # packed-fp32 VALU forms are kept out of generated code on purpose

@@ -212,6 +212,60 @@ def test_weight_gradients_of_a_layer_in_one_launch(h, nq, nk, f, b, s, main_grad
         assert (got[n] - want[n]).norm() <= (1e-5 if main_grads else 2.0 ** -8) * want[n].norm(), n
 
 
+def attention_reference(q, k, v, do, cu):
+    """(out, lse, dq, dk, dv) in float64 on the GPU; documents cu over the (b s) tokens."""
+    s, b, nq, d = q.shape
+    nk, scale = k.shape[2], d ** -0.5
+    Q, KK, V, DO = (x.transpose(0, 1).reshape(s * b, -1, d).transpose(0, 1).double().contiguous() for x in (q, k, v, do))
+    out, dq, dk, dv = torch.zeros_like(Q), torch.zeros_like(Q), torch.zeros_like(KK), torch.zeros_like(V)
+    lse = torch.zeros(nq, s * b, device=q.device, dtype=torch.float64)
+    for a, e in zip(cu[:-1], cu[1:]):
+        later = torch.ones(e - a, e - a, dtype=torch.bool, device=q.device).triu(1)
+        for h in range(nq):
+            g = h // (nq // nk)
+            S = (Q[h, a:e] @ KK[g, a:e].t() * scale).masked_fill(later, float("-inf"))
+            P, dP = S.softmax(-1), DO[h, a:e] @ V[g, a:e].t()
+            lse[h, a:e] = S.logsumexp(-1)
+            out[h, a:e] = P @ V[g, a:e]
+            dS = P * (dP - (dP * P).sum(-1, keepdim=True)) * scale
+            dq[h, a:e] = dS @ KK[g, a:e]
+            dk[g, a:e] += dS.t() @ Q[h, a:e]
+            dv[g, a:e] += P.t() @ DO[h, a:e]
+    back = lambda x: x.transpose(0, 1).reshape(b, s, -1, d).transpose(0, 1)
+    return back(out), lse, back(dq), back(dk), back(dv)
+
+
+@pytest.mark.parametrize("d,nq,nk,b,s,cu", [
+    # 32 rows per workgroup: tile edges, waves without a tile, more tiles than waves, grouped queries, documents
+    (64, 2, 2, 1, 1, None), (64, 4, 1, 3, 31, None), (128, 2, 2, 2, 33, None), (64, 3, 3, 1, 255, None), (128, 2, 1, 1, 257, None),
+    (64, 4, 4, 2, 512, None), (128, 3, 1, 1, 640, None), (64, 8, 2, 1, 389, [0, 1, 2, 65, 129, 200, 389]), (128, 4, 2, 1, 330, [0, 96, 97, 330]),
+    (64, 2, 2, 2, 128, [0, 100, 128, 200, 256]),
+    # 128 rows, forward with two key groups, dQ and dK/dV in one launch (the last tile missing for a group, documents, split groups)
+    (64, 24, 24, 2, 385, None), (128, 16, 4, 3, 449, None), (128, 24, 24, 1, 513, None), (64, 40, 8, 1, 641, [0, 63, 64, 330, 641]),
+    (128, 40, 40, 1, 700, [0, 129, 700]),
+    # 128 rows, one launch for the backward only, then neither
+    (64, 60, 60, 2, 100, None), (128, 30, 15, 4, 130, None), (64, 64, 64, 8, 140, None)])
+def test_attention_for_every_split_of_the_work(K, d, nq, nk, b, s, cu):
+    """Against float64.  Inputs are exact; probabilities, dS and the results are rounded to bf16 (2^-9 each): 1e-2 of a result's norm.
+    dS is a difference that may cancel (a document of one token: exactly), off by scale |K| |dO . (O - its bf16 value)|."""
+    print("attention", d, nq, nk, b, s, cu, flush=True)
+    q, do = rnd(s, b, nq, d, seed=1), rnd(s, b, nq, d, seed=2)
+    kv = rnd(s, b, 2 * nk + 1, d, seed=3)  # strides other than the heads' width
+    k, v = kv[:, :, :nk], kv[:, :, nk:2 * nk]
+    cut = None if cu is None else torch.tensor(cu, device="cuda", dtype=torch.int32)
+    want = attention_reference(q, k, v, do, cu or [i * s for i in range(b + 1)])
+    out, lse = K.attn_fwd(q, k, v, cut)
+    got = (out, lse) + tuple(K.attn_bwd(q, k, v, out, do, lse, cut))
+    assert (lse - want[1]).abs().max() <= 1e-4
+    for name, x, w, cancels in zip(("out", "lse", "dq", "dk", "dv"), got, want, (0, 0, 1, 1, 0)):
+        assert (x.double() - w).norm() <= 1e-2 * w.norm() + cancels * 2.0 ** -8 * do.double().norm(), name
+    q[s // 2, 0, 0, 3] = float("nan")  # one query: its row of the result, nobody else's
+    out2, _ = K.attn_fwd(q, k, v, cut)
+    assert out2[s // 2, 0, 0].isnan().all()
+    out2[s // 2, 0, 0] = out[s // 2, 0, 0]
+    assert torch.equal(out2, out)
+
+
 @pytest.mark.parametrize("sizes", [[1], [4096, 4095, 4097, 3], [0, 8, 0, 70001], [1 + 37 * i for i in range(101)]])
 def test_optimizer_over_lists_of_tensors(K, sizes):
     """Chunk edges, empty tensors and more tensors than one launch takes: the norm against fp64, the update bit for bit against
