@@ -52,10 +52,9 @@ struct alignas(16) bf16x8_raw {
 
 __device__ __forceinline__ bf16x8 ld_bf16x8(const bf16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 __device__ __forceinline__ void st_bf16x8(bf16_t* p, bf16x8 v) { *reinterpret_cast<bf16x8*>(p) = v; }
-// Streaming forms for large tensors that are read or written once per kernel.  Measured inside the training step: they help
-// the kernels that move hundreds of MB (SwiGLU backward 92 -> 78 us, RMSNorm backward 42 -> 34 us) and hurt where a 33 MB
-// tensor goes from one kernel straight into the next (the consumer then misses the last-level cache), so only the former
-// use them.
+// Streaming forms: loads of what nobody reads again soon; stores only of results that do not fit the last-level cache anyway.  A kernel
+// that moves hundreds of MB gains from them by itself (SwiGLU backward 92 -> 78 us), but the kernels that read the result next lose
+// more than that where it would have stayed in the cache.
 __device__ __forceinline__ bf16x8 ld_bf16x8_nt(const bf16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)); }
 __device__ __forceinline__ void st_bf16x8_nt(bf16_t* p, bf16x8 v) { __builtin_nontemporal_store(v, reinterpret_cast<bf16x8*>(p)); }
 

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __r
                     if (HAS_DRES) o[i] += (float)drr[c][i];
                     dwacc[c][i] += dyv * xhat;
                 }
-                st_bf16x8_nt(dx + base + col, pack8(o));
+                st_bf16x8(dx + base + col, pack8(o));
             }
         }
     }
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_bwd_split_kernel(const bf16_t*
                     if (HAS_DRES) o[i] += (float)drr[c][i];
                     dwacc[c][i] += dyv * xhat;
                 }
-                st_bf16x8_nt(dxrow + c * 512, pack8(o));
+                st_bf16x8(dxrow + c * 512, pack8(o));
             }
         }
     }

@@ -266,6 +266,17 @@ def test_attention_for_every_split_of_the_work(K, d, nq, nk, b, s, cu):
     assert torch.equal(out2, out)
 
 
+def test_swiglu_results_larger_than_the_last_level_cache(K):
+    """Written past the caches: the same bits as in two calls of half the size."""
+    print("swiglu beyond the cache", flush=True)
+    n = (128 << 20) + 16
+    g, u, do = (rnd(n // 8, 8, seed=i) for i in (1, 2, 3))
+    out, (dg, du) = K.swiglu_fwd(g, u), K.swiglu_bwd(do, g, u)
+    for half in (slice(0, n // 16), slice(n // 16, n // 8)):
+        a, b = K.swiglu_bwd(do[half], g[half], u[half])
+        assert torch.equal(out[half], K.swiglu_fwd(g[half], u[half])) and torch.equal(dg[half], a) and torch.equal(du[half], b)
+
+
 @pytest.mark.parametrize("sizes", [[1], [4096, 4095, 4097, 3], [0, 8, 0, 70001], [1 + 37 * i for i in range(101)]])
 def test_optimizer_over_lists_of_tensors(K, sizes):
     """Chunk edges, empty tensors and more tensors than one launch takes: the norm against fp64, the update bit for bit against
