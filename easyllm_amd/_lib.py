@@ -84,6 +84,7 @@ _SPECIAL = {
     "ezl_attn_bwd_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64], _i64),
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
     "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
+    "ezl_gemm_group_form_workspace_bytes": ([_i32, _i32, _i64p, _i64p, _i64], _i64),
     "ezl_layer_bytes": ([_layerp, _i32], _i64),
     "ezl_sumsq_partials": ([], _i64),
     "ezl_sumsq_list_partials": ([_i32], _i64),
@@ -155,6 +156,12 @@ def gemm_workspace_bytes(M, N, K):
 def gemm_group_workspace_bytes(Ms, Ns, K):
     n = len(Ms)
     return load().ezl_gemm_group_workspace_bytes(n, (_i64 * n)(*Ms), (_i64 * n)(*Ns), K)
+
+
+@functools.lru_cache(maxsize=1024)
+def gemm_group_form_workspace_bytes(a_kc, Ms, Ns, K):
+    n = len(Ms)
+    return load().ezl_gemm_group_form_workspace_bytes(1 if a_kc else 0, n, (_i64 * n)(*Ms), (_i64 * n)(*Ns), K)
 
 
 def layer_bytes(layer, which):

@@ -524,26 +524,30 @@ SplitPlan make_plan(int64_t tiles, int64_t nk, void* workspace, int64_t workspac
 }
 
 // ---- which tile shape, and over how many workgroups a tile's reduction is split ------------------------------------------
-// The time of a launch is estimated for every shape as rounds x (K tiles x rate + fixed) and the cheapest one taken.  The
-// rates (us per 64-wide K tile of one workgroup per CU, or of two sharing a CU; the lower figure with the chip nearly empty,
-// the higher one full: clock and L2 bandwidth give way) and fixed costs (us: first load, epilogue, a workgroup's start) are
-// fits to products timed back to back:
-//                 few workgroups      chip full         fixed     from (M x N x K, us)
-//   256 x 256     1.00                1.30              12        4096^3 96, 4096 x 4096 x 11008 239, 1531 x 11008 x 4096 115
-//   256 x 128     0.60                0.77               6        2048 x 768 x 768 12.5, x 2048 25; 4000 x 2048 x 2048 31, x 5504 71;
-//                                                                 1531 x 4096 x 4096 (3/4 full) 46, x 22016 227
-//   128 x 128     0.64 (one per CU)   0.98 (two)         3        2048 x 768 x 768 10.4, x 2048 23; 4000 x 2048 x 2048 35, x 5504 87
-//   64 x 64       0.33 (one per CU)   0.40 (two)         3        1024 x 256 x 256 3.8, x 768 6.4; 1167 x 1024 x 1024 8.9, x 5632 38
-//   64 x 64 by 8 waves  0.19          0.27               3.2      1024 x 256 x 768 5.3, 256 x 256 x 1024 5.7, 1024 x 1024 x 1167 7.3
+// The time of a launch is estimated for every shape as rounds x (K tiles x rate + ends) and the cheapest one taken.  The rates are us per
+// 64-wide K tile of one workgroup per CU (two sharing a CU for 128 and 64 tiles), the lower one with the chip nearly empty, the higher one full:
+// clock and L2 bandwidth give way; the ends (first load, epilogue, a workgroup's start) us per round.  Weight gradients have rates of their
+// own: both operands go through transposing LDS reads, and results are mostly fp32.  Fits to 850 products of 256 - 8192 wide operands and
+// 200 - 16384 tokens, weights not in cache, each timed with every shape and several splits: the shape that is taken is 0.2 % (weight gradients
+// 0.6 %) slower than the best one on average.  M x N x K, us for 256 x 256, 256 x 128, 192 x 128, 128 x 128:
+//   1531 x 4096 x 4096     65, 50, 44, 57         1531 x 11008 x 4096   111, 152, 129, 153      4000 x 2048 x 2048    42, 32, 43, 34
+//   1531 x 4096 x 22016   248, 249, 226, 309      4000 x 5504 x 2048     90, 90, 95, 94         4096 x 4096 x 4096    93, 114, 129, 124
+//   as weight gradients:  4096 x 4096 x 1531  52, 59, 69, 54;  11008 x 4096 x 1531  135, 164, 179, 146;  5120 x 5120 x 4096  178, 222, 227, 213
 // A split reduction adds a launch and a trip of the fp32 partial tiles through the caches (2048 x 768 x 4096 as 256 x 128 tiles
 // split four ways: 26, of which 10 for that).
+struct Rates {
+    double low, high, ends;
+};
+constexpr Rates kRates[2][kGemmKinds] = {
+    {{0.72, 1.30, 8.8}, {0.57, 0.71, 6.5}, {0.54, 0.57, 5.4}, {0.69, 0.94, 3.25}, {0.275, 0.43, 2.6}, {0.187, 0.20, 3.3}},  // forward, input gradient
+    {{1.18, 1.30, 12.5}, {0.74, 0.83, 8}, {0.61, 0.695, 6}, {0.64, 0.80, 5}, {0.265, 0.45, 2.7}, {0.21, 0.218, 3.1}}};       // weight gradient
 constexpr double kReduceFixed = 4.0, kReduceBytesPerUs = 8e6;
 double reduce_cost(int64_t tiles, int64_t tile_elems, int64_t nsplit) {
     return kReduceFixed + (double)tiles * tile_elems * nsplit * 8 / kReduceBytesPerUs;
 }
-double cost_256(int64_t tiles, int64_t nk, bool split_ok) {
+double cost_256(const Rates& rate, int64_t tiles, int64_t nk, bool split_ok) {
     const SplitPlan p = make_plan(tiles, nk, split_ok ? (void*)16 : nullptr, INT64_MAX);
-    auto round = [&](int64_t groups, int64_t k) { return k * (1.0 + 0.3 * groups / kCus) + 12; };
+    auto round = [&](int64_t groups, int64_t k) { return k * (rate.low + (rate.high - rate.low) * groups / kCus) + rate.ends; };
     double t = (p.full / kCus) * round(kCus, nk);
     if (p.full % kCus) t += round(p.full % kCus, nk);
     if (p.nsplit > 1) {
@@ -552,16 +556,13 @@ double cost_256(int64_t tiles, int64_t nk, bool split_ok) {
     }
     return t;
 }
-double cost_small(int kind, int64_t tiles, int64_t nk, int64_t nsplit) {
+double cost_small(const Rates& rate, int kind, int64_t tiles, int64_t nk, int64_t nsplit) {
     const int64_t groups = tiles * nsplit, share = (nk + nsplit - 1) / nsplit;
     const bool two = kind == kTile128 || kind == kTile64;  // workgroups per CU
-    const double low = kind == kTile256x128 ? 0.60 : kind == kTile128 ? 0.64 : kind == kTile64 ? 0.33 : 0.19;
-    const double high = kind == kTile256x128 ? 0.77 : kind == kTile128 ? 0.98 : kind == kTile64 ? 0.40 : 0.27;
-    const double fixed = kind == kTile256x128 ? 6 : kind == kTile64Waves ? 3.2 : 3;
     const int64_t slots = two ? 2 * kCus : kCus, rest = groups % slots;
-    double t = (groups / slots) * (share * high + fixed);
+    double t = (groups / slots) * (share * rate.high + rate.ends);
     const double fill = (double)rest / kCus;  // (one workgroup per CU: the rate holds until the chip is nearly full)
-    if (rest) t += share * (two ? (rest > kCus ? high : low) : low + (high - low) * fill * fill * fill) + fixed;
+    if (rest) t += share * (two ? (rest > kCus ? rate.high : rate.low) : rate.low + (rate.high - rate.low) * fill * fill * fill) + rate.ends;
     if (nsplit > 1) t += reduce_cost(tiles, gemm_kind_bm(kind) * gemm_kind_bn(kind), nsplit);
     return t;
 }
@@ -571,14 +572,18 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
     return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 // `count` products over the same nk K tiles in one launch (256 x 256 takes one product); `room`: workspace bytes
-GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr) {
+GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr) {
+    const Rates* rates = kRates[wgrad];
+    // 128 x 128 tiles read every operand most often, which lists of weight gradients over many tokens feel: a layer's seven over 11918 tokens at
+    // h = 1024 400 us (estimate 309), with 256 x 128 tiles 354 (315).
+    const double list_128 = wgrad && count > 3 ? 1.05 : 1;
     GemmPlan best = {kTile256, 1};
     double t_best = 1e30;
     if (count == 1) {
         const int64_t tiles = tiles_of(kTile256, M[0], N[0]);
         const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
         const int64_t need = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * 4 : 0;
-        t_best = cost_256(tiles, nk, need <= room);
+        t_best = cost_256(rates[kTile256], tiles, nk, need <= room);
     }
     for (int kind = kTile256x128; kind < kGemmKinds; ++kind) {
         int64_t tiles = 0;
@@ -588,7 +593,7 @@ GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, in
             if (s > 1 && (kind == kTile64Waves || nk / s < 4 || tiles * s > 4 * kCus ||
                           tiles * s * gemm_kind_bm(kind) * gemm_kind_bn(kind) * 4 > room))
                 break;
-            const double t = cost_small(kind, tiles, nk, s);
+            const double t = cost_small(rates[kind], kind, tiles, nk, s) * (kind == kTile128 ? list_128 : 1);
             if (t < t_best) {
                 t_best = t;
                 best.kind = kind;
@@ -600,14 +605,14 @@ GemmPlan find_plan(int count, const int64_t* M, const int64_t* N, int64_t nk, in
     return best;
 }
 // The search takes 3 us, as long as a small product: a thread remembers its last 256 products by their sizes.
-GemmPlan choose_plan(int64_t M, int64_t N, int64_t nk, int64_t room) {
+GemmPlan choose_plan(bool wgrad, int64_t M, int64_t N, int64_t nk, int64_t room) {
     struct Entry {
         int64_t M, N, nk, room;
         GemmPlan plan;
     };
-    static thread_local Entry memo[256] = {};
-    Entry& e = memo[(uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ nk * 0x165667B19E3779F9ull) >> 56];
-    if (e.M != M || e.N != N || e.nk != nk || e.room != room) e = {M, N, nk, room, find_plan(1, &M, &N, nk, room)};
+    static thread_local Entry memo[2][256] = {};
+    Entry& e = memo[wgrad][(uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ nk * 0x165667B19E3779F9ull) >> 56];
+    if (e.M != M || e.N != N || e.nk != nk || e.room != room) e = {M, N, nk, room, find_plan(wgrad, 1, &M, &N, nk, room)};
     return e.plan;
 }
 int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const int64_t* N) {
@@ -618,36 +623,36 @@ int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const i
 // Products that share a reduction length (q / k / v or gate / up of one input, and their weight gradients) in one launch?  Worth
 // it where each of them leaves CUs idle: 1024 tokens at h = 256, q + k + v forward 3 x 4.7 us alone.  The launches of a long
 // batch fill the chip one by one, with the better 256 x 256 tiles (at 4096 tokens and h = 4096 one launch for q / k / v
-// measured 0.14 ms per four-layer step slower).  Between launches of the smaller tiles the estimates compare well; against the 256 x 256
-// kernels they flatter the one launch, which has to win by a tenth where each product alone takes those.  Estimated ratio -> measured
-// time apart and together, us (T tokens, width / widths; f forward, w weight gradient):
-//   smaller tiles alone     f 3072, 8192 / 8192, 2 x 1024 0.93 -> 462, 429; w 512, 8192 / 8192, 2 x 1024 0.96 -> 145, 134; f 8192, 1024 /
-//                           2 x 2816 0.98 -> 115, 104; w 1378, 4608 / 2 x 12288 0.99 -> 380, 370; at worst w 9200, 2048 / 3 x 2048 0.94 ->
-//                           242, 254
-//   256 x 256, to 0.9       f 2048, 5120 / 3 x 5120 0.81 -> 300, 286; w 14955, 3200 / 3 x 3200 0.82 -> 1028, 960; w 8192, 2048 / 2 x 5504
-//                           0.90 -> 361, 337; at worst w 2792, 1664 / 2 x 5504 0.86 -> 126, 132
-//   256 x 256, above        f 3072, 2048 / 2 x 5504 0.91 -> 140, 154; f 3600, 3072 / 3 x 3072 0.96 -> 188, 209; f 4797, 1664 / 2 x 5792 0.99 ->
-//                           151, 184; f 4096, 5120 / 3 x 5120 1.00 -> 537, 551; at best f 270, 7552 / 2 x 23872 0.91 -> 365, 330
-// Over 220 groups of widths 256 - 8192 and 256 - 16384 tokens with ratios of 0.72 - 1.08: 0.27 % behind the faster of the two on
-// average; by any estimated gain 0.74 %, by any gain where the products apart take under 115 us and a tenth above 0.65 %.
+// measured 0.14 ms per four-layer step slower).  The estimates compare well; where each product alone takes 256 x 256 tiles they still
+// flatter the one launch a little, which has to win by a twenty-fifth there.
+// Estimated ratio -> measured time apart and together, us (T tokens, width / widths; f forward, w weight gradient):
+//   smaller tiles alone     w 10604, 2176 / 2176, 2 x 512 0.76 -> 186, 132; f 1601, 4096 / 4096, 2 x 512 0.96 -> 85, 78; w 926, 6400 / 3 x 6400 0.98
+//                           -> 314, 281; at worst f 15975, 1664 / 1664, 2 x 384 0.94 -> 121, 132
+//   256 x 256, to 0.96      w 1910, 3072 / 3 x 3072 0.73 -> 170, 117; f 684, 4992 / 2 x 14744 0.92 -> 223, 199; w 4301, 4352 / 3 x 4352 0.95 -> 514,
+//                           443; at worst f 12911, 640 / 2 x 2160 0.96 -> 80, 83
+//   256 x 256, above        w 8316, 5888 / 5888, 2 x 1472 0.98 -> 868, 821; w 1221, 5504 / 3 x 5504 0.99 -> 255, 257; f 3298, 3840 / 2 x 11968 1.02
+//                           -> 491, 531; f 5851, 1664 / 2 x 4512 1.05 -> 147, 178
+// Over 240 groups of widths 256 - 8192 and 256 - 16384 tokens with estimated ratios of 0.7 - 1.1: 0.25 % (forward) and 0.39 % (weight gradients)
+// behind the faster of the two on average; without the margin 0.31 and 0.33 %, with one of a tenth 0.79 and 0.88 %.
 constexpr double kLaunchGap = 2.5;  // us between two launches of a stream: ramp down, ramp up
-constexpr double kMargin256 = 0.9;
+constexpr double kMargin256 = 0.96;
 struct GroupTimes {
     GemmPlan plan;           // of the one launch
     double together, apart;  // estimated us
     bool one;
 };
-GroupTimes group_times(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room) {
+GroupTimes group_times(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room) {
     struct Entry {
         int64_t M[kMaxProblems], N[kMaxProblems], K, room;
         GroupTimes times;
         int count;
+        bool wgrad;
     };
     static thread_local Entry memo[64] = {};
-    uint64_t hash = K * 0x165667B19E3779F9ull + count;
+    uint64_t hash = K * 0x165667B19E3779F9ull + 2 * count + wgrad;
     for (int i = 0; i < count; ++i) hash = (hash ^ (uint64_t)M[i]) * 0x9E3779B97F4A7C15ull + (uint64_t)N[i] * 0xC2B2AE3D27D4EB4Full;
     Entry& e = memo[hash >> 58];
-    bool same = e.count == count && e.K == K && e.room == room;
+    bool same = e.count == count && e.wgrad == wgrad && e.K == K && e.room == room;
     for (int i = 0; i < count && same; ++i) same = e.M[i] == M[i] && e.N[i] == N[i];
     if (!same) {
         const int64_t nk = (K + BK - 1) / BK;
@@ -656,34 +661,38 @@ GroupTimes group_times(int count, const int64_t* M, const int64_t* N, int64_t K,
         bool all_256 = true;
         for (int i = 0; i < count; ++i) {
             double t;
-            all_256 = find_plan(1, &M[i], &N[i], nk, room, &t).kind == kTile256 && all_256;
+            all_256 = find_plan(wgrad, 1, &M[i], &N[i], nk, room, &t).kind == kTile256 && all_256;
             g.apart += t;
             e.M[i] = M[i];
             e.N[i] = N[i];
         }
-        g.plan = find_plan(count, M, N, nk, room, &g.together);
+        g.plan = find_plan(wgrad, count, M, N, nk, room, &g.together);
         if (all_256) g.together /= kMargin256;
         g.one = g.together < g.apart;
         e.K = K;
         e.room = room;
         e.count = count;
+        e.wgrad = wgrad;
     }
     return e.times;
 }
-bool group_plan(int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
-    const GroupTimes g = group_times(count, M, N, K, room);
+bool group_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
+    const GroupTimes g = group_times(wgrad, count, M, N, K, room);
     plan = g.plan;
     return g.one;
 }
-// workspace of a product's plan; the 256 x 256 kernels' own where a launch has to fall back to them
+// workspace of a product's plan, whichever form it has; the 256 x 256 kernels' own where a launch has to fall back to them
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int64_t nk = (K + BK - 1) / BK, tiles = tiles_of(kTile256, M, N);
     const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
-    const int64_t big = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
-    const GemmPlan q = choose_plan(M, N, nk, INT64_MAX);
-    const int64_t small = small_plan_bytes(q, 1, &M, &N);
-    return q.kind == kTile256 ? big : (big > small ? big : small);
+    int64_t most = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
+    for (int wgrad = 0; wgrad < 2; ++wgrad) {
+        const GemmPlan q = choose_plan(wgrad, M, N, nk, INT64_MAX);
+        const int64_t small = q.kind == kTile256 ? 0 : small_plan_bytes(q, 1, &M, &N);
+        most = small > most ? small : most;
+    }
+    return most;
 }
 
 // Which 256 x 256 kernel: the 4-wave one moves a third fewer LDS bytes (the chip is bound by power on long products) and, with
@@ -753,7 +762,7 @@ void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t 
     constexpr int form = A_KC ? (B_KC ? (sizeof(OutT) == 4 ? 4 : 0) : 1) : (sizeof(OutT) == 4 ? 2 : 3);
     if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC) {
         if (small_stores_ok<OutT>(ldc)) {
-            const GemmPlan plan = choose_plan(M, N, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
+            const GemmPlan plan = choose_plan(!A_KC, M, N, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
             if (plan.kind != kTile256) {
                 GemmSmallArgs a = {};
                 a.p[0] = {(const bf16_t*)A, (const bf16_t*)B, C, lda, ldb, ldc, M, N, 0, 0, 0, accumulate};
@@ -893,7 +902,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
     if (small_stores_ok<bf16_t>(ldc)) {
-        const GemmPlan small = choose_plan(M, N, (ktot + BK - 1) / BK, workspace ? workspace_bytes : 0);
+        const GemmPlan small = choose_plan(false, M, N, (ktot + BK - 1) / BK, workspace ? workspace_bytes : 0);
         if (small.kind != kTile256) {
             GemmSmallArgs a = {};
             a.p[0] = {(const bf16_t*)A[0], (const bf16_t*)B[0], C, lda, ldb, ldc, (int)M, (int)N, 0, 0, 0, accumulate};
@@ -946,16 +955,24 @@ bool results_meet(int count, void* const* C, const int64_t* M, const int64_t* N,
 
 // Up to three independent products C[i] (=|+=) A[i] * B[i] over one reduction length K in one launch; one after the other where their
 // results share memory or have rows too far apart.
-// ezl_gemm_group_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
+// ezl_gemm_group_form_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
 constexpr int kGroupMax = 3;  // q / k / v
 static_assert(kGemmListMax == kMaxProblems, "a list goes out in one launch");
-extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
+extern "C" int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K) {
     if (count < 2 || count > kGroupMax || !M || !N || K <= 0) return -1;
     for (int i = 0; i < count; ++i)
         if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
     GemmPlan plan;
-    if (!group_plan(count, M, N, K, INT64_MAX, plan)) return -1;
+    if (!group_plan(!a_kc, count, M, N, K, INT64_MAX, plan)) return -1;
     return small_plan_bytes(plan, count, M, N);
+}
+// The form is not said: products with K = N are taken for the forward of square weights, others for weight gradients (gate and up are
+// long in both).  The workspace is enough for either form's plan.
+extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
+    const int64_t fwd = ezl_gemm_group_form_workspace_bytes(1, count, M, N, K), wgrad = ezl_gemm_group_form_workspace_bytes(0, count, M, N, K);
+    if (fwd < 0 && wgrad < 0) return -1;
+    if ((N[0] == K ? fwd : wgrad) < 0) return -1;
+    return fwd > wgrad ? fwd : wgrad;
 }
 
 extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
@@ -971,11 +988,11 @@ int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* 
     double in_pieces = kLaunchGap * (pieces - 1);
     int count = 0;
     for (int p = 0; p < pieces; ++p) {
-        const GroupTimes g = group_times(counts[p], M + count, N + count, K, INT64_MAX);
+        const GroupTimes g = group_times(true, counts[p], M + count, N + count, K, INT64_MAX);
         in_pieces += g.one ? g.together : g.apart;
         count += counts[p];
     }
-    const GroupTimes all = group_times(count, M, N, K, INT64_MAX);
+    const GroupTimes all = group_times(true, count, M, N, K, INT64_MAX);
     return all.together < in_pieces ? small_plan_bytes(all.plan, count, M, N) : -1;
 }
 
@@ -1007,8 +1024,8 @@ int gemm_list(int count, const void* const* A, const void* const* B, void* const
         return EZL_OK;
     }
     GemmPlan plan;
-    group_plan(count, M, N, K, INT64_MAX, plan);
-    if (small_plan_bytes(plan, count, M, N) > (workspace ? workspace_bytes : 0)) group_plan(count, M, N, K, 0, plan);
+    group_plan(!a_kc, count, M, N, K, INT64_MAX, plan);
+    if (small_plan_bytes(plan, count, M, N) > (workspace ? workspace_bytes : 0)) group_plan(!a_kc, count, M, N, K, 0, plan);
     if (plan.kind == kTile256) plan = {kTile256x128, 1};  // (a group of one: these kernels take one or more)
     a.K = (int)K;
     a.partial = (float*)workspace;

@@ -81,15 +81,15 @@ __device__ __forceinline__ void zero_acc(f32x4 (&acc)[TM][TN]) {
 }
 
 // =================================================================================================
-// 256 x 128 tile, 4 waves of 128 x 64, three LDS stages
+// 256 x 128 and 192 x 128 tiles, 2 x 2 waves, three LDS stages
 // =================================================================================================
-// The 4-wave kernel of gemm.hip (one wave per SIMD, one MFMA per compile-time step) with half the columns.  The three stages
-// (144 KiB) let the 12 wave loads of a K tile go out over both phases, one every fifth MFMA (the address unit needs 48 of the
+// The 4-wave kernel of gemm.hip (one wave per SIMD, one MFMA per compile-time step) with smaller tiles.  The three stages (256 x 128:
+// 144 KiB) let the wave loads of a K tile (12) go out over both phases, one every fifth MFMA (the address unit needs 48 of the
 // 64 MFMA slots of a K tile), two K tiles ahead of their use; a stage is free from the barrier in front of its K tile's second
 // phase on, because that phase works on fragments already in registers.
-template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
-__global__ __launch_bounds__(256, 1) void gemm_256x128_kernel(const GemmSmallArgs args) {
-    constexpr int TBM = 256, TBN = 128, TM = 8, TN = 4;
+template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL, int TBM, int TBN>
+__global__ __launch_bounds__(256, 1) void gemm_wide_kernel(const GemmSmallArgs args) {
+    constexpr int TM = TBM / 32, TN = TBN / 32;
     constexpr int STAGE = (TBM + TBN) * BK;
     __shared__ __attribute__((aligned(1024))) bf16_t smem[3 * STAGE];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256, 1) void gemm_256x128_kernel(const GemmSmallArg
     int tm, tn;
     tile_of(tile - p.first, p.tiles_m, p.tiles_n, tm, tn);
     const int m0 = tm * TBM, n0 = tn * TBN;
-    const int arow = (wave >> 1) * 128, brow = (wave & 1) * 64;
+    const int arow = (wave >> 1) * (TBM / 2), brow = (wave & 1) * (TBN / 2);
     TileLoader<A_KC, TBM, 4, KTAIL> la;
     TileLoader<B_KC, TBN, 4, KTAIL> lb;
     const int64_t a_blk = A_KC ? (int64_t)m0 * p.lda : (int64_t)m0;
@@ -114,10 +114,11 @@ __global__ __launch_bounds__(256, 1) void gemm_256x128_kernel(const GemmSmallArg
     f32x4 acc[TM][TN];
     zero_acc(acc);
 
-    constexpr int NA = 8, NL = 12;       // wave loads per K tile: A, and A + B
+    constexpr int NA = TM, NL = TM + TN;  // wave loads per K tile: A, and A + B
     constexpr int NF = TM + TN;          // fragments per k half
     constexpr int NM = TM * TN;          // MFMAs per phase
-    constexpr int RSTEP = 2, LSTEP = 5;  // a fragment read every RSTEP MFMAs of a phase, a load every LSTEP of both
+    constexpr int RSTEP = 2, LSTEP = 2 * NM / NL;  // a fragment read every RSTEP MFMAs of a phase, a load every LSTEP of both
+    static_assert(RSTEP * NF <= NM + RSTEP - 1, "all fragments of a k half are read during the other one");
     bf16x8 fa[2][TM], fb[2][TN];
     auto read_frag = [&](const bf16_t* sA, int ks, int buf, auto F) {
         constexpr int f = decltype(F)::value;
@@ -411,10 +412,13 @@ template <bool A_KC, bool B_KC, typename OutT, bool MULTI>
 void launch_kind(int kind, const GemmSmallArgs& a, bool tail, hipStream_t st) {
     const dim3 grid((unsigned)(a.ntiles * a.nsplit));
     switch (kind) {
-        case kTile256x128:
-            if (tail) hipLaunchKernelGGL((gemm_256x128_kernel<A_KC, B_KC, OutT, MULTI, true>), grid, dim3(256), 0, st, a);
-            else hipLaunchKernelGGL((gemm_256x128_kernel<A_KC, B_KC, OutT, MULTI, false>), grid, dim3(256), 0, st, a);
-            break;
+#define EZL_WIDE(BM_, BN_)                                                                                                                 \
+    if (tail) hipLaunchKernelGGL((gemm_wide_kernel<A_KC, B_KC, OutT, MULTI, true, BM_, BN_>), grid, dim3(256), 0, st, a);                  \
+    else hipLaunchKernelGGL((gemm_wide_kernel<A_KC, B_KC, OutT, MULTI, false, BM_, BN_>), grid, dim3(256), 0, st, a);                      \
+    break
+        case kTile256x128: EZL_WIDE(256, 128);
+        case kTile192x128: EZL_WIDE(192, 128);
+#undef EZL_WIDE
         case kTile128: hipLaunchKernelGGL((gemm_square_kernel<A_KC, B_KC, OutT, MULTI, 128, 2>), grid, dim3(256), 0, st, a); break;
         case kTile64: hipLaunchKernelGGL((gemm_square_kernel<A_KC, B_KC, OutT, MULTI, 64, 4>), grid, dim3(256), 0, st, a); break;
         default: hipLaunchKernelGGL((gemm_64_waves_kernel<A_KC, B_KC, OutT, MULTI>), grid, dim3(512), 0, st, a); break;

@@ -39,18 +39,19 @@ __device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int& 
 }
 
 // chunk (16 B) permutation of a k-major tile row: keeps the transpose reads of one wave instruction (four k rows x 32 B in each
-// of four k octets) on distinct banks.  Rows of 128 or more columns all start at bank 0; a 64-column row is half the banks
-// wide, so the row's parity already separates two of the four rows.
+// of four k octets) on distinct banks.  Rows of 128 or 256 columns all start at bank 0; a row of 64 (192) columns is half (one and a
+// half times) the banks wide, so the row's parity already separates two of the four rows.
 template <int R>
 __device__ __forceinline__ int kmajor_swizzle(int krow) {
-    if (R >= 128) return ((krow & 3) << 2) ^ (((krow >> 3) & 1) << 1);
+    if (R % 128 == 0) return ((krow & 3) << 2) ^ (((krow >> 3) & 1) << 1);
     return (((krow >> 1) & 1) << 2) ^ (((krow >> 3) & 1) << 1);
 }
 
 // One operand tile of R rows (k-contiguous) or columns (k-major) = R / 8 wave-instructions of 1 KiB each
 // (buffer_load_dwordx4 ... lds: lane l lands at base + 16 l).
 //   k-contiguous tile [R rows][64 k]:  instruction q covers rows 8q..8q+7; chunk c of row r sits in slot c ^ ((r>>1)&7)
-//   k-major tile      [64 k][R cols]:  instruction q covers 512 / R k rows; chunk c of k row sits in slot c ^ kmajor_swizzle(k)
+//   k-major tile      [64 k][R cols]:  instruction q covers 512 / R k rows (not whole ones with R = 192); chunk c of k row sits in slot
+//                                      c ^ kmajor_swizzle(k)
 // Wave w issues instructions q = w*NI .. w*NI+NI-1, i.e. one contiguous NI KiB piece of the tile: M0 (the LDS base) is
 // written once per 4 KiB and the instruction offset (i & 3) * 1024 selects the KiB.  That offset is also added to the global
 // address, so the per-lane byte offsets are stored with it already subtracted; they are kept 4 KiB high (and the
@@ -65,7 +66,6 @@ template <bool KC, int R, int NW, bool KTAIL>
 struct TileLoader {
     static constexpr int NI = R / 8 / NW;
     static constexpr int CPR = R / 8;       // k-major: chunks per k row
-    static constexpr int KPI = 64 / CPR;    // k-major: k rows per instruction
     uint32_t off[NI];  // byte offsets from (operand base + k advance - 4096)
     // dim: rows (columns) of the operand from this tile's first on; those past the edge re-read the last one, their results
     // are never stored
@@ -80,8 +80,8 @@ struct TileLoader {
                 const int gr = row < dim ? row : dim - 1;
                 e = (int64_t)gr * ld + c * 8;
             } else {
-                const int krow = KPI * q + lane / CPR;
-                const int c = (lane % CPR) ^ kmajor_swizzle<R>(krow);
+                const int krow = (q * 64 + lane) / CPR;
+                const int c = ((q * 64 + lane) % CPR) ^ kmajor_swizzle<R>(krow);
                 int col = c * 8;
                 col = col + 8 <= dim ? col : dim - 8;
                 e = (int64_t)krow * ld + col;
@@ -99,7 +99,7 @@ struct TileLoader {
         uint32_t o = off[I];
         if (KTAIL && kv < BK) {
             const int q = wave * NI + I;
-            const int k = KC ? ((lane & 7) ^ (((8 * q + (lane >> 3)) >> 1) & 7)) * 8 : KPI * q + lane / CPR;
+            const int k = KC ? ((lane & 7) ^ (((8 * q + (lane >> 3)) >> 1) & 7)) * 8 : (q * 64 + lane) / CPR;
             o = k < kv ? o : kBufBytes;
         }
         __builtin_amdgcn_raw_ptr_buffer_load_lds(g, (lds_void*)(stage + wave * (NI * 512) + (I >> 2) * 2048), 16, o, 0, (I & 3) * 1024, 0);
@@ -346,7 +346,8 @@ struct GemmSmallArgs {
 };
 
 // Tile shapes of gemm_small.hip, and 0 for the 256 x 256 kernels of gemm.hip.
-enum GemmKind { kTile256 = 0, kTile256x128 = 1, kTile128 = 2, kTile64 = 3, kTile64Waves = 4, kGemmKinds = 5 };
+enum GemmKind { kTile256 = 0, kTile256x128, kTile192x128, kTile128, kTile64, kTile64Waves, kGemmKinds };
+constexpr int kKindRows[kGemmKinds] = {256, 256, 192, 128, 64, 64}, kKindCols[kGemmKinds] = {256, 128, 128, 128, 64, 64};
 struct GemmPlan {
     int kind, nsplit;
 };
@@ -354,5 +355,5 @@ struct GemmPlan {
 // result; 4: as 0 with an fp32 result.  Sets the tile grids in `a` and launches; 256 rows of every problem's C must span less than 2 GiB.
 __attribute__((visibility("hidden"))) void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs& a, int count,
                                                              hipStream_t stream);
-inline int64_t gemm_kind_bm(int kind) { return kind <= kTile256x128 ? 256 : (kind == kTile128 ? 128 : 64); }
-inline int64_t gemm_kind_bn(int kind) { return kind == kTile256 ? 256 : (kind <= kTile128 ? 128 : 64); }
+inline int64_t gemm_kind_bm(int kind) { return kKindRows[kind]; }
+inline int64_t gemm_kind_bn(int kind) { return kKindCols[kind]; }

@@ -48,8 +48,8 @@ struct Saved {
 int64_t max64(int64_t a, int64_t b) { return a > b ? a : b; }
 
 // workspace of up to three products over one K, however they are launched
-int64_t products_ws(int count, const int64_t* M, const int64_t* N, int64_t K) {
-    const int64_t group = count > 1 ? ezl_gemm_group_workspace_bytes(count, M, N, K) : -1;
+int64_t products_ws(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K) {
+    const int64_t group = count > 1 ? ezl_gemm_group_form_workspace_bytes(a_kc, count, M, N, K) : -1;
     if (group >= 0) return group;
     int64_t w = 0;
     for (int i = 0; i < count; ++i) w = max64(w, ezl_gemm_workspace_bytes(M[i], N[i], K));
@@ -82,7 +82,7 @@ struct ForwardTemp {
         wide = b.take(m.T * m.h * 2);                                     // o / down result
         bias_in = l.bq ? b.take(m.T * (m.qw + 2 * m.kw) * 2) : nullptr;  // q, k, v before their bias
         const int64_t Tq[3] = {m.T, m.T, m.T}, nqkv[3] = {m.qw, m.kw, m.kw}, ngu[2] = {m.f, m.f};
-        ws_bytes = max64(products_ws(3, Tq, nqkv, m.h), products_ws(2, Tq, ngu, m.h));
+        ws_bytes = max64(products_ws(1, 3, Tq, nqkv, m.h), products_ws(1, 2, Tq, ngu, m.h));
         ws_bytes = max64(ws_bytes, max64(ezl_gemm_workspace_bytes(m.T, m.h, m.qw), ezl_gemm_workspace_bytes(m.T, m.h, m.f)));
         ws = b.take(ws_bytes);
         bytes = b.used;
@@ -100,7 +100,7 @@ struct BackwardTemp {
         dqkv = b.take(m.T * (m.qw + 2 * m.kw) * 2);  // dq | dk | dv in one row, so that one launch can reduce over all three
         delta = b.take(m.nq * m.T * 4);
         const int64_t mqkv[3] = {m.qw, m.kw, m.kw}, hh[3] = {m.h, m.h, m.h}, mgu[2] = {m.f, m.f};
-        int64_t w = max64(products_ws(3, mqkv, hh, m.T), products_ws(2, mgu, hh, m.T));
+        int64_t w = max64(products_ws(0, 3, mqkv, hh, m.T), products_ws(0, 2, mgu, hh, m.T));
         w = max64(w, max64(ezl_gemm_workspace_bytes(m.qw, m.h, m.T), ezl_gemm_workspace_bytes(m.f, m.h, m.T)));  // (also one by one)
         w = max64(w, max64(ezl_gemm_workspace_bytes(m.kw, m.h, m.T), ezl_gemm_workspace_bytes(m.h, m.qw, m.T)));
         w = max64(w, max64(ezl_gemm_workspace_bytes(m.h, m.f, m.T), ezl_gemm_workspace_bytes(m.T, m.f, m.h)));
@@ -127,7 +127,7 @@ int forward_products(int count, const void* x, const void* const* w, void* const
     const int64_t Ts[3] = {T, T, T}, ks[3] = {k, k, k};
     const void* xs[3] = {x, x, x};
     const int zero[3] = {0, 0, 0};
-    if (count > 1 && ezl_gemm_group_workspace_bytes(count, Ts, n, k) >= 0)
+    if (count > 1 && ezl_gemm_group_form_workspace_bytes(1, count, Ts, n, k) >= 0)
         return ezl_gemm_bf16_group(count, xs, w, y, Ts, n, k, ks, ks, n, 1, 1, 0, zero, ws, ws_bytes, st);
     for (int i = 0; i < count; ++i) EZL_TRY(ezl_gemm_bf16(x, w[i], y[i], T, n[i], k, k, k, n[i], 1, 1, 0, 0, ws, ws_bytes, st));
     return EZL_OK;
@@ -146,7 +146,7 @@ int weight_gradients(int count, const void* const* dy, int64_t ld, const void* x
         acc[i] = g[i].accumulate;
         one = one && out[i] && (g[i].f32 != nullptr) == (g[0].f32 != nullptr);
     }
-    if (one && ezl_gemm_group_workspace_bytes(count, n, ks, T) >= 0)
+    if (one && ezl_gemm_group_form_workspace_bytes(0, count, n, ks, T) >= 0)
         return ezl_gemm_bf16_group(count, dy, xs, out, n, ks, T, lds, ks, ks, 0, 0, g[0].f32 ? 1 : 0, acc, ws, ws_bytes, st);
     for (int i = 0; i < count; ++i)
         if (out[i])

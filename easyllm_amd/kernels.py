@@ -345,7 +345,7 @@ def linear_wgrad(dy2d, x2d, out=None, accumulate=False):
 
 
 def gemm_group(As, Bs, Ms, Ns, K, ldas, ldbs, a_kc, b_kc, outs, accumulates, ws_bytes):
-    """Products over one reduction length in one launch; ws_bytes as gemm_group_workspace_bytes says for these sizes.  Operands
+    """Products over one reduction length in one launch; ws_bytes as gemm_group_form_workspace_bytes says for these sizes.  Operands
     and outputs have been checked by the callers below."""
     n = len(As)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=outs[0].device) if ws_bytes else None
@@ -356,18 +356,18 @@ def gemm_group(As, Bs, Ms, Ns, K, ldas, ldbs, a_kc, b_kc, outs, accumulates, ws_
               _stream())
 
 
-def _group_ws(Ms, Ns, K):
+def _group_ws(a_kc, Ms, Ns, K):
     """Workspace bytes of one launch for these products, or -1: separate launches (also for empty ones)."""
     if not 2 <= len(Ms) <= 3 or K == 0:
         return -1
-    return _lib.gemm_group_workspace_bytes(Ms, Ns, K)
+    return _lib.gemm_group_form_workspace_bytes(a_kc, Ms, Ns, K)
 
 
 def linear_fwd_multi(x2d, ws):
     """[x2d @ w_i^T]: linears that share their input, in one launch where that is faster."""
     T, n_in = x2d.shape
     Ns = tuple(w.shape[0] for w in ws)
-    nbytes = _group_ws((T,) * len(ws), Ns, n_in)
+    nbytes = _group_ws(True, (T,) * len(ws), Ns, n_in)
     if nbytes < 0:
         return [linear_fwd(x2d, w) for w in ws]
     lda, ldbs = _rows_ld(x2d, "x"), [_rows_ld(w, "w") for w in ws]
@@ -383,7 +383,7 @@ def linear_wgrad_multi(dy2ds, x2d, outs, accumulates):
     T, n_in = x2d.shape
     Ms = tuple(dy.shape[1] for dy in dy2ds)
     n = len(dy2ds)
-    nbytes = _group_ws(Ms, (n_in,) * n, T) if len({None if o is None else o.dtype for o in outs}) == 1 else -1
+    nbytes = _group_ws(False, Ms, (n_in,) * n, T) if len({None if o is None else o.dtype for o in outs}) == 1 else -1
     if nbytes < 0:
         return [linear_wgrad(dy, x2d, out=o, accumulate=acc) for dy, o, acc in zip(dy2ds, outs, accumulates)]
     ldas, ldb = [_rows_ld(dy, "dy") for dy in dy2ds], _rows_ld(x2d, "x")

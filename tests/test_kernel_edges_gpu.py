@@ -97,6 +97,23 @@ def test_gemm_smaller_tiles(K, form, M, N, Kd):
     check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
 
 
+@pytest.mark.parametrize("form,M,N,Kd", [
+    # 192 x 128: K tails, ragged edges, element-wise stores, reductions split two to nine ways
+    (0, 1780, 2328, 344), (1, 742, 2720, 904), (0, 1099, 3819, 368), (0, 1531, 4096, 4096), (0, 392, 4688, 2680), (1, 453, 2752, 3368),
+    (0, 556, 952, 5752), (2, 3456, 1336, 400), (2, 2224, 2168, 403), (3, 904, 4848, 467), (2, 904, 2488, 2160), (3, 384, 3240, 2765),
+    # 256 x 128
+    (0, 1195, 4816, 696), (1, 1209, 5008, 672), (0, 3872, 1648, 720), (0, 1009, 2808, 3040), (1, 423, 4704, 3568)])
+def test_gemm_wide_tiles(K, form, M, N, Kd):
+    print("gemm", form, M, N, Kd, flush=True)
+    check_gemm(K, form, M, N, Kd)
+    check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
+    if form == 0:
+        x, w = rnd(M, Kd, seed=1), rnd(N, Kd, seed=2)
+        f = K.linear_fwd(x, w, fp32_output=True)
+        tol = gemm_bound(x, w.t()) + f.abs() * 2.0 ** -8 + 1e-6
+        assert torch.equal(f, f.bfloat16().float()) and ((f - x.float() @ w.float().t()).abs() <= tol).all()
+
+
 @pytest.mark.parametrize("T,n_in,outs", [(1167, 1024, (1024, 256, 256)), (2048, 768, (2048, 2056)), (700, 3072, (3072, 1024, 1032)),
                                          (4000, 2048, (2048, 2048, 2056)), (1024, 256, (256, 256, 256))])
 def test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs):
@@ -110,6 +127,11 @@ def test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs):
     assert ((dx.float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
     K.linear_dgrad_multi(dys, ws, out=dx, accumulate=True)
     assert ((dx.float() - 2 * ref).abs() <= 2 * gemm_bound(A, B) + ref.abs() * 2.0 ** -6 + 1e-6).all()
+
+
+@pytest.mark.parametrize("T,n_in,outs", [(742, 2720, (304, 304, 296)), (453, 2752, (1128, 1120, 1120))])
+def test_gemm_input_gradient_over_pairs_on_wide_tiles(K, T, n_in, outs):
+    test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs)
 
 
 def test_gemm_smaller_tiles_leave_what_is_outside_the_result_alone(K):
