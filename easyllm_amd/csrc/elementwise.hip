@@ -260,6 +260,74 @@ __global__ __launch_bounds__(kBlock) void embed_bucket_kernel(const int64_t* __r
     }
 }
 
+// The four kernels above as one workgroup, for batches of up to kSmallRows: each of those launches costs more than its work there
+// (2 x 512 tokens at V = 32000: 2.7, 3.3, 5.8, 3.2 us and the gaps between them, now 6.8).  Ids are looked up in a hash table in LDS, so the global
+// tables are only written: cnt / first / off of the ids that occur, and, with zero_all, cnt = 0 of all others.
+constexpr int kSmallRows = 4096, kSmallSlots = 2 * kSmallRows, kSmallThreads = 1024;
+constexpr int64_t kSmallVocab = 131072;  // a single workgroup clears that many counts in 3 us
+__global__ __launch_bounds__(kSmallThreads) void embed_tables_small_kernel(const int64_t* __restrict__ ids, int* __restrict__ cnt, int* __restrict__ first,
+                                                                           int* __restrict__ off, int* __restrict__ bucket, int* __restrict__ cursor,
+                                                                           int* __restrict__ heavy, int rows, int64_t V, int zero_all) {
+    __shared__ int s_id[kSmallSlots], s_cnt[kSmallSlots], s_first[kSmallSlots], s_off[kSmallSlots];
+    __shared__ int s_next, s_heavy;
+    constexpr int PER = kSmallRows / kSmallThreads;
+    const int tid = threadIdx.x;
+    int row_id[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int r = k * kSmallThreads + tid;
+        const int64_t id = r < rows ? ids[r] : -1;
+        row_id[k] = id >= 0 && id < V ? (int)id : -1;
+    }
+    // (2048, 4096 or 8192 slots, the hash's highest bits: at most half of them are ever taken)
+    const int shift = rows <= kSmallSlots / 8 ? 21 : (rows <= kSmallSlots / 4 ? 20 : 19), slots = 1 << (32 - shift);
+    for (int i = tid; i < slots; i += kSmallThreads) {
+        s_id[i] = -1;
+        s_cnt[i] = 0;
+        s_first[i] = 0x7fffffff;
+    }
+    if (tid == 0) s_next = s_heavy = 0;
+    if (zero_all)
+        for (int64_t i = tid; i < V; i += kSmallThreads) cnt[i] = 0;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the zeros have arrived before the counts below are stored
+    __syncthreads();
+    int slot[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int r = k * kSmallThreads + tid;
+        slot[k] = -1;
+        const int id = row_id[k];
+        if (id < 0) continue;
+        unsigned i = ((unsigned)id * 0x9E3779B1u) >> shift;
+        for (;;) {  // ends: half of the slots stay free
+            const int old = atomicCAS(&s_id[i], -1, id);
+            if (old == -1 || old == id) break;
+            i = (i + 1) & (slots - 1);
+        }
+        slot[k] = (int)i;
+        atomicAdd(&s_cnt[i], 1);
+        atomicMin(&s_first[i], r);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int r = k * kSmallThreads + tid;
+        if (slot[k] < 0 || s_first[slot[k]] != r) continue;
+        const int id = s_id[slot[k]], n = s_cnt[slot[k]], o = atomicAdd(&s_next, n);
+        s_off[slot[k]] = o;
+        cnt[id] = n;
+        first[id] = r;
+        off[id] = o;
+        if (n > kOwnedRows) heavy[atomicAdd(&s_heavy, 1)] = id;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (slot[k] >= 0) bucket[atomicAdd(&s_off[slot[k]], 1)] = k * kSmallThreads + tid;
+    if (tid == 0) cursor[1] = s_heavy;
+}
+static_assert(kSmallSlots == 1 << (32 - 19), "the largest table");
+
 // p[0 .. n4) = 0 in 16-byte pieces: a block clears one contiguous 16 KiB chunk (4 stores per thread), chunks dealt to blocks in
 // order, so the blocks running at any moment sweep one window of the buffer.
 __global__ __launch_bounds__(kBlock) void zero_f32x4_kernel(f32x4* __restrict__ p, int64_t n4) {
@@ -903,14 +971,6 @@ int embed_gradient(const char* name, const void* ids, const void* dy, void* dwei
     int* cursor = bucket + rows;
     int* heavy = cursor + 4;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(embed_tables_init_kernel, dim3(grid_for(vocab, kBlock, 1024)), dim3(kBlock), 0, st, cnt, first, fill, cursor, vocab);
-    hipLaunchKernelGGL(embed_count_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, cnt, first,
-                       rows, vocab);
-    hipLaunchKernelGGL(embed_assign_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, cnt, first, off,
-                       cursor, heavy, rows, vocab);
-    hipLaunchKernelGGL(embed_bucket_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, off, fill,
-                       bucket, rows, vocab);
-    EZL_LAUNCH_CHECK(name);
     // one workgroup per token row (accumulate) or per vocabulary row, whichever is more: the zero fill of the rows that
     // received nothing is most of the traffic when the result overwrites the buffer
     // Overwriting a large table ([152064, 5120] fp32 = 3.1 GB, say) is mostly a zero fill, and a flat fill kernel in front
@@ -922,6 +982,19 @@ int embed_gradient(const char* name, const void* ids, const void* dy, void* dwei
         hipLaunchKernelGGL(zero_f32x4_kernel, dim3(grid_for(n4, 4 * kBlock, (int64_t)1 << 20)), dim3(kBlock), 0, st, (f32x4*)dweight, n4);
     }
     const int overwrite = accumulate || flat_fill ? 0 : 1;
+    if (rows <= kSmallRows && (!overwrite || vocab <= kSmallVocab)) {
+        hipLaunchKernelGGL(embed_tables_small_kernel, dim3(1), dim3(kSmallThreads), 0, st, (const int64_t*)ids, cnt, first, off, bucket, cursor,
+                           heavy, (int)rows, vocab, overwrite);
+    } else {
+        hipLaunchKernelGGL(embed_tables_init_kernel, dim3(grid_for(vocab, kBlock, 1024)), dim3(kBlock), 0, st, cnt, first, fill, cursor, vocab);
+        hipLaunchKernelGGL(embed_count_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, cnt, first,
+                           rows, vocab);
+        hipLaunchKernelGGL(embed_assign_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, cnt, first, off,
+                           cursor, heavy, rows, vocab);
+        hipLaunchKernelGGL(embed_bucket_kernel, dim3(grid_for(rows, kBlock, 1024)), dim3(kBlock), 0, st, (const int64_t*)ids, off, fill,
+                           bucket, rows, vocab);
+    }
+    EZL_LAUNCH_CHECK(name);
     const dim3 grid(grid_for(overwrite ? (rows > vocab ? rows : vocab) : rows, 1));
     if (h <= 8 * kBlock * 2)
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<2, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,

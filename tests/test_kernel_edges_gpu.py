@@ -513,3 +513,29 @@ def test_embedding_gradient_in_bf16_is_the_fp32_one_rounded(K, V, h, rows, frequ
     K.embed_scatter_add(ids, dy, ref, accumulate=False)
     got = K.embed_grad_bf16(ids, dy, V)
     assert got.dtype is torch.bfloat16 and torch.equal(got, ref.bfloat16())
+
+
+@pytest.mark.parametrize("V,h,rows,ids", [(32000, 256, 1024, "random"), (5000, 64, 4096, "distinct"), (50304, 72, 1167, "padding"), (131072, 64, 4095, "far apart"),
+                                          (40, 128, 3000, "few"), (1, 8, 33, "random"), (131073, 64, 900, "random"), (300, 64, 500, "out of range")])
+def test_embedding_gradient_with_and_without_the_one_workgroup_tables(K, V, h, rows, ids):
+    """Batches of up to 4096 rows build their tables in one workgroup.  Rows with an id outside the table are skipped, so the same
+    batch with 4097 of them behind it goes the general way: equal bit for bit, overwriting and adding."""
+    print("embedding tables", V, h, rows, ids, flush=True)
+    g = torch.Generator().manual_seed(rows)
+    t = torch.randint(0, V, (rows,), generator=g)
+    if ids == "distinct":
+        t = torch.randperm(V, generator=g)[:rows]
+    elif ids == "padding":
+        t[rows // 2:] = 0
+    elif ids == "far apart":
+        t = torch.arange(rows) * 32 % V
+    elif ids == "out of range":
+        t[::7], t[::11] = V, -1
+    long = torch.cat([t, torch.full((4097,), V)]).cuda()
+    dy = torch.cat([rnd(rows, h, seed=4), torch.full((4097, h), float("nan"), device="cuda", dtype=torch.bfloat16)])
+    for accumulate in (False, True):
+        got, want = torch.full((V, h), 2.5, device="cuda"), torch.full((V, h), 2.5, device="cuda")
+        K.embed_scatter_add(t.cuda(), dy[:rows].contiguous(), got, accumulate=accumulate)
+        K.embed_scatter_add(long, dy, want, accumulate=accumulate)
+        assert torch.equal(got, want)
+    assert torch.equal(K.embed_grad_bf16(t.cuda(), dy[:rows].contiguous(), V), K.embed_grad_bf16(long, dy, V))
