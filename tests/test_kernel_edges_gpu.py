@@ -539,3 +539,33 @@ def test_embedding_gradient_with_and_without_the_one_workgroup_tables(K, V, h, r
         K.embed_scatter_add(long, dy, want, accumulate=accumulate)
         assert torch.equal(got, want)
     assert torch.equal(K.embed_grad_bf16(t.cuda(), dy[:rows].contiguous(), V), K.embed_grad_bf16(long, dy, V))
+
+
+@pytest.mark.parametrize("rows,V,cut", [(3, 32776, 0), (700, 40960, 0), (2100, 40968, 0), (5, 50304, 304), (1167, 53256, 0), (9, 65536, 9), (4, 65544, 0),
+                                        (6, 73720, 1000)])
+def test_loss_and_gradient_of_rows_kept_as_bf16_in_registers(K, rows, V, cut):
+    """Edges of the register counts, cut columns, ignored rows, labels in the cut, more rows than blocks; against float64.  The sum of V
+    fp32 exponentials is off by V 2^-24 at most, the gradient by that and one rounding to bf16."""
+    print("loss", rows, V, cut, flush=True)
+    x = rnd(rows, V, seed=3, scale=2.0)
+    labels = torch.randint(0, V - cut, (rows,), generator=torch.Generator().manual_seed(1)).cuda()
+    labels[::5] = -100
+    if cut:
+        labels[1] = V - 1
+    w, count = K.ce_prepare(labels, None, -100)
+    loss, grad = K.ce_fused(x, labels, w, count, cut, inplace=False)
+    for r in list(range(min(rows, 12))) + [rows - 1]:
+        xd, t = x[r].double(), labels[r].item()
+        if t == -100:
+            assert loss[r] == 0 and (grad[r] == 0).all()
+            continue
+        masked = t >= V - cut
+        lse = xd[:V - cut].logsumexp(0)
+        want = lse - (xd[:V - cut].max() if masked else xd[t])
+        assert abs(loss[r].double() - want) <= V * 2.0 ** -24 + 1e-5
+        g = (xd - lse).exp()
+        if not masked:
+            g[t] -= 1
+        g /= count.double()
+        assert ((grad[r].double() - g).abs() <= g.abs() * (2.0 ** -8 + V * 2.0 ** -23) + 2.0 ** -126).all()
+    assert torch.equal(K.ce_fused(x, labels, w, count, cut)[1], grad)  # in place: the same bits
