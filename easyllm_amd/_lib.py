@@ -40,7 +40,9 @@ SIGNATURES = {
     "ezl_rope_apply": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _vp],
     "ezl_rope_apply_pair": [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "ezl_ids_in_range": [_vp, _i64, _i64, _vp, _vp],
+    "ezl_ids_in_range_host_flag": [_vp, _i64, _i64, _vp, _vp],
     "ezl_embed_gather": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "ezl_embed_gather_host_flag": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "ezl_embed_scatter_add": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "ezl_embed_grad_bf16": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "ezl_transpose01": [_vp, _vp, _i64, _i64, _i64, _vp],

@@ -140,29 +140,43 @@ __global__ __launch_bounds__(kBlock) void rope_kernel(RopeSide a, RopeSide b2, c
 // ---------------------------------------------------------------------------------------------
 // Token embedding (base_modules/layers/vocab_parallel_emb.py:106-137, TP=1)
 // ---------------------------------------------------------------------------------------------
-// ORs 1 into *bad_flag if some id >= limit, 2 if some id < 0 (the range test of an index tensor, without a host sync)
-__global__ __launch_bounds__(kBlock) void ids_in_range_kernel(const int64_t* __restrict__ ids, int64_t n, int64_t limit,
-                                                              int* __restrict__ bad_flag) {
+// What a range test found, 1 for an id >= limit and 2 for a negative one: ORed into a word of device memory, or, HOST, byte 0 and
+// byte 1 of pinned host memory set by plain stores.  Those need neither a clearing launch before the kernel nor a copy behind it,
+// which cost a host-bound step 8 us of host time and the GPU a copy-engine hand-over; an atomic OR on host memory is not among
+// those that PCIe carries.
+template <bool HOST>
+__device__ __forceinline__ void raise_id_flag(void* flag, int bad) {
+    if constexpr (HOST) {
+        if (bad & 1) ((volatile unsigned char*)flag)[0] = 1;
+        if (bad & 2) ((volatile unsigned char*)flag)[1] = 1;
+    } else if (bad) {
+        atomicOr((int*)flag, bad);
+    }
+}
+
+// the range test of an index tensor, without a host sync
+template <bool HOST>
+__global__ __launch_bounds__(kBlock) void ids_in_range_kernel(const int64_t* __restrict__ ids, int64_t n, int64_t limit, void* bad_flag) {
     int bad = 0;
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
         const int64_t id = ids[i];
         bad |= id >= limit ? 1 : (id < 0 ? 2 : 0);
     }
-    if (bad) atomicOr(bad_flag, bad);
+    raise_id_flag<HOST>(bad_flag, bad);
 }
 
 // out[r, :] = W[ids[r], :]; an id outside [0, V) raises the flag and yields a zero row.
 // One wave per row; a lane's loads (up to 8 vectors of 8 at a time: a row of 4096 in one go) are all in flight before its
 // first store.
+template <bool HOST>
 __global__ __launch_bounds__(kBlock) void embed_gather_kernel(const int64_t* __restrict__ ids, const bf16_t* __restrict__ W,
-                                                              bf16_t* __restrict__ out, int64_t rows, int h, int64_t V,
-                                                              int* __restrict__ bad_flag) {
+                                                              bf16_t* __restrict__ out, int64_t rows, int h, int64_t V, void* bad_flag) {
     const int h8 = h >> 3;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int64_t r = (int64_t)blockIdx.x * 4 + wave; r < rows; r += (int64_t)gridDim.x * 4) {
         const int64_t id = ids[r];
         const bool ok = id >= 0 && id < V;
-        if (!ok && lane == 0) atomicOr(bad_flag, id >= V ? 1 : 2);
+        if (!ok && lane == 0) raise_id_flag<HOST>(bad_flag, id >= V ? 1 : 2);
         const bf16_t* src = W + (ok ? id : 0) * h;
         bf16_t* dst = out + r * h;
         for (int c0 = lane; c0 < h8; c0 += 512) {
@@ -921,26 +935,50 @@ extern "C" int ezl_rope_apply_pair(const void* q, void* q_out, int64_t nq, int64
                        cos_table, sin_table, position_ids, s, b, d, npos, backward, stream);
 }
 
-extern "C" int ezl_ids_in_range(const void* ids, int64_t n, int64_t limit, void* bad_flag, void* stream) {
-    EZL_REQUIRE(n >= 0 && bad_flag && (n == 0 || ids), EZL_EINVAL, "ezl_ids_in_range: null pointer");
+namespace {
+
+template <bool HOST>
+int launch_ids_in_range(const char* name, const void* ids, int64_t n, int64_t limit, void* bad_flag, void* stream) {
+    EZL_REQUIRE(n >= 0 && bad_flag && (n == 0 || ids), EZL_EINVAL, "%s: null pointer", name);
     if (n == 0) return EZL_OK;
-    hipLaunchKernelGGL(ids_in_range_kernel, dim3(grid_for(n, kBlock, 256)), dim3(kBlock), 0, (hipStream_t)stream, (const int64_t*)ids,
-                       n, limit, (int*)bad_flag);
-    EZL_LAUNCH_CHECK("ezl_ids_in_range");
+    hipLaunchKernelGGL((ids_in_range_kernel<HOST>), dim3(grid_for(n, kBlock, 256)), dim3(kBlock), 0, (hipStream_t)stream,
+                       (const int64_t*)ids, n, limit, bad_flag);
+    EZL_LAUNCH_CHECK(name);
     return EZL_OK;
+}
+
+template <bool HOST>
+int launch_embed_gather(const char* name, const void* ids, const void* weight, void* out, void* bad_flag, int64_t rows, int64_t h,
+                        int64_t vocab, void* stream) {
+    EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h < (1LL << 31) && vocab > 0, EZL_EUNSUPPORTED,
+                "%s: h must be a multiple of 8", name);
+    EZL_REQUIRE(bad_flag && (rows == 0 || (ids && weight && out)) && ezl_aligned16(weight) && ezl_aligned16(out), EZL_EINVAL,
+                "%s: null or misaligned pointer", name);
+    if (rows == 0) return EZL_OK;
+    hipLaunchKernelGGL((embed_gather_kernel<HOST>), dim3(grid_for((rows + 3) / 4, 1)), dim3(kBlock), 0, (hipStream_t)stream,
+                       (const int64_t*)ids, (const bf16_t*)weight, (bf16_t*)out, rows, (int)h, vocab, bad_flag);
+    EZL_LAUNCH_CHECK(name);
+    return EZL_OK;
+}
+
+}  // namespace
+
+extern "C" int ezl_ids_in_range(const void* ids, int64_t n, int64_t limit, void* bad_flag, void* stream) {
+    return launch_ids_in_range<false>("ezl_ids_in_range", ids, n, limit, bad_flag, stream);
+}
+
+extern "C" int ezl_ids_in_range_host_flag(const void* ids, int64_t n, int64_t limit, void* host_flag, void* stream) {
+    return launch_ids_in_range<true>("ezl_ids_in_range_host_flag", ids, n, limit, host_flag, stream);
 }
 
 extern "C" int ezl_embed_gather(const void* ids, const void* weight, void* out, void* bad_flag, int64_t rows, int64_t h,
                                 int64_t vocab, void* stream) {
-    EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h < (1LL << 31) && vocab > 0, EZL_EUNSUPPORTED,
-                "ezl_embed_gather: h must be a multiple of 8");
-    EZL_REQUIRE(bad_flag && (rows == 0 || (ids && weight && out)) && ezl_aligned16(weight) && ezl_aligned16(out), EZL_EINVAL,
-                "ezl_embed_gather: null or misaligned pointer");
-    if (rows == 0) return EZL_OK;
-    hipLaunchKernelGGL(embed_gather_kernel, dim3(grid_for((rows + 3) / 4, 1)), dim3(kBlock), 0, (hipStream_t)stream, (const int64_t*)ids,
-                       (const bf16_t*)weight, (bf16_t*)out, rows, (int)h, vocab, (int*)bad_flag);
-    EZL_LAUNCH_CHECK("ezl_embed_gather");
-    return EZL_OK;
+    return launch_embed_gather<false>("ezl_embed_gather", ids, weight, out, bad_flag, rows, h, vocab, stream);
+}
+
+extern "C" int ezl_embed_gather_host_flag(const void* ids, const void* weight, void* out, void* host_flag, int64_t rows, int64_t h,
+                                          int64_t vocab, void* stream) {
+    return launch_embed_gather<true>("ezl_embed_gather_host_flag", ids, weight, out, host_flag, rows, h, vocab, stream);
 }
 
 extern "C" int64_t ezl_embed_scatter_add_workspace_bytes(int64_t rows, int64_t vocab) {

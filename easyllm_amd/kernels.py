@@ -162,20 +162,28 @@ def rope_apply_pair(q, k, cos, sin, position_ids=None, backward=False):
     return qo, ko
 
 
-def ids_in_range_flag(ids, limit):
-    """-> int32 [1] GPU flag: bit 0 set if some id >= limit, bit 1 if some id < 0."""
+def ids_in_range_flag(ids, limit, host_flag=None):
+    """-> int32 [1] GPU flag: bit 0 set if some id >= limit, bit 1 if some id < 0.  With host_flag (int32 [1], pinned, zero): None, and
+    bits 0 and 8 of that, once the launch has run."""
     _need(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous(), "ids must be contiguous int64 on the GPU")
+    if host_flag is not None:
+        _lib.call("ezl_ids_in_range_host_flag", _p(ids), ids.numel(), int(limit), _p(host_flag), _stream())
+        return None
     flag = torch.zeros(1, dtype=torch.int32, device=ids.device)
     _lib.call("ezl_ids_in_range", _p(ids), ids.numel(), int(limit), _p(flag), _stream())
     return flag
 
 
 # ------------------------------------------------------------------------------------- embedding
-def embed_gather(ids, weight):
+def embed_gather(ids, weight, host_flag=None):
+    """-> rows, flag (as `ids_in_range_flag`)"""
     _need(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous(), "ids must be contiguous int64 on the GPU")
     _bf16c(weight, "weight")
     V, h = weight.shape
     out = torch.empty(tuple(ids.shape) + (h,), dtype=BF16, device=weight.device)
+    if host_flag is not None:
+        _lib.call("ezl_embed_gather_host_flag", _p(ids), _p(weight), _p(out), _p(host_flag), ids.numel(), h, V, _stream())
+        return out, None
     flag = torch.zeros(1, dtype=torch.int32, device=weight.device)
     _lib.call("ezl_embed_gather", _p(ids), _p(weight), _p(out), _p(flag), ids.numel(), h, V, _stream())
     return out, flag

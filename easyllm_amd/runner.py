@@ -9,6 +9,7 @@ number of accumulation steps and ZeRO partitioning are DeepSpeed's and are not r
 import torch
 
 from .registry import MODULE_ZOO_REGISTRY
+from . import functional as _F
 from . import llama as _llama  # (registers the model builders)
 from .losses import CrossEntropy
 from .transformer import is_plain
@@ -51,8 +52,9 @@ def _logits_stay_inside(model):
 
 def forward_step(model, inputs, labels):
     """One micro-batch: returns the loss tensor after backward has run."""
-    output = model(inputs, cast_logits=False) if _logits_stay_inside(model) else model(inputs)
-    loss = model.loss_fn(output, labels)
+    with _F.input_checks_at_the_end():  # (before any gradient is written)
+        output = model(inputs, cast_logits=False) if _logits_stay_inside(model) else model(inputs)
+        loss = model.loss_fn(output, labels)
     loss.backward()
     return loss
 

@@ -74,6 +74,11 @@ int ezl_rope_apply(const void* x, void* out, const void* cos_table, const void* 
  * fails on an index past the table): ORs 1 into *bad_flag (device int32) if some id >= limit, 2 if some id < 0.  The apply
  * kernels themselves clamp. */
 int ezl_ids_in_range(const void* ids_i64, int64_t n, int64_t limit, void* bad_flag, void* stream);
+/* ezl_ids_in_range / ezl_embed_gather with the flag in pinned host memory that the caller holds at zero: byte 0 becomes 1 for an id
+ * at or past the limit, byte 1 for a negative one; to be read after an event recorded behind the call */
+int ezl_ids_in_range_host_flag(const void* ids_i64, int64_t n, int64_t limit, void* host_flag, void* stream);
+int ezl_embed_gather_host_flag(const void* ids, const void* weight, void* out, void* host_flag, int64_t rows, int64_t h, int64_t vocab,
+                               void* stream);
 /* the same rotation of q [.., nq, d] and k [.., nk, d] of one layer (llama/transformer.py:437-448) in one launch */
 int ezl_rope_apply_pair(const void* q, void* q_out, int64_t nq, int64_t q_in_stride, int64_t q_out_stride, const void* k,
                         void* k_out, int64_t nk, int64_t k_in_stride, int64_t k_out_stride, const void* cos_table,

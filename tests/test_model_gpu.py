@@ -209,6 +209,31 @@ def test_bad_token_id_raises_value_error(gpu_device):
         functional.set_input_check("sync")
 
 
+@pytest.mark.parametrize("bad", ["id", "negative", "both", "position"])
+def test_a_step_with_a_bad_index_raises_before_any_gradient(gpu_device, bad):
+    """forward_step waits for its index checks behind the forward pass: same errors as a plain call, and nothing is written."""
+    from easyllm_amd import runner
+    model = runner.build_model({"type": "llama_custom", "kwargs": dict(
+        num_layers=1, hidden_size=256, num_attention_heads=4, intermediate_size=512, vocab_size=512, seq_length=64, bf16=True)}).cuda()
+    runner.attach_main_grads(model)
+    gen = torch.Generator().manual_seed(3)
+    tokens, labels = (torch.randint(1, 512, (1, 64), generator=gen).to(gpu_device) for _ in range(2))
+    pos, cu = torch.arange(64, device=gpu_device)[None], torch.tensor([0, 64], device=gpu_device)
+    target = labels, torch.ones(1, 64, device=gpu_device)
+    good = runner.forward_step(model, (tokens, pos, None, cu), target)
+    before = [p.main_grad.clone() for p in model.parameters()]
+    ids = tokens.clone()
+    if bad != "position":
+        ids[0, 5], ids[0, 41] = (512, -1) if bad == "both" else ((512, 3) if bad == "id" else (3, -1))
+    wrong = ids, pos + (bad == "position"), None, cu
+    for call in (lambda: runner.forward_step(model, wrong, target), lambda: model(wrong)):
+        with pytest.raises(ValueError if bad in ("id", "both") else IndexError):
+            call()
+    assert all(torch.equal(p.main_grad, b) for p, b in zip(model.parameters(), before))
+    runner.zero_main_grads(model)
+    assert torch.equal(runner.forward_step(model, (tokens, pos, None, cu), target), good)
+
+
 def test_position_id_beyond_the_rotary_table_raises_index_error(gpu_device):
     """The reference indexes its cos / sin tables (one row per sequence position) with the position ids; an id past the
     table is an indexing error there (positional_embeddings.py:109-117).  Same here, from the embedding stage."""
