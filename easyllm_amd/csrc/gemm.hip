@@ -271,10 +271,17 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // 4096 911 -> 885.  What is left there is the power limit: longer K loops run at 1.2 - 1.35 us per K tile instead of 0.96.
 // C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base), its tile-relative byte offsets
 // must fit 31 bits, and every item must have two K tiles or more: the host side checks.
-template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
+// LIST (weight gradients): the tiles of several products over one K; what is said per product comes from the list then, not from the other
+// arguments.  A decoder layer's seven over 4000 tokens (h = 2048, f = 5504: 784 tiles, three rounds and 16 tiles) went out as 128 x 128 tiles in
+// 453 us, as these in 387.  (One product in a list of one would save the form without it, but costs 6 us a launch: a tile's scalar loads
+// depend on one another.)
+struct NoList {};
+template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL, bool LIST = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                          int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
-                                                         int tiles_m, int tiles_n, int items, const SplitPlan plan, const KSegments seg) {
+                                                         int tiles_m, int tiles_n, int items, const SplitPlan plan, const KSegments seg,
+                                                         const std::conditional_t<LIST, GemmSmallArgs, NoList> list) {
+    static_assert(!LIST || (!A_KC && !B_KC && !MULTI), "lists are of weight gradients");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[4 * DTILE];  // A0 B0 A1 B1
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -284,7 +291,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     const int64_t bstep = B_KC ? BK : (int64_t)BK * ldb;
     const int arow = wm * 128, brow = wn * 128;
 
-    struct Item {  // a whole tile, or a tile of the split last round with this workgroup's share of its K tiles
+    struct ListItem {  // its product, its operands from the tile's corner on, their strides, the tile's rows and columns
+        int product, lda, ldb, mrem, nrem;
+        const bf16_t *a, *b;
+    };
+    struct Item : std::conditional_t<LIST, ListItem, NoList> {  // a whole tile, or a tile of the split last round with this workgroup's share of its K tiles
         int m0, n0, kt0, nk;
         int slot;  // >= 0: place of the partial tile
         int64_t a_blk, b_blk;
@@ -304,7 +315,16 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             it.nk = (int)((int64_t)nk_all * (part + 1) / plan.nsplit) - it.kt0;
         }
         int tm, tn;
-        tile_of(pid, tiles_m, tiles_n, tm, tn);
+        if constexpr (LIST) {
+            pid = __builtin_amdgcn_readfirstlane(pid);
+            it.product = 0;
+#pragma unroll
+            for (int j = 1; j < kMaxProblems; ++j) it.product += pid >= list.first[j];
+            const GemmProblem& p = list.p[it.product];
+            tile_of(pid - p.first, p.tiles_m, p.tiles_n, tm, tn);
+        } else {
+            tile_of(pid, tiles_m, tiles_n, tm, tn);
+        }
         // (scalar registers: the buffer bases are made of them)
         it.m0 = __builtin_amdgcn_readfirstlane(tm * BM);
         it.n0 = __builtin_amdgcn_readfirstlane(tn * BN);
@@ -313,15 +333,48 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
         it.slot = __builtin_amdgcn_readfirstlane(it.slot);
         it.a_blk = A_KC ? (int64_t)it.m0 * lda : (int64_t)it.m0;
         it.b_blk = B_KC ? (int64_t)it.n0 * ldb : (int64_t)it.n0;
+        if constexpr (LIST) {
+            const GemmProblem& p = list.p[it.product];
+            it.a = p.A + it.m0;
+            it.b = p.B + it.n0;
+            it.lda = (int)p.lda;
+            it.ldb = (int)p.ldb;
+            it.mrem = min(p.M - it.m0, BM);
+            it.nrem = min(p.N - it.n0, BN);
+            // (these scalar loads are waited for here, not inside the K loop)
+            asm volatile("" ::"s"(it.a), "s"(it.b), "s"(it.lda), "s"(it.ldb), "s"(it.mrem), "s"(it.nrem));
+        }
         return it;
     };
+    auto rows_left = [&](const Item& x) {
+        if constexpr (LIST) return x.mrem;
+        else return M - x.m0;
+    };
+    auto cols_left = [&](const Item& x) {
+        if constexpr (LIST) return x.nrem;
+        else return N - x.n0;
+    };
+    auto a_stride = [&](const Item& x) {
+        if constexpr (LIST) return (int64_t)x.lda;
+        else return lda;
+    };
+    auto b_stride = [&](const Item& x) {
+        if constexpr (LIST) return (int64_t)x.ldb;
+        else return ldb;
+    };
+    if constexpr (LIST) {  // every cache line of the list, fetched at once: the loads below depend on one another
+        int line[kMaxProblems];
+#pragma unroll
+        for (int j = 0; j < kMaxProblems; ++j) line[j] = list.p[j].M;
+        asm volatile("" ::"s"(line[0]), "s"(line[1]), "s"(line[2]), "s"(line[3]), "s"(line[4]), "s"(line[5]), "s"(line[6]), "s"(list.first[6]));
+    }
     int u = blockIdx.x;
     Item it = item_of(u);
 
     TileLoader<A_KC, BM, 4, KTAIL> la;
     TileLoader<B_KC, BN, 4, KTAIL> lb;
-    la.init(lane, wave, M - it.m0, lda);
-    lb.init(lane, wave, N - it.n0, ldb);
+    la.init(lane, wave, rows_left(it), a_stride(it));
+    lb.init(lane, wave, cols_left(it), b_stride(it));
 
     FragReader<A_KC> ra;
     FragReader<B_KC> rb;
@@ -341,6 +394,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     auto tile_bases = [&](const Item& x, int t) {
         const bf16_t *Ab, *Bb;
         t += x.kt0;
+        if constexpr (LIST) {
+            kv = K - t * BK;
+            ga = la.base(x.a + (int64_t)t * BK * x.lda);
+            gb = lb.base(x.b + (int64_t)t * BK * x.ldb);
+            return;
+        }
         pick_segment<MULTI>(A, B, K, seg, t, kv, Ab, Bb);
         ga = la.base(Ab + x.a_blk + (int64_t)t * astep);
         gb = lb.base(Bb + x.b_blk + (int64_t)t * bstep);
@@ -419,8 +478,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             flip();
         }
         // the last two K tiles bring in the first two of the next tile (the last item's: its own again, into stages nobody reads)
-        if (min(M - next.m0, BM) != min(M - it.m0, BM)) la.init(lane, wave, M - next.m0, lda);
-        if (min(N - next.n0, BN) != min(N - it.n0, BN)) lb.init(lane, wave, N - next.n0, ldb);
+        if (min(rows_left(next), BM) != min(rows_left(it), BM) || (LIST && a_stride(next) != a_stride(it))) la.init(lane, wave, rows_left(next), a_stride(next));
+        if (min(cols_left(next), BN) != min(cols_left(it), BN) || (LIST && b_stride(next) != b_stride(it))) lb.init(lane, wave, cols_left(next), b_stride(next));
         tile_bases(next, 0);
         phase_b(smem + s1, smem + s0);
         phase_a(smem + s1);
@@ -442,6 +501,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
                     *reinterpret_cast<f32x4*>(tile + (arow + i * 16 + (lane & 15)) * BN + brow + j * 16 + 4 * (lane >> 4)) = from_agprs<64>(acc[i][j]);
+        } else if constexpr (LIST) {
+            const GemmProblem& p = list.p[it.product];
+            OutT* Ct = (OutT*)p.C + (int64_t)it.m0 * p.ldc + it.n0;
+            store_tile_flags<8, 8, OutT, true, false>(acc, Ct, p.ldc, it.mrem, it.nrem, arow, brow, lane, p.accumulate);
         } else {
             const int mrem = M - it.m0 < BM ? M - it.m0 : BM;
             OutT* Ct = C + (int64_t)it.m0 * ld + it.n0;
@@ -571,19 +634,28 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
     const int64_t bm = gemm_kind_bm(kind), bn = gemm_kind_bn(kind);
     return ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
-// `count` products over the same nk K tiles in one launch (256 x 256 takes one product); `room`: workspace bytes
-GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr) {
+// A list on 256 x 256 tiles has to win by a fourteenth: its tiles cost a chain of scalar loads each, and many rounds of short reductions are
+// bound by the results' way to memory, whatever the launches.  Forward and backward of a layer with its weight gradients in such a list
+// against without, by estimated ratio of the weight gradients (T, h, kv heads, f; us):
+//   0.76 - 0.80   8192, 2048, 16, 5504 3867 -> 3680; 4000, 2048, 16, 5504 1905 -> 1835; 10086, 1024, 8, 3328 2471 -> 2432
+//   0.80 - 0.93   4810, 2560, 20, 7744 3443 -> 3313; 1691, 2944, 23, 9216 1667 -> 1631; 2048, 4096, 8, 14336 2900 -> 2860; 2780, 2688, 21, 9408
+//                 2283 -> 2205; at worst 2963, 1024, 2, 3392 707 -> 716
+//   0.93 - 1.00   1531, 4096, 32, 11008 2180 -> 2216; 8569, 896, 14, 2976 1772 -> 1787; 1331, 3200, 25, 9984 1589 -> 1550
+constexpr double kMarginList256 = 0.93;
+// `count` products over the same nk K tiles in one launch; `room`: workspace bytes.  256 x 256 tiles take one product, or with list_256 all
+GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr, bool list_256 = false) {
     const Rates* rates = kRates[wgrad];
     // 128 x 128 tiles read every operand most often, which lists of weight gradients over many tokens feel: a layer's seven over 11918 tokens at
     // h = 1024 400 us (estimate 309), with 256 x 128 tiles 354 (315).
     const double list_128 = wgrad && count > 3 ? 1.05 : 1;
     GemmPlan best = {kTile256, 1};
     double t_best = 1e30;
-    if (count == 1) {
-        const int64_t tiles = tiles_of(kTile256, M[0], N[0]);
+    if (count == 1 || list_256) {
+        int64_t tiles = 0;
+        for (int i = 0; i < count; ++i) tiles += tiles_of(kTile256, M[i], N[i]);
         const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
         const int64_t need = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * 4 : 0;
-        t_best = cost_256(rates[kTile256], tiles, nk, need <= room);
+        t_best = cost_256(rates[kTile256], tiles, nk, need <= room) / (list_256 ? kMarginList256 : 1);
     }
     for (int kind = kTile256x128; kind < kGemmKinds; ++kind) {
         int64_t tiles = 0;
@@ -641,18 +713,18 @@ struct GroupTimes {
     double together, apart;  // estimated us
     bool one;
 };
-GroupTimes group_times(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room) {
+GroupTimes group_times(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, bool list_256 = false) {
     struct Entry {
         int64_t M[kMaxProblems], N[kMaxProblems], K, room;
         GroupTimes times;
         int count;
-        bool wgrad;
+        bool wgrad, list_256;
     };
     static thread_local Entry memo[64] = {};
     uint64_t hash = K * 0x165667B19E3779F9ull + 2 * count + wgrad;
     for (int i = 0; i < count; ++i) hash = (hash ^ (uint64_t)M[i]) * 0x9E3779B97F4A7C15ull + (uint64_t)N[i] * 0xC2B2AE3D27D4EB4Full;
     Entry& e = memo[hash >> 58];
-    bool same = e.count == count && e.wgrad == wgrad && e.K == K && e.room == room;
+    bool same = e.count == count && e.wgrad == wgrad && e.list_256 == list_256 && e.K == K && e.room == room;
     for (int i = 0; i < count && same; ++i) same = e.M[i] == M[i] && e.N[i] == N[i];
     if (!same) {
         const int64_t nk = (K + BK - 1) / BK;
@@ -666,18 +738,19 @@ GroupTimes group_times(bool wgrad, int count, const int64_t* M, const int64_t* N
             e.M[i] = M[i];
             e.N[i] = N[i];
         }
-        g.plan = find_plan(wgrad, count, M, N, nk, room, &g.together);
-        if (all_256) g.together /= kMargin256;
+        g.plan = find_plan(wgrad, count, M, N, nk, room, &g.together, list_256);
+        if (all_256 && g.plan.kind != kTile256) g.together /= kMargin256;
         g.one = g.together < g.apart;
         e.K = K;
         e.room = room;
         e.count = count;
         e.wgrad = wgrad;
+        e.list_256 = list_256;
     }
     return e.times;
 }
-bool group_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan) {
-    const GroupTimes g = group_times(wgrad, count, M, N, K, room);
+bool group_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K, int64_t room, GemmPlan& plan, bool list_256 = false) {
+    const GroupTimes g = group_times(wgrad, count, M, N, K, room, list_256);
     plan = g.plan;
     return g.one;
 }
@@ -727,6 +800,42 @@ bool w4_stores_ok(const void* C, int64_t N, int64_t ldc) {
     return N % vec == 0 && ldc % vec == 0 && ezl_aligned16(C) && ldc * (int64_t)sizeof(OutT) * BM < (1LL << 31);
 }
 
+// Lists of weight gradients on 256 x 256 tiles (4-wave kernel, fp32 results)
+int64_t list_256_tiles(int count, const int64_t* M, const int64_t* N) {
+    int64_t tiles = 0;
+    for (int i = 0; i < count; ++i) tiles += tiles_of(kTile256, M[i], N[i]);
+    return tiles;
+}
+bool list_256_pays(int count, const int64_t* M, const int64_t* N, int64_t K) {
+    const int64_t nk = (K + BK - 1) / BK, tiles = list_256_tiles(count, M, N);
+    bool pays = tiles < (1LL << 26);
+    for (int i = 0; i < count; ++i) pays = pays && w4_pays(Form::weight_gradient, nk, tiles, N[i]);
+    return pays;
+}
+int64_t list_256_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
+    const int64_t tiles = list_256_tiles(count, M, N);
+    const SplitPlan p = make_plan(tiles, (K + BK - 1) / BK, (void*)16, INT64_MAX);
+    return p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
+}
+// the main launch of a list
+template <bool KTAIL>
+void launch_w4_list(GemmSmallArgs& a, int count, const SplitPlan& plan, hipStream_t st) {
+    gemm_tile_grids({kTile256, 1}, a, count);
+    const int items = plan.full + (a.ntiles - plan.full) * plan.nsplit;
+    hipLaunchKernelGGL((gemm_w4_kernel<false, false, float, false, KTAIL, true>), w4_grid((a.K + BK - 1) / BK, items), dim3(256), 0, st, nullptr, nullptr,
+                       (float*)nullptr, 0, 0, a.K, (int64_t)0, (int64_t)0, (int64_t)0, 0, 0, 0, items, plan, KSegments(), a);
+}
+void launch_list_256(GemmSmallArgs& a, int count, int64_t tiles, void* workspace, int64_t workspace_bytes, hipStream_t st) {
+    const SplitPlan plan = make_plan(tiles, (a.K + BK - 1) / BK, workspace, workspace_bytes);
+    if (a.K % BK == 0) launch_w4_list<false>(a, count, plan, st);
+    else launch_w4_list<true>(a, count, plan, st);
+    if (plan.nsplit > 1) {
+        a.nsplit = plan.nsplit;
+        a.partial = plan.partial;
+        gemm_small_reduce_fp32(kTile256, plan.full, a, st);
+    }
+}
+
 template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
 void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
                  void* workspace, int64_t workspace_bytes, hipStream_t st) {
@@ -742,7 +851,7 @@ void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int
         w4 = w4_pays(form, plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk, items, ldb) && w4_stores_ok<OutT>(C, N, ldc);
         if (w4)
             hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, false, KTAIL>), w4_grid(nk, items), dim3(256), 0, st, (const bf16_t*)A,
-                               (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, items, plan, KSegments());
+                               (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, items, plan, KSegments(), NoList());
     }
     if (!w4)
         hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, false, KTAIL>), dim3((unsigned)items), dim3(512), 0, st, (const bf16_t*)A,
@@ -924,7 +1033,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
         if (w4)                                                                                                                              \
             hipLaunchKernelGGL((gemm_w4_kernel<true, false, bf16_t, true, KT>), w4_grid(seg.nk, items), dim3(256), 0, (hipStream_t)stream,    \
                                (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate,    \
-                               tiles_m, tiles_n, items, plan, seg);                                                                          \
+                               tiles_m, tiles_n, items, plan, seg, NoList());                                                                          \
         else                                                                                                                                 \
             hipLaunchKernelGGL((gemm_d2l_kernel<true, false, bf16_t, true, KT>), dim3((unsigned)items), dim3(512), 0, (hipStream_t)stream,   \
                                (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate,    \
@@ -984,7 +1093,7 @@ extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* 
 
 // A decoder layer's weight gradients all reduce over its tokens.  Behind one another each of them is a launch that fills a part of the
 // chip (2 x 512 tokens at h = 256: 16 to 132 workgroups, four launches of 8 us), as one list of tiles they fill it together.
-int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* M, const int64_t* N, int64_t K) {
+int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* M, const int64_t* N, int64_t K, bool fp32, bool beyond_cache) {
     double in_pieces = kLaunchGap * (pieces - 1);
     int count = 0;
     for (int p = 0; p < pieces; ++p) {
@@ -992,8 +1101,9 @@ int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* 
         in_pieces += g.one ? g.together : g.apart;
         count += counts[p];
     }
-    const GroupTimes all = group_times(true, count, M, N, K, INT64_MAX);
-    return all.together < in_pieces ? small_plan_bytes(all.plan, count, M, N) : -1;
+    const GroupTimes all = group_times(true, count, M, N, K, INT64_MAX, fp32 && list_256_pays(count, M, N, K));
+    if (all.together >= in_pieces || (beyond_cache && all.plan.kind != kTile256)) return -1;
+    return all.plan.kind == kTile256 ? list_256_bytes(count, M, N, K) : small_plan_bytes(all.plan, count, M, N);
 }
 
 int gemm_list(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N, int64_t K,
@@ -1024,10 +1134,17 @@ int gemm_list(int count, const void* const* A, const void* const* B, void* const
         return EZL_OK;
     }
     GemmPlan plan;
-    group_plan(!a_kc, count, M, N, K, INT64_MAX, plan);
+    bool list_256 = out_dtype == 1 && count > kGroupMax && list_256_pays(count, M, N, K);
+    for (int i = 0; i < count; ++i) list_256 = list_256 && w4_stores_ok<float>(C[i], N[i], ldc[i]);
+    group_plan(!a_kc, count, M, N, K, INT64_MAX, plan, list_256);
+    a.K = (int)K;
+    if (list_256 && plan.kind == kTile256) {
+        launch_list_256(a, count, list_256_tiles(count, M, N), workspace, workspace_bytes, (hipStream_t)stream);
+        EZL_LAUNCH_CHECK("ezl_gemm_bf16_group");
+        return EZL_OK;
+    }
     if (small_plan_bytes(plan, count, M, N) > (workspace ? workspace_bytes : 0)) group_plan(!a_kc, count, M, N, K, 0, plan);
     if (plan.kind == kTile256) plan = {kTile256x128, 1};  // (a group of one: these kernels take one or more)
-    a.K = (int)K;
     a.partial = (float*)workspace;
     const int form = a_kc ? (b_kc ? 0 : 1) : (out_dtype == 1 ? 2 : 3);
     gemm_small_launch(form, false, plan, a, count, (hipStream_t)stream);

@@ -358,13 +358,13 @@ __global__ __launch_bounds__(512) void gemm_64_waves_kernel(const GemmSmallArgs 
 
 // C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order; a thread owns 8 consecutive columns of one row
 template <typename OutT>
-__global__ __launch_bounds__(256) void small_reduce_kernel(const GemmSmallArgs args, int tbm, int tbn) {
+__global__ __launch_bounds__(256) void small_reduce_kernel(const GemmSmallArgs args, int tbm, int tbn, int first_tile) {
     const int per_tile = tbm * tbn / 2048;  // workgroups per tile
-    const int tile = blockIdx.x / per_tile;
+    const int local = blockIdx.x / per_tile, tile = first_tile + local;
     const GemmProblem p = problem_of(args, tile);
     int tm, tn;
     tile_of(tile - p.first, p.tiles_m, p.tiles_n, tm, tn);
-    const int e = ((blockIdx.x - tile * per_tile) * 256 + threadIdx.x) * 8;  // element of the tile
+    const int e = ((blockIdx.x - local * per_tile) * 256 + threadIdx.x) * 8;  // element of the tile
     const int rl = e / tbn, cl = e - rl * tbn;
     const int row = tm * tbm + rl, col = tn * tbn + cl;
     if (row >= p.M || col >= p.N) return;
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(256) void small_reduce_kernel(const GemmSmallArgs a
 #pragma unroll
     for (int r = 0; r < 8; ++r) v[r] = 0.f;
     const size_t stride = (size_t)tbm * tbn;
-    const float* src = args.partial + (size_t)tile * args.nsplit * stride + e;
+    const float* src = args.partial + (size_t)local * args.nsplit * stride + e;
 #pragma unroll 4
     for (int q = 0; q < args.nsplit; ++q, src += stride) {
         const f32x4 x = *reinterpret_cast<const f32x4*>(src), y = *reinterpret_cast<const f32x4*>(src + 4);
@@ -425,13 +425,13 @@ void launch_kind(int kind, const GemmSmallArgs& a, bool tail, hipStream_t st) {
     }
     if (a.nsplit > 1) {
         const int tbm = (int)gemm_kind_bm(kind), tbn = (int)gemm_kind_bn(kind);
-        hipLaunchKernelGGL((small_reduce_kernel<OutT>), dim3((unsigned)(a.ntiles * (tbm * tbn / 2048))), dim3(256), 0, st, a, tbm, tbn);
+        hipLaunchKernelGGL((small_reduce_kernel<OutT>), dim3((unsigned)(a.ntiles * (tbm * tbn / 2048))), dim3(256), 0, st, a, tbm, tbn, 0);
     }
 }
 
 }  // namespace
 
-void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs& a, int count, hipStream_t stream) {
+void gemm_tile_grids(const GemmPlan& plan, GemmSmallArgs& a, int count) {
     const int bm = (int)gemm_kind_bm(plan.kind), bn = (int)gemm_kind_bn(plan.kind);
     a.ntiles = 0;
     for (int i = 0; i < kMaxProblems; ++i) {
@@ -446,6 +446,16 @@ void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs
         a.ntiles += p.tiles_m * p.tiles_n;
     }
     a.nsplit = plan.nsplit;
+}
+
+void gemm_small_reduce_fp32(int kind, int first_tile, const GemmSmallArgs& a, hipStream_t stream) {
+    const int bm = (int)gemm_kind_bm(kind), bn = (int)gemm_kind_bn(kind);
+    hipLaunchKernelGGL((small_reduce_kernel<float>), dim3((unsigned)((a.ntiles - first_tile) * (bm * bn / 2048))), dim3(256), 0, stream, a, bm, bn,
+                       first_tile);
+}
+
+void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs& a, int count, hipStream_t stream) {
+    gemm_tile_grids(plan, a, count);
     bool tail = a.K % BK != 0;
     if (multi) tail = tail || a.seg.K1 % BK != 0 || a.seg.K2 % BK != 0;
     if (form == 0) launch_kind<true, true, bf16_t, false>(plan.kind, a, tail, stream);

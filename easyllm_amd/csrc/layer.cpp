@@ -62,7 +62,7 @@ struct WeightGradients {
     explicit WeightGradients(const Dims& m)
         : n{m.qw, m.kw, m.kw, m.h, m.f, m.f, m.h}, k{m.h, m.h, m.h, m.qw, m.h, m.h, m.f} {}
     // workspace of all of them in one launch behind everything else; -1 where it is faster to launch them as their operands
-    // appear (q / k / v, o, gate / up, down).  elem: bytes of a result.  Results of much more than the last-level cache (256 MB)
+    // appear (q / k / v, o, gate / up, down).  elem: bytes of a result.  On the smaller tiles, results of much more than the last-level cache (256 MB)
     // are better written in pieces, which drain into memory under the products between them: a layer's backward with 309 and 356 MB of
     // them in one launch and in pieces 301 against 312 us, 1060 against 1102; with 410 - 670 MB 406 against 398, 790 against 779, 968
     // against 1006, 524 against 484, 575 against 534.
@@ -70,7 +70,7 @@ struct WeightGradients {
         static const int counts[4] = {3, 1, 2, 1};
         int64_t results = 0;
         for (int i = 0; i < kGemmListMax; ++i) results += n[i] * k[i] * elem;
-        return results > (384LL << 20) ? -1 : gemm_list_workspace_bytes(4, counts, n, k, T);
+        return gemm_list_workspace_bytes(4, counts, n, k, T, elem == 4, results > (384LL << 20));
     }
 };
 
@@ -109,7 +109,7 @@ struct BackwardTemp {
         w = max64(w, ezl_rmsnorm_bwd_workspace_bytes(m.T, m.h));
         w = max64(w, ezl_attn_bwd_workspace_bytes(m.T, l.ndocs, m.nq, m.nk, m.d));
         if (l.bq) w = max64(w, ezl_bias_grad_workspace_bytes(m.T, m.qw + 2 * m.kw));
-        w = max64(w, WeightGradients(m).list_bytes(m.T, 2));
+        w = max64(w, max64(WeightGradients(m).list_bytes(m.T, 2), WeightGradients(m).list_bytes(m.T, 4)));
         ws_bytes = w;
         ws = b.take(ws_bytes);
         bytes = b.used;

@@ -206,10 +206,15 @@ def test_gemm_products_in_one_launch(K, T, n_in, outs):
 
 @pytest.mark.parametrize("h,nq,nk,f,b,s,main_grads", [(64, 1, 1, 72, 1, 3, True), (256, 4, 1, 688, 2, 511, True), (768, 12, 12, 2048, 2, 1024, True),
                                                       (1024, 16, 4, 2816, 3, 389, False), (1024, 8, 8, 2816, 1, 4000, True),
-                                                      (256, 4, 4, 1000, 1, 16001, True)])
+                                                      (256, 4, 4, 1000, 1, 16001, True),
+                                                      # 256 x 256 tiles: a split last round, with a K tail, ragged tiles, less than a round,
+                                                      # more results than the cache holds
+                                                      (2048, 16, 16, 5504, 1, 2048, True), (2048, 16, 4, 5504, 2, 1001, True),
+                                                      (1920, 15, 15, 5056, 1, 2503, True), (1024, 8, 2, 3328, 1, 4003, True),
+                                                      (2944, 23, 23, 9216, 1, 1691, True)])
 def test_weight_gradients_of_a_layer_in_one_launch(h, nq, nk, f, b, s, main_grads):
-    """A layer's seven weight gradients as one list of tiles (at these sizes: one, two or several K tiles per wave, K tails, 64, 128 and
-    256 x 128 tiles, split reductions), overwritten and then added to, against the composed layer's separate products: activations and
+    """A layer's seven weight gradients as one list of tiles (at these sizes: one, two or several K tiles per wave, K tails, 64, 128,
+    256 x 128 and 256 x 256 tiles, split reductions), overwritten and then added to, against the composed layer's separate products: activations and
     their gradients are the same bits, the sums over the tokens are in fp32 in another order (bf16 results: one rounding apart)."""
     from easyllm_amd import runner
     print("weight gradients of a layer", h, f, b, s, flush=True)
