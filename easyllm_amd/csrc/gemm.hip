@@ -271,17 +271,17 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // 4096 911 -> 885.  What is left there is the power limit: longer K loops run at 1.2 - 1.35 us per K tile instead of 0.96.
 // C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base), its tile-relative byte offsets
 // must fit 31 bits, and every item must have two K tiles or more: the host side checks.
-// LIST (weight gradients): the tiles of several products over one K; what is said per product comes from the list then, not from the other
-// arguments.  A decoder layer's seven over 4000 tokens (h = 2048, f = 5504: 784 tiles, three rounds and 16 tiles) went out as 128 x 128 tiles in
-// 453 us, as these in 387.  (One product in a list of one would save the form without it, but costs 6 us a launch: a tile's scalar loads
-// depend on one another.)
+// LIST (forward, weight gradients): the tiles of several products over one K; what is said per product comes from the list then, not from the
+// other arguments.  A decoder layer's seven weight gradients over 4000 tokens (h = 2048, f = 5504: 784 tiles, three rounds and 16 tiles) went out
+// as 128 x 128 tiles in 453 us, as these in 387; its gate and up products (704 tiles) as 256 x 128 tiles in 208, as these in 155.  (One
+// product in a list of one would save the form without it, but costs 6 us a launch: a tile's scalar loads depend on one another.)
 struct NoList {};
 template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL, bool LIST = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                          int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
                                                          int tiles_m, int tiles_n, int items, const SplitPlan plan, const KSegments seg,
                                                          const std::conditional_t<LIST, GemmSmallArgs, NoList> list) {
-    static_assert(!LIST || (!A_KC && !B_KC && !MULTI), "lists are of weight gradients");
+    static_assert(!LIST || (A_KC == B_KC && !MULTI), "lists are of forward products or weight gradients");
     __shared__ __attribute__((aligned(1024))) bf16_t smem[4 * DTILE];  // A0 B0 A1 B1
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -335,8 +335,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
         it.b_blk = B_KC ? (int64_t)it.n0 * ldb : (int64_t)it.n0;
         if constexpr (LIST) {
             const GemmProblem& p = list.p[it.product];
-            it.a = p.A + it.m0;
-            it.b = p.B + it.n0;
+            it.a = p.A + (A_KC ? it.m0 * p.lda : it.m0);
+            it.b = p.B + (B_KC ? it.n0 * p.ldb : it.n0);
             it.lda = (int)p.lda;
             it.ldb = (int)p.ldb;
             it.mrem = min(p.M - it.m0, BM);
@@ -396,8 +396,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
         t += x.kt0;
         if constexpr (LIST) {
             kv = K - t * BK;
-            ga = la.base(x.a + (int64_t)t * BK * x.lda);
-            gb = lb.base(x.b + (int64_t)t * BK * x.ldb);
+            ga = la.base(x.a + (int64_t)t * BK * (A_KC ? 1 : x.lda));
+            gb = lb.base(x.b + (int64_t)t * BK * (B_KC ? 1 : x.ldb));
             return;
         }
         pick_segment<MULTI>(A, B, K, seg, t, kv, Ab, Bb);
@@ -640,7 +640,10 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
 //   0.76 - 0.80   8192, 2048, 16, 5504 3867 -> 3680; 4000, 2048, 16, 5504 1905 -> 1835; 10086, 1024, 8, 3328 2471 -> 2432
 //   0.80 - 0.93   4810, 2560, 20, 7744 3443 -> 3313; 1691, 2944, 23, 9216 1667 -> 1631; 2048, 4096, 8, 14336 2900 -> 2860; 2780, 2688, 21, 9408
 //                 2283 -> 2205; at worst 2963, 1024, 2, 3392 707 -> 716
-//   0.93 - 1.00   1531, 4096, 32, 11008 2180 -> 2216; 8569, 896, 14, 2976 1772 -> 1787; 1331, 3200, 25, 9984 1589 -> 1550
+//   0.93 - 1.00   (before the margin) 1531, 4096, 32, 11008 2180 -> 2216; 8569, 896, 14, 2976 1772 -> 1787; 1331, 3200, 25, 9984 1589 -> 1550
+// Gate and up in a forward list, by the same margin: 1726, 3072, 24, 9920 1760 -> 1709; 4952, 1792, 14, 4800 1968 -> 1923; 4000, 2048, 16, 5504
+// 1748 -> 1716; 24 random layers 0.7 % faster in the mean, none slower.  bf16 weight gradients, whether list or single: 5183, 2048, 16, 6912 2641 -> 2526;
+// 2961, 2048, 4, 5504 1288 -> 1231; 24 random layers 1.7 %, none slower.
 constexpr double kMarginList256 = 0.93;
 // `count` products over the same nk K tiles in one launch; `room`: workspace bytes.  256 x 256 tiles take one product, or with list_256 all
 GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr, bool list_256 = false) {
@@ -800,16 +803,16 @@ bool w4_stores_ok(const void* C, int64_t N, int64_t ldc) {
     return N % vec == 0 && ldc % vec == 0 && ezl_aligned16(C) && ldc * (int64_t)sizeof(OutT) * BM < (1LL << 31);
 }
 
-// Lists of weight gradients on 256 x 256 tiles (4-wave kernel, fp32 results)
+// Lists of forward products or weight gradients on 256 x 256 tiles (4-wave kernel)
 int64_t list_256_tiles(int count, const int64_t* M, const int64_t* N) {
     int64_t tiles = 0;
     for (int i = 0; i < count; ++i) tiles += tiles_of(kTile256, M[i], N[i]);
     return tiles;
 }
-bool list_256_pays(int count, const int64_t* M, const int64_t* N, int64_t K) {
+bool list_256_pays(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K) {
     const int64_t nk = (K + BK - 1) / BK, tiles = list_256_tiles(count, M, N);
     bool pays = tiles < (1LL << 26);
-    for (int i = 0; i < count; ++i) pays = pays && w4_pays(Form::weight_gradient, nk, tiles, N[i]);
+    for (int i = 0; i < count; ++i) pays = pays && w4_pays(wgrad ? Form::weight_gradient : Form::forward, nk, tiles, N[i]);
     return pays;
 }
 int64_t list_256_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
@@ -817,22 +820,22 @@ int64_t list_256_bytes(int count, const int64_t* M, const int64_t* N, int64_t K)
     const SplitPlan p = make_plan(tiles, (K + BK - 1) / BK, (void*)16, INT64_MAX);
     return p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
 }
-// the main launch of a list
-template <bool KTAIL>
-void launch_w4_list(GemmSmallArgs& a, int count, const SplitPlan& plan, hipStream_t st) {
+template <bool KC, typename OutT>
+void launch_list_256(GemmSmallArgs& a, int count, void* workspace, int64_t workspace_bytes, hipStream_t st) {
     gemm_tile_grids({kTile256, 1}, a, count);
+    const int nk = (a.K + BK - 1) / BK;
+    const SplitPlan plan = make_plan(a.ntiles, nk, workspace, workspace_bytes);
     const int items = plan.full + (a.ntiles - plan.full) * plan.nsplit;
-    hipLaunchKernelGGL((gemm_w4_kernel<false, false, float, false, KTAIL, true>), w4_grid((a.K + BK - 1) / BK, items), dim3(256), 0, st, nullptr, nullptr,
-                       (float*)nullptr, 0, 0, a.K, (int64_t)0, (int64_t)0, (int64_t)0, 0, 0, 0, items, plan, KSegments(), a);
-}
-void launch_list_256(GemmSmallArgs& a, int count, int64_t tiles, void* workspace, int64_t workspace_bytes, hipStream_t st) {
-    const SplitPlan plan = make_plan(tiles, (a.K + BK - 1) / BK, workspace, workspace_bytes);
-    if (a.K % BK == 0) launch_w4_list<false>(a, count, plan, st);
-    else launch_w4_list<true>(a, count, plan, st);
+#define EZL_LIST(KTAIL)                                                                                                                 \
+    hipLaunchKernelGGL((gemm_w4_kernel<KC, KC, OutT, false, KTAIL, true>), w4_grid(nk, items), dim3(256), 0, st, nullptr, nullptr,       \
+                       (OutT*)nullptr, 0, 0, a.K, (int64_t)0, (int64_t)0, (int64_t)0, 0, 0, 0, items, plan, KSegments(), a)
+    if (a.K % BK == 0) EZL_LIST(false);
+    else EZL_LIST(true);
+#undef EZL_LIST
     if (plan.nsplit > 1) {
         a.nsplit = plan.nsplit;
         a.partial = plan.partial;
-        gemm_small_reduce_fp32(kTile256, plan.full, a, st);
+        gemm_small_reduce(kTile256, sizeof(OutT) == 4, plan.full, a, st);
     }
 }
 
@@ -844,8 +847,8 @@ void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int
     const int split_tiles = tiles_m * tiles_n - plan.full;
     const int items = plan.full + split_tiles * plan.nsplit;
     bool w4 = false;
-    // (bf16 weight gradients and fp32 input gradients stay with the 8-wave kernel)
-    if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC && sizeof(OutT) == 4) {
+    // (fp32 input gradients stay with the 8-wave kernel)
+    if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC) {
         constexpr Form form = !A_KC ? Form::weight_gradient : (B_KC ? Form::forward : Form::input_gradient);
         // (a launch that is split tiles only is judged by the length of a share)
         w4 = w4_pays(form, plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk, items, ldb) && w4_stores_ok<OutT>(C, N, ldc);
@@ -1072,8 +1075,8 @@ extern "C" int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, cons
     for (int i = 0; i < count; ++i)
         if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
     GemmPlan plan;
-    if (!group_plan(!a_kc, count, M, N, K, INT64_MAX, plan)) return -1;
-    return small_plan_bytes(plan, count, M, N);
+    if (!group_plan(!a_kc, count, M, N, K, INT64_MAX, plan, a_kc && list_256_pays(false, count, M, N, K))) return -1;
+    return plan.kind == kTile256 ? list_256_bytes(count, M, N, K) : small_plan_bytes(plan, count, M, N);
 }
 // The form is not said: products with K = N are taken for the forward of square weights, others for weight gradients (gate and up are
 // long in both).  The workspace is enough for either form's plan.
@@ -1093,7 +1096,7 @@ extern "C" int ezl_gemm_bf16_group(int count, const void* const* A, const void* 
 
 // A decoder layer's weight gradients all reduce over its tokens.  Behind one another each of them is a launch that fills a part of the
 // chip (2 x 512 tokens at h = 256: 16 to 132 workgroups, four launches of 8 us), as one list of tiles they fill it together.
-int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* M, const int64_t* N, int64_t K, bool fp32, bool beyond_cache) {
+int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* M, const int64_t* N, int64_t K, bool beyond_cache) {
     double in_pieces = kLaunchGap * (pieces - 1);
     int count = 0;
     for (int p = 0; p < pieces; ++p) {
@@ -1101,7 +1104,7 @@ int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* 
         in_pieces += g.one ? g.together : g.apart;
         count += counts[p];
     }
-    const GroupTimes all = group_times(true, count, M, N, K, INT64_MAX, fp32 && list_256_pays(count, M, N, K));
+    const GroupTimes all = group_times(true, count, M, N, K, INT64_MAX, list_256_pays(true, count, M, N, K));
     if (all.together >= in_pieces || (beyond_cache && all.plan.kind != kTile256)) return -1;
     return all.plan.kind == kTile256 ? list_256_bytes(count, M, N, K) : small_plan_bytes(all.plan, count, M, N);
 }
@@ -1134,12 +1137,13 @@ int gemm_list(int count, const void* const* A, const void* const* B, void* const
         return EZL_OK;
     }
     GemmPlan plan;
-    bool list_256 = out_dtype == 1 && count > kGroupMax && list_256_pays(count, M, N, K);
-    for (int i = 0; i < count; ++i) list_256 = list_256 && w4_stores_ok<float>(C[i], N[i], ldc[i]);
+    bool list_256 = (a_kc ? b_kc && count > 1 : count > kGroupMax) && list_256_pays(!a_kc, count, M, N, K);
+    for (int i = 0; i < count; ++i) list_256 = list_256 && (out_dtype ? w4_stores_ok<float> : w4_stores_ok<bf16_t>)(C[i], N[i], ldc[i]);
     group_plan(!a_kc, count, M, N, K, INT64_MAX, plan, list_256);
     a.K = (int)K;
     if (list_256 && plan.kind == kTile256) {
-        launch_list_256(a, count, list_256_tiles(count, M, N), workspace, workspace_bytes, (hipStream_t)stream);
+        (a_kc ? launch_list_256<true, bf16_t> : (out_dtype ? launch_list_256<false, float> : launch_list_256<false, bf16_t>))(
+            a, count, workspace, workspace_bytes, (hipStream_t)stream);
         EZL_LAUNCH_CHECK("ezl_gemm_bf16_group");
         return EZL_OK;
     }

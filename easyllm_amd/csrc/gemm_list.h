@@ -5,9 +5,9 @@
 constexpr int kGemmListMax = 7;  // the weight gradients of a decoder layer: q, k, v, o, gate, up, down
 
 // Workspace of C[i] (=|+=) A[i] * B[i], i < sum of counts, as one launch; -1 where the products are estimated to be faster in
-// `pieces` pieces of counts[p] consecutive ones, each in one launch or one by one.  fp32: the results are (else bf16); beyond_cache: only as 256 x 256 tiles.
+// `pieces` pieces of counts[p] consecutive ones, each in one launch or one by one.  beyond_cache: only as 256 x 256 tiles.
 __attribute__((visibility("hidden"))) int64_t gemm_list_workspace_bytes(int pieces, const int* counts, const int64_t* M, const int64_t* N,
-                                                                        int64_t K, bool fp32, bool beyond_cache);
+                                                                        int64_t K, bool beyond_cache);
 // as ezl_gemm_bf16_group, for up to kGemmListMax products
 __attribute__((visibility("hidden"))) int gemm_list(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M,
                                                     const int64_t* N, int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc,

@@ -448,10 +448,11 @@ void gemm_tile_grids(const GemmPlan& plan, GemmSmallArgs& a, int count) {
     a.nsplit = plan.nsplit;
 }
 
-void gemm_small_reduce_fp32(int kind, int first_tile, const GemmSmallArgs& a, hipStream_t stream) {
+void gemm_small_reduce(int kind, bool fp32, int first_tile, const GemmSmallArgs& a, hipStream_t stream) {
     const int bm = (int)gemm_kind_bm(kind), bn = (int)gemm_kind_bn(kind);
-    hipLaunchKernelGGL((small_reduce_kernel<float>), dim3((unsigned)((a.ntiles - first_tile) * (bm * bn / 2048))), dim3(256), 0, stream, a, bm, bn,
-                       first_tile);
+    const dim3 grid((unsigned)((a.ntiles - first_tile) * (bm * bn / 2048)));
+    if (fp32) hipLaunchKernelGGL((small_reduce_kernel<float>), grid, dim3(256), 0, stream, a, bm, bn, first_tile);
+    else hipLaunchKernelGGL((small_reduce_kernel<bf16_t>), grid, dim3(256), 0, stream, a, bm, bn, first_tile);
 }
 
 void gemm_small_launch(int form, bool multi, const GemmPlan& plan, GemmSmallArgs& a, int count, hipStream_t stream) {

@@ -357,7 +357,7 @@ __attribute__((visibility("hidden"))) void gemm_small_launch(int form, bool mult
                                                              hipStream_t stream);
 // tile grids of a launch on tiles of that plan's shape (K is set)
 __attribute__((visibility("hidden"))) void gemm_tile_grids(const GemmPlan& plan, GemmSmallArgs& a, int count);
-// fp32 results of tiles first_tile.. of a launch from their partial tiles (a.partial: of first_tile on, a.nsplit of each)
-__attribute__((visibility("hidden"))) void gemm_small_reduce_fp32(int kind, int first_tile, const GemmSmallArgs& a, hipStream_t stream);
+// results (fp32, else bf16) of tiles first_tile.. of a launch from their partial tiles (a.partial: of first_tile on, a.nsplit of each)
+__attribute__((visibility("hidden"))) void gemm_small_reduce(int kind, bool fp32, int first_tile, const GemmSmallArgs& a, hipStream_t stream);
 inline int64_t gemm_kind_bm(int kind) { return kKindRows[kind]; }
 inline int64_t gemm_kind_bn(int kind) { return kKindCols[kind]; }

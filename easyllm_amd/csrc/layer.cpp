@@ -70,7 +70,7 @@ struct WeightGradients {
         static const int counts[4] = {3, 1, 2, 1};
         int64_t results = 0;
         for (int i = 0; i < kGemmListMax; ++i) results += n[i] * k[i] * elem;
-        return gemm_list_workspace_bytes(4, counts, n, k, T, elem == 4, results > (384LL << 20));
+        return gemm_list_workspace_bytes(4, counts, n, k, T, results > (384LL << 20));
     }
 };
 

@@ -101,6 +101,8 @@ def test_gemm_smaller_tiles(K, form, M, N, Kd):
     # 192 x 128: K tails, ragged edges, element-wise stores, reductions split two to nine ways
     (0, 1780, 2328, 344), (1, 742, 2720, 904), (0, 1099, 3819, 368), (0, 1531, 4096, 4096), (0, 392, 4688, 2680), (1, 453, 2752, 3368),
     (0, 556, 952, 5752), (2, 3456, 1336, 400), (2, 2224, 2168, 403), (3, 904, 4848, 467), (2, 904, 2488, 2160), (3, 384, 3240, 2765),
+    # 256 x 256, bf16 weight gradients: several tiles per workgroup, K tails, a long reduction
+    (3, 4872, 5128, 1040), (3, 5000, 6000, 1101), (3, 4096, 4096, 3205),
     # 256 x 128
     (0, 1195, 4816, 696), (1, 1209, 5008, 672), (0, 3872, 1648, 720), (0, 1009, 2808, 3040), (1, 423, 4704, 3568)])
 def test_gemm_wide_tiles(K, form, M, N, Kd):
@@ -180,6 +182,18 @@ def test_gemm_four_wave_kernel_over_pairs(K):
     assert ((dx.float() - 2 * ref).abs() <= 2 * bound + ref.abs() * 2.0 ** -6 + 1e-6).all()
 
 
+# split last rounds, K tails, ragged tiles, widths that differ
+@pytest.mark.parametrize("T,n_in,outs", [(1726, 3072, (9920, 9920)), (1726, 3080, (9920, 9912)), (2050, 2056, (5504, 5504, 2056)), (4000, 2048, (5504, 5504))])
+def test_gemm_forward_products_in_one_launch_on_the_largest_tiles(K, T, n_in, outs):
+    print("gemm forward list", T, n_in, outs, flush=True)
+    from easyllm_amd import _lib
+    x, ws = rnd(T, n_in, seed=1), [rnd(o, n_in, seed=2 + i) for i, o in enumerate(outs)]
+    assert _lib.gemm_group_form_workspace_bytes(True, (T,) * len(outs), outs, n_in) >= 0
+    for y, w in zip(K.linear_fwd_multi(x, ws), ws):
+        ref = x.float() @ w.float().t()
+        assert ((y.float() - ref).abs() <= gemm_bound(x, w.t()) + ref.abs() * 2.0 ** -8 + 1e-6).all()
+
+
 @pytest.mark.parametrize("T,n_in,outs", [(1024, 256, (256, 256, 256)), (1167, 1024, (1024, 256, 264)), (389, 768, (2048, 2056)),
                                          (17, 264, (8, 1000, 72)), (4000, 2048, (2048, 512, 512)), (9000, 256, (256, 512))])
 def test_gemm_products_in_one_launch(K, T, n_in, outs):
@@ -211,7 +225,8 @@ def test_gemm_products_in_one_launch(K, T, n_in, outs):
                                                       # more results than the cache holds
                                                       (2048, 16, 16, 5504, 1, 2048, True), (2048, 16, 4, 5504, 2, 1001, True),
                                                       (1920, 15, 15, 5056, 1, 2503, True), (1024, 8, 2, 3328, 1, 4003, True),
-                                                      (2944, 23, 23, 9216, 1, 1691, True)])
+                                                      (2944, 23, 23, 9216, 1, 1691, True), (2048, 16, 4, 5504, 1, 2961, False),
+                                                      (1792, 14, 14, 4672, 1, 4608, False)])
 def test_weight_gradients_of_a_layer_in_one_launch(h, nq, nk, f, b, s, main_grads):
     """A layer's seven weight gradients as one list of tiles (at these sizes: one, two or several K tiles per wave, K tails, 64, 128,
     256 x 128 and 256 x 256 tiles, split reductions), overwritten and then added to, against the composed layer's separate products: activations and
