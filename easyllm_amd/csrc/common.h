@@ -83,10 +83,8 @@ __device__ __forceinline__ float wave_max(float v) {
 // out[col] (+)= sum_r partial[r][col];  64 columns per block, 16 row groups (loads of a group issued eight at a time)
 // folded through LDS in a fixed order.
 constexpr int kColsumThreads = 1024;
-template <int UNUSED>
-__global__ __launch_bounds__(kColsumThreads) void ezl_colsum_kernel(const float* __restrict__ partial, int nrows, int ncols,
-                                                                    bf16_t* __restrict__ out_bf16, float* __restrict__ out_f32,
-                                                                    int accumulate) {
+__device__ __forceinline__ void ezl_colsum(const float* __restrict__ partial, int nrows, int ncols, bf16_t* __restrict__ out_bf16,
+                                           float* __restrict__ out_f32, int accumulate) {
     constexpr int G = kColsumThreads / 64;
     __shared__ float s[G][64];
     const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
@@ -112,5 +110,11 @@ __global__ __launch_bounds__(kColsumThreads) void ezl_colsum_kernel(const float*
         if (out_f32) out_f32[col] = accumulate ? out_f32[col] + v : v;
         else out_bf16[col] = (bf16_t)v;
     }
+}
+template <int UNUSED>
+__global__ __launch_bounds__(kColsumThreads) void ezl_colsum_kernel(const float* __restrict__ partial, int nrows, int ncols,
+                                                                    bf16_t* __restrict__ out_bf16, float* __restrict__ out_f32,
+                                                                    int accumulate) {
+    ezl_colsum(partial, nrows, ncols, out_bf16, out_f32, accumulate);
 }
 #endif

@@ -10,6 +10,7 @@
 // and laid out by the same arithmetic in forward and backward (bump allocation, 256-byte steps).
 #include "common.h"
 #include "gemm_list.h"
+#include "norm_pair.h"
 #include "qkv_bias.h"
 #include "../../include/ezl.h"
 
@@ -90,7 +91,7 @@ struct ForwardTemp {
 };
 
 struct BackwardTemp {
-    void *dact, *dgate, *dup, *dn, *dsum, *dctx, *dqkv, *delta, *ws;
+    void *dact, *dgate, *dup, *dn, *dsum, *dctx, *dqkv, *delta, *ln2_sums, *ws;
     int64_t ws_bytes, bytes;
     BackwardTemp(const ezl_layer& l, const Dims& m, void* base) {
         Bump b(base);
@@ -99,6 +100,7 @@ struct BackwardTemp {
         dctx = b.take(m.T * m.qw * 2);
         dqkv = b.take(m.T * (m.qw + 2 * m.kw) * 2);  // dq | dk | dv in one row, so that one launch can reduce over all three
         delta = b.take(m.nq * m.T * 4);
+        ln2_sums = b.take(ezl_rmsnorm_bwd_workspace_bytes(m.T, m.h));
         const int64_t mqkv[3] = {m.qw, m.kw, m.kw}, hh[3] = {m.h, m.h, m.h}, mgu[2] = {m.f, m.f};
         int64_t w = max64(products_ws(0, 3, mqkv, hh, m.T), products_ws(0, 2, mgu, hh, m.T));
         w = max64(w, max64(ezl_gemm_workspace_bytes(m.qw, m.h, m.T), ezl_gemm_workspace_bytes(m.f, m.h, m.T)));  // (also one by one)
@@ -267,8 +269,9 @@ extern "C" int ezl_layer_bwd(const ezl_layer* l, const void* x, const void* dy, 
         EZL_TRY(ezl_gemm_bf16_ksplit(2, d, w, t.dn, m.T, m.h, n, m.f, m.h, m.h, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
         if (!one_list) EZL_TRY(weight_gradients(2, d, m.f, a.n2, &g[EZL_G_GATE], m.T, n, m.h, t.ws, t.ws_bytes, st));
     }
-    EZL_TRY(ezl_rmsnorm_bwd(t.dn, a.sum, l->ln2, a.rstd2, dy, t.dsum, g[EZL_G_LN2].f32 ? nullptr : g[EZL_G_LN2].bf16, g[EZL_G_LN2].f32,
-                            g[EZL_G_LN2].accumulate, t.ws, t.ws_bytes, m.T, m.h, st));
+    NormWeightGrad ln1, ln2;
+    EZL_TRY(rmsnorm_bwd_rows(t.dn, a.sum, l->ln2, a.rstd2, dy, t.dsum, g[EZL_G_LN2].f32 ? nullptr : g[EZL_G_LN2].bf16, g[EZL_G_LN2].f32,
+                             g[EZL_G_LN2].accumulate, t.ln2_sums, m.T, m.h, ln2, st));
     // sum = x + o(ctx)
     EZL_TRY(ezl_gemm_bf16(t.dsum, l->wo, t.dctx, m.T, m.qw, m.h, m.h, m.qw, m.qw, 1, 0, 0, 0, t.ws, t.ws_bytes, st));
     if (!one_list) {
@@ -311,6 +314,7 @@ extern "C" int ezl_layer_bwd(const ezl_layer* l, const void* x, const void* dy, 
         }
         EZL_TRY(gemm_list(kGemmListMax, d, x, out, w.n, w.k, m.T, ld, w.k, w.k, 0, 0, g[EZL_G_Q].f32 ? 1 : 0, acc, t.ws, t.ws_bytes, st));
     }
-    return ezl_rmsnorm_bwd(t.dn, x, l->ln1, a.rstd1, t.dsum, dx, g[EZL_G_LN1].f32 ? nullptr : g[EZL_G_LN1].bf16, g[EZL_G_LN1].f32,
-                           g[EZL_G_LN1].accumulate, t.ws, t.ws_bytes, m.T, m.h, st);
+    EZL_TRY(rmsnorm_bwd_rows(t.dn, x, l->ln1, a.rstd1, t.dsum, dx, g[EZL_G_LN1].f32 ? nullptr : g[EZL_G_LN1].bf16, g[EZL_G_LN1].f32,
+                             g[EZL_G_LN1].accumulate, t.ws, m.T, m.h, ln1, st));
+    return norm_weight_grads(ln1, ln2, m.h, st);
 }
