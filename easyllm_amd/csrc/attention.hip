@@ -880,7 +880,18 @@ bool fwd_key_groups_pay(int64_t blocks, int64_t s_len) { return blocks <= 256 ? 
 bool bwd_one_launch_pays(int64_t blocks, int64_t s_len, int64_t d) {
     return blocks <= 128 || (blocks <= 256 && s_len >= 384) || (blocks <= (d == 64 ? 384 : 288) && s_len >= 1024);
 }
+enum AttnPlan { kRows128, kRows128Shared, kRows32 };  // as ezl_attn_plan returns them
+AttnPlan attn_plan(bool backward, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d) {
+    if (attn_small_pays(total_tokens, s_len, nq, nk, d, backward)) return kRows32;
+    const int64_t blocks = total_tokens / s_len * ((s_len + 127) / 128) * nq;
+    return (backward ? bwd_one_launch_pays(blocks, s_len, d) : fwd_key_groups_pay(blocks, s_len)) ? kRows128Shared : kRows128;
+}
 }  // namespace
+
+extern "C" int ezl_attn_plan(int backward, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d) {
+    if (total_tokens <= 0 || s_len <= 0 || nk <= 0 || nq <= 0 || nq % nk != 0) return -1;
+    return attn_plan(backward != 0, total_tokens, s_len, nq, nk, d);
+}
 
 // strides[8]: q_seq, q_batch, k_seq, k_batch, v_seq, v_batch, out_seq, out_batch (elements)
 extern "C" int ezl_attn_fwd(const void* q, const void* k, const void* v, void* out, void* lse, const void* cu_seqlens, int64_t ndocs,
@@ -897,14 +908,15 @@ extern "C" int ezl_attn_fwd(const void* q, const void* k, const void* v, void* o
     p.scale = scale;
     p.q_ss = strides[0]; p.q_sb = strides[1]; p.k_ss = strides[2]; p.k_sb = strides[3];
     p.v_ss = strides[4]; p.v_sb = strides[5]; p.o_ss = strides[6]; p.o_sb = strides[7];
-    if (attn_small_pays(total_tokens, s_len, nq, d, false)) {
+    const AttnPlan plan = attn_plan(false, total_tokens, s_len, nq, nk, d);
+    if (plan == kRows32) {
         attn_small_fwd(p, (int)d, (hipStream_t)stream);
         EZL_LAUNCH_CHECK("ezl_attn_fwd");
         return EZL_OK;
     }
     const dim3 grid((unsigned)((total_tokens + 127) / 128 + ndocs + total_tokens / s_len), (unsigned)nq);
     hipStream_t st = (hipStream_t)stream;
-    if (fwd_key_groups_pay(total_tokens / s_len * ((s_len + 127) / 128) * nq, s_len)) {
+    if (plan == kRows128Shared) {
         if (d == 128) hipLaunchKernelGGL((attn_fwd_kernel<128, 2>), grid, dim3(2 * kThreads), 0, st, p);
         else hipLaunchKernelGGL((attn_fwd_kernel<64, 2>), grid, dim3(2 * kThreads), 0, st, p);
     } else {
@@ -961,7 +973,8 @@ extern "C" int ezl_attn_bwd(const void* q, const void* k, const void* v, const v
     p.do_ss = strides[8]; p.do_sb = strides[9]; p.dq_ss = strides[10]; p.dq_sb = strides[11];
     p.dk_ss = strides[12]; p.dk_sb = strides[13]; p.dv_ss = strides[14]; p.dv_sb = strides[15];
     hipStream_t st = (hipStream_t)stream;
-    if (attn_small_pays(total_tokens, s_len, nq, d, true)) {
+    const AttnPlan plan = attn_plan(true, total_tokens, s_len, nq, nk, d);
+    if (plan == kRows32) {
         attn_small_bwd(p, (int)d, st);
         EZL_LAUNCH_CHECK("ezl_attn_bwd");
         return EZL_OK;
@@ -971,9 +984,8 @@ extern "C" int ezl_attn_bwd(const void* q, const void* k, const void* v, const v
     const dim3 gridk(nblk, (unsigned)(nk * p.nsplit));
     int64_t gc = (total_tokens * nk * d / 8 + kThreads - 1) / kThreads;
     if (gc > 256 * 16) gc = 256 * 16;
-    const bool both = bwd_one_launch_pays(total_tokens / s_len * ((s_len + 127) / 128) * nq, s_len, d);
     // otherwise the dQ kernel goes first: it also produces delta = rowsum(dO * O), which the dK/dV kernel reads
-    if (both) {
+    if (plan == kRows128Shared) {
         const int key_blocks = (int)(nblk * nk * p.nsplit);
         const dim3 grid((unsigned)(key_blocks + nblk * nq));
         if (d == 128) {

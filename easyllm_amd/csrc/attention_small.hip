@@ -430,10 +430,15 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 //             (130) 19.5, 21.9
 //             d 128:  6 / 2 x 145 (18) 15.8, 11.5; 19 / 2 x 128 (38) 14.2, 16.5; 3 / 4 x 428 (42) 26.8, 20.9; 2 / 3 x 1455 (70) 71, 51; 5 / 8 x 209
 //             (70) 19.3, 25.5; 4 / 3 x 1281 (124) 66, 73
-bool attn_small_pays(int64_t total_tokens, int64_t s_len, int64_t nq, int64_t d, bool backward) {
+// A block of keys walks the queries of every head of its group, which the 128-row kernel deals to several workgroups: with more than two heads
+// a group only short chains pay.  Query / kv heads, documents x length, us with dQ and dK/dV of 128 rows in one launch against these:
+//   d 64:  8 / 1, 2 x 500 23.2, 54.7; 28 / 7, 3 x 83 13.5, 11.2; 14 / 7, 728 27.9, 28.4; 2 / 1, 3 x 561 21.8, 19.4
+//   d 128: 4 / 1, 2 x 802 47.5, 67.5 (two launches 62.2); 12 / 3, 175 20.2, 21.6; 32 / 4, 79 17.1, 21.2; 68 / 17, 114 21.6, 18.4; 2 / 1, 4326 189, 165
+bool attn_small_pays(int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d, bool backward) {
     const int64_t rows = total_tokens / s_len;
     if (!backward) return rows * ((s_len + 31) / 32) * nq <= (d == 64 ? 512 : 256);
-    return rows * ((s_len + 127) / 128) * nq <= (d == 64 ? 64 : 32) + s_len / 32;
+    const int64_t group = nq / nk;
+    return rows * ((s_len + 127) / 128) * nq <= (d == 64 ? 64 : 32) + s_len / 32 && (group <= 2 || (s_len + 31) / 32 * group <= 16);
 }
 
 void attn_small_fwd(const AttnParams& p, int d, hipStream_t stream) {

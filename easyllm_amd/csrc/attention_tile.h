@@ -309,6 +309,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 }  // namespace
 
 // attention_small.hip: the same results with 32 queries (or keys) per workgroup
-__attribute__((visibility("hidden"))) bool attn_small_pays(int64_t total_tokens, int64_t s_len, int64_t nq, int64_t d, bool backward);
+__attribute__((visibility("hidden"))) bool attn_small_pays(int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d,
+                                                            bool backward);
 __attribute__((visibility("hidden"))) void attn_small_fwd(const AttnParams& p, int d, hipStream_t stream);
 __attribute__((visibility("hidden"))) void attn_small_bwd(const AttnParams& p, int d, hipStream_t stream);

@@ -109,3 +109,15 @@ def test_products_of_256_tiles_share_a_launch_only_by_a_margin(T, h, outs, forwa
     n = len(outs)
     assert (_lib.gemm_group_workspace_bytes((T,) * n, outs, h) >= 0) == forward
     assert (_lib.gemm_group_workspace_bytes(outs, (h,) * n, T) >= 0) == weight_gradient
+
+
+# (measured, us: one launch of 128 rows against workgroups of 32)
+@pytest.mark.parametrize("d,nq,nk,b,s,plan", [
+    (64, 8, 1, 2, 500, 1),     # 23.2, 54.7
+    (128, 4, 1, 2, 802, 1),    # 47.5, 67.5
+    (128, 32, 4, 1, 79, 1),    # 17.1, 21.2
+    (64, 2, 1, 3, 561, 2),     # 21.8, 19.4
+    (64, 28, 7, 1, 83, 2),     # (three rows: 13.5, 11.2)
+    (64, 4, 4, 2, 512, 2)])
+def test_attention_backward_of_grouped_queries_on_32_rows_only_with_short_chains(d, nq, nk, b, s, plan):
+    assert _lib.attn_plan(True, b * s, s, nq, nk, d) == plan
