@@ -84,7 +84,7 @@ _SPECIAL = {
     "ezl_bias_grad_workspace_bytes": ([_i64, _i64], _i64),
     "ezl_embed_scatter_add_workspace_bytes": ([_i64, _i64], _i64),
     "ezl_attn_bwd_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64], _i64),
-    "ezl_attn_plan": ([_i32, _i64, _i64, _i64, _i64, _i64], _i32),
+    "ezl_attn_plan": ([_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64], _i32),
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
     "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
     "ezl_gemm_group_form_workspace_bytes": ([_i32, _i32, _i64p, _i64p, _i64], _i64),
@@ -150,8 +150,10 @@ def attn_bwd_workspace_bytes(total_tokens, ndocs, nq, nk, d):
     return load().ezl_attn_bwd_workspace_bytes(total_tokens, ndocs, nq, nk, d)
 
 
-def attn_plan(backward, total_tokens, s_len, nq, nk, d):
-    return load().ezl_attn_plan(1 if backward else 0, total_tokens, s_len, nq, nk, d)
+def attn_plan(backward, ndocs, total_tokens, s_len, nq, nk, d):
+    """ndocs: None without cu_seqlens"""
+    documents = 0 if ndocs is None else 1
+    return load().ezl_attn_plan(1 if backward else 0, documents, ndocs if documents else total_tokens // s_len, total_tokens, s_len, nq, nk, d)
 
 
 @functools.lru_cache(maxsize=1024)  # a function of the sizes alone

@@ -23,7 +23,8 @@
 //
 // Launches that leave CUs idle: the forward and the dQ kernel also exist with the key tiles shared out to two groups of four
 // waves, dQ and dK/dV as one launch, and attention_small.hip has both with 32 rows per workgroup.  Which is taken follows from
-// the number of blocks and the document length alone (attn_small_pays, fwd_key_groups_pay, bwd_one_launch_pays).
+// the number of blocks and the length of the rows, or of the documents on average, alone (attn_small_pays, fwd_key_groups_pay,
+// bwd_one_launch_pays).
 #include "attention_tile.h"
 
 namespace {
@@ -862,7 +863,7 @@ int check_common(const char* name, int64_t T, int64_t s_len, int64_t nq, int64_t
 }  // namespace
 
 namespace {
-// blocks: 128-row blocks of the launch; s_len: the longest document there can be.  While about every CU has one workgroup, a launch takes
+// Batches of whole rows.  blocks: 128-row blocks of the launch.  While about every CU has one workgroup, a launch takes
 // its longest chain of tiles: sharing it out to two groups of waves pays for their sums being brought together where it has
 // six tiles or more, and with some CUs having two workgroups where it has many.  us, one group against two:
 //   d 64:  13 / 3 x 400 (130 blocks) 10.5, 9.8; 19 / 8 x 222 (266) 9.7, 12.9; 12 / 2 x 1024 (192) 18.9, 15.8; 22 / 3 x 558 (308) 14.4, 16.8;
@@ -880,17 +881,38 @@ bool fwd_key_groups_pay(int64_t blocks, int64_t s_len) { return blocks <= 256 ? 
 bool bwd_one_launch_pays(int64_t blocks, int64_t s_len, int64_t d) {
     return blocks <= 128 || (blocks <= 256 && s_len >= 384) || (blocks <= (d == 64 ? 384 : 288) && s_len >= 1024);
 }
+// Packed batches, by the workgroups that are launched and the mean length of the documents: every workgroup of these forms holds a CU by itself, also while
+// it searches the documents and when it finds no block.  Heads, documents x length (mean, longest) of one row, us with two groups or one launch after
+// those without:
+//   forward   d 64:  12 / 64 x 64 13.5, 30.7; 12 / 8 x 512 19.2, 25.7; 2 / 128 x 128 14.3, 16.0; 2 / 32 x 512 19.4, 18.0; 12 / 4 x 512 16.6, 15.6
+//             d 128: 4 / 128 x 64 16.6, 27.7; 4 / 16 x 512 23.3, 22.5; 8 / 4 x 512 20.1, 19.6; 10 / 27 (179, 445) 33.6, 43.7
+//   backward  d 64:  12 / 64 x 64 49, 68; 12 / 8 x 512 53, 54; 2 / 128 x 128 32.7, 35.2; 4 / 16 x 256 31, 18; 16 / 4 x 256 28, 17; 12 / 4 (512, 1010) 57, 38
+//             d 128: 4 / 64 x 128 42, 47; 4 / 16 x 512 59, 58; 8 / 8 x 256 39, 25; 3 / 72 (51, 85) 29.8, 31.4
+// 430 batches of 1 - 93 heads, 256 - 16384 tokens and log-uniform lengths, with attn_small_pays: forward 0.9 %, backward 1.3 % behind the fastest of
+// the three, at worst 4 % behind the 128-row kernels and 4 % and 28 % faster on average; by the rules for whole rows 8.7 and 15 % behind, at worst 2.3 and
+// 3.0 times the 128-row kernels.
+bool fwd_key_groups_pay_documents(int64_t launched, int64_t mean) { return launched <= 320 ? mean >= 192 : launched <= 384 && mean >= 768; }
+bool bwd_one_launch_pays_documents(int64_t launched, int64_t mean) {
+    return launched <= 256 || (launched <= 320 && mean >= 128) || (launched <= 384 && mean >= 384);
+}
 enum AttnPlan { kRows128, kRows128Shared, kRows32 };  // as ezl_attn_plan returns them
-AttnPlan attn_plan(bool backward, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d) {
-    if (attn_small_pays(total_tokens, s_len, nq, nk, d, backward)) return kRows32;
-    const int64_t blocks = total_tokens / s_len * ((s_len + 127) / 128) * nq;
-    return (backward ? bwd_one_launch_pays(blocks, s_len, d) : fwd_key_groups_pay(blocks, s_len)) ? kRows128Shared : kRows128;
+AttnPlan attn_plan(bool backward, const AttnSizes& z) {
+    if (attn_small_pays(z, backward)) return kRows32;
+    bool shared;
+    if (z.documents) {
+        const int64_t launched = z.launched(128) * z.nq, mean = z.mean_length();
+        shared = backward ? bwd_one_launch_pays_documents(launched, mean) : fwd_key_groups_pay_documents(launched, mean);
+    } else {
+        const int64_t blocks = z.rows() * ((z.s_len + 127) / 128) * z.nq;
+        shared = backward ? bwd_one_launch_pays(blocks, z.s_len, z.d) : fwd_key_groups_pay(blocks, z.s_len);
+    }
+    return shared ? kRows128Shared : kRows128;
 }
 }  // namespace
 
-extern "C" int ezl_attn_plan(int backward, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d) {
-    if (total_tokens <= 0 || s_len <= 0 || nk <= 0 || nq <= 0 || nq % nk != 0) return -1;
-    return attn_plan(backward != 0, total_tokens, s_len, nq, nk, d);
+extern "C" int ezl_attn_plan(int backward, int documents, int64_t ndocs, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d) {
+    if (total_tokens <= 0 || s_len <= 0 || ndocs <= 0 || nk <= 0 || nq <= 0 || nq % nk != 0) return -1;
+    return attn_plan(backward != 0, {documents != 0, ndocs, total_tokens, s_len, nq, nk, d});
 }
 
 // strides[8]: q_seq, q_batch, k_seq, k_batch, v_seq, v_batch, out_seq, out_batch (elements)
@@ -908,7 +930,7 @@ extern "C" int ezl_attn_fwd(const void* q, const void* k, const void* v, void* o
     p.scale = scale;
     p.q_ss = strides[0]; p.q_sb = strides[1]; p.k_ss = strides[2]; p.k_sb = strides[3];
     p.v_ss = strides[4]; p.v_sb = strides[5]; p.o_ss = strides[6]; p.o_sb = strides[7];
-    const AttnPlan plan = attn_plan(false, total_tokens, s_len, nq, nk, d);
+    const AttnPlan plan = attn_plan(false, {cu_seqlens != nullptr, ndocs, total_tokens, s_len, nq, nk, d});
     if (plan == kRows32) {
         attn_small_fwd(p, (int)d, (hipStream_t)stream);
         EZL_LAUNCH_CHECK("ezl_attn_fwd");
@@ -973,7 +995,7 @@ extern "C" int ezl_attn_bwd(const void* q, const void* k, const void* v, const v
     p.do_ss = strides[8]; p.do_sb = strides[9]; p.dq_ss = strides[10]; p.dq_sb = strides[11];
     p.dk_ss = strides[12]; p.dk_sb = strides[13]; p.dv_ss = strides[14]; p.dv_sb = strides[15];
     hipStream_t st = (hipStream_t)stream;
-    const AttnPlan plan = attn_plan(true, total_tokens, s_len, nq, nk, d);
+    const AttnPlan plan = attn_plan(true, {cu_seqlens != nullptr, ndocs, total_tokens, s_len, nq, nk, d});
     if (plan == kRows32) {
         attn_small_bwd(p, (int)d, st);
         EZL_LAUNCH_CHECK("ezl_attn_bwd");

@@ -434,11 +434,20 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 // a group only short chains pay.  Query / kv heads, documents x length, us with dQ and dK/dV of 128 rows in one launch against these:
 //   d 64:  8 / 1, 2 x 500 23.2, 54.7; 28 / 7, 3 x 83 13.5, 11.2; 14 / 7, 728 27.9, 28.4; 2 / 1, 3 x 561 21.8, 19.4
 //   d 128: 4 / 1, 2 x 802 47.5, 67.5 (two launches 62.2); 12 / 3, 175 20.2, 21.6; 32 / 4, 79 17.1, 21.2; 68 / 17, 114 21.6, 18.4; 2 / 1, 4326 189, 165
-bool attn_small_pays(int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d, bool backward) {
-    const int64_t rows = total_tokens / s_len;
-    if (!backward) return rows * ((s_len + 31) / 32) * nq <= (d == 64 ? 512 : 256);
-    const int64_t group = nq / nk;
-    return rows * ((s_len + 127) / 128) * nq <= (d == 64 ? 64 : 32) + s_len / 32 && (group <= 2 || (s_len + 31) / 32 * group <= 16);
+// Every workgroup of a packed batch first searches the documents for its block, so that four times the workgroups cost more than with whole rows; these
+// kernels have to fit the launched ones at once and gain from documents that are long on average.  Heads, documents x length (mean, longest) of one
+// row, us with 128-row kernels (two launches backward), key groups / one launch, these:
+//   forward   d 64:  8 / 31 (59, 72) 10.5, 11.2, 20.2; 4 / 64 x 64 10.5, 11.8, 13.4; 4 / 8 x 512 17.0, 16.0, 16.8; 1 / 29 (414, 507) 18.1, 17.1, 17.2; 4 / 7 (586, 2132)
+//             37.1, 31.2, 27.9
+//             d 128: 2 / 32 x 128 14.2, 15.1, 14.5; 2 / 16 x 256 16.3, 16.8, 15.6; 2 / 7 (586, 2132) 45.8, 39.7, 36.3
+//   backward  d 64:  4 / 32 x 512 63, 74, 144; 4 / 16 x 256 30.8, 17.9, 31.5; 4 / 7 (586, 2132) 95, 58, 56; 1 / 45 (188, 752) 48, 28.2, 28.3
+//             d 128: 4 / 64 x 128 42, 47, 127; 2 / 16 x 256 39, 24.5, 34.6; 1 / 16 (320, 736) 63, 43, 33; 2 / 7 (586, 2132) 135, 101, 65
+bool attn_small_pays(const AttnSizes& z, bool backward) {
+    const int64_t length = z.documents ? z.mean_length() : z.s_len, group = z.nq / z.nk;
+    auto blocks = [&](int64_t n) { return (z.documents ? z.launched(n) : z.rows() * ((z.s_len + n - 1) / n)) * z.nq; };
+    if (!backward) return blocks(32) <= (z.d == 64 ? 512 : 256) && (!z.documents || length >= 256);
+    if (group > 2 && (length + 31) / 32 * group > 16) return false;
+    return blocks(128) <= (z.documents ? 48 + length / 8 : (z.d == 64 ? 64 : 32) + length / 32);
 }
 
 void attn_small_fwd(const AttnParams& p, int d, hipStream_t stream) {

@@ -308,8 +308,21 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 }  // namespace
 
+// Sizes of a call, from which its kernels are chosen.
+struct AttnSizes {
+    bool documents;  // cu_seqlens given
+    int64_t ndocs, total_tokens, s_len, nq, nk, d;
+    int64_t rows() const { return total_tokens / s_len; }
+    // workgroups of `block` queries or keys per head: as many as any documents can need, hence as many as are launched with documents
+    int64_t launched(int64_t block) const { return (total_tokens + block - 1) / block + ndocs + rows(); }
+    // documents lie on the device: the host knows how long they are on average, and that none is longer than a batch row
+    int64_t mean_length() const {
+        const int64_t mean = (total_tokens + ndocs - 1) / ndocs;
+        return mean < s_len ? mean : s_len;
+    }
+};
+
 // attention_small.hip: the same results with 32 queries (or keys) per workgroup
-__attribute__((visibility("hidden"))) bool attn_small_pays(int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d,
-                                                            bool backward);
+__attribute__((visibility("hidden"))) bool attn_small_pays(const AttnSizes& z, bool backward);
 __attribute__((visibility("hidden"))) void attn_small_fwd(const AttnParams& p, int d, hipStream_t stream);
 __attribute__((visibility("hidden"))) void attn_small_bwd(const AttnParams& p, int d, hipStream_t stream);

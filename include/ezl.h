@@ -165,8 +165,9 @@ int ezl_attn_fwd(const void* q, const void* k, const void* v, void* out, void* l
                  int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d, float scale, const int64_t* strides,
                  void* stream);
 /* Which kernels a call takes, for tests and profiles (host only): 2 workgroups of 32 queries or keys; 1 of 128, the forward's and dQ's key
- * tiles shared out to two groups of waves and dQ and dK/dV in one launch; 0 of 128, two launches backward.  -1: bad sizes. */
-int ezl_attn_plan(int backward, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d);
+ * tiles shared out to two groups of waves and dQ and dK/dV in one launch; 0 of 128, two launches backward.  documents: cu_seqlens is
+ * given.  -1: bad sizes. */
+int ezl_attn_plan(int backward, int documents, int64_t ndocs, int64_t total_tokens, int64_t s_len, int64_t nq, int64_t nk, int64_t d);
 int64_t ezl_attn_bwd_workspace_bytes(int64_t total_tokens, int64_t ndocs, int64_t nq, int64_t nk, int64_t d);
 int ezl_attn_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout, const void* lse, void* delta,
                  void* dq, void* dk, void* dv, const void* cu_seqlens, int64_t ndocs, int64_t total_tokens, int64_t s_len,

@@ -120,4 +120,23 @@ def test_products_of_256_tiles_share_a_launch_only_by_a_margin(T, h, outs, forwa
     (64, 28, 7, 1, 83, 2),     # (three rows: 13.5, 11.2)
     (64, 4, 4, 2, 512, 2)])
 def test_attention_backward_of_grouped_queries_on_32_rows_only_with_short_chains(d, nq, nk, b, s, plan):
-    assert _lib.attn_plan(True, b * s, s, nq, nk, d) == plan
+    assert _lib.attn_plan(True, None, b * s, s, nq, nk, d) == plan
+
+
+# (measured, us: 128-row kernels, key groups / one launch, 32-row kernels)
+@pytest.mark.parametrize("backward,d,heads,tokens,ndocs,plan", [
+    (False, 64, 12, 4096, 64, 0),   # 13.5, 30.7, 35.6
+    (False, 64, 8, 1811, 31, 0),    # 10.5, 11.2, 20.2
+    (False, 64, 12, 2048, 4, 1),    # 16.6, 15.6, 26.4
+    (False, 64, 2, 4096, 7, 2),     # (four heads: 37.1, 31.2, 27.9)
+    (False, 128, 4, 8192, 128, 0),  # 16.6, 27.7, 53.8
+    (True, 64, 4, 16384, 256, 0),   # 79, 102, 122
+    (True, 64, 4, 16384, 32, 0),    # 63, 74, 144
+    (True, 64, 12, 4096, 64, 0),    # 49, 68, 83
+    (True, 64, 4, 4096, 16, 1),     # 30.8, 17.9, 31.5
+    (True, 128, 4, 8192, 64, 0),    # 42, 47, 127
+    (True, 128, 1, 5115, 16, 2),    # 63, 43, 33
+    # empty documents: launches of 2^32 threads or more along one axis are refused, which 128-row kernels reach last
+    (False, 64, 512, 16, 33000, 0), (True, 64, 512, 16, 33000, 0), (True, 64, 128, 129, 70000, 0)])
+def test_attention_of_packed_rows_goes_by_the_length_of_the_documents(backward, d, heads, tokens, ndocs, plan):
+    assert _lib.attn_plan(backward, ndocs, tokens, tokens, heads, heads, d) == plan

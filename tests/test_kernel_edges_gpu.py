@@ -308,6 +308,22 @@ def test_attention_for_every_split_of_the_work(K, d, nq, nk, b, s, cu):
     assert torch.equal(out2, out)
 
 
+@pytest.mark.parametrize("nq,s,ndocs", [(512, 16, 33000), (128, 129, 70000)])
+def test_attention_with_more_documents_than_one_axis_of_a_launch_holds(K, nq, s, ndocs):
+    """All but the first document are empty.  Workgroups for all documents and heads on one axis would be 2^32 threads or more, which no launch
+    takes.  Against the one document by itself: other kernels at these sizes, so 1e-2 of a result's norm as for every split of the work."""
+    print("attention, empty documents", nq, s, ndocs, flush=True)
+    q, k, v, do = (rnd(s, 1, n, 64, seed=i) for i, n in ((1, nq), (2, nq // 4), (3, nq // 4), (4, nq)))
+    one = torch.tensor([0, s], device="cuda", dtype=torch.int32)
+    many = torch.cat([one, torch.full((ndocs - 1,), s, device="cuda", dtype=torch.int32)])
+    results = []
+    for cu in (one, many):
+        out, lse = K.attn_fwd(q, k, v, cu)
+        results.append((out, lse) + tuple(K.attn_bwd(q, k, v, out, do, lse, cu)))
+    for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), *results):
+        assert (a.double() - b.double()).norm() <= 1e-2 * a.double().norm(), name
+
+
 def test_swiglu_results_larger_than_the_last_level_cache(K):
     """Written past the caches: the same bits as in two calls of half the size."""
     print("swiglu beyond the cache", flush=True)
