@@ -419,8 +419,8 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 
 }  // namespace
 
-// Where these kernels win, by the number of 128-row blocks of the launch (each four workgroups here) and the longest document there can
-// be: while all workgroups run at once (two per CU at d = 64, one at d = 128, by their registers) a launch takes its longest chain of
+// Where these kernels win, on whole rows by the number of 128-row blocks of the launch (each four workgroups here) and the rows' length:
+// while all workgroups run at once (two per CU at d = 64, one at d = 128, by their registers) a launch takes its longest chain of
 // tiles; beyond that it takes the sum, and the larger blocks do the same work with a quarter of the reads.  us, 128-row kernels
 // (as attention.hip would launch them) against these, d / heads / documents x length (blocks):
 //   forward   d 64:   4 / 2 x 512 (32) 9.9, 7.2; 6 / 4 x 454 (90) 9.8, 8.5; 5 / 2902 (115) 33.6, 29.6; 13 / 3 x 511 (156) 10.9, 13.4; 12 / 2 x 1024
@@ -430,6 +430,11 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 //             (130) 19.5, 21.9
 //             d 128:  6 / 2 x 145 (18) 15.8, 11.5; 19 / 2 x 128 (38) 14.2, 16.5; 3 / 4 x 428 (42) 26.8, 20.9; 2 / 3 x 1455 (70) 71, 51; 5 / 8 x 209
 //             (70) 19.3, 25.5; 4 / 3 x 1281 (124) 66, 73
+// A row of up to 64 tokens is one tile, which there is nothing to share out of; one of two tiles gains only while a CU has one workgroup.  Forward, heads /
+// rows x length (32-row workgroups):
+//   d 64:  4 / 64 (8) 4.9, 5.3; 41 / 3 x 33 (246) 5.0, 5.6; 16 / 4 x 65 (192) 6.2, 5.5; 24 / 4 x 65 (288) 6.3, 6.8; 16 / 4 x 97 (256) 6.6, 5.7; 64 / 2 x 97 (512) 6.6,
+//          6.9; 24 / 4 x 128 (384) 7.1, 7.0
+//   d 128: 16 / 2 x 33 (64) 5.8, 6.5; 64 / 2 x 64 (256) 6.5, 7.2; 16 / 65 (48) 7.7, 6.8
 // A block of keys walks the queries of every head of its group, which the 128-row kernel deals to several workgroups: with more than two heads
 // a group only short chains pay.  Query / kv heads, documents x length, us with dQ and dK/dV of 128 rows in one launch against these:
 //   d 64:  8 / 1, 2 x 500 23.2, 54.7; 28 / 7, 3 x 83 13.5, 11.2; 14 / 7, 728 27.9, 28.4; 2 / 1, 3 x 561 21.8, 19.4
@@ -445,7 +450,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 bool attn_small_pays(const AttnSizes& z, bool backward) {
     const int64_t length = z.documents ? z.mean_length() : z.s_len, group = z.nq / z.nk;
     auto blocks = [&](int64_t n) { return (z.documents ? z.launched(n) : z.rows() * ((z.s_len + n - 1) / n)) * z.nq; };
-    if (!backward) return blocks(32) <= (z.d == 64 ? 512 : 256) && (!z.documents || length >= 256);
+    if (!backward) return length > (z.documents ? 255 : 64) && blocks(32) <= (z.d == 64 && length >= 128 ? 512 : 256);
     if (group > 2 && (length + 31) / 32 * group > 16) return false;
     return blocks(128) <= (z.documents ? 48 + length / 8 : (z.d == 64 ? 64 : 32) + length / 32);
 }

@@ -140,3 +140,16 @@ def test_attention_backward_of_grouped_queries_on_32_rows_only_with_short_chains
     (False, 64, 512, 16, 33000, 0), (True, 64, 512, 16, 33000, 0), (True, 64, 128, 129, 70000, 0)])
 def test_attention_of_packed_rows_goes_by_the_length_of_the_documents(backward, d, heads, tokens, ndocs, plan):
     assert _lib.attn_plan(backward, ndocs, tokens, tokens, heads, heads, d) == plan
+
+
+# (measured, us: 128-row kernel, 32-row kernel)
+@pytest.mark.parametrize("d,heads,b,s,plan", [
+    (64, 4, 1, 64, 0),    # 4.9, 5.3
+    (64, 41, 3, 33, 0),   # 5.0, 5.6
+    (64, 16, 4, 65, 2),   # 6.2, 5.5
+    (64, 24, 4, 65, 0),   # 6.3, 6.8
+    (64, 24, 4, 128, 2),  # 7.1, 7.0
+    (128, 64, 2, 64, 0),  # 6.5, 7.2
+    (128, 16, 1, 65, 2)])  # 7.7, 6.8
+def test_attention_forward_of_short_rows(d, heads, b, s, plan):
+    assert _lib.attn_plan(False, None, b * s, s, heads, heads, d) == plan
