@@ -578,7 +578,9 @@ def test_embedding_gradient_with_and_without_the_one_workgroup_tables(K, V, h, r
 
 
 @pytest.mark.parametrize("rows,V,cut", [(3, 32776, 0), (700, 40960, 0), (2100, 40968, 0), (5, 50304, 304), (1167, 53256, 0), (9, 65536, 9), (4, 65544, 0),
-                                        (6, 73720, 1000)])
+                                        (6, 73720, 1000),
+                                        # little more than a vector left, less than one, a whole number of them, all but the last column
+                                        (3, 40960, 40951), (4, 50304, 50299), (3, 36872, 4104), (520, 65536, 1)])
 def test_loss_and_gradient_of_rows_kept_as_bf16_in_registers(K, rows, V, cut):
     """Edges of the register counts, cut columns, ignored rows, labels in the cut, more rows than blocks; against float64.  The sum of V
     fp32 exponentials is off by V 2^-24 at most, the gradient by that and one rounding to bf16."""
