@@ -274,18 +274,26 @@ __global__ __launch_bounds__(kBlock) void embed_bucket_kernel(const int64_t* __r
     }
 }
 
-// The four kernels above as one workgroup, for batches of up to kSmallRows: each of those launches costs more than its work there
-// (2 x 512 tokens at V = 32000: 2.7, 3.3, 5.8, 3.2 us and the gaps between them, now 6.8).  Ids are looked up in a hash table in LDS, so the global
-// tables are only written: cnt / first / off of the ids that occur, and, with zero_all, cnt = 0 of all others.
-constexpr int kSmallRows = 4096, kSmallSlots = 2 * kSmallRows, kSmallThreads = 1024;
-constexpr int64_t kSmallVocab = 131072;  // a single workgroup clears that many counts in 3 us
+// The four kernels above as one workgroup, for short batches: each of those launches costs more than its work there.  Ids are looked up in a hash
+// table in LDS, so the global tables are only written: cnt / first / off of the ids that occur, and, with zero_all, cnt = 0 of all others.
+// Bound by LDS atomics, hence by the rows (and with zero_all by one workgroup's stores, hence by the vocabulary).  The whole gradient, h = 256, us,
+// four launches against this, adding / overwriting; ids drawn evenly, as frequent as words (1 / rank), all the same (padding):
+//   V = 32000    512 rows 16.2 / 23.3, 9.6 / 17.9; 18.3 / 22.7, 11.4 / 16.8; 26.6 / 28.3, 20.5 / 23.1
+//               1531      17.0 / 23.8, 13.3 / 21.3; 21.5 / 24.1, 16.0 / 19.9; 51.1 / 52.5, 45.1 / 47.5
+//               2048      17.9 / 24.1, 17.4 / 25.1; 25.1 / 27.6, 21.6 / 24.7; 63.0 / 64.4, 56.9 / 59.0
+//               4096      20.0 / 25.6, 27.7 / 34.4; 29.1 / 30.9, 29.1 / 31.6; 114 / 116, 109 / 110
+//   V = 131072  1531      17.0 / 43.1, 13.5 / 41.9; 21.2 / 44.5, 15.7 / 39.9
+//               2048      17.4 / 42.2, 17.0 / 45.2; 22.0 / 42.4, 18.0 / 41.5
+// (Without the lanes of a wave that hold one id sharing their atomics 2048 equal ids took 62.5 / 65.1.)
+constexpr int kSmallRows = 2048, kSmallRowsZero = 1536, kSmallSlots = 2 * kSmallRows, kSmallThreads = 1024;
+constexpr int64_t kSmallVocab = 131072;  // with zero_all
 __global__ __launch_bounds__(kSmallThreads) void embed_tables_small_kernel(const int64_t* __restrict__ ids, int* __restrict__ cnt, int* __restrict__ first,
                                                                            int* __restrict__ off, int* __restrict__ bucket, int* __restrict__ cursor,
                                                                            int* __restrict__ heavy, int rows, int64_t V, int zero_all) {
     __shared__ int s_id[kSmallSlots], s_cnt[kSmallSlots], s_first[kSmallSlots], s_off[kSmallSlots];
     __shared__ int s_next, s_heavy;
     constexpr int PER = kSmallRows / kSmallThreads;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     int row_id[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
@@ -293,8 +301,8 @@ __global__ __launch_bounds__(kSmallThreads) void embed_tables_small_kernel(const
         const int64_t id = r < rows ? ids[r] : -1;
         row_id[k] = id >= 0 && id < V ? (int)id : -1;
     }
-    // (2048, 4096 or 8192 slots, the hash's highest bits: at most half of them are ever taken)
-    const int shift = rows <= kSmallSlots / 8 ? 21 : (rows <= kSmallSlots / 4 ? 20 : 19), slots = 1 << (32 - shift);
+    // (2048 or 4096 slots, the hash's highest bits: at most half of them are ever taken)
+    const int shift = rows <= kSmallRows / 4 ? 21 : 20, slots = 1 << (32 - shift);
     for (int i = tid; i < slots; i += kSmallThreads) {
         s_id[i] = -1;
         s_cnt[i] = 0;
@@ -312,15 +320,22 @@ __global__ __launch_bounds__(kSmallThreads) void embed_tables_small_kernel(const
         slot[k] = -1;
         const int id = row_id[k];
         if (id < 0) continue;
-        unsigned i = ((unsigned)id * 0x9E3779B1u) >> shift;
-        for (;;) {  // ends: half of the slots stay free
-            const int old = atomicCAS(&s_id[i], -1, id);
-            if (old == -1 || old == id) break;
-            i = (i + 1) & (slots - 1);
+        unsigned long long mask;
+        const bool same = same_as_first_lane(id, mask);
+        const int leader = __builtin_ctzll(mask);
+        if (!same || lane == leader) {
+            unsigned i = ((unsigned)id * 0x9E3779B1u) >> shift;
+            for (;;) {  // ends: half of the slots stay free
+                const int old = atomicCAS(&s_id[i], -1, id);
+                if (old == -1 || old == id) break;
+                i = (i + 1) & (slots - 1);
+            }
+            slot[k] = (int)i;
+            atomicAdd(&s_cnt[i], same ? (int)__popcll(mask) : 1);
+            atomicMin(&s_first[i], r);  // (the lowest lane holds the smallest row)
         }
-        slot[k] = (int)i;
-        atomicAdd(&s_cnt[i], 1);
-        atomicMin(&s_first[i], r);
+        const int shared = __builtin_amdgcn_readlane(slot[k], leader);
+        if (same) slot[k] = shared;
     }
     __syncthreads();
 #pragma unroll
@@ -336,11 +351,20 @@ __global__ __launch_bounds__(kSmallThreads) void embed_tables_small_kernel(const
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < PER; ++k)
-        if (slot[k] >= 0) bucket[atomicAdd(&s_off[slot[k]], 1)] = k * kSmallThreads + tid;
+    for (int k = 0; k < PER; ++k) {
+        if (slot[k] < 0) continue;
+        unsigned long long mask;
+        const bool same = same_as_first_lane(slot[k], mask);
+        const int leader = __builtin_ctzll(mask);
+        int at = 0;
+        if (!same || lane == leader) at = atomicAdd(&s_off[slot[k]], same ? (int)__popcll(mask) : 1);
+        const int base = __builtin_amdgcn_readlane(at, leader);
+        if (same) at = base + (int)__popcll(mask & ((1ull << lane) - 1));
+        bucket[at] = k * kSmallThreads + tid;
+    }
     if (tid == 0) cursor[1] = s_heavy;
 }
-static_assert(kSmallSlots == 1 << (32 - 19), "the largest table");
+static_assert(kSmallSlots == 1 << (32 - 20), "the largest table");
 
 // p[0 .. n4) = 0 in 16-byte pieces: a block clears one contiguous 16 KiB chunk (4 stores per thread), chunks dealt to blocks in
 // order, so the blocks running at any moment sweep one window of the buffer.
@@ -1020,7 +1044,7 @@ int embed_gradient(const char* name, const void* ids, const void* dy, void* dwei
         hipLaunchKernelGGL(zero_f32x4_kernel, dim3(grid_for(n4, 4 * kBlock, (int64_t)1 << 20)), dim3(kBlock), 0, st, (f32x4*)dweight, n4);
     }
     const int overwrite = accumulate || flat_fill ? 0 : 1;
-    if (rows <= kSmallRows && (!overwrite || vocab <= kSmallVocab)) {
+    if (overwrite ? rows <= kSmallRowsZero && vocab <= kSmallVocab : rows <= kSmallRows) {
         hipLaunchKernelGGL(embed_tables_small_kernel, dim3(1), dim3(kSmallThreads), 0, st, (const int64_t*)ids, cnt, first, off, bucket, cursor,
                            heavy, (int)rows, vocab, overwrite);
     } else {

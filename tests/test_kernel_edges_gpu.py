@@ -552,9 +552,12 @@ def test_embedding_gradient_in_bf16_is_the_fp32_one_rounded(K, V, h, rows, frequ
 
 
 @pytest.mark.parametrize("V,h,rows,ids", [(32000, 256, 1024, "random"), (5000, 64, 4096, "distinct"), (50304, 72, 1167, "padding"), (131072, 64, 4095, "far apart"),
-                                          (40, 128, 3000, "few"), (1, 8, 33, "random"), (131073, 64, 900, "random"), (300, 64, 500, "out of range")])
+                                          (40, 128, 3000, "few"), (1, 8, 33, "random"), (131073, 64, 900, "random"), (300, 64, 500, "out of range"),
+                                          # the largest of one workgroup, runs of equal ids, and between them ids out of range
+                                          (5000, 64, 2048, "distinct"), (131072, 64, 1536, "far apart"), (3000, 72, 2047, "padding"),
+                                          (40, 64, 1537, "few"), (700, 64, 1530, "runs"), (700, 64, 2049, "runs")])
 def test_embedding_gradient_with_and_without_the_one_workgroup_tables(K, V, h, rows, ids):
-    """Batches of up to 4096 rows build their tables in one workgroup.  Rows with an id outside the table are skipped, so the same
+    """Batches of up to 2048 rows (1536 where the buffer is overwritten) build their tables in one workgroup.  Rows with an id outside the table are skipped, so the same
     batch with 4097 of them behind it goes the general way: equal bit for bit, overwriting and adding."""
     print("embedding tables", V, h, rows, ids, flush=True)
     g = torch.Generator().manual_seed(rows)
@@ -565,6 +568,9 @@ def test_embedding_gradient_with_and_without_the_one_workgroup_tables(K, V, h, r
         t[rows // 2:] = 0
     elif ids == "far apart":
         t = torch.arange(rows) * 32 % V
+    elif ids == "runs":
+        t = torch.arange(rows) // 100 * 37 % V
+        t[::9], t[5::64] = V, 3
     elif ids == "out of range":
         t[::7], t[::11] = V, -1
     long = torch.cat([t, torch.full((4097,), V)]).cuda()
