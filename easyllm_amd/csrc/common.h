@@ -52,11 +52,19 @@ struct alignas(16) bf16x8_raw {
 
 __device__ __forceinline__ bf16x8 ld_bf16x8(const bf16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 __device__ __forceinline__ void st_bf16x8(bf16_t* p, bf16x8 v) { *reinterpret_cast<bf16x8*>(p) = v; }
-// Streaming forms: loads of what nobody reads again soon; stores only of results that do not fit the last-level cache anyway.  A kernel
-// that moves hundreds of MB gains from them by itself (SwiGLU backward 92 -> 78 us), but the kernels that read the result next lose
-// more than that where it would have stayed in the cache.
+// Streaming forms: loads of what nobody reads again soon; stores only of results that do not fit the last-level cache (256 MB) anyway, for
+// the kernels that read a result next lose more where it would have stayed there than the writing one gains.
 __device__ __forceinline__ bf16x8 ld_bf16x8_nt(const bf16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)); }
 __device__ __forceinline__ void st_bf16x8_nt(bf16_t* p, bf16x8 v) { __builtin_nontemporal_store(v, reinterpret_cast<bf16x8*>(p)); }
+template <bool STREAM>
+__device__ __forceinline__ void st_result(bf16_t* p, bf16x8 v) {
+    if constexpr (STREAM) st_bf16x8_nt(p, v);
+    else st_bf16x8(p, v);
+}
+// All results of a launch together.  The kernels by themselves, results in MB, us with plain and with streaming stores: SwiGLU forward 172 87, 92;
+// 251 125, 137; 344 222, 196; backward 258 106, 115; 344 175, 158; 502 275, 245; 688 390, 347; RMSNorm backward 128 90, 92; 273 220, 212; 312 227, 213; 512
+// 368, 346.  In a layer's forward and backward of 4096 - 40960 tokens the two differ by less than runs do above 256 MB.
+inline bool ezl_streams(int64_t bytes) { return bytes > (264LL << 20); }
 
 __device__ __forceinline__ void unpack8(bf16x8 v, float* f) {
 #pragma unroll

@@ -25,17 +25,9 @@ __device__ __forceinline__ float sigmoidf_fast(float x) {
 // ---------------------------------------------------------------------------------------------
 // SwiGLU: out = silu(gate) * up     (llama/transformer.py:220-222, glu_activations.py:56-61)
 // ---------------------------------------------------------------------------------------------
-// STREAM: results past the caches.  They are read next by products whose operands every XCD fetches for itself, so it pays to leave
-// them in the last-level cache (256 MB) where one of them fits: input gradient over gate and up behind the backward kernel, 1531 x 4096 x
-// 22016, 349 -> 303 us; a layer's forward and backward over 1531 tokens at h = 4096 687 -> 672 and 1535 -> 1483 us, over 4096 tokens 1511 ->
-// 1490 and 3339 -> 3325.  Larger ones (16384 tokens) would only push each other out: 7304 us with streaming stores, 7316 without.
-template <bool STREAM>
-__device__ __forceinline__ void st_result(bf16_t* p, bf16x8 v) {
-    if constexpr (STREAM) st_bf16x8_nt(p, v);
-    else st_bf16x8(p, v);
-}
-inline bool streams(int64_t n) { return n * 2 > (256LL << 20); }
-
+// STREAM: results past the caches (ezl_streams).  Where one of them fits it is read next by products whose operands every XCD fetches for itself: input
+// gradient over gate and up behind the backward kernel, 1531 x 4096 x 22016, 349 -> 303 us with plain stores; a layer's forward and backward over
+// 1531 tokens at h = 4096 687 -> 672 and 1535 -> 1483 us, over 4096 tokens 1511 -> 1490 and 3339 -> 3325.
 template <bool STREAM>
 __global__ __launch_bounds__(kBlock) void swiglu_fwd_kernel(const bf16_t* __restrict__ gate, const bf16_t* __restrict__ up,
                                                             bf16_t* __restrict__ out, int64_t n8) {
@@ -888,7 +880,7 @@ extern "C" int ezl_swiglu_fwd(const void* gate, const void* up, void* out, int64
     EZL_REQUIRE(ezl_aligned16(gate) && ezl_aligned16(up) && ezl_aligned16(out) && (n == 0 || (gate && up && out)), EZL_EINVAL,
                 "ezl_swiglu_fwd: null or misaligned pointer");
     if (n == 0) return EZL_OK;
-    hipLaunchKernelGGL(streams(n) ? swiglu_fwd_kernel<true> : swiglu_fwd_kernel<false>, dim3(grid_for(n / 8, kBlock)), dim3(kBlock), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(ezl_streams(n * 2) ? swiglu_fwd_kernel<true> : swiglu_fwd_kernel<false>, dim3(grid_for(n / 8, kBlock)), dim3(kBlock), 0, (hipStream_t)stream,
                        (const bf16_t*)gate, (const bf16_t*)up, (bf16_t*)out, n / 8);
     EZL_LAUNCH_CHECK("ezl_swiglu_fwd");
     return EZL_OK;
@@ -901,7 +893,7 @@ extern "C" int ezl_swiglu_bwd(const void* dout, const void* gate, const void* up
                     (n == 0 || (dout && gate && up && dgate && dup)),
                 EZL_EINVAL, "ezl_swiglu_bwd: null or misaligned pointer");
     if (n == 0) return EZL_OK;
-    hipLaunchKernelGGL(streams(n) ? swiglu_bwd_kernel<true> : swiglu_bwd_kernel<false>, dim3(grid_for(n / 8, kBlock)), dim3(kBlock), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(ezl_streams(n * 4) ? swiglu_bwd_kernel<true> : swiglu_bwd_kernel<false>, dim3(grid_for(n / 8, kBlock)), dim3(kBlock), 0, (hipStream_t)stream,
                        (const bf16_t*)dout, (const bf16_t*)gate, (const bf16_t*)up, (bf16_t*)dgate, (bf16_t*)dup, n / 8);
     EZL_LAUNCH_CHECK("ezl_swiglu_bwd");
     return EZL_OK;

@@ -84,12 +84,12 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
 // ---- backward with one wave per row (h <= 2048) ----------------------------------------------------------------
 // A row is owned by ONE wave: lane l holds the 8 columns (c * 64 + l) * 8 .. + 7 of chunk c, so every chunk is one
 // coalesced 1 KiB access, the row sums need wave shuffles only and there is no barrier inside the row loop: the waves
-// of a CU run out of step and keep HBM busy while others compute.  Loads and stores carry the streaming hint (in the
-// step: 42 -> 34 us); the forward kernel keeps the block-per-row form and plain accesses, which measured faster there
-// (its input was written by the kernel before it and its output is read by the one after, 33 MB each).
+// of a CU run out of step and keep HBM busy while others compute.  Loads carry the streaming hint, stores only of results that
+// do not fit the last-level cache (STREAM, see ezl_streams); the forward kernel keeps the block-per-row form and plain accesses, which
+// measured faster there (its input was written by the kernel before it and its output is read by the one after, 33 MB each).
 // Backward, 8 waves per block: each wave keeps the dw partial of its lanes' columns over all rows it visits; at the end the
 // 8 waves of a block are folded through LDS in a fixed order and one partial row per block goes to HBM.
-template <int NCHUNK, bool HAS_DRES>
+template <int NCHUNK, bool HAS_DRES, bool STREAM>
 __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x,
                                                                const bf16_t* __restrict__ w, const float* __restrict__ rstd,
                                                                const bf16_t* __restrict__ dres, bf16_t* __restrict__ dx,
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __r
                     if (HAS_DRES) o[i] += (float)drr[c][i];
                     dwacc[c][i] += dyv * xhat;
                 }
-                st_bf16x8(dx + base + col, pack8(o));
+                st_result<STREAM>(dx + base + col, pack8(o));
             }
         }
     }
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __r
 // waits, computes and stores in turn, and at T = h = 4096 each wave sees only two rows: 45 us for backward + column sum
 // against 29 us with the prefetch.)  The partial sums of a row meet in an LDS cell (double buffered by iteration parity:
 // one barrier per row).  A block is 4 waves = 4 / NSPLIT rows per pass, two blocks per CU.
-template <int NCHUNK, int NSPLIT, bool HAS_DRES>
+template <int NCHUNK, int NSPLIT, bool HAS_DRES, bool STREAM>
 __global__ __launch_bounds__(256, 2) void rmsnorm_bwd_split_kernel(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x,
                                                                    const bf16_t* __restrict__ w, const float* __restrict__ rstd,
                                                                    const bf16_t* __restrict__ dres, bf16_t* __restrict__ dx,
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_bwd_split_kernel(const bf16_t*
                     if (HAS_DRES) o[i] += (float)drr[c][i];
                     dwacc[c][i] += dyv * xhat;
                 }
-                st_bf16x8(dxrow + c * 512, pack8(o));
+                st_result<STREAM>(dxrow + c * 512, pack8(o));
             }
         }
     }
@@ -467,8 +467,9 @@ int rmsnorm_bwd_check(const char* name, const void* dy, const void* x, const voi
 int rmsnorm_bwd_launch_rows(const void* dy, const void* x, const void* weight, const void* rstd, const void* dresidual, void* dx,
                             float* partials, int64_t max_blocks, int64_t rows, int64_t h, int64_t& grid, hipStream_t st) {
     const size_t smem = (size_t)h * sizeof(float);
+    const bool stream = ezl_streams(rows * h * 2);
 #define LAUNCH_SPLIT(NC, NS, DR)                                                                                           \
-    hipLaunchKernelGGL((rmsnorm_bwd_split_kernel<NC, NS, DR>), dim3((unsigned)grid), dim3(256), smem, st, (const bf16_t*)dy, \
+    hipLaunchKernelGGL((stream ? rmsnorm_bwd_split_kernel<NC, NS, DR, true> : rmsnorm_bwd_split_kernel<NC, NS, DR, false>), dim3((unsigned)grid), dim3(256), smem, st, (const bf16_t*)dy, \
                        (const bf16_t*)x, (const bf16_t*)weight, (const float*)rstd, (const bf16_t*)dresidual, (bf16_t*)dx,  \
                        partials, (int)rows, (int)h)
     if (h <= 2048) {  // one wave per row, 8 rows per block
@@ -477,7 +478,7 @@ int rmsnorm_bwd_launch_rows(const void* dy, const void* x, const void* weight, c
         if (grid > max_blocks) grid = max_blocks;
         if (grid < 1) grid = 1;  // rows == 0 still produces a zero dw
 #define LAUNCH(NC, DR)                                                                                                    \
-    hipLaunchKernelGGL((rmsnorm_bwd_wave_kernel<NC, DR>), dim3((unsigned)grid), dim3(512), smem, st, (const bf16_t*)dy,    \
+    hipLaunchKernelGGL((stream ? rmsnorm_bwd_wave_kernel<NC, DR, true> : rmsnorm_bwd_wave_kernel<NC, DR, false>), dim3((unsigned)grid), dim3(512), smem, st, (const bf16_t*)dy,    \
                        (const bf16_t*)x, (const bf16_t*)weight, (const float*)rstd, (const bf16_t*)dresidual, (bf16_t*)dx, \
                        partials, (int)rows, (int)h)
 #define LAUNCH_NC(DR)                                  \

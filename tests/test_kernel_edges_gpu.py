@@ -325,14 +325,32 @@ def test_attention_with_more_documents_than_one_axis_of_a_launch_holds(K, nq, s,
 
 
 def test_swiglu_results_larger_than_the_last_level_cache(K):
-    """Written past the caches: the same bits as in two calls of half the size."""
+    """Written past the caches: the same bits as in four calls of a quarter of the size."""
     print("swiglu beyond the cache", flush=True)
-    n = (128 << 20) + 16
+    n = (140 << 20) + 32
     g, u, do = (rnd(n // 8, 8, seed=i) for i in (1, 2, 3))
     out, (dg, du) = K.swiglu_fwd(g, u), K.swiglu_bwd(do, g, u)
-    for half in (slice(0, n // 16), slice(n // 16, n // 8)):
-        a, b = K.swiglu_bwd(do[half], g[half], u[half])
-        assert torch.equal(out[half], K.swiglu_fwd(g[half], u[half])) and torch.equal(dg[half], a) and torch.equal(du[half], b)
+    for i in range(4):
+        part = slice(i * n // 32, (i + 1) * n // 32)
+        a, b = K.swiglu_bwd(do[part], g[part], u[part])
+        assert torch.equal(out[part], K.swiglu_fwd(g[part], u[part])) and torch.equal(dg[part], a) and torch.equal(du[part], b)
+
+
+@pytest.mark.parametrize("rows,h", [(270000, 520), (70001, 2048), (50000, 3080), (34608, 4096), (23001, 6144), (17500, 8192)])
+def test_rmsnorm_backward_with_results_larger_than_the_last_level_cache(K, rows, h):
+    """Written past the caches: the same bits as for its parts; the weight's gradient over all rows against float64 sums of the parts' (partial sums of
+    up to rows / 256 products each in fp32: 1e-4)."""
+    print("rmsnorm backward beyond the cache", rows, h, flush=True)
+    x, dy, dr, w = rnd(rows, h, seed=1), rnd(rows, h, seed=2), rnd(rows, h, seed=3), rnd(h, seed=4)
+    rstd = (x.float().square().mean(1) + 1e-5).rsqrt()
+    mg = torch.empty(h, device="cuda")
+    dx, _ = K.rmsnorm_bwd(dy, x, w, rstd, dresidual=dr, main_grad=mg)
+    total = torch.zeros(h, device="cuda", dtype=torch.float64)
+    for i in range(4):
+        part, sub = slice(i * rows // 4, (i + 1) * rows // 4), torch.empty(h, device="cuda")
+        assert torch.equal(dx[part], K.rmsnorm_bwd(dy[part], x[part], w, rstd[part], dresidual=dr[part], main_grad=sub)[0])
+        total += sub.double()
+    assert (mg.double() - total).norm() <= 1e-4 * total.norm()
 
 
 @pytest.mark.parametrize("sizes", [[1], [4096, 4095, 4097, 3], [0, 8, 0, 70001], [1 + 37 * i for i in range(101)]])
