@@ -723,10 +723,10 @@ GroupTimes group_times(bool wgrad, int count, const int64_t* M, const int64_t* N
         int count;
         bool wgrad, list_256;
     };
-    static thread_local Entry memo[64] = {};
+    static thread_local Entry memo[2][64] = {};  // (by list_256: group_bytes asks for one set of sizes both ways, each time)
     uint64_t hash = K * 0x165667B19E3779F9ull + 2 * count + wgrad;
     for (int i = 0; i < count; ++i) hash = (hash ^ (uint64_t)M[i]) * 0x9E3779B97F4A7C15ull + (uint64_t)N[i] * 0xC2B2AE3D27D4EB4Full;
-    Entry& e = memo[hash >> 58];
+    Entry& e = memo[list_256][hash >> 58];
     bool same = e.count == count && e.wgrad == wgrad && e.list_256 == list_256 && e.K == K && e.room == room;
     for (int i = 0; i < count && same; ++i) same = e.M[i] == M[i] && e.N[i] == N[i];
     if (!same) {

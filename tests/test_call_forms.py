@@ -1,5 +1,6 @@
 """Forms of calls that a fast path must answer as the general one does, where that can be seen without a GPU."""
 import ctypes
+import time
 
 import pytest
 import torch
@@ -153,3 +154,19 @@ def test_attention_of_packed_rows_goes_by_the_length_of_the_documents(backward, 
     (128, 16, 1, 65, 2)])  # 7.7, 6.8
 def test_attention_forward_of_short_rows(d, heads, b, s, plan):
     assert _lib.attn_plan(False, None, b * s, s, heads, heads, d) == plan
+
+
+@pytest.mark.parametrize("T,h,f", [(512, 3072, 8192), (512, 4096, 11008)])
+def test_a_decision_about_products_in_one_launch_is_remembered(T, h, f):
+    """A layer asks several times per pass.  Where lists on 256 x 256 tiles come into question the forward form is looked up twice, with and without
+    them; neither may push the other out (a repeated query then took twice as long as the weight gradients' one lookup)."""
+    lib, two = _lib.load(), ctypes.c_int64 * 2
+    queries = [(1, 2, two(T, T), two(f, f), h), (0, 2, two(f, f), two(h, h), T)]
+    best = [float("inf")] * 2
+    for _ in range(30):
+        for i, q in enumerate(queries):
+            start = time.perf_counter()
+            for _ in range(300):
+                lib.ezl_gemm_group_form_workspace_bytes(*q)
+            best[i] = min(best[i], time.perf_counter() - start)
+    assert best[0] <= 1.4 * best[1]
