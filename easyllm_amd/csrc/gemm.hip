@@ -1070,9 +1070,7 @@ bool results_meet(int count, void* const* C, const int64_t* M, const int64_t* N,
 // ezl_gemm_group_form_workspace_bytes: -1 where separate ezl_gemm_bf16 calls are estimated to be faster, else the workspace.
 constexpr int kGroupMax = 3;  // q / k / v
 static_assert(kGemmListMax == kMaxProblems, "a list goes out in one launch");
-namespace {
-// with_lists: lists on 256 x 256 tiles count in the decision (in the workspace always: a launch may take them)
-int64_t group_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K, bool with_lists) {
+extern "C" int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K) {
     if (count < 2 || count > kGroupMax || !M || !N || K <= 0) return -1;
     for (int i = 0; i < count; ++i)
         if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
@@ -1080,21 +1078,16 @@ int64_t group_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int
     bool one = group_plan(!a_kc, count, M, N, K, INT64_MAX, plan);
     int64_t bytes = small_plan_bytes(plan, count, M, N);  // (an input gradient, or results that the large tiles cannot store)
     if (a_kc && list_256_pays(false, count, M, N, K)) {
-        const bool list = group_plan(false, count, M, N, K, INT64_MAX, plan, true);
+        one = group_plan(false, count, M, N, K, INT64_MAX, plan, true);
         const int64_t large = plan.kind == kTile256 ? list_256_bytes(count, M, N, K) : 0;
         bytes = bytes > large ? bytes : large;
-        if (with_lists) one = list;
     }
     return one ? bytes : -1;
-}
-}  // namespace
-extern "C" int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K) {
-    return group_bytes(a_kc, count, M, N, K, true);
 }
 // The form is not said: products with K = N are taken for the forward of square weights, others for weight gradients (gate and up are
 // long in both).  The workspace is enough for either form's plan.
 extern "C" int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
-    const int64_t fwd = group_bytes(1, count, M, N, K, false), wgrad = group_bytes(0, count, M, N, K, false);
+    const int64_t fwd = ezl_gemm_group_form_workspace_bytes(1, count, M, N, K), wgrad = ezl_gemm_group_form_workspace_bytes(0, count, M, N, K);
     if (fwd < 0 && wgrad < 0) return -1;
     if ((N[0] == K ? fwd : wgrad) < 0) return -1;
     return fwd > wgrad ? fwd : wgrad;

@@ -138,7 +138,8 @@ int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void* const* B, 
  * share memory, or any with result rows 8 MiB or more apart, go out one after the other, in the order of the list).  Forms: forward,
  * input gradient (bf16 results) and weight gradient (bf16 or fp32); all arrays are HOST arrays of `count` entries. */
 int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_t* N, int64_t K);
-/* the same for a given form: a_kc = 1 forward or input gradient, 0 weight gradient (the former guesses it from the sizes) */
+/* the same for a given form: a_kc = 1 forward, 0 weight gradient (the query above guesses it from the sizes: forward where N[0] = K).  An input
+ * gradient is answered for as a forward product of its sizes, with workspace enough for it. */
 int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K);
 int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
                         int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,

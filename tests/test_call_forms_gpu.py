@@ -55,7 +55,7 @@ def test_weight_gradients_of_one_weight_used_several_times(K, T, n_in, n_out, co
     """One buffer for several products, at sizes where they would otherwise share a launch: they are added one after the other."""
     from easyllm_amd import _lib
     print("one weight, several uses", T, n_in, n_out, count, flush=True)
-    assert _lib.gemm_group_workspace_bytes((n_out,) * count, (n_in,) * count, T) >= 0
+    assert _lib.gemm_group_form_workspace_bytes(False, (n_out,) * count, (n_in,) * count, T) >= 0
     x, dys = rnd(T, n_in, seed=1), [rnd(T, n_out, seed=2 + i) for i in range(count)]
     total = sum(dys[i].double().t() @ x.double() for i in range(count))
     bound = sum(product_bound(dy.t(), x) for dy in dys) + total.abs() * 2.0 ** -20 + 1e-5
@@ -82,7 +82,7 @@ def test_weight_gradients_into_buffers_with_far_apart_rows(K):
     """Rows 8 MiB apart are more than the smaller-tile kernels' offsets reach: such results are stored by the others."""
     from easyllm_amd import _lib
     T, n_in, outs, ld = 1024, 264, (8, 16), 1 << 21
-    assert _lib.gemm_group_workspace_bytes(outs, (n_in,) * 2, T) >= 0
+    assert _lib.gemm_group_form_workspace_bytes(False, outs, (n_in,) * 2, T) >= 0
     x, dys = rnd(T, n_in, seed=1), [rnd(T, o, seed=2 + i) for i, o in enumerate(outs)]
     bufs = [torch.full((o * ld,), 5.0, device="cuda") for o in outs]
     mgs = [b.as_strided((o, n_in), (ld, 1)) for b, o in zip(bufs, outs)]

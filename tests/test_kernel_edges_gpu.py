@@ -203,7 +203,8 @@ def test_gemm_products_in_one_launch(K, T, n_in, outs):
     from easyllm_amd import _lib
     x, ws = rnd(T, n_in, seed=1), [rnd(o, n_in, seed=2 + i) for i, o in enumerate(outs)]
     n = len(outs)
-    assert _lib.gemm_group_workspace_bytes((T,) * n, outs, n_in) >= 0 and _lib.gemm_group_workspace_bytes(outs, (n_in,) * n, T) >= 0
+    assert _lib.gemm_group_form_workspace_bytes(True, (T,) * n, outs, n_in) >= 0
+    assert _lib.gemm_group_form_workspace_bytes(False, outs, (n_in,) * n, T) >= 0
     for y, w in zip(K.linear_fwd_multi(x, ws), ws):
         ref = x.float() @ w.float().t()
         assert ((y.float() - ref).abs() <= gemm_bound(x, w.t()) + ref.abs() * 2.0 ** -8 + 1e-6).all()
