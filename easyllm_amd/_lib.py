@@ -88,6 +88,8 @@ _SPECIAL = {
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
     "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
     "ezl_gemm_group_form_workspace_bytes": ([_i32, _i32, _i64p, _i64p, _i64], _i64),
+    "ezl_gemm_plan": ([_i32, _i32, _i64p, _i64p, _i64] + [ctypes.POINTER(_i32)] * 4, _i32),
+    "ezl_layer_plan": ([_layerp, _i32], _i32),
     "ezl_layer_bytes": ([_layerp, _i32], _i64),
     "ezl_sumsq_partials": ([], _i64),
     "ezl_sumsq_list_partials": ([_i32], _i64),
@@ -171,6 +173,23 @@ def gemm_group_workspace_bytes(Ms, Ns, K):
 def gemm_group_form_workspace_bytes(a_kc, Ms, Ns, K):
     n = len(Ms)
     return load().ezl_gemm_group_form_workspace_bytes(1 if a_kc else 0, n, (_i64 * n)(*Ms), (_i64 * n)(*Ns), K)
+
+
+GEMM_FORMS = {"forward": 0, "weight gradient": 1, "input gradient": 2, "input gradient over pairs": 3}
+
+
+def gemm_plan(form, Ms, Ns, K):
+    """(one launch?, tile rows, tile columns, split, waves) of products of contiguous operands"""
+    n, out = len(Ms), [_i32() for _ in range(4)]
+    one = load().ezl_gemm_plan(GEMM_FORMS[form], n, (_i64 * n)(*Ms), (_i64 * n)(*Ns), K, *(ctypes.byref(x) for x in out))
+    if one < 0:
+        raise ValueError("gemm_plan: bad sizes")
+    return (one == 1,) + tuple(x.value for x in out)
+
+
+def layer_plan(layer, fp32):
+    """whether a layer's weight gradients go out as one list of tiles"""
+    return load().ezl_layer_plan(ctypes.byref(layer), 1 if fp32 else 0) == 1
 
 
 def layer_bytes(layer, which):

@@ -791,6 +791,11 @@ bool w4_pays(Form form, int64_t nk, int64_t items, int64_t ldb) {
         default: return nk >= 512;
     }
 }
+// the same for a product's launch: one that is split tiles only is judged by the length of a share
+bool w4_pays(Form form, const SplitPlan& plan, int64_t tiles, int64_t nk, int64_t ldb) {
+    const int64_t items = plan.full + (tiles - plan.full) * plan.nsplit;
+    return w4_pays(form, plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk, items, ldb);
+}
 // Workgroups of a 4-wave launch: one per CU, each walking over its tiles, while the K loop is short against a tile's ends; one per
 // tile on longer ones and over many rounds, where the hardware's order of dispatch keeps the workgroups that share operands together
 // (as weight gradients, one per tile against one per CU: 32000 x 5120 x 8192, 128 K tiles, 2164 us against 2314; 11008 x 4096 x
@@ -850,8 +855,7 @@ void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int
     // (fp32 input gradients stay with the 8-wave kernel)
     if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC) {
         constexpr Form form = !A_KC ? Form::weight_gradient : (B_KC ? Form::forward : Form::input_gradient);
-        // (a launch that is split tiles only is judged by the length of a share)
-        w4 = w4_pays(form, plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk, items, ldb) && w4_stores_ok<OutT>(C, N, ldc);
+        w4 = w4_pays(form, plan, (int64_t)tiles_m * tiles_n, nk, ldb) && w4_stores_ok<OutT>(C, N, ldc);
         if (w4)
             hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, false, KTAIL>), w4_grid(nk, items), dim3(256), 0, st, (const bf16_t*)A,
                                (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, items, plan, KSegments(), NoList());
@@ -1029,8 +1033,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     const SplitPlan plan = make_plan(tiles, (ktot + BK - 1) / BK, workspace, workspace_bytes);
     const int split_tiles = (int)tiles - plan.full;
     const int items = plan.full + split_tiles * plan.nsplit;
-    const int share = plan.nsplit > 1 && plan.full == 0 ? seg.nk / plan.nsplit : seg.nk;
-    const bool w4 = w4_pays(Form::input_gradient_segments, share, items, ldb) && w4_stores_ok<bf16_t>(C, N, ldc);
+    const bool w4 = w4_pays(Form::input_gradient_segments, plan, tiles, seg.nk, ldb) && w4_stores_ok<bf16_t>(C, N, ldc);
 #define EZL_MULTI(KT)                                                                                                                        \
     do {                                                                                                                                     \
         if (w4)                                                                                                                              \
@@ -1160,4 +1163,32 @@ int gemm_list(int count, const void* const* A, const void* const* B, void* const
     gemm_small_launch(form, false, plan, a, count, (hipStream_t)stream);
     EZL_LAUNCH_CHECK("ezl_gemm_bf16_group");
     return EZL_OK;
+}
+
+extern "C" int ezl_gemm_plan(int form, int count, const int64_t* M, const int64_t* N, int64_t K, int* rows, int* cols, int* split, int* waves) {
+    if (form < 0 || form > 3 || count < 1 || count > kMaxProblems || (form > 1 && count > 1) || !M || !N || K <= 0 || !rows || !cols || !split || !waves)
+        return -1;
+    for (int i = 0; i < count; ++i)
+        if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
+    const bool wgrad = form == 1;
+    const Form forms[4] = {Form::forward, Form::weight_gradient, Form::input_gradient, Form::input_gradient_segments};
+    const int64_t nk = (K + BK - 1) / BK;
+    GemmPlan plan;
+    bool one = true;
+    if (count == 1) {
+        plan = choose_plan(wgrad, M[0], N[0], nk, INT64_MAX);
+    } else {
+        one = group_plan(wgrad, count, M, N, K, INT64_MAX, plan, (!wgrad || count > kGroupMax) && list_256_pays(wgrad, count, M, N, K));
+    }
+    *rows = kKindRows[plan.kind];
+    *cols = kKindCols[plan.kind];
+    *split = plan.nsplit;
+    *waves = plan.kind == kTile64Waves ? 8 : 4;
+    if (plan.kind == kTile256) {
+        const int64_t tiles = list_256_tiles(count, M, N);
+        const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
+        *split = p.nsplit;
+        if (count == 1) *waves = w4_pays(forms[form], p, tiles, nk, form == 0 ? K : N[0]) ? 4 : 8;
+    }
+    return one;
 }

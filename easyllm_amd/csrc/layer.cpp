@@ -208,6 +208,12 @@ extern "C" int64_t ezl_layer_bytes(const ezl_layer* l, int which) {
     return -1;
 }
 
+extern "C" int ezl_layer_plan(const ezl_layer* l, int fp32) {
+    if (check("ezl_layer_plan", l)) return -1;
+    const Dims m(*l);
+    return WeightGradients(m).list_bytes(m.T, fp32 ? 4 : 2) >= 0;
+}
+
 extern "C" int ezl_layer_fwd(const ezl_layer* l, const void* x, void* y, void* saved, void* temp, void* st) {
     EZL_TRY(check("ezl_layer_fwd", l));
     EZL_REQUIRE(x && y && saved && temp, EZL_EINVAL, "ezl_layer_fwd: null pointer");

@@ -141,6 +141,11 @@ int64_t ezl_gemm_group_workspace_bytes(int count, const int64_t* M, const int64_
 /* the same for a given form: a_kc = 1 forward, 0 weight gradient (the query above guesses it from the sizes: forward where N[0] = K).  An input
  * gradient is answered for as a forward product of its sizes, with workspace enough for it. */
 int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, const int64_t* M, const int64_t* N, int64_t K);
+/* Which kernel products of contiguous operands with workspace enough take, for tests and profiles (host only).  form: 0 forward, 1 weight gradient, 2
+ * input gradient, 3 input gradient over pairs (one product, K the sum over the pairs).  A tile's rows and columns, over how many workgroups a tile's
+ * reduction is split (of 256 x 256 tiles: of those in the last round), waves of a workgroup (of 256 x 256 tiles: 4, or 8 for the kernel
+ * that takes one tile each).  Returns 1, or 0 where several products go out one by one (then as what they would take in one launch); -1: bad sizes. */
+int ezl_gemm_plan(int form, int count, const int64_t* M, const int64_t* N, int64_t K, int* rows, int* cols, int* split, int* waves);
 int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
                         int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,
                         const int* accumulate, void* workspace, int64_t workspace_bytes, void* stream);
@@ -266,6 +271,9 @@ typedef struct {
 enum { EZL_G_LN1, EZL_G_Q, EZL_G_K, EZL_G_V, EZL_G_O, EZL_G_LN2, EZL_G_GATE, EZL_G_UP, EZL_G_DOWN, EZL_G_BQ, EZL_G_BK, EZL_G_BV, EZL_G_COUNT };
 /* device bytes of the blocks below (256-byte aligned bases): which 0 = saved, 1 = forward temp, 2 = backward temp; -1: bad sizes */
 int64_t ezl_layer_bytes(const ezl_layer* layer, int which);
+/* for tests and profiles: 1 where the backward's weight gradients, all wanted and in one type (fp32, else bf16), go out as one list of tiles (ezl_gemm_plan
+ * of the seven says on which), 0 where as their operands appear; -1: bad sizes */
+int ezl_layer_plan(const ezl_layer* layer, int fp32);
 /* y = layer(x); `saved` is what ezl_layer_bwd needs, `temp` is free again when the call's work is done */
 int ezl_layer_fwd(const ezl_layer* layer, const void* x, void* y, void* saved, void* temp, void* stream);
 /* grads: EZL_G_COUNT entries, no two of which share memory (they are written in the kernels' order, several in one launch) */

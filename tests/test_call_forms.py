@@ -5,6 +5,7 @@ import time
 import pytest
 import torch
 
+import test_kernel_edges_gpu as edges
 from easyllm_amd import _lib
 from easyllm_amd import functional as F_
 
@@ -183,3 +184,48 @@ def test_a_decision_about_products_in_one_launch_is_remembered(T, h, f):
                 lib.ezl_gemm_group_form_workspace_bytes(*q)
             best[i] = min(best[i], time.perf_counter() - start)
     assert best[0] <= 1.4 * best[1]
+
+
+# ---- the GPU tests of single kernels reach the kernels they are about -----------------------------------------------------
+FORMS = ("forward", "input gradient", "weight gradient", "weight gradient")
+
+
+def listed(table):
+    return [(want, case) for want, cases in table.items() for case in cases]
+
+
+@pytest.mark.parametrize("want,case", listed(edges.SMALLER_TILES) + listed(edges.WIDE_TILES) + listed(edges.LARGEST_TILES))
+def test_products_at_tile_edges_take_the_tiles_they_are_listed_under(want, case):
+    form, M, N, K = case
+    _, rows, cols, _, waves = _lib.gemm_plan(FORMS[form], [M], [N], K)
+    assert (rows, cols, waves) == want
+
+
+@pytest.mark.parametrize("want,case", listed(edges.PAIRS) + listed(edges.PAIRS_WIDE))
+def test_products_over_pairs_take_the_tiles_they_are_listed_under(want, case):
+    T, h, widths = case
+    _, rows, cols, _, waves = _lib.gemm_plan("input gradient over pairs", [T], [h], sum(widths))
+    assert (rows, cols, waves) == want
+
+
+@pytest.mark.parametrize("T,h,widths", edges.FORWARD_LISTS)
+def test_forward_products_on_the_largest_tiles_are_one_launch(T, h, widths):
+    assert _lib.gemm_plan("forward", [T] * len(widths), widths, h)[:3] == (True, 256, 256)
+
+
+@pytest.mark.parametrize("want,case", listed(edges.LAYER_LISTS))
+def test_weight_gradients_of_a_layer_go_out_as_they_are_listed(want, case):
+    h, nq, nk, f, b, s, fp32 = case
+    layer = _lib.Layer(s=s, b=b, h=h, nq=nq, nk=nk, d=h // nq, f=f, ndocs=b, npos=s)
+    assert _lib.layer_plan(layer, fp32) == (want is not None)
+    if want:
+        kv = h // nq * nk
+        _, rows, cols, _, waves = _lib.gemm_plan("weight gradient", [h, kv, kv, h, f, f, h], [h] * 6 + [f], b * s)
+        assert (rows, cols, waves) == want
+
+
+@pytest.mark.parametrize("want,case", listed(edges.ATTENTION))
+def test_attention_takes_the_kernels_it_is_listed_under(want, case):
+    d, nq, nk, b, s, cu = case
+    ndocs = None if cu is None else len(cu) - 1
+    assert tuple(_lib.attn_plan(backward, ndocs, b * s, s, nq, nk, d) for backward in (False, True)) == want

@@ -81,30 +81,47 @@ def test_gemm_input_gradient_over_pairs_with_k_tails(K, T, n_in, outs):
     assert ((dx.float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
 
 
-@pytest.mark.parametrize("form,M,N,Kd", [
-    # 64 x 64, the waves share the reduction: fewer and more K tiles than waves, a ragged tail, one row, one vector of columns
-    (0, 65, 72, 1000), (2, 256, 264, 1531), (1, 1, 8, 520), (3, 8, 64, 449), (0, 64, 64, 64),
-    # 64 x 64: one and several K tiles per stage ring
-    (0, 1167, 1024, 1024), (1, 1000, 2056, 200), (2, 2048, 776, 2048), (3, 1544, 1032, 64),
-    # 128 x 128, whole and split
-    (1, 1167, 2816, 1032), (2, 2824, 1000, 1167), (0, 4100, 1800, 512), (2, 1024, 1032, 12000), (3, 1024, 1024, 9001),
-    # 256 x 128: one to four K tiles, tails, ragged edges, split
-    (0, 4001, 2056, 2048), (1, 1531, 4096, 712), (0, 4096, 2048, 64), (1, 4096, 2048, 128), (2, 4096, 2048, 192), (0, 4096, 2048, 200),
-    (1, 700, 3080, 5128), (3, 2048, 2048, 4000)])
+# (form, M, N, K) by the tile rows, columns and waves that a product of that size takes (test_call_forms.py holds the rule to this);
+# forms: 0 forward, 1 input gradient, 2 weight gradient in fp32, 3 in bf16
+SMALLER_TILES = {
+    # the waves share the reduction: fewer and more K tiles than waves, a ragged tail, one row, one vector of columns
+    (64, 64, 8): [(0, 65, 72, 1000), (2, 256, 264, 1531), (1, 1, 8, 520), (3, 8, 64, 449)],
+    # one and several K tiles per stage ring
+    (64, 64, 4): [(0, 64, 64, 64), (0, 1167, 1024, 1024), (2, 2048, 776, 2048), (3, 1544, 1032, 64)],
+    # whole and split, one to four K tiles, tails, ragged edges
+    (128, 128, 4): [(1, 1000, 2056, 200), (2, 2824, 1000, 1167), (0, 4100, 1800, 512), (2, 1024, 1032, 12000), (3, 1024, 1024, 9001), (0, 4096, 2048, 64),
+                    (1, 4096, 2048, 128), (2, 4096, 2048, 192), (0, 4096, 2048, 200), (3, 2048, 2048, 4000)],
+    (192, 128, 4): [(1, 1167, 2816, 1032), (1, 1531, 4096, 712)],
+    (256, 128, 4): [(1, 700, 3080, 5128)],
+    (256, 256, 8): [(0, 4001, 2056, 2048)]}
+WIDE_TILES = {
+    # K tails, ragged edges, element-wise stores, reductions split two to nine ways
+    (192, 128, 4): [(0, 1780, 2328, 344), (1, 742, 2720, 904), (0, 1099, 3819, 368), (0, 1531, 4096, 4096), (0, 392, 4688, 2680), (1, 453, 2752, 3368),
+                    (0, 556, 952, 5752), (2, 3456, 1336, 400), (2, 2224, 2168, 403), (3, 904, 4848, 467), (2, 904, 2488, 2160), (3, 384, 3240, 2765)],
+    # bf16 weight gradients: several tiles per workgroup, K tails, a long reduction
+    (256, 256, 4): [(3, 4872, 5128, 1040), (3, 5000, 6000, 1101), (3, 4096, 4096, 3205)],
+    (256, 128, 4): [(0, 1195, 4816, 696), (1, 1209, 5008, 672), (0, 3872, 1648, 720), (0, 1009, 2808, 3040), (1, 423, 4704, 3568)]}
+LARGEST_TILES = {
+    # several tiles per workgroup: ragged edges, K tails, a split last round, one K tile more or less than where the rule changes; one workgroup
+    # per tile: whole rounds and split ones, input gradients
+    (256, 256, 4): [(0, 5000, 20000, 1096), (0, 4096, 8192, 1024), (0, 4000, 17000, 4096), (0, 4000, 17000, 4104), (2, 5000, 20008, 1100),
+                    (2, 4096, 4352, 4160), (0, 4096, 4096, 8200), (2, 3000, 3080, 9000), (1, 4096, 4096, 10240), (1, 4100, 6152, 10248)],
+    (256, 256, 8): [(2, 8192, 8192, 2048)],  # rows of B a multiple of 16 KiB apart
+    (256, 128, 4): [(1, 4100, 5128, 10248)]}
+
+
+def products(table):
+    return [case for cases in table.values() for case in cases]
+
+
+@pytest.mark.parametrize("form,M,N,Kd", products(SMALLER_TILES))
 def test_gemm_smaller_tiles(K, form, M, N, Kd):
     print("gemm", form, M, N, Kd, flush=True)
     check_gemm(K, form, M, N, Kd)
     check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
 
 
-@pytest.mark.parametrize("form,M,N,Kd", [
-    # 192 x 128: K tails, ragged edges, element-wise stores, reductions split two to nine ways
-    (0, 1780, 2328, 344), (1, 742, 2720, 904), (0, 1099, 3819, 368), (0, 1531, 4096, 4096), (0, 392, 4688, 2680), (1, 453, 2752, 3368),
-    (0, 556, 952, 5752), (2, 3456, 1336, 400), (2, 2224, 2168, 403), (3, 904, 4848, 467), (2, 904, 2488, 2160), (3, 384, 3240, 2765),
-    # 256 x 256, bf16 weight gradients: several tiles per workgroup, K tails, a long reduction
-    (3, 4872, 5128, 1040), (3, 5000, 6000, 1101), (3, 4096, 4096, 3205),
-    # 256 x 128
-    (0, 1195, 4816, 696), (1, 1209, 5008, 672), (0, 3872, 1648, 720), (0, 1009, 2808, 3040), (1, 423, 4704, 3568)])
+@pytest.mark.parametrize("form,M,N,Kd", products(WIDE_TILES))
 def test_gemm_wide_tiles(K, form, M, N, Kd):
     print("gemm", form, M, N, Kd, flush=True)
     check_gemm(K, form, M, N, Kd)
@@ -116,8 +133,13 @@ def test_gemm_wide_tiles(K, form, M, N, Kd):
         assert torch.equal(f, f.bfloat16().float()) and ((f - x.float() @ w.float().t()).abs() <= tol).all()
 
 
-@pytest.mark.parametrize("T,n_in,outs", [(1167, 1024, (1024, 256, 256)), (2048, 768, (2048, 2056)), (700, 3072, (3072, 1024, 1032)),
-                                         (4000, 2048, (2048, 2048, 2056)), (1024, 256, (256, 256, 256))])
+# (T, h, widths) of dx = sum of dy_i w_i by tile and waves
+PAIRS = {(64, 64, 4): [(1167, 1024, (1024, 256, 256))], (64, 64, 8): [(1024, 256, (256, 256, 256))], (192, 128, 4): [(2048, 768, (2048, 2056))],
+         (256, 128, 4): [(700, 3072, (3072, 1024, 1032)), (4000, 2048, (2048, 2048, 2056))]}
+PAIRS_WIDE = {(192, 128, 4): [(742, 2720, (304, 304, 296)), (453, 2752, (1128, 1120, 1120))]}
+
+
+@pytest.mark.parametrize("T,n_in,outs", products(PAIRS))
 def test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs):
     print("dgrad multi", T, n_in, outs, flush=True)
     ld = max(outs)
@@ -131,7 +153,7 @@ def test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs):
     assert ((dx.float() - 2 * ref).abs() <= 2 * gemm_bound(A, B) + ref.abs() * 2.0 ** -6 + 1e-6).all()
 
 
-@pytest.mark.parametrize("T,n_in,outs", [(742, 2720, (304, 304, 296)), (453, 2752, (1128, 1120, 1120))])
+@pytest.mark.parametrize("T,n_in,outs", products(PAIRS_WIDE))
 def test_gemm_input_gradient_over_pairs_on_wide_tiles(K, T, n_in, outs):
     test_gemm_input_gradient_over_pairs_on_smaller_tiles(K, T, n_in, outs)
 
@@ -153,11 +175,7 @@ def test_gemm_smaller_tiles_leave_what_is_outside_the_result_alone(K):
         assert (border == 7.0).all(), (form, M, N, Kd)
 
 
-@pytest.mark.parametrize("form,M,N,Kd", [
-    # several tiles per workgroup: ragged edges, K tails, a split last round, one K tile more or less than where the rule changes
-    (0, 5000, 20000, 1096), (0, 4096, 8192, 1024), (0, 4000, 17000, 4096), (0, 4000, 17000, 4104), (2, 5000, 20008, 1100), (2, 4096, 4352, 4160),
-    # one workgroup per tile: whole rounds and split ones, input gradients
-    (0, 4096, 4096, 8200), (2, 3000, 3080, 9000), (1, 4100, 5128, 10248), (1, 4096, 4096, 10240), (2, 8192, 8192, 2048)])
+@pytest.mark.parametrize("form,M,N,Kd", products(LARGEST_TILES))
 def test_gemm_four_wave_kernel(K, form, M, N, Kd):
     print("gemm", form, M, N, Kd, flush=True)
     check_gemm(K, form, M, N, Kd)
@@ -182,8 +200,11 @@ def test_gemm_four_wave_kernel_over_pairs(K):
     assert ((dx.float() - 2 * ref).abs() <= 2 * bound + ref.abs() * 2.0 ** -6 + 1e-6).all()
 
 
-# split last rounds, K tails, ragged tiles, widths that differ
-@pytest.mark.parametrize("T,n_in,outs", [(1726, 3072, (9920, 9920)), (1726, 3080, (9920, 9912)), (2050, 2056, (5504, 5504, 2056)), (4000, 2048, (5504, 5504))])
+# split last rounds, K tails, ragged tiles, widths that differ: all in one launch of 256 x 256 tiles
+FORWARD_LISTS = [(1726, 3072, (9920, 9920)), (1726, 3080, (9920, 9912)), (2050, 2056, (5504, 5504, 2056)), (4000, 2048, (5504, 5504))]
+
+
+@pytest.mark.parametrize("T,n_in,outs", FORWARD_LISTS)
 def test_gemm_forward_products_in_one_launch_on_the_largest_tiles(K, T, n_in, outs):
     print("gemm forward list", T, n_in, outs, flush=True)
     from easyllm_amd import _lib
@@ -219,18 +240,23 @@ def test_gemm_products_in_one_launch(K, T, n_in, outs):
             assert ((dw.float() - ref).abs() <= tol).all()
 
 
-@pytest.mark.parametrize("h,nq,nk,f,b,s,main_grads", [(64, 1, 1, 72, 1, 3, True), (256, 4, 1, 688, 2, 511, True), (768, 12, 12, 2048, 2, 1024, True),
-                                                      (1024, 16, 4, 2816, 3, 389, False), (1024, 8, 8, 2816, 1, 4000, True),
-                                                      (256, 4, 4, 1000, 1, 16001, True),
-                                                      # 256 x 256 tiles: a split last round, with a K tail, ragged tiles, less than a round,
-                                                      # more results than the cache holds
-                                                      (2048, 16, 16, 5504, 1, 2048, True), (2048, 16, 4, 5504, 2, 1001, True),
-                                                      (1920, 15, 15, 5056, 1, 2503, True), (1024, 8, 2, 3328, 1, 4003, True),
-                                                      (2944, 23, 23, 9216, 1, 1691, True), (2048, 16, 4, 5504, 1, 2961, False),
-                                                      (1792, 14, 14, 4672, 1, 4608, False)])
+# (h, nq, nk, f, b, s, fp32) of a layer by the tile and waves of its seven weight gradients in one list; None: in pieces
+LAYER_LISTS = {
+    (64, 64, 4): [(64, 1, 1, 72, 1, 3, True)],
+    (64, 64, 8): [(256, 4, 1, 688, 2, 511, True)],
+    # one, two or several K tiles per wave, K tails, split reductions
+    (128, 128, 4): [(768, 12, 12, 2048, 2, 1024, True), (256, 4, 4, 1000, 1, 16001, True)],
+    (192, 128, 4): [(1024, 16, 4, 2816, 3, 389, False)],
+    # a split last round, with a K tail, ragged tiles, less than a round, more results than the cache holds, bf16
+    (256, 256, 4): [(1024, 8, 8, 2816, 1, 4000, True), (2048, 16, 16, 5504, 1, 2048, True), (2048, 16, 4, 5504, 2, 1001, True),
+                    (1920, 15, 15, 5056, 1, 2503, True), (1024, 8, 2, 3328, 1, 4003, True), (2944, 23, 23, 8360, 1, 987, True),
+                    (2048, 16, 4, 5504, 1, 2961, False), (1792, 14, 14, 4672, 1, 4608, False)],
+    None: [(2944, 23, 23, 9216, 1, 1691, True)]}
+
+
+@pytest.mark.parametrize("h,nq,nk,f,b,s,main_grads", products(LAYER_LISTS))
 def test_weight_gradients_of_a_layer_in_one_launch(h, nq, nk, f, b, s, main_grads):
-    """A layer's seven weight gradients as one list of tiles (at these sizes: one, two or several K tiles per wave, K tails, 64, 128,
-    256 x 128 and 256 x 256 tiles, split reductions), overwritten and then added to, against the composed layer's separate products: activations and
+    """A layer's seven weight gradients as one list of tiles, overwritten and then added to, against the composed layer's separate products: activations and
     their gradients are the same bits, the sums over the tokens are in fp32 in another order (bf16 results: one rounding apart)."""
     from easyllm_amd import runner
     print("weight gradients of a layer", h, f, b, s, flush=True)
@@ -278,16 +304,23 @@ def attention_reference(q, k, v, do, cu):
     return back(out), lse, back(dq), back(dk), back(dv)
 
 
-@pytest.mark.parametrize("d,nq,nk,b,s,cu", [
-    # 32 rows per workgroup: tile edges, waves without a tile, more tiles than waves, grouped queries, documents
-    (64, 2, 2, 1, 1, None), (64, 4, 1, 3, 31, None), (128, 2, 2, 2, 33, None), (64, 3, 3, 1, 255, None), (128, 2, 1, 1, 257, None),
-    (64, 4, 4, 2, 512, None), (128, 3, 1, 1, 640, None), (64, 8, 2, 1, 389, [0, 1, 2, 65, 129, 200, 389]), (128, 4, 2, 1, 330, [0, 96, 97, 330]),
-    (64, 2, 2, 2, 128, [0, 100, 128, 200, 256]),
-    # 128 rows, forward with two key groups, dQ and dK/dV in one launch (the last tile missing for a group, documents, split groups)
-    (64, 24, 24, 2, 385, None), (128, 16, 4, 3, 449, None), (128, 24, 24, 1, 513, None), (64, 40, 8, 1, 641, [0, 63, 64, 330, 641]),
-    (128, 40, 40, 1, 700, [0, 129, 700]),
-    # 128 rows, one launch for the backward only, then neither
-    (64, 60, 60, 2, 100, None), (128, 30, 15, 4, 130, None), (64, 64, 64, 8, 140, None)])
+# (d, nq, nk, b, s, documents) by what forward and backward take: 0 workgroups of 128 rows, 1 the same with key groups / in one launch, 2 of 32 rows
+ATTENTION = {
+    # one tile, tile edges, waves without a tile, more tiles than waves, grouped queries, documents
+    (0, 2): [(64, 2, 2, 1, 1, None), (64, 4, 1, 3, 31, None), (128, 2, 2, 2, 33, None), (128, 4, 2, 1, 330, [0, 96, 97, 330]),
+             (64, 2, 2, 2, 128, [0, 100, 128, 200, 256])],
+    (2, 2): [(64, 3, 3, 1, 255, None), (128, 2, 1, 1, 257, None), (64, 4, 4, 2, 512, None), (128, 3, 3, 1, 65, None), (64, 8, 8, 1, 97, None),
+             (64, 4, 2, 1, 700, [0, 300, 700]), (128, 6, 6, 1, 900, [0, 1, 450, 900]), (64, 2, 1, 1, 2048, [0, 600, 601, 2048])],
+    (2, 1): [(128, 3, 1, 1, 640, None), (64, 12, 4, 1, 1000, [0, 255, 1000]), (64, 16, 16, 1, 800, [0, 97, 800])],
+    # the last tile missing for a key group, documents, split groups
+    (1, 1): [(64, 24, 24, 2, 385, None), (128, 16, 4, 3, 449, None), (128, 24, 24, 1, 513, None), (64, 12, 12, 1, 2048, [0, 1, 66, 700, 2048]),
+             (128, 8, 8, 1, 1030, [0, 64, 193, 1030])],
+    (0, 1): [(64, 60, 60, 2, 100, None), (64, 8, 2, 1, 389, [0, 1, 2, 65, 129, 200, 389])],
+    (1, 0): [(128, 38, 38, 1, 1025, None)],
+    (0, 0): [(128, 30, 15, 4, 130, None), (64, 64, 64, 8, 140, None), (64, 40, 8, 1, 641, [0, 63, 64, 330, 641]), (128, 40, 40, 1, 700, [0, 129, 700])]}
+
+
+@pytest.mark.parametrize("d,nq,nk,b,s,cu", products(ATTENTION))
 def test_attention_for_every_split_of_the_work(K, d, nq, nk, b, s, cu):
     """Against float64.  Inputs are exact; probabilities, dS and the results are rounded to bf16 (2^-9 each): 1e-2 of a result's norm.
     dS is a difference that may cancel (a document of one token: exactly), off by scale |K| |dO . (O - its bf16 value)|."""
