@@ -651,11 +651,17 @@ GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, in
     // 128 x 128 tiles read every operand most often, which lists of weight gradients over many tokens feel: a layer's seven over 11918 tokens at
     // h = 1024 400 us (estimate 309), with 256 x 128 tiles 354 (315).
     const double list_128 = wgrad && count > 3 ? 1.05 : 1;
+    // Weight gradients of two rounds of 256 x 256 tiles or more, as of a vocabulary, are bound by their results' way to memory as much as by the tiles,
+    // which the rates of one round do not know: the smaller tiles have to win by a twelfth.  50304 x 1024 x 1167, 256 x 256 against 128 x 128 tiles: 147, 175 us
+    // (bf16 122, 131); bf16 70528 x 2176 x 477 198, 221; 151808 x 1024 x 711 299, 319.  160 such products: what is taken is 2.2 % behind the fastest, without
+    // this 3.3 (those that overwrite fp32 2.9 and 5.4).
+    double margin = 1;
     GemmPlan best = {kTile256, 1};
     double t_best = 1e30;
     if (count == 1 || list_256) {
         int64_t tiles = 0;
         for (int i = 0; i < count; ++i) tiles += tiles_of(kTile256, M[i], N[i]);
+        if (wgrad && count == 1 && tiles >= 2 * kCus) margin = 1.08;
         const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
         const int64_t need = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * 4 : 0;
         t_best = cost_256(rates[kTile256], tiles, nk, need <= room) / (list_256 ? kMarginList256 : 1);
@@ -669,14 +675,14 @@ GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, in
                           tiles * s * gemm_kind_bm(kind) * gemm_kind_bn(kind) * 4 > room))
                 break;
             const double t = cost_small(rates[kind], kind, tiles, nk, s) * (kind == kTile128 ? list_128 : 1);
-            if (t < t_best) {
-                t_best = t;
+            if (t * margin < t_best) {
+                t_best = t * margin;
                 best.kind = kind;
                 best.nsplit = (int)s;
             }
         }
     }
-    if (time) *time = t_best;
+    if (time) *time = best.kind == kTile256 ? t_best : t_best / margin;
     return best;
 }
 // The search takes 3 us, as long as a small product: a thread remembers its last 256 products by their sizes.

@@ -229,3 +229,13 @@ def test_attention_takes_the_kernels_it_is_listed_under(want, case):
     d, nq, nk, b, s, cu = case
     ndocs = None if cu is None else len(cu) - 1
     assert tuple(_lib.attn_plan(backward, ndocs, b * s, s, nq, nk, d) for backward in (False, True)) == want
+
+
+# (measured, us, 256 x 256 against the smaller tiles whose estimate is lower)
+@pytest.mark.parametrize("M,N,T,tile", [
+    (50304, 1024, 1167, 256),  # 147, 175
+    (70528, 2176, 477, 256),   # (bf16) 198, 221
+    (151808, 1024, 711, 256),  # (bf16) 299, 319
+    (11008, 4096, 1531, 256), (32000, 768, 1024, 128)])
+def test_weight_gradients_of_a_vocabulary_take_smaller_tiles_only_by_a_margin(M, N, T, tile):
+    assert _lib.gemm_plan("weight gradient", [M], [N], T)[1] == tile
