@@ -430,6 +430,10 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 //             (130) 19.5, 21.9
 //             d 128:  6 / 2 x 145 (18) 15.8, 11.5; 19 / 2 x 128 (38) 14.2, 16.5; 3 / 4 x 428 (42) 26.8, 20.9; 2 / 3 x 1455 (70) 71, 51; 5 / 8 x 209
 //             (70) 19.3, 25.5; 4 / 3 x 1281 (124) 66, 73
+// Long rows pay up to 128 blocks (512 workgroups of keys, 512 of queries), not beyond.  Backward, heads / rows x length (128-row blocks), us with two launches, one,
+// these:
+//   d 64:  1 / 16384 (128) 570, 353, 257; 3 / 8192 (192) 293, 181, 198; 1 / 4 x 8192 (256) 294, 181, 237; 4 / 16384 (512) 621, 609, 868
+//   d 128: 1 / 16384 (128) 856, 705, 540; 3 / 8192 (192) 440, 371, 443; 1 / 4 x 8192 (256) 435, 368, 529; 4 / 16384 (512) 1007, 1118, 1987
 // A row of up to 64 tokens is one tile, which there is nothing to share out of; one of two tiles gains only while a CU has one workgroup.  Forward, heads /
 // rows x length (32-row workgroups):
 //   d 64:  4 / 64 (8) 4.9, 5.3; 41 / 3 x 33 (246) 5.0, 5.6; 16 / 4 x 65 (192) 6.2, 5.5; 24 / 4 x 65 (288) 6.3, 6.8; 16 / 4 x 97 (256) 6.6, 5.7; 64 / 2 x 97 (512) 6.6,
@@ -445,14 +449,17 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_small_kernel(AttnParams p, i
 //   forward   d 64:  8 / 31 (59, 72) 10.5, 11.2, 20.2; 4 / 64 x 64 10.5, 11.8, 13.4; 4 / 8 x 512 17.0, 16.0, 16.8; 1 / 29 (414, 507) 18.1, 17.1, 17.2; 4 / 7 (586, 2132)
 //             37.1, 31.2, 27.9
 //             d 128: 2 / 32 x 128 14.2, 15.1, 14.5; 2 / 16 x 256 16.3, 16.8, 15.6; 2 / 7 (586, 2132) 45.8, 39.7, 36.3
-//   backward  d 64:  4 / 32 x 512 63, 74, 144; 4 / 16 x 256 30.8, 17.9, 31.5; 4 / 7 (586, 2132) 95, 58, 56; 1 / 45 (188, 752) 48, 28.2, 28.3
-//             d 128: 4 / 64 x 128 42, 47, 127; 2 / 16 x 256 39, 24.5, 34.6; 1 / 16 (320, 736) 63, 43, 33; 2 / 7 (586, 2132) 135, 101, 65
+//   backward  d 64:  4 / 32 x 512 63, 74, 144; 4 / 16 x 256 30.8, 17.9, 31.5; 4 / 7 (586, 2132) 95, 58, 56; 1 / 45 (188, 752) 48, 28.2, 28.3;
+//             2 / 8 x 1024 58, 35, 44; 2 / 4 x 4096 165, 111, 163; 2 / 2 x 2048 91, 56, 44
+//             d 128: 4 / 64 x 128 42, 47, 127; 2 / 16 x 256 39, 24.5, 34.6; 1 / 16 (320, 736) 63, 43, 33; 2 / 7 (586, 2132) 135, 101, 65;
+//             2 / 8 x 1024 80, 59, 93; 2 / 4 x 4096 239, 184, 359; 2 / 2 x 2048 129, 96, 69
 bool attn_small_pays(const AttnSizes& z, bool backward) {
     const int64_t length = z.documents ? z.mean_length() : z.s_len, group = z.nq / z.nk;
     auto blocks = [&](int64_t n) { return (z.documents ? z.launched(n) : z.rows() * ((z.s_len + n - 1) / n)) * z.nq; };
     if (!backward) return length > (z.documents ? 255 : 64) && blocks(32) <= (z.d == 64 && length >= 128 ? 512 : 256);
     if (group > 2 && (length + 31) / 32 * group > 16) return false;
-    return blocks(128) <= (z.documents ? 48 + length / 8 : (z.d == 64 ? 64 : 32) + length / 32);
+    const int64_t limit = (z.documents || z.d == 64 ? 64 : 32) + length / 32;
+    return blocks(128) <= (limit < 128 ? limit : 128);
 }
 
 void attn_small_fwd(const AttnParams& p, int d, hipStream_t stream) {

@@ -151,10 +151,26 @@ def test_attention_backward_of_grouped_queries_on_32_rows_only_with_short_chains
     (True, 64, 4, 4096, 16, 1),     # 30.8, 17.9, 31.5
     (True, 128, 4, 8192, 64, 0),    # 42, 47, 127
     (True, 128, 1, 5115, 16, 2),    # 63, 43, 33
+    (True, 64, 2, 8192, 8, 1),      # 58, 35, 44
+    (True, 128, 2, 16384, 4, 1),    # 239, 184, 359
+    (True, 128, 2, 4096, 2, 2),     # 129, 96, 69
     # empty documents: launches of 2^32 threads or more along one axis are refused, which 128-row kernels reach last
     (False, 64, 512, 16, 33000, 0), (True, 64, 512, 16, 33000, 0), (True, 64, 128, 129, 70000, 0)])
 def test_attention_of_packed_rows_goes_by_the_length_of_the_documents(backward, d, heads, tokens, ndocs, plan):
     assert _lib.attn_plan(backward, ndocs, tokens, tokens, heads, heads, d) == plan
+
+
+# (measured, us: 128 rows in two launches, in one, 32 rows)
+@pytest.mark.parametrize("d,heads,b,s,plan", [
+    (64, 1, 1, 16384, 2),   # 570, 353, 257
+    (64, 1, 4, 8192, 1),    # 294, 181, 237
+    (64, 4, 1, 16384, 0),   # 621, 609, 868
+    (128, 1, 1, 16384, 2),  # 856, 705, 540
+    (128, 1, 4, 8192, 1),   # 435, 368, 529
+    (128, 3, 1, 12000, 1),  # 646, 546, 881
+    (128, 4, 1, 16384, 0)])  # 1007, 1118, 1987
+def test_attention_backward_of_long_rows(d, heads, b, s, plan):
+    assert _lib.attn_plan(True, None, b * s, s, heads, heads, d) == plan
 
 
 # (measured, us: 128-row kernel, 32-row kernel)
