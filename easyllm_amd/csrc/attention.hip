@@ -885,13 +885,13 @@ bool bwd_one_launch_pays(int64_t blocks, int64_t s_len, int64_t d) {
 // it searches the documents and when it finds no block.  Heads, documents x length (mean, longest) of one row, us with two groups or one launch after
 // those without:
 //   forward   d 64:  12 / 64 x 64 13.5, 30.7; 12 / 8 x 512 19.2, 25.7; 2 / 128 x 128 14.3, 16.0; 2 / 32 x 512 19.4, 18.0; 12 / 4 x 512 16.6, 15.6
-//             d 128: 4 / 128 x 64 16.6, 27.7; 4 / 16 x 512 23.3, 22.5; 8 / 4 x 512 20.1, 19.6; 10 / 27 (179, 445) 33.6, 43.7
+//             d 128: 4 / 128 x 64 16.6, 27.7; 4 / 16 x 512 23.3, 22.5; 8 / 4 x 512 20.1, 19.6; 10 / 27 (179, 445) 33.6, 43.7; 4 / 20 (349, 547) 24.3, 30.0
 //   backward  d 64:  12 / 64 x 64 49, 68; 12 / 8 x 512 53, 54; 2 / 128 x 128 32.7, 35.2; 4 / 16 x 256 31, 18; 16 / 4 x 256 28, 17; 12 / 4 (512, 1010) 57, 38
 //             d 128: 4 / 64 x 128 42, 47; 4 / 16 x 512 59, 58; 8 / 8 x 256 39, 25; 3 / 72 (51, 85) 29.8, 31.4
-// 430 batches of 1 - 93 heads, 256 - 16384 tokens and log-uniform lengths, with attn_small_pays: forward 0.9 %, backward 1.4 % behind the fastest of
-// the three, at worst 4 % behind the 128-row kernels and 4 % and 28 % faster on average; by the rules for whole rows 8.7 and 15 % behind, at worst 2.3 and
+// 430 batches of 1 - 93 heads, 256 - 16384 tokens and log-uniform lengths, with attn_small_pays: forward 1.1 %, backward 1.4 % behind the fastest of
+// the three, at worst 4 % behind the 128-row kernels and 4 % and 27 % faster on average; by the rules for whole rows 8.7 and 15 % behind, at worst 2.3 and
 // 3.0 times the 128-row kernels.
-bool fwd_key_groups_pay_documents(int64_t launched, int64_t mean) { return launched <= 320 ? mean >= 192 : launched <= 384 && mean >= 768; }
+bool fwd_key_groups_pay_documents(int64_t launched, int64_t mean) { return launched <= 272 ? mean >= 192 : launched <= 384 && mean >= 768; }
 bool bwd_one_launch_pays_documents(int64_t launched, int64_t mean) {
     return launched <= 256 || (launched <= 320 && mean >= 128) || (launched <= 384 && mean >= 384);
 }

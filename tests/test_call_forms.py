@@ -143,6 +143,7 @@ def test_attention_backward_of_grouped_queries_on_32_rows_only_with_short_chains
     (False, 64, 12, 4096, 64, 0),   # 13.5, 30.7, 35.6
     (False, 64, 8, 1811, 31, 0),    # 10.5, 11.2, 20.2
     (False, 64, 12, 2048, 4, 1),    # 16.6, 15.6, 26.4
+    (False, 128, 4, 6968, 20, 0),   # 24.3, 30.0
     (False, 64, 2, 4096, 7, 2),     # (four heads: 37.1, 31.2, 27.9)
     (False, 128, 4, 8192, 128, 0),  # 16.6, 27.7, 53.8
     (True, 64, 4, 16384, 256, 0),   # 79, 102, 122
