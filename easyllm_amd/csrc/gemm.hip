@@ -252,18 +252,23 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // One wave per SIMD with 8 x 8 MFMA 16x16x32 tiles: the 256 accumulator registers live in AGPRs, a K tile costs a third
 // fewer LDS fragment reads than with 128 x 64 wave tiles, and nothing else runs on the SIMD to cover a stall, so the K loop
 // is laid out step by step (one MFMA per step, a sched_barrier after each):
-//   phase A of tile kt: 64 MFMAs on k half 0 (fragment set 0); the 16 fragments of k half 1 are read meanwhile
-//   wait for the loads in flight + barrier: tile kt + 1 has landed, every wave is done reading the stage of tile kt
-//   phase B of tile kt: 64 MFMAs on k half 1 (set 1); the fragments of tile kt + 1, k half 0 are read meanwhile and the
-//                       16 wave loads of tile kt + 2 go out into the stage of tile kt
+//   phase A of tile kt: 64 MFMAs on k half 0 (fragment set 0); the 16 fragments of k half 1 are read meanwhile and the 8 wave
+//                       loads of B tile kt + 2 go out into the stage of B tile kt - 1
+//   wait for A tile kt + 1 (B tile kt + 1 is older, B tile kt + 2 stays in flight) + barrier: tile kt + 1 has landed, every wave is
+//                       done reading the stages of tile kt
+//   phase B of tile kt: 64 MFMAs on k half 1 (set 1); the fragments of tile kt + 1, k half 0 are read meanwhile and the 8 wave
+//                       loads of A tile kt + 2 go out into the stage of A tile kt
+// What bounds it is the way of the operands' lines to the CU.  With two stages of both operands, all 16 loads in phase B and waited for
+// behind the next phase A, operands from HBM (weights, in every step) cost as much with zeros in them, where no clock gives way, as with
+// random data: loads alone took 1.45 us per K tile, from the last-level cache 1.0, the products 1.25.  The 160 KiB hold two stages
+// of A and three of B, loads go out in the first half of each phase (one every fourth MFMA: the CU's address unit takes 16 cycles per 1 KiB wave
+// load, the four waves' keep it busy for just that half; every second MFMA 99 us where this takes 96, B's over all of phase A 97), and B
+// has more than a K tile's time on the way, A three quarters.  Operands from HBM, us before and now: 4096 x 4096 x 4096 109 -> 96,
+// 4096 x 4096 x 11008 277 -> 240, 2048 x 4096 x 11008 271 -> 206, weight gradient 11008 x 4096 x 4096 314 -> 288; from the cache 94 -> 94, 233 -> 230.
 // The loop's back edge sits right behind the barrier, where no LDS read is in flight, so inside the body the compiler's
 // waits on the fragment reads are exact counts.  Reads are issued in the first half of a phase (one every second MFMA) and
-// have landed long before the next phase needs them; loads are issued one every fourth MFMA over the whole of phase B:
-// the CU's address unit takes 16 cycles per 1 KiB wave load, i.e. the four waves' loads keep it busy for all of phase B,
-// and issued any faster they fill its queue and the issuing wave stalls with its MFMAs behind it (measured on all-zero
-// operands, 4096 x 4096 x K: 0.96 us per K tile with this spacing, 1.12 with one load every second MFMA, 1.23 back to
-// back; the 8-wave kernel 1.05).
-// A workgroup works off items blockIdx.x, + gridDim.x, ... as one stream of K tiles: the last two K tiles of an item bring in the
+// have landed long before the next phase needs them.
+// A workgroup works off items blockIdx.x, + gridDim.x, ... as one stream of K tiles: the last K tiles of an item bring in the
 // first two of the next, and the finished accumulators are stored while those are on their way (their wait is a count that
 // leaves the stores in flight).  With one workgroup per tile a tile cost 14 us on top of its K tiles - a workgroup's start, the first
 // loads, the stores drained before its LDS is free - which is a third of it at 32 K tiles: 4000 x 32000 x 2048 444 -> 407 us,
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
                                                          int tiles_m, int tiles_n, int items, const SplitPlan plan, const KSegments seg,
                                                          const std::conditional_t<LIST, GemmSmallArgs, NoList> list) {
     static_assert(!LIST || (A_KC == B_KC && !MULTI), "lists are of forward products or weight gradients");
-    __shared__ __attribute__((aligned(1024))) bf16_t smem[4 * DTILE];  // A0 B0 A1 B1
+    __shared__ __attribute__((aligned(1024))) bf16_t smem[5 * DTILE];  // A0 A1 B0 B1 B2
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
@@ -384,109 +389,137 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     f32x4 acc[8][8];
     bf16x8 fa[2][8], fb[2][8];
     // fragment f of a k half: f < 8 the B fragment f, else the A fragment f - 8
-    auto read_frag = [&](const bf16_t* sA, int ks, int buf, auto F) {
+    auto read_frag = [&](const bf16_t* sA, const bf16_t* sB, int ks, int buf, auto F) {
         constexpr int f = decltype(F)::value;
-        if constexpr (f < 8) fb[buf][f] = rb.template read<f>(sA + DTILE, ks);
+        if constexpr (f < 8) fb[buf][f] = rb.template read<f>(sB, ks);
         else fa[buf][f - 8] = ra.template read<f - 8>(sA, ks);
     };
     __amdgpu_buffer_rsrc_t ga, gb;
-    int kv = BK;
-    auto tile_bases = [&](const Item& x, int t) {
-        const bf16_t *Ab, *Bb;
+    int kva = BK, kvb = BK;
+    auto a_base = [&](const Item& x, int t) {
         t += x.kt0;
         if constexpr (LIST) {
-            kv = K - t * BK;
+            kva = K - t * BK;
             ga = la.base(x.a + (int64_t)t * BK * (A_KC ? 1 : x.lda));
-            gb = lb.base(x.b + (int64_t)t * BK * (B_KC ? 1 : x.ldb));
-            return;
+        } else {
+            const bf16_t *Ab, *Bb;
+            pick_segment<MULTI>(A, B, K, seg, t, kva, Ab, Bb);
+            ga = la.base(Ab + x.a_blk + (int64_t)t * astep);
         }
-        pick_segment<MULTI>(A, B, K, seg, t, kv, Ab, Bb);
-        ga = la.base(Ab + x.a_blk + (int64_t)t * astep);
-        gb = lb.base(Bb + x.b_blk + (int64_t)t * bstep);
+    };
+    auto b_base = [&](const Item& x, int t) {
+        t += x.kt0;
+        if constexpr (LIST) {
+            kvb = K - t * BK;
+            gb = lb.base(x.b + (int64_t)t * BK * (B_KC ? 1 : x.ldb));
+        } else {
+            const bf16_t *Ab, *Bb;
+            pick_segment<MULTI>(A, B, K, seg, t, kvb, Ab, Bb);
+            gb = lb.base(Bb + x.b_blk + (int64_t)t * bstep);
+        }
     };
     // load l of a tile pair: l < 8 piece l of the A tile, else piece l - 8 of the B tile
-    auto issue_load = [&](bf16_t* st, auto L) {
+    auto issue_load = [&](bf16_t* sA, bf16_t* sB, auto L) {
         constexpr int l = decltype(L)::value;
-        if constexpr (l < 8) la.template issue_at<l>(ga, st, lane, wave, kv);
-        else lb.template issue_at<l - 8>(gb, st + DTILE, lane, wave, kv);
+        if constexpr (l < 8) la.template issue_at<l>(ga, sA, lane, wave, kva);
+        else lb.template issue_at<l - 8>(gb, sB, lane, wave, kvb);
     };
 
-    tile_bases(it, 0);
-    static_for<0, 16>([&](auto L) { issue_load(smem, L); });
-    tile_bases(it, 1);
-    static_for<0, 16>([&](auto L) { issue_load(smem + 2 * DTILE, L); });
+    int a0 = 0, a1 = DTILE, b0 = 2 * DTILE, b1 = 3 * DTILE, b2 = 4 * DTILE;  // stages of K tiles kt, kt + 1 (and kt + 2)
+    a_base(it, 0);
+    b_base(it, 0);
+    static_for<0, 16>([&](auto L) { issue_load(smem + a0, smem + b0, L); });
+    a_base(it, 1);
+    b_base(it, 1);
+    static_for<0, 16>([&](auto L) { issue_load(smem + a1, smem + b1, L); });
     // the remaining kernel arguments, pulled into registers now (a scalar load in flight inside the K loop would share the
     // counter of the LDS reads)
     asm volatile("" ::"s"(C), "s"(ldc), "s"(accumulate), "s"(plan.partial), "s"(plan.full), "s"(plan.nsplit), "s"(items), "s"(M), "s"(N),
                  "s"(tiles_m), "s"(tiles_n));
     if constexpr (MULTI) asm volatile("" ::"s"(seg.A1), "s"(seg.B1), "s"(seg.A2), "s"(seg.B2), "s"(seg.t1), "s"(seg.t2), "s"(seg.K1), "s"(seg.K2));
-    __builtin_amdgcn_s_waitcnt(0x4070);  // vmcnt(16) lgkmcnt(0): K tile 0 has landed, K tile 1 is still on its way
-    __syncthreads();
-    static_for<0, 16>([&](auto F) { read_frag(smem, 0, 0, F); });
+    __builtin_amdgcn_s_waitcnt(0x4070);  // vmcnt(16) lgkmcnt(0): K tile 0 has landed, what is newer is still on its way
+    wave_barrier();
+    static_for<0, 16>([&](auto F) { read_frag(smem + a0, smem + b0, 0, 0, F); });
 
     constexpr int RSTEP = 2;  // a fragment read every RSTEP MFMAs (16 reads: the first half of a phase)
-    constexpr int LSTEP = 4;  // a tile load every LSTEP MFMAs (16 loads: all of phase B)
-    auto phase_a = [&](const bf16_t* sA) {
+    constexpr int LSTEP = 4;  // a tile load every LSTEP MFMAs (8 loads: the first half of a phase)
+    auto phase_a = [&](const bf16_t* sA, const bf16_t* sB, bf16_t* lB) {
         static_for<0, 64>([&](auto S) {
             constexpr int m = decltype(S)::value, i = m >> 3, j = m & 7;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0][i], acc[i][j], 0, 0, 0);
-            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sA, 1, 1, std::integral_constant<int, m / RSTEP>{});
+            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sA, sB, 1, 1, std::integral_constant<int, m / RSTEP>{});
+            if constexpr (m % LSTEP == LSTEP - 1 && m / LSTEP < 8) issue_load(smem, lB, std::integral_constant<int, 8 + m / LSTEP>{});
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-    auto phase_b = [&](const bf16_t* sN, bf16_t* sL) {
+    auto phase_b = [&](const bf16_t* sA, const bf16_t* sB, bf16_t* lA) {
         static_for<0, 64>([&](auto S) {
             constexpr int m = decltype(S)::value, i = m >> 3, j = m & 7;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[1][i], acc[i][j], 0, 0, 0);
-            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sN, 0, 0, std::integral_constant<int, m / RSTEP>{});
-            if constexpr (m % LSTEP == LSTEP - 1) issue_load(sL, std::integral_constant<int, m / LSTEP>{});
+            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sA, sB, 0, 0, std::integral_constant<int, m / RSTEP>{});
+            if constexpr (m % LSTEP == LSTEP - 1 && m / LSTEP < 8) issue_load(lA, smem, std::integral_constant<int, m / LSTEP>{});
             __builtin_amdgcn_sched_barrier(0);
         });
     };
     auto publish = [&](auto LEFT) {  // all but this wave's LEFT newest accesses are done: the next K tile has landed; so are its LDS reads
         constexpr int left = decltype(LEFT)::value;
         __builtin_amdgcn_s_waitcnt(0x0070 | (left & 15) | ((left >> 4) << 14));
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
+        wave_barrier();
     };
-    // stores of a finished tile that are newer than the loads of the next tile's second K tile (a count holds at most 63)
-    constexpr int STORES = sizeof(OutT) == 2 ? 32 : 63;
-    typedef std::integral_constant<int, 0> none;
-    int s0 = 0, s1 = 2 * DTILE;  // stages of K tiles kt and kt + 1
+    // newer than the A tile that is waited for: the B tile behind the next, and where an item begins the stores of the one before (a count
+    // holds at most 63)
+    typedef std::integral_constant<int, 8> ahead;
+    typedef std::integral_constant<int, sizeof(OutT) == 2 ? 40 : 63> ahead_and_stores;
     auto flip = [&]() {
-        const int x = s0;
-        s0 = s1;
-        s1 = x;
-        asm volatile("" : "+s"(s0), "+s"(s1));  // (the fragment reads are restrict-qualified: a refilled stage must not look like the same address)
+        const int x = a0, y = b0;
+        a0 = a1;
+        a1 = x;
+        b0 = b1;
+        b1 = b2;
+        b2 = y;
+        asm volatile("" : "+s"(a0), "+s"(a1), "+s"(b0), "+s"(b1), "+s"(b2));  // (the fragment reads are restrict-qualified: a refilled stage must not look like the same address)
+    };
+    // the next A and B tile to bring in: K tile ta (tb) of item ia (ib)
+    Item ia = it, ib = it;
+    int ta = 2, tb = 2;
+    auto advance_a = [&](const Item& next) __attribute__((always_inline)) {
+        if (ta == ia.nk) {
+            if (min(rows_left(next), BM) != min(rows_left(ia), BM) || (LIST && a_stride(next) != a_stride(ia))) la.init(lane, wave, rows_left(next), a_stride(next));
+            ia = next;
+            ta = 0;
+        }
+        a_base(ia, ta++);
+    };
+    auto advance_b = [&](const Item& next) __attribute__((always_inline)) {
+        if (tb == ib.nk) {
+            if (min(cols_left(next), BN) != min(cols_left(ib), BN) || (LIST && b_stride(next) != b_stride(ib))) lb.init(lane, wave, cols_left(next), b_stride(next));
+            ib = next;
+            tb = 0;
+        }
+        b_base(ib, tb++);
     };
     for (bool first = true;; first = false) {
         const int next_u = u + (int)gridDim.x;
         const bool more = next_u < items;
-        const Item next = more ? item_of(next_u) : it;
+        const Item next = more ? item_of(next_u) : it;  // (behind the last item its own first tiles again, into stages nobody reads)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        phase_a(smem + s0);
-        if (first) publish(none{});
-        else publish(std::integral_constant<int, STORES>{});
-        for (int kt = 2; kt < it.nk; ++kt) {
-            tile_bases(it, kt);
-            phase_b(smem + s1, smem + s0);
-            phase_a(smem + s1);
-            publish(none{});
+        advance_b(next);
+        phase_a(smem + a0, smem + b0, smem + b2);
+        if (first) publish(ahead{});
+        else publish(ahead_and_stores{});
+        for (int left = it.nk - 1; left > 0; --left) {
+            advance_a(next);
+            phase_b(smem + a1, smem + b1, smem + a0);
+            advance_b(next);
+            phase_a(smem + a1, smem + b1, smem + b0);
+            publish(ahead{});
             flip();
         }
-        // the last two K tiles bring in the first two of the next tile (the last item's: its own again, into stages nobody reads)
-        if (min(rows_left(next), BM) != min(rows_left(it), BM) || (LIST && a_stride(next) != a_stride(it))) la.init(lane, wave, rows_left(next), a_stride(next));
-        if (min(cols_left(next), BN) != min(cols_left(it), BN) || (LIST && b_stride(next) != b_stride(it))) lb.init(lane, wave, cols_left(next), b_stride(next));
-        tile_bases(next, 0);
-        phase_b(smem + s1, smem + s0);
-        phase_a(smem + s1);
-        publish(none{});
-        flip();
-        tile_bases(next, 1);
-        phase_b(smem + s1, smem + s0);
+        advance_a(next);
+        phase_b(smem + a1, smem + b1, smem + a0);
         flip();
 #pragma unroll
         for (int i = 0; i < 8; ++i)

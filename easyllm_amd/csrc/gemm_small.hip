@@ -19,13 +19,6 @@ __device__ __forceinline__ int opaque(int x) {
     asm volatile("" : "+s"(x));
     return x;
 }
-// the loads another wave issued are visible behind it: every wave waits for its own first
-__device__ __forceinline__ void wave_barrier() {
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 // workgroup id -> (tile, part): XCD-aware, parts outermost, so that an XCD's workgroups share operand bands and K range
 __device__ __forceinline__ void tile_and_part(const GemmSmallArgs& a, int& tile, int& part) {
     const int total = a.ntiles * a.nsplit;

@@ -202,6 +202,16 @@ __device__ __forceinline__ void pick_segment(const bf16_t* A, const bf16_t* B, i
     kv = K - t * BK;
 }
 
+// A barrier that waits for nothing: what is in flight is each wave's to wait for first, by a count.  (In front of a __syncthreads the
+// compiler puts a wait for all loads that go straight to LDS, those of later K tiles included.)
+__device__ __forceinline__ void wave_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+}
+
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
     if constexpr (I < N) {
