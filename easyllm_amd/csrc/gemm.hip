@@ -26,9 +26,12 @@
 // by splitting the reduction of the tiles of that last round over several workgroups (given a workspace): each writes an
 // fp32 partial tile and a small kernel adds the partials in a fixed order, so results stay bit-reproducible.
 //
-// Products that do not fill the chip with 256 x 256 tiles run on the smaller tiles of gemm_small.hip (see choose_plan).
+// Where that leaves fewer CUs idle the 4-wave kernel runs on tiles of 192 rows; products that do not fill the chip with either run on the smaller
+// tiles of gemm_small.hip (see choose_plan).
 #include "gemm_tile.h"
 #include "gemm_list.h"
+
+#include <math.h>
 
 namespace {
 
@@ -48,9 +51,18 @@ constexpr int DTILE = 256 * 64;  // elements per operand per stage of the swizzl
 // Work split of a launch: tile ids below `full` are one workgroup each; every later
 // tile is computed by `nsplit` workgroups that each take a contiguous share of the K tiles and leave an fp32 partial tile.
 struct SplitPlan {
-    int full, nsplit;
-    float* partial;  // [tiles - full][nsplit][256 x 256]
+    int full, rest, nsplit;  // rest: tiles - full
+    float* partial;          // [rest][nsplit][tile]
 };
+// Split tile and share of workgroup-sized piece u >= full: like the whole tiles, an XCD's pieces are neighbours, all of one share where they can
+// be (product in two shares, 1531 x 4096 x 11008, tile by tile 179 us, share by share 159; x 32000 403, 384).
+__device__ __forceinline__ void split_piece(const SplitPlan& plan, int u, int& tile, int& part) {
+    u -= plan.full;
+    const int n = plan.rest * plan.nsplit, per = n >> 3, rem = n & 7, xcd = u & 7;
+    u = xcd * per + (xcd < rem ? xcd : rem) + (u >> 3);
+    part = u / plan.rest;
+    tile = u - part * plan.rest;
+}
 
 
 #define SG_MFMA 0x008
@@ -99,9 +111,8 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
         const int per = plan.full >> 3, rem = plan.full & 7, xcd = pid & 7, idx = pid >> 3;
         pid = xcd * per + (xcd < rem ? xcd : rem) + idx;
     } else {
-        const int u = pid - plan.full;
-        pid = plan.full + u / plan.nsplit;
-        part = u - (pid - plan.full) * plan.nsplit;
+        split_piece(plan, pid, pid, part);
+        pid += plan.full;
     }
     int tm, tn;
     tile_of(pid, tiles_m, tiles_n, tm, tn);
@@ -274,6 +285,7 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // loads, the stores drained before its LDS is free - which is a third of it at 32 K tiles: 4000 x 32000 x 2048 444 -> 407 us,
 // 8192 x 32000 x 1024 517 -> 460, 4096 x 11008 x 2048 143 -> 134, 8192 x 32000 x 5120 1974 -> 1947; the weight gradient 32000 x 4096 x
 // 4096 911 -> 885.  What is left there is the power limit: longer K loops run at 1.2 - 1.35 us per K tile instead of 0.96.
+// TBM = 192: six tiles of 16 rows per wave, 144 KiB, for products whose 256 x 256 tiles leave more CUs idle (see kRates).
 // C must allow 16-byte stores (N and ldc multiples of 8 for bf16, of 4 for fp32, aligned base), its tile-relative byte offsets
 // must fit 31 bits, and every item must have two K tiles or more: the host side checks.
 // LIST (forward, weight gradients): the tiles of several products over one K; what is said per product comes from the list then, not from the
@@ -281,20 +293,22 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
 // as 128 x 128 tiles in 453 us, as these in 387; its gate and up products (704 tiles) as 256 x 128 tiles in 208, as these in 155.  (One
 // product in a list of one would save the form without it, but costs 6 us a launch: a tile's scalar loads depend on one another.)
 struct NoList {};
-template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL, bool LIST = false>
+template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL, bool LIST = false, int TBM = 256>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, OutT* __restrict__ C,
                                                          int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
                                                          int tiles_m, int tiles_n, int items, const SplitPlan plan, const KSegments seg,
                                                          const std::conditional_t<LIST, GemmSmallArgs, NoList> list) {
     static_assert(!LIST || (A_KC == B_KC && !MULTI), "lists are of forward products or weight gradients");
-    __shared__ __attribute__((aligned(1024))) bf16_t smem[5 * DTILE];  // A0 A1 B0 B1 B2
+    constexpr int TM = TBM / 32, NA = TM, NB = 8;  // MFMA tiles of a wave, one below the other; wave loads of an A and a B tile
+    constexpr int ASTAGE = TBM * BK;
+    __shared__ __attribute__((aligned(1024))) bf16_t smem[2 * ASTAGE + 3 * DTILE];  // A0 A1 B0 B1 B2
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int nk_all = MULTI ? seg.nk : (K + BK - 1) / BK;
     const int64_t astep = A_KC ? BK : (int64_t)BK * lda;
     const int64_t bstep = B_KC ? BK : (int64_t)BK * ldb;
-    const int arow = wm * 128, brow = wn * 128;
+    const int arow = wm * (TBM / 2), brow = wn * 128;
 
     struct ListItem {  // its product, its operands from the tile's corner on, their strides, the tile's rows and columns
         int product, lda, ldb, mrem, nrem;
@@ -313,8 +327,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             const int per = plan.full >> 3, rem = plan.full & 7, xcd = u & 7, idx = u >> 3;
             pid = xcd * per + (xcd < rem ? xcd : rem) + idx;
         } else {
-            it.slot = u - plan.full;
-            const int t = it.slot / plan.nsplit, part = it.slot - t * plan.nsplit;
+            int t, part;
+            split_piece(plan, u, t, part);
+            it.slot = t * plan.nsplit + part;
             pid = plan.full + t;
             it.kt0 = (int)((int64_t)nk_all * part / plan.nsplit);
             it.nk = (int)((int64_t)nk_all * (part + 1) / plan.nsplit) - it.kt0;
@@ -331,7 +346,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             tile_of(pid, tiles_m, tiles_n, tm, tn);
         }
         // (scalar registers: the buffer bases are made of them)
-        it.m0 = __builtin_amdgcn_readfirstlane(tm * BM);
+        it.m0 = __builtin_amdgcn_readfirstlane(tm * TBM);
         it.n0 = __builtin_amdgcn_readfirstlane(tn * BN);
         it.kt0 = __builtin_amdgcn_readfirstlane(it.kt0);
         it.nk = __builtin_amdgcn_readfirstlane(it.nk);
@@ -344,7 +359,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             it.b = p.B + (B_KC ? it.n0 * p.ldb : it.n0);
             it.lda = (int)p.lda;
             it.ldb = (int)p.ldb;
-            it.mrem = min(p.M - it.m0, BM);
+            it.mrem = min(p.M - it.m0, TBM);
             it.nrem = min(p.N - it.n0, BN);
             // (these scalar loads are waited for here, not inside the K loop)
             asm volatile("" ::"s"(it.a), "s"(it.b), "s"(it.lda), "s"(it.ldb), "s"(it.mrem), "s"(it.nrem));
@@ -376,18 +391,18 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     int u = blockIdx.x;
     Item it = item_of(u);
 
-    TileLoader<A_KC, BM, 4, KTAIL> la;
+    TileLoader<A_KC, TBM, 4, KTAIL> la;
     TileLoader<B_KC, BN, 4, KTAIL> lb;
     la.init(lane, wave, rows_left(it), a_stride(it));
     lb.init(lane, wave, cols_left(it), b_stride(it));
 
-    FragReader<A_KC> ra;
-    FragReader<B_KC> rb;
+    FragReader<A_KC, TBM> ra;
+    FragReader<B_KC, BN> rb;
     ra.init(arow, lane);
     rb.init(brow, lane);
 
-    f32x4 acc[8][8];
-    bf16x8 fa[2][8], fb[2][8];
+    f32x4 acc[TM][8];
+    bf16x8 fa[2][TM], fb[2][8];
     // fragment f of a k half: f < 8 the B fragment f, else the A fragment f - 8
     auto read_frag = [&](const bf16_t* sA, const bf16_t* sB, int ks, int buf, auto F) {
         constexpr int f = decltype(F)::value;
@@ -418,46 +433,47 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
             gb = lb.base(Bb + x.b_blk + (int64_t)t * bstep);
         }
     };
-    // load l of a tile pair: l < 8 piece l of the A tile, else piece l - 8 of the B tile
+    // load l of a tile pair: l < NA piece l of the A tile, else of the B tile
     auto issue_load = [&](bf16_t* sA, bf16_t* sB, auto L) {
         constexpr int l = decltype(L)::value;
-        if constexpr (l < 8) la.template issue_at<l>(ga, sA, lane, wave, kva);
-        else lb.template issue_at<l - 8>(gb, sB, lane, wave, kvb);
+        if constexpr (l < NA) la.template issue_at<l>(ga, sA, lane, wave, kva);
+        else lb.template issue_at<l - NA>(gb, sB, lane, wave, kvb);
     };
 
-    int a0 = 0, a1 = DTILE, b0 = 2 * DTILE, b1 = 3 * DTILE, b2 = 4 * DTILE;  // stages of K tiles kt, kt + 1 (and kt + 2)
+    int a0 = 0, a1 = ASTAGE, b0 = 2 * ASTAGE, b1 = b0 + DTILE, b2 = b1 + DTILE;  // stages of K tiles kt, kt + 1 (and kt + 2)
     a_base(it, 0);
     b_base(it, 0);
-    static_for<0, 16>([&](auto L) { issue_load(smem + a0, smem + b0, L); });
+    static_for<0, NA + NB>([&](auto L) { issue_load(smem + a0, smem + b0, L); });
     a_base(it, 1);
     b_base(it, 1);
-    static_for<0, 16>([&](auto L) { issue_load(smem + a1, smem + b1, L); });
+    static_for<0, NA + NB>([&](auto L) { issue_load(smem + a1, smem + b1, L); });
     // the remaining kernel arguments, pulled into registers now (a scalar load in flight inside the K loop would share the
     // counter of the LDS reads)
     asm volatile("" ::"s"(C), "s"(ldc), "s"(accumulate), "s"(plan.partial), "s"(plan.full), "s"(plan.nsplit), "s"(items), "s"(M), "s"(N),
                  "s"(tiles_m), "s"(tiles_n));
     if constexpr (MULTI) asm volatile("" ::"s"(seg.A1), "s"(seg.B1), "s"(seg.A2), "s"(seg.B2), "s"(seg.t1), "s"(seg.t2), "s"(seg.K1), "s"(seg.K2));
-    __builtin_amdgcn_s_waitcnt(0x4070);  // vmcnt(16) lgkmcnt(0): K tile 0 has landed, what is newer is still on its way
+    static_assert(NA + NB <= 16, "a count's low bits, and bit 4 alone");
+    __builtin_amdgcn_s_waitcnt(NA + NB == 16 ? 0x4070 : 0x0070 | (NA + NB));  // lgkmcnt(0): K tile 0 has landed, K tile 1 is still on its way
     wave_barrier();
-    static_for<0, 16>([&](auto F) { read_frag(smem + a0, smem + b0, 0, 0, F); });
+    static_for<0, TM + 8>([&](auto F) { read_frag(smem + a0, smem + b0, 0, 0, F); });
 
-    constexpr int RSTEP = 2;  // a fragment read every RSTEP MFMAs (16 reads: the first half of a phase)
+    constexpr int RSTEP = 2;  // a fragment read every RSTEP MFMAs (of 8 x 8 MFMA tiles 16 reads: the first half of a phase)
     constexpr int LSTEP = 4;  // a tile load every LSTEP MFMAs (8 loads: the first half of a phase)
     auto phase_a = [&](const bf16_t* sA, const bf16_t* sB, bf16_t* lB) {
-        static_for<0, 64>([&](auto S) {
+        static_for<0, TM * 8>([&](auto S) {
             constexpr int m = decltype(S)::value, i = m >> 3, j = m & 7;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0][i], acc[i][j], 0, 0, 0);
-            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sA, sB, 1, 1, std::integral_constant<int, m / RSTEP>{});
-            if constexpr (m % LSTEP == LSTEP - 1 && m / LSTEP < 8) issue_load(smem, lB, std::integral_constant<int, 8 + m / LSTEP>{});
+            if constexpr (m % RSTEP == 0 && m / RSTEP < TM + 8) read_frag(sA, sB, 1, 1, std::integral_constant<int, m / RSTEP>{});
+            if constexpr (m % LSTEP == LSTEP - 1 && m / LSTEP < NB) issue_load(smem, lB, std::integral_constant<int, NA + m / LSTEP>{});
             __builtin_amdgcn_sched_barrier(0);
         });
     };
     auto phase_b = [&](const bf16_t* sA, const bf16_t* sB, bf16_t* lA) {
-        static_for<0, 64>([&](auto S) {
+        static_for<0, TM * 8>([&](auto S) {
             constexpr int m = decltype(S)::value, i = m >> 3, j = m & 7;
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[1][i], acc[i][j], 0, 0, 0);
-            if constexpr (m % RSTEP == 0 && m / RSTEP < 16) read_frag(sA, sB, 0, 0, std::integral_constant<int, m / RSTEP>{});
-            if constexpr (m % LSTEP == LSTEP - 1 && m / LSTEP < 8) issue_load(lA, smem, std::integral_constant<int, m / LSTEP>{});
+            if constexpr (m % RSTEP == 0 && m / RSTEP < TM + 8) read_frag(sA, sB, 0, 0, std::integral_constant<int, m / RSTEP>{});
+            if constexpr (m % LSTEP == LSTEP - 1 && m / LSTEP < NA) issue_load(lA, smem, std::integral_constant<int, m / LSTEP>{});
             __builtin_amdgcn_sched_barrier(0);
         });
     };
@@ -468,8 +484,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     };
     // newer than the A tile that is waited for: the B tile behind the next, and where an item begins the stores of the one before (a count
     // holds at most 63)
-    typedef std::integral_constant<int, 8> ahead;
-    typedef std::integral_constant<int, sizeof(OutT) == 2 ? 40 : 63> ahead_and_stores;
+    typedef std::integral_constant<int, NB> ahead;
+    constexpr int STORES = TM * 8 * (int)sizeof(OutT) / 4;
+    typedef std::integral_constant<int, NB + STORES <= 63 ? NB + STORES : 63> ahead_and_stores;
     auto flip = [&]() {
         const int x = a0, y = b0;
         a0 = a1;
@@ -484,7 +501,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     int ta = 2, tb = 2;
     auto advance_a = [&](const Item& next) __attribute__((always_inline)) {
         if (ta == ia.nk) {
-            if (min(rows_left(next), BM) != min(rows_left(ia), BM) || (LIST && a_stride(next) != a_stride(ia))) la.init(lane, wave, rows_left(next), a_stride(next));
+            if (min(rows_left(next), TBM) != min(rows_left(ia), TBM) || (LIST && a_stride(next) != a_stride(ia))) la.init(lane, wave, rows_left(next), a_stride(next));
             ia = next;
             ta = 0;
         }
@@ -503,7 +520,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
         const bool more = next_u < items;
         const Item next = more ? item_of(next_u) : it;  // (behind the last item its own first tiles again, into stages nobody reads)
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         advance_b(next);
@@ -522,26 +539,26 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
         phase_b(smem + a1, smem + b1, smem + a0);
         flip();
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
         int64_t ld = ldc;
         asm volatile("" : "+s"(ld));  // (the stores' offsets are not kept over the K loop)
         if (it.slot >= 0) {  // a share of the reduction, as a dense fp32 tile; gemm_split_reduce_kernel adds the shares
-            float* tile = plan.partial + (size_t)it.slot * (size_t)(BM * BN);
+            float* tile = plan.partial + (size_t)it.slot * (size_t)(TBM * BN);
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    *reinterpret_cast<f32x4*>(tile + (arow + i * 16 + (lane & 15)) * BN + brow + j * 16 + 4 * (lane >> 4)) = from_agprs<64>(acc[i][j]);
+                    *reinterpret_cast<f32x4*>(tile + (arow + i * 16 + (lane & 15)) * BN + brow + j * 16 + 4 * (lane >> 4)) = from_agprs<TM * 8>(acc[i][j]);
         } else if constexpr (LIST) {
             const GemmProblem& p = list.p[it.product];
             OutT* Ct = (OutT*)p.C + (int64_t)it.m0 * p.ldc + it.n0;
-            store_tile_flags<8, 8, OutT, true, false>(acc, Ct, p.ldc, it.mrem, it.nrem, arow, brow, lane, p.accumulate);
+            store_tile_flags<TM, 8, OutT, true, false>(acc, Ct, p.ldc, it.mrem, it.nrem, arow, brow, lane, p.accumulate);
         } else {
-            const int mrem = M - it.m0 < BM ? M - it.m0 : BM;
+            const int mrem = M - it.m0 < TBM ? M - it.m0 : TBM;
             OutT* Ct = C + (int64_t)it.m0 * ld + it.n0;
-            store_tile_flags<8, 8, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ld, mrem, N - it.n0, arow, brow, lane, accumulate);
+            store_tile_flags<TM, 8, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ld, mrem, N - it.n0, arow, brow, lane, accumulate);
         }
         if (!more) break;
         it = next;
@@ -552,20 +569,21 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
 
 // C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order.  One block per 16 rows of a tile: a thread owns 16
 // consecutive columns of one row.
-template <typename OutT>
+template <typename OutT, int TBM>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(OutT* __restrict__ C, int M, int N, int64_t ldc, int accumulate,
                                                                 int tiles_m, int tiles_n, const SplitPlan plan) {
-    const int t = blockIdx.x >> 4;  // split tile
+    constexpr int PIECES = TBM / 16;
+    const int t = blockIdx.x / PIECES;  // split tile
     int tm, tn;
     tile_of(plan.full + t, tiles_m, tiles_n, tm, tn);
-    const int rl = (blockIdx.x & 15) * 16 + (threadIdx.x >> 4), cl = (threadIdx.x & 15) * 16;
-    const int row = tm * BM + rl, col = tn * BN + cl;
+    const int rl = (blockIdx.x - t * PIECES) * 16 + (threadIdx.x >> 4), cl = (threadIdx.x & 15) * 16;
+    const int row = tm * TBM + rl, col = tn * BN + cl;
     if (row >= M || col >= N) return;
     float v[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) v[e] = 0.f;
-    const float* src = plan.partial + (size_t)t * plan.nsplit * (size_t)(BM * BN) + (size_t)rl * BN + cl;
-    for (int p = 0; p < plan.nsplit; ++p, src += BM * BN) {
+    const float* src = plan.partial + (size_t)t * plan.nsplit * (size_t)(TBM * BN) + (size_t)rl * BN + cl;
+    for (int p = 0; p < plan.nsplit; ++p, src += TBM * BN) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const f32x4 x = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src) + q);
@@ -602,63 +620,82 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(OutT* __restrict
         if (col + e < N) store_out<OutT>(dst + e, v[e], accumulate != 0);
 }
 
-// Split the tiles of a mostly empty last round?  cus workgroups run at a time (one per CU: the kernel uses 128 KiB of LDS).
+enum Class { kForward, kInputGradient, kWeightGradient };
+// Products whose operands' rows are whole cache lines (128 bytes): what the rates, the 192 x 256 tiles and the wider rule for split rounds below were
+// measured on.  Rows that straddle lines cost up to 30 % more (4096 x 4096 x 4096 from rows of 8192 + 16 bytes 139 us, + 128 bytes 107), and weight
+// gradients over up to 16 K tiles are bound by their results; both keep the rates that were fitted to all widths.
+bool whole_lines(Class cls, int64_t M, int64_t N, int64_t K) {
+    return N % 64 == 0 && (cls == kWeightGradient ? M % 64 == 0 && K > 16 * BK : K % 64 == 0);
+}
+
+// Split the tiles of a mostly empty last round?  cus workgroups run at a time (one per CU: the kernels use 128 KiB of LDS and more).
 constexpr int kCus = 256;
-SplitPlan make_plan(int64_t tiles, int64_t nk, void* workspace, int64_t workspace_bytes) {
+int64_t tile_bytes(int kind) { return gemm_kind_bm(kind) * gemm_kind_bn(kind) * (int64_t)sizeof(float); }
+SplitPlan make_plan(int kind, bool lines, int64_t tiles, int64_t nk, void* workspace, int64_t workspace_bytes) {
     SplitPlan p;
-    p.full = (int)tiles; p.nsplit = 1; p.partial = nullptr;
+    p.full = (int)tiles; p.rest = 0; p.nsplit = 1; p.partial = nullptr;
     const int64_t r = tiles % kCus;
-    // A last round that is more than 3/8 full is left alone: split two ways it measured slower (128 tiles, K = 4096: 88 against
-    // 81 us -- under the power limit a half-empty round runs at a higher clock, and the partial tiles cost a pass of their own).
-    if (r == 0 || r > 96) return p;
+    // Up to 96 tiles always: two shares and more of them.  97 - 128 are half a chip's worth, in two shares; time of them split over whole, 1400 products,
+    // by K tiles 16 - 31 1.36, 32 - 47 1.07, 48 - 63 0.93, 96 - 127 0.75, 256 - 399 0.63 (behind whole rounds 1.12, 1.03, 0.98, 0.91, 0.82).
+    if (r == 0 || r > (lines && nk >= 48 ? kCus / 2 : 96)) return p;
     int s = (int)(kCus / r);
     while (s > 1 && nk / s < 8) --s;  // a share of fewer than 8 K tiles is mostly prologue
     if (s < 2) return p;
-    if (!workspace || workspace_bytes < r * s * (int64_t)(BM * BN) * (int64_t)sizeof(float)) return p;
-    p.full = (int)(tiles - r); p.nsplit = s; p.partial = (float*)workspace;
+    if (!workspace || workspace_bytes < r * s * tile_bytes(kind)) return p;
+    p.full = (int)(tiles - r); p.rest = (int)r; p.nsplit = s; p.partial = (float*)workspace;
     return p;
+}
+int64_t split_bytes(int kind, bool lines, int64_t tiles, int64_t nk) {
+    const SplitPlan p = make_plan(kind, lines, tiles, nk, (void*)16, INT64_MAX);
+    return p.nsplit > 1 ? p.rest * p.nsplit * tile_bytes(kind) : 0;
 }
 
 // ---- which tile shape, and over how many workgroups a tile's reduction is split ------------------------------------------
-// The time of a launch is estimated for every shape as rounds x (K tiles x rate + ends) and the cheapest one taken.  The rates are us per
-// 64-wide K tile of one workgroup per CU (two sharing a CU for 128 and 64 tiles), the lower one with the chip nearly empty, the higher one full:
-// clock and L2 bandwidth give way; the ends (first load, epilogue, a workgroup's start) us per round.  Weight gradients have rates of their
-// own: both operands go through transposing LDS reads, and results are mostly fp32.  Fits to 850 products of 256 - 8192 wide operands and
-// 200 - 16384 tokens, weights not in cache, each timed with every shape and several splits: the shape that is taken is 0.2 % (weight gradients
-// 0.6 %) slower than the best one on average.  M x N x K, us for 256 x 256, 256 x 128, 192 x 128, 128 x 128:
-//   1531 x 4096 x 4096     65, 50, 44, 57         1531 x 11008 x 4096   111, 152, 129, 153      4000 x 2048 x 2048    42, 32, 43, 34
-//   1531 x 4096 x 22016   248, 249, 226, 309      4000 x 5504 x 2048     90, 90, 95, 94         4096 x 4096 x 4096    93, 114, 129, 124
-//   as weight gradients:  4096 x 4096 x 1531  52, 59, 69, 54;  11008 x 4096 x 1531  135, 164, 179, 146;  5120 x 5120 x 4096  178, 222, 227, 213
+// The time of a launch is estimated for every shape as first + rounds x (K tiles x rate + next) + out x MB of results and the cheapest one taken: us per
+// 64-wide K tile of one workgroup per CU (two sharing a CU for 128 and 64 tiles), `low` with the chip nearly empty, `high` full, in between by a
+// power of the share of it that is filled; the two ends of a round, and what the launch and its results cost.  Fits to 6000 products of 64 - 96000 wide
+// operands, 100 - 16384 rows and 2 - 1100 K tiles, weights from HBM, each timed with every shape and several splits in changing order: what is
+// taken is 1.0 % (forward, input gradients) and 0.9 % (weight gradients) slower than the fastest, and was 2.0 and 4.5 % with rates fitted to
+// products alone on the chip, out of its caches (kOtherRates; still those of rows that are not whole lines and of lists).  M x N x K, us for
+// 256 x 256 (the better of whole and split), 192 x 256, 256 x 128, 192 x 128, 128 x 128:
+//   forward          1774 x 4096 x 3584 68, 59, 51, 76, 57        1556 x 3520 x 10752 123, 111, 124, 111, 148    3664 x 2368 x 2048 45, 38, 57, 47, 54
+//   input gradient   1636 x 3840 x 30464 317, 445, 387, 483, 429  3033 x 1856 x 34432 374, 316, 456, 355, 469    4193 x 10048 x 4224 272, 277, 346, 330, 371
+//   weight gradient  4032 x 3712 x 1664 51, 69, 67, 75, 68        1856 x 2176 x 4096 64, 60, 61, 51, 51          4480 x 5760 x 4160 194, 195, 234, 237, 235
+// Without the 192 x 256 tiles the best of the others is 2.0 % slower in the mean, 3 % and more for every sixth product.  What makes the large tiles win is
+// LDS traffic: a K tile of 256 x 128 (192 x 128) takes the LDS 1152 (960) cycles of 128 bytes, written and read, and its MFMAs 1024 (768); 192 x 256
+// 1344 and 1536, 256 x 256 1536 and 2048.
 // A split reduction adds a launch and a trip of the fp32 partial tiles through the caches (2048 x 768 x 4096 as 256 x 128 tiles
 // split four ways: 26, of which 10 for that).
 struct Rates {
-    double low, high, ends;
+    double low, high, first, next, power, out;
 };
-constexpr Rates kRates[2][kGemmKinds] = {
-    {{0.72, 1.30, 8.8}, {0.57, 0.71, 6.5}, {0.54, 0.57, 5.4}, {0.69, 0.94, 3.25}, {0.275, 0.43, 2.6}, {0.187, 0.20, 3.3}},  // forward, input gradient
-    {{1.18, 1.30, 12.5}, {0.74, 0.83, 8}, {0.61, 0.695, 6}, {0.64, 0.80, 5}, {0.265, 0.45, 2.7}, {0.21, 0.218, 3.1}}};       // weight gradient
+constexpr Rates kRates[3][kGemmKinds] = {
+    {{0.904, 1.35, 5.789, 4.753, 1.329, 0.003}, {0.735, 1.058, 4.794, 3.77, 1.19, 0.011}, {0.68, 0.822, 3.52, 2.587, 2.252, 0.182}, {0.457, 0.67, 3.006, 2.612, 0.739, 0.137}, {0.56, 0.93, 2.444, 1.883, 2.136, 0.119}, {0.286, 0.405, 2.848, 0.321, 6, 0.466}, {0.096, 0.205, 2.107, 2.546, 0.3, 0.183}},
+    {{0.986, 1.397, 6.138, 4.844, 1.422, 0}, {0.824, 1.098, 5.446, 3.786, 1.472, 0.01}, {0.713, 0.833, 3.462, 2.866, 2.656, 0.187}, {0.5, 0.66, 2.704, 3.02, 0.992, 0.143}, {0.637, 0.943, 3.112, 1.208, 4.766, 0.184}, {0.307, 0.464, 2.735, 0.783, 6, 0.372}, {0.115, 0.203, 2.294, 2.438, 0.3, 0.259}},
+    {{1.088, 1.404, 7.566, 6.16, 1.4, 0.063}, {0.909, 1.098, 7.463, 3.783, 1.767, 0.087}, {0.665, 0.815, 5.6, 2.887, 0.602, 0.184}, {0.426, 0.669, 3.605, 2.771, 0.3, 0.189}, {0.553, 0.931, 2.861, 2.219, 1.454, 0.16}, {0.276, 0.457, 3.539, 0.1, 6, 0.263}, {0.148, 0.228, 2.623, 2.118, 0.3, 0.309}}};
+constexpr Rates kOtherRates[2][kGemmKinds] = {
+    {{0.72, 1.3, 0, 8.8, 1, 0}, {1e6, 1e6, 0, 0, 1, 0}, {0.57, 0.71, 0, 6.5, 3, 0}, {0.54, 0.57, 0, 5.4, 3, 0}, {0.69, 0.94, 0, 3.25, 99, 0}, {0.275, 0.43, 0, 2.6, 99, 0}, {0.187, 0.2, 0, 3.3, 3, 0}},
+    {{1.18, 1.3, 0, 12.5, 1, 0}, {1e6, 1e6, 0, 0, 1, 0}, {0.74, 0.83, 0, 8, 3, 0}, {0.61, 0.695, 0, 6, 3, 0}, {0.64, 0.8, 0, 5, 99, 0}, {0.265, 0.45, 0, 2.7, 99, 0}, {0.21, 0.218, 0, 3.1, 3, 0}}};
 constexpr double kReduceFixed = 4.0, kReduceBytesPerUs = 8e6;
 double reduce_cost(int64_t tiles, int64_t tile_elems, int64_t nsplit) {
     return kReduceFixed + (double)tiles * tile_elems * nsplit * 8 / kReduceBytesPerUs;
 }
-double cost_256(const Rates& rate, int64_t tiles, int64_t nk, bool split_ok) {
-    const SplitPlan p = make_plan(tiles, nk, split_ok ? (void*)16 : nullptr, INT64_MAX);
-    auto round = [&](int64_t groups, int64_t k) { return k * (rate.low + (rate.high - rate.low) * groups / kCus) + rate.ends; };
-    double t = (p.full / kCus) * round(kCus, nk);
+// us of a launch of `tiles` tiles, results of out_mb MB
+double cost_large(const Rates& rate, int kind, bool lines, int64_t tiles, int64_t nk, int64_t room, double out_mb) {
+    const SplitPlan p = make_plan(kind, lines, tiles, nk, (void*)16, room);
+    auto round = [&](int64_t groups, int64_t k) { return k * (rate.low + (rate.high - rate.low) * pow((double)groups / kCus, rate.power)) + rate.next; };
+    double t = rate.first + rate.out * out_mb + (p.full / kCus) * (nk * rate.high + rate.next);
     if (p.full % kCus) t += round(p.full % kCus, nk);
-    if (p.nsplit > 1) {
-        const int64_t r = tiles - p.full;
-        t += round(r * p.nsplit, (nk + p.nsplit - 1) / p.nsplit) + reduce_cost(r, BM * BN, p.nsplit);
-    }
+    if (p.nsplit > 1) t += round(p.rest * p.nsplit, (nk + p.nsplit - 1) / p.nsplit) + reduce_cost(p.rest, tile_bytes(kind) / 4, p.nsplit);
     return t;
 }
-double cost_small(const Rates& rate, int kind, int64_t tiles, int64_t nk, int64_t nsplit) {
+double cost_small(const Rates& rate, int kind, int64_t tiles, int64_t nk, int64_t nsplit, double out_mb) {
     const int64_t groups = tiles * nsplit, share = (nk + nsplit - 1) / nsplit;
     const bool two = kind == kTile128 || kind == kTile64;  // workgroups per CU
     const int64_t slots = two ? 2 * kCus : kCus, rest = groups % slots;
-    double t = (groups / slots) * (share * rate.high + rate.ends);
-    const double fill = (double)rest / kCus;  // (one workgroup per CU: the rate holds until the chip is nearly full)
-    if (rest) t += share * (two ? (rest > kCus ? rate.high : rate.low) : rate.low + (rate.high - rate.low) * fill * fill * fill) + rate.ends;
+    double t = rate.first + rate.out * out_mb + (groups / slots) * (share * rate.high + rate.next);
+    const double fill = rest < kCus ? (double)rest / kCus : 1.0;
+    if (rest) t += share * (rate.low + (rate.high - rate.low) * pow(fill, rate.power)) + rate.next;
     if (nsplit > 1) t += reduce_cost(tiles, gemm_kind_bm(kind) * gemm_kind_bn(kind), nsplit);
     return t;
 }
@@ -679,8 +716,11 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
 // 2961, 2048, 4, 5504 1288 -> 1231; 24 random layers 1.7 %, none slower.
 constexpr double kMarginList256 = 0.93;
 // `count` products over the same nk K tiles in one launch; `room`: workspace bytes.  256 x 256 tiles take one product, or with list_256 all
-GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr, bool list_256 = false) {
-    const Rates* rates = kRates[wgrad];
+GemmPlan find_plan(Class cls, bool lines, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr, bool list_256 = false) {
+    const bool wgrad = cls == kWeightGradient;
+    const Rates* rates = lines ? kRates[cls] : kOtherRates[wgrad];
+    double out_mb = 0;
+    for (int i = 0; i < count; ++i) out_mb += (double)M[i] * N[i] * (wgrad ? 4e-6 : 2e-6);
     // 128 x 128 tiles read every operand most often, which lists of weight gradients over many tokens feel: a layer's seven over 11918 tokens at
     // h = 1024 400 us (estimate 309), with 256 x 128 tiles 354 (315).
     const double list_128 = wgrad && count > 3 ? 1.05 : 1;
@@ -695,9 +735,14 @@ GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, in
         int64_t tiles = 0;
         for (int i = 0; i < count; ++i) tiles += tiles_of(kTile256, M[i], N[i]);
         if (wgrad && count == 1 && tiles >= 2 * kCus) margin = 1.08;
-        const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
-        const int64_t need = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * 4 : 0;
-        t_best = cost_256(rates[kTile256], tiles, nk, need <= room) / (list_256 ? kMarginList256 : 1);
+        t_best = cost_large(rates[kTile256], kTile256, lines, tiles, nk, room, out_mb) / (list_256 ? kMarginList256 : 1);
+    }
+    if (count == 1) {
+        const double t = cost_large(rates[kTile192x256], kTile192x256, lines, tiles_of(kTile192x256, M[0], N[0]), nk, room, out_mb);
+        if (t * margin < t_best && nk >= 2) {
+            t_best = t * margin;
+            best.kind = kTile192x256;
+        }
     }
     for (int kind = kTile256x128; kind < kGemmKinds; ++kind) {
         int64_t tiles = 0;
@@ -707,7 +752,7 @@ GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, in
             if (s > 1 && (kind == kTile64Waves || nk / s < 4 || tiles * s > 4 * kCus ||
                           tiles * s * gemm_kind_bm(kind) * gemm_kind_bn(kind) * 4 > room))
                 break;
-            const double t = cost_small(rates[kind], kind, tiles, nk, s) * (kind == kTile128 ? list_128 : 1);
+            const double t = cost_small(rates[kind], kind, tiles, nk, s, out_mb) * (kind == kTile128 ? list_128 : 1);
             if (t * margin < t_best) {
                 t_best = t * margin;
                 best.kind = kind;
@@ -719,14 +764,15 @@ GemmPlan find_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, in
     return best;
 }
 // The search takes 3 us, as long as a small product: a thread remembers its last 256 products by their sizes.
-GemmPlan choose_plan(bool wgrad, int64_t M, int64_t N, int64_t nk, int64_t room) {
+GemmPlan choose_plan(Class cls, int64_t M, int64_t N, int64_t K, int64_t room) {
+    const int64_t nk = (K + BK - 1) / BK;
     struct Entry {
-        int64_t M, N, nk, room;
+        int64_t M, N, K, room;
         GemmPlan plan;
     };
-    static thread_local Entry memo[2][256] = {};
-    Entry& e = memo[wgrad][(uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ nk * 0x165667B19E3779F9ull) >> 56];
-    if (e.M != M || e.N != N || e.nk != nk || e.room != room) e = {M, N, nk, room, find_plan(wgrad, 1, &M, &N, nk, room)};
+    static thread_local Entry memo[3][256] = {};
+    Entry& e = memo[cls][(uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ K * 0x165667B19E3779F9ull) >> 56];
+    if (e.M != M || e.N != N || e.K != K || e.room != room) e = {M, N, K, room, find_plan(cls, whole_lines(cls, M, N, K), 1, &M, &N, nk, room)};
     return e.plan;
 }
 int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const int64_t* N) {
@@ -775,12 +821,12 @@ GroupTimes group_times(bool wgrad, int count, const int64_t* M, const int64_t* N
         bool all_256 = true;
         for (int i = 0; i < count; ++i) {
             double t;
-            all_256 = find_plan(wgrad, 1, &M[i], &N[i], nk, room, &t).kind == kTile256 && all_256;
+            all_256 = gemm_kind_large(find_plan(wgrad ? kWeightGradient : kForward, false, 1, &M[i], &N[i], nk, room, &t).kind) && all_256;
             g.apart += t;
             e.M[i] = M[i];
             e.N[i] = N[i];
         }
-        g.plan = find_plan(wgrad, count, M, N, nk, room, &g.together, list_256);
+        g.plan = find_plan(wgrad ? kWeightGradient : kForward, false, count, M, N, nk, room, &g.together, list_256);
         if (all_256 && g.plan.kind != kTile256) g.together /= kMargin256;
         g.one = g.together < g.apart;
         e.K = K;
@@ -800,46 +846,46 @@ bool group_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64
 int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int64_t nk = (K + BK - 1) / BK, tiles = tiles_of(kTile256, M, N);
-    const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
-    int64_t most = p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
-    for (int wgrad = 0; wgrad < 2; ++wgrad) {
-        const GemmPlan q = choose_plan(wgrad, M, N, nk, INT64_MAX);
-        const int64_t small = q.kind == kTile256 ? 0 : small_plan_bytes(q, 1, &M, &N);
+    int64_t most = split_bytes(kTile256, false, tiles, nk);
+    for (int cls = 0; cls < 3; ++cls) {
+        const GemmPlan q = choose_plan((Class)cls, M, N, K, INT64_MAX);
+        const bool lines = whole_lines((Class)cls, M, N, K);
+        const int64_t large = split_bytes(kTile256, lines, tiles, nk);  // (also where its results have to be stored by the 8-wave kernel)
+        most = large > most ? large : most;
+        const int64_t small = gemm_kind_large(q.kind) ? split_bytes(q.kind, lines, tiles_of(q.kind, M, N), nk) : small_plan_bytes(q, 1, &M, &N);
         most = small > most ? small : most;
     }
     return most;
 }
 
-// Which 256 x 256 kernel: the 4-wave one moves a third fewer LDS bytes (the chip is bound by power on long products) and, with
-// one workgroup per CU walking over several tiles, hides a tile's first loads and its stores; the 8-wave one hides more inside a
-// single tile.  Speed of the 4-wave kernel over the 8-wave one, M x N x K:
-//   forward            one tile per CU: 4096 x 4096 x 2048 (32 K tiles) 0.95, x 4096 1.05, x 8192 1.08
-//                      several: 8192 x 32000 x 1024 (16) 1.12, 8192 x 8192 x 1536 1.10, 4000 x 32000 x 2048 1.09
-//   weight gradient    11008 x 4096 x 1024 (16) 1.08, 32000 x 4096 x 1024 1.13, 13824 x 5120 x 2048 1.04, but with the rows of B 16 KiB
-//                      (or a multiple) apart 32000 x 8192 x 1536 0.94, 28672 x 8192 x 1536 0.96
-//   input gradient     4096 x 8192 x 8192 (128) 1.01, 4096 x 28672 x 8192 0.97, 8192 x 13824 x 5120 0.95; 4096 x 4096 x 11008 (172) 1.02,
-//                      4096 x 8192 x 28672 1.04, 16384 x 4096 x 32000 1.03
-//   ... over segments  4096 x 4096 x 2 * 11008 (344) 0.97, 16384 x 4096 x 2 * 4096 0.95; 4096 x 8192 x 2 * 20480 (640) 1.03, x 2 * 28672 1.04
-// items: workgroup-sized pieces of the launch; nk: K tiles of a piece
+// Which 256 x 256 kernel: the 4-wave one moves a third fewer LDS bytes and has its operands longer on the way; the 8-wave one hides more inside a
+// tile, which shows where a launch is one round of short reductions.  Time of the 8-wave kernel over that of the 4-wave one, 17000 products of 256 - 96000 wide
+// operands, by K tiles:
+//                        2 - 7   8 - 15  16 - 31  32 - 63  64 - 127  128 - 399
+//   forward, one round   1.01    1.03    1.04     1.09     1.15      1.19          several rounds 1.13 - 1.16
+//   input gradient       0.99    0.98    0.98     1.00     1.04      1.06          1.06 - 1.15
+//   ... over pairs       0.99    0.98    0.97     0.99     1.02      1.06          1.05 - 1.15
+//   weight gradient      1.00    1.02    1.05     1.09     1.13      1.17          1.09 - 1.12
+// (forward in one round under 48 K tiles: the 256 x 256 tiles are hardly ever the choice there).  Several rounds of a weight gradient with the rows of B 16 KiB (or a
+// multiple) apart, under 48 K tiles: 32000 x 8192 x 1536 0.94, 28672 x 8192 x 1536 0.96.
+// items: workgroup-sized pieces of the launch; nk: K tiles of a piece; shares: pieces are shares of a reduction
 enum class Form { forward, weight_gradient, input_gradient, input_gradient_segments };
-bool w4_pays(Form form, int64_t nk, int64_t items, int64_t ldb) {
+bool w4_pays(Form form, int64_t nk, int64_t items, int64_t ldb, bool shares = false) {
+    const bool rounds = items > kCus;
     switch (form) {
-        case Form::forward: return nk >= 48 || (nk >= 16 && items > kCus);
-        case Form::weight_gradient: return nk >= 48 || (nk >= 16 && items > kCus && ldb % 8192 != 0);
-        case Form::input_gradient: return nk >= 160;
-        default: return nk >= 512;
+        case Form::forward: return nk >= 48 || rounds || (shares && nk >= 12);
+        case Form::weight_gradient: return nk >= 48 || (nk >= 8 && !(rounds && ldb % 8192 == 0));
+        default: return nk >= 128 || rounds || (shares && nk >= 12);
     }
 }
 // the same for a product's launch: one that is split tiles only is judged by the length of a share
-bool w4_pays(Form form, const SplitPlan& plan, int64_t tiles, int64_t nk, int64_t ldb) {
-    const int64_t items = plan.full + (tiles - plan.full) * plan.nsplit;
-    return w4_pays(form, plan.nsplit > 1 && plan.full == 0 ? nk / plan.nsplit : nk, items, ldb);
+bool w4_pays(Form form, const SplitPlan& plan, int64_t nk, int64_t ldb) {
+    const bool shares = plan.nsplit > 1 && plan.full == 0;
+    if (shares) nk /= plan.nsplit;
+    return nk >= 2 && w4_pays(form, nk, plan.full + plan.rest * plan.nsplit, ldb, shares);
 }
-// Workgroups of a 4-wave launch: one per CU, each walking over its tiles, while the K loop is short against a tile's ends; one per
-// tile on longer ones and over many rounds, where the hardware's order of dispatch keeps the workgroups that share operands together
-// (as weight gradients, one per tile against one per CU: 32000 x 5120 x 8192, 128 K tiles, 2164 us against 2314; 11008 x 4096 x
-// 4096, 64 K tiles, 291 against 283).
-dim3 w4_grid(int64_t nk, int64_t items) { return dim3((unsigned)(nk <= 64 && items > kCus && items <= 16 * kCus ? kCus : items)); }
+// Workgroups of a 4-wave launch: one per CU, each walking over its tiles (one per tile costs, by K tiles, 2 - 7 7 - 12 %, 8 - 31 3 - 8, 32 - 63 2 - 3, from 64 on 0 - 1).
+dim3 w4_grid(int64_t items) { return dim3((unsigned)(items > kCus ? kCus : items)); }
 // its stores: 16 bytes each, at 31-bit byte offsets inside a tile
 template <typename OutT>
 bool w4_stores_ok(const void* C, int64_t N, int64_t ldc) {
@@ -855,23 +901,22 @@ int64_t list_256_tiles(int count, const int64_t* M, const int64_t* N) {
 }
 bool list_256_pays(bool wgrad, int count, const int64_t* M, const int64_t* N, int64_t K) {
     const int64_t nk = (K + BK - 1) / BK, tiles = list_256_tiles(count, M, N);
-    bool pays = tiles < (1LL << 26);
+    bool pays = tiles < (1LL << 26) && (nk >= 48 || (nk >= 16 && tiles > kCus));
     for (int i = 0; i < count; ++i) pays = pays && w4_pays(wgrad ? Form::weight_gradient : Form::forward, nk, tiles, N[i]);
     return pays;
 }
 int64_t list_256_bytes(int count, const int64_t* M, const int64_t* N, int64_t K) {
     const int64_t tiles = list_256_tiles(count, M, N);
-    const SplitPlan p = make_plan(tiles, (K + BK - 1) / BK, (void*)16, INT64_MAX);
-    return p.nsplit > 1 ? (tiles - p.full) * p.nsplit * (int64_t)(BM * BN) * (int64_t)sizeof(float) : 0;
+    return split_bytes(kTile256, false, tiles, (K + BK - 1) / BK);
 }
 template <bool KC, typename OutT>
 void launch_list_256(GemmSmallArgs& a, int count, void* workspace, int64_t workspace_bytes, hipStream_t st) {
     gemm_tile_grids({kTile256, 1}, a, count);
     const int nk = (a.K + BK - 1) / BK;
-    const SplitPlan plan = make_plan(a.ntiles, nk, workspace, workspace_bytes);
-    const int items = plan.full + (a.ntiles - plan.full) * plan.nsplit;
+    const SplitPlan plan = make_plan(kTile256, false, a.ntiles, nk, workspace, workspace_bytes);
+    const int items = plan.full + plan.rest * plan.nsplit;
 #define EZL_LIST(KTAIL)                                                                                                                 \
-    hipLaunchKernelGGL((gemm_w4_kernel<KC, KC, OutT, false, KTAIL, true>), w4_grid(nk, items), dim3(256), 0, st, nullptr, nullptr,       \
+    hipLaunchKernelGGL((gemm_w4_kernel<KC, KC, OutT, false, KTAIL, true>), w4_grid(items), dim3(256), 0, st, nullptr, nullptr,       \
                        (OutT*)nullptr, 0, 0, a.K, (int64_t)0, (int64_t)0, (int64_t)0, 0, 0, 0, items, plan, KSegments(), a)
     if (a.K % BK == 0) EZL_LIST(false);
     else EZL_LIST(true);
@@ -883,28 +928,44 @@ void launch_list_256(GemmSmallArgs& a, int count, void* workspace, int64_t works
     }
 }
 
-template <bool A_KC, bool B_KC, typename OutT, bool KTAIL>
-void launch_form(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
-                 void* workspace, int64_t workspace_bytes, hipStream_t st) {
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, nk = (K + BK - 1) / BK;
-    const SplitPlan plan = make_plan((int64_t)tiles_m * tiles_n, nk, workspace, workspace_bytes);
-    const int split_tiles = tiles_m * tiles_n - plan.full;
-    const int items = plan.full + split_tiles * plan.nsplit;
-    bool w4 = false;
+// large tiles: the 4-wave kernel in either height, or the 8-wave one
+template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
+void launch_large(int kind, bool lines, const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
+                  void* workspace, int64_t workspace_bytes, const KSegments& seg, hipStream_t st) {
+    const int nk = MULTI ? seg.nk : (K + BK - 1) / BK;
     // (fp32 input gradients stay with the 8-wave kernel)
-    if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC) {
-        constexpr Form form = !A_KC ? Form::weight_gradient : (B_KC ? Form::forward : Form::input_gradient);
-        w4 = w4_pays(form, plan, (int64_t)tiles_m * tiles_n, nk, ldb) && w4_stores_ok<OutT>(C, N, ldc);
-        if (w4)
-            hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, false, KTAIL>), w4_grid(nk, items), dim3(256), 0, st, (const bf16_t*)A,
-                               (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, items, plan, KSegments(), NoList());
+    constexpr bool HAS_W4 = A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC;
+    constexpr Form form = !A_KC ? Form::weight_gradient : (B_KC ? Form::forward : (MULTI ? Form::input_gradient_segments : Form::input_gradient));
+    bool w4 = false;
+    if constexpr (HAS_W4) w4 = w4_stores_ok<OutT>(C, N, ldc);
+    constexpr bool HAS_192 = HAS_W4 && (!KTAIL || !A_KC || MULTI);  // (whole_lines: the others' reductions are whole K tiles)
+    if (!w4 || !HAS_192) kind = kTile256;
+    const int tiles_m = (int)((M + gemm_kind_bm(kind) - 1) / gemm_kind_bm(kind)), tiles_n = (N + BN - 1) / BN;
+    const SplitPlan plan = make_plan(kind, lines, (int64_t)tiles_m * tiles_n, nk, workspace, workspace_bytes);
+    const int items = plan.full + plan.rest * plan.nsplit;
+    w4 = w4 && (kind == kTile192x256 || w4_pays(form, plan, nk, ldb));
+    if constexpr (HAS_W4) {
+#define EZL_W4(TBM)                                                                                                                            \
+    hipLaunchKernelGGL((gemm_w4_kernel<A_KC, B_KC, OutT, MULTI, KTAIL, false, TBM>), w4_grid(items), dim3(256), 0, st, (const bf16_t*)A,     \
+                       (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, items, plan, seg, NoList())
+        if (w4 && kind == kTile192x256) {
+            if constexpr (HAS_192) EZL_W4(192);
+        } else if (w4) {
+            EZL_W4(256);
+        }
+#undef EZL_W4
     }
     if (!w4)
-        hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, false, KTAIL>), dim3((unsigned)items), dim3(512), 0, st, (const bf16_t*)A,
-                           (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan, KSegments());
-    if (plan.nsplit > 1)
-        hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, st, (OutT*)C, M, N, ldc,
-                           accumulate, tiles_m, tiles_n, plan);
+        hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, MULTI, KTAIL>), dim3((unsigned)items), dim3(512), 0, st, (const bf16_t*)A,
+                           (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan, seg);
+#define EZL_REDUCE(TBM)                                                                                                                    \
+    hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT, TBM>), dim3((unsigned)(plan.rest * (TBM / 16))), dim3(256), 0, st, (OutT*)C, M, N, ldc, \
+                       accumulate, tiles_m, tiles_n, plan)
+    if (plan.nsplit > 1) {
+        if (kind == kTile192x256) EZL_REDUCE(192);
+        else EZL_REDUCE(256);
+    }
+#undef EZL_REDUCE
 }
 // the smaller-tile kernels store at 31-bit byte offsets inside a tile
 template <typename OutT>
@@ -915,10 +976,14 @@ template <bool A_KC, bool B_KC, typename OutT>
 void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
             void* workspace, int64_t workspace_bytes, hipStream_t st) {
     constexpr int form = A_KC ? (B_KC ? (sizeof(OutT) == 4 ? 4 : 0) : 1) : (sizeof(OutT) == 4 ? 2 : 3);
+    constexpr Class cls = !A_KC ? kWeightGradient : (B_KC ? kForward : kInputGradient);
+    const bool lines = whole_lines(cls, M, N, K);
+    int kind = kTile256;
     if constexpr (A_KC ? B_KC || sizeof(OutT) == 2 : !B_KC) {
         if (small_stores_ok<OutT>(ldc)) {
-            const GemmPlan plan = choose_plan(!A_KC, M, N, (K + BK - 1) / BK, workspace ? workspace_bytes : 0);
-            if (plan.kind != kTile256) {
+            const GemmPlan plan = choose_plan(cls, M, N, K, workspace ? workspace_bytes : 0);
+            kind = plan.kind;
+            if (!gemm_kind_large(kind)) {
                 GemmSmallArgs a = {};
                 a.p[0] = {(const bf16_t*)A, (const bf16_t*)B, C, lda, ldb, ldc, M, N, 0, 0, 0, accumulate};
                 a.K = K;
@@ -929,9 +994,9 @@ void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t 
         }
     }
     if (K % BK == 0)
-        launch_form<A_KC, B_KC, OutT, false>(A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
+        launch_large<A_KC, B_KC, OutT, false, false>(kind, lines, A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, KSegments(), st);
     else
-        launch_form<A_KC, B_KC, OutT, true>(A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
+        launch_large<A_KC, B_KC, OutT, false, true>(kind, lines, A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, KSegments(), st);
 }
 
 // C = 0 for an empty reduction (a fill kernel rather than a memset node, so the call can be captured into a graph)
@@ -1054,11 +1119,12 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
     seg.t2 = seg.nk = seg.t1 + ktiles(1);
     if (count > 2) seg.nk += ktiles(2);
     seg.A2 = count > 2 ? (const bf16_t*)A[2] : seg.A1; seg.B2 = count > 2 ? (const bf16_t*)B[2] : seg.B1; seg.K2 = count > 2 ? (int)K[2] : 0;
-    const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
     EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
+    int kind = kTile256;
     if (small_stores_ok<bf16_t>(ldc)) {
-        const GemmPlan small = choose_plan(false, M, N, (ktot + BK - 1) / BK, workspace ? workspace_bytes : 0);
-        if (small.kind != kTile256) {
+        const GemmPlan small = choose_plan(kInputGradient, M, N, ktot, workspace ? workspace_bytes : 0);
+        kind = small.kind;
+        if (!gemm_kind_large(kind)) {
             GemmSmallArgs a = {};
             a.p[0] = {(const bf16_t*)A[0], (const bf16_t*)B[0], C, lda, ldb, ldc, (int)M, (int)N, 0, 0, 0, accumulate};
             a.K = (int)K[0];
@@ -1069,27 +1135,8 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
             return EZL_OK;
         }
     }
-    const SplitPlan plan = make_plan(tiles, (ktot + BK - 1) / BK, workspace, workspace_bytes);
-    const int split_tiles = (int)tiles - plan.full;
-    const int items = plan.full + split_tiles * plan.nsplit;
-    const bool w4 = w4_pays(Form::input_gradient_segments, plan, tiles, seg.nk, ldb) && w4_stores_ok<bf16_t>(C, N, ldc);
-#define EZL_MULTI(KT)                                                                                                                        \
-    do {                                                                                                                                     \
-        if (w4)                                                                                                                              \
-            hipLaunchKernelGGL((gemm_w4_kernel<true, false, bf16_t, true, KT>), w4_grid(seg.nk, items), dim3(256), 0, (hipStream_t)stream,    \
-                               (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate,    \
-                               tiles_m, tiles_n, items, plan, seg, NoList());                                                                          \
-        else                                                                                                                                 \
-            hipLaunchKernelGGL((gemm_d2l_kernel<true, false, bf16_t, true, KT>), dim3((unsigned)items), dim3(512), 0, (hipStream_t)stream,   \
-                               (const bf16_t*)A[0], (const bf16_t*)B[0], (bf16_t*)C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate,    \
-                               tiles_m, tiles_n, plan, seg);                                                                                 \
-    } while (0)
-    if (tail) EZL_MULTI(true);
-    else EZL_MULTI(false);
-#undef EZL_MULTI
-    if (plan.nsplit > 1)
-        hipLaunchKernelGGL((gemm_split_reduce_kernel<bf16_t>), dim3((unsigned)(split_tiles * 16)), dim3(256), 0, (hipStream_t)stream,
-                           (bf16_t*)C, (int)M, (int)N, ldc, accumulate, tiles_m, tiles_n, plan);
+    (tail ? launch_large<true, false, bf16_t, true, true> : launch_large<true, false, bf16_t, true, false>)(
+        kind, whole_lines(kInputGradient, M, N, ktot), A[0], B[0], C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate, workspace, workspace_bytes, seg, (hipStream_t)stream);
     EZL_LAUNCH_CHECK("ezl_gemm_bf16_ksplit");
     return EZL_OK;
 }
@@ -1196,7 +1243,7 @@ int gemm_list(int count, const void* const* A, const void* const* B, void* const
         return EZL_OK;
     }
     if (small_plan_bytes(plan, count, M, N) > (workspace ? workspace_bytes : 0)) group_plan(!a_kc, count, M, N, K, 0, plan);
-    if (plan.kind == kTile256) plan = {kTile256x128, 1};  // (a group of one: these kernels take one or more)
+    if (gemm_kind_large(plan.kind)) plan = {kTile256x128, 1};  // (a group of one: these kernels take one or more)
     a.partial = (float*)workspace;
     const int form = a_kc ? (b_kc ? 0 : 1) : (out_dtype == 1 ? 2 : 3);
     gemm_small_launch(form, false, plan, a, count, (hipStream_t)stream);
@@ -1210,12 +1257,13 @@ extern "C" int ezl_gemm_plan(int form, int count, const int64_t* M, const int64_
     for (int i = 0; i < count; ++i)
         if (M[i] <= 0 || N[i] <= 0 || M[i] >= (1LL << 31) || N[i] >= (1LL << 31)) return -1;
     const bool wgrad = form == 1;
+    const Class cls = wgrad ? kWeightGradient : (form == 0 ? kForward : kInputGradient);
     const Form forms[4] = {Form::forward, Form::weight_gradient, Form::input_gradient, Form::input_gradient_segments};
     const int64_t nk = (K + BK - 1) / BK;
     GemmPlan plan;
     bool one = true;
     if (count == 1) {
-        plan = choose_plan(wgrad, M[0], N[0], nk, INT64_MAX);
+        plan = choose_plan(cls, M[0], N[0], K, INT64_MAX);
     } else {
         one = group_plan(wgrad, count, M, N, K, INT64_MAX, plan, (!wgrad || count > kGroupMax) && list_256_pays(wgrad, count, M, N, K));
     }
@@ -1223,11 +1271,11 @@ extern "C" int ezl_gemm_plan(int form, int count, const int64_t* M, const int64_
     *cols = kKindCols[plan.kind];
     *split = plan.nsplit;
     *waves = plan.kind == kTile64Waves ? 8 : 4;
-    if (plan.kind == kTile256) {
-        const int64_t tiles = list_256_tiles(count, M, N);
-        const SplitPlan p = make_plan(tiles, nk, (void*)16, INT64_MAX);
+    if (gemm_kind_large(plan.kind)) {
+        const int64_t tiles = count == 1 ? tiles_of(plan.kind, M[0], N[0]) : list_256_tiles(count, M, N);
+        const SplitPlan p = make_plan(plan.kind, count == 1 && whole_lines(cls, M[0], N[0], K), tiles, nk, (void*)16, INT64_MAX);
         *split = p.nsplit;
-        if (count == 1) *waves = w4_pays(forms[form], p, tiles, nk, form == 0 ? K : N[0]) ? 4 : 8;
+        if (count == 1 && plan.kind == kTile256) *waves = w4_pays(forms[form], p, nk, form == 0 ? K : N[0]) ? 4 : 8;
     }
     return one;
 }

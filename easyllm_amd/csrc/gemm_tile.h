@@ -147,13 +147,13 @@ __device__ __forceinline__ bf16x8 sfrag(const bf16_t* __restrict__ s, int row0, 
     }
 }
 
-// The eight fragments of a wave's 128 rows (columns) in a 256-wide tile.  What a fragment's address is made of per lane is computed once and hidden
+// The fragments of a wave's half of a tile's rows (columns), R in all.  What a fragment's address is made of per lane is computed once and hidden
 // from the compiler, which otherwise rebuilds it per read in a loop over stages (48 vector instructions per K tile of the 4-wave
 // kernel, 5 % of its time); the rest is the read's immediate offset.
-template <bool KC>
+template <bool KC, int R>
 struct FragReader {
-    static constexpr int R = 256;
-    int off[KC ? 2 : 8];  // elements: k-contiguous per k half, k-major per fragment (its chunk permutation mixes with the fragment's index)
+    static constexpr int NF = R / 32;
+    int off[KC ? 2 : NF];  // elements: k-contiguous per k half, k-major per fragment (its chunk permutation mixes with the fragment's index)
     __device__ __forceinline__ void init(int row0, int lane) {
         if constexpr (KC) {
             const int row = row0 + (lane & 15);
@@ -162,7 +162,7 @@ struct FragReader {
         } else {
             const int krow = (lane >> 4) * 8 + ((lane & 15) >> 2);
 #pragma unroll
-            for (int f = 0; f < 8; ++f) {
+            for (int f = 0; f < NF; ++f) {
                 const int col = row0 + f * 16 + ((lane & 3) << 2);
                 off[f] = krow * R + ((col >> 3) ^ kmajor_swizzle<R>(krow)) * 8 + (col & 7);
             }
@@ -220,11 +220,11 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-// Tiles of 64 accumulators are the 4-wave kernel's, which take all AGPRs: they are copied out here, row by row (with a
+// Tiles of 48 accumulators and more are the 4-wave kernel's, which lie in AGPRs: they are copied out here, row by row (with a
 // scheduling barrier behind each).  Copied any earlier, behind their MFMA or all of them before the first store, they spill.
 template <int ACCUMULATORS>
 __device__ __forceinline__ f32x4 from_agprs(f32x4 x) {
-    if constexpr (ACCUMULATORS >= 64) asm volatile("" : "+a"(x));
+    if constexpr (ACCUMULATORS >= 48) asm volatile("" : "+a"(x));
     return x;
 }
 
@@ -299,7 +299,7 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
                 }
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, offset(jp) + i * row_step, 0, 0);
             }
-            if constexpr (TM * TN >= 64) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (TM * TN >= 48) __builtin_amdgcn_sched_barrier(0);
         }
     } else {
         const auto offset = [&](int j) {
@@ -329,7 +329,7 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
                 }
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), cbuf, offset(j) + i * row_step, 0, 0);
             }
-            if constexpr (TM * TN >= 64) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (TM * TN >= 48) __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
@@ -367,9 +367,10 @@ struct GemmSmallArgs {
     KSegments seg;
 };
 
-// Tile shapes of gemm_small.hip, and 0 for the 256 x 256 kernels of gemm.hip.
-enum GemmKind { kTile256 = 0, kTile256x128, kTile192x128, kTile128, kTile64, kTile64Waves, kGemmKinds };
-constexpr int kKindRows[kGemmKinds] = {256, 256, 192, 128, 64, 64}, kKindCols[kGemmKinds] = {256, 128, 128, 128, 64, 64};
+// Tile shapes: the first two of gemm.hip, the others of gemm_small.hip.
+enum GemmKind { kTile256 = 0, kTile192x256, kTile256x128, kTile192x128, kTile128, kTile64, kTile64Waves, kGemmKinds };
+constexpr int kKindRows[kGemmKinds] = {256, 192, 256, 192, 128, 64, 64}, kKindCols[kGemmKinds] = {256, 256, 128, 128, 128, 64, 64};
+inline bool gemm_kind_large(int kind) { return kind <= kTile192x256; }
 struct GemmPlan {
     int kind, nsplit;
 };

@@ -1,0 +1,60 @@
+"""Products on 192 x 256 tiles, short reductions on the 4-wave kernel and half a chip's worth of tiles in two shares, each against fp32."""
+import pytest
+import torch
+
+from easyllm_amd import _lib
+from test_kernel_edges_gpu import K, check_gemm, gemm_bound, products, rnd  # noqa: F401
+
+FORMS = ("forward", "input gradient", "weight gradient", "weight gradient")
+# (form, M, N, K) by (tile rows, columns, waves, shares of a reduction in the last round); forms as in check_gemm
+TILES = {
+    # two and more K tiles, ragged rows, one round and several
+    (192, 256, 4, 1): [(0, 2100, 4096, 128), (0, 6000, 3072, 128), (1, 1531, 6144, 128), (0, 3664, 2368, 2048), (0, 2303, 8192, 128), (2, 3008, 3072, 1105),
+                       (2, 3008, 6144, 1169), (3, 2304, 4096, 1105)],
+    # the last round's tiles in shares, with a K tail
+    (192, 256, 4, 5): [(0, 700, 3072, 8192), (1, 2100, 1024, 8192), (2, 1536, 1536, 9233), (3, 768, 3072, 9233)],
+    (192, 256, 4, 2): [(0, 1500, 4096, 11008), (1, 1531, 4096, 11008)],
+    # half the chip in two shares; one round of a short weight gradient
+    (256, 256, 4, 2): [(1, 4000, 2048, 32000), (0, 2048, 4096, 20032)],
+    (256, 256, 4, 1): [(2, 4096, 4096, 1531), (3, 4096, 4096, 1100)]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("want,case", [(w, c) for w, cs in TILES.items() for c in cs])
+def test_products_on_large_tiles(K, want, case):  # noqa: F811
+    print("gemm", want, case, flush=True)
+    form, M, N, Kd = case
+    check_gemm(K, form, M, N, Kd)
+    check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
+    if form == 0:  # bf16 values in fp32: the same sums, rounded the same way
+        x, w = rnd(M, Kd, seed=1), rnd(N, Kd, seed=2)
+        assert torch.equal(K.linear_fwd(x, w, fp32_output=True), K.linear_fwd(x, w).float())
+
+
+@pytest.mark.parametrize("want,case", [(w, c) for w, cs in TILES.items() for c in cs])
+def test_products_take_the_large_tiles_they_are_listed_under(want, case):
+    form, M, N, Kd = case
+    _, rows, cols, split, waves = _lib.gemm_plan(FORMS[form], [M], [N], Kd)
+    assert (rows, cols, waves, split) == want
+
+
+PAIRS = [(1531, 4096, (5504, 5504)), (2100, 4096, (72, 56)), (1531, 4096, (4096, 3464, 3448))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n_in,outs", PAIRS)
+def test_input_gradient_over_pairs_on_large_tiles(K, T, n_in, outs):  # noqa: F811
+    """Whole K tiles, and K tails inside the reduction."""
+    print("dgrad multi", T, n_in, outs, flush=True)
+    ld = max(outs)
+    dys = [torch.empty(T, ld, device="cuda", dtype=torch.bfloat16)[:, :o].copy_(rnd(T, o, seed=i)) for i, o in enumerate(outs)]
+    ws = [rnd(o, n_in, seed=10 + i) for i, o in enumerate(outs)]
+    A, B = torch.cat([d.contiguous() for d in dys], 1), torch.cat(ws, 0)
+    ref = A.float() @ B.float()
+    dx = K.linear_dgrad_multi(dys, ws)
+    assert ((dx.float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
+
+
+@pytest.mark.parametrize("T,n_in,outs", PAIRS)
+def test_pairs_take_the_large_tiles(T, n_in, outs):
+    assert _lib.gemm_plan("input gradient over pairs", [T], [n_in], sum(outs))[1:3] == (192, 256)
