@@ -34,6 +34,8 @@ SIGNATURES = {
     "ezl_rmsnorm_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp],
     "ezl_rmsnorm_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp],
     "ezl_rmsnorm_bwd_noalloc": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _vp],
+    "ezl_rmsnorm_fwd_swapped": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp],
+    "ezl_rmsnorm_bwd_swapped": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _vp],
     "ezl_swiglu_fwd": [_vp, _vp, _vp, _i64, _vp],
     "ezl_swiglu_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "ezl_rope_table": [_vp, _vp, _vp, _i64, _i64, _f32, _vp],
@@ -45,6 +47,8 @@ SIGNATURES = {
     "ezl_embed_gather_host_flag": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "ezl_embed_scatter_add": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "ezl_embed_grad_bf16": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
+    "ezl_embed_gather_swapped": [_vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _vp],
+    "ezl_embed_grad_swapped": [_vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp],
     "ezl_transpose01": [_vp, _vp, _i64, _i64, _i64, _vp],
     "ezl_add": [_vp, _vp, _vp, _i64, _vp],
     "ezl_cast_bf16_to_f32": [_vp, _vp, _i64, _vp],

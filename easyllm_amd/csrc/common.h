@@ -88,6 +88,14 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// Rows that lie in memory in the other order of their two indices: row r of [d0, d1] is row (r % d1) * d0 + r / d1 there.  d1 = 0: as they are.
+struct RowSwap {
+    int d0, d1;
+};
+__device__ __forceinline__ int swapped_row(int r, const RowSwap& s) {
+    return s.d1 ? (int)((unsigned)r % (unsigned)s.d1 * (unsigned)s.d0 + (unsigned)r / (unsigned)s.d1) : r;
+}
+
 // out[col] (+)= sum_r partial[r][col];  64 columns per block, 16 row groups (loads of a group issued eight at a time)
 // folded through LDS in a fixed order.
 constexpr int kColsumThreads = 1024;

@@ -162,7 +162,8 @@ __global__ __launch_bounds__(kBlock) void ids_in_range_kernel(const int64_t* __r
 // first store.
 template <bool HOST>
 __global__ __launch_bounds__(kBlock) void embed_gather_kernel(const int64_t* __restrict__ ids, const bf16_t* __restrict__ W,
-                                                              bf16_t* __restrict__ out, int64_t rows, int h, int64_t V, void* bad_flag) {
+                                                              bf16_t* __restrict__ out, int64_t rows, int h, int64_t V, void* bad_flag,
+                                                              const RowSwap swap) {
     const int h8 = h >> 3;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int64_t r = (int64_t)blockIdx.x * 4 + wave; r < rows; r += (int64_t)gridDim.x * 4) {
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(kBlock) void embed_gather_kernel(const int64_t* __r
         const bool ok = id >= 0 && id < V;
         if (!ok && lane == 0) raise_id_flag<HOST>(bad_flag, id >= V ? 1 : 2);
         const bf16_t* src = W + (ok ? id : 0) * h;
-        bf16_t* dst = out + r * h;
+        bf16_t* dst = out + (swap.d1 ? (int64_t)swapped_row((int)r, swap) : r) * h;
         for (int c0 = lane; c0 < h8; c0 += 512) {
             bf16x8 v[8];
 #pragma unroll
@@ -391,7 +392,7 @@ struct EmbedOrder {
 // 334, 3473, 340 us; 300 times 474, 1043, 310; 3000 times 3335, 922, 636; T = 16384, ids by Zipf's law 950, 164, 148.
 template <typename OutT>
 __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY, OutT* __restrict__ dW, const int* __restrict__ mine, int n,
-                                                  int64_t id, int col0, int64_t rows, int h, int overwrite, EmbedOrder& o) {
+                                                  int64_t id, int col0, int64_t rows, int h, int overwrite, EmbedOrder& o, const RowSwap& swap) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int col = col0 + 2 * tid;
     const bool live = col < h;
@@ -409,7 +410,7 @@ __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY,
             __syncthreads();
             int rank = 0;
             for (int j = 0; j < n; ++j) rank += o.raw[j] < v;
-            if (tid < n) o.list[rank] = v;
+            if (tid < n) o.list[rank] = swapped_row(v, swap);
             m = n;
         } else {
             for (int i = tid; i < words; i += kBlock) o.bits[i] = 0u;
@@ -448,7 +449,7 @@ __device__ __forceinline__ void embed_frequent_id(const bf16_t* __restrict__ dY,
                         continue;
                     }
                     for (; w; w &= w - 1, ++q)
-                        if (q >= 0 && q < kListRows) o.list[q] = (int)w0 + 32 * i + __builtin_ctz(w);
+                        if (q >= 0 && q < kListRows) o.list[q] = swapped_row((int)w0 + 32 * i + __builtin_ctz(w), swap);
                 }
             }
             __syncthreads();
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
                                                                       const int* __restrict__ first, const int* __restrict__ off,
                                                                       const int* __restrict__ bucket, const int* __restrict__ cursor,
                                                                       const int* __restrict__ heavy, int64_t rows, int h, int64_t V,
-                                                                      int overwrite) {
+                                                                      int overwrite, const RowSwap swap) {
     __shared__ EmbedOrder order;
     int *const raw = order.raw, *const sorted = order.list;  // rows of the current id as they are found, and in increasing order
     const int h8 = h >> 3;
@@ -514,7 +515,7 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
         const int slices = (h + 2 * kBlock - 1) / (2 * kBlock), items = cursor[1] * slices;
         for (int it = blockIdx.x; it < items; it += helpers) {
             const int id = heavy[it / slices];
-            embed_frequent_id(dY, dW, bucket + off[id], cnt[id], id, (it % slices) * 2 * kBlock, rows, h, overwrite, order);
+            embed_frequent_id(dY, dW, bucket + off[id], cnt[id], id, (it % slices) * 2 * kBlock, rows, h, overwrite, order, swap);
         }
         __syncthreads();
     }
@@ -570,7 +571,7 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
             for (; i < m; ++i) add_row(lst[i]);
         };
         if (n == 1) {
-            add_row(t);
+            add_row(swapped_row((int)t, swap));
         } else {
             __syncthreads();  // the previous id's LDS use is over
             if ((int)threadIdx.x < n) raw[threadIdx.x] = mine[threadIdx.x];
@@ -579,7 +580,7 @@ __global__ __launch_bounds__(kBlock, MAXC == 2 ? 6 : 1) void embed_scatter_bucke
                 const int v = raw[threadIdx.x];
                 int rank = 0;
                 for (int j = 0; j < n; ++j) rank += raw[j] < v;
-                sorted[rank] = v;
+                sorted[rank] = swapped_row(v, swap);
             }
             __syncthreads();
             add_rows(sorted, n);
@@ -965,14 +966,14 @@ int launch_ids_in_range(const char* name, const void* ids, int64_t n, int64_t li
 
 template <bool HOST>
 int launch_embed_gather(const char* name, const void* ids, const void* weight, void* out, void* bad_flag, int64_t rows, int64_t h,
-                        int64_t vocab, void* stream) {
+                        int64_t vocab, void* stream, const RowSwap& swap = RowSwap{0, 0}) {
     EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h < (1LL << 31) && vocab > 0, EZL_EUNSUPPORTED,
                 "%s: h must be a multiple of 8", name);
     EZL_REQUIRE(bad_flag && (rows == 0 || (ids && weight && out)) && ezl_aligned16(weight) && ezl_aligned16(out), EZL_EINVAL,
                 "%s: null or misaligned pointer", name);
     if (rows == 0) return EZL_OK;
     hipLaunchKernelGGL((embed_gather_kernel<HOST>), dim3(grid_for((rows + 3) / 4, 1)), dim3(kBlock), 0, (hipStream_t)stream,
-                       (const int64_t*)ids, (const bf16_t*)weight, (bf16_t*)out, rows, (int)h, vocab, bad_flag);
+                       (const int64_t*)ids, (const bf16_t*)weight, (bf16_t*)out, rows, (int)h, vocab, bad_flag, swap);
     EZL_LAUNCH_CHECK(name);
     return EZL_OK;
 }
@@ -997,6 +998,23 @@ extern "C" int ezl_embed_gather_host_flag(const void* ids, const void* weight, v
     return launch_embed_gather<true>("ezl_embed_gather_host_flag", ids, weight, out, host_flag, rows, h, vocab, stream);
 }
 
+namespace {
+int embed_swap_check(const char* name, int64_t d0, int64_t d1) {
+    EZL_REQUIRE(d0 > 0 && d1 > 0 && d0 < (1LL << 31) && d1 < (1LL << 31) && d0 * d1 < (1LL << 31), EZL_EUNSUPPORTED, "%s: need 0 < d0 * d1 < 2^31",
+                name);
+    return EZL_OK;
+}
+}  // namespace
+
+extern "C" int ezl_embed_gather_swapped(const void* ids, const void* weight, void* out, void* bad_flag, int host_flag, int64_t d0, int64_t d1,
+                                        int64_t h, int64_t vocab, void* stream) {
+    const char* name = "ezl_embed_gather_swapped";
+    if (const int rc = embed_swap_check(name, d0, d1)) return rc;
+    const RowSwap swap{(int)d0, (int)d1};
+    return host_flag ? launch_embed_gather<true>(name, ids, weight, out, bad_flag, d0 * d1, h, vocab, stream, swap)
+                     : launch_embed_gather<false>(name, ids, weight, out, bad_flag, d0 * d1, h, vocab, stream, swap);
+}
+
 extern "C" int64_t ezl_embed_scatter_add_workspace_bytes(int64_t rows, int64_t vocab) {
     if (rows < 0 || vocab <= 0) return -1;
     return (4 * vocab + rows + 4 + embed_heavy_max(rows)) * (int64_t)sizeof(int);
@@ -1005,7 +1023,7 @@ extern "C" int64_t ezl_embed_scatter_add_workspace_bytes(int64_t rows, int64_t v
 namespace {
 template <typename OutT>
 int embed_gradient(const char* name, const void* ids, const void* dy, void* dweight, void* workspace, int64_t workspace_bytes, int64_t rows,
-                   int64_t h, int64_t vocab, int accumulate, void* stream) {
+                   int64_t h, int64_t vocab, int accumulate, void* stream, const RowSwap& swap = RowSwap{0, 0}) {
     EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h < (1LL << 31) && vocab > 0, EZL_EUNSUPPORTED,
                 "%s: h must be a multiple of 8", name);
     EZL_REQUIRE((rows == 0 || (ids && dy && dweight)) && ezl_aligned16(dy), EZL_EINVAL,
@@ -1052,13 +1070,13 @@ int embed_gradient(const char* name, const void* ids, const void* dy, void* dwei
     const dim3 grid(grid_for(overwrite ? (rows > vocab ? rows : vocab) : rows, 1));
     if (h <= 8 * kBlock * 2)
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<2, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
+                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite, swap);
     else if (h <= 8 * kBlock * 4)
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<4, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
+                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite, swap);
     else
         hipLaunchKernelGGL((embed_scatter_bucket_kernel<8, OutT>), grid, dim3(kBlock), 0, st, (const int64_t*)ids, (const bf16_t*)dy,
-                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite);
+                           (OutT*)dweight, cnt, first, off, bucket, cursor, heavy, rows, (int)h, vocab, overwrite, swap);
     EZL_LAUNCH_CHECK(name);
     return EZL_OK;
 }
@@ -1072,6 +1090,16 @@ extern "C" int ezl_embed_scatter_add(const void* ids, const void* dy, void* dwei
 extern "C" int ezl_embed_grad_bf16(const void* ids, const void* dy, void* dweight_bf16, void* workspace, int64_t workspace_bytes,
                                    int64_t rows, int64_t h, int64_t vocab, void* stream) {
     return embed_gradient<bf16_t>("ezl_embed_grad_bf16", ids, dy, dweight_bf16, workspace, workspace_bytes, rows, h, vocab, 0, stream);
+}
+
+extern "C" int ezl_embed_grad_swapped(const void* ids, const void* dy, void* dweight, int fp32, void* workspace, int64_t workspace_bytes, int64_t d0,
+                                      int64_t d1, int64_t h, int64_t vocab, int accumulate, void* stream) {
+    const char* name = "ezl_embed_grad_swapped";
+    if (const int rc = embed_swap_check(name, d0, d1)) return rc;
+    EZL_REQUIRE(fp32 || !accumulate, EZL_EUNSUPPORTED, "%s: a bf16 gradient is overwritten", name);
+    const RowSwap swap{(int)d0, (int)d1};
+    return fp32 ? embed_gradient<float>(name, ids, dy, dweight, workspace, workspace_bytes, d0 * d1, h, vocab, accumulate, stream, swap)
+                : embed_gradient<bf16_t>(name, ids, dy, dweight, workspace, workspace_bytes, d0 * d1, h, vocab, 0, stream, swap);
 }
 
 extern "C" int ezl_transpose01(const void* x, void* y, int64_t d0, int64_t d1, int64_t inner, void* stream) {

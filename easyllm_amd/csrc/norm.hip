@@ -19,7 +19,7 @@ template <int NCHUNK, bool HAS_RES>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                           const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
                                                           bf16_t* __restrict__ sum_out, float* __restrict__ rstd_out,
-                                                          int T, int h, float eps, int tpr) {
+                                                          int T, int h, float eps, int tpr, const RowSwap swap) {
     __shared__ float red[2][4][4];  // [parity][row slot][wave in slot]
     const int rpb = 256 / tpr;             // row slots per block
     const int slot = threadIdx.x / tpr;    // which row slot
@@ -38,14 +38,14 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
     for (int row0 = blockIdx.x * rpb; row0 < T; row0 += gridDim.x * rpb) {
         const int row = row0 + slot;
         const bool live = row < T;
-        const size_t base = (size_t)row * h;
+        const size_t base = (size_t)row * h, xbase = HAS_RES ? base : (size_t)swapped_row(row, swap) * h;
         float xv[NCHUNK][8];
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < NCHUNK; ++c) {
             const int col = (c * tpr + tin) * 8;
             if (live && col < h) {
-                unpack8(ld_bf16x8(x + base + col), xv[c]);
+                unpack8(ld_bf16x8(x + xbase + col), xv[c]);
                 if (HAS_RES) {
                     float r[8];
                     unpack8(ld_bf16x8(res + base + col), r);
@@ -93,7 +93,7 @@ template <int NCHUNK, bool HAS_DRES, bool STREAM>
 __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x,
                                                                const bf16_t* __restrict__ w, const float* __restrict__ rstd,
                                                                const bf16_t* __restrict__ dres, bf16_t* __restrict__ dx,
-                                                               float* __restrict__ dw_partial, int T, int h) {
+                                                               float* __restrict__ dw_partial, int T, int h, const RowSwap swap) {
     extern __shared__ float fold[];  // h floats
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     bf16x8 wr[NCHUNK];
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __r
     }
     const float inv_h = 1.0f / (float)h;
     for (int row = blockIdx.x * 8 + wave; row < T; row += gridDim.x * 8) {
-        const size_t base = (size_t)row * h;
+        const size_t base = (size_t)row * h, xbase = HAS_DRES ? base : (size_t)swapped_row(row, swap) * h;
         const float rs = rstd[row];
         bf16x8 xr[NCHUNK], dyr[NCHUNK], drr[NCHUNK];
 #pragma unroll
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __r
 #pragma unroll
             for (int i = 0; i < 8; ++i) { xr[c][i] = (bf16_t)0.0f; dyr[c][i] = (bf16_t)0.0f; }
             if (col < h) {
-                xr[c] = ld_bf16x8_nt(x + base + col);
+                xr[c] = ld_bf16x8_nt(x + xbase + col);
                 dyr[c] = ld_bf16x8_nt(dy + base + col);
                 if (HAS_DRES) drr[c] = ld_bf16x8_nt(dres + base + col);
             }
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_wave_kernel(const bf16_t* __r
                     if (HAS_DRES) o[i] += (float)drr[c][i];
                     dwacc[c][i] += dyv * xhat;
                 }
-                st_result<STREAM>(dx + base + col, pack8(o));
+                st_result<STREAM>(dx + xbase + col, pack8(o));
             }
         }
     }
@@ -178,7 +178,7 @@ template <int NCHUNK, int NSPLIT, bool HAS_DRES, bool STREAM>
 __global__ __launch_bounds__(256, 2) void rmsnorm_bwd_split_kernel(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x,
                                                                    const bf16_t* __restrict__ w, const float* __restrict__ rstd,
                                                                    const bf16_t* __restrict__ dres, bf16_t* __restrict__ dx,
-                                                                   float* __restrict__ dw_partial, int T, int h) {
+                                                                   float* __restrict__ dw_partial, int T, int h, const RowSwap swap) {
     constexpr int RPB = 4 / NSPLIT;  // rows per block pass
     extern __shared__ float fold[];  // h floats
     __shared__ float cell[2][RPB][NSPLIT];  // [parity][row slot][part]
@@ -201,13 +201,14 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_bwd_split_kernel(const bf16_t*
     float nrs = 0.f;
     auto fetch = [&](int row) {  // the operands of this wave's share of `row` into the next-row registers
         const bool live = row < T;
+        const bf16_t* xrow = x + (size_t)(HAS_DRES ? row : swapped_row(row, swap)) * h + col0;
         nrs = live ? rstd[row] : 0.f;
 #pragma unroll
         for (int c = 0; c < NCHUNK; ++c) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) { nxr[c][i] = (bf16_t)0.0f; ndyr[c][i] = (bf16_t)0.0f; }
             if (live && col0 + c * 512 < h) {
-                nxr[c] = ld_bf16x8_nt(x + (size_t)row * h + col0 + c * 512);
+                nxr[c] = ld_bf16x8_nt(xrow + c * 512);
                 ndyr[c] = ld_bf16x8_nt(dy + (size_t)row * h + col0 + c * 512);
                 if (HAS_DRES) ndrr[c] = ld_bf16x8_nt(dres + (size_t)row * h + col0 + c * 512);
             }
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_bwd_split_kernel(const bf16_t*
         for (int q = 1; q < NSPLIT; ++q) rowdot += cell[parity][slot][q];
         const float cmean = rowdot * inv_h;
         parity ^= 1;
-        bf16_t* dxrow = dx + (size_t)row * h + col0;
+        bf16_t* dxrow = dx + (size_t)(HAS_DRES ? row : swapped_row(row, swap)) * h + col0;
 #pragma unroll
         for (int c = 0; c < NCHUNK; ++c) {
             asm volatile("" : "+v"(xr[c]), "+v"(dyr[c]));  // do not keep the fp32 copies of the dot product alive
@@ -392,10 +393,8 @@ int tpr_for(int h) {
     return t < 64 ? 64 : (t > 256 ? 256 : t);
 }
 
-}  // namespace
-
-extern "C" int ezl_rmsnorm_fwd(const void* x, const void* residual, const void* weight, void* y, void* sum_out,
-                               void* rstd, int64_t rows, int64_t h, float eps, void* stream) {
+int rmsnorm_fwd_launch(const void* x, const void* residual, const void* weight, void* y, void* sum_out, void* rstd, int64_t rows, int64_t h,
+                       float eps, const RowSwap& swap, void* stream) {
     EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h <= kWideMaxH, EZL_EUNSUPPORTED,
                 "ezl_rmsnorm_fwd: need h %% 8 == 0 and h <= %d (got h=%lld)", kWideMaxH, (long long)h);
     EZL_REQUIRE(rows == 0 || (x && weight && y && rstd), EZL_EINVAL, "ezl_rmsnorm_fwd: null pointer");
@@ -427,7 +426,7 @@ extern "C" int ezl_rmsnorm_fwd(const void* x, const void* residual, const void* 
 #define LAUNCH(NC, RES)                                                                                             \
     hipLaunchKernelGGL((rmsnorm_fwd_kernel<NC, RES>), dim3((unsigned)grid), dim3(rpb * tpr), 0, st, (const bf16_t*)x, \
                        (const bf16_t*)residual, (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, \
-                       (int)rows, (int)h, eps, tpr)
+                       (int)rows, (int)h, eps, tpr, swap)
     if (residual) {
         if (nchunk == 1) LAUNCH(1, true); else if (nchunk == 2) LAUNCH(2, true); else LAUNCH(4, true);
     } else {
@@ -436,6 +435,26 @@ extern "C" int ezl_rmsnorm_fwd(const void* x, const void* residual, const void* 
 #undef LAUNCH
     EZL_LAUNCH_CHECK("ezl_rmsnorm_fwd");
     return EZL_OK;
+}
+
+// sizes of [d0, d1, h] whose rows lie swapped (those kernels hold a row in registers)
+int swap_check(const char* name, int64_t d0, int64_t d1, int64_t h) {
+    EZL_REQUIRE(d0 > 0 && d1 > 0 && d0 < (1LL << 31) && d1 < (1LL << 31) && d0 * d1 < (1LL << 31) && h <= 8192, EZL_EUNSUPPORTED,
+                "%s: need 0 < d0 * d1 < 2^31 and h <= 8192", name);
+    return EZL_OK;
+}
+
+}  // namespace
+
+extern "C" int ezl_rmsnorm_fwd(const void* x, const void* residual, const void* weight, void* y, void* sum_out,
+                               void* rstd, int64_t rows, int64_t h, float eps, void* stream) {
+    return rmsnorm_fwd_launch(x, residual, weight, y, sum_out, rstd, rows, h, eps, RowSwap{0, 0}, stream);
+}
+
+extern "C" int ezl_rmsnorm_fwd_swapped(const void* x, const void* weight, void* y, void* rstd, int64_t d0, int64_t d1, int64_t h, float eps,
+                                       void* stream) {
+    if (const int rc = swap_check("ezl_rmsnorm_fwd_swapped", d0, d1, h)) return rc;
+    return rmsnorm_fwd_launch(x, nullptr, weight, y, nullptr, rstd, d0 * d1, h, eps, RowSwap{(int)d0, (int)d1}, stream);
 }
 
 namespace {
@@ -465,13 +484,13 @@ int rmsnorm_bwd_check(const char* name, const void* dy, const void* x, const voi
 // both entry points: `partials` holds one fp32 row of h per block (at most max_blocks blocks; the narrow-row kernel uses up
 // to 256, the wide-row one up to 512), every used row fully written
 int rmsnorm_bwd_launch_rows(const void* dy, const void* x, const void* weight, const void* rstd, const void* dresidual, void* dx,
-                            float* partials, int64_t max_blocks, int64_t rows, int64_t h, int64_t& grid, hipStream_t st) {
+                            float* partials, int64_t max_blocks, int64_t rows, int64_t h, const RowSwap& swap, int64_t& grid, hipStream_t st) {
     const size_t smem = (size_t)h * sizeof(float);
     const bool stream = ezl_streams(rows * h * 2);
 #define LAUNCH_SPLIT(NC, NS, DR)                                                                                           \
     hipLaunchKernelGGL((stream ? rmsnorm_bwd_split_kernel<NC, NS, DR, true> : rmsnorm_bwd_split_kernel<NC, NS, DR, false>), dim3((unsigned)grid), dim3(256), smem, st, (const bf16_t*)dy, \
                        (const bf16_t*)x, (const bf16_t*)weight, (const float*)rstd, (const bf16_t*)dresidual, (bf16_t*)dx,  \
-                       partials, (int)rows, (int)h)
+                       partials, (int)rows, (int)h, swap)
     if (h <= 2048) {  // one wave per row, 8 rows per block
         const int nchunk = ((int)h + 511) / 512;
         grid = (rows + 7) / 8;
@@ -480,7 +499,7 @@ int rmsnorm_bwd_launch_rows(const void* dy, const void* x, const void* weight, c
 #define LAUNCH(NC, DR)                                                                                                    \
     hipLaunchKernelGGL((stream ? rmsnorm_bwd_wave_kernel<NC, DR, true> : rmsnorm_bwd_wave_kernel<NC, DR, false>), dim3((unsigned)grid), dim3(512), smem, st, (const bf16_t*)dy,    \
                        (const bf16_t*)x, (const bf16_t*)weight, (const float*)rstd, (const bf16_t*)dresidual, (bf16_t*)dx, \
-                       partials, (int)rows, (int)h)
+                       partials, (int)rows, (int)h, swap)
 #define LAUNCH_NC(DR)                                  \
     do {                                               \
         if (nchunk <= 1) LAUNCH(1, DR);                \
@@ -518,9 +537,9 @@ int rmsnorm_bwd_launch_rows(const void* dy, const void* x, const void* weight, c
 
 int rmsnorm_bwd_launch(const void* dy, const void* x, const void* weight, const void* rstd, const void* dresidual, void* dx,
                        void* dw_bf16, void* dw_f32, int accumulate, float* partials, int64_t max_blocks, int64_t rows, int64_t h,
-                       hipStream_t st) {
+                       hipStream_t st, const RowSwap& swap = RowSwap{0, 0}) {
     int64_t grid;
-    if (const int rc = rmsnorm_bwd_launch_rows(dy, x, weight, rstd, dresidual, dx, partials, max_blocks, rows, h, grid, st)) return rc;
+    if (const int rc = rmsnorm_bwd_launch_rows(dy, x, weight, rstd, dresidual, dx, partials, max_blocks, rows, h, swap, grid, st)) return rc;
     hipLaunchKernelGGL(ezl_colsum_kernel<0>, dim3((unsigned)((h + 63) / 64)), dim3(kColsumThreads), 0, st, (const float*)partials,
                        (int)grid, (int)h, (bf16_t*)dw_bf16, (float*)dw_f32, accumulate);
     EZL_LAUNCH_CHECK("ezl_rmsnorm_bwd(colsum)");
@@ -539,6 +558,18 @@ extern "C" int ezl_rmsnorm_bwd(const void* dy, const void* x, const void* weight
                               rmsnorm_bwd_blocks(h), rows, h, (hipStream_t)stream);
 }
 
+extern "C" int ezl_rmsnorm_bwd_swapped(const void* dy, const void* x, const void* weight, const void* rstd, void* dx, void* dw_bf16, void* dw_f32,
+                                       int accumulate, void* workspace, int64_t workspace_bytes, int64_t d0, int64_t d1, int64_t h,
+                                       void* stream) {
+    const char* name = "ezl_rmsnorm_bwd_swapped";
+    if (const int rc = swap_check(name, d0, d1, h)) return rc;
+    const int64_t rows = d0 * d1;
+    if (const int rc = rmsnorm_bwd_check(name, dy, x, weight, rstd, nullptr, dx, dw_bf16, dw_f32, rows, h)) return rc;
+    EZL_REQUIRE(workspace && workspace_bytes >= ezl_rmsnorm_bwd_workspace_bytes(rows, h), EZL_EINVAL, "%s: workspace missing or too small", name);
+    return rmsnorm_bwd_launch(dy, x, weight, rstd, nullptr, dx, dw_bf16, dw_f32, accumulate, (float*)workspace, rmsnorm_bwd_blocks(h), rows, h,
+                              (hipStream_t)stream, RowSwap{(int)d0, (int)d1});
+}
+
 // A layer's two norms leave their partial sums and one launch behind the second adds up both: a column sum takes 4 - 5 us at any width, nearly
 // all of it the launch and the latency of one pass over the partials.  Per pass:
 // captured two-layer stack of h = 256 437 -> 431 us, training iteration at h = 768 2449 -> 2438.
@@ -554,8 +585,8 @@ int rmsnorm_bwd_rows(const void* dy, const void* x, const void* weight, const vo
                      void* dw_f32, int accumulate, void* workspace, int64_t rows, int64_t h, NormWeightGrad& grad, void* stream) {
     if (const int rc = rmsnorm_bwd_check("ezl_rmsnorm_bwd", dy, x, weight, rstd, dresidual, dx, dw_bf16, dw_f32, rows, h)) return rc;
     int64_t grid;
-    if (const int rc = rmsnorm_bwd_launch_rows(dy, x, weight, rstd, dresidual, dx, (float*)workspace, rmsnorm_bwd_blocks(h), rows, h, grid,
-                                               (hipStream_t)stream))
+    if (const int rc = rmsnorm_bwd_launch_rows(dy, x, weight, rstd, dresidual, dx, (float*)workspace, rmsnorm_bwd_blocks(h), rows, h,
+                                               RowSwap{0, 0}, grid, (hipStream_t)stream))
         return rc;
     grad = {(const float*)workspace, dw_bf16, dw_f32, accumulate, (int)grid};
     return EZL_OK;

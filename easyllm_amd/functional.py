@@ -142,9 +142,20 @@ def bias_add(x, bias):
 # --------------------------------------------------------------------------------------------
 # RMSNorm (+ fused residual add): base_modules/layers/fused_layer_norm.py:49-71, transformer.py:786
 # --------------------------------------------------------------------------------------------
+def _norm_reads_swapped(x):
+    return K.rows_swapped(x) and x.shape[2] <= 8192
+
+
 class RMSNormFunction(torch.autograd.Function):
+    """An x whose first two dimensions are swapped in memory (a transposed view) is read where it lies, and its gradient is laid out
+    alike: the norm behind the layers, which run in sequence order."""
+
     @staticmethod
     def forward(ctx, x, weight, eps):
+        if _norm_reads_swapped(x):
+            y, rstd = K.rmsnorm_fwd_swapped(x, weight, eps)
+            ctx.save_for_backward(x, weight, rstd)
+            return y
         xc = x.contiguous()
         y, rstd, _ = K.rmsnorm_fwd(xc, weight, eps)
         ctx.save_for_backward(xc, weight, rstd)
@@ -154,7 +165,8 @@ class RMSNormFunction(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, rstd = ctx.saved_tensors
         mg, acc = _main_grad_target(weight)
-        dx, dw = K.rmsnorm_bwd(dy.contiguous(), x, weight, rstd, main_grad=mg, accumulate=acc)
+        bwd = K.rmsnorm_bwd_swapped if _norm_reads_swapped(x) else K.rmsnorm_bwd
+        dx, dw = bwd(dy.contiguous(), x, weight, rstd, main_grad=mg, accumulate=acc)
         return dx, dw, None
 
 
@@ -384,9 +396,9 @@ def decoder_layer(x, plan, cos, sin, position_ids, cu_seqlens, params):
 # --------------------------------------------------------------------------------------------
 class EmbeddingFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, ids, weight, host_flag=None):
+    def forward(ctx, ids, weight, host_flag=None, swapped=False):
         ids = ids.contiguous()
-        out, flag = K.embed_gather(ids, weight, host_flag)
+        out, flag = K.embed_gather(ids, weight, host_flag, swapped)
         ctx.save_for_backward(ids, weight)
         if flag is not None:
             ctx.mark_non_differentiable(flag)
@@ -396,10 +408,12 @@ class EmbeddingFunction(torch.autograd.Function):
     def backward(ctx, dout, _dflag):
         ids, weight = ctx.saved_tensors
         mg, acc = _main_grad_target(weight)
+        if ids.dim() == 2 and K.rows_swapped(dout):
+            return None, K.embed_grad_swapped(ids, dout, weight.shape[0], mg, acc), None, None
         if mg is not None:
             K.embed_scatter_add(ids, dout.contiguous(), mg, accumulate=acc)
-            return None, None, None
-        return None, K.embed_grad_bf16(ids, dout.contiguous(), weight.shape[0]), None
+            return None, None, None, None
+        return None, K.embed_grad_bf16(ids, dout.contiguous(), weight.shape[0]), None, None
 
 
 def _raise_for_id_flag(bad, ids, num_embeddings):
@@ -517,14 +531,16 @@ def check_position_ids(position_ids, table_len):
         _dispatch_flag(flag, position_ids, limit_tag)
 
 
-def embedding(ids, weight):
-    """Row gather; raises ValueError for an id >= vocab like the reference (:107-109)."""
+def embedding(ids, weight, sequence_first=False):
+    """Row gather; raises ValueError for an id >= vocab like the reference (:107-109).  sequence_first (ids [b, s]): the rows of the
+    result [b, s, h] lie in memory as [s, b, h], so that its transposition costs nothing."""
     pair = _held_pair(weight.device)
+    swapped = sequence_first and ids.dim() == 2 and ids.shape[0] > 1 and ids.shape[1] > 1 and ids.numel() < 2 ** 31
     if pair:
-        out, _ = EmbeddingFunction.apply(ids, weight, pair[1])
+        out, _ = EmbeddingFunction.apply(ids, weight, pair[1], swapped)
         _hold(weight.device, pair, ids, weight.shape[0])
         return out
-    out, flag = EmbeddingFunction.apply(ids, weight)
+    out, flag = EmbeddingFunction.apply(ids, weight, None, swapped)
     # inside a graph capture nothing may synchronise: the flag tensor is handed to whoever captures (runner.GraphedStep),
     # which reads it back after each replay
     _dispatch_flag(flag, ids, weight.shape[0])
@@ -548,6 +564,8 @@ def transpose01(x):
     """[d0, d1, ...] -> contiguous [d1, d0, ...]; a free view when either extent is 1."""
     if x.shape[0] == 1 or x.shape[1] == 1:
         return x.contiguous().view((x.shape[1], x.shape[0]) + tuple(x.shape[2:]))
+    if x.dim() >= 3 and x.transpose(0, 1).is_contiguous():  # it lies that way already
+        return x.transpose(0, 1)
     return Transpose01Function.apply(x)
 
 

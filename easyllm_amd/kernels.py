@@ -86,6 +86,45 @@ def rmsnorm_bwd(dy, x, weight, rstd, dresidual=None, main_grad=None, accumulate=
     return dx, dw
 
 
+def rows_swapped(x):
+    """x [d0, d1, h] lies in memory as [d1, d0, h] (and not also as it is), on 16 bytes: the kernels can read it there."""
+    return (x.dim() == 3 and not x.is_contiguous() and x.shape[0] > 1 and x.shape[1] > 1 and x.transpose(0, 1).is_contiguous()
+            and x.data_ptr() % 16 == 0 and x.shape[0] * x.shape[1] < 2 ** 31)
+
+
+def _swapped_bf16(t, name):
+    _need(t.dtype is BF16 and t.is_cuda and rows_swapped(t), "%s must be a bf16 GPU tensor with its rows in the other order" % name)
+
+
+def rmsnorm_fwd_swapped(x, weight, eps):
+    """rmsnorm_fwd of an x with swapped rows -> (y, rstd), y contiguous."""
+    _swapped_bf16(x, "x"); _bf16c(weight, "weight")
+    d0, d1, h = x.shape
+    _need(weight.numel() == h, "weight size mismatch")
+    y = torch.empty(x.shape, dtype=BF16, device=x.device)
+    rstd = torch.empty(d0 * d1, dtype=torch.float32, device=x.device)
+    _lib.call("ezl_rmsnorm_fwd_swapped", _p(x), _p(weight), _p(y), _p(rstd), d0, d1, h, float(eps), _stream())
+    return y, rstd
+
+
+def rmsnorm_bwd_swapped(dy, x, weight, rstd, main_grad=None, accumulate=False):
+    """rmsnorm_bwd of an x with swapped rows, which dx has too; dy is contiguous."""
+    _bf16c(dy, "dy"); _swapped_bf16(x, "x"); _bf16c(weight, "weight")
+    d0, d1, h = x.shape
+    _need(dy.shape == x.shape and rstd.numel() == d0 * d1 and rstd.dtype == torch.float32 and weight.numel() == h, "rmsnorm_bwd: shape mismatch")
+    dx = torch.empty((d1, d0, h), dtype=BF16, device=x.device).transpose(0, 1)
+    dw = None
+    if main_grad is None:
+        dw = torch.empty(h, dtype=BF16, device=x.device)
+    else:
+        _need(main_grad.dtype == torch.float32 and main_grad.is_contiguous() and main_grad.numel() == h, "bad main_grad")
+    ws_bytes = _lib.rmsnorm_bwd_workspace_bytes(d0 * d1, h)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    _lib.call("ezl_rmsnorm_bwd_swapped", _p(dy), _p(x), _p(weight), _p(rstd), _p(dx), _p(dw), _p(main_grad), 1 if accumulate else 0, _p(ws),
+              ws_bytes, d0, d1, h, _stream())
+    return dx, dw
+
+
 # ------------------------------------------------------------------------------------- SwiGLU
 def swiglu_fwd(gate, up):
     _bf16c(gate, "gate"); _bf16c(up, "up")
@@ -175,11 +214,18 @@ def ids_in_range_flag(ids, limit, host_flag=None):
 
 
 # ------------------------------------------------------------------------------------- embedding
-def embed_gather(ids, weight, host_flag=None):
-    """-> rows, flag (as `ids_in_range_flag`)"""
+def embed_gather(ids, weight, host_flag=None, swapped=False):
+    """-> rows, flag (as `ids_in_range_flag`).  swapped (ids [d0, d1]): the rows lie in memory as [d1, d0, h]."""
     _need(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous(), "ids must be contiguous int64 on the GPU")
     _bf16c(weight, "weight")
     V, h = weight.shape
+    if swapped:
+        d0, d1 = ids.shape
+        out = torch.empty((d1, d0, h), dtype=BF16, device=weight.device).transpose(0, 1)
+        flag = torch.zeros(1, dtype=torch.int32, device=weight.device) if host_flag is None else None
+        _lib.call("ezl_embed_gather_swapped", _p(ids), _p(weight), _p(out), _p(flag if host_flag is None else host_flag), 0 if host_flag is None else 1,
+                  d0, d1, h, V, _stream())
+        return out, flag
     out = torch.empty(tuple(ids.shape) + (h,), dtype=BF16, device=weight.device)
     if host_flag is not None:
         _lib.call("ezl_embed_gather_host_flag", _p(ids), _p(weight), _p(out), _p(host_flag), ids.numel(), h, V, _stream())
@@ -199,6 +245,22 @@ def embed_scatter_add(ids, dy, dweight_f32, accumulate=True):
     ws_bytes = _lib.embed_scatter_add_workspace_bytes(ids.numel(), V)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dy.device)
     _lib.call("ezl_embed_scatter_add", _p(ids), _p(dy), _p(dweight_f32), _p(ws), ws_bytes, ids.numel(), h, V, 1 if accumulate else 0, _stream())
+
+
+def embed_grad_swapped(ids, dy, vocab, main_grad=None, accumulate=False):
+    """embed_scatter_add into main_grad (-> None), or embed_grad_bf16, of a dy with swapped rows."""
+    _need(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and ids.dim() == 2, "ids must be contiguous int64 [d0, d1] on the GPU")
+    _swapped_bf16(dy, "dy")
+    (d0, d1), h = ids.shape, dy.shape[-1]
+    _need(dy.shape == (d0, d1, h), "one dy row per id")
+    if main_grad is not None:
+        _need(main_grad.dtype == torch.float32 and main_grad.is_contiguous() and main_grad.shape == (vocab, h), "bad dweight")
+    out = torch.empty((vocab, h), dtype=BF16, device=dy.device) if main_grad is None else main_grad
+    ws_bytes = _lib.embed_scatter_add_workspace_bytes(d0 * d1, vocab)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dy.device)
+    _lib.call("ezl_embed_grad_swapped", _p(ids), _p(dy), _p(out), 0 if main_grad is None else 1, _p(ws), ws_bytes, d0, d1, h, vocab,
+              1 if accumulate else 0, _stream())
+    return out if main_grad is None else None
 
 
 def embed_grad_bf16(ids, dy, vocab):

@@ -251,9 +251,9 @@ class VocabParallelEmbedding(torch.nn.Module):
         with torch.no_grad():
             init_method(self.weight)
 
-    def forward(self, input_):
+    def forward(self, input_, sequence_first=False):
         # the range check of :107-109 happens inside the gather kernel (flag -> ValueError)
-        return dist_env.reduce_from_tensor_model_parallel_region(F_.embedding(input_, self.weight))
+        return dist_env.reduce_from_tensor_model_parallel_region(F_.embedding(input_, self.weight, sequence_first))
 
 
 # ---- GLU activations --------------------------------------------------------------------------

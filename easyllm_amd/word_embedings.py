@@ -26,17 +26,18 @@ class Embedding(torch.nn.Module):
         self.position_embeddings = None
         self.sequence_parallel = sequence_parallel
 
-    def forward(self, input_ids, position_ids):
-        embeddings = self.word_embeddings(input_ids)  # [b, s, h]
+    def forward(self, input_ids, position_ids, sequence_first=False):
+        embeddings = self.word_embeddings(input_ids, sequence_first=True) if sequence_first else self.word_embeddings(input_ids)  # [b, s, h]
         if self.sequence_parallel:
             embeddings = dist_env.scatter_to_sequence_parallel_region(embeddings)
         return embeddings
 
 
 class EmbeddingPipe(Embedding):
-    def forward(self, inputs, **kwargs):
+    def forward(self, inputs, sequence_first=False, **kwargs):
+        """sequence_first: the rows of the embeddings [b, s, h] lie in memory as [s, b, h], for a transposition right behind."""
         input_ids, position_ids, attention_mask = inputs[0], inputs[1], inputs[2]
-        embeddings = super().forward(input_ids, position_ids)
+        embeddings = super().forward(input_ids, position_ids, True) if sequence_first else super().forward(input_ids, position_ids)
         if len(inputs) == 4:
             # the layers index their rotary tables (one row per sequence position) with these ids
             F_.check_position_ids(position_ids, input_ids.shape[1])

@@ -46,6 +46,12 @@ int ezl_rmsnorm_bwd(const void* dy, const void* x, const void* weight, const voi
                     void* dw_bf16, void* dw_f32, int accumulate, void* workspace, int64_t workspace_bytes, int64_t rows,
                     int64_t h, void* stream);
 
+/* The two for an x [d0, d1, h] whose rows lie in memory in the order [d1, d0] (dx is written in that order; y, dy and rstd are in
+ * [d0, d1]): the norm behind a change between batch and sequence order without a pass of its own for that.  h <= 8192. */
+int ezl_rmsnorm_fwd_swapped(const void* x, const void* weight, void* y, void* rstd, int64_t d0, int64_t d1, int64_t h, float eps, void* stream);
+int ezl_rmsnorm_bwd_swapped(const void* dy, const void* x, const void* weight, const void* rstd, void* dx, void* dw_bf16, void* dw_f32,
+                            int accumulate, void* workspace, int64_t workspace_bytes, int64_t d0, int64_t d1, int64_t h, void* stream);
+
 /* ezl_rmsnorm_bwd without the workspace argument.  No counterpart in the reference: it exists for callers that cannot
  * obtain device memory at the call site (code under HIP graph capture, tight serving loops, harnesses that forbid
  * allocation).  The per-block dw partials go to a device array built into the library (16 MiB per GPU, held until the
@@ -103,6 +109,13 @@ int ezl_embed_scatter_add(const void* ids, const void* dy, void* dweight_f32, vo
 /* the overwriting form into a bf16 gradient: the same fp32 sums, rounded once */
 int ezl_embed_grad_bf16(const void* ids, const void* dy, void* dweight_bf16, void* workspace, int64_t workspace_bytes,
                         int64_t rows, int64_t h, int64_t vocab, void* stream);
+
+/* The same for ids [d0, d1] and rows (out, dy) that lie in the order [d1, d0]; sums are taken in the order of the ids, as above.  host_flag: the flag
+ * is pinned host memory, as in ezl_embed_gather_host_flag.  fp32: dweight is fp32, else bf16 and overwritten. */
+int ezl_embed_gather_swapped(const void* ids, const void* weight, void* out, void* bad_flag, int host_flag, int64_t d0, int64_t d1, int64_t h,
+                             int64_t vocab, void* stream);
+int ezl_embed_grad_swapped(const void* ids, const void* dy, void* dweight, int fp32, void* workspace, int64_t workspace_bytes, int64_t d0, int64_t d1,
+                           int64_t h, int64_t vocab, int accumulate, void* stream);
 
 /* ---- layout / dtype plumbing of llama/llama.py:145-188 (transpose, undo, float16_to_fp32) ---- */
 int ezl_transpose01(const void* x, void* y, int64_t d0, int64_t d1, int64_t inner, void* stream); /* y[j,i,:] = x[i,j,:] */

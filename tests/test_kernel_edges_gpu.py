@@ -665,3 +665,46 @@ def test_loss_and_gradient_of_rows_kept_as_bf16_in_registers(K, rows, V, cut):
         g /= count.double()
         assert ((grad[r].double() - g).abs() <= g.abs() * (2.0 ** -8 + V * 2.0 ** -23) + 2.0 ** -126).all()
     assert torch.equal(K.ce_fused(x, labels, w, count, cut)[1], grad)  # in place: the same bits
+
+
+@pytest.mark.parametrize("d0,d1,h", [(2, 3, 8), (2, 512, 256), (3, 389, 1024), (5, 7, 1032), (1000, 4, 2048), (2, 33, 2056), (3, 301, 4096), (7, 5, 5120), (2, 129, 8192)])
+def test_rmsnorm_of_rows_in_the_other_order(K, d0, d1, h):
+    """x [d0, d1, h] stored as [d1, d0, h]: what the norm of its contiguous copy gives, forward and backward, bit for bit."""
+    print("rmsnorm swapped", d0, d1, h, flush=True)
+    x, w, dy = rnd(d1, d0, h, seed=1).transpose(0, 1), rnd(h, seed=2), rnd(d0, d1, h, seed=3)
+    assert K.rows_swapped(x)
+    y, rstd = K.rmsnorm_fwd_swapped(x, w, 1e-6)
+    want_y, want_rstd, _ = K.rmsnorm_fwd(x.contiguous(), w, 1e-6)
+    assert y.is_contiguous() and torch.equal(y, want_y) and torch.equal(rstd, want_rstd)
+    dx, dw = K.rmsnorm_bwd_swapped(dy, x, w, rstd)
+    want_dx, want_dw = K.rmsnorm_bwd(dy, x.contiguous(), w, rstd)
+    assert K.rows_swapped(dx) and torch.equal(dx, want_dx) and torch.equal(dw, want_dw)
+    mg, want_mg = torch.full((h,), 0.5, device="cuda"), torch.full((h,), 0.5, device="cuda")
+    K.rmsnorm_bwd_swapped(dy, x, w, rstd, main_grad=mg, accumulate=True)
+    K.rmsnorm_bwd(dy, x.contiguous(), w, rstd, main_grad=want_mg, accumulate=True)
+    assert torch.equal(mg, want_mg)
+
+
+@pytest.mark.parametrize("d0,d1,h,V,same", [(2, 3, 8, 5, 0), (2, 512, 256, 32000, 0), (3, 389, 1024, 4099, 40), (4, 1000, 72, 900, 1500), (700, 3, 4104, 130, 300),
+                                            (2, 257, 8200, 64, 33), (2, 33000, 8, 50, 65999)])
+def test_embedding_of_rows_in_the_other_order(K, d0, d1, h, V, same):
+    """ids [d0, d1], rows stored as [d1, d0, h]: the gather, its flags and every form of the gradient as of contiguous rows, bit for bit.  Ids that occur once,
+    a few times, and (`same` of them) often enough for the kernel's lists and its bitmap over two windows of row numbers."""
+    print("embedding swapped", d0, d1, h, V, same, flush=True)
+    ids = torch.randint(0, V, (d0 * d1,), generator=torch.Generator().manual_seed(d0 + d1))
+    ids[d0 * d1 - same:] = V // 2
+    ids[0], ids[-1] = V, -1  # out of range
+    ids, W, dy = ids.view(d0, d1).cuda(), rnd(V, h, seed=1), rnd(d1, d0, h, seed=2).transpose(0, 1)
+    out, flag = K.embed_gather(ids, W, swapped=True)
+    want, want_flag = K.embed_gather(ids, W)
+    assert K.rows_swapped(out) and torch.equal(out, want) and flag.item() == want_flag.item() == 3
+    host = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    out, none = K.embed_gather(ids, W, host, swapped=True)
+    torch.cuda.synchronize()
+    assert none is None and torch.equal(out, want) and host.item() == 0x101
+    for accumulate in (False, True):
+        got, ref = torch.full((V, h), 2.5, device="cuda"), torch.full((V, h), 2.5, device="cuda")
+        assert K.embed_grad_swapped(ids, dy, V, got, accumulate) is None
+        K.embed_scatter_add(ids, dy.contiguous(), ref, accumulate=accumulate)
+        assert torch.equal(got, ref)
+    assert torch.equal(K.embed_grad_swapped(ids, dy, V), K.embed_grad_bf16(ids, dy.contiguous(), V))

@@ -281,3 +281,39 @@ def test_qkv_pack_and_bias_variants(gpu_device):
     close(xg.grad, xr.grad, "packed layer dx")
     close(layer.self_attn.wqkv.weight.grad, Wg["3.self_attn.wqkv.weight"].grad, "wqkv grad")
     close(layer.self_attn.wqkv.bias.grad, Wg["3.self_attn.wqkv.bias"].grad, "wqkv bias grad")
+
+
+@pytest.mark.parametrize("b,s,main_grads,checkpoint", [(2, 160, True, False), (3, 77, False, True), (1, 64, True, False), (5, 1, True, False)])
+def test_rows_change_their_order_inside_the_embedding_and_the_final_norm(gpu_device, b, s, main_grads, checkpoint):
+    """A hook on either module brings the separate transpositions back, and sees contiguous tensors: the same logits, loss and gradients bit for bit, also
+    where what is saved for backward comes back laid out otherwise."""
+    from easyllm_amd import runner, workloads as W
+    w = dict(num_layers=2, hidden_size=256, num_attention_heads=2, num_kv_attention_heads=2, intermediate_size=512, vocab_size=1024, seq=s, batch=b,
+             seed=5)
+    model, _ = build_pair(w, gpu_device, checkpoint_activations=checkpoint)
+    inputs, (labels, loss_mask), _ = W.make_inputs(w)
+    inputs, labels = to_dev(inputs, gpu_device), (labels.to(gpu_device), loss_mask.to(gpu_device))
+    if not main_grads:
+        for p in model.parameters():
+            del p.main_grad
+
+    def step():
+        runner.zero_main_grads(model)
+        loss = runner.forward_step(model, inputs, labels)
+        with torch.no_grad():
+            logits = model(inputs)
+        return [loss.detach(), logits] + [(p.main_grad if main_grads else p.grad).clone() for p in model.parameters()]
+
+    got = step()
+    seen = []
+    norm, embedding = model.forward_funcs[-3 if model.fp32_logits else -2], model.forward_funcs[1]
+    hooks = [norm.register_forward_pre_hook(lambda m, x: seen.append(x[0].is_contiguous())),
+             embedding.register_forward_hook(lambda m, i, x: seen.append((x[0] if isinstance(x, tuple) else x).is_contiguous()))]
+    want = step()
+    for h in hooks:
+        h.remove()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(memory_format=torch.contiguous_format), lambda t: t):
+        saved = step()
+    assert len(seen) == 4 and all(seen)
+    for a, c, e in zip(got, want, saved):
+        assert torch.equal(a, c) and torch.equal(a, e)
