@@ -567,56 +567,67 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the last item's loads of a next tile (its own again) may not outlive the workgroup's LDS
 }
 
-// C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order.  One block per 16 rows of a tile: a thread owns 16
-// consecutive columns of one row.
+// Sum in index order of the vectors at src, src + stride, ...: `count` partial results, read once, up to eight at a time.
+__device__ __forceinline__ f32x4 sum_partials(const float* __restrict__ src, size_t stride, int count) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    const auto add = [&](auto COUNT) {
+        constexpr int n = decltype(COUNT)::value;
+        for (; count >= n; count -= n, src += n * stride) {
+            f32x4 x[n];
+#pragma unroll
+            for (int p = 0; p < n; ++p) x[p] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + p * stride));
+#pragma unroll
+            for (int p = 0; p < n; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += x[p][e];
+        }
+    };
+    add(std::integral_constant<int, 8>{});
+    add(std::integral_constant<int, 4>{});
+    add(std::integral_constant<int, 2>{});
+    add(std::integral_constant<int, 1>{});
+    return v;
+}
+
+// C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order.  A wave owns a row of a tile, a lane four consecutive columns
+// of it.  What bounds it is the read of the partial tiles, which comes from the last-level cache mostly: every load instruction is 1 KiB of one row, and
+// up to eight of a lane's are in flight.  (With 16 consecutive columns a thread, whose loads of a wave lay 64 bytes apart, and a part at a time, us before and now, M x N of a
+// product, tiles x shares: 1531 x 4096, 128 of 192 rows x 2 16.3 -> 10.2; 2048 x 768, 24 x 10 18.0 -> 10.4; 1167 x 1024, 20 x 12 17.1 -> 9.3; 4000 x 2048, 128 x 2
+// 22.3 -> 12.8; fp32, 50304 x 1024, 20 x 2 5.8 -> 4.6.)
+constexpr int kReduceRows = 4;  // rows of a block
 template <typename OutT, int TBM>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(OutT* __restrict__ C, int M, int N, int64_t ldc, int accumulate,
                                                                 int tiles_m, int tiles_n, const SplitPlan plan) {
-    constexpr int PIECES = TBM / 16;
+    constexpr int PIECES = TBM / kReduceRows;
     const int t = blockIdx.x / PIECES;  // split tile
     int tm, tn;
     tile_of(plan.full + t, tiles_m, tiles_n, tm, tn);
-    const int rl = (blockIdx.x - t * PIECES) * 16 + (threadIdx.x >> 4), cl = (threadIdx.x & 15) * 16;
+    const int rl = (blockIdx.x - t * PIECES) * kReduceRows + (threadIdx.x >> 6), cl = (threadIdx.x & 63) * 4;
     const int row = tm * TBM + rl, col = tn * BN + cl;
     if (row >= M || col >= N) return;
-    float v[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = 0.f;
-    const float* src = plan.partial + (size_t)t * plan.nsplit * (size_t)(TBM * BN) + (size_t)rl * BN + cl;
-    for (int p = 0; p < plan.nsplit; ++p, src += TBM * BN) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 x = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src) + q);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * q + e] += x[e];
-        }
-    }
+    f32x4 v = sum_partials(plan.partial + (size_t)t * plan.nsplit * (TBM * BN) + (size_t)rl * BN + cl, TBM * BN, plan.nsplit);
     if (accumulate & kRoundResult) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = (float)(bf16_t)v[e];
+        for (int e = 0; e < 4; ++e) v[e] = (float)(bf16_t)v[e];
         accumulate = 0;
     }
     OutT* dst = C + (int64_t)row * ldc + col;
-    if (col + 16 <= N && ldc % 8 == 0 && ((uintptr_t)C & 15) == 0) {  // whole 16-column piece, 16-byte aligned
-        constexpr int VE = 16 / (int)sizeof(OutT);  // elements per 16-byte vector
-        typedef OutT vec_t __attribute__((ext_vector_type(VE)));
+    if (col + 4 <= N && ldc % 8 == 0 && ((uintptr_t)C & 15) == 0) {
+        typedef OutT vec_t __attribute__((ext_vector_type(4)));
+        vec_t o;
+        if (accumulate) {
+            const vec_t old = *reinterpret_cast<const vec_t*>(dst);
 #pragma unroll
-        for (int q = 0; q < 16 / VE; ++q) {
-            vec_t o;
-            if (accumulate) {
-                const vec_t old = *reinterpret_cast<const vec_t*>(dst + q * VE);
+            for (int e = 0; e < 4; ++e) o[e] = (OutT)(v[e] + (float)old[e]);
+        } else {
 #pragma unroll
-                for (int e = 0; e < VE; ++e) o[e] = (OutT)(v[q * VE + e] + (float)old[e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < VE; ++e) o[e] = (OutT)v[q * VE + e];
-            }
-            *reinterpret_cast<vec_t*>(dst + q * VE) = o;
+            for (int e = 0; e < 4; ++e) o[e] = (OutT)v[e];
         }
+        *reinterpret_cast<vec_t*>(dst) = o;
         return;
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
+    for (int e = 0; e < 4; ++e)
         if (col + e < N) store_out<OutT>(dst + e, v[e], accumulate != 0);
 }
 
@@ -959,7 +970,7 @@ void launch_large(int kind, bool lines, const void* A, const void* B, void* C, i
         hipLaunchKernelGGL((gemm_d2l_kernel<A_KC, B_KC, OutT, MULTI, KTAIL>), dim3((unsigned)items), dim3(512), 0, st, (const bf16_t*)A,
                            (const bf16_t*)B, (OutT*)C, M, N, K, lda, ldb, ldc, accumulate, tiles_m, tiles_n, plan, seg);
 #define EZL_REDUCE(TBM)                                                                                                                    \
-    hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT, TBM>), dim3((unsigned)(plan.rest * (TBM / 16))), dim3(256), 0, st, (OutT*)C, M, N, ldc, \
+    hipLaunchKernelGGL((gemm_split_reduce_kernel<OutT, TBM>), dim3((unsigned)(plan.rest * (TBM / kReduceRows))), dim3(256), 0, st, (OutT*)C, M, N, ldc, \
                        accumulate, tiles_m, tiles_n, plan)
     if (plan.nsplit > 1) {
         if (kind == kTile192x256) EZL_REDUCE(192);

@@ -58,3 +58,27 @@ def test_input_gradient_over_pairs_on_large_tiles(K, T, n_in, outs):  # noqa: F8
 @pytest.mark.parametrize("T,n_in,outs", PAIRS)
 def test_pairs_take_the_large_tiles(T, n_in, outs):
     assert _lib.gemm_plan("input gradient over pairs", [T], [n_in], sum(outs))[1:3] == (192, 256)
+
+
+# (form, M, N, K, shares): every count of partial tiles that are added at a time (8, 4, 2, 1), edges inside the last vector
+SHARES = [(0, 2048, 2304, 8192, 3), (0, 1500, 1800, 32768, 5), (0, 1500, 1536, 32768, 7), (0, 1024, 1280, 32768, 12), (1, 1167, 2048, 32768, 6),
+          (2, 2048, 1800, 16445, 4), (2, 904, 1800, 32829, 8)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,M,N,Kd,shares", SHARES)
+def test_partial_tiles_are_added(K, form, M, N, Kd, shares):  # noqa: F811
+    """Whole vectors, and results of which no row but the first starts on 16 bytes: element by element, the same bits."""
+    print("gemm shares", form, M, N, Kd, flush=True)
+    check_gemm(K, form, M, N, Kd)
+    check_gemm(K, form, M, N, Kd, accumulate=True, seed=5)
+    A, B = rnd(M, Kd) if form < 2 else rnd(Kd, M), rnd(N, Kd, seed=1) if form == 0 else rnd(Kd, N, seed=1)
+    wide = torch.zeros(M, N + 1, device="cuda", dtype=torch.float32 if form == 2 else torch.bfloat16)
+    args = A, B, M, N, Kd, A.stride(0), B.stride(0), form < 2, form == 0
+    K.gemm(*args, out=wide[:, :N])
+    assert torch.equal(wide[:, :N], K.gemm(*args, out=torch.zeros_like(wide)[:, 1:].contiguous())) and not wide[:, N].any()
+
+
+@pytest.mark.parametrize("form,M,N,Kd,shares", SHARES)
+def test_products_are_split_as_they_are_listed(form, M, N, Kd, shares):
+    assert _lib.gemm_plan(FORMS[form], [M], [N], Kd)[1:4] == (256, 256, shares)
