@@ -649,8 +649,7 @@ SplitPlan make_plan(int kind, bool lines, int64_t tiles, int64_t nk, void* works
     // Up to 96 tiles always: two shares and more of them.  97 - 128 are half a chip's worth, in two shares; time of them split over whole, 1400 products,
     // by K tiles 16 - 31 1.36, 32 - 47 1.07, 48 - 63 0.93, 96 - 127 0.75, 256 - 399 0.63 (behind whole rounds 1.12, 1.03, 0.98, 0.91, 0.82).
     if (r == 0 || r > (lines && nk >= 48 ? kCus / 2 : 96)) return p;
-    int s = (int)(kCus / r);
-    while (s > 1 && nk / s < 8) --s;  // a share of fewer than 8 K tiles is mostly prologue
+    const int s = (int)(kCus / r < nk / 8 ? kCus / r : nk / 8);  // a share of fewer than 8 K tiles is mostly prologue
     if (s < 2) return p;
     if (!workspace || workspace_bytes < r * s * tile_bytes(kind)) return p;
     p.full = (int)(tiles - r); p.rest = (int)r; p.nsplit = s; p.partial = (float*)workspace;
