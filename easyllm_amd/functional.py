@@ -564,7 +564,7 @@ def transpose01(x):
     """[d0, d1, ...] -> contiguous [d1, d0, ...]; a free view when either extent is 1."""
     if x.shape[0] == 1 or x.shape[1] == 1:
         return x.contiguous().view((x.shape[1], x.shape[0]) + tuple(x.shape[2:]))
-    if x.dim() >= 3 and x.transpose(0, 1).is_contiguous():  # it lies that way already
+    if K.rows_swapped(x):  # it lies that way already
         return x.transpose(0, 1)
     return Transpose01Function.apply(x)
 

@@ -88,8 +88,11 @@ def rmsnorm_bwd(dy, x, weight, rstd, dresidual=None, main_grad=None, accumulate=
 
 def rows_swapped(x):
     """x [d0, d1, h] lies in memory as [d1, d0, h] (and not also as it is), on 16 bytes: the kernels can read it there."""
-    return (x.dim() == 3 and not x.is_contiguous() and x.shape[0] > 1 and x.shape[1] > 1 and x.transpose(0, 1).is_contiguous()
-            and x.data_ptr() % 16 == 0 and x.shape[0] * x.shape[1] < 2 ** 31)
+    shape = x.shape
+    if len(shape) != 3:
+        return False
+    d0, d1, h = shape
+    return d0 > 1 and d1 > 1 and x.stride() == (h, d0 * h, 1) and x.data_ptr() % 16 == 0 and d0 * d1 < 2 ** 31
 
 
 def _swapped_bf16(t, name):

@@ -64,12 +64,14 @@ def _run_spec(f, following, x):
     """f(x), laid out as the spec behind it (None: nothing is) takes it for free where both are the framework's own: the embedding's rows in
     the layers' order, the last layer's rows left in place for a norm that reads them in the batch's order, logits in fp32 from the
     product.  Passes over memory, four of a training step's launches (captured two-layer stack of h = 256 431 -> 424 us a step, 4 x 1000 tokens of h = 2048 2822 -> 2794)."""
-    if (following is sequence_first and type(f) is EmbeddingPipe and Embedding.forward is _EMBEDDING_FORWARD
+    if (following is sequence_first and type(f) is EmbeddingPipe and x[0].shape[0] > 1 and Embedding.forward is _EMBEDDING_FORWARD
             and are_plain(((f, EmbeddingPipe), (f.word_embeddings, VocabParallelEmbedding)))):
         return f(x, sequence_first=True)
-    if f is batch_first and is_plain(following, RMSNorm):
+    if f is batch_first and type(following) is RMSNorm:
         x = x[0] if isinstance(x, (tuple, list)) else x
-        return x.transpose(0, 1) if x.dim() == 3 else batch_first(x)
+        if x.dim() == 3 and x.shape[1] > 1 and is_plain(following, RMSNorm):
+            return x.transpose(0, 1)
+        return batch_first(x)
     if following is float16_to_fp32 and is_plain(f, EmbedddingPipeNoTied):
         return f(x, fp32_output=True)  # (the cast then has nothing to do)
     return f(x)
