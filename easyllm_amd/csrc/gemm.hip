@@ -237,7 +237,7 @@ __global__ __launch_bounds__(512) void gemm_d2l_kernel(const bf16_t* __restrict_
     const int mrem = M - m0 < BM ? M - m0 : BM, nrem = N - n0;
     OutT* Ct = C + (int64_t)m0 * ldc + n0;
     if (N % 8 == 0 && ldc % (16 / (int)sizeof(OutT)) == 0 && ((uintptr_t)C & 15) == 0 && ldc < (1 << 21) / ((int)sizeof(OutT) / 2)) {
-        store_tile_flags<8, 4, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ldc, mrem, nrem, arow, brow, lane, accumulate);
+        store_tile_flags<8, 4, OutT, true, A_KC && B_KC>(acc, Ct, ldc, mrem, nrem, arow, brow, lane, accumulate);
         return;
     }
 #pragma unroll
@@ -558,7 +558,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const bf16_t* __restric
         } else {
             const int mrem = M - it.m0 < TBM ? M - it.m0 : TBM;
             OutT* Ct = C + (int64_t)it.m0 * ld + it.n0;
-            store_tile_flags<TM, 8, OutT, true, A_KC && B_KC && sizeof(OutT) == 4>(acc, Ct, ld, mrem, N - it.n0, arow, brow, lane, accumulate);
+            store_tile_flags<TM, 8, OutT, true, A_KC && B_KC>(acc, Ct, ld, mrem, N - it.n0, arow, brow, lane, accumulate);
         }
         if (!more) break;
         it = next;
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(OutT* __restrict
     if (accumulate & kRoundResult) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = (float)(bf16_t)v[e];
-        accumulate = 0;
+        accumulate &= 1;
     }
     OutT* dst = C + (int64_t)row * ldc + col;
     if (col + 4 <= N && ldc % 8 == 0 && ((uintptr_t)C & 15) == 0) {
@@ -1086,6 +1086,15 @@ extern "C" int ezl_gemm_bf16(const void* A, const void* B, void* C, int64_t M, i
         else EZL_GEMM_CASE(false, true, float);
     }
 #undef EZL_GEMM_CASE
+    EZL_LAUNCH_CHECK("ezl_gemm_bf16");
+    return EZL_OK;
+}
+
+int gemm_forward_add(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
+    EZL_REQUIRE(M > 0 && N > 0 && K > 0 && C, EZL_EINVAL, "ezl_gemm_bf16: null pointer or empty product");
+    if (const int rc = check_operands(A, B, M, N, K, K, K, N, 1, 1)) return rc;
+    EZL_REQUIRE(!workspace || ezl_aligned16(workspace), EZL_EINVAL, "ezl_gemm_bf16: workspace must be 16-byte aligned");
+    launch<true, true, bf16_t>(A, B, C, (int)M, (int)N, (int)K, K, K, N, 1 | kRoundResult, workspace, workspace_bytes, (hipStream_t)stream);
     EZL_LAUNCH_CHECK("ezl_gemm_bf16");
     return EZL_OK;
 }

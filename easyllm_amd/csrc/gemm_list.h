@@ -13,3 +13,7 @@ __attribute__((visibility("hidden"))) int gemm_list(int count, const void* const
                                                     const int64_t* N, int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc,
                                                     int a_kc, int b_kc, int out_dtype, const int* accumulate, void* workspace,
                                                     int64_t workspace_bytes, void* stream);
+
+// C[M, N] += A[M, K] * B[N, K]^T, all contiguous bf16, the product rounded to bf16 before it is added: the bits of a product and an addition
+__attribute__((visibility("hidden"))) int gemm_forward_add(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, void* workspace,
+                                                           int64_t workspace_bytes, void* stream);

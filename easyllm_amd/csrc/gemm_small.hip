@@ -38,12 +38,12 @@ template <typename OutT>
 __device__ __forceinline__ bool vector_stores(const GemmProblem& p) {
     return p.N % 8 == 0 && p.ldc % (16 / (int)sizeof(OutT)) == 0 && ((uintptr_t)p.C & 15) == 0;
 }
-template <int TM, int TN, typename OutT>
+template <bool FORWARD, int TM, int TN, typename OutT>
 __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], const GemmProblem& p, int m0, int n0, int row0, int col0, int lane) {
     OutT* C = (OutT*)p.C + (int64_t)m0 * p.ldc + n0;
     const int mrem = p.M - m0 < 256 ? p.M - m0 : 256, nrem = p.N - n0;  // (no tile is taller: the range fits 31 bits)
-    if (vector_stores<OutT>(p)) store_tile_flags<TM, TN, OutT, true, sizeof(OutT) == 4>(acc, C, p.ldc, mrem, nrem, row0, col0, lane, p.accumulate);
-    else store_tile_flags<TM, TN, OutT, false, sizeof(OutT) == 4>(acc, C, p.ldc, mrem, nrem, row0, col0, lane, p.accumulate);
+    if (vector_stores<OutT>(p)) store_tile_flags<TM, TN, OutT, true, FORWARD>(acc, C, p.ldc, mrem, nrem, row0, col0, lane, p.accumulate);
+    else store_tile_flags<TM, TN, OutT, false, FORWARD>(acc, C, p.ldc, mrem, nrem, row0, col0, lane, p.accumulate);
 }
 
 // this workgroup's share of the reduction, as a dense fp32 tile; small_reduce_kernel adds the shares
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(const GemmSmallArgs a
     }
     phase_b(smem, smem, no{}, no{});
     if (args.nsplit > 1) store_partial<TM, TN, TBM, TBN>(acc, args, tile, part, arow, brow, lane);
-    else store_tile<TM, TN, OutT>(acc, p, m0, n0, arow, brow, lane);
+    else store_tile<A_KC && B_KC, TM, TN, OutT>(acc, p, m0, n0, arow, brow, lane);
 }
 
 // =================================================================================================
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256) void gemm_square_kernel(const GemmSmallArgs ar
         free_stage = free_stage + 1 == ST ? 0 : free_stage + 1;
     }
     if (args.nsplit > 1) store_partial<T, T, TB, TB>(acc, args, tile, part, arow, brow, lane);
-    else store_tile<T, T, OutT>(acc, p, m0, n0, arow, brow, lane);
+    else store_tile<A_KC && B_KC, T, T, OutT>(acc, p, m0, n0, arow, brow, lane);
 }
 
 // =================================================================================================
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(512) void gemm_64_waves_kernel(const GemmSmallArgs 
 #pragma unroll
             for (int r = 0; r < 4; ++r) sum[0][q][r] += x[r];
         }
-    store_tile<1, 2, OutT>(sum, p, m0, n0, (wave >> 1) * 16, (wave & 1) * 32, lane);
+    store_tile<A_KC && B_KC, 1, 2, OutT>(sum, p, m0, n0, (wave >> 1) * 16, (wave & 1) * 32, lane);
 }
 
 // C tile (=|+=) sum of the nsplit fp32 partial tiles, added in index order; a thread owns 8 consecutive columns of one row

@@ -17,7 +17,8 @@ struct KSegments {
     int K1, K2;
 };
 
-// Kernels take it in place of `accumulate`: an fp32 result is rounded to bf16 first (logits that are handed out in fp32).
+// Kernels take it in the bits of `accumulate`: the product is rounded to bf16 first (logits that are handed out in fp32; with bit 0, a forward product
+// added to a bf16 tensor as a launch of its own would add the two).
 constexpr int kRoundResult = 2;
 
 namespace {
@@ -295,7 +296,7 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
                 if constexpr (ACC) {
                     const bf16x8 o = __builtin_bit_cast(bf16x8, old[i & 1][jp]);
 #pragma unroll
-                    for (int r = 0; r < 8; ++r) v[r] += (float)o[r];
+                    for (int r = 0; r < 8; ++r) v[r] = (ROUND ? (float)(bf16_t)v[r] : v[r]) + (float)o[r];
                 }
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, pack8(v)), cbuf, offset(jp) + i * row_step, 0, 0);
             }
@@ -334,12 +335,14 @@ __device__ __forceinline__ void store_tile_impl(const f32x4 (&acc)[TM][TN], OutT
     }
 }
 
-// as above with the kernel's flags: bit 0 accumulate, kRoundResult (only where the form has it: MAY_ROUND)
+// as above with the kernel's flags: bit 0 accumulate, kRoundResult (only where the form has it: MAY_ROUND; an fp32 result has it without bit 0, a bf16
+// one, which is rounded as it is stored, with it)
 template <int TM, int TN, typename OutT, bool VEC, bool MAY_ROUND>
 __device__ __forceinline__ void store_tile_flags(const f32x4 (&acc)[TM][TN], OutT* C, int64_t ldc, int mrem, int nrem, int row0, int col0,
                                                  int lane, int flags) {
-    if (flags & 1) store_tile_impl<TM, TN, OutT, true, VEC>(acc, C, ldc, mrem, nrem, row0, col0, lane);
-    else if (MAY_ROUND && (flags & kRoundResult)) store_tile_impl<TM, TN, OutT, false, VEC, true>(acc, C, ldc, mrem, nrem, row0, col0, lane);
+    if (MAY_ROUND && sizeof(OutT) == 2 && flags == (1 | kRoundResult)) store_tile_impl<TM, TN, OutT, true, VEC, MAY_ROUND && sizeof(OutT) == 2>(acc, C, ldc, mrem, nrem, row0, col0, lane);
+    else if (flags & 1) store_tile_impl<TM, TN, OutT, true, VEC>(acc, C, ldc, mrem, nrem, row0, col0, lane);
+    else if (MAY_ROUND && sizeof(OutT) == 4 && (flags & kRoundResult)) store_tile_impl<TM, TN, OutT, false, VEC, true>(acc, C, ldc, mrem, nrem, row0, col0, lane);
     else store_tile_impl<TM, TN, OutT, false, VEC>(acc, C, ldc, mrem, nrem, row0, col0, lane);
 }
 

@@ -239,7 +239,13 @@ extern "C" int ezl_layer_fwd(const ezl_layer* l, const void* x, void* y, void* s
     const int64_t strides[8] = {row_q[0], b1 * row_q[1], row_k[0], b1 * row_k[1], row_k[0], b1 * row_k[1], row_q[0], b1 * row_q[1]};
     EZL_TRY(ezl_attn_fwd(a.q, a.k, a.v, a.ctx, a.lse, l->cu_seqlens, l->ndocs, m.T, l->s, m.nq, m.nk, m.d, l->scale, strides, st));
     EZL_TRY(ezl_gemm_bf16(a.ctx, l->wo, t.wide, m.T, m.h, m.qw, m.qw, m.qw, m.h, 1, 1, 0, 0, t.ws, t.ws_bytes, st));
-    EZL_TRY(ezl_rmsnorm_fwd(t.wide, x, l->ln2, a.n2, a.sum, a.rstd2, m.T, m.h, l->eps2, st));
+    // A small layer's result begins as the residual sum, to which the down projection adds its product in its epilogue: a launch that adds the two takes 4 us
+    // there, nearly all of it the launch.  With more to add, the epilogue waits longer for the sum than that launch takes.  us of a layer, launch and epilogue: 1024 x 256
+    // 209.4, 207.2; 2048 x 768 576, 573.4; 1531 x 4096 3020, 3027; 4000 x 2048 2662, 2675 (whole passes per layer): the lines cross between 1.6 and 6.3 million elements.
+    const int64_t bytes = m.T * m.h * 2;
+    const bool apart = (const char*)y + bytes <= (const char*)x || (const char*)x + bytes <= (const char*)y;  // (y is written before x is read for the last time)
+    const bool sum_in_epilogue = apart && m.T * m.h <= 5 << 19;
+    EZL_TRY(rmsnorm_fwd_keep_sum(t.wide, x, l->ln2, a.n2, a.sum, sum_in_epilogue ? y : nullptr, a.rstd2, m.T, m.h, l->eps2, st));
     {
         const void* w[2] = {l->wg, l->wu};
         const int64_t n[2] = {m.f, m.f};
@@ -247,6 +253,7 @@ extern "C" int ezl_layer_fwd(const ezl_layer* l, const void* x, void* y, void* s
         EZL_TRY(forward_products(2, a.n2, w, out, m.T, n, m.h, t.ws, t.ws_bytes, st));
     }
     EZL_TRY(ezl_swiglu_fwd(a.gate, a.up, a.act, m.T * m.f, st));
+    if (sum_in_epilogue) return gemm_forward_add(a.act, l->wd, y, m.T, m.h, m.f, t.ws, t.ws_bytes, st);
     EZL_TRY(ezl_gemm_bf16(a.act, l->wd, t.wide, m.T, m.h, m.f, m.f, m.f, m.h, 1, 1, 0, 0, t.ws, t.ws_bytes, st));
     return ezl_add(t.wide, a.sum, y, m.T * m.h, st);
 }

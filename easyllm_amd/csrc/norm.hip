@@ -19,7 +19,7 @@ template <int NCHUNK, bool HAS_RES>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                           const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
                                                           bf16_t* __restrict__ sum_out, float* __restrict__ rstd_out,
-                                                          int T, int h, float eps, int tpr, const RowSwap swap) {
+                                                          int T, int h, float eps, int tpr, const RowSwap swap, bf16_t* __restrict__ sum_copy) {
     __shared__ float red[2][4][4];  // [parity][row slot][wave in slot]
     const int rpb = 256 / tpr;             // row slots per block
     const int slot = threadIdx.x / tpr;    // which row slot
@@ -52,6 +52,7 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
 #pragma unroll
                     for (int i = 0; i < 8; ++i) xv[c][i] = (float)(bf16_t)(xv[c][i] + r[i]);
                     st_bf16x8(sum_out + base + col, pack8(xv[c]));
+                    if (sum_copy) st_bf16x8(sum_copy + base + col, pack8(xv[c]));
                 }
 #pragma unroll
                 for (int i = 0; i < 8; ++i) ss += xv[c][i] * xv[c][i];
@@ -301,7 +302,7 @@ template <bool HAS_RES>
 __global__ __launch_bounds__(kWideThreads) void rmsnorm_fwd_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                                         const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
                                                                         bf16_t* __restrict__ sum_out, float* __restrict__ rstd_out,
-                                                                        int T, int h, float eps) {
+                                                                        int T, int h, float eps, bf16_t* __restrict__ sum_copy) {
     __shared__ float red[2][kWideThreads / 64];
     const int h8 = h >> 3;
     int parity = 0;
@@ -317,6 +318,7 @@ __global__ __launch_bounds__(kWideThreads) void rmsnorm_fwd_wide_kernel(const bf
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = (float)(bf16_t)(v[i] + r[i]);
                 st_bf16x8(sum_out + base + c * 8, pack8(v));
+                if (sum_copy) st_bf16x8(sum_copy + base + c * 8, pack8(v));
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
@@ -394,7 +396,7 @@ int tpr_for(int h) {
 }
 
 int rmsnorm_fwd_launch(const void* x, const void* residual, const void* weight, void* y, void* sum_out, void* rstd, int64_t rows, int64_t h,
-                       float eps, const RowSwap& swap, void* stream) {
+                       float eps, const RowSwap& swap, void* stream, void* sum_copy = nullptr) {
     EZL_REQUIRE(rows >= 0 && h > 0 && h % 8 == 0 && h <= kWideMaxH, EZL_EUNSUPPORTED,
                 "ezl_rmsnorm_fwd: need h %% 8 == 0 and h <= %d (got h=%lld)", kWideMaxH, (long long)h);
     EZL_REQUIRE(rows == 0 || (x && weight && y && rstd), EZL_EINVAL, "ezl_rmsnorm_fwd: null pointer");
@@ -410,10 +412,10 @@ int rmsnorm_fwd_launch(const void* x, const void* residual, const void* weight, 
         const unsigned g = (unsigned)(rows < 512 ? rows : 512);
         if (residual)
             hipLaunchKernelGGL(rmsnorm_fwd_wide_kernel<true>, dim3(g), dim3(kWideThreads), 0, st, (const bf16_t*)x, (const bf16_t*)residual,
-                               (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, (int)rows, (int)h, eps);
+                               (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, (int)rows, (int)h, eps, (bf16_t*)sum_copy);
         else
             hipLaunchKernelGGL(rmsnorm_fwd_wide_kernel<false>, dim3(g), dim3(kWideThreads), 0, st, (const bf16_t*)x, (const bf16_t*)residual,
-                               (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, (int)rows, (int)h, eps);
+                               (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, (int)rows, (int)h, eps, (bf16_t*)sum_copy);
         EZL_LAUNCH_CHECK("ezl_rmsnorm_fwd");
         return EZL_OK;
     }
@@ -426,7 +428,7 @@ int rmsnorm_fwd_launch(const void* x, const void* residual, const void* weight, 
 #define LAUNCH(NC, RES)                                                                                             \
     hipLaunchKernelGGL((rmsnorm_fwd_kernel<NC, RES>), dim3((unsigned)grid), dim3(rpb * tpr), 0, st, (const bf16_t*)x, \
                        (const bf16_t*)residual, (const bf16_t*)weight, (bf16_t*)y, (bf16_t*)sum_out, (float*)rstd, \
-                       (int)rows, (int)h, eps, tpr, swap)
+                       (int)rows, (int)h, eps, tpr, swap, (bf16_t*)sum_copy)
     if (residual) {
         if (nchunk == 1) LAUNCH(1, true); else if (nchunk == 2) LAUNCH(2, true); else LAUNCH(4, true);
     } else {
@@ -455,6 +457,11 @@ extern "C" int ezl_rmsnorm_fwd_swapped(const void* x, const void* weight, void* 
                                        void* stream) {
     if (const int rc = swap_check("ezl_rmsnorm_fwd_swapped", d0, d1, h)) return rc;
     return rmsnorm_fwd_launch(x, nullptr, weight, y, nullptr, rstd, d0 * d1, h, eps, RowSwap{(int)d0, (int)d1}, stream);
+}
+
+int rmsnorm_fwd_keep_sum(const void* x, const void* residual, const void* weight, void* y, void* sum_out, void* sum_copy, void* rstd, int64_t rows,
+                         int64_t h, float eps, void* stream) {
+    return rmsnorm_fwd_launch(x, residual, weight, y, sum_out, rstd, rows, h, eps, RowSwap{0, 0}, stream, sum_copy);
 }
 
 namespace {

@@ -1,4 +1,4 @@
-// RMSNorm backward in two parts, for the whole-layer backward (layer.cpp; defined in norm.hip).
+// RMSNorm for the whole-layer calls (layer.cpp; defined in norm.hip): the forward that writes its sum twice, the backward in two parts.
 #pragma once
 #include "common.h"
 
@@ -8,6 +8,10 @@ struct NormWeightGrad {
     void *bf16, *f32;
     int accumulate, blocks;
 };
+
+// ezl_rmsnorm_fwd with a residual, the sum also to sum_copy (null, or 16-byte aligned and none of the other tensors)
+__attribute__((visibility("hidden"))) int rmsnorm_fwd_keep_sum(const void* x, const void* residual, const void* weight, void* y, void* sum_out,
+                                                               void* sum_copy, void* rstd, int64_t rows, int64_t h, float eps, void* stream);
 
 // ezl_rmsnorm_bwd up to the partial sums, which it leaves in `workspace` (as large as there)
 __attribute__((visibility("hidden"))) int rmsnorm_bwd_rows(const void* dy, const void* x, const void* weight, const void* rstd, const void* dresidual,

@@ -708,3 +708,29 @@ def test_embedding_of_rows_in_the_other_order(K, d0, d1, h, V, same):
         K.embed_scatter_add(ids, dy.contiguous(), ref, accumulate=accumulate)
         assert torch.equal(got, ref)
     assert torch.equal(K.embed_grad_swapped(ids, dy, V), K.embed_grad_bf16(ids, dy.contiguous(), V))
+
+
+@pytest.mark.parametrize("s,b,h,f", [(192, 2, 256, 688), (1280, 2, 1024, 1024), (1281, 2, 1024, 1024), (40, 1, 8200, 256), (301, 1, 8192, 512), (130, 3, 264, 8192)])
+def test_the_residual_sum_in_the_down_projections_epilogue(s, b, h, f):
+    """On either side of the size where a launch adds the two, norms of every kind, split reductions: the composed layer's bits, and a contiguous x of which
+    y shares nothing stays as it was."""
+    from easyllm_amd import functional as F_
+    from easyllm_amd import kernels as K_
+    print("residual sum", s, b, h, f, flush=True)
+    heads, d = 2, 64
+    sizes = [(h,), (heads * d, h), (heads * d, h), (heads * d, h), (h, heads * d), (h,), (f, h), (f, h), (h, f)]
+    ws = [rnd(*n, seed=i, scale=0.05 if len(n) > 1 else 1.0) for i, n in enumerate(sizes)]
+    x = rnd(s, b, h, seed=20)
+    before, angles = x.clone(), torch.rand(s, d // 2, device="cuda")
+    with torch.no_grad():
+        y = F_.decoder_layer(x, ((heads, heads, d), f, (1e-5, 1e-5), d ** -0.5), angles.cos(), angles.sin(), None, None, tuple(ws))
+        n1 = F_.rmsnorm(x, ws[0], 1e-5)
+        q, k, v = (F_.linear(n1, w).view(s, b, heads, d) for w in ws[1:4])
+        q, k = F_.apply_rotary_pair(q, k, angles.cos(), angles.sin(), None)
+        o = F_.linear(F_.flash_attention(q, k, v, None, d ** -0.5).view(s, b, heads * d), ws[4])
+        total, n2 = F_.add_rmsnorm(o, x, ws[5], 1e-5)
+        down = F_.linear(K_.swiglu_fwd(F_.linear(n2, ws[6]), F_.linear(n2, ws[7])), ws[8])
+        want = F_.add(down, total)
+    assert torch.equal(x, before)
+    # (the grouped launches of the one call may sum q / k / v and gate / up in another order: a rounding of bf16 in the worst element)
+    assert (y.float() - want.float()).norm() <= 4e-3 * want.float().norm() and (y.float() - want.float()).abs().max() <= 2 ** -5 * want.float().abs().max()
