@@ -50,6 +50,7 @@ SIGNATURES = {
     "ezl_embed_gather_swapped": [_vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _vp],
     "ezl_embed_grad_swapped": [_vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp],
     "ezl_transpose01": [_vp, _vp, _i64, _i64, _i64, _vp],
+    "ezl_copy_list": [_i32, _vpp, _vpp, _i64p, _vp],
     "ezl_add": [_vp, _vp, _vp, _i64, _vp],
     "ezl_cast_bf16_to_f32": [_vp, _vp, _i64, _vp],
     "ezl_cast_f32_to_bf16": [_vp, _vp, _i64, _vp],

@@ -290,6 +290,17 @@ def transpose01(x):
     return y
 
 
+def copy_list(dsts, srcs):
+    """dsts[i].copy_(srcs[i]) of contiguous GPU tensors of one shape and type each, in one launch per eight."""
+    for d, s in zip(dsts, srcs):
+        _need(d.is_cuda and s.device == d.device and d.dtype is s.dtype and d.shape == s.shape and d.is_contiguous() and s.is_contiguous(),
+              "copy_list: contiguous tensors of one shape, type and GPU")
+    n = len(dsts)
+    vp = ctypes.c_void_p * n
+    _lib.call("ezl_copy_list", n, vp(*[s.data_ptr() for s in srcs]), vp(*[d.data_ptr() for d in dsts]),
+              (ctypes.c_int64 * n)(*[d.numel() * d.element_size() for d in dsts]), _stream())
+
+
 def add(a, b):
     _bf16c(a, "a"); _bf16c(b, "b")
     _need(a.shape == b.shape, "add shape mismatch")

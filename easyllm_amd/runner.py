@@ -10,6 +10,7 @@ import torch
 
 from .registry import MODULE_ZOO_REGISTRY
 from . import functional as _F
+from . import kernels as _K
 from . import llama as _llama  # (registers the model builders)
 from .losses import CrossEntropy
 from .transformer import is_plain
@@ -67,12 +68,27 @@ def _tree_map(fn, x):
     return x
 
 
-def _tree_copy(dst, src):
+def _tree_pairs(dst, src):
     if isinstance(dst, torch.Tensor):
-        dst.copy_(src, non_blocking=True)
-    elif isinstance(dst, (tuple, list)):
-        for d, s_ in zip(dst, src):
-            _tree_copy(d, s_)
+        return [(dst, src)]
+    return [p for d, s in zip(dst, src) for p in _tree_pairs(d, s)] if isinstance(dst, (tuple, list)) else []
+
+
+def _tree_copy(dst, src):
+    """Tensors that lie alike on the current GPU in one launch; others (from the host, of another type or layout), and all of them where one is
+    part of what another is copied to, one by one in their order."""
+    pairs = _tree_pairs(dst, src)
+    device = torch.cuda.current_device()
+    alike = [type(s) is torch.Tensor and s.dtype is d.dtype and s.shape == d.shape and s.get_device() == d.get_device() == device
+             and s.is_contiguous() and d.is_contiguous() and not s.is_neg() and not s.is_conj() for d, s in pairs]
+    targets = {d.untyped_storage().data_ptr() for d, _ in pairs}
+    if any(a and s.untyped_storage().data_ptr() in targets for a, (_, s) in zip(alike, pairs)):
+        alike = [False] * len(pairs)
+    for a, (d, s) in zip(alike, pairs):
+        if not a:
+            d.copy_(s, non_blocking=True)
+    if any(alike):
+        _K.copy_list([d for a, (d, _) in zip(alike, pairs) if a], [s for a, (_, s) in zip(alike, pairs) if a])
 
 
 class GraphedStep:
@@ -141,10 +157,7 @@ class GraphedStep:
 
     def __call__(self, inputs=None, labels=None):
         self._check_previous()
-        if inputs is not None:
-            _tree_copy(self.inputs, inputs)
-        if labels is not None:
-            _tree_copy(self.labels, labels)
+        _tree_copy(*zip(*[(own, new) for own, new in ((self.inputs, inputs), (self.labels, labels)) if new is not None] or [((), ())]))
         if self._accumulate:
             for p in self._grads:  # the graph adds: a buffer marked fresh (zero_main_grads) starts from zero
                 if getattr(p, "main_grad_fresh", False):

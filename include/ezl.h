@@ -119,6 +119,8 @@ int ezl_embed_grad_swapped(const void* ids, const void* dy, void* dweight, int f
 
 /* ---- layout / dtype plumbing of llama/llama.py:145-188 (transpose, undo, float16_to_fp32) ---- */
 int ezl_transpose01(const void* x, void* y, int64_t d0, int64_t d1, int64_t inner, void* stream); /* y[j,i,:] = x[i,j,:] */
+/* bytes[i] bytes from src[i] to dst[i] (device memory, any alignment; no dst overlaps another tensor of the list), up to eight of them per launch */
+int ezl_copy_list(int count, const void* const* src, void* const* dst, const int64_t* bytes, void* stream);
 int ezl_add(const void* a, const void* b, void* out, int64_t n, void* stream); /* residual add, transformer.py:797 */
 int ezl_cast_bf16_to_f32(const void* in, void* out, int64_t n, void* stream);
 int ezl_cast_f32_to_bf16(const void* in, void* out, int64_t n, void* stream);

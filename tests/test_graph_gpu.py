@@ -92,3 +92,31 @@ def test_graphed_accumulating_step_adds_to_what_the_buffers_hold(gpu_device):
     torch.cuda.synchronize()
     for n, p in model.named_parameters():
         assert torch.equal(p.main_grad, expect_b[n]), n
+
+
+@pytest.mark.parametrize("sizes", [[1], [7, 16, 33], [4096, 4095, 1, 0, 65537], [3] * 20])
+def test_tensors_copied_in_one_launch(gpu_device, sizes):
+    """Odd numbers of bytes, tensors that do not start on 16 bytes, an empty one, more than one launch's worth: what they held, and nothing around it changed."""
+    from easyllm_amd import kernels as K
+    print("copy list", len(sizes), flush=True)
+    for dtype, offset in ((torch.int64, 0), (torch.int64, 1), (torch.uint8, 3), (torch.float32, 0)):
+        src = [torch.randint(0, 100, (n + 2 * offset,), device=gpu_device).to(dtype) for n in sizes]
+        dst = [torch.full((n + 2 * offset + 5,), 101, device=gpu_device).to(dtype) for n in sizes]
+        K.copy_list([d[offset:offset + n] for d, n in zip(dst, sizes)], [s[offset:offset + n] for s, n in zip(src, sizes)])
+        for d, s, n in zip(dst, src, sizes):
+            assert torch.equal(d[offset:offset + n], s[offset:offset + n]) and bool((d[:offset] == 101).all()) and bool((d[offset + n:] == 101).all())
+
+
+def test_inputs_of_a_graphed_step_are_copied_whatever_they_are(gpu_device):
+    """From the host, of another type, strided, part of a buffer that is copied to: as copy_ one after the other."""
+    from easyllm_amd import runner
+    own = [torch.zeros(4, 6, device=gpu_device, dtype=torch.int64) for _ in range(3)]
+    news = [torch.arange(24).view(4, 6), torch.arange(24, device=gpu_device).view(6, 4).t(), torch.ones(4, 6, device=gpu_device)]
+    runner._tree_copy(tuple(own), (news[0], news[1], news[2]))
+    assert all(torch.equal(o.cpu(), n.cpu().long()) for o, n in zip(own, news))
+    fresh = torch.arange(100, 124, device=gpu_device).view(4, 6)
+    runner._tree_copy((own[0], (own[1], None), own[2]), (fresh, (own[0], None), own[2]))  # own[0] is copied to before it is copied from
+    assert torch.equal(own[0], fresh) and torch.equal(own[1], fresh) and torch.equal(own[2].cpu(), news[2].cpu().long())
+    again = torch.arange(24, device=gpu_device).view(4, 6)
+    runner._tree_copy((own[0], [own[1]]), (again, [again + 1]))
+    assert torch.equal(own[0], again) and torch.equal(own[1], again + 1)
