@@ -75,14 +75,15 @@ def _tree_pairs(dst, src):
 
 
 def _tree_copy(dst, src):
-    """Tensors that lie alike on the current GPU in one launch; others (from the host, of another type or layout), and all of them where one is
-    part of what another is copied to, one by one in their order."""
+    """Tensors that lie alike on the current GPU in one launch; others (from the host, of another type or layout), and all of them where one (alike
+    or not) is part of what another is copied to, one by one in their order."""
     pairs = _tree_pairs(dst, src)
     device = torch.cuda.current_device()
     alike = [type(s) is torch.Tensor and s.dtype is d.dtype and s.shape == d.shape and s.get_device() == d.get_device() == device
              and s.is_contiguous() and d.is_contiguous() and not s.is_neg() and not s.is_conj() for d, s in pairs]
     targets = {d.untyped_storage().data_ptr() for d, _ in pairs}
-    if any(a and s.untyped_storage().data_ptr() in targets for a, (_, s) in zip(alike, pairs)):
+    if any(isinstance(s, torch.Tensor) and (type(s) is not torch.Tensor or s.layout is not torch.strided or s.untyped_storage().data_ptr() in targets)
+           for _, s in pairs):  # (other kinds of tensors do not say what memory they read)
         alike = [False] * len(pairs)
     for a, (d, s) in zip(alike, pairs):
         if not a:

@@ -117,6 +117,16 @@ def test_inputs_of_a_graphed_step_are_copied_whatever_they_are(gpu_device):
     fresh = torch.arange(100, 124, device=gpu_device).view(4, 6)
     runner._tree_copy((own[0], (own[1], None), own[2]), (fresh, (own[0], None), own[2]))  # own[0] is copied to before it is copied from
     assert torch.equal(own[0], fresh) and torch.equal(own[1], fresh) and torch.equal(own[2].cpu(), news[2].cpu().long())
+    sq, other = torch.zeros(5, 5, device=gpu_device), torch.zeros(5, 5, device=gpu_device)
+    whole = torch.zeros(5, 5, device=gpu_device, dtype=torch.int64)
+    news = torch.arange(25., device=gpu_device).view(5, 5)
+    for source, want in ((sq.t(), news.t()), (sq[:1].expand(5, 5), news[:1].expand(5, 5))):  # strided parts of an earlier target
+        sq.zero_()
+        runner._tree_copy((sq, other), (news, source))
+        assert torch.equal(sq, news) and torch.equal(other, want)
+    sq.zero_()
+    runner._tree_copy((sq, whole, other), (news, sq, news + 1))  # of another type, with an alike one behind it
+    assert torch.equal(whole, news.long()) and torch.equal(other, news + 1)
     again = torch.arange(24, device=gpu_device).view(4, 6)
     runner._tree_copy((own[0], [own[1]]), (again, [again + 1]))
     assert torch.equal(own[0], again) and torch.equal(own[1], again + 1)

@@ -47,6 +47,31 @@ def test_forward_without_gpu_fails_loudly():
         kernels.swiglu_fwd(torch.zeros(8, dtype=torch.bfloat16), torch.zeros(8, dtype=torch.bfloat16))
 
 
+@pytest.mark.parametrize("part", [lambda a: a.t(), lambda a: a[:1].expand(4, 4), lambda a: a.to(torch.int32).fill_(7), lambda a: a[1:].reshape(-1)[:4].expand(4, 4),
+                                  lambda a: torch.nn.Parameter(a.view(4, 4), requires_grad=False), lambda a: a])
+def test_inputs_that_are_parts_of_earlier_targets_are_copied_in_order(part, monkeypatch):
+    """As copy_ one after the other, whatever goes out in one launch (on the CPU: a list of copies, which runs last)."""
+    from easyllm_amd import runner
+
+    def copy_list(dsts, srcs):
+        for d, s in zip(dsts, srcs):
+            d.copy_(s)
+    monkeypatch.setattr(runner._K, "copy_list", copy_list)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: -1)  # (what get_device() says on the CPU)
+
+    def buffers():
+        return [torch.zeros(4, 4), torch.zeros(4, 4), torch.zeros(4, 4, dtype=torch.int64), torch.zeros(4, 4)]
+
+    def sources(own):
+        fresh = torch.arange(16.).view(4, 4)
+        return [fresh, part(own[0]), part(own[0]), fresh + 1]
+    got, want = buffers(), buffers()
+    runner._tree_copy(got, sources(got))
+    for d, s in zip(want, sources(want)):
+        d.copy_(s)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def _tiny_kwargs(**over):
     kw = dict(num_layers=2, hidden_size=64, num_attention_heads=4, vocab_size=128, seq_length=16, bf16=True,
               use_cpu_initialization=True)
