@@ -395,10 +395,13 @@ def decoder_layer(x, plan, cos, sin, position_ids, cu_seqlens, params):
 # embedding: base_modules/layers/vocab_parallel_emb.py:106-137
 # --------------------------------------------------------------------------------------------
 class EmbeddingFunction(torch.autograd.Function):
+    """transposed (ids [b, s]): the rows as [s, b, h].  (The tensor itself, no view of it: a view made in here could not be changed in place.)"""
+
     @staticmethod
-    def forward(ctx, ids, weight, host_flag=None, swapped=False):
+    def forward(ctx, ids, weight, host_flag=None, transposed=False):
         ids = ids.contiguous()
-        out, flag = K.embed_gather(ids, weight, host_flag, swapped)
+        out, flag = (K.embed_gather_transposed if transposed else K.embed_gather)(ids, weight, host_flag)
+        ctx.transposed = transposed
         ctx.save_for_backward(ids, weight)
         if flag is not None:
             ctx.mark_non_differentiable(flag)
@@ -408,6 +411,8 @@ class EmbeddingFunction(torch.autograd.Function):
     def backward(ctx, dout, _dflag):
         ids, weight = ctx.saved_tensors
         mg, acc = _main_grad_target(weight)
+        if ctx.transposed:
+            dout = dout.transpose(0, 1)
         if ids.dim() == 2 and K.rows_swapped(dout):
             return None, K.embed_grad_swapped(ids, dout, weight.shape[0], mg, acc), None, None
         if mg is not None:
@@ -533,18 +538,29 @@ def check_position_ids(position_ids, table_len):
 
 def embedding(ids, weight, sequence_first=False):
     """Row gather; raises ValueError for an id >= vocab like the reference (:107-109).  sequence_first (ids [b, s]): the rows of the
-    result [b, s, h] lie in memory as [s, b, h], so that its transposition costs nothing."""
+    result [b, s, h] lie in memory as [s, b, h], and `transposed_rows` gives them in that order at no cost."""
     pair = _held_pair(weight.device)
-    swapped = sequence_first and ids.dim() == 2 and ids.shape[0] > 1 and ids.shape[1] > 1 and ids.numel() < 2 ** 31
+    transposed = sequence_first and ids.dim() == 2 and ids.shape[0] > 1 and ids.shape[1] > 1 and ids.numel() < 2 ** 31
     if pair:
-        out, _ = EmbeddingFunction.apply(ids, weight, pair[1], swapped)
+        out, _ = EmbeddingFunction.apply(ids, weight, pair[1], transposed)
         _hold(weight.device, pair, ids, weight.shape[0])
-        return out
-    out, flag = EmbeddingFunction.apply(ids, weight, None, swapped)
-    # inside a graph capture nothing may synchronise: the flag tensor is handed to whoever captures (runner.GraphedStep),
-    # which reads it back after each replay
-    _dispatch_flag(flag, ids, weight.shape[0])
-    return out
+    else:
+        out, flag = EmbeddingFunction.apply(ids, weight, None, transposed)
+        # inside a graph capture nothing may synchronise: the flag tensor is handed to whoever captures (runner.GraphedStep),
+        # which reads it back after each replay
+        _dispatch_flag(flag, ids, weight.shape[0])
+    return out.transpose(0, 1) if transposed else out
+
+
+def transposed_rows(x):
+    """What `transpose01` gives, of an x [b, s, h] that nobody else has seen: where its rows lie in that order already, the tensor that it is a view of
+    (which, unlike a view, allows whatever the result of a kernel allows), not a copy."""
+    base = x._base
+    if not K.rows_swapped(x):
+        return transpose01(x)
+    if base is not None and base.shape == (x.shape[1], x.shape[0], x.shape[2]) and base.is_contiguous() and base.data_ptr() == x.data_ptr():
+        return base
+    return x.transpose(0, 1)  # (inference mode keeps no base)
 
 
 # --------------------------------------------------------------------------------------------
@@ -564,8 +580,6 @@ def transpose01(x):
     """[d0, d1, ...] -> contiguous [d1, d0, ...]; a free view when either extent is 1."""
     if x.shape[0] == 1 or x.shape[1] == 1:
         return x.contiguous().view((x.shape[1], x.shape[0]) + tuple(x.shape[2:]))
-    if K.rows_swapped(x):  # it lies that way already
-        return x.transpose(0, 1)
     return Transpose01Function.apply(x)
 
 

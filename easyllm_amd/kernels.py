@@ -223,18 +223,26 @@ def embed_gather(ids, weight, host_flag=None, swapped=False):
     _bf16c(weight, "weight")
     V, h = weight.shape
     if swapped:
-        d0, d1 = ids.shape
-        out = torch.empty((d1, d0, h), dtype=BF16, device=weight.device).transpose(0, 1)
-        flag = torch.zeros(1, dtype=torch.int32, device=weight.device) if host_flag is None else None
-        _lib.call("ezl_embed_gather_swapped", _p(ids), _p(weight), _p(out), _p(flag if host_flag is None else host_flag), 0 if host_flag is None else 1,
-                  d0, d1, h, V, _stream())
-        return out, flag
+        out, flag = embed_gather_transposed(ids, weight, host_flag)
+        return out.transpose(0, 1), flag
     out = torch.empty(tuple(ids.shape) + (h,), dtype=BF16, device=weight.device)
     if host_flag is not None:
         _lib.call("ezl_embed_gather_host_flag", _p(ids), _p(weight), _p(out), _p(host_flag), ids.numel(), h, V, _stream())
         return out, None
     flag = torch.zeros(1, dtype=torch.int32, device=weight.device)
     _lib.call("ezl_embed_gather", _p(ids), _p(weight), _p(out), _p(flag), ids.numel(), h, V, _stream())
+    return out, flag
+
+
+def embed_gather_transposed(ids, weight, host_flag=None):
+    """ids [d0, d1] -> rows [d1, d0, h], flag (as `ids_in_range_flag`)"""
+    _need(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and ids.dim() == 2, "ids must be contiguous int64 [d0, d1] on the GPU")
+    _bf16c(weight, "weight")
+    (d0, d1), (V, h) = ids.shape, weight.shape
+    out = torch.empty((d1, d0, h), dtype=BF16, device=weight.device)
+    flag = torch.zeros(1, dtype=torch.int32, device=weight.device) if host_flag is None else None
+    _lib.call("ezl_embed_gather_swapped", _p(ids), _p(weight), _p(out), _p(flag if host_flag is None else host_flag), 0 if host_flag is None else 1,
+              d0, d1, h, V, _stream())
     return out, flag
 
 

@@ -45,11 +45,11 @@ def float16_to_fp32(val):
     return val
 
 
-def sequence_first(x):
+def sequence_first(x, transpose=F_.transpose01):
     """[b, s, h] -> [s, b, h], of a tensor or the first of several"""
     if isinstance(x, (tuple, list)):
-        return (F_.transpose01(x[0]), *x[1:])
-    return F_.transpose01(x)
+        return (transpose(x[0]), *x[1:])
+    return transpose(x)
 
 
 def batch_first(x):
@@ -60,13 +60,20 @@ def batch_first(x):
 _EMBEDDING_FORWARD = Embedding.forward
 
 
-def _run_spec(f, following, x):
-    """f(x), laid out as the spec behind it (None: nothing is) takes it for free where both are the framework's own: the embedding's rows in
+def _plain_embedding(f):
+    return (type(f) is EmbeddingPipe and Embedding.forward is _EMBEDDING_FORWARD
+            and are_plain(((f, EmbeddingPipe), (f.word_embeddings, VocabParallelEmbedding))))
+
+
+def _run_spec(preceding, f, following, x):
+    """f(x), laid out as the spec behind it takes it for free where both are the framework's own (None: there is none): the embedding's rows in
     the layers' order, the last layer's rows left in place for a norm that reads them in the batch's order, logits in fp32 from the
-    product.  Passes over memory, four of a training step's launches (captured two-layer stack of h = 256 431 -> 424 us a step, 4 x 1000 tokens of h = 2048 2822 -> 2794)."""
-    if (following is sequence_first and type(f) is EmbeddingPipe and x[0].shape[0] > 1 and Embedding.forward is _EMBEDDING_FORWARD
-            and are_plain(((f, EmbeddingPipe), (f.word_embeddings, VocabParallelEmbedding)))):
+    product.  Passes over memory, four of a training step's launches (captured two-layer stack of h = 256 431 -> 424 us a step, 4 x 1000 tokens of h = 2048 2822 -> 2794).
+    The first layer's input is a tensor of its own, which a hook may change in place."""
+    if following is sequence_first and _plain_embedding(f) and x[0].shape[0] > 1:
         return f(x, sequence_first=True)
+    if f is sequence_first and _plain_embedding(preceding):
+        return sequence_first(x, F_.transposed_rows)
     if f is batch_first and type(following) is RMSNorm:
         x = x[0] if isinstance(x, (tuple, list)) else x
         if x.dim() == 3 and x.shape[1] > 1 and is_plain(following, RMSNorm):
@@ -154,7 +161,7 @@ class LlamaModelPipe(torch.nn.Module):
             def run(*inputs):
                 inputs = inputs[0] if len(inputs) == 1 else inputs
                 for i in range(start, end):
-                    inputs = _run_spec(funcs_all[i], funcs_all[i + 1] if i + 1 < n else None, inputs)
+                    inputs = _run_spec(funcs_all[i - 1] if i else None, funcs_all[i], funcs_all[i + 1] if i + 1 < n else None, inputs)
                 return inputs
             return run
 

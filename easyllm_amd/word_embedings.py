@@ -35,7 +35,7 @@ class Embedding(torch.nn.Module):
 
 class EmbeddingPipe(Embedding):
     def forward(self, inputs, sequence_first=False, **kwargs):
-        """sequence_first: the rows of the embeddings [b, s, h] lie in memory as [s, b, h], for a transposition right behind."""
+        """sequence_first: the rows of the embeddings [b, s, h] lie in memory as [s, b, h], for `functional.transposed_rows` right behind."""
         input_ids, position_ids, attention_mask = inputs[0], inputs[1], inputs[2]
         embeddings = super().forward(input_ids, position_ids, True) if sequence_first else super().forward(input_ids, position_ids)
         if len(inputs) == 4:

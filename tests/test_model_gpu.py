@@ -317,3 +317,44 @@ def test_rows_change_their_order_inside_the_embedding_and_the_final_norm(gpu_dev
     assert len(seen) == 4 and all(seen)
     for a, c, e in zip(got, want, saved):
         assert torch.equal(a, c) and torch.equal(a, e)
+
+
+@pytest.mark.parametrize("b,s", [(2, 160), (1, 64)])
+def test_hooks_may_change_the_first_layers_input_in_place(gpu_device, b, s):
+    """Noise added to the embeddings in place, by a hook on the first layer, against the same by a new tensor."""
+    from easyllm_amd import runner, workloads as W
+    w = dict(num_layers=2, hidden_size=256, num_attention_heads=2, num_kv_attention_heads=2, intermediate_size=512, vocab_size=1024, seq=s, batch=b,
+             seed=5)
+    model, _ = build_pair(w, gpu_device, checkpoint_activations=False)
+    inputs, (labels, loss_mask), _ = W.make_inputs(w)
+    inputs, labels = to_dev(inputs, gpu_device), (labels.to(gpu_device), loss_mask.to(gpu_device))
+    noise = torch.randn(s, b, 256, generator=torch.Generator().manual_seed(3)).bfloat16().to(gpu_device)
+    first = model.forward_funcs[3]
+
+    def result(hook):
+        handle = first.register_forward_pre_hook(hook)
+        runner.zero_main_grads(model)
+        loss = runner.forward_step(model, inputs, labels)
+        handle.remove()
+        return [loss.detach()] + [p.main_grad.clone() for p in model.parameters()]
+
+    def in_place(module, args):
+        x = args[0][0] if isinstance(args[0], tuple) else args[0]
+        assert x.is_contiguous() and x.shape == (s, b, 256) and (b == 1 or x._base is None)
+        x.add_(noise)
+
+    def anew(module, args):
+        x = args[0][0] if isinstance(args[0], tuple) else args[0]
+        return ((x + noise, *args[0][1:]) if isinstance(args[0], tuple) else x + noise,)
+
+    for got, want in zip(result(in_place), result(anew)):
+        assert torch.equal(got, want)
+
+
+def test_transposed_tensors_are_not_aliased(gpu_device):
+    """What the public transposition returns of a tensor whose rows are swapped is its own."""
+    from easyllm_amd import functional as F_
+    base = torch.randn(5, 3, 64, device=gpu_device).bfloat16()
+    x = base.transpose(0, 1)
+    y = F_.transpose01(x)
+    assert torch.equal(y, base) and y.data_ptr() != base.data_ptr()
