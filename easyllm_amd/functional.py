@@ -147,12 +147,14 @@ def _norm_reads_swapped(x):
 
 
 class RMSNormFunction(torch.autograd.Function):
-    """An x whose first two dimensions are swapped in memory (a transposed view) is read where it lies, and its gradient is laid out
-    alike: the norm behind the layers, which run in sequence order."""
+    """rows_in_place: an x whose first two dimensions are swapped in memory (a transposed view) is read where it lies, and its gradient is laid out
+    alike: the norm behind the layers, which run in sequence order.  x itself is then saved for backward, as a contiguous one is; only a caller
+    who knows that nobody changes it meanwhile asks for that.  Otherwise such an x is copied."""
 
     @staticmethod
-    def forward(ctx, x, weight, eps):
-        if _norm_reads_swapped(x):
+    def forward(ctx, x, weight, eps, rows_in_place=False):
+        ctx.rows_in_place = rows_in_place and _norm_reads_swapped(x)
+        if ctx.rows_in_place:
             y, rstd = K.rmsnorm_fwd_swapped(x, weight, eps)
             ctx.save_for_backward(x, weight, rstd)
             return y
@@ -165,9 +167,9 @@ class RMSNormFunction(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, rstd = ctx.saved_tensors
         mg, acc = _main_grad_target(weight)
-        bwd = K.rmsnorm_bwd_swapped if _norm_reads_swapped(x) else K.rmsnorm_bwd
+        bwd = K.rmsnorm_bwd_swapped if ctx.rows_in_place and _norm_reads_swapped(x) else K.rmsnorm_bwd  # (hooks may have saved it otherwise)
         dx, dw = bwd(dy.contiguous(), x, weight, rstd, main_grad=mg, accumulate=acc)
-        return dx, dw, None
+        return dx, dw, None, None
 
 
 class AddRMSNormFunction(torch.autograd.Function):
@@ -207,8 +209,8 @@ class RMSNormPassFunction(torch.autograd.Function):
         return dx, dw, None
 
 
-def rmsnorm(x, weight, eps):
-    return RMSNormFunction.apply(x, weight, eps)
+def rmsnorm(x, weight, eps, rows_in_place=False):
+    return RMSNormFunction.apply(x, weight, eps, rows_in_place)
 
 
 def rmsnorm_pass(x, weight, eps):

@@ -103,11 +103,11 @@ class RMSNorm(torch.nn.Module):
     def reset_parameters(self):
         torch.nn.init.ones_(self.weight)
 
-    def forward(self, input):
+    def forward(self, input, rows_in_place=False):
         if self.layernorm_tp_auto_sync or self.sequence_parallel:
             dist_env.sync_tp_duplicated_parameter(self.weight)  # AVG over a 1-rank group (:51-54)
         _require_bf16(input, "RMSNorm")
-        return F_.rmsnorm(input, self.weight, self.eps)
+        return F_.rmsnorm(input, self.weight, self.eps, rows_in_place)
 
     def forward_keep_input(self, x):
         """(x, norm(x)): x is returned as the residual branch so that its gradient is fused into the norm's backward."""

@@ -320,8 +320,9 @@ def test_rows_change_their_order_inside_the_embedding_and_the_final_norm(gpu_dev
 
 
 @pytest.mark.parametrize("b,s", [(2, 160), (1, 64)])
-def test_hooks_may_change_the_first_layers_input_in_place(gpu_device, b, s):
-    """Noise added to the embeddings in place, by a hook on the first layer, against the same by a new tensor."""
+def test_hooks_may_change_the_first_layers_input_and_the_last_layers_output_in_place(gpu_device, b, s):
+    """Noise added to the embeddings in place, by a hook on the first layer, against the same by a new tensor; and a kept output of the last layer that is
+    overwritten before the backward pass (of one row, where it is the norm's own input, autograd refuses that, as ever)."""
     from easyllm_amd import runner, workloads as W
     w = dict(num_layers=2, hidden_size=256, num_attention_heads=2, num_kv_attention_heads=2, intermediate_size=512, vocab_size=1024, seq=s, batch=b,
              seed=5)
@@ -329,10 +330,10 @@ def test_hooks_may_change_the_first_layers_input_in_place(gpu_device, b, s):
     inputs, (labels, loss_mask), _ = W.make_inputs(w)
     inputs, labels = to_dev(inputs, gpu_device), (labels.to(gpu_device), loss_mask.to(gpu_device))
     noise = torch.randn(s, b, 256, generator=torch.Generator().manual_seed(3)).bfloat16().to(gpu_device)
-    first = model.forward_funcs[3]
+    first, last = model.forward_funcs[3], model.forward_funcs[4]
 
-    def result(hook):
-        handle = first.register_forward_pre_hook(hook)
+    def result(hook, module=first, register="register_forward_pre_hook"):
+        handle = getattr(module, register)(hook)
         runner.zero_main_grads(model)
         loss = runner.forward_step(model, inputs, labels)
         handle.remove()
@@ -349,12 +350,32 @@ def test_hooks_may_change_the_first_layers_input_in_place(gpu_device, b, s):
 
     for got, want in zip(result(in_place), result(anew)):
         assert torch.equal(got, want)
+    if b > 1:
+        want = result(lambda m, a, out: None, last, "register_forward_hook")
+        kept = []
+        handle = model.forward_funcs[-2 if model.fp32_logits else -1].register_forward_hook(lambda m, a, out: [kept[0].zero_(), None][1])
+        got = result(lambda m, a, out: kept.append((out[0] if isinstance(out, tuple) else out).detach()), last, "register_forward_hook")
+        handle.remove()
+        for g, r in zip(got, want):
+            assert torch.equal(g, r)
 
 
 def test_transposed_tensors_are_not_aliased(gpu_device):
-    """What the public transposition returns of a tensor whose rows are swapped is its own."""
+    """What the public functions return of a tensor whose rows are swapped is its own, and what they saved of it is, too."""
     from easyllm_amd import functional as F_
     base = torch.randn(5, 3, 64, device=gpu_device).bfloat16()
     x = base.transpose(0, 1)
     y = F_.transpose01(x)
     assert torch.equal(y, base) and y.data_ptr() != base.data_ptr()
+    w = torch.randn(64, device=gpu_device).bfloat16()
+    grads = []
+    for change in (False, True):
+        leaf = base.clone().requires_grad_(True)
+        z = leaf * 1.0
+        out = F_.rmsnorm(z.transpose(0, 1), w, 1e-6)
+        if change:
+            with torch.no_grad():
+                z.zero_()
+        out.backward(torch.ones_like(out))
+        grads.append(leaf.grad)
+    assert torch.equal(*grads)
