@@ -217,6 +217,7 @@ extern "C" int ezl_layer_plan(const ezl_layer* l, int fp32) {
 extern "C" int ezl_layer_fwd(const ezl_layer* l, const void* x, void* y, void* saved, void* temp, void* st) {
     EZL_TRY(check("ezl_layer_fwd", l));
     EZL_REQUIRE(x && y && saved && temp, EZL_EINVAL, "ezl_layer_fwd: null pointer");
+    EZL_REQUIRE(ezl_aligned16(y), EZL_EINVAL, "ezl_layer_fwd: y must be 16-byte aligned");
     const Dims m(*l);
     const Saved a(m, saved);
     const ForwardTemp t(*l, m, temp);

@@ -403,7 +403,7 @@ int rmsnorm_fwd_launch(const void* x, const void* residual, const void* weight, 
     EZL_REQUIRE((residual == nullptr) == (sum_out == nullptr), EZL_EINVAL,
                 "ezl_rmsnorm_fwd: residual and sum_out go together");
     EZL_REQUIRE(ezl_aligned16(x) && ezl_aligned16(weight) && ezl_aligned16(y) && ezl_aligned16(residual) &&
-                    ezl_aligned16(sum_out),
+                    ezl_aligned16(sum_out) && ezl_aligned16(sum_copy),
                 EZL_EINVAL, "ezl_rmsnorm_fwd: pointers must be 16-byte aligned");
     if (rows == 0) return EZL_OK;
     hipStream_t st = (hipStream_t)stream;

@@ -289,7 +289,7 @@ int64_t ezl_layer_bytes(const ezl_layer* layer, int which);
 /* for tests and profiles: 1 where the backward's weight gradients, all wanted and in one type (fp32, else bf16), go out as one list of tiles (ezl_gemm_plan
  * of the seven says on which), 0 where as their operands appear; -1: bad sizes */
 int ezl_layer_plan(const ezl_layer* layer, int fp32);
-/* y = layer(x); `saved` is what ezl_layer_bwd needs, `temp` is free again when the call's work is done */
+/* y = layer(x), y on 16 bytes; `saved` is what ezl_layer_bwd needs, `temp` is free again when the call's work is done */
 int ezl_layer_fwd(const ezl_layer* layer, const void* x, void* y, void* saved, void* temp, void* stream);
 /* grads: EZL_G_COUNT entries, no two of which share memory (they are written in the kernels' order, several in one launch) */
 int ezl_layer_bwd(const ezl_layer* layer, const void* x, const void* dy, void* dx, const void* saved, void* temp,

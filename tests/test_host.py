@@ -41,6 +41,17 @@ def test_bad_arguments_are_rejected_without_a_gpu():
     assert rc == -2
 
 
+@pytest.mark.parametrize("tokens", [8, 1 << 20])
+def test_a_layers_result_has_to_be_aligned_whatever_writes_it(tokens):
+    """Small layers write it from the norm and the down projection, large ones from the addition.  (x is misaligned too: nothing is launched either way.)"""
+    from easyllm_amd import _lib
+    lib = _lib.load()
+    layer = _lib.Layer(s=tokens, b=1, h=256, nq=4, nk=4, d=64, f=512, ndocs=1, npos=tokens, eps1=1e-5, eps2=1e-5, scale=0.125, ln1=4096)
+    for y, said in ((4096 + 8, b"y must be 16-byte aligned"), (4096 + 2, b"y must be 16-byte aligned"), (4096, b"rmsnorm")):
+        assert lib.ezl_layer_fwd(ctypes.byref(layer), 4096 + 8, y, 1 << 20, 1 << 21, None) == -1
+        assert said in lib.ezl_last_error()
+
+
 def test_forward_without_gpu_fails_loudly():
     from easyllm_amd import kernels
     with pytest.raises(ValueError):
