@@ -943,9 +943,10 @@ void launch_list_256(GemmSmallArgs& a, int count, void* workspace, int64_t works
     }
 }
 
-// large tiles: the 4-wave kernel in either height, or the 8-wave one
+// large tiles: the 4-wave kernel in either height, or the 8-wave one.  ktot: length of the whole reduction, from which the workspace was sized (the K tiles of
+// several pairs can be one or two more)
 template <bool A_KC, bool B_KC, typename OutT, bool MULTI, bool KTAIL>
-void launch_large(int kind, bool lines, const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
+void launch_large(int kind, bool lines, int64_t ktot, const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int accumulate,
                   void* workspace, int64_t workspace_bytes, const KSegments& seg, hipStream_t st) {
     const int nk = MULTI ? seg.nk : (K + BK - 1) / BK;
     // (fp32 input gradients stay with the 8-wave kernel)
@@ -956,7 +957,7 @@ void launch_large(int kind, bool lines, const void* A, const void* B, void* C, i
     constexpr bool HAS_192 = HAS_W4 && (!KTAIL || !A_KC || MULTI);  // (whole_lines: the others' reductions are whole K tiles)
     if (!w4 || !HAS_192) kind = kTile256;
     const int tiles_m = (int)((M + gemm_kind_bm(kind) - 1) / gemm_kind_bm(kind)), tiles_n = (N + BN - 1) / BN;
-    const SplitPlan plan = make_plan(kind, lines, (int64_t)tiles_m * tiles_n, nk, workspace, workspace_bytes);
+    const SplitPlan plan = make_plan(kind, lines, (int64_t)tiles_m * tiles_n, (ktot + BK - 1) / BK, workspace, workspace_bytes);
     const int items = plan.full + plan.rest * plan.nsplit;
     w4 = w4 && (kind == kTile192x256 || w4_pays(form, plan, nk, ldb));
     if constexpr (HAS_W4) {
@@ -1009,9 +1010,9 @@ void launch(const void* A, const void* B, void* C, int M, int N, int K, int64_t 
         }
     }
     if (K % BK == 0)
-        launch_large<A_KC, B_KC, OutT, false, false>(kind, lines, A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, KSegments(), st);
+        launch_large<A_KC, B_KC, OutT, false, false>(kind, lines, K, A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, KSegments(), st);
     else
-        launch_large<A_KC, B_KC, OutT, false, true>(kind, lines, A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, KSegments(), st);
+        launch_large<A_KC, B_KC, OutT, false, true>(kind, lines, K, A, B, C, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, KSegments(), st);
 }
 
 // C = 0 for an empty reduction (a fill kernel rather than a memset node, so the call can be captured into a graph)
@@ -1160,7 +1161,7 @@ extern "C" int ezl_gemm_bf16_ksplit(int count, const void* const* A, const void*
         }
     }
     (tail ? launch_large<true, false, bf16_t, true, true> : launch_large<true, false, bf16_t, true, false>)(
-        kind, whole_lines(kInputGradient, M, N, ktot), A[0], B[0], C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate, workspace, workspace_bytes, seg, (hipStream_t)stream);
+        kind, whole_lines(kInputGradient, M, N, ktot), ktot, A[0], B[0], C, (int)M, (int)N, (int)K[0], lda, ldb, ldc, accumulate, workspace, workspace_bytes, seg, (hipStream_t)stream);
     EZL_LAUNCH_CHECK("ezl_gemm_bf16_ksplit");
     return EZL_OK;
 }

@@ -1,4 +1,6 @@
 """Products on 192 x 256 tiles, short reductions on the 4-wave kernel and half a chip's worth of tiles in two shares, each against fp32."""
+import ctypes
+
 import pytest
 import torch
 
@@ -58,6 +60,31 @@ def test_input_gradient_over_pairs_on_large_tiles(K, T, n_in, outs):  # noqa: F8
 @pytest.mark.parametrize("T,n_in,outs", PAIRS)
 def test_pairs_take_the_large_tiles(T, n_in, outs):
     assert _lib.gemm_plan("input gradient over pairs", [T], [n_in], sum(outs))[1:3] == (192, 256)
+
+
+# K tails that make the pairs' K tiles, rounded up one by one, enough for one share more than the workspace is for
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n_in,outs", [(201, 768, (21032, 17816)), (214, 256, (19480, 10192, 20952))])
+def test_pairs_with_tails_are_split_as_their_workspace_says(K, T, n_in, outs):  # noqa: F811
+    """The workspace that is asked for is enough for the plan: more of it changes no bit (a reduction that is not split is another sum)."""
+    print("dgrad multi, shares", T, n_in, outs, flush=True)
+    rows, cols, split = _lib.gemm_plan("input gradient over pairs", [T], [n_in], sum(outs))[1:4]
+    tiles = (T + rows - 1) // rows * ((n_in + cols - 1) // cols)
+    need = _lib.gemm_workspace_bytes(T, n_in, sum(outs))
+    assert split > 64 and need == tiles * split * rows * cols * 4 and sum((o + 63) // 64 for o in outs) // 8 == split + 1
+    dys = [rnd(T, max(outs), seed=i)[:, :o] for i, o in enumerate(outs)]
+    ws = [rnd(o, n_in, seed=10 + i) for i, o in enumerate(outs)]
+    n = len(outs)
+    ptrs, got = ctypes.c_void_p * n, []
+    for size in (need, 2 * need):
+        room, dx = torch.empty(size, dtype=torch.uint8, device="cuda"), torch.empty(T, n_in, dtype=torch.bfloat16, device="cuda")
+        _lib.call("ezl_gemm_bf16_ksplit", n, ptrs(*[d.data_ptr() for d in dys]), ptrs(*[w.data_ptr() for w in ws]), dx.data_ptr(), T, n_in,
+                  (ctypes.c_int64 * n)(*outs), max(outs), n_in, n_in, 1, 0, 0, 0, room.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+        got.append(dx)
+    assert torch.equal(*got)
+    A, B = torch.cat([d.contiguous() for d in dys], 1), torch.cat(ws, 0)
+    ref = A.float() @ B.float()
+    assert ((got[0].float() - ref).abs() <= gemm_bound(A, B) + ref.abs() * 2.0 ** -8 + 1e-6).all()
 
 
 # (form, M, N, K, shares): every count of partial tiles that are added at a time (8, 4, 2, 1), edges inside the last vector
