@@ -93,6 +93,7 @@ _SPECIAL = {
     "ezl_gemm_workspace_bytes": ([_i64, _i64, _i64], _i64),
     "ezl_gemm_group_workspace_bytes": ([_i32, _i64p, _i64p, _i64], _i64),
     "ezl_gemm_group_form_workspace_bytes": ([_i32, _i32, _i64p, _i64p, _i64], _i64),
+    "ezl_gemm_searches": ([], _i64),
     "ezl_gemm_plan": ([_i32, _i32, _i64p, _i64p, _i64] + [ctypes.POINTER(_i32)] * 4, _i32),
     "ezl_layer_plan": ([_layerp, _i32], _i32),
     "ezl_layer_bytes": ([_layerp, _i32], _i64),

@@ -684,8 +684,8 @@ constexpr Rates kRates[3][kGemmKinds] = {
     {{0.986, 1.397, 6.138, 4.844, 1.422, 0}, {0.824, 1.098, 5.446, 3.786, 1.472, 0.01}, {0.713, 0.833, 3.462, 2.866, 2.656, 0.187}, {0.5, 0.66, 2.704, 3.02, 0.992, 0.143}, {0.637, 0.943, 3.112, 1.208, 4.766, 0.184}, {0.307, 0.464, 2.735, 0.783, 6, 0.372}, {0.115, 0.203, 2.294, 2.438, 0.3, 0.259}},
     {{1.088, 1.404, 7.566, 6.16, 1.4, 0.063}, {0.909, 1.098, 7.463, 3.783, 1.767, 0.087}, {0.665, 0.815, 5.6, 2.887, 0.602, 0.184}, {0.426, 0.669, 3.605, 2.771, 0.3, 0.189}, {0.553, 0.931, 2.861, 2.219, 1.454, 0.16}, {0.276, 0.457, 3.539, 0.1, 6, 0.263}, {0.148, 0.228, 2.623, 2.118, 0.3, 0.309}}};
 constexpr Rates kOtherRates[2][kGemmKinds] = {
-    {{0.72, 1.3, 0, 8.8, 1, 0}, {1e6, 1e6, 0, 0, 1, 0}, {0.57, 0.71, 0, 6.5, 3, 0}, {0.54, 0.57, 0, 5.4, 3, 0}, {0.69, 0.94, 0, 3.25, 99, 0}, {0.275, 0.43, 0, 2.6, 99, 0}, {0.187, 0.2, 0, 3.3, 3, 0}},
-    {{1.18, 1.3, 0, 12.5, 1, 0}, {1e6, 1e6, 0, 0, 1, 0}, {0.74, 0.83, 0, 8, 3, 0}, {0.61, 0.695, 0, 6, 3, 0}, {0.64, 0.8, 0, 5, 99, 0}, {0.265, 0.45, 0, 2.7, 99, 0}, {0.21, 0.218, 0, 3.1, 3, 0}}};
+    {{0.72, 1.3, 0, 8.8, 1, 0}, {}, {0.57, 0.71, 0, 6.5, 3, 0}, {0.54, 0.57, 0, 5.4, 3, 0}, {0.69, 0.94, 0, 3.25, 99, 0}, {0.275, 0.43, 0, 2.6, 99, 0}, {0.187, 0.2, 0, 3.3, 3, 0}},
+    {{1.18, 1.3, 0, 12.5, 1, 0}, {}, {0.74, 0.83, 0, 8, 3, 0}, {0.61, 0.695, 0, 6, 3, 0}, {0.64, 0.8, 0, 5, 99, 0}, {0.265, 0.45, 0, 2.7, 99, 0}, {0.21, 0.218, 0, 3.1, 3, 0}}};
 // The partial tiles of 256 and 192 x 256 are added faster (gemm_split_reduce_kernel): 11 MB/us is the rate between 8 and 18 with the least loss over 80
 // products whose plan it decides, 2.1 % faster in the mean than with 8, at worst 2.4 % slower.  Of 20000 other products it changes the plan of 640; 110 of those are 5.8 % faster
 // in the mean, 18 slower by 1 - 7 % and one by 16 (14933 x 256 x 5504).  M x N x K, us with tiles x shares as with 8 and now: input gradient 3175 x 512 x
@@ -695,22 +695,33 @@ constexpr double kReduceFixed = 4.0, kReduceBytesPerUs = 8e6, kLargeReduceBytesP
 double reduce_cost(int64_t tiles, int64_t tile_elems, int64_t nsplit, double bytes_per_us = kReduceBytesPerUs) {
     return kReduceFixed + (double)tiles * tile_elems * nsplit * 8 / bytes_per_us;
 }
+// What share of the way from `low` to `high` the rate goes with `groups` of kCus workgroups on the chip, of kRates' three rows and kOtherRates' two: the powers
+// would be most of a search.
+double way_up(int row, int kind, int64_t groups) {
+    static const auto table = [] {
+        static double t[5][kGemmKinds][kCus + 1];
+        for (int r = 0; r < 5; ++r)
+            for (int k = 0; k < kGemmKinds; ++k)
+                for (int g = 0; g <= kCus; ++g) t[r][k][g] = pow((double)g / kCus, (r < 3 ? kRates[r] : kOtherRates[r - 3])[k].power);
+        return &t;
+    }();
+    return (*table)[row][kind][groups];
+}
 // us of a launch of `tiles` tiles, results of out_mb MB
-double cost_large(const Rates& rate, int kind, bool lines, int64_t tiles, int64_t nk, int64_t room, double out_mb) {
+double cost_large(const Rates& rate, int row, int kind, bool lines, int64_t tiles, int64_t nk, int64_t room, double out_mb) {
     const SplitPlan p = make_plan(kind, lines, tiles, nk, (void*)16, room);
-    auto round = [&](int64_t groups, int64_t k) { return k * (rate.low + (rate.high - rate.low) * pow((double)groups / kCus, rate.power)) + rate.next; };
+    auto round = [&](int64_t groups, int64_t k) { return k * (rate.low + (rate.high - rate.low) * way_up(row, kind, groups)) + rate.next; };
     double t = rate.first + rate.out * out_mb + (p.full / kCus) * (nk * rate.high + rate.next);
     if (p.full % kCus) t += round(p.full % kCus, nk);
     if (p.nsplit > 1) t += round(p.rest * p.nsplit, (nk + p.nsplit - 1) / p.nsplit) + reduce_cost(p.rest, tile_bytes(kind) / 4, p.nsplit, lines ? kLargeReduceBytesPerUs : kReduceBytesPerUs);
     return t;
 }
-double cost_small(const Rates& rate, int kind, int64_t tiles, int64_t nk, int64_t nsplit, double out_mb) {
+double cost_small(const Rates& rate, int row, int kind, int64_t tiles, int64_t nk, int64_t nsplit, double out_mb) {
     const int64_t groups = tiles * nsplit, share = (nk + nsplit - 1) / nsplit;
     const bool two = kind == kTile128 || kind == kTile64;  // workgroups per CU
     const int64_t slots = two ? 2 * kCus : kCus, rest = groups % slots;
     double t = rate.first + rate.out * out_mb + (groups / slots) * (share * rate.high + rate.next);
-    const double fill = rest < kCus ? (double)rest / kCus : 1.0;
-    if (rest) t += share * (rate.low + (rate.high - rate.low) * pow(fill, rate.power)) + rate.next;
+    if (rest) t += share * (rate.low + (rate.high - rate.low) * way_up(row, kind, rest < kCus ? rest : kCus)) + rate.next;
     if (nsplit > 1) t += reduce_cost(tiles, gemm_kind_bm(kind) * gemm_kind_bn(kind), nsplit);
     return t;
 }
@@ -734,6 +745,7 @@ constexpr double kMarginList256 = 0.93;
 GemmPlan find_plan(Class cls, bool lines, int count, const int64_t* M, const int64_t* N, int64_t nk, int64_t room, double* time = nullptr, bool list_256 = false) {
     const bool wgrad = cls == kWeightGradient;
     const Rates* rates = lines ? kRates[cls] : kOtherRates[wgrad];
+    const int row = lines ? cls : 3 + wgrad;
     double out_mb = 0;
     for (int i = 0; i < count; ++i) out_mb += (double)M[i] * N[i] * (wgrad ? 4e-6 : 2e-6);
     // 128 x 128 tiles read every operand most often, which lists of weight gradients over many tokens feel: a layer's seven over 11918 tokens at
@@ -750,10 +762,10 @@ GemmPlan find_plan(Class cls, bool lines, int count, const int64_t* M, const int
         int64_t tiles = 0;
         for (int i = 0; i < count; ++i) tiles += tiles_of(kTile256, M[i], N[i]);
         if (wgrad && count == 1 && tiles >= 2 * kCus) margin = 1.08;
-        t_best = cost_large(rates[kTile256], kTile256, lines, tiles, nk, room, out_mb) / (list_256 ? kMarginList256 : 1);
+        t_best = cost_large(rates[kTile256], row, kTile256, lines, tiles, nk, room, out_mb) / (list_256 ? kMarginList256 : 1);
     }
-    if (count == 1) {
-        const double t = cost_large(rates[kTile192x256], kTile192x256, lines, tiles_of(kTile192x256, M[0], N[0]), nk, room, out_mb);
+    if (count == 1 && lines) {  // (no rates for others)
+        const double t = cost_large(rates[kTile192x256], row, kTile192x256, lines, tiles_of(kTile192x256, M[0], N[0]), nk, room, out_mb);
         if (t * margin < t_best && nk >= 2) {
             t_best = t * margin;
             best.kind = kTile192x256;
@@ -767,7 +779,7 @@ GemmPlan find_plan(Class cls, bool lines, int count, const int64_t* M, const int
             if (s > 1 && (kind == kTile64Waves || nk / s < 4 || tiles * s > 4 * kCus ||
                           tiles * s * gemm_kind_bm(kind) * gemm_kind_bn(kind) * 4 > room))
                 break;
-            const double t = cost_small(rates[kind], kind, tiles, nk, s, out_mb) * (kind == kTile128 ? list_128 : 1);
+            const double t = cost_small(rates[kind], row, kind, tiles, nk, s, out_mb) * (kind == kTile128 ? list_128 : 1);
             if (t * margin < t_best) {
                 t_best = t * margin;
                 best.kind = kind;
@@ -778,7 +790,14 @@ GemmPlan find_plan(Class cls, bool lines, int count, const int64_t* M, const int
     if (time) *time = best.kind == kTile256 ? t_best : t_best / margin;
     return best;
 }
-// The search takes 3 us, as long as a small product: a thread remembers its last 256 products by their sizes.
+// A search takes 0.3 us and more, and each product of a step is asked for twice, when its workspace is sized and when it is launched: a thread remembers
+// 256 products of a class by sizes and room, and 256 workspaces (below).  The planning of a layer's nine products, each sized and launched, 1167 tokens, h = 256,
+// 768, 1024: 0.1 us each, the first time 4.4, 7.1, 6.3; with one slot for whatever room, where the two questions throw each other out, and the powers computed
+// in every search 6.9, 10.8, 10.4 and 14, 21, 20.
+uint64_t memo_slot(int64_t M, int64_t N, int64_t K, int64_t room) {
+    return (uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ K * 0x165667B19E3779F9ull ^ room * 0xD6E8FEB86659FD93ull) >> 56;
+}
+thread_local int64_t searches = 0;  // (ezl_gemm_searches)
 GemmPlan choose_plan(Class cls, int64_t M, int64_t N, int64_t K, int64_t room) {
     const int64_t nk = (K + BK - 1) / BK;
     struct Entry {
@@ -786,8 +805,11 @@ GemmPlan choose_plan(Class cls, int64_t M, int64_t N, int64_t K, int64_t room) {
         GemmPlan plan;
     };
     static thread_local Entry memo[3][256] = {};
-    Entry& e = memo[cls][(uint64_t)(M * 0x9E3779B97F4A7C15ull ^ N * 0xC2B2AE3D27D4EB4Full ^ K * 0x165667B19E3779F9ull) >> 56];
-    if (e.M != M || e.N != N || e.K != K || e.room != room) e = {M, N, K, room, find_plan(cls, whole_lines(cls, M, N, K), 1, &M, &N, nk, room)};
+    Entry& e = memo[cls][memo_slot(M, N, K, room)];
+    if (e.M != M || e.N != N || e.K != K || e.room != room) {
+        e = {M, N, K, room, find_plan(cls, whole_lines(cls, M, N, K), 1, &M, &N, nk, room)};
+        ++searches;
+    }
     return e.plan;
 }
 int64_t small_plan_bytes(const GemmPlan& p, int count, const int64_t* M, const int64_t* N) {
@@ -858,19 +880,30 @@ bool group_plan(bool wgrad, int count, const int64_t* M, const int64_t* N, int64
     return g.one;
 }
 // workspace of a product's plan, whichever form it has; the 256 x 256 kernels' own where a launch has to fall back to them
-int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
+int64_t find_bytes(int64_t M, int64_t N, int64_t K) {
     const int64_t nk = (K + BK - 1) / BK, tiles = tiles_of(kTile256, M, N);
     int64_t most = split_bytes(kTile256, false, tiles, nk);
-    for (int cls = 0; cls < 3; ++cls) {
-        const GemmPlan q = choose_plan((Class)cls, M, N, K, INT64_MAX);
-        const bool lines = whole_lines((Class)cls, M, N, K);
+    for (const Class cls : {kForward, kInputGradient, kWeightGradient}) {
+        const bool lines = whole_lines(cls, M, N, K);
+        if (cls == kInputGradient && !lines) continue;  // (the rates of a forward product)
+        const GemmPlan q = find_plan(cls, lines, 1, &M, &N, nk, INT64_MAX);
+        ++searches;
         const int64_t large = split_bytes(kTile256, lines, tiles, nk);  // (also where its results have to be stored by the 8-wave kernel)
         most = large > most ? large : most;
         const int64_t small = gemm_kind_large(q.kind) ? split_bytes(q.kind, lines, tiles_of(q.kind, M, N), nk) : small_plan_bytes(q, 1, &M, &N);
         most = small > most ? small : most;
     }
     return most;
+}
+int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    struct Entry {
+        int64_t M, N, K, bytes;
+    };
+    static thread_local Entry memo[256] = {};
+    Entry& e = memo[memo_slot(M, N, K, 0)];
+    if (e.M != M || e.N != N || e.K != K) e = {M, N, K, find_bytes(M, N, K)};
+    return e.bytes;
 }
 
 // Which 256 x 256 kernel: the 4-wave one moves a third fewer LDS bytes and has its operands longer on the way; the 8-wave one hides more inside a
@@ -1276,6 +1309,7 @@ int gemm_list(int count, const void* const* A, const void* const* B, void* const
     return EZL_OK;
 }
 
+extern "C" int64_t ezl_gemm_searches(void) { return searches; }
 extern "C" int ezl_gemm_plan(int form, int count, const int64_t* M, const int64_t* N, int64_t K, int* rows, int* cols, int* split, int* waves) {
     if (form < 0 || form > 3 || count < 1 || count > kMaxProblems || (form > 1 && count > 1) || !M || !N || K <= 0 || !rows || !cols || !split || !waves)
         return -1;

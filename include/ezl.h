@@ -161,6 +161,8 @@ int64_t ezl_gemm_group_form_workspace_bytes(int a_kc, int count, const int64_t* 
  * reduction is split (of 256 x 256 tiles: of those in the last round), waves of a workgroup (of 256 x 256 tiles: 4, or 8 for the kernel
  * that takes one tile each).  Returns 1, or 0 where several products go out one by one (then as what they would take in one launch); -1: bad sizes. */
 int ezl_gemm_plan(int form, int count, const int64_t* M, const int64_t* N, int64_t K, int* rows, int* cols, int* split, int* waves);
+/* for tests and profiles: how often the calling thread has searched for the plan of a single product (a repeated question is answered from memory) */
+int64_t ezl_gemm_searches(void);
 int ezl_gemm_bf16_group(int count, const void* const* A, const void* const* B, void* const* C, const int64_t* M, const int64_t* N,
                         int64_t K, const int64_t* lda, const int64_t* ldb, const int64_t* ldc, int a_kc, int b_kc, int out_dtype,
                         const int* accumulate, void* workspace, int64_t workspace_bytes, void* stream);

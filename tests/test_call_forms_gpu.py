@@ -395,3 +395,26 @@ def test_embedding_gradient_with_frequent_ids(K, V, h, rows, counts, accumulate)
     assert torch.equal(out.cpu(), ref + old if accumulate else ref)
     if not accumulate:
         assert torch.equal(K.embed_grad_bf16(ids.cuda(), dy.cuda(), V).cpu(), ref.bfloat16())
+
+
+@pytest.mark.parametrize("s,b,h,f", [(512, 2, 256, 688), (389, 3, 1024, 2816), (389, 1, 768, 2048)])
+def test_plans_of_a_repeated_step_are_not_searched_for_again(gpu_device, s, b, h, f):
+    """A layer in one native call, forward and backward, which sizes its products' workspaces and launches them in turn: the second time nothing is searched for."""
+    from easyllm_amd import _lib
+    from easyllm_amd import functional as F_
+    print("searches", s, b, h, f, flush=True)
+    heads, d = h // 64, 64
+    sizes = [(h,), (h, h), (h, h), (h, h), (h, h), (h,), (f, h), (f, h), (h, f)]
+    ws = [rnd(*n, seed=i, scale=0.05 if len(n) > 1 else 1.0).requires_grad_(True) for i, n in enumerate(sizes)]
+    x, angles = rnd(s, b, h, seed=20).requires_grad_(True), torch.rand(s, d // 2, device=gpu_device)
+
+    def step():
+        before = _lib.load().ezl_gemm_searches()
+        y = F_.decoder_layer(x, ((heads, heads, d), f, (1e-5, 1e-5), d ** -0.5), angles.cos(), angles.sin(), None, None, tuple(ws))
+        grads = torch.autograd.grad(y, [x] + ws, y.detach())
+        assert all(torch.isfinite(g).all() for g in grads)
+        return _lib.load().ezl_gemm_searches() - before
+
+    with torch.autograd.set_multithreading_enabled(False):  # (a thread remembers its own)
+        assert step() > 0
+        assert step() == 0 and step() == 0
