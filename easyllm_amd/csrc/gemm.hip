@@ -790,6 +790,17 @@ GemmPlan find_plan(Class cls, bool lines, int count, const int64_t* M, const int
     if (time) *time = best.kind == kTile256 ? t_best : t_best / margin;
     return best;
 }
+// One product.  kRates take too little for what a split costs where the tiles are 64 x 64: they ask for twice the shares that are fastest, or for whole tiles
+// of eight waves where shares are faster.  Where they end at such tiles and kOtherRates at shares, the latter's plan is taken.  Time of kRates' plan over that one, 600 such
+// products of 128 - 8192 wide operands and 64 - 16384 rows, everything in the caches and weights from HBM: 64 x 64 in more shares 1.09, 1.12 (forward), 1.08, 1.11
+// (input gradients) and 1.06, 1.09 (weight gradients), whole 64 x 64 tiles instead of shares 0.91, 1.26 (forward and input gradients).  M x N x K, weights from HBM, us:
+// 605 x 384 x 2560 in 8 shares 12.9, in 4 11.2; 376 x 576 x 3328 9, 4 14.0, 11.8; weight gradient 576 x 512 x 2989 7, 3 14.6, 12.8; 191 x 320 x 1728 whole 11.4, in 6 9.0.
+GemmPlan find_plan(Class cls, bool lines, int64_t M, int64_t N, int64_t nk, int64_t room) {
+    const GemmPlan plan = find_plan(cls, lines, 1, &M, &N, nk, room);
+    if (!lines || (plan.kind != kTile64 && plan.kind != kTile64Waves)) return plan;
+    const GemmPlan other = find_plan(cls, false, 1, &M, &N, nk, room);
+    return other.nsplit > 1 ? other : plan;
+}
 // A search takes 0.3 us and more, and each product of a step is asked for twice, when its workspace is sized and when it is launched: a thread remembers
 // 256 products of a class by sizes and room, and 256 workspaces (below).  The planning of a layer's nine products, each sized and launched, 1167 tokens, h = 256,
 // 768, 1024: 0.1 us each, the first time 4.4, 7.1, 6.3; with one slot for whatever room, where the two questions throw each other out, and the powers computed
@@ -807,7 +818,7 @@ GemmPlan choose_plan(Class cls, int64_t M, int64_t N, int64_t K, int64_t room) {
     static thread_local Entry memo[3][256] = {};
     Entry& e = memo[cls][memo_slot(M, N, K, room)];
     if (e.M != M || e.N != N || e.K != K || e.room != room) {
-        e = {M, N, K, room, find_plan(cls, whole_lines(cls, M, N, K), 1, &M, &N, nk, room)};
+        e = {M, N, K, room, find_plan(cls, whole_lines(cls, M, N, K), M, N, nk, room)};
         ++searches;
     }
     return e.plan;
@@ -886,7 +897,7 @@ int64_t find_bytes(int64_t M, int64_t N, int64_t K) {
     for (const Class cls : {kForward, kInputGradient, kWeightGradient}) {
         const bool lines = whole_lines(cls, M, N, K);
         if (cls == kInputGradient && !lines) continue;  // (the rates of a forward product)
-        const GemmPlan q = find_plan(cls, lines, 1, &M, &N, nk, INT64_MAX);
+        const GemmPlan q = find_plan(cls, lines, M, N, nk, INT64_MAX);
         ++searches;
         const int64_t large = split_bytes(kTile256, lines, tiles, nk);  // (also where its results have to be stored by the 8-wave kernel)
         most = large > most ? large : most;

@@ -256,3 +256,19 @@ def test_attention_takes_the_kernels_it_is_listed_under(want, case):
     (11008, 4096, 1531, 256), (32000, 768, 1024, 128)])
 def test_weight_gradients_of_a_vocabulary_take_smaller_tiles_only_by_a_margin(M, N, T, tile):
     assert _lib.gemm_plan("weight gradient", [M], [N], T)[1] == tile
+
+
+# (form, M, N, K, shares): us in these and in the shares that the rates of operands on whole lines ask for
+SHARES_OF_64 = [(0, 605, 384, 2560, 4),   # 11.2, 8 shares 12.9
+                (0, 376, 576, 3328, 4),   # 11.8, 9 shares 14.0
+                (1, 1551, 128, 3072, 5),  # 11.4, 10 shares 13.8
+                (1, 768, 256, 4480, 5),   # 12.7, 10 shares 14.8
+                (2, 576, 512, 2989, 3),   # 12.8, 7 shares 14.6
+                (2, 1728, 192, 3250, 3),  # 13.3, 6 shares 15.0
+                (0, 191, 320, 1728, 6),   # 9.0, whole (8 waves) 11.4
+                (1, 386, 256, 1920, 6)]   # 9.6, whole 11.9
+
+
+@pytest.mark.parametrize("form,M,N,K,shares", SHARES_OF_64)
+def test_short_products_are_split_as_finely_as_pays(form, M, N, K, shares):
+    assert _lib.gemm_plan(FORMS[form], [M], [N], K) == (True, 64, 64, shares, 4)
