@@ -551,18 +551,18 @@ def embedding(ids, weight, sequence_first=False):
         # inside a graph capture nothing may synchronise: the flag tensor is handed to whoever captures (runner.GraphedStep),
         # which reads it back after each replay
         _dispatch_flag(flag, ids, weight.shape[0])
-    return out.transpose(0, 1) if transposed else out
+    if not transposed:
+        return out
+    x = out.transpose(0, 1)
+    x.rows_in_memory_order = out
+    return x
 
 
 def transposed_rows(x):
-    """What `transpose01` gives, of an x [b, s, h] that nobody else has seen: where its rows lie in that order already, the tensor that it is a view of
-    (which, unlike a view, allows whatever the result of a kernel allows), not a copy."""
-    base = x._base
-    if not K.rows_swapped(x):
-        return transpose01(x)
-    if base is not None and base.shape == (x.shape[1], x.shape[0], x.shape[2]) and base.is_contiguous() and base.data_ptr() == x.data_ptr():
-        return base
-    return x.transpose(0, 1)  # (inference mode keeps no base)
+    """`transpose01`, but of what `embedding` returned with sequence_first the tensor that it is a view of: no copy, and, unlike a view, it allows whatever
+    the result of a kernel allows."""
+    rows = getattr(x, "rows_in_memory_order", None)
+    return transpose01(x) if rows is None else rows
 
 
 # --------------------------------------------------------------------------------------------

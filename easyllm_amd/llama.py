@@ -13,7 +13,6 @@ import torch
 
 from . import dist_env
 from . import functional as F_
-from . import kernels as K
 from .checkpointing import checkpoint
 from .default_cfg import update_model_cfg
 from .layers import LayerSpec, RMSNorm, VocabParallelEmbedding, build_layer_norm
@@ -46,11 +45,11 @@ def float16_to_fp32(val):
     return val
 
 
-def sequence_first(x, transpose=F_.transpose01):
+def sequence_first(x):
     """[b, s, h] -> [s, b, h], of a tensor or the first of several"""
     if isinstance(x, (tuple, list)):
-        return (transpose(x[0]), *x[1:])
-    return transpose(x)
+        return (F_.transposed_rows(x[0]), *x[1:])
+    return F_.transposed_rows(x)
 
 
 def batch_first(x):
@@ -61,27 +60,21 @@ def batch_first(x):
 _EMBEDDING_FORWARD = Embedding.forward
 
 
-def _plain_embedding(f):
-    return (type(f) is EmbeddingPipe and Embedding.forward is _EMBEDDING_FORWARD
-            and are_plain(((f, EmbeddingPipe), (f.word_embeddings, VocabParallelEmbedding))))
-
-
 def _run_spec(preceding, f, following, x):
     """f(x), laid out as the spec behind it takes it for free where both are the framework's own (None: there is none): the embedding's rows in
     the layers' order, the last layer's rows left in place for a norm that reads them in the batch's order, logits in fp32 from the
     product.  Passes over memory, four of a training step's launches (captured two-layer stack of h = 256 431 -> 424 us a step, 4 x 1000 tokens of h = 2048 2822 -> 2794).
     Where a hook sees a tensor that a pass made, the pass stays: the first layer's input is a tensor of its own, which may be changed in place, and so is the final
     norm's, whatever becomes of the last layer's output."""
-    if following is sequence_first and _plain_embedding(f) and x[0].shape[0] > 1:
+    if (following is sequence_first and type(f) is EmbeddingPipe and x[0].shape[0] > 1 and Embedding.forward is _EMBEDDING_FORWARD
+            and are_plain(((f, EmbeddingPipe), (f.word_embeddings, VocabParallelEmbedding)))):
         return f(x, sequence_first=True)
-    if f is sequence_first and _plain_embedding(preceding):
-        return sequence_first(x, F_.transposed_rows)
     if f is batch_first and type(following) is RMSNorm:
         x = x[0] if isinstance(x, (tuple, list)) else x
         if x.dim() == 3 and x.shape[1] > 1 and are_plain(((preceding, ParallelTransformerLayerPipe), (following, RMSNorm))):
             return x.transpose(0, 1)
         return batch_first(x)
-    if preceding is batch_first and type(f) is RMSNorm and K.rows_swapped(x):  # (batch_first itself leaves no such rows: the branch above did)
+    if preceding is batch_first and type(f) is RMSNorm and not x.is_contiguous():  # (batch_first itself leaves no such x: the branch above did)
         return f(x, rows_in_place=True)
     if following is float16_to_fp32 and is_plain(f, EmbedddingPipeNoTied):
         return f(x, fp32_output=True)  # (the cast then has nothing to do)
