@@ -632,9 +632,11 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(OutT* __restrict
 }
 
 enum Class { kForward, kInputGradient, kWeightGradient };
-// Products whose operands' rows are whole cache lines (128 bytes): what the rates, the 192 x 256 tiles and the wider rule for split rounds below were
-// measured on.  Rows that straddle lines cost up to 30 % more (4096 x 4096 x 4096 from rows of 8192 + 16 bytes 139 us, + 128 bytes 107), and weight
-// gradients over up to 16 K tiles are bound by their results; both keep the rates that were fitted to all widths.
+// Products whose widths are whole cache lines (128 bytes): what the rates, the 192 x 256 tiles and the wider rule for split rounds below were
+// measured on.  Other widths, and weight gradients over up to 16 K tiles, which are bound by their results, keep the rates that were fitted to all widths.
+// Only the widths are looked at, not how the rows lie: rows of a whole width that straddle lines (a column slice, a pitch of 8 elements more, a base 16 bytes off) cost up to 30 %
+// more on any tile (4096 x 4096 x 4096 103 us with such an A, 111 with both, 120 with both bases off), and the plans for whole lines are the better ones there too: of
+// 156 such products 5 - 8 % (forward), 5 - 9 % (input gradients) and 2 % (weight gradients) faster than with the rates for other widths.
 bool whole_lines(Class cls, int64_t M, int64_t N, int64_t K) {
     return N % 64 == 0 && (cls == kWeightGradient ? M % 64 == 0 && K > 16 * BK : K % 64 == 0);
 }
@@ -738,7 +740,8 @@ int64_t tiles_of(int kind, int64_t M, int64_t N) {
 //                 2283 -> 2205; at worst 2963, 1024, 2, 3392 707 -> 716
 //   0.93 - 1.00   (before the margin) 1531, 4096, 32, 11008 2180 -> 2216; 8569, 896, 14, 2976 1772 -> 1787; 1331, 3200, 25, 9984 1589 -> 1550
 // Gate and up in a forward list, by the same margin: 1726, 3072, 24, 9920 1760 -> 1709; 4952, 1792, 14, 4800 1968 -> 1923; 4000, 2048, 16, 5504
-// 1748 -> 1716; 24 random layers 0.7 % faster in the mean, none slower.  bf16 weight gradients, whether list or single: 5183, 2048, 16, 6912 2641 -> 2526;
+// 1748 -> 1716; 24 random layers 0.7 % faster in the mean, none slower.  (All of these, and kMargin256's below, with the 4-wave kernel's first form and against separate launches
+// on kOtherRates' plans, by which the two are still compared.  Separate launches of whole lines that fill the chip have become 5 - 18 % faster since, so the decision leans to lists.)  bf16 weight gradients, whether list or single: 5183, 2048, 16, 6912 2641 -> 2526;
 // 2961, 2048, 4, 5504 1288 -> 1231; 24 random layers 1.7 %, none slower.
 constexpr double kMarginList256 = 0.93;
 // `count` products over the same nk K tiles in one launch; `room`: workspace bytes.  256 x 256 tiles take one product, or with list_256 all
@@ -925,7 +928,9 @@ int64_t plan_bytes(int64_t M, int64_t N, int64_t K) {
 //   input gradient       0.99    0.98    0.98     1.00     1.04      1.06          1.06 - 1.15
 //   ... over pairs       0.99    0.98    0.97     0.99     1.02      1.06          1.05 - 1.15
 //   weight gradient      1.00    1.02    1.05     1.09     1.13      1.17          1.09 - 1.12
-// (forward in one round under 48 K tiles: the 256 x 256 tiles are hardly ever the choice there).  Several rounds of a weight gradient with the rows of B 16 KiB (or a
+// (forward in one round under 48 K tiles: the 256 x 256 tiles are hardly ever the choice there; input gradients in one round of 64 - 127 K tiles: the 4 and 2 % are not
+// taken, one line for both forms where both gain more).  The figures are of operands from HBM; with both in the caches one round of 8 - 47 K tiles of a weight gradient is 5 - 8 % slower on the
+// 4-wave kernel, with one from HBM 3 - 7 % faster, with both 6 - 10 (90 products).  Several rounds of a weight gradient with the rows of B 16 KiB (or a
 // multiple) apart, under 48 K tiles: 32000 x 8192 x 1536 0.94, 28672 x 8192 x 1536 0.96.
 // items: workgroup-sized pieces of the launch; nk: K tiles of a piece; shares: pieces are shares of a reduction
 enum class Form { forward, weight_gradient, input_gradient, input_gradient_segments };
