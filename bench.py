@@ -30,11 +30,11 @@ PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA peak
 # HBM-side bytes per GEMM launch (average over the launches of one step), from two rocprofv3 --pmc runs of this script
 # (FETCH_SIZE, WRITE_SIZE) scaled by what the same counters read for the streaming kernels of known size in the same
 # run (factor 2.0 for FETCH_SIZE, 1.0 for WRITE_SIZE); see profiles/c2_step_gemm_hbm_traffic.txt.
-GEMM_HBM_BYTES_PER_LAUNCH = {"C2": 600.9e6}
+GEMM_HBM_BYTES_PER_LAUNCH = {"C2": 592.7e6}
 
 
 def cpu_baseline(w, flops):
-    """fp32 oracle on the host cores (the thread count the box gives this process: torch's default, i.e. OMP_NUM_THREADS).
+    """fp32 oracle on the host cores (the thread count the machine gives this process: torch's default, i.e. OMP_NUM_THREADS).
     Workloads of up to 3e13 FLOPs per step run one whole fwd+bwd step; larger ones one decoder layer + final norm + LM head
     + loss, with t_step ~= L * t_layer + t_head.  Returns the dict that goes into the JSON line."""
     import torch
@@ -207,7 +207,7 @@ def measure(name, steps, warmup, mode, input_check):
 
 
 def gemm_vs_library(workload):
-    """Every GEMM launch of one training step of `workload`, this library's kernel against the box's own GEMM library
+    """Every GEMM launch of one training step of `workload`, this library's kernel against the machine's own GEMM library
     (torch.matmul / torch.mm -> hipBLASLt), timed alternately in one process on the same operands.  Prints a table and the
     step's total GEMM time under three choices: this kernel everywhere, the library everywhere, the faster of the two per
     launch -- the last is what a step could reach if every launch ran at the better of the two kernels."""
@@ -282,7 +282,7 @@ def gemm_vs_library(workload):
     wgrad("gate/up", f, h, 2 * L)
     wgrad("down", h, f, L)
     wgrad("head", V, h, 1)
-    print("GEMM launches of one %s step (M = %d tokens), this kernel against the library GEMM of the box" % (workload, T))
+    print("GEMM launches of one %s step (M = %d tokens), this kernel against the library GEMM of the machine" % (workload, T))
     print("%-66s %6s %10s %11s %8s %8s" % ("launch", "count", "this us", "library us", "this TF", "lib TF"))
     ta = tb = tm = fl = 0.0
     for name, flops, count, a, b in rows:
@@ -309,7 +309,7 @@ def main():
                          "`configs` array of the same JSON line; empty string to skip")
     ap.add_argument("--other-steps", type=int, default=6)
     ap.add_argument("--gemm-vs-library", action="store_true",
-                    help="instead of the benchmark: time every GEMM launch of one step against the box's library GEMM and print a table")
+                    help="instead of the benchmark: time every GEMM launch of one step against the machine's library GEMM and print a table")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py: this build measures one GPU's share only (TP=1, one MI355X); --gpus %d is not supported. "

@@ -16,7 +16,7 @@ OUT_DIR = os.path.join(HERE, "_ref")
 
 
 def build(verbose=True):
-    """Returns the path of the built module, or None when the reference tree is not present (e.g. on the GPU box)."""
+    """Returns the path of the built module, or None when the reference tree is not present (e.g. on a machine that only runs)."""
     if not os.path.exists(REF_SRC):
         return None
     import pybind11

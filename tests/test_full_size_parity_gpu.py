@@ -1,4 +1,4 @@
-"""Parity of the full-size benchmark workloads (C2, C3, C4, and layers 0 and 7 + head of the packed C5) with the CPU oracle, run on the host cores of the GPU box
+"""Parity of the full-size benchmark workloads (C2, C3, C4, and layers 0 and 7 + head of the packed C5) with the CPU oracle, run on the host cores beside the GPU
 on the same weights, token ids and labels.  The comparison rule (stated bar against the fp32 oracle; where a chain of
 bf16-stored ops cannot meet it, no farther from fp32 than the oracle's exact-arithmetic bf16-storage evaluation) is in
 tests/_parity.py.
